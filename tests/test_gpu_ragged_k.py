@@ -100,3 +100,25 @@ def test_ragged_k_rejections(device):
         mm.matmul(a.float(), a.float(), None, a_ragged_metadata=md, b_ragged_metadata=md)
     with pytest.raises(ValueError):
         mm.matmul(a, a, None, b_ragged_metadata=md)
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("m, n", [(8, 8), (128, 136), (264, 1032)])
+def test_ragged_k_stage_and_tile_edges(device, m, n, out_dtype):
+    """Aligned k-slow operands (transposed by the LDS reads): slice lengths around the 16-row stages and the five stage
+    buffers, tiles around 128, more and fewer tiles than XCDs, each output type."""
+    import triton_amd.matmul as mm
+    g = torch.Generator().manual_seed(m + n)
+    sizes = torch.tensor([0, 1, 15, 16, 17, 48, 64, 65, 80, 81, 96, 200], dtype=torch.int32)
+    offs = _offsets(sizes, 24)
+    k = int(offs[-1])
+    a, b = torch.randn((k, m), generator=g).to(torch.bfloat16), torch.randn((k, n), generator=g).to(torch.bfloat16)
+    for e, s in enumerate(sizes.tolist()):
+        a[int(offs[e]) + s:int(offs[e + 1])] = float("nan")
+        b[int(offs[e]) + s:int(offs[e + 1])] = float("nan")
+    out = torch.full((len(sizes), m, n), float("nan"), dtype=out_dtype, device=device)
+    md = _metadata(sizes, offs, device)
+    mm.matmul(a.to(device).t(), b.to(device), None, a_ragged_metadata=md, b_ragged_metadata=md, c=out,
+              precision_config=mm.PrecisionConfig(out_dtype=out_dtype))
+    ref = omoe.matmul_ragged_k(a.t(), b, sizes, offs, offs, out_dtype=torch.float32)
+    assert_allclose_gate(ref, out.float(), what="ragged-K matmul")

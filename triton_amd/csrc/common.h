@@ -57,6 +57,31 @@ __device__ inline uint16_t f32_to_f16_bits(float f) {
   return b;
 }
 
+// ---- memory straight into LDS ------------------------------------------------------------------
+// `u32x4` buffer resource over [base, base + bytes): loads past the range read zero.
+typedef uint32_t buf_desc_t __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ buf_desc_t make_buf_desc(const void* base, uint32_t bytes) {
+  const uint64_t a = reinterpret_cast<uint64_t>(base);
+  return buf_desc_t{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xFFFFu)),
+                    (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+}
+// 16 bytes per lane from `desc` at byte offset `off` + `soff` into LDS at `dst` (wave-uniform byte address) + 16 * lane.  Written
+// as assembly because the compiler puts a wait for ALL outstanding memory operations in front of every LDS read that
+// follows the builtin form; here the kernel places its own vmcnt waits (the instruction counts as one).
+__device__ __forceinline__ void lds_dma16(buf_desc_t desc, uint32_t dst, uint32_t off, uint32_t soff = 0) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(off), "s"(desc), "s"(soff) : "memory");
+}
+// LDS byte address of a __shared__ object
+__device__ __forceinline__ uint32_t lds_addr(const void* p) {
+  return (uint32_t)reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void*)p);
+}
+// four consecutive k of this lane's row, transposed by the LDS read: sixteen lanes read four rows (lane >> 2 of the group) of
+// sixteen 16-bit columns (four per lane) and lane i receives column i of the four rows
+__device__ __forceinline__ uint64_t lds_read_tr16(uint32_t at) {
+  typedef __attribute__((ext_vector_type(4))) short s16x4_t;
+  return __builtin_bit_cast(uint64_t, __builtin_amdgcn_ds_read_tr16_b64_v4i16(reinterpret_cast<__attribute__((address_space(3))) s16x4_t*>((uintptr_t)at)));
+}
+
 __device__ inline uint32_t f32_bits(float f) { return __builtin_bit_cast(uint32_t, f); }
 __device__ inline float bits_f32(uint32_t u) { return __builtin_bit_cast(float, u); }
 

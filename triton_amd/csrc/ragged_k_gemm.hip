@@ -36,8 +36,9 @@ struct RaggedKParams {
   const int32_t* b_offs;
   int M, N;
   int tiles_m, tiles_n;
+  int chunk, n_slices;  // aligned variant: tiles per XCD and turn
   int y_dtype;
-  uint32_t a_bytes, b_bytes;  // extents for the buffer resources of the fast variant
+  uint32_t a_bytes, b_bytes, y_bytes;  // extents for the buffer resources of the aligned variant (y: one slice)
   int a_vec, b_vec;  // the operand's base and strides allow 16-byte loads along its contiguous dimension
 };
 
@@ -46,6 +47,13 @@ constexpr int kKC = 32;     // k per pipeline stage
 constexpr int kRing = 3;   // stages of global loads in flight per thread
 constexpr int kPitch = kKC * 2 + 16;  // bytes per LDS row: 32 k + a pad that keeps 16-byte alignment and spreads banks
 
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for_n(F&& f) {
+  if constexpr (I < N) {
+    f(std::integral_constant<int, I>{});
+    static_for_n<N, I + 1>(f);
+  }
+}
 template <class F>
 __device__ __forceinline__ void static_for_ring(F&& f) {
   f(std::integral_constant<int, 0>{});
@@ -54,11 +62,8 @@ __device__ __forceinline__ void static_for_ring(F&& f) {
   static_assert(kRing == 3, "static_for_ring lists the slots");
 }
 
-// FAST: both operands are stored with the reduction index slow, 16-byte loads are possible everywhere and M and N are
-// multiples of 8 (so a thread's eight rows are all inside or all outside).  The loads then go through a buffer
-// resource with an out-of-range offset for pieces past the slice end or the matrix edge (the hardware returns zeros),
-// so no branch surrounds a load and the compiler's wait counts let all kRing stages stay in flight.
-template <int DT, bool FAST>
+// Any layout and alignment (the aligned k-slow pair runs ragged_k_tr_kernel below).
+template <int DT>
 __global__ __launch_bounds__(256) void ragged_k_gemm_kernel(const RaggedKParams p) {
   __shared__ __attribute__((aligned(16))) uint8_t lds[2][2][kTile * kPitch];  // [buffer][operand][row][k]
   const int tid = threadIdx.x;
@@ -107,28 +112,8 @@ __global__ __launch_bounds__(256) void ragged_k_gemm_kernel(const RaggedKParams 
   auto load_elem = [&](int64_t r, int64_t k) __attribute__((always_inline)) -> uint32_t {
     return *reinterpret_cast<const uint16_t*>(base + ((r0 + r) * stride_r + (k_first + k) * stride_k) * 2);
   };
-  const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(is_b ? p.b : p.a), 0,
-                                                                        is_b ? p.b_bytes : p.a_bytes, 0x00020000);
-  // byte offset of this thread's eight rows at k = 0 of the slice; kOutOfRange when the rows lie past the edge
-  constexpr uint32_t kOutOfRange = 0x80000000u;
-  const bool rows_in = r0 + rb * 8 < rows_total;
-  const uint32_t off0 = (uint32_t)(((int64_t)(r0 + rb * 8) + (int64_t)k_first * stride_k) * 2);
-  const uint32_t kstep = (uint32_t)(stride_k * 2);
   auto load_stage = [&](auto slot_c, int kc) __attribute__((always_inline)) {
     uint32_t(&pr)[16] = ring[decltype(slot_c)::value];
-    if constexpr (FAST) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int k = kc + kq * 4 + q;
-        const uint32_t off = (rows_in && k < ksz) ? off0 + (uint32_t)k * kstep : kOutOfRange;
-        const u32x4_t v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0);
-        pr[4 * q + 0] = v.x;
-        pr[4 * q + 1] = v.y;
-        pr[4 * q + 2] = v.z;
-        pr[4 * q + 3] = v.w;
-      }
-      return;
-    }
     if (k_slow) {
       const int rr = rb * 8;
       const bool full_rows = r0 + rr + 8 <= rows_total;
@@ -185,7 +170,7 @@ __global__ __launch_bounds__(256) void ragged_k_gemm_kernel(const RaggedKParams 
   auto store_stage = [&](auto slot_c, int buf) __attribute__((always_inline)) {
     uint32_t(&pr)[16] = ring[decltype(slot_c)::value];
     uint8_t* dst = my_lds0 + buf * (2 * kTile * kPitch);
-    if (FAST || k_slow) {
+    if (k_slow) {
       // pr[4q + d] = rows (2d, 2d+1) at k = kq*4 + q  ->  row i gets its four k as one 8-byte piece
 #pragma unroll
       for (int d = 0; d < 4; ++d) {
@@ -319,6 +304,210 @@ __global__ __launch_bounds__(256) void ragged_k_gemm_kernel(const RaggedKParams 
   }
 }
 
+// ---- both operands k-slow and aligned (the weight-gradient layout): transposition by the LDS read --------------------
+// A stage is kTrK k rows x 128 m (and 128 n) in the operands' own order: the rows go from memory straight into LDS
+// (buffer_load ... lds, 1 KiB = 4 k rows per wave instruction, no registers, no VALU) and ds_read_b64_tr_b16 hands a
+// lane four consecutive k of ITS row, so nothing is transposed in registers.  Row pitch 256 bytes without padding (the
+// DMA writes lane-contiguously): the 16-byte pieces of k row r are stored at piece ^ 2 * (r & 3), which puts the four
+// rows that sixteen lanes of a transposing read touch on disjoint banks.  Pieces past the slice end or the matrix edge
+// get an offset beyond the buffer resource; the hardware then writes zeros to LDS.
+//
+// What bounds it: writing y.  The same kernel without its loads writes 128 x [2880, 5760] bf16 in 0.77 ms (5.5 TB/s),
+// without its stores it takes 0.85 ms; together 1.21 ms (3.1 ms with the transposition in registers; 2880 x 2880: 1.5 -> 0.62).
+//   * the results go through LDS so that a store instruction writes whole 128-byte lines, with the non-temporal hint
+//     (pieces of 32 bytes: 1.76 ms; with the hint on such pieces 4.0, plain whole lines 1.55, whole lines with the hint 1.40);
+//   * stages of 16 k, five buffers, four workgroups per CU: four fifths of the LDS are loads in flight (three buffers
+//     of 32 k and three workgroups: 1.44), and a slice is padded to 16 k only;
+//   * every XCD gets an eighth of EVERY slice: slices differ in length by factors, and with whole slices dealt to the
+//     XCDs the longest sum decided (1.40 -> 1.21 ms); columns of tiles run first, so an XCD's eighth touches all of a and
+//     an eighth of b.
+constexpr int kTrK = 16;
+constexpr int kTrBufs = 5;
+constexpr int kTrOperand = kTrK * kTile * 2;   // bytes of one operand's stage
+constexpr int kTrStage = 2 * kTrOperand;
+constexpr int kNonTemporal = 2;  // buffer store: streaming
+
+__device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
+  const f32x2_t v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
+}
+__device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
+  const f32x2_t v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
+}
+
+template <int DT>
+__device__ __forceinline__ f32x16_t mfma_k16(u32x4_t a, u32x4_t b, f32x16_t c) {
+  if constexpr (DT == TK_BF16)
+    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
+  else
+    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
+}
+
+// YT = element type of y (TK_BF16, TK_F16, TK_F32)
+template <int DT, int YT>
+__global__ __launch_bounds__(256, 4) void ragged_k_tr_kernel(const RaggedKParams p) {
+  __shared__ __attribute__((aligned(1024))) uint8_t lds[kTrBufs * kTrStage];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int lr = lane & 31, h = lane >> 5;
+  const int mw = wave & 1, nw = wave >> 1;  // the wave's 64 x 64 quadrant
+  // chunks of an eighth of a slice's tiles, dealt to the XCDs in turn (workgroup b runs on XCD b % 8)
+  const int per_e = p.tiles_m * p.tiles_n;
+  int pid;
+  {
+    const int q = p.chunk, x = blockIdx.x & 7, l = blockIdx.x >> 3;
+    const int round = l / q;
+    pid = (round * 8 + x) * q + (l - round * q);
+  }
+  if (pid >= p.n_slices * per_e) return;
+  const int e = pid / per_e;
+  pid -= e * per_e;
+  const int tn = pid / p.tiles_m;
+  const int tm = pid - tn * p.tiles_m;
+  const int ksz = p.sizes[e];
+  const int a_k0 = p.a_offs[e], b_k0 = p.b_offs[e];
+  const int m0 = tm * kTile, n0 = tn * kTile;
+  const int nst = (ksz + kTrK - 1) / kTrK;
+  const uint32_t lds0 = lds_addr(lds);
+
+  // ---- staging: a wave's instruction covers four k rows of an operand ---------------------------------------------------
+  const buf_desc_t ra = make_buf_desc(p.a, p.a_bytes), rb = make_buf_desc(p.b, p.b_bytes);
+  constexpr uint32_t kOutOfRange = 0x80000000u;
+  const int krow = lane >> 4;                  // k row within the instruction's four
+  const int piece = (lane & 15) ^ (krow * 2);  // the 16-byte piece of the row this lane fetches
+  const int k_lane = wave * 4 + krow;
+  static_assert(kTrK == 16, "one instruction per wave, operand and stage");
+  const uint32_t a_step = (uint32_t)p.a_stride_k * 2u, b_step = (uint32_t)p.b_stride_k * 2u;
+  // (a lane whose columns lie past the edge has no k in range)
+  const int a_k = m0 + piece * 8 < p.M ? k_lane : ksz, b_k = n0 + piece * 8 < p.N ? k_lane : ksz;
+  const uint32_t a_off = (uint32_t)(a_k0 + k_lane) * a_step + (uint32_t)(m0 + piece * 8) * 2u;
+  const uint32_t b_off = (uint32_t)(b_k0 + k_lane) * b_step + (uint32_t)(n0 + piece * 8) * 2u;
+  auto issue = [&](int c, uint32_t buf) __attribute__((always_inline)) {
+    const uint32_t dst = lds0 + buf + wave * 1024;
+    const int k = c * kTrK;
+    lds_dma16(ra, dst, a_k + k < ksz ? a_off + (uint32_t)k * a_step : kOutOfRange);
+    lds_dma16(rb, dst + kTrOperand, b_k + k < ksz ? b_off + (uint32_t)k * b_step : kOutOfRange);
+  };
+
+  f32x16_t acc[2][2];  // [n fragment][m fragment]
+#pragma unroll
+  for (int f = 0; f < 2; ++f)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) acc[f][j][i] = 0.f;
+
+  // ---- fragment reads: lane addresses of a transposing read (row (lane & 15) >> 2 of four k, four columns) ------------
+  const int l16 = lane & 15;
+  const int v = ((((lane >> 4) & 1) * 2) + ((l16 & 3) >> 1)) ^ ((l16 >> 2) * 2);
+  const uint32_t rd0 = lds0 + (uint32_t)((h * 8 + (l16 >> 2)) * (kTile * 2) + (l16 & 1) * 8);
+  // (the second fragment of a quadrant flips piece bit 2, which the rows' exclusive-or also touches)
+  const uint32_t frag_a[2] = {rd0 + mw * 128 + v * 16, rd0 + mw * 128 + (v ^ 4) * 16};
+  const uint32_t frag_b[2] = {rd0 + kTrOperand + nw * 128 + v * 16, rd0 + kTrOperand + nw * 128 + (v ^ 4) * 16};
+  auto read_frag = [&](uint32_t at) __attribute__((always_inline)) -> u32x4_t {
+    const uint64_t lo = lds_read_tr16(at), hi = lds_read_tr16(at + 4 * kTile * 2);
+    return u32x4_t{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
+  };
+  auto compute = [&](uint32_t buf) __attribute__((always_inline)) {
+    u32x4_t af[2], bf[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) af[j] = read_frag(frag_a[j] + buf);
+#pragma unroll
+    for (int f = 0; f < 2; ++f) bf[f] = read_frag(frag_b[f] + buf);
+#pragma unroll
+    for (int f = 0; f < 2; ++f)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[f][j] = mfma_k16<DT>(bf[f], af[j], acc[f][j]);
+  };
+
+  constexpr uint32_t kLast = (kTrBufs - 1) * kTrStage;
+  uint32_t rd = 0, wr = kLast;
+  if (nst > 0) {
+    static_for_n<kTrBufs - 1>([&](auto i_c) __attribute__((always_inline)) {
+      if (decltype(i_c)::value < nst) issue(decltype(i_c)::value, decltype(i_c)::value * kTrStage);
+    });
+    static_assert(kTrBufs == 5, "the wait counts below list the stages that may be outstanding");
+    for (int c = 0; c < nst; ++c) {
+      // this wave's two pieces of stage c have landed when only those of the younger stages are outstanding
+      const int ahead = nst - 1 - c;
+      if (ahead >= 3)
+        asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+      else if (ahead == 2)
+        asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+      else if (ahead == 1)
+        asm volatile("s_waitcnt vmcnt(2)" ::: "memory");
+      else
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      // ... and everybody's behind the barrier; the buffer of stage c - 1 has been read
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (c + kTrBufs - 1 < nst) issue(c + kTrBufs - 1, wr);
+      compute(rd);
+      rd = rd == kLast ? 0 : rd + kTrStage;
+      wr = wr == kLast ? 0 : wr + kTrStage;
+    }
+  }
+  // ---- store: a lane's accumulator quad is four columns of one row; the lane halves exchange quads, so a lane stores
+  // eight consecutive columns (16-bit) or four (fp32), through a resource that drops rows past M and columns past N ----
+  constexpr uint32_t ES = YT == TK_F32 ? 4 : 2;
+  uint8_t* ye = p.y + (int64_t)e * p.y_stride_e * ES;
+  const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(ye, 0, p.y_bytes, 0x00020000);
+  if constexpr (YT == TK_F32) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int m = m0 + mw * 64 + j * 32 + lr;
+      const uint32_t row = (uint32_t)m * (uint32_t)p.y_stride_m * ES;
+#pragma unroll
+      for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int n = n0 + nw * 64 + f * 32 + u * 8 + h * 4;
+          const uint32_t off = (m < p.M && n < p.N) ? row + (uint32_t)n * ES : kOutOfRange;
+          __builtin_amdgcn_raw_buffer_store_b128(u32x4_t{f32_bits(acc[f][j][4 * u]), f32_bits(acc[f][j][4 * u + 1]),
+                                                         f32_bits(acc[f][j][4 * u + 2]), f32_bits(acc[f][j][4 * u + 3])}, ry, off, 0, 0);
+        }
+    }
+  } else {
+    // through LDS (16-byte pieces exchanged by row to spread the banks), so that a store instruction writes eight whole
+    // 128-byte lines of the quadrant
+    static_assert(kTrBufs * kTrStage >= 4 * 8192, "the four quadrants fit the operand buffers");
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    uint8_t* sp = lds + wave * 8192;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int f = 0; f < 2; ++f)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          uint32_t q[4];  // columns 16u + 4h + {01, 23} and 16u + 8 + 4h + {01, 23}
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            q[i] = YT == TK_BF16 ? pack_bf16x2(acc[f][j][8 * u + 2 * i], acc[f][j][8 * u + 2 * i + 1])
+                                 : pack_f16x2(acc[f][j][8 * u + 2 * i], acc[f][j][8 * u + 2 * i + 1]);
+          // after the exchange lanes 0..31 hold columns 16u .. 16u + 7 of their row, lanes 32..63 columns 16u + 8 .. 16u + 15
+          const auto s0 = __builtin_amdgcn_permlane32_swap(q[0], q[2], false, false);
+          const auto s1 = __builtin_amdgcn_permlane32_swap(q[1], q[3], false, false);
+          const int r = j * 32 + lr;
+          *reinterpret_cast<u32x4_t*>(sp + r * 128 + (((f * 4 + u * 2 + h) ^ (r & 7)) * 16)) = u32x4_t{s0[0], s1[0], s0[1], s1[1]};
+        }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+    for (int it = 0; it < 8; ++it) {
+      const int r = it * 8 + (lane >> 3), pc = lane & 7;
+      const u32x4_t q = *reinterpret_cast<const u32x4_t*>(sp + r * 128 + ((pc ^ (r & 7)) * 16));
+      const int m = m0 + mw * 64 + r, n = n0 + nw * 64 + pc * 8;
+      const uint32_t off = (m < p.M && n < p.N) ? ((uint32_t)m * (uint32_t)p.y_stride_m + (uint32_t)n) * ES : kOutOfRange;
+      __builtin_amdgcn_raw_buffer_store_b128(q, ry, off, 0, kNonTemporal);
+    }
+  }
+}
+
 }  // namespace
 }  // namespace tk
 
@@ -356,27 +545,40 @@ extern "C" int32_t tk_ragged_k_gemm(const tk_ragged_k_desc* d, tk_stream_t strea
   };
   p.a_vec = vec(d->a, d->a_stride_m == 1 ? d->a_stride_m : d->a_stride_k, d->a_stride_m == 1 ? d->a_stride_k : d->a_stride_m);
   p.b_vec = vec(d->b, d->b_stride_n == 1 ? d->b_stride_n : d->b_stride_k, d->b_stride_n == 1 ? d->b_stride_k : d->b_stride_n);
-  const int64_t grid = (int64_t)d->n_slices * p.tiles_m * p.tiles_n;
-  if (grid > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_ragged_k_gemm: grid too large");
+  int64_t grid = (int64_t)d->n_slices * p.tiles_m * p.tiles_n;
+  if (grid > 0x7FFF0000) return fail(TK_ERR_UNSUPPORTED, "tk_ragged_k_gemm: grid too large");
   hipStream_t st = static_cast<hipStream_t>(stream);
   // extents (bytes from the base to one past the last element) when both operands are k-slow and within 2 GiB
   const bool k_slow_both = d->a_stride_m == 1 && d->b_stride_n == 1 && d->a_stride_k > 0 && d->b_stride_k > 0;
   const int64_t a_extent = d->a_k_extent * d->a_stride_k * 2, b_extent = d->b_k_extent * d->b_stride_k * 2;
   const bool fast = k_slow_both && p.a_vec && p.b_vec && d->M % 8 == 0 && d->N % 8 == 0 && d->a_k_extent > 0 && d->b_k_extent > 0 &&
                     a_extent < (int64_t(1) << 31) && b_extent < (int64_t(1) << 31) && d->M <= d->a_stride_k && d->N <= d->b_stride_k;
+  const int64_t es = d->y_dtype == TK_F32 ? 4 : 2, y_extent = ((int64_t)(d->M - 1) * d->y_stride_m + d->N) * es;
+  const bool y_ok = d->y_stride_m >= d->N && y_extent < (int64_t(1) << 31) && d->y_stride_m * es % 16 == 0 && d->y_stride_e * es % 16 == 0 &&
+                    (reinterpret_cast<uintptr_t>(d->y) & 15) == 0;
   p.a_bytes = fast ? (uint32_t)a_extent : 0;
   p.b_bytes = fast ? (uint32_t)b_extent : 0;
+  p.y_bytes = y_ok ? (uint32_t)y_extent : 0;
   auto launch = [&](auto kern) { hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(256), 0, st, p); };
-  if (d->dtype == TK_BF16) {
-    if (fast)
-      launch(ragged_k_gemm_kernel<TK_BF16, true>);
-    else
-      launch(ragged_k_gemm_kernel<TK_BF16, false>);
-  } else {
-    if (fast)
-      launch(ragged_k_gemm_kernel<TK_F16, true>);
-    else
-      launch(ragged_k_gemm_kernel<TK_F16, false>);
+  const bool bf16 = d->dtype == TK_BF16;
+  if (fast && y_ok) {
+    const int per_e = p.tiles_m * p.tiles_n;
+    p.chunk = per_e >= 8 ? per_e / 8 : 1;
+    p.n_slices = d->n_slices;
+    const int64_t chunks = cdiv((int64_t)d->n_slices * per_e, p.chunk);
+    grid = cdiv(chunks, 8) * 8 * p.chunk;
+    auto with_y = [&](auto dt) {
+      constexpr int DT = decltype(dt)::value;
+      if (d->y_dtype == TK_BF16)
+        launch(ragged_k_tr_kernel<DT, TK_BF16>);
+      else if (d->y_dtype == TK_F16)
+        launch(ragged_k_tr_kernel<DT, TK_F16>);
+      else
+        launch(ragged_k_tr_kernel<DT, TK_F32>);
+    };
+    bf16 ? with_y(std::integral_constant<int, TK_BF16>{}) : with_y(std::integral_constant<int, TK_F16>{});
+    return check_launch("ragged_k_tr_kernel");
   }
+  bf16 ? launch(ragged_k_gemm_kernel<TK_BF16>) : launch(ragged_k_gemm_kernel<TK_F16>);
   return check_launch("ragged_k_gemm_kernel");
 }
