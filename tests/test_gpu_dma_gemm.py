@@ -1,0 +1,67 @@
+"""GPU parity of the expert GEMM that stages both operands by memory-to-LDS transfers (bf16, fp16, e4m3; row blocks of 128 and 256)
+against the CPU oracle, at the sizes where it can go wrong: row blocks that are empty, nearly empty, nearly and exactly
+full; one stage of K, a stage and a remainder, more stages than LDS buffers; columns around the tile; all its slice registers."""
+import pytest
+import torch
+
+from oracle import moe as omoe
+from oracle.checks import assert_allclose_gate
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [0, 1, 31, 33, 127, 128, 129, 0, 255, 256, 257, 390]
+
+
+def _check(device, dtype, block_m, sizes, k, n, swiglu=False):
+    import triton_amd.matmul as mm
+    from triton_amd.swiglu import swiglu_fn
+    from triton_amd.tensor import convert_layout, make_ragged_tensor_metadata, wrap_torch_tensor
+    from triton_amd.tensor_details.layout import make_default_matmul_fp8_w_layout
+    g = torch.Generator().manual_seed(k * 7 + n)
+    E, m = len(sizes), sum(sizes)
+    sizes = torch.tensor(sizes, dtype=torch.int32)
+    x, w = torch.randn((m, k), generator=g), torch.randn((E, n, k), generator=g) * 0.1
+    bias, gam = torch.randn((E, n), generator=g), torch.rand((m, ), generator=g) + 0.5
+    gi, sc = torch.randint(0, m, (m, ), generator=g).to(torch.int32), torch.randperm(m, generator=g).to(torch.int32)
+    pc, scales = mm.PrecisionConfig(), {}
+    if dtype == "e4m3":
+        scales = dict(x_row_scale=torch.rand((m, ), generator=g) + 0.5, w_col_scale=torch.rand((E, n), generator=g) + 0.5)
+        x, w = x.to(torch.float8_e4m3fn), w.to(torch.float8_e4m3fn).transpose(1, 2)
+        w_dev = convert_layout(wrap_torch_tensor(w.transpose(1, 2).contiguous().to(device).transpose(1, 2)), make_default_matmul_fp8_w_layout())
+        pc = mm.PrecisionConfig(a_mx_tensor_scale=scales["x_row_scale"].to(device), b_mx_tensor_scale=scales["w_col_scale"].to(device),
+                                out_dtype=torch.bfloat16)
+        out_dtype = torch.bfloat16
+    else:
+        out_dtype = getattr(torch, dtype)
+        x, w = x.to(out_dtype), w.to(out_dtype).transpose(1, 2)
+        w_dev = w.transpose(1, 2).contiguous().to(device).transpose(1, 2)
+    act = mm.FusedActivation(mm.FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0)) if swiglu else None
+    out = torch.full((m, n // 2 if swiglu else n), float("nan"), dtype=out_dtype, device=device)
+    with mm.scoped_opt_flags_constraints({"block_m": block_m}):
+        mm.matmul(x.to(device), w_dev, bias.to(device), make_ragged_tensor_metadata(sizes.to(device), m), gather_indx=gi.to(device),
+                  scatter_indx=sc.to(device), gammas=gam.to(device), precision_config=pc, fused_activation=act, c=out)
+    ref = omoe.matmul(x, w, bias, sizes, gather_indx=gi, out_dtype=torch.float32, **scales)
+    ref = (omoe.swiglu(ref, 1.702, 7.0).float() if swiglu else ref) * gam[:, None]
+    want = torch.empty_like(ref)
+    want[sc.long()] = ref
+    assert_allclose_gate(want, out, what=f"{dtype} block_m {block_m}")
+
+
+@pytest.mark.parametrize("k, n", [(32, 8), (64, 264), (208, 520), (1040, 248)])
+@pytest.mark.parametrize("block_m", [128, 256])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16", "e4m3"])
+def test_tile_and_stage_edges(device, dtype, block_m, k, n):
+    _check(device, dtype, block_m, SIZES, k, n)
+
+
+@pytest.mark.parametrize("block_m", [128, 256])
+@pytest.mark.parametrize("dtype", ["bfloat16", "e4m3"])
+def test_swiglu(device, dtype, block_m):
+    _check(device, dtype, block_m, SIZES, 272, 528, swiglu=True)
+
+
+@pytest.mark.parametrize("n_slices", [64, 65, 256, 257])
+def test_slice_registers(device, n_slices):
+    """257 slices run on the kernel without registers for them."""
+    _check(device, "e4m3", 128, [(i * 37) % 9 for i in range(n_slices)], 192, 160)
+    _check(device, "bfloat16", 128, [(i * 37) % 9 for i in range(n_slices)], 192, 160)

@@ -176,6 +176,22 @@ def stream_ptr(device=None) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
+_current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device
+
+
+def submit(entry, desc, device: torch.device, what: str = ""):
+    """`entry(desc, stream)` on the current stream of `device` (made current for the call if it is not), for the entry points
+    that take one descriptor; errors as `check` says."""
+    idx = device.index
+    if idx is None or idx == _current_device():
+        status = entry(desc, stream_ptr(device))
+    else:
+        with torch.cuda.device(idx):
+            status = entry(desc, stream_ptr(device))
+    if status != TK_OK:
+        check(status, what)
+
+
 class on_device:
     """`with on_device(t.device):` makes that device current for the launch, like `torch.cuda.device`, but costs
     next to nothing in the common case that it already is."""
@@ -183,7 +199,7 @@ class on_device:
 
     def __init__(self, device):
         idx = device.index if isinstance(device, torch.device) else device
-        self.ctx = None if idx is None or idx == torch.cuda.current_device() else torch.cuda.device(idx)
+        self.ctx = None if idx is None or idx == _current_device() else torch.cuda.device(idx)
 
     def __enter__(self):
         if self.ctx is not None:

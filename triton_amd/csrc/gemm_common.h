@@ -70,20 +70,23 @@ struct GemmParams {
   float out_alpha;
   const uint16_t* acc_in;     // tensor of the output's shape and type added to the result (behind the gate weight), or null
   int64_t acc_in_stride_m;
+  uint32_t x_bytes;           // extent of x for a buffer resource (kernels that address x through one), 0 = not below 2 GiB
 };
 
 // one entry per kernel family; each returns a TK_* status
 int32_t gemm_launch_strided(const GemmParams& p, int wk, int block_m, int grid_m, bool swiglu, hipStream_t st);
+int32_t gemm_launch_dma(const GemmParams& p, int wk, int block_m, int grid_m, bool swiglu, hipStream_t st);  // block_m 128 / 256
 int32_t gemm_launch_mxn(const GemmParams& p, int block_m, int grid_m, bool swiglu, hipStream_t st);
 int32_t gemm_launch_mxn_mx(const GemmParams& p, int block_m, int grid_m, bool swiglu, hipStream_t st);  // block_m 128 / 256, MX-quantised output
 int32_t gemm_launch_mxd(const GemmParams& p, int block_m, int grid_m, bool swiglu, hipStream_t st);
 int32_t gemm_launch_f8n(const GemmParams& p, int block_m, int grid_m, bool swiglu, hipStream_t st);
-int32_t gemm_launch_f8w(const GemmParams& p, int grid_m, bool swiglu, hipStream_t st);  // 256 x 256 tiles (row blocks of 256)
 int32_t gemm_launch_mx8n(const GemmParams& p, int block_m, int grid_m, bool swiglu, bool mx_out, hipStream_t st);
 
 // Slices (experts) whose row and block offsets the persistent MXFP4 prefill kernel keeps in LDS: a tile's coordinates
 // then cost LDS reads instead of a chain of dependent global loads.  The host refuses more slices than this.
 constexpr int kMetaSlices = 1024;
+// Slices whose sizes and offsets the memory-to-LDS kernel keeps in registers; other kernels run with more.
+constexpr int kDmaSlices = 256;
 
 namespace {
 

@@ -8,6 +8,12 @@
 
 using namespace tk;
 
+// Can the kernel that stages both operands through memory-to-LDS transfers run this?  x and an expert's weights (`w_bytes`) have to lie within
+// 2 GiB (buffer resources) and the slices' sizes in its registers.
+static bool dma_ok(const GemmParams& p, const tk_gemm_desc* d, int64_t w_bytes) {
+  return p.x_bytes && (!d->slice_sizes || d->n_slices <= kDmaSlices) && w_bytes < (int64_t)1 << 31 && (d->block_m == 128 || d->block_m == 256);
+}
+
 extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
   if (!d) return fail(TK_ERR_INVALID, "tk_moe_gemm: null descriptor");
   if (d->M < 0 || d->N < 0 || d->K < 0) return fail(TK_ERR_INVALID, "tk_moe_gemm: negative size");
@@ -112,6 +118,12 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
   p.y_mx_kind = d->y_dtype;
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool swiglu = d->activation == TK_ACT_SWIGLU;
+  {
+    // extent of x for the kernels that address it through a buffer resource
+    const int64_t rows = d->x_rows > 0 ? d->x_rows : (d->gather_indx ? 0 : d->M);
+    const int64_t bytes = rows * d->x_stride_m * (d->x_dtype == TK_E4M3 ? 1 : 2);
+    p.x_bytes = bytes > 0 && d->x_stride_m >= d->K && bytes < (int64_t)1 << 31 ? (uint32_t)bytes : 0u;
+  }
   if (d->w_layout == TK_W_TILED && d->w_dtype == TK_E4M3) {
     if (d->w_mx_scale) return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: MX scales with e4m3 weights");
     if (d->block_m != 128 && d->block_m != 256) return fail(TK_ERR_INVALID, "tk_moe_gemm: tiled e4m3 weights take block_m 128 or 256 (got %d)", d->block_m);
@@ -121,11 +133,7 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
     if (d->n_slices > 1 && d->w_stride_e < nfr * nst * 8192) return fail(TK_ERR_INVALID, "tk_moe_gemm: expert stride smaller than one tiled expert");
     p.w_stride_e = d->w_stride_e;
     p.w_nst = (int32_t)nst;
-    if (d->block_m == 256) {
-      // 256 x 256 tiles; the kernel addresses activation rows with 32-bit byte offsets from x
-      const int64_t x_rows = d->x_rows > 0 ? d->x_rows : (d->gather_indx ? 0 : d->M);
-      if (x_rows > 0 && d->x_stride_m >= 0 && x_rows * d->x_stride_m < ((int64_t)1 << 32)) return gemm_launch_f8w(p, d->grid_m, swiglu, st);
-    }
+    if (dma_ok(p, d, nfr * nst * 8192)) return gemm_launch_dma(p, WK_FP8, d->block_m, d->grid_m, swiglu, st);
     return gemm_launch_f8n(p, d->block_m, d->grid_m, swiglu, st);
   }
   if (mx_act) {
@@ -229,6 +237,7 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
     if (d->w_stride_n % 8 || d->w_stride_e % 8 || (reinterpret_cast<uintptr_t>(d->w) & 15)) return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: weight columns must be 16-byte aligned");
     p.w_stride_e = d->w_stride_e * 2;
     p.w_stride_n = d->w_stride_n * 2;
+    if (dma_ok(p, d, (int64_t)(d->N - 1) * p.w_stride_n + d->K * 2) && p.w_stride_n >= d->K * 2) return gemm_launch_dma(p, WK_BF16, d->block_m, d->grid_m, swiglu, st);
     return gemm_launch_strided(p, WK_BF16, d->block_m, d->grid_m, swiglu, st);
   }
   if (d->w_dtype == TK_F16) {
@@ -238,6 +247,7 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
     if (d->w_stride_n % 8 || d->w_stride_e % 8 || (reinterpret_cast<uintptr_t>(d->w) & 15)) return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: weight columns must be 16-byte aligned");
     p.w_stride_e = d->w_stride_e * 2;
     p.w_stride_n = d->w_stride_n * 2;
+    if (dma_ok(p, d, (int64_t)(d->N - 1) * p.w_stride_n + d->K * 2) && p.w_stride_n >= d->K * 2) return gemm_launch_dma(p, WK_F16, d->block_m, d->grid_m, swiglu, st);
     return gemm_launch_strided(p, WK_F16, d->block_m, d->grid_m, swiglu, st);
   }
   if (d->w_dtype == TK_E4M3) {

@@ -1,0 +1,390 @@
+// Expert GEMM for full row blocks with both operands staged by memory-to-LDS transfers: bf16 / fp16 (strided, K-contiguous weights)
+// and e4m3 (tiled weights), fp32 accumulation, the shared epilogue.
+//
+//   * A workgroup multiplies BM rows of one expert by BN columns: 256 x 256 with eight waves of 128 x 64 (one workgroup per CU), or
+//     128 x 128 with four waves of 64 x 64 (two per CU).  Either way a SIMD holds two waves: while one waits for LDS or at the
+//     barrier the other feeds the matrix pipe.
+//   * A stage is 128 bytes of K of every row and column, i.e. whole cache lines: with 64-byte stages every line crossed from L2 to
+//     the CU twice, 37 bytes per cycle for 18 useful ones.  The LDS holds two stages of activations and three of weights (which come
+//     from further away).  Every transfer is a `buffer_load ... lds` of 1 KiB per wave, eight rows of a line each: no registers, no VALU, no
+//     LDS write instructions; gathered rows, rows past the slice, columns past N and k past K are a matter of the lanes'
+//     offsets (past the resource's range the hardware writes zeros).
+//   * Rows lie 128 bytes apart without padding (the transfer writes lane-contiguously); the 16-byte pieces of row r are stored at
+//     piece ^ (r >> 1 & 7), so that sixteen rows read at one k occupy all banks once.  Tiled e4m3 blocks arrive in fragment order
+//     and are read as they are.
+//   * A stage is multiplied in four quarters; the operand fragments of a quarter are read from LDS during the one before.  The one
+//     barrier of a stage sits in front of its last quarter: behind it the next stage is complete, this stage's buffers have been
+//     read and are filled again.
+//   * Workgroups are persistent and the ring runs on across tiles: the first stages of the next tile are on their way during the
+//     last stages and the epilogue of this one.
+//
+// What bounds it: the board's power with the matrix pipe about 65 % busy at 1.85 GHz (a square bf16 product of 8192 runs at 1390 TFLOP/s,
+// 0.93 of what the vendor's library reaches on the same board), then the epilogues (12 % of the e4m3 GEMM with K = 4096).  16384 routed rows
+// of 8 experts in e4m3: K 4096, N 28672, swiglu 1840 -> 1590 us (2.42 PFLOP/s), K 14336, N 4096 850 -> 805 us; 4096 rows of 16
+// experts in bf16, K 2048: N 4096 231 -> 94 us, N 2048 133 -> 51 us (the kernels before: weights in registers with one wave
+// per SIMD, and both operands through registers into LDS).
+#include "gemm_common.h"
+#include "route_common.h"
+
+namespace tk {
+namespace {
+
+constexpr uint32_t kOutOfRange = 0x80000000u;
+constexpr int kSliceRegs = kDmaSlices / 64;
+
+template <bool LARGE>
+struct DmaCfg {
+  static constexpr int WM = 2, WN = LARGE ? 4 : 2;       // waves along rows / columns
+  static constexpr int MFW = LARGE ? 4 : 2, NFW = 2;     // fragments of a wave
+  static constexpr int BM = WM * MFW * 32, BN = WN * NFW * 32;
+  static constexpr int NW = WM * WN;
+  static constexpr int ABYTES = BM * 128, BBYTES = BN * 128;
+  static constexpr int ABUFS = 2, BBUFS = 3;
+  static constexpr int LDS = ABUFS * ABYTES + BBUFS * BBYTES;
+  static constexpr int AI = BM / 8 / NW, BI = BN / 8 / NW;  // transfers of a wave and stage
+};
+static_assert(DmaCfg<true>::LDS == 160 * 1024 && DmaCfg<false>::LDS == 80 * 1024, "one / two workgroups fill a CU's LDS");
+
+template <int WK, bool LARGE, bool SWIGLU>
+__global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel(const GemmParams p) {
+  typedef DmaCfg<LARGE> C;
+  constexpr bool F8 = WK == WK_FP8;
+  constexpr int ES = F8 ? 1 : 2;
+  constexpr int MFW = C::MFW, NFW = C::NFW;
+  extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int mw = wave % C::WM, nw = wave / C::WM;
+  const int lr = lane & 31, h = lane >> 5;
+  const int KB = p.K * ES;                // bytes of a row
+  const int nst = (KB + 127) >> 7;
+  const uint32_t lds0 = lds_addr(lds);
+
+  // ---- tiles ---------------------------------------------------------------------------------------------------------------------------------------
+  // Two lists: row blocks that are more than half full, then the short last blocks of the experts, which cost a fraction of a tile;
+  // with the short ones in between, a workgroup's share was up to a whole tile longer than the next one's.  Of each list every
+  // XCD (workgroup b runs on XCD b % 8) takes a contiguous part, walked side by side by its workgroups, the short tiles behind the
+  // others: the workgroups without a tile in the last round of full ones begin with them.
+  // Slice sizes and offsets stay in registers, lane l of register c holding slice c * 64 + l.
+  int sz[kSliceRegs], so[kSliceRegs];
+#pragma unroll
+  for (int c = 0; c < kSliceRegs; ++c) {
+    const int e = c * 64 + lane;
+    sz[c] = so[c] = 0;
+    if (p.slice_sizes) {
+      if (e < p.n_slices) {
+        sz[c] = p.slice_sizes[e];
+        so[c] = p.slice_offs[e];
+      }
+    } else if (e == 0) {
+      sz[c] = p.M;
+    }
+  }
+  auto n_full = [&](int rows) __attribute__((always_inline)) { return (rows + C::BM / 2 - 1) / C::BM; };
+  auto n_short = [&](int rows) __attribute__((always_inline)) { return rows > n_full(rows) * C::BM ? 1 : 0; };
+  int full = 0, brief = 0;
+#pragma unroll
+  for (int c = 0; c < kSliceRegs; ++c) {
+    full += __builtin_amdgcn_readlane(wave_scan_i32(n_full(sz[c])), 63);
+    brief += __builtin_amdgcn_readlane(wave_scan_i32(n_short(sz[c])), 63);
+  }
+  const int xcd = blockIdx.x & 7, t_step = gridDim.x >> 3;
+  const int f_beg = (int)(((int64_t)full * p.grid_n * xcd) >> 3), f_len = (int)(((int64_t)full * p.grid_n * (xcd + 1)) >> 3) - f_beg;
+  const int s_beg = (int)(((int64_t)brief * p.grid_n * xcd) >> 3), s_len = (int)(((int64_t)brief * p.grid_n * (xcd + 1)) >> 3) - s_beg;
+  const int t_end = f_len + s_len;
+  int tile = (int)(blockIdx.x >> 3);
+  if (tile >= t_end) return;
+
+  struct Tile {
+    int expert, off_m, start_m, eM, n_tile;
+  };
+  auto locate = [&](int t) __attribute__((always_inline)) -> Tile {
+    Tile r = {0, 0, 0, 0, 0};
+    const bool is_full = t < f_len;
+    const int g = is_full ? f_beg + t : s_beg + t - f_len;
+    int q = g / p.grid_n, base = 0;
+    bool found = false;
+#pragma unroll
+    for (int c = 0; c < kSliceRegs; ++c) {
+      if (found) continue;
+      const int cnt = is_full ? n_full(sz[c]) : n_short(sz[c]);
+      const int inc = wave_scan_i32(cnt);
+      const int total = __builtin_amdgcn_readlane(inc, 63);
+      if (q < base + total) {
+        found = true;
+        const int l = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(base + inc > q));
+        const int nb = __builtin_amdgcn_readlane(cnt, l);
+        int i = g - (base + __builtin_amdgcn_readlane(inc, l) - nb) * p.grid_n;
+        r.expert = c * 64 + l;
+        r.eM = __builtin_amdgcn_readlane(sz[c], l);
+        r.start_m = __builtin_amdgcn_readlane(so[c], l);
+        // bands of eight row blocks, in a band column by column, so that the tiles an XCD has in hand share eight blocks of
+        // activations and a few of weights through its L2
+        const int band = i / (8 * p.grid_n);
+        const int bh = nb - band * 8 < 8 ? nb - band * 8 : 8;
+        i -= band * 8 * p.grid_n;
+        const int pn = i / bh;
+        r.n_tile = pn * C::BN;
+        r.off_m = (is_full ? band * 8 + i - pn * bh : n_full(r.eM)) * C::BM;
+      }
+      base += total;
+    }
+    return r;
+  };
+
+  // ---- transfer side ------------------------------------------------------------------------------------------------------------------------------
+  // transfer i of an operand: rows i * 8 .. + 7, lane -> row lane / 8, LDS position lane % 8, i.e. piece (lane % 8) ^ (row >> 1 & 7);
+  // with eight rows a transfer, row >> 1 & 7 = (i & 1) * 4 + (lane >> 4)
+  // (a wave's transfers start at an even index, so the parity of i counts)
+  const int pc0 = (lane & 7) ^ (lane >> 4), pc1 = pc0 ^ 4;
+  const buf_desc_t xdesc = make_buf_desc(p.x, p.x_bytes);
+  buf_desc_t wdesc;
+  uint32_t a_off[C::AI], b_off[C::BI];
+  const uint32_t x_row = (uint32_t)(p.x_stride_m * ES);
+  static_assert(C::AI % 2 == 0 && C::BI % 2 == 0, "a transfer's parity is that of its index in the wave");
+  auto aim = [&](const Tile& c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < C::AI; ++i) {
+      const int row = c.off_m + (wave * C::AI + i) * 8 + (lane >> 3);
+      const int sr = c.start_m + (row < c.eM ? row : c.eM - 1);
+      const uint32_t src = p.gather ? (uint32_t)p.gather[sr] : (uint32_t)sr;
+      a_off[i] = row < c.eM ? src * x_row + (uint32_t)((i & 1) ? pc1 : pc0) * 16u : kOutOfRange;
+    }
+    const uint8_t* w = p.w + (int64_t)c.expert * p.w_stride_e;
+    if constexpr (F8) {
+      const int f0 = c.n_tile >> 5, nfr = (p.N + 31) >> 5, nf = C::BN / 32;
+      const uint32_t fsz = (uint32_t)p.w_nst * 8192u;  // bytes of a column fragment
+      wdesc = make_buf_desc(w + (int64_t)f0 * fsz, (uint32_t)(nfr - f0 < nf ? nfr - f0 : nf) * fsz);
+#pragma unroll
+      for (int i = 0; i < C::BI; ++i) {
+        const int id = wave * C::BI + i;  // KiB id % 4 of fragment id / 4's block
+        b_off[i] = (uint32_t)(id >> 2) * fsz + (uint32_t)(id & 3) * 1024u + (uint32_t)lane * 16u;
+      }
+    } else {
+      const int cols = p.N - c.n_tile < C::BN ? p.N - c.n_tile : C::BN;
+      wdesc = make_buf_desc(w + (int64_t)c.n_tile * p.w_stride_n, (uint32_t)(cols - 1) * (uint32_t)p.w_stride_n + (uint32_t)KB);
+#pragma unroll
+      for (int i = 0; i < C::BI; ++i) {
+        const int n = (wave * C::BI + i) * 8 + (lane >> 3);
+        b_off[i] = n < cols ? (uint32_t)n * (uint32_t)p.w_stride_n + (uint32_t)((i & 1) ? pc1 : pc0) * 16u : kOutOfRange;
+      }
+    }
+  };
+  // transfer i of this wave for stage s of the tile aimed at (none left: zeros into a buffer that nobody reads)
+  auto fetch_a = [&](int i, int s, uint32_t buf, bool more) __attribute__((always_inline)) {
+    const uint32_t kb = (uint32_t)s * 128u;
+    const bool in = more && (int)kb + ((i & 1) ? pc1 : pc0) * 16 < KB;
+    lds_dma16(xdesc, lds0 + buf + (wave * C::AI + i) * 1024, in ? a_off[i] + kb : kOutOfRange);
+  };
+  auto fetch_b = [&](int i, int s, uint32_t buf, bool more) __attribute__((always_inline)) {
+    const uint32_t kb = (uint32_t)s * (F8 ? 4096u : 128u);
+    const bool in = more && (F8 || (int)kb + ((i & 1) ? pc1 : pc0) * 16 < KB);  // (tiled weights are padded with zeros)
+    lds_dma16(wdesc, lds0 + buf + (wave * C::BI + i) * 1024, in ? b_off[i] + kb : kOutOfRange);
+  };
+
+  // ---- LDS read side ----------------------------------------------------------------------------------------------------------------------------
+  // 16-bit: step t of four, the lane's piece 2t + h;  e4m3: step u of two, the lane's pieces 4u + 2h + {0, 1} (32 consecutive k)
+  const int sw = (lr >> 1) & 7;
+  uint32_t pos[4];
+#pragma unroll
+  for (int t = 0; t < 4; ++t) pos[t] = (uint32_t)(((F8 ? (t >> 1) * 4 + 2 * h + (t & 1) : 2 * t + h) ^ sw) * 16 + lr * 128);
+  auto ld = [&](uint32_t at) __attribute__((always_inline)) -> u32x4_t { return *reinterpret_cast<const u32x4_t*>(lds + at); };
+  auto read_a = [&](uint32_t buf, int j, int t) __attribute__((always_inline)) -> u32x4_t {
+    return ld(buf + (uint32_t)(mw * 4096) + pos[t] + j * (C::WM * 4096));
+  };
+  auto read_b = [&](uint32_t buf, int f, int t) __attribute__((always_inline)) -> u32x4_t {
+    return F8 ? ld(buf + (uint32_t)(nw * NFW * 4096) + (uint32_t)lane * 16u + f * 4096 + t * 1024) : ld(buf + (uint32_t)(nw * NFW * 4096) + pos[t] + f * 4096);
+  };
+
+  // ---- the rings: one cursor, two stages ahead of the multiplication --------------------------------------------------------------------------
+  constexpr uint32_t kAEnd = C::ABUFS * C::ABYTES, kBEnd = kAEnd + C::BBUFS * C::BBYTES;
+  Tile cur = locate(tile);
+  aim(cur);
+  uint32_t aw = 0, bw = kAEnd;  // buffers the next transfers fill
+  int fs = 0;                   // next stage to fetch
+  bool more = true;
+  int f_tile = tile;
+  auto advance = [&]() __attribute__((always_inline)) {
+    aw = aw + C::ABYTES == kAEnd ? 0 : aw + C::ABYTES;
+    bw = bw + C::BBYTES == kBEnd ? kAEnd : bw + C::BBYTES;
+    if (++fs == nst) {
+      fs = 0;
+      f_tile += t_step;
+      more = more && f_tile < t_end;
+      if (more) aim(locate(f_tile));
+    }
+  };
+
+  f32x16_t acc[NFW][MFW];
+  auto mma16 = [&](u32x4_t w, u32x4_t x, f32x16_t c) __attribute__((always_inline)) -> f32x16_t {
+    if constexpr (WK == WK_F16)
+      return Frag<32>::mma_f16(__builtin_bit_cast(bf16x8_t, w), __builtin_bit_cast(bf16x8_t, x), c);
+    else
+      return Frag<32>::mma(__builtin_bit_cast(bf16x8_t, w), __builtin_bit_cast(bf16x8_t, x), c);
+  };
+  auto both = [&](u32x4_t lo, u32x4_t hi) __attribute__((always_inline)) -> i32x8_t {
+    return __builtin_bit_cast(i32x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  };
+  // Operand registers of the even and the odd quarters.  16-bit: quarter t multiplies step t, all row fragments.  e4m3: quarters 2u and
+  // 2u + 1 multiply the lower and the upper half of the row fragments of step u; the weights of a step live in w8[u].
+  u32x4_t ar[2][F8 ? 1 : MFW], wr[2][F8 ? 1 : NFW];
+  i32x8_t a8[2][F8 ? MFW / 2 : 1], w8[2][F8 ? NFW : 1];
+  // quarter Q of the stage at (abuf, bbuf), while the operands of the next quarter are read: of the same stage, or for Q = 3 of the next
+  auto quarter = [&](auto full_c, auto q_c, int jc, uint32_t abuf, uint32_t bbuf) __attribute__((always_inline)) {
+    constexpr bool FULL = decltype(full_c)::value;
+    constexpr int Q = decltype(q_c)::value, QN = (Q + 1) & 3, P = Q & 1;
+    // A wave's transfers are spread over the stage (the CU takes one per sixteen cycles or so; all eight behind the barrier held up
+    // its first multiplications): activations, which the next barrier waits for, in quarter 3, weights in quarters 0 and 1.
+    auto transfer = [&](int k) __attribute__((always_inline)) {
+      if constexpr (Q == 3) {
+        fetch_a(2 * k, fs, aw, more);
+        fetch_a(2 * k + 1, fs, aw, more);
+      }
+      if constexpr (Q < 2) fetch_b(2 * Q + k, fs, bw, more);
+    };
+    if constexpr (!F8) {
+#pragma unroll
+      for (int f = 0; f < NFW; ++f) wr[1 - P][f] = read_b(bbuf, f, QN);
+#pragma unroll
+      for (int j = 0; j < MFW; ++j) {
+        ar[1 - P][j] = read_a(abuf, j, QN);
+        if (FULL || j < jc) {
+#pragma unroll
+          for (int f = 0; f < NFW; ++f) acc[f][j] = mma16(wr[P][f], ar[P][j], acc[f][j]);
+        }
+        if (j % (MFW / 2) == MFW / 2 - 1) transfer(j / (MFW / 2));
+        if constexpr (FULL) __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      constexpr int U = Q >> 1, UN = QN >> 1, HJ = MFW / 2;
+#pragma unroll
+      for (int j = 0; j < HJ; ++j) {
+        a8[1 - P][j] = both(read_a(abuf, (1 - P) * HJ + j, 2 * UN), read_a(abuf, (1 - P) * HJ + j, 2 * UN + 1));
+        if constexpr (P == 1) {  // the weights of the next step
+#pragma unroll
+          for (int f = j * NFW / HJ; f < (j + 1) * NFW / HJ; ++f) w8[1 - U][f] = both(read_b(bbuf, f, 2 * UN), read_b(bbuf, f, 2 * UN + 1));
+        }
+        if (FULL || P * HJ + j < jc) {
+#pragma unroll
+          for (int f = 0; f < NFW; ++f)
+            acc[f][P * HJ + j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w8[U][f], a8[P][j], acc[f][P * HJ + j], 0, 0, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
+        }
+#pragma unroll
+        for (int k = 0; k < 2 / HJ; ++k) transfer(HJ == 2 ? j : k);
+        if constexpr (FULL) {
+          // (an empty use of the results: the compiler otherwise sinks the multiplications to the end of the loop)
+#pragma unroll
+          for (int f = 0; f < NFW; ++f) asm volatile("" : "+v"(acc[f][P * HJ + j]));
+        }
+        if constexpr (FULL) __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+
+  auto barrier = [&]() __attribute__((always_inline)) {
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // stages 0 and 1 of both operands: as the loop finds them in front of its quarter 0
+  static_assert(C::AI == 4 && C::BI == 4, "transfers as dealt to the quarters");
+#pragma unroll
+  for (int n = 0; n < 2; ++n) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) fetch_b(i, fs, bw, more);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) fetch_a(i, fs, aw, more);
+    advance();
+  }
+  asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+  barrier();
+  uint32_t ab = 0, bb = kAEnd;
+  // the operands of a tile's first quarter (read again behind an epilogue, which needs the registers)
+  auto prime = [&]() __attribute__((always_inline)) {
+    if constexpr (!F8) {
+#pragma unroll
+      for (int f = 0; f < NFW; ++f) wr[0][f] = read_b(bb, f, 0);
+#pragma unroll
+      for (int j = 0; j < MFW; ++j) ar[0][j] = read_a(ab, j, 0);
+    } else {
+#pragma unroll
+      for (int f = 0; f < NFW; ++f) w8[0][f] = both(read_b(bb, f, 0), read_b(bb, f, 1));
+#pragma unroll
+      for (int j = 0; j < MFW / 2; ++j) a8[0][j] = both(read_a(ab, j, 0), read_a(ab, j, 1));
+    }
+  };
+  while (true) {
+    prime();
+#pragma unroll
+    for (int f = 0; f < NFW; ++f)
+#pragma unroll
+      for (int j = 0; j < MFW; ++j)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[f][j][i] = 0.f;
+    const int rows = cur.eM - cur.off_m < C::BM ? cur.eM - cur.off_m : C::BM;
+    const int jc = __builtin_amdgcn_readfirstlane((((rows + 31) >> 5) - mw + C::WM - 1) / C::WM);  // this wave's row fragments (j * WM + mw) that hold rows
+    auto stages = [&](auto full_c) __attribute__((always_inline)) {
+      for (int s = 0; s < nst; ++s) {
+        quarter(full_c, template_int<0>{}, jc, ab, bb);
+        quarter(full_c, template_int<1>{}, jc, ab, bb);
+        quarter(full_c, template_int<2>{}, jc, ab, bb);
+        // the next stage has landed (this wave's part) when only the four transfers of quarters 0 and 1 are outstanding
+        asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        barrier();
+        ab = ab + C::ABYTES == kAEnd ? 0 : ab + C::ABYTES;
+        bb = bb + C::BBYTES == kBEnd ? kAEnd : bb + C::BBYTES;
+        quarter(full_c, template_int<3>{}, jc, ab, bb);
+        // (the one branch of a stage stands at its end: with one in between, the compiler moves the multiplications in front of it
+        // down behind it, and their operands pile up)
+        advance();
+      }
+    };
+    if (jc >= MFW)
+      stages(std::true_type{});
+    else
+      stages(std::false_type{});
+    gemm_epilogue<32, C::WM, MFW, NFW, SWIGLU, WK == WK_F16>(p, acc, cur.expert, cur.off_m, cur.start_m, cur.eM, cur.n_tile + nw * NFW * 32,
+                                                             cur.n_tile + C::BN <= p.N, mw, lr, h);
+    tile += t_step;
+    if (tile >= t_end) break;
+    cur = locate(tile);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no transfer into this workgroup's LDS is left behind
+}
+
+template <int WK, bool LARGE>
+int32_t launch_cfg(const GemmParams& p, int grid_m, bool swiglu, hipStream_t st) {
+  typedef DmaCfg<LARGE> C;
+  GemmParams q = p;
+  q.grid_n = (int)cdiv(p.N, C::BN);
+  const int64_t tiles = (int64_t)grid_m * q.grid_n;
+  if (tiles <= 0) return TK_OK;
+  if (tiles > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: grid too large");
+  q.total_tiles = (int32_t)tiles;
+  // a multiple of 8 workgroups (every XCD walks its share of the tiles), one or two per CU
+  int64_t grid = (int64_t)busy_cu_count(p.idle_cus) * (LARGE ? 1 : 2) / 8 * 8;
+  grid = grid < 8 ? 8 : grid;
+  grid = grid < cdiv(tiles, 8) * 8 ? grid : cdiv(tiles, 8) * 8;
+  auto launch = [&](auto kern) -> int32_t {
+    if (const int32_t rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), C::LDS)) return rc;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NW * 64), C::LDS, st, q);
+    return check_launch("moe_gemm_dma_kernel");
+  };
+  return swiglu ? launch(moe_gemm_dma_kernel<WK, LARGE, true>) : launch(moe_gemm_dma_kernel<WK, LARGE, false>);
+}
+
+}  // namespace
+
+int32_t gemm_launch_dma(const GemmParams& p, int wk, int block_m, int grid_m, bool swiglu, hipStream_t st) {
+  switch (wk) {
+    case WK_BF16:
+      return block_m == 256 ? launch_cfg<WK_BF16, true>(p, grid_m, swiglu, st) : launch_cfg<WK_BF16, false>(p, grid_m, swiglu, st);
+    case WK_F16:
+      return block_m == 256 ? launch_cfg<WK_F16, true>(p, grid_m, swiglu, st) : launch_cfg<WK_F16, false>(p, grid_m, swiglu, st);
+    case WK_FP8:
+      return block_m == 256 ? launch_cfg<WK_FP8, true>(p, grid_m, swiglu, st) : launch_cfg<WK_FP8, false>(p, grid_m, swiglu, st);
+  }
+  return fail(TK_ERR_INVALID, "tk_moe_gemm: bad weight kind %d", wk);
+}
+
+}  // namespace tk

@@ -32,14 +32,16 @@ from typing import Callable
 import torch
 
 from . import _native as nt
-from .matmul_details.opt_flags import (InapplicableConstraint, OptFlags, make_opt_flags, scoped_opt_flags,  # noqa: F401
-                                        scoped_opt_flags_constraints, set_idle_sms)
+from .matmul_details.opt_flags import (InapplicableConstraint, OptFlags, _get_idle_sms, _get_opt_flags_constraints,  # noqa: F401
+                                        default_block_m, make_opt_flags, scoped_opt_flags, scoped_opt_flags_constraints, set_idle_sms,
+                                        unconstrained)
 from .numerics import InFlexData, OutFlexData
 from .specialize import FnSpecs
 from .tensor import FP4, RaggedTensorMetadata, Tensor, convert_layout, torch_dtype_to_dtype, wrap_torch_tensor
 from .tensor_details.layout_details.cdna4_scale import CDNA4MXScaleLayout
 from .tensor_details.layout_details.gfx950_mx import GFX950FP8ValueLayout, GFX950MXScaleLayout, GFX950MXValueLayout
 from .tensor_details.layout_details.strided import StridedLayout
+from .tensor_details.ragged_tensor import _BLOCK_SIZES
 
 MXFP_BLOCK_SIZE = 32
 
@@ -104,6 +106,14 @@ class PrecisionConfig:
     enforce_bitwise_invariance: bool = False
 
 
+# defaults shared by all calls (never written to)
+_NO_PRECISION = PrecisionConfig()
+_NO_ACTIVATION = FusedActivation()
+_NO_EPILOGUE = Epilogue()
+_DEFAULT_FLEX = _NO_PRECISION.flex_ctx
+_BF16, _F16, _F32, _U8, _I32, _E4M3 = torch.bfloat16, torch.float16, torch.float32, torch.uint8, torch.int32, torch.float8_e4m3fn
+
+
 def matmul_set_idle_sms(num_idle_sms):
     set_idle_sms(num_idle_sms)
 
@@ -112,13 +122,13 @@ _TILE_COUNTERS: dict = {}
 _STATIC_TILES = False  # True: the persistent kernels walk their static tile schedule (for comparisons)
 
 
-def _tile_counters(device: torch.device) -> torch.Tensor:
+def _tile_counters(device: torch.device, stream: int | None = None) -> torch.Tensor:
     """Zeroed int32 words the persistent kernels claim tiles with (`tk_gemm_desc.tile_counters`): one small buffer
     per (device, stream), made on first use and kept for the life of the process.  A kernel leaves the words zero, so
     launches in stream order share them; launches on different streams get different buffers.  (A buffer first made
     while a HIP graph is being captured belongs to the capture stream: graphs captured on one stream must not be
     replayed concurrently with each other.)"""
-    key = (device.index, nt.stream_ptr(device))
+    key = (device.index, nt.stream_ptr(device) if stream is None else stream)
     buf = _TILE_COUNTERS.get(key)
     if buf is None:
         buf = torch.zeros(32, dtype=torch.int32, device=device)
@@ -142,7 +152,7 @@ def _combine_counters(device: torch.device) -> torch.Tensor:
 
 
 def _flex_out_is_trivial(flex: FlexCtx) -> bool:
-    return (flex.acc_data.scale is None and flex.out_data.expected_scale is None and flex.out_data.actual_scale is None
+    return flex is _DEFAULT_FLEX or (flex.acc_data.scale is None and flex.out_data.expected_scale is None and flex.out_data.actual_scale is None
             and flex.out_data.checksum_scale is None)
 
 
@@ -442,6 +452,20 @@ def _matmul_ragged_k(a, b, bias, a_ragged_metadata, b_ragged_metadata, gather_in
     return c
 
 
+def _dma_block_m(rows: int, row_bytes: int, N: int, n_slices: int) -> int:
+    """Row blocks of the memory-to-LDS kernel: 256 (256 x 256 tiles, one workgroup per CU) or 128 (128 x 128, two per CU).  The large
+    tile moves half the operand bytes per product, the small one fills the chip with fewer rows.  Measured on 8 to 32 slices: up to
+    64 rows per slice the small tile is as fast or faster (e4m3, 8 rows, K 4096: 174 against 183 us), from 192 on the large one
+    is (e4m3, 256 rows: 350 against 456 us); in between it depends on the large tiles there are for the 256 CUs (bf16, 128
+    rows, K 2048: N 4096, 256 tiles, 56 against 72 us; N 2048, 128 tiles, 44 against 38 us) and, with fewer, on the length
+    of a row, which a tile's start and end have to be paid from (e4m3, 128 tiles, K 14336: 168 against 214 us)."""
+    per_slice = rows // max(n_slices, 1)
+    if per_slice <= 64:
+        return 128
+    tiles = n_slices * ((per_slice + 255) // 256) * ((N + 255) // 256)
+    return 256 if per_slice >= 192 or tiles >= 192 or row_bytes >= 8192 else 128
+
+
 def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
            b_ragged_metadata: RaggedTensorMetadata | None = None, gather_indx: torch.Tensor | None = None,
            scatter_indx: torch.Tensor | None = None, precision_config: PrecisionConfig | None = None,
@@ -474,12 +498,15 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
     if c_acc_in is not None and scatter_indx is not None:
         raise AssertionError("c_acc_in + scatter is not supported.")  # triton_kernels/matmul.py:531
     if precision_config is None:
-        precision_config = PrecisionConfig()
+        precision_config = _NO_PRECISION
     if fused_activation is None:
-        fused_activation = FusedActivation(FnSpecs.default(), tuple())
+        fused_activation = _NO_ACTIVATION
     if epilogue is None:
-        epilogue = Epilogue(FnSpecs.default(), tuple(), tuple(), False)
-    a, b, precision_config = _expand_operands(a, b, precision_config)
+        epilogue = _NO_EPILOGUE
+    # (bf16 / fp16 activations with weights that are not strided fp8 need no look at the operand pair)
+    b_data = b.storage.data if isinstance(b, Tensor) else b
+    if a_data.dtype not in (_BF16, _F16) or b_data.dtype in _FP8_TYPES or precision_config.a_mx_scale is not None:
+        a, b, precision_config = _expand_operands(a, b, precision_config)
     # MXFP8 activations (`a_mx_scale`): e4m3 values with one e8m0 scale per 32 k, multiplied with tiled MXFP4 weights
     # on the scaled MFMA (triton_kernels/matmul.py:130-132,783-795)
     a_scale = precision_config.a_mx_scale
@@ -496,7 +523,9 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
         assert precision_config.a_microblock_size in (None, MXFP_BLOCK_SIZE), \
             f"Unsupported microscale block size {precision_config.a_microblock_size}"
     mx_out_fused = False
-    if epilogue.specs.name in (FnName.QUANTIZE_MXFP8.name, FnName.QUANTIZE_MXFP4.name):
+    if epilogue is _NO_EPILOGUE and precision_config.c_mx_scale is None:
+        pass
+    elif epilogue.specs.name in (FnName.QUANTIZE_MXFP8.name, FnName.QUANTIZE_MXFP4.name):
         # with MXFP8 activations the kernel quantises its fp32 accumulator itself; otherwise the bf16 GEMM is followed
         # by the MX quantiser
         mx_out_fused = (mx_act and epilogue.specs.name == FnName.QUANTIZE_MXFP8.name
@@ -530,56 +559,62 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
     a = flex.lhs_data.reinterpret(a)
     assert a.ndim == 2
     nt.require_gpu(a, "a")
+    device = a.device
     # ---- weights -------------------------------------------------------------------------------
     b_scale = precision_config.b_mx_scale
-    if not isinstance(b, Tensor):
-        b = wrap_torch_tensor(b, dtype=FP4 if b.dtype == torch.uint8 else None)
-    tiled = isinstance(b.storage.layout, GFX950MXValueLayout)
-    tiled_fp8 = isinstance(b.storage.layout, GFX950FP8ValueLayout)
-    if not tiled and not tiled_fp8 and not isinstance(b.storage.layout, StridedLayout):
-        raise NotImplementedError(f"weight layout {type(b.storage.layout).__name__} is not supported")
-    if b_scale is not None and not isinstance(b_scale, Tensor):
-        b_scale = wrap_torch_tensor(b_scale)
-    if b_scale is not None and isinstance(b_scale.storage.layout, CDNA4MXScaleLayout):
-        # the reference's scale pre-shuffle: converted once to the order that goes with the values' layout and
-        # kept on the wrapper (weights are static; re-wrap the tensor after changing its storage in place)
-        want = GFX950MXScaleLayout() if tiled else StridedLayout(-2)
-        cached = getattr(b_scale, "_tk_converted", None)
-        if cached is None or cached[0] != want:
-            cached = (want, convert_layout(b_scale, want))
-            b_scale._tk_converted = cached
-        b_scale = cached[1]
+    if isinstance(b, Tensor):
+        w, layout, fp4, (K_W, N) = b.storage.data, type(b.storage.layout), b.dtype == FP4, b.shape[-2:]
+    elif b.dtype == _U8:
+        b = wrap_torch_tensor(b, dtype=FP4)
+        w, layout, fp4, (K_W, N) = b.storage.data, StridedLayout, True, b.shape[-2:]
+    else:
+        w, layout, fp4, (K_W, N) = b, StridedLayout, False, b.shape[-2:]
+    tiled, tiled_fp8 = layout is GFX950MXValueLayout, layout is GFX950FP8ValueLayout
+    strided = layout is StridedLayout
+    if not (tiled or tiled_fp8 or strided):
+        raise NotImplementedError(f"weight layout {layout.__name__} is not supported")
     if b_scale is not None:
+        if not isinstance(b_scale, Tensor):
+            b_scale = wrap_torch_tensor(b_scale)
+        if isinstance(b_scale.storage.layout, CDNA4MXScaleLayout):
+            # the reference's scale pre-shuffle: converted once to the order that goes with the values' layout and
+            # kept on the wrapper (weights are static; re-wrap the tensor after changing its storage in place)
+            want = GFX950MXScaleLayout() if tiled else StridedLayout(-2)
+            cached = getattr(b_scale, "_tk_converted", None)
+            if cached is None or cached[0] != want:
+                cached = (want, convert_layout(b_scale, want))
+                b_scale._tk_converted = cached
+            b_scale = cached[1]
         if tiled != isinstance(b_scale.storage.layout, GFX950MXScaleLayout):
             raise NotImplementedError("tiled MXFP4 values go with tiled scales (convert both with convert_layout)")
         if not tiled and not isinstance(b_scale.storage.layout, StridedLayout):
             raise NotImplementedError(f"scale layout {type(b_scale.storage.layout).__name__} is not supported")
-        assert b_scale.storage.data.dtype == torch.uint8, f"Unsupported microscale dtype {b_scale.storage.data.dtype}"
+        assert b_scale.storage.data.dtype == _U8, f"Unsupported microscale dtype {b_scale.storage.data.dtype}"
         assert precision_config.b_microblock_size is None or precision_config.b_microblock_size == MXFP_BLOCK_SIZE, \
             f"Unsupported microscale block size {precision_config.b_microblock_size}"
-    w = b.storage.data
-    if not tiled and not tiled_fp8 and b.dtype != FP4:
-        w = _k_contiguous(w)  # before any view is taken: the converted copy is cached on the caller's tensor
-    if w.ndim == 2 and not tiled and not tiled_fp8:
-        w = w[None]
-    K_W, N = b.shape[-2:]
-    M = a.shape[-2] if gather_indx is None else gather_indx.shape[0]
-    K = a.shape[-1]
+    if strided:
+        if not fp4:
+            w = _k_contiguous(w)  # before any view is taken: the converted copy is cached on the caller's tensor
+        if w.ndim == 2:
+            w = w[None]
+    n_w = w.shape[0]
+    M = a.shape[0] if gather_indx is None else gather_indx.shape[0]
+    K = a.shape[1]
     assert K == K_W, f"reduction dims differ: a has K={K}, b has K={K_W}"
     is_ragged = a_ragged_metadata is not None
     if is_ragged and getattr(a_ragged_metadata, "remapped_from", None) is not None:
         _combine_k = None  # only the local experts' rows arrive: tokens are incomplete
-        a_ragged_metadata = _localise_remapped_metadata(a_ragged_metadata, w.shape[0], M)
-    n_slices = a_ragged_metadata.n_slices if is_ragged else w.shape[0]
-    if not is_ragged and w.shape[0] != 1:
+        a_ragged_metadata = _localise_remapped_metadata(a_ragged_metadata, n_w, M)
+    n_slices = a_ragged_metadata.n_slices if is_ragged else n_w
+    if not is_ragged and n_w != 1:
         raise NotImplementedError("batched weights need ragged metadata")
     if is_ragged:
-        assert w.shape[0] == n_slices, f"{w.shape[0]} weight slices for {n_slices} ragged slices"
+        assert n_w == n_slices, f"{n_w} weight slices for {n_slices} ragged slices"
     # ---- output --------------------------------------------------------------------------------
     reduction_n = fused_activation.specs.reduction_n
     act = nt.TK_ACT_NONE
     alpha, limit, has_limit = 0.0, 0.0, 0
-    if fused_activation.specs.fn is not None or fused_activation.specs.name != "dflt":
+    if fused_activation is not _NO_ACTIVATION and (fused_activation.specs.fn is not None or fused_activation.specs.name != "dflt"):
         if fused_activation.specs.name != "swiglu" or reduction_n != 2:
             raise NotImplementedError(f"fused activation {fused_activation.specs.name!r} is not supported")
         act = nt.TK_ACT_SWIGLU
@@ -588,10 +623,11 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
         has_limit = int(lim is not None)
         limit = float(lim) if lim is not None else 0.0
     out_dtype = precision_config.out_dtype or a.dtype
-    f16 = a.dtype == torch.float16 or w.dtype == torch.float16
-    if f16 and not (a.dtype == w.dtype == out_dtype == torch.float16 and not (tiled or tiled_fp8 or mx_act) and b_scale is None):
+    a_dtype, w_dtype = a.dtype, w.dtype
+    f16 = a_dtype == _F16 or w_dtype == _F16
+    if f16 and not (a_dtype == w_dtype == out_dtype == _F16 and not (tiled or tiled_fp8 or mx_act) and b_scale is None):
         raise NotImplementedError(f"fp16 activations go with strided fp16 weights and an fp16 output (got {a.dtype} x {w.dtype} -> {out_dtype})")
-    if out_dtype != torch.bfloat16 and not mx_out_fused and not f16:
+    if out_dtype != _BF16 and not mx_out_fused and not f16:
         raise NotImplementedError(f"output dtype {out_dtype} is not supported (bf16, or fp16 for fp16 operands); set precision_config.out_dtype")
     y_rows = scatter_indx.shape[0] if scatter_indx is not None else M
     out_shape = (y_rows, N // reduction_n)
@@ -611,162 +647,143 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
             out_shape = (y_rows, out_shape[1] // 2)  # two e2m1 codes per byte
     caller_c = c is not None
     if c is None:
-        c = torch.empty(out_shape, dtype=out_dtype, device=a.device)
+        c = torch.empty(out_shape, dtype=out_dtype, device=device)
     else:
         assert tuple(c.shape[-2:]) == out_shape and c.dtype == out_dtype and c.stride(-1) == 1
         c = c.view(out_shape) if c.ndim > 2 else c
-    opt_flags = make_opt_flags(torch_dtype_to_dtype(out_dtype), torch_dtype_to_dtype(a.dtype), b.dtype, precision_config,
-                               1, M, N, K, a_ragged_metadata, epilogue_reduction_n=reduction_n)
+    if unconstrained():
+        block_m, forced, idle = default_block_m(M, a_ragged_metadata), None, _get_idle_sms()
+    else:
+        opt_flags = make_opt_flags(torch_dtype_to_dtype(out_dtype), torch_dtype_to_dtype(a_dtype),
+                                   FP4 if fp4 else torch_dtype_to_dtype(w_dtype if strided else _E4M3), precision_config, 1, M, N, K, a_ragged_metadata, epilogue_reduction_n=reduction_n)
+        block_m, forced, idle = opt_flags.block_m, _get_opt_flags_constraints().get("block_m"), opt_flags.idle_sms
     if M * N == 0:
         return c
-    if a.stride(-1) != 1:
+    if a.stride(1) != 1:
         a = a.contiguous()
+    a_rows, a_stride = a.shape[0], a.stride(0)
     d = nt.GemmDesc()
-    d.x = a.data_ptr()
-    d.x_dtype = nt.TORCH_TO_TK[a.dtype]
-    d.x_stride_m = a.stride(0)
-    d.x_rows = a.shape[0]
+    d.x, d.x_dtype, d.x_stride_m, d.x_rows = a.data_ptr(), nt.TORCH_TO_TK[a_dtype], a_stride, a_rows
+    keep = []  # tensors made here that the launch reads
     a_ts = precision_config.a_mx_tensor_scale
     if a_ts is not None:
-        a_ts = a_ts.to(torch.float32).reshape(-1).contiguous()
-        assert a_ts.numel() == a.shape[0], "a_mx_tensor_scale must hold one scale per row of a"
-    if flex.lhs_data.scale is not None:
+        a_ts = a_ts.to(_F32).reshape(-1).contiguous()
+        assert a_ts.numel() == a_rows, "a_mx_tensor_scale must hold one scale per row of a"
+    if flex is not _DEFAULT_FLEX and flex.lhs_data.scale is not None:
         # flexpoint input scale (`acc *= x_scale * w_scale` before the bias, matmul_details/_matmul.py:540-547): a
         # one-element device tensor, folded into the per-row scale the kernel already applies (no host read)
-        xs = flex.lhs_data.scale.to(torch.float32).reshape(-1)
+        xs = flex.lhs_data.scale.to(_F32).reshape(-1)
         if xs.numel() != 1:
             raise NotImplementedError("per-batch flexpoint scales need batched activations, which are not supported")
-        a_ts = a_ts * xs if a_ts is not None else xs.expand(a.shape[0]).contiguous()
+        a_ts = a_ts * xs if a_ts is not None else xs.expand(a_rows).contiguous()
     if a_ts is not None:
         d.x_row_scale = a_ts.data_ptr()
-    keep = [a_ts]
+        keep.append(a_ts)
     if mx_act:
-        if a.dtype != torch.float8_e4m3fn:
-            raise NotImplementedError(f"MX-quantised activations must be float8_e4m3fn (got {a.dtype})")
+        if a_dtype != _E4M3:
+            raise NotImplementedError(f"MX-quantised activations must be float8_e4m3fn (got {a_dtype})")
         if a_ts is not None:
             raise NotImplementedError("a_mx_tensor_scale / flexpoint scales are not supported with a_mx_scale")
-        assert tuple(a_scale.shape) == (a.shape[0], (K + MXFP_BLOCK_SIZE - 1) // MXFP_BLOCK_SIZE), \
-            f"a_mx_scale must be [{a.shape[0]}, {(K + 31) // 32}], got {tuple(a_scale.shape)}"
+        assert tuple(a_scale.shape) == (a_rows, (K + MXFP_BLOCK_SIZE - 1) // MXFP_BLOCK_SIZE), \
+            f"a_mx_scale must be [{a_rows}, {(K + 31) // 32}], got {tuple(a_scale.shape)}"
         if a_scale.stride(-1) != 1:
             a_scale = a_scale.contiguous()
-        d.x_mx_scale = a_scale.data_ptr()
-        d.xs_stride_m = a_scale.stride(0)
+        d.x_mx_scale, d.xs_stride_m = a_scale.data_ptr(), a_scale.stride(0)
         keep.append(a_scale)
+    d.w = w.data_ptr()
+    if strided:
+        d.w_stride_e, d.w_stride_k, d.w_stride_n = w.stride()
+    else:
+        assert w.is_contiguous() and w_dtype == _U8
+        d.w_layout, d.w_stride_e = nt.TK_W_TILED, w.stride(0)
     if tiled_fp8:
         if b_scale is not None:
             raise NotImplementedError("MX scales are supported with mxfp4 (uint8) weights only")
-        if a.dtype != torch.float8_e4m3fn:
+        if a_dtype != _E4M3:
             raise NotImplementedError("tiled e4m3 weights take e4m3 activations (quantise with quantize_fp8_rowwise)")
-        assert w.is_contiguous() and w.dtype == torch.uint8
         d.w_dtype = nt.TK_E4M3
-        d.w_layout = nt.TK_W_TILED
     elif tiled:
-        assert b.dtype == FP4 and b_scale is not None, "tiled weights are MXFP4 and need precision_config.b_mx_scale"
+        assert fp4 and b_scale is not None, "tiled weights are MXFP4 and need precision_config.b_mx_scale"
         ws = b_scale.storage.data
-        assert w.is_contiguous() and ws.is_contiguous() and ws.shape[0] == w.shape[0]
-        d.w_dtype = nt.TK_E2M1
-        d.w_layout = nt.TK_W_TILED
-        d.w_mx_scale = ws.data_ptr()
-        d.ws_stride_e = ws.stride(0)
-        keep.append(ws)
-    elif b.dtype == FP4:
+        assert ws.is_contiguous() and ws.shape[0] == n_w
+        d.w_dtype, d.w_mx_scale, d.ws_stride_e = nt.TK_E2M1, ws.data_ptr(), ws.stride(0)
+    elif fp4:
         assert b_scale is not None, "mxfp4 weights need precision_config.b_mx_scale"
-        assert w.dtype == torch.uint8
+        assert w_dtype == _U8
         if w.stride(-2) != 1:
             raise NotImplementedError("mxfp4 weights must be packed along K (stride(-2) == 1)")
         ws = _k_contiguous(b_scale.storage.data)
         ws = ws[None] if ws.ndim == 2 else ws
-        d.w_dtype = nt.TK_E2M1
-        d.w_mx_scale = ws.data_ptr()
+        d.w_dtype, d.w_mx_scale = nt.TK_E2M1, ws.data_ptr()
         d.ws_stride_e, d.ws_stride_k, d.ws_stride_n = ws.stride()
         keep.append(ws)
     else:
         if b_scale is not None:
             raise NotImplementedError("MX scales are supported with mxfp4 (uint8) weights only")
-        d.w_dtype = nt.TORCH_TO_TK.get(w.dtype, -1)
-    d.w = w.data_ptr()
-    if tiled or tiled_fp8:
-        d.w_stride_e = w.stride(0)
-    else:
-        d.w_stride_e, d.w_stride_k, d.w_stride_n = w.stride()
-    keep.append(w)
+        d.w_dtype = nt.TORCH_TO_TK.get(w_dtype, -1)
     b_ts = precision_config.b_mx_tensor_scale
     if b_ts is not None:
-        b_ts = b_ts.to(torch.float32).reshape(w.shape[0], N).contiguous()
-    if flex.rhs_data.scale is not None:
+        b_ts = b_ts.to(_F32).reshape(n_w, N).contiguous()
+    if flex is not _DEFAULT_FLEX and flex.rhs_data.scale is not None:
         # one scale for all experts or one per expert (PER_BATCH_W_SCALE), folded into the per-column scale
-        ws_ = flex.rhs_data.scale.to(torch.float32).reshape(-1)
-        if ws_.numel() not in (1, w.shape[0]):
-            raise ValueError(f"rhs flexpoint scale must hold 1 or {w.shape[0]} values, got {ws_.numel()}")
-        col = ws_.reshape(-1, 1).expand(w.shape[0], N)
+        ws_ = flex.rhs_data.scale.to(_F32).reshape(-1)
+        if ws_.numel() not in (1, n_w):
+            raise ValueError(f"rhs flexpoint scale must hold 1 or {n_w} values, got {ws_.numel()}")
+        col = ws_.reshape(-1, 1).expand(n_w, N)
         b_ts = b_ts * col if b_ts is not None else col.contiguous()
     if b_ts is not None:
-        d.w_col_scale = b_ts.data_ptr()
-        d.wcs_stride_e = b_ts.stride(0)
+        d.w_col_scale, d.wcs_stride_e = b_ts.data_ptr(), b_ts.stride(0)
         keep.append(b_ts)
     if bias is not None:
         bias2 = bias[None] if bias.ndim == 1 else bias
-        if bias2.stride(-1) != 1 or bias2.dtype not in (torch.float32, torch.bfloat16):
-            bias2 = bias2.to(torch.float32).contiguous()
-        d.bias = bias2.data_ptr()
-        d.bias_dtype = nt.TORCH_TO_TK[bias2.dtype]
-        d.bias_stride_e = bias2.stride(0)
+        if bias2.stride(-1) != 1 or bias2.dtype not in (_F32, _BF16):
+            bias2 = bias2.to(_F32).contiguous()
+        d.bias, d.bias_dtype, d.bias_stride_e = bias2.data_ptr(), nt.TORCH_TO_TK[bias2.dtype], bias2.stride(0)
         keep.append(bias2)
     if gather_indx is not None:
-        assert gather_indx.dtype == torch.int32
+        assert gather_indx.dtype == _I32
         gather_indx = gather_indx.contiguous()
         d.gather_indx = gather_indx.data_ptr()
     if scatter_indx is not None:
-        assert scatter_indx.dtype == torch.int32
+        assert scatter_indx.dtype == _I32
         scatter_indx = scatter_indx.contiguous()
-        d.scatter_indx = scatter_indx.data_ptr()
-        d.scatter_len = scatter_indx.shape[0]
+        d.scatter_indx, d.scatter_len = scatter_indx.data_ptr(), y_rows
     if gammas is not None:
-        g = gammas if gammas.dtype in (torch.float32, torch.bfloat16) else gammas.to(torch.float32)
+        g = gammas if gammas.dtype in (_F32, _BF16) else gammas.to(_F32)
         g = g.contiguous()
-        d.gammas = g.data_ptr()
-        d.gammas_dtype = nt.TORCH_TO_TK[g.dtype]
+        d.gammas, d.gammas_dtype = g.data_ptr(), nt.TORCH_TO_TK[g.dtype]
         keep.append(g)
-    block_m = opt_flags.block_m
     if tiled_fp8:
-        from .matmul_details.opt_flags import _get_opt_flags_constraints
-        forced = _get_opt_flags_constraints().get("block_m")
-        # the FP8 MFMA kernels' row blocks: 256 x 256 tiles from 512 rows per slice on (every row fragment of a block is
-        # multiplied there, so blocks should be mostly full) when K is long enough to pay for the larger tile's set-up
-        # and epilogue (measured at 16384 rows: K 14336 12 % faster, K 4096 2 % slower), 128-row tiles otherwise
-        rows_per_slice = M // max(n_slices, 1) if is_ragged else M
-        block_m = 256 if (forced == 256 or (forced is None and rows_per_slice >= 512 and K >= 8192)) else 128
-    elif mx_act:
-        from .matmul_details.opt_flags import _get_opt_flags_constraints
-        forced = _get_opt_flags_constraints().get("block_m")
+        block_m = forced if forced in (128, 256) else 128 if forced is not None else _dma_block_m(M, K, N, n_slices)
+    elif mx_act or (tiled and mx_out_fused):
+        # the tile shapes that take MXFP8 activations / have an MX-output epilogue
         block_m = 256 if (forced == 256 or (forced is None and is_ragged and M <= 144 * n_slices)) else 128
-    elif tiled and mx_out_fused:
-        from .matmul_details.opt_flags import _get_opt_flags_constraints
-        forced = _get_opt_flags_constraints().get("block_m")
-        block_m = 256 if (forced == 256 or (forced is None and is_ragged and M <= 144 * n_slices)) else 128  # the tile shapes with an MX-output epilogue
-    elif tiled and extras:
-        block_m = min(block_m, 32)  # the decode kernel carries the shared epilogue; the prefill kernels do not take these options
     elif tiled:
-        from .matmul_details.opt_flags import _get_opt_flags_constraints
-        if block_m == 128 and _get_opt_flags_constraints().get("block_m") is None and is_ragged and M <= 144 * n_slices:
+        if extras:
+            block_m = min(block_m, 32)  # the decode kernel carries the shared epilogue; the prefill kernels do not take these options
+        elif block_m == 128 and forced is None and is_ragged and M <= 144 * n_slices:
             block_m = 256  # about 128 rows per expert: one tile per expert, the weights are read once
+    elif w_dtype in (_BF16, _F16):
+        # (the conditions of the memory-to-LDS kernel: x and an expert's weights within 2 GiB, up to 256 slices)
+        dma = a_rows * a_stride < 1 << 30 and n_slices <= 256 and N * w.stride(-1) < 1 << 30
+        if not dma:
+            block_m = min(block_m, 128)
+        elif forced is None and block_m > 16:
+            block_m = _dma_block_m(M, 2 * K, N, n_slices)
     elif block_m == 256:
         block_m = 128
     if is_ragged:
         md = a_ragged_metadata
-        d.slice_sizes = md.slice_sizes.data_ptr()
-        d.slice_offs = md.slice_offs.data_ptr()
-        bo, bs = md.block_offs(block_m), md.block_schedule(block_m)
-        assert bo.stride(0) == 1 and (bs.numel() == 0 or bs.stride(0) == 1)
-        d.block_offs = bo.data_ptr()
-        d.block_schedule = bs.data_ptr()
+        bo, bs, i = md.block_offs_data, md.block_schedule_data, _BLOCK_SIZES.index(block_m)
+        assert bo.stride(1) == 1 and (bs.numel() == 0 or bs.stride(1) == 1)
+        d.slice_sizes, d.slice_offs = md.slice_sizes.data_ptr(), md.slice_offs.data_ptr()
+        d.block_offs, d.block_schedule = bo.data_ptr() + 4 * i * bo.stride(0), bs.data_ptr() + 4 * i * bs.stride(0)
         d.n_slices = n_slices
-        d.grid_m = min(RaggedTensorMetadata.n_blocks(n_slices, M, block_m), bs.shape[0])
+        d.grid_m = min(RaggedTensorMetadata.n_blocks(n_slices, M, block_m), bs.shape[1])
     else:
         d.n_slices = 1
         d.grid_m = (M + block_m - 1) // block_m
-    d.block_m = block_m
-    d.M, d.N, d.K = M, N, K
+    d.block_m, d.M, d.N, d.K = block_m, M, N, K
     y_buf = c
     if tiled and block_m >= 64 and not mx_act and not mx_out_fused:
         # the prefill kernels write whole 16-byte pieces through a buffer resource: rows 16-byte aligned and padded to
@@ -774,55 +791,47 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
         # caller's own `c` whose last piece would spill past its columns (they may belong to a wider tensor).
         n_pad = (out_shape[1] + 7) // 8 * 8
         if c.stride(0) % 8 or c.data_ptr() % 16 or c.stride(0) < n_pad or (caller_c and out_shape[1] % 8):
-            y_buf = torch.empty((out_shape[0], n_pad), dtype=c.dtype, device=c.device)[:, :out_shape[1]]
-    d.y = y_buf.data_ptr()
-    d.y_dtype = nt.TK_E2M1 if fp4_out else nt.TORCH_TO_TK[c.dtype]
-    d.y_stride_m = y_buf.stride(0)
-    d.activation = act
-    d.act_alpha, d.act_limit, d.act_has_limit = alpha, limit, has_limit
-    d.idle_cus = max(0, int(opt_flags.idle_sms or 0))
+            y_buf = torch.empty((out_shape[0], n_pad), dtype=c.dtype, device=device)[:, :out_shape[1]]
+    d.y, d.y_dtype, d.y_stride_m = y_buf.data_ptr(), nt.TK_E2M1 if fp4_out else nt.TORCH_TO_TK[out_dtype], y_buf.stride(0)
+    if act:
+        d.activation, d.act_alpha, d.act_limit, d.act_has_limit = act, alpha, limit, has_limit
+    if idle:
+        d.idle_cus = max(0, int(idle))
     if c_scale is not None:
-        d.y_mx_scale = c_scale.data_ptr()
-        d.ys_stride_m = c_scale.stride(-2)
+        d.y_mx_scale, d.ys_stride_m = c_scale.data_ptr(), c_scale.stride(-2)
     if betas is not None:
         assert betas.shape[0] == M, f"betas must hold one value per row ({M}), got {tuple(betas.shape)}"
-        be = betas if betas.dtype in (torch.float32, torch.bfloat16) else betas.to(torch.float32)
+        be = betas if betas.dtype in (_F32, _BF16) else betas.to(_F32)
         be = be.contiguous()
-        d.betas = be.data_ptr()
-        d.betas_dtype = nt.TORCH_TO_TK[be.dtype]
+        d.betas, d.betas_dtype = be.data_ptr(), nt.TORCH_TO_TK[be.dtype]
         keep.append(be)
     if out_alpha is not None:
-        d.has_out_alpha = 1
-        d.out_alpha = float(out_alpha)
+        d.has_out_alpha, d.out_alpha = 1, float(out_alpha)
     if c_acc_in is not None:
         acc_in = c_acc_in.view(out_shape) if c_acc_in.ndim > 2 else c_acc_in
         if tuple(acc_in.shape) != out_shape or acc_in.dtype != c.dtype or acc_in.stride(-1) != 1:
             raise NotImplementedError(f"c_acc_in must have the output's shape {out_shape} and dtype {c.dtype} with unit stride along N")
-        d.acc_in = acc_in.data_ptr()
-        d.acc_in_stride_m = acc_in.stride(0)
+        d.acc_in, d.acc_in_stride_m = acc_in.data_ptr(), acc_in.stride(0)
         keep.append(acc_in)
     if (tiled or tiled_fp8) and block_m >= 64 and not _STATIC_TILES and not mx_act:
-        d.tile_counters = _tile_counters(a.device).data_ptr()
+        d.tile_counters = _tile_counters(device).data_ptr()
     combined = None
     # (not with MXFP8 activations: at the end of that kernel's launch the combine measured 22 us slower than `reduce` in a
     # launch of its own at the gpt-oss shape)
-    can_combine = (_combine_k and not extras and tiled and not mx_act and act == nt.TK_ACT_NONE and scatter_indx is not None
-                   and scatter_indx.shape[0] % _combine_k == 0 and a.dtype == torch.bfloat16)
+    can_combine = (_combine_k and tiled and not extras and not mx_act and act == nt.TK_ACT_NONE and scatter_indx is not None
+                   and y_rows % _combine_k == 0 and a_dtype == _BF16)
     if can_combine and block_m <= 32:
         # decode kernel: the wave that completes a token's rows last sums them (arrival counters per token and fragment)
-        can_combine = (scatter_indx.shape[0] // _combine_k) * ((N + 31) // 32) <= _COMBINE_COUNTER_WORDS
+        can_combine = (y_rows // _combine_k) * ((N + 31) // 32) <= _COMBINE_COUNTER_WORDS
     elif can_combine:
         # prefill kernel: the persistent grid sums when all its workgroups have written their tiles
         can_combine = bool(d.tile_counters) and N % 8 == 0 and y_buf is c
     if can_combine:
-        combined = torch.empty((scatter_indx.shape[0] // _combine_k, N), dtype=c.dtype, device=c.device)
-        d.combine_k = int(_combine_k)
-        d.combine_out = combined.data_ptr()
-        d.combine_stride_m = combined.stride(0)
+        combined = torch.empty((y_rows // _combine_k, N), dtype=out_dtype, device=device)
+        d.combine_k, d.combine_out, d.combine_stride_m = int(_combine_k), combined.data_ptr(), combined.stride(0)
         if block_m <= 32:
-            d.combine_counters = _combine_counters(a.device).data_ptr()
-    with nt.on_device(a.device):
-        nt.check(nt.lib().tk_moe_gemm(d, nt.stream_ptr(a.device)))
+            d.combine_counters = _combine_counters(device).data_ptr()
+    nt.submit(nt.lib().tk_moe_gemm, d, device)
     del keep
     if y_buf is not c:
         c.copy_(y_buf)

@@ -10,7 +10,8 @@ workgroup) and the weight format:
       32        128      256      4        128      128
       64        256      128      4        128      128
      128        256      128      4        128      128         prefill: ~128 rows per expert
-     256        256      128      4         -        -          pre-tiled MXFP4 only: a whole expert (<= 160 rows) per tile
+     256        256      128      4        256       64         pre-tiled MXFP4: a whole expert (<= 160 rows) per tile; 16-bit and
+                                                                tiled e4m3 weights: from about 128 rows per expert on
 
 so only `block_m` can be forced; `block_n`, `block_k` and `num_warps` constraints must match the table.
 `split_k > 1` and `is_persistent=True` cannot be honoured and raise `InapplicableConstraint`, which is
@@ -88,6 +89,11 @@ def set_idle_sms(num_idle_sms: int):
 def _get_opt_flags_constraints() -> dict:
     c = _opt_flags_constraints.get()
     return {} if c is None else c
+
+
+def unconstrained() -> bool:
+    """Neither constraints nor forced flags are in effect: the tile follows from the problem alone."""
+    return not _opt_flags_constraints.get() and _opt_flags.get() is None
 
 
 def update_opt_flags_constraints(constraints: dict):

@@ -14,6 +14,9 @@ import torch
 from .. import _native as nt
 
 
+_BLOCK_SIZES = (16, 32, 64, 128, 256)
+
+
 @dataclass
 class RaggedTensorMetadata:
     slice_sizes: torch.Tensor  # [n_slices] int32 rows per slice
@@ -24,7 +27,7 @@ class RaggedTensorMetadata:
     slice_sizes_divisibility: int = None
 
     def __post_init__(self):
-        n = len(RaggedTensorMetadata.block_sizes())
+        n = len(_BLOCK_SIZES)
         assert self.block_offs_data.shape[0] == n
         assert self.block_schedule_data.shape[0] == n
         assert self.block_offs_data.dtype == torch.int32
@@ -39,10 +42,10 @@ class RaggedTensorMetadata:
         return self.slice_sizes.shape[0]
 
     def block_offs(self, block_size):
-        return self.block_offs_data[RaggedTensorMetadata.block_sizes().index(block_size)]
+        return self.block_offs_data[_BLOCK_SIZES.index(block_size)]
 
     def block_schedule(self, block_size):
-        return self.block_schedule_data[RaggedTensorMetadata.block_sizes().index(block_size)]
+        return self.block_schedule_data[_BLOCK_SIZES.index(block_size)]
 
     @staticmethod
     def n_blocks(n_slices, n_total_rows, block_size):
@@ -53,7 +56,7 @@ class RaggedTensorMetadata:
 
     @staticmethod
     def max_n_blocks(n_slices, n_total_rows):
-        return RaggedTensorMetadata.n_blocks(n_slices, n_total_rows, min(RaggedTensorMetadata.block_sizes()))
+        return RaggedTensorMetadata.n_blocks(n_slices, n_total_rows, _BLOCK_SIZES[0])
 
     @staticmethod
     def block_sizes_log2():
@@ -61,7 +64,7 @@ class RaggedTensorMetadata:
 
     @staticmethod
     def block_sizes():
-        return [2**x for x in RaggedTensorMetadata.block_sizes_log2()]
+        return list(_BLOCK_SIZES)
 
 
 def ragged_metadata_fields(metadata, block_size):
@@ -71,7 +74,7 @@ def ragged_metadata_fields(metadata, block_size):
 
 def _alloc(n_slices, n_total_rows, device):
     """(slice_offs, block_offs_data, block_schedule_data) as rows of two int32 buffers."""
-    n_bs = len(RaggedTensorMetadata.block_sizes())
+    n_bs = len(_BLOCK_SIZES)
     width = RaggedTensorMetadata.max_n_blocks(n_slices, n_total_rows)
     offs = torch.empty((n_bs + 1, n_slices + 1), dtype=torch.int32, device=device)
     sched = torch.empty((n_bs, max(width, 0)), dtype=torch.int32, device=device)
