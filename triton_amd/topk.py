@@ -22,6 +22,12 @@ def _cdiv(a, b):
     return (a + b - 1) // b
 
 
+def check_topk(k: int, E: int):
+    assert E < 32768
+    if k & (k - 1) or k > 32:
+        raise ValueError(f"k must be a power of two <= 32 (got {k})")
+
+
 def _topk_route(x, k, apply_softmax, y_indx, n_rows, *, want_meta, want_extras=False, ragged=None):
     if isinstance(x, Tensor):
         n_rows = x.shape[0] if n_rows is None else n_rows
@@ -29,11 +35,9 @@ def _topk_route(x, k, apply_softmax, y_indx, n_rows, *, want_meta, want_extras=F
     assert x.ndim == 2
     nt.require_gpu(x, "x")
     T, E = x.shape
-    assert E < 32768
+    check_topk(k, E)
     if x.stride(1) != 1:
         x = x.contiguous()
-    if k & (k - 1) or k > 32:
-        raise ValueError(f"k must be a power of two <= 32 (got {k})")
     dev = x.device
     y_vals = torch.empty((T, k), dtype=x.dtype, device=dev)
     provided = y_indx is not None
