@@ -65,11 +65,24 @@ __device__ __forceinline__ buf_desc_t make_buf_desc(const void* base, uint32_t b
   return buf_desc_t{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(a >> 32) & 0xFFFFu)),
                     (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
 }
-// 16 bytes per lane from `desc` at byte offset `off` + `soff` into LDS at `dst` (wave-uniform byte address) + 16 * lane.  Written
+// 16 bytes per lane from `desc` at byte offset `off` into LDS at `dst` (wave-uniform byte address) + 16 * lane.  Written
 // as assembly because the compiler puts a wait for ALL outstanding memory operations in front of every LDS read that
 // follows the builtin form; here the kernel places its own vmcnt waits (the instruction counts as one).
-__device__ __forceinline__ void lds_dma16(buf_desc_t desc, uint32_t dst, uint32_t off, uint32_t soff = 0) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(dst), "v"(off), "s"(desc), "s"(soff) : "memory");
+// NT = with the non-temporal hint (streams that are read once).
+template <bool NT = false>
+__device__ __forceinline__ void lds_dma16(buf_desc_t desc, uint32_t dst, uint32_t off) {
+  if constexpr (NT)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"s"(dst), "v"(off), "s"(desc) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(dst), "v"(off), "s"(desc) : "memory");
+}
+// the same with 4 bytes per lane
+template <bool NT = false>
+__device__ __forceinline__ void lds_dma4(buf_desc_t desc, uint32_t dst, uint32_t off) {
+  if constexpr (NT)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen nt lds" ::"s"(dst), "v"(off), "s"(desc) : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(dst), "v"(off), "s"(desc) : "memory");
 }
 // LDS byte address of a __shared__ object
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {

@@ -1,0 +1,96 @@
+// Tiles of the persistent kernels that fetch their operands by memory-to-LDS transfers, found from the slice sizes alone.
+#pragma once
+#include "gemm_common.h"
+#include "route_common.h"
+
+namespace tk {
+namespace {
+
+constexpr uint32_t kOutOfRange = 0x80000000u;  // byte offset that every buffer resource here (below 2 GiB) treats as out of range
+constexpr int kSliceRegs = kDmaSlices / 64;
+
+struct Tile {
+  int expert, off_m, start_m, eM, n_tile;
+};
+
+// Two lists: row blocks that are more than half full, then the short last blocks of the experts, which cost a fraction of a tile;
+// with the short ones in between, a workgroup's share was up to a whole tile longer than the next one's.  Of each list every
+// XCD (workgroup b runs on XCD b % 8) takes a contiguous part, walked side by side by its workgroups, the short tiles behind the
+// others: the workgroups without a tile in the last round of full ones begin with them.
+// Slice sizes and offsets stay in registers, lane l of register c holding slice c * 64 + l.
+template <int BM, int BN>
+struct TileList {
+  int sz[kSliceRegs], so[kSliceRegs];
+  int f_beg, f_len, s_beg, t_end, t_step, grid_n;
+
+  static __device__ __forceinline__ int n_full(int rows) { return (rows + BM / 2 - 1) / BM; }
+  static __device__ __forceinline__ int n_short(int rows) { return rows > n_full(rows) * BM ? 1 : 0; }
+
+  // returns this workgroup's first index (it has none if that is not below t_end; the following ones are t_step apart)
+  __device__ __forceinline__ int init(const GemmParams& p, int lane) {
+    int full = 0, brief = 0;
+#pragma unroll
+    for (int c = 0; c < kSliceRegs; ++c) {
+      const int e = c * 64 + lane;
+      sz[c] = so[c] = 0;
+      if (p.slice_sizes) {
+        if (e < p.n_slices) {
+          sz[c] = p.slice_sizes[e];
+          so[c] = p.slice_offs[e];
+        }
+      } else if (e == 0) {
+        sz[c] = p.M;
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < kSliceRegs; ++c) {
+      full += __builtin_amdgcn_readlane(wave_scan_i32(n_full(sz[c])), 63);
+      brief += __builtin_amdgcn_readlane(wave_scan_i32(n_short(sz[c])), 63);
+    }
+    grid_n = p.grid_n;
+    const int xcd = blockIdx.x & 7;
+    t_step = gridDim.x >> 3;
+    f_beg = (int)(((int64_t)full * grid_n * xcd) >> 3), f_len = (int)(((int64_t)full * grid_n * (xcd + 1)) >> 3) - f_beg;
+    s_beg = (int)(((int64_t)brief * grid_n * xcd) >> 3);
+    t_end = f_len + (int)(((int64_t)brief * grid_n * (xcd + 1)) >> 3) - s_beg;
+    return (int)(blockIdx.x >> 3);
+  }
+
+  __device__ __forceinline__ Tile locate(int t) const {
+    Tile r = {0, 0, 0, 0, 0};
+    const bool is_full = t < f_len;
+    const int g = is_full ? f_beg + t : s_beg + t - f_len;
+    const int q = g / grid_n;
+    int base = 0;
+    bool found = false;
+#pragma unroll
+    for (int c = 0; c < kSliceRegs; ++c) {
+      if (found) continue;
+      const int cnt = is_full ? n_full(sz[c]) : n_short(sz[c]);
+      const int inc = wave_scan_i32(cnt);
+      const int total = __builtin_amdgcn_readlane(inc, 63);
+      if (q < base + total) {
+        found = true;
+        const int l = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(base + inc > q));
+        const int nb = __builtin_amdgcn_readlane(cnt, l);
+        int i = g - (base + __builtin_amdgcn_readlane(inc, l) - nb) * grid_n;
+        r.expert = c * 64 + l;
+        r.eM = __builtin_amdgcn_readlane(sz[c], l);
+        r.start_m = __builtin_amdgcn_readlane(so[c], l);
+        // bands of eight row blocks, in a band column by column, so that the tiles an XCD has in hand share eight blocks of
+        // activations and a few of weights through its L2
+        const int band = i / (8 * grid_n);
+        const int bh = nb - band * 8 < 8 ? nb - band * 8 : 8;
+        i -= band * 8 * grid_n;
+        const int pn = i / bh;
+        r.n_tile = pn * BN;
+        r.off_m = (is_full ? band * 8 + i - pn * bh : n_full(r.eM)) * BM;
+      }
+      base += total;
+    }
+    return r;
+  }
+};
+
+}  // namespace
+}  // namespace tk

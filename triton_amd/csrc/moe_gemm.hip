@@ -217,6 +217,10 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
     if (d->n_slices > 1 && (d->w_stride_e < nfr * nst * 2048 || d->ws_stride_e < nfr * nst * 128)) return fail(TK_ERR_INVALID, "tk_moe_gemm: expert stride smaller than one tiled expert");
     p.w_stride_e = d->w_stride_e;
     p.w_nst = (int32_t)nst;
+    // row blocks of 32: the streaming kernel, unless something asks for the decode kernel's epilogue or fused combine (or x is too large
+    // for a buffer resource, or there are more slices than it has registers for)
+    if (d->block_m == 32 && p.x_bytes && (!d->slice_sizes || d->n_slices <= kDmaSlices) && !extras && d->combine_k <= 0 && !d->x_row_scale && !d->w_col_scale)
+      return gemm_launch_mxs(p, d->grid_m, swiglu, (int64_t)d->M <= (int64_t)d->n_slices * 16, st);
     if (d->block_m <= 32) return gemm_launch_mxd(p, d->block_m, d->grid_m, swiglu, st);
     if (mx_out_bf16) return gemm_launch_mxn_mx(p, d->block_m, d->grid_m, swiglu, st);
     return gemm_launch_mxn(p, d->block_m, d->grid_m, swiglu, st);

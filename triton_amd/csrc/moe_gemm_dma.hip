@@ -23,14 +23,10 @@
 // of 8 experts in e4m3: K 4096, N 28672, swiglu 1840 -> 1590 us (2.42 PFLOP/s), K 14336, N 4096 850 -> 805 us; 4096 rows of 16
 // experts in bf16, K 2048: N 4096 231 -> 94 us, N 2048 133 -> 51 us (the kernels before: weights in registers with one wave
 // per SIMD, and both operands through registers into LDS).
-#include "gemm_common.h"
-#include "route_common.h"
+#include "gemm_tiles.h"
 
 namespace tk {
 namespace {
-
-constexpr uint32_t kOutOfRange = 0x80000000u;
-constexpr int kSliceRegs = kDmaSlices / 64;
 
 template <bool LARGE>
 struct DmaCfg {
@@ -60,77 +56,10 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
   const int nst = (KB + 127) >> 7;
   const uint32_t lds0 = lds_addr(lds);
 
-  // ---- tiles ---------------------------------------------------------------------------------------------------------------------------------------
-  // Two lists: row blocks that are more than half full, then the short last blocks of the experts, which cost a fraction of a tile;
-  // with the short ones in between, a workgroup's share was up to a whole tile longer than the next one's.  Of each list every
-  // XCD (workgroup b runs on XCD b % 8) takes a contiguous part, walked side by side by its workgroups, the short tiles behind the
-  // others: the workgroups without a tile in the last round of full ones begin with them.
-  // Slice sizes and offsets stay in registers, lane l of register c holding slice c * 64 + l.
-  int sz[kSliceRegs], so[kSliceRegs];
-#pragma unroll
-  for (int c = 0; c < kSliceRegs; ++c) {
-    const int e = c * 64 + lane;
-    sz[c] = so[c] = 0;
-    if (p.slice_sizes) {
-      if (e < p.n_slices) {
-        sz[c] = p.slice_sizes[e];
-        so[c] = p.slice_offs[e];
-      }
-    } else if (e == 0) {
-      sz[c] = p.M;
-    }
-  }
-  auto n_full = [&](int rows) __attribute__((always_inline)) { return (rows + C::BM / 2 - 1) / C::BM; };
-  auto n_short = [&](int rows) __attribute__((always_inline)) { return rows > n_full(rows) * C::BM ? 1 : 0; };
-  int full = 0, brief = 0;
-#pragma unroll
-  for (int c = 0; c < kSliceRegs; ++c) {
-    full += __builtin_amdgcn_readlane(wave_scan_i32(n_full(sz[c])), 63);
-    brief += __builtin_amdgcn_readlane(wave_scan_i32(n_short(sz[c])), 63);
-  }
-  const int xcd = blockIdx.x & 7, t_step = gridDim.x >> 3;
-  const int f_beg = (int)(((int64_t)full * p.grid_n * xcd) >> 3), f_len = (int)(((int64_t)full * p.grid_n * (xcd + 1)) >> 3) - f_beg;
-  const int s_beg = (int)(((int64_t)brief * p.grid_n * xcd) >> 3), s_len = (int)(((int64_t)brief * p.grid_n * (xcd + 1)) >> 3) - s_beg;
-  const int t_end = f_len + s_len;
-  int tile = (int)(blockIdx.x >> 3);
+  TileList<C::BM, C::BN> tiles;
+  int tile = tiles.init(p, lane);
+  const int t_step = tiles.t_step, t_end = tiles.t_end;
   if (tile >= t_end) return;
-
-  struct Tile {
-    int expert, off_m, start_m, eM, n_tile;
-  };
-  auto locate = [&](int t) __attribute__((always_inline)) -> Tile {
-    Tile r = {0, 0, 0, 0, 0};
-    const bool is_full = t < f_len;
-    const int g = is_full ? f_beg + t : s_beg + t - f_len;
-    int q = g / p.grid_n, base = 0;
-    bool found = false;
-#pragma unroll
-    for (int c = 0; c < kSliceRegs; ++c) {
-      if (found) continue;
-      const int cnt = is_full ? n_full(sz[c]) : n_short(sz[c]);
-      const int inc = wave_scan_i32(cnt);
-      const int total = __builtin_amdgcn_readlane(inc, 63);
-      if (q < base + total) {
-        found = true;
-        const int l = (int)__builtin_ctzll(__builtin_amdgcn_ballot_w64(base + inc > q));
-        const int nb = __builtin_amdgcn_readlane(cnt, l);
-        int i = g - (base + __builtin_amdgcn_readlane(inc, l) - nb) * p.grid_n;
-        r.expert = c * 64 + l;
-        r.eM = __builtin_amdgcn_readlane(sz[c], l);
-        r.start_m = __builtin_amdgcn_readlane(so[c], l);
-        // bands of eight row blocks, in a band column by column, so that the tiles an XCD has in hand share eight blocks of
-        // activations and a few of weights through its L2
-        const int band = i / (8 * p.grid_n);
-        const int bh = nb - band * 8 < 8 ? nb - band * 8 : 8;
-        i -= band * 8 * p.grid_n;
-        const int pn = i / bh;
-        r.n_tile = pn * C::BN;
-        r.off_m = (is_full ? band * 8 + i - pn * bh : n_full(r.eM)) * C::BM;
-      }
-      base += total;
-    }
-    return r;
-  };
 
   // ---- transfer side ------------------------------------------------------------------------------------------------------------------------------
   // transfer i of an operand: rows i * 8 .. + 7, lane -> row lane / 8, LDS position lane % 8, i.e. piece (lane % 8) ^ (row >> 1 & 7);
@@ -198,7 +127,7 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
 
   // ---- the rings: one cursor, two stages ahead of the multiplication --------------------------------------------------------------------------
   constexpr uint32_t kAEnd = C::ABUFS * C::ABYTES, kBEnd = kAEnd + C::BBUFS * C::BBYTES;
-  Tile cur = locate(tile);
+  Tile cur = tiles.locate(tile);
   aim(cur);
   uint32_t aw = 0, bw = kAEnd;  // buffers the next transfers fill
   int fs = 0;                   // next stage to fetch
@@ -211,7 +140,7 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
       fs = 0;
       f_tile += t_step;
       more = more && f_tile < t_end;
-      if (more) aim(locate(f_tile));
+      if (more) aim(tiles.locate(f_tile));
     }
   };
 
@@ -347,7 +276,7 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
                                                              cur.n_tile + C::BN <= p.N, mw, lr, h);
     tile += t_step;
     if (tile >= t_end) break;
-    cur = locate(tile);
+    cur = tiles.locate(tile);
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no transfer into this workgroup's LDS is left behind
 }

@@ -466,6 +466,15 @@ def _dma_block_m(rows: int, row_bytes: int, N: int, n_slices: int) -> int:
     return 256 if per_slice >= 192 or tiles >= 192 or row_bytes >= 8192 else 128
 
 
+def _mxfp4_block_m(rows: int, n_slices: int, default: int) -> int:
+    """Row blocks for tiled MXFP4 weights with more routed rows than the decode kernel is made for.  32 = the streaming kernel, faster than
+    the decode kernel's 16-row blocks from 160 rows on (128 slices, K 2880, N 5760: 300 tokens 210 against 232 us, 32 slices, 200
+    tokens 28 against 57 us) and than the prefill kernel's 64-row blocks up to about 20 rows per slice (18: 245 against 258 us,
+    31: 331 against 290 us); those give way to the larger ones at about 56 (47: 340 against 372 us, 62: 410 against 399 us)."""
+    per_slice = rows // max(n_slices, 1)
+    return 32 if per_slice <= 20 else 64 if per_slice <= 56 else max(default, 128)
+
+
 def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
            b_ragged_metadata: RaggedTensorMetadata | None = None, gather_indx: torch.Tensor | None = None,
            scatter_indx: torch.Tensor | None = None, precision_config: PrecisionConfig | None = None,
@@ -761,8 +770,12 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
     elif tiled:
         if extras:
             block_m = min(block_m, 32)  # the decode kernel carries the shared epilogue; the prefill kernels do not take these options
-        elif block_m == 128 and forced is None and is_ragged and M <= 144 * n_slices:
-            block_m = 256  # about 128 rows per expert: one tile per expert, the weights are read once
+        elif forced is None and is_ragged:
+            if (M > 256 and a_rows * a_stride < 1 << 30 and n_slices <= 256 and a_ts is None and b_ts is None
+                    and a_ragged_metadata.expected_slice_size is None):
+                block_m = _mxfp4_block_m(M, n_slices, block_m)
+            if block_m == 128 and M <= 144 * n_slices:
+                block_m = 256  # about 128 rows per expert: one tile per expert, the weights are read once
     elif w_dtype in (_BF16, _F16):
         # (the conditions of the memory-to-LDS kernel: x and an expert's weights within 2 GiB, up to 256 slices)
         dma = a_rows * a_stride < 1 << 30 and n_slices <= 256 and N * w.stride(-1) < 1 << 30
@@ -820,7 +833,9 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
     # launch of its own at the gpt-oss shape)
     can_combine = (_combine_k and tiled and not extras and not mx_act and act == nt.TK_ACT_NONE and scatter_indx is not None
                    and y_rows % _combine_k == 0 and a_dtype == _BF16)
-    if can_combine and block_m <= 32:
+    if can_combine and block_m == 32 and forced is None:
+        can_combine = False  # the streaming kernel has no combine
+    elif can_combine and block_m <= 32:
         # decode kernel: the wave that completes a token's rows last sums them (arrival counters per token and fragment)
         can_combine = (y_rows // _combine_k) * ((N + 31) // 32) <= _COMBINE_COUNTER_WORDS
     elif can_combine:
