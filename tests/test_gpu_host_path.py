@@ -1,0 +1,161 @@
+"""The native host path against the general Python path, bit for bit, over the forms of a call that it serves and at its edges: both fill
+a descriptor for the same kernels, so values, shapes, strides and types have to agree; and calls it has to leave to the general path."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _same(a, b):
+    if isinstance(a, torch.Tensor):
+        assert a.shape == b.shape and a.dtype == b.dtype and a.stride() == b.stride() and a._version == b._version == 0
+        assert torch.equal(a.contiguous().view(torch.uint8), b.contiguous().view(torch.uint8))
+    elif isinstance(a, (list, tuple)):
+        assert type(a) is type(b) and len(a) == len(b)
+        for x, y in zip(a, b):
+            _same(x, y)
+    else:
+        assert a == b and type(a) is type(b)
+
+
+def _both(monkeypatch, f, served=True):
+    """f() through the native path and through the general one."""
+    from triton_amd import _native as nt
+    real, seen = nt.host(), []
+
+    class Watch:
+        def __getattr__(self, name):
+            def call(*args):
+                r = getattr(real, name)(*args)
+                seen.append((name, r is not None))
+                return r
+            return call
+
+    with monkeypatch.context() as m:
+        m.setattr(nt, "host", lambda: Watch())
+        fast = f()
+    assert seen and all(ok == served for _, ok in seen), seen
+    with monkeypatch.context() as m:
+        m.setattr(nt, "host", lambda: None)
+        slow = f()
+    _same(fast, slow)
+    return fast
+
+
+@pytest.mark.parametrize("tokens, e, k", [(1, 1, 1), (1, 128, 4), (3, 20, 2), (300, 128, 8), (33, 700, 32)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_routing(device, monkeypatch, tokens, e, k, dtype):
+    from triton_amd.legacy import routing
+    logits = torch.randn((tokens, e), generator=torch.Generator().manual_seed(e)).to(dtype).to(device)
+    for softmax in (True, False):
+        rd, gather, scatter = routing(logits, k, softmax)
+        from triton_amd import _native as nt
+        with monkeypatch.context() as m:
+            m.setattr(nt, "host", lambda: None)
+            rd2, gather2, scatter2 = routing(logits, k, softmax)
+        md, md2 = rd.expt_data, rd2.expt_data
+        _same([gather.src_indx, gather.dst_indx, scatter.src_indx, scatter.dst_indx], [gather2.src_indx, gather2.dst_indx, scatter2.src_indx, scatter2.dst_indx])
+        _same([rd.gate_scal, rd.expt_hist, rd.token_indx, rd.expt_indx, rd.gate_vals, rd.all_rows_live, rd.n_expts_tot, rd.n_expts_act],
+              [rd2.gate_scal, rd2.expt_hist, rd2.token_indx, rd2.expt_indx, rd2.gate_vals, rd2.all_rows_live, rd2.n_expts_tot, rd2.n_expts_act])
+        _same([md.slice_offs, md.block_offs_data, md.block_schedule_data, md.n_slices], [md2.slice_offs, md2.block_offs_data, md2.block_schedule_data, md2.n_slices])
+    with pytest.raises(ValueError):
+        routing(logits, 3)
+
+
+def _weights(kind, e, k, n, g, device):
+    from triton_amd.numerics_details.mxfp import downcast_to_mxfp
+    from triton_amd.tensor import FP4, convert_layout, wrap_torch_tensor
+    from triton_amd.tensor_details import layout as L
+    w = (torch.randn((e, n, k), generator=g) * 0.1).to(device)
+    if kind in ("bf16", "fp16"):
+        return w.to(torch.bfloat16 if kind == "bf16" else torch.float16).transpose(1, 2), None
+    if kind == "fp8":
+        return convert_layout(wrap_torch_tensor(w.to(torch.float8_e4m3fn).transpose(1, 2)), L.make_default_matmul_fp8_w_layout()), None
+    q, s = downcast_to_mxfp(w.to(torch.bfloat16).transpose(1, 2), torch.uint8, axis=1)
+    return (convert_layout(wrap_torch_tensor(q, dtype=FP4), L.make_default_matmul_mxfp4_w_layout(mx_axis=1)),
+            convert_layout(wrap_torch_tensor(s), L.make_default_matmul_mxfp4_w_scale_layout(mx_axis=1)))
+
+
+@pytest.mark.parametrize("kind", ["bf16", "fp16", "fp8", "mxfp4", "mxfp8", "mxfp8_out"])
+@pytest.mark.parametrize("tokens", [1, 40, 200, 500, 1200])
+def test_layer_gemms(device, monkeypatch, kind, tokens):
+    """16 experts, 2 choices: 2 to 2400 rows, so that every row block is chosen; with activation and gather, scatter and combine."""
+    import triton_amd.matmul as mm
+    from triton_amd.legacy import matmul_ogs, routing
+    from triton_amd.numerics_details.mxfp import downcast_to_mxfp, quantize_mxfp8_fn
+    from triton_amd.numerics_details.rowwise_fp8 import quantize_fp8_rowwise
+    from triton_amd.swiglu import swiglu_fn
+    e, k, d, f = 16, 2, 256, 320
+    g = torch.Generator().manual_seed(tokens)
+    x = torch.randn((tokens, d), generator=g).to(torch.float16 if kind == "fp16" else torch.bfloat16).to(device)
+    rd, gather, scatter = routing(torch.randn((tokens, e), generator=g).to(device), k)
+    w1, s1 = _weights(kind, e, d, 2 * f, g, device)
+    w2, s2 = _weights(kind, e, f, d, g, device)
+    b1, b2 = torch.randn((e, 2 * f), generator=g).to(device), torch.randn((e, d), generator=g).to(torch.bfloat16).to(device)
+    act = mm.FusedActivation(mm.FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0))
+    P, bf16, e4m3 = mm.PrecisionConfig, torch.bfloat16, torch.float8_e4m3fn
+    epi = None
+    if kind == "fp8":
+        x, sx = quantize_fp8_rowwise(x)
+        col = torch.rand((e, 2 * f), generator=g).to(device)
+        pc1 = P(a_mx_tensor_scale=sx, b_mx_tensor_scale=col, out_dtype=bf16)
+    elif kind.startswith("mxfp8"):
+        x, sx = downcast_to_mxfp(x, e4m3, axis=-1)
+        pc1 = P(a_mx_scale=sx, b_mx_scale=s1, out_dtype=bf16)
+        if kind == "mxfp8_out":
+            pc1.c_mx_scale, pc1.out_dtype = torch.zeros((tokens * k, f // 32), dtype=torch.uint8, device=device), e4m3
+            epi = mm.Epilogue(mm.FnSpecs(mm.FnName.QUANTIZE_MXFP8.name, quantize_mxfp8_fn, (), ()), (), (), effective_itemsize=1.0)
+    else:
+        pc1 = P(b_mx_scale=s1) if s1 is not None else None
+    h = _both(monkeypatch, lambda: matmul_ogs(x, w1, b1, rd, gather_indx=gather, precision_config=pc1, fused_activation=act, epilogue=epi))
+    if kind == "fp8":
+        h, sh = _both(monkeypatch, lambda: quantize_fp8_rowwise(h))
+        pc2 = P(a_mx_tensor_scale=sh, out_dtype=bf16)
+    elif kind == "mxfp8":
+        h, sh = _both(monkeypatch, lambda: downcast_to_mxfp(h, e4m3, axis=-1))
+        pc2 = P(a_mx_scale=sh, b_mx_scale=s2, out_dtype=bf16)
+    elif kind == "mxfp8_out":
+        pc2 = P(a_mx_scale=pc1.c_mx_scale, b_mx_scale=s2, out_dtype=bf16)
+    else:
+        pc2 = P(b_mx_scale=s2) if s2 is not None else P()
+    gam = rd.gate_scal
+    _both(monkeypatch, lambda: matmul_ogs(h, w2, b2, rd, scatter_indx=scatter, precision_config=pc2, gammas=gam))
+    # left to the general path: operands and options that are not of the plain form
+    xt = x.t().contiguous().t()
+    _both(monkeypatch, lambda: matmul_ogs(xt, w1, b1, rd, gather_indx=gather, precision_config=pc1, fused_activation=act, epilogue=epi), served=tokens == 1)
+    with pytest.raises(AssertionError):
+        matmul_ogs(x[:, :-32], w1, b1, rd, gather_indx=gather, precision_config=P(b_mx_scale=s1, out_dtype=bf16), fused_activation=act)
+
+
+@pytest.mark.parametrize("shape, axis", [((1, 32), 1), ((3, 64), -1), ((64, 5), 0), ((2, 96, 7), 1), ((2, 96, 64), -2), ((1, 32, 1), 1), ((4, 3, 32), 2)])
+@pytest.mark.parametrize("to", [torch.uint8, torch.float8_e4m3fn, torch.float8_e5m2])
+def test_mx(device, monkeypatch, shape, axis, to):
+    from triton_amd.numerics_details.mxfp import downcast_to_mxfp, upcast_from_mxfp
+    x = torch.randn(shape, generator=torch.Generator().manual_seed(sum(shape))).to(torch.bfloat16).to(device)
+    q, s = _both(monkeypatch, lambda: downcast_to_mxfp(x, to, axis=axis))
+    _both(monkeypatch, lambda: upcast_from_mxfp(q, s, torch.float16, axis=axis))
+
+
+@pytest.mark.parametrize("m, n, sizes", [(8, 40, [3, 0, 17]), (64, 64, [0, 4])])
+def test_ragged_k(device, monkeypatch, m, n, sizes):
+    from triton_amd.matmul import matmul
+    from triton_amd.tensor import make_ragged_tensor_metadata
+    g, r = torch.Generator().manual_seed(m), sum(sizes)
+    a, b = torch.randn((r, m), generator=g).to(torch.bfloat16).to(device), torch.randn((r, n), generator=g).to(torch.bfloat16).to(device)
+    md = make_ragged_tensor_metadata(torch.tensor(sizes, dtype=torch.int32, device=device), r)
+    _both(monkeypatch, lambda: matmul(a.t(), b, None, a_ragged_metadata=md, b_ragged_metadata=md))
+
+
+@pytest.mark.parametrize("tokens, skip_bias", [(8, False), (61, True)])
+def test_decode_layer(device, monkeypatch, tokens, skip_bias):
+    import triton_amd.matmul as mm
+    from triton_amd.moe_decode import moe_mlp
+    from triton_amd.swiglu import swiglu_fn
+    e, k, d, f = 32, 4, 256, 320
+    g = torch.Generator().manual_seed(tokens)
+    (w1, s1), (w2, s2) = _weights("mxfp4", e, d, 2 * f, g, device), _weights("mxfp4", e, f, d, g, device)
+    x, logits = torch.randn((tokens, d), generator=g).to(torch.bfloat16).to(device), torch.randn((tokens, e), generator=g).to(device)
+    b1 = None if skip_bias else torch.randn((e, 2 * f), generator=g).to(device)
+    act = mm.FusedActivation(mm.FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0))
+    pc1, pc2 = mm.PrecisionConfig(b_mx_scale=s1), mm.PrecisionConfig(b_mx_scale=s2)
+    _both(monkeypatch, lambda: moe_mlp(x, logits, k, w1, b1, w2, None, pc1, pc2, act))

@@ -1,6 +1,7 @@
-"""ctypes binding of `libtriton_amd.so` (the C ABI declared in include/triton_amd.h).
+"""ctypes binding of `libtriton_amd.so` (the C ABI declared in include/triton_amd.h) and `_host.so`, the native half of the
+host path.
 
-The library is loaded lazily on first use and a missing library is a hard error: there is no
+The libraries are loaded lazily on first use and a missing one is a hard error: there is no
 fallback implementation.
 """
 from __future__ import annotations
@@ -149,6 +150,49 @@ def lib():
     return _lib
 
 
+_host = None
+_HOST_ENTRIES = ("tk_moe_gemm", "tk_route", "tk_route_workspace_bytes", "tk_reduce_mid", "tk_quant_fp8_rows", "tk_mx_downcast",
+                 "tk_mx_upcast", "tk_ragged_k_gemm", "tk_moe_decode_layer")
+
+
+def _load_host():
+    global _host
+    handle = lib()
+    path = os.path.join(HERE, "_host.so")
+    if not os.path.exists(path):
+        raise NativeLibraryMissing(f"{path} not found: build it with `python -m triton_amd.build`. There is no fallback implementation.")
+    from . import _host as module, legacy, matmul, moe_decode
+    from .tensor import FP4, Tensor
+    from .tensor_details.layout_details.gfx950_mx import GFX950FP8ValueLayout, GFX950MXScaleLayout, GFX950MXValueLayout
+    from .tensor_details.ragged_tensor import RaggedTensorMetadata
+    with _lock:
+        if _host is None:
+            table = {name: _c.cast(getattr(handle, name), _ptr).value for name in _HOST_ENTRIES}
+            table.update(check=check, raw_stream=_raw_stream, current_device=_current_device, tile_counters=matmul._tile_counters,
+                         combine_counters=matmul._combine_counters, decode_workspace=moe_decode._workspace, tensor_type=Tensor,
+                         mx_value=GFX950MXValueLayout, mx_scale=GFX950MXScaleLayout, fp8_value=GFX950FP8ValueLayout, fp4=FP4,
+                         metadata_type=RaggedTensorMetadata, routing_type=legacy.RoutingData, gather_type=legacy.GatherIndx,
+                         scatter_type=legacy.ScatterIndx, default_flex=matmul._DEFAULT_FLEX, no_activation=matmul._NO_ACTIVATION,
+                         no_epilogue=matmul._NO_EPILOGUE)
+            module.bind(table)
+            _host = module
+
+
+def host():
+    """The native host path, bound to the loaded library.  None where `lib` hands out something else (an object that watches
+    the calls, say): then every call is made through that."""
+    if _host is None:
+        _load_host()
+    return _host if lib() is _lib else None
+
+
+def rules():
+    """The module that holds the row-block rules, whatever `lib` hands out."""
+    if _host is None:
+        _load_host()
+    return _host
+
+
 def last_error() -> str:
     return lib().tk_last_error().decode("utf-8", "replace")
 
@@ -165,15 +209,15 @@ def check(status: int, what: str = ""):
     raise RuntimeError(msg)
 
 
-_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)  # a fraction of a microsecond instead of several
+if _raw_stream is None:
+    def _raw_stream(idx):
+        return torch.cuda.current_stream(idx).cuda_stream
 
 
 def stream_ptr(device=None) -> int:
     """The current PyTorch HIP stream of `device` as a raw hipStream_t."""
-    if _raw_stream is not None:  # the direct binding: a fraction of a microsecond instead of several
-        idx = device.index if isinstance(device, torch.device) and device.index is not None else torch.cuda.current_device()
-        return _raw_stream(idx)
-    return torch.cuda.current_stream(device).cuda_stream
+    return _raw_stream(device.index if isinstance(device, torch.device) and device.index is not None else torch.cuda.current_device())
 
 
 _current_device = getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device

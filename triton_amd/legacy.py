@@ -8,7 +8,9 @@ python/triton_kernels/tests/test_distributed.py:203-220 composes them:
     y        = matmul(x, w, bias, metadata, gather_indx=gather, scatter_indx=scatter, gammas=...)
     out      = reduce(y.view(T, k, -1), dim=1)                   when scattering
 
-`routing` obtains all of it from ONE fused routing pass (three kernel launches).
+`routing` obtains all of it from ONE fused routing pass (three kernel launches).  The router's own choice for every row
+is served by the native host path, where the integer results are views of one allocation and the bitmatrix, which
+`RoutingData` does not carry, is not made (36 -> 8 us of host time).
 """
 from __future__ import annotations
 
@@ -18,10 +20,10 @@ import torch
 
 from . import _native as nt
 from .matmul import FusedActivation, PrecisionConfig, matmul
-from .reduce import _reduce_forward
+from .reduce import combine_rows
 from .tensor import RaggedTensorMetadata
 from .tensor_details.ragged_tensor import _alloc
-from .topk import _topk_route, check_topk
+from .topk import _topk_route
 
 
 @dataclass
@@ -53,10 +55,13 @@ class RoutingData:
 
 def routing(logits, n_expts_act, apply_softmax: bool = True, expt_indx=None, n_rows=None):
     """Router for a mixture-of-experts layer: returns `(RoutingData, GatherIndx, ScatterIndx)`."""
+    if expt_indx is None and n_rows is None:
+        host = nt.host()
+        r = host.route(logits, n_expts_act, apply_softmax) if host is not None else None
+        if r is not None:
+            return r
     T, E = logits.shape
     k = n_expts_act
-    if expt_indx is None and n_rows is None and T > 0 and isinstance(logits, torch.Tensor):
-        return _routing_of_logits(logits, T, E, k, apply_softmax)
     ragged = _alloc(E, T * k, logits.device)
     vals, indx, _mask, r = _topk_route(logits, k, apply_softmax, expt_indx, n_rows, want_meta=True, want_extras=True,
                                        ragged=ragged)
@@ -67,43 +72,6 @@ def routing(logits, n_expts_act, apply_softmax: bool = True, expt_indx=None, n_r
                         token_indx=r["gather_indx"], expt_indx=indx, gate_vals=vals,
                         all_rows_live=expt_indx is None and n_rows is None)
     return rdata, GatherIndx(src_indx=col, dst_indx=row), ScatterIndx(src_indx=row, dst_indx=col)
-
-
-def _routing_of_logits(logits, T: int, E: int, k: int, apply_softmax: bool):
-    """`routing` with the router's own choice for every row: the integer results are views of one allocation, and the
-    bitmatrix, which `RoutingData` does not carry, is not made."""
-    nt.require_gpu(logits, "logits")
-    if logits.stride(1) != 1:
-        logits = logits.contiguous()
-    check_topk(k, E)
-    device, dtype, R = logits.device, logits.dtype, T * k
-    lib = nt.lib()
-    width = RaggedTensorMetadata.max_n_blocks(E, R)
-    # [E] histogram, the two permutations, [R] gather index, [E + 1] row offsets, [5, E + 1] block offsets, [5, width] schedules
-    # (the schedules' readers load single words), and the kernels' scratch, which starts on 16 bytes
-    sizes = [E, R, R, R, E + 1, 5 * (E + 1), 5 * width]
-    used = sum(sizes)
-    pad = -used & 3
-    words = (max(1, lib.tk_route_workspace_bytes(T, E)) + 3) // 4
-    buf = torch.empty(used + pad + words, dtype=torch.int32, device=device)
-    hist, col, row, gather, slice_offs, block_offs, sched, _ws = buf.split([*sizes, pad + words])
-    block_offs, sched = block_offs.view(5, E + 1), sched.view(5, width)
-    vals, indx = torch.empty((T, k), dtype=dtype, device=device), torch.empty((T, k), dtype=torch.int16, device=device)
-    gammas = torch.empty(R, dtype=dtype, device=device)
-    base = buf.data_ptr()
-    d = nt.RouteDesc()
-    d.logits, d.logits_dtype, d.logits_stride_m = logits.data_ptr(), nt.TORCH_TO_TK[dtype], logits.stride(0)
-    d.n_tokens, d.n_rows, d.n_experts, d.k, d.apply_softmax = T, -1, E, k, int(bool(apply_softmax))
-    d.vals, d.indx, d.indx_dtype, d.gammas = vals.data_ptr(), indx.data_ptr(), nt.TK_I16, gammas.data_ptr()
-    d.col_sum, at = base, base + 4 * E
-    d.col_sorted_indx, d.row_sorted_indx, d.gather_indx = at, at + 4 * R, at + 8 * R
-    at += 12 * R
-    d.slice_offs, d.block_offs, d.block_offs_stride = at, at + 4 * (E + 1), E + 1
-    d.block_schedule, d.block_schedule_stride, d.max_n_blocks = at + 24 * (E + 1), width, width
-    d.workspace = base + 4 * (used + pad)
-    nt.submit(lib.tk_route, d, device)
-    rdata = RoutingData(gammas, hist, E, k, RaggedTensorMetadata(hist, slice_offs, block_offs, sched), gather, indx, vals, True)
-    return rdata, GatherIndx(col, row), ScatterIndx(row, col)
 
 
 def matmul_ogs(x, w, bias, routing_data: RoutingData | None = None, gather_indx: GatherIndx | None = None,
@@ -133,7 +101,7 @@ def matmul_ogs(x, w, bias, routing_data: RoutingData | None = None, gather_indx:
     combined = getattr(y, "_tk_combined", None)
     if combined is not None:  # decode shapes: the GEMM's last wave per token has already summed its k rows
         return combined
-    return _reduce_forward(y.view(y.shape[0] // k, k, y.shape[-1]), None, None, None)[0]
+    return combine_rows(y, k)
 
 
 from .torch_twins import matmul_ogs_torch, routing_torch  # noqa: E402,F401  (reference twins)

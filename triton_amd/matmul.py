@@ -452,29 +452,6 @@ def _matmul_ragged_k(a, b, bias, a_ragged_metadata, b_ragged_metadata, gather_in
     return c
 
 
-def _dma_block_m(rows: int, row_bytes: int, N: int, n_slices: int) -> int:
-    """Row blocks of the memory-to-LDS kernel: 256 (256 x 256 tiles, one workgroup per CU) or 128 (128 x 128, two per CU).  The large
-    tile moves half the operand bytes per product, the small one fills the chip with fewer rows.  Measured on 8 to 32 slices: up to
-    64 rows per slice the small tile is as fast or faster (e4m3, 8 rows, K 4096: 174 against 183 us), from 192 on the large one
-    is (e4m3, 256 rows: 350 against 456 us); in between it depends on the large tiles there are for the 256 CUs (bf16, 128
-    rows, K 2048: N 4096, 256 tiles, 56 against 72 us; N 2048, 128 tiles, 44 against 38 us) and, with fewer, on the length
-    of a row, which a tile's start and end have to be paid from (e4m3, 128 tiles, K 14336: 168 against 214 us)."""
-    per_slice = rows // max(n_slices, 1)
-    if per_slice <= 64:
-        return 128
-    tiles = n_slices * ((per_slice + 255) // 256) * ((N + 255) // 256)
-    return 256 if per_slice >= 192 or tiles >= 192 or row_bytes >= 8192 else 128
-
-
-def _mxfp4_block_m(rows: int, n_slices: int, default: int) -> int:
-    """Row blocks for tiled MXFP4 weights with more routed rows than the decode kernel is made for.  32 = the streaming kernel, faster than
-    the decode kernel's 16-row blocks from 160 rows on (128 slices, K 2880, N 5760: 300 tokens 210 against 232 us, 32 slices, 200
-    tokens 28 against 57 us) and than the prefill kernel's 64-row blocks up to about 20 rows per slice (18: 245 against 258 us,
-    31: 331 against 290 us); those give way to the larger ones at about 56 (47: 340 against 372 us, 62: 410 against 399 us)."""
-    per_slice = rows // max(n_slices, 1)
-    return 32 if per_slice <= 20 else 64 if per_slice <= 56 else max(default, 128)
-
-
 def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
            b_ragged_metadata: RaggedTensorMetadata | None = None, gather_indx: torch.Tensor | None = None,
            scatter_indx: torch.Tensor | None = None, precision_config: PrecisionConfig | None = None,
@@ -492,6 +469,18 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
     the returned tensor as `._tk_combined` ([tokens, N]) and the caller skips its `reduce`.  The caller vouches that
     EVERY token has exactly k routed rows: a token with fewer leaves its arrival counter non-zero for the next launch.
     """
+    if betas is None and out_alpha is None and c is None and fused_comm is None and c_acc_in is None and a_ragged_metadata is not None:
+        # (`host` is the same steps in native code for the plain forms of a call; None = not one of those)
+        host, y = nt.host(), None
+        if b_ragged_metadata is not None:
+            if (host is not None and bias is None and gather_indx is None and scatter_indx is None and precision_config is None
+                    and gammas is None and fused_activation is None and epilogue is None):
+                y = host.ragged_k(a, b, a_ragged_metadata, b_ragged_metadata)
+        elif host is not None and not _STATIC_TILES and unconstrained():
+            y = host.gemm(a, b, bias, a_ragged_metadata, gather_indx, scatter_indx, precision_config, gammas, fused_activation,
+                          epilogue, _combine_k, _get_idle_sms())
+        if y is not None:
+            return y
     if b_ragged_metadata is not None:
         return _matmul_ragged_k(a, b, bias, a_ragged_metadata, b_ragged_metadata, gather_indx, scatter_indx, precision_config,
                                 betas, gammas, out_alpha, c, fused_comm, fused_activation, epilogue, c_acc_in)
@@ -763,7 +752,7 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
         d.gammas, d.gammas_dtype = g.data_ptr(), nt.TORCH_TO_TK[g.dtype]
         keep.append(g)
     if tiled_fp8:
-        block_m = forced if forced in (128, 256) else 128 if forced is not None else _dma_block_m(M, K, N, n_slices)
+        block_m = forced if forced in (128, 256) else 128 if forced is not None else nt.rules().dma_block_m(M, K, N, n_slices)
     elif mx_act or (tiled and mx_out_fused):
         # the tile shapes that take MXFP8 activations / have an MX-output epilogue
         block_m = 256 if (forced == 256 or (forced is None and is_ragged and M <= 144 * n_slices)) else 128
@@ -773,7 +762,7 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
         elif forced is None and is_ragged:
             if (M > 256 and a_rows * a_stride < 1 << 30 and n_slices <= 256 and a_ts is None and b_ts is None
                     and a_ragged_metadata.expected_slice_size is None):
-                block_m = _mxfp4_block_m(M, n_slices, block_m)
+                block_m = nt.rules().mxfp4_block_m(M, n_slices, block_m)
             if block_m == 128 and M <= 144 * n_slices:
                 block_m = 256  # about 128 rows per expert: one tile per expert, the weights are read once
     elif w_dtype in (_BF16, _F16):
@@ -782,7 +771,7 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
         if not dma:
             block_m = min(block_m, 128)
         elif forced is None and block_m > 16:
-            block_m = _dma_block_m(M, 2 * K, N, n_slices)
+            block_m = nt.rules().dma_block_m(M, 2 * K, N, n_slices)
     elif block_m == 256:
         block_m = 128
     if is_ragged:

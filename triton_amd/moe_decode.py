@@ -17,6 +17,7 @@ from __future__ import annotations
 import torch
 
 from . import _native as nt
+from .legacy import matmul_ogs, routing
 from .matmul import FusedActivation, PrecisionConfig, _flex_out_is_trivial
 from .tensor import FP4, Tensor
 from .tensor_details.layout_details.gfx950_mx import GFX950MXScaleLayout, GFX950MXValueLayout
@@ -160,9 +161,16 @@ def moe_mlp(x, logits, n_expts_act, w1, b1, w2, b2, pc1: PrecisionConfig, pc2: P
     call: one kernel launch at decode sizes, the three calls otherwise.  Returns `[tokens, d_model]`."""
     # (with fewer than 8 routed rows the launch's fixed part, every workgroup routing the batch before its first weight
     # byte, outweighs the two launch boundaries it saves: 41 against 29 us for one token at the gpt-oss shape)
-    if logits.shape[0] * n_expts_act >= MIN_ROWS and one_launch_reason(x, logits, n_expts_act, w1, b1, w2, b2, pc1, pc2, fused_activation) is None:
-        return moe_decode_layer(x, logits, n_expts_act, w1, b1, w2, b2, pc1, pc2, fused_activation)
-    from .legacy import matmul_ogs, routing
+    rows = logits.shape[0] * n_expts_act
+    if MIN_ROWS <= rows <= MAX_ROWS:
+        host = nt.host()
+        out = None
+        if host is not None:
+            out = host.decode_layer(x, logits, n_expts_act, w1, b1, w2, b2, pc1, pc2, fused_activation, MAX_ROWS, MAX_EXPERTS, MAX_DIM)
+        if out is None and one_launch_reason(x, logits, n_expts_act, w1, b1, w2, b2, pc1, pc2, fused_activation) is None:
+            out = moe_decode_layer(x, logits, n_expts_act, w1, b1, w2, b2, pc1, pc2, fused_activation)
+        if out is not None:
+            return out
     rdata, gather, scatter = routing(logits, n_expts_act)
     h = matmul_ogs(x, w1, b1, rdata, gather_indx=gather, precision_config=pc1, fused_activation=fused_activation)
     return matmul_ogs(h, w2, b2, rdata, scatter_indx=scatter, precision_config=pc2, gammas=rdata.gate_scal)

@@ -54,6 +54,7 @@ def get_max_quant_val(dtype: torch.dtype):
 
 
 _KIND = {FP4: nt.TK_E2M1, FP8_E4M3FN: nt.TK_E4M3, FP8_E5M2: nt.TK_E5M2}
+_KIND_OF_TORCH = {torch.uint8: nt.TK_E2M1, torch.float8_e4m3fn: nt.TK_E4M3, torch.float8_e5m2: nt.TK_E5M2}
 _FLOAT_SRC = {torch.float32: nt.TK_F32, torch.bfloat16: nt.TK_BF16, torch.float16: nt.TK_F16}
 
 
@@ -93,6 +94,12 @@ def downcast_to_mxfp(x, out_dtype, axis: int, scale_dtype: torch.dtype = torch.u
     """Quantises `x` along `axis` in blocks of 32.  Returns `(values, scales)` torch tensors whose
     unit-stride dimension is `axis`; `torch.uint8` output means e2m1 packed two per byte."""
     if not isinstance(x, Tensor):
+        kind = _KIND_OF_TORCH.get(out_dtype)
+        if kind is not None and scale_dtype is torch.uint8 and microblock_size == 32:
+            host = nt.host()
+            r = host.mx_downcast(x, kind, axis, DEQUANT_SCALE_ROUNDING_MODE.value) if host is not None else None
+            if r is not None:
+                return r
         x = wrap_torch_tensor(x)
     if scale_dtype != torch.uint8:
         if scale_dtype == torch.float8_e4m3fn:
@@ -136,6 +143,11 @@ def downcast_to_mxfp(x, out_dtype, axis: int, scale_dtype: torch.dtype = torch.u
 def upcast_from_mxfp(tensor: torch.Tensor, scale: torch.Tensor, target_dtype: torch.dtype, axis: int,
                      tensor_scale: torch.Tensor | None = None):
     """Dequantises along `axis`; the result is a standard-contiguous tensor of `target_dtype`."""
+    if tensor_scale is None:
+        host = nt.host()
+        out = host.mx_upcast(tensor, scale, target_dtype, axis) if host is not None else None
+        if out is not None:
+            return out
     ndim = tensor.ndim
     assert -ndim <= axis < ndim, f"Invalid axis {axis=}"
     axis = axis % ndim
@@ -163,7 +175,7 @@ def upcast_from_mxfp(tensor: torch.Tensor, scale: torch.Tensor, target_dtype: to
         outer = _prod(out_shape[:axis])
         inner = _prod(out_shape[axis + 1:])
         inner_last = out_shape[-1] if axis < ndim - 1 else 1
-        kind = {torch.uint8: nt.TK_E2M1, torch.float8_e4m3fn: nt.TK_E4M3, torch.float8_e5m2: nt.TK_E5M2}[tensor.dtype]
+        kind = _KIND_OF_TORCH[tensor.dtype]
         with nt.on_device(tensor.device):
             nt.check(
                 nt.lib().tk_mx_upcast(v.data_ptr(), s.data_ptr(), kind, outer, L, inner, inner_last, out.data_ptr(),

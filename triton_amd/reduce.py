@@ -107,6 +107,13 @@ def reduce(x: torch.Tensor, dim: int, mask: Optional[torch.Tensor] = None, scale
     return _reduce_forward(x, mask, scale, y)
 
 
+def combine_rows(y, k: int):
+    """`reduce(y.view(T, k, -1), dim=1)` without mask, scale or gradient."""
+    host = nt.host()
+    out = host.combine(y, k) if host is not None else None
+    return out if out is not None else _reduce_forward(y.view(y.shape[0] // k, k, y.shape[-1]), None, None, None)[0]
+
+
 def _reduce_forward(x, mask, scale, y):
     nt.require_gpu(x, "x")
     if x.stride(2) != 1:

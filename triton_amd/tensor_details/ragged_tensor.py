@@ -25,6 +25,7 @@ class RaggedTensorMetadata:
     block_schedule_data: torch.Tensor  # [n_block_sizes, max_n_blocks] int32, (block << 16) | slice, -1 padded
     expected_slice_size: int | None = None
     slice_sizes_divisibility: int = None
+    remapped_from = None  # set by `remap_ragged_tensor_metadata`: the number of slices of the source tensor
 
     def __post_init__(self):
         n = len(_BLOCK_SIZES)
