@@ -76,6 +76,10 @@ __device__ __forceinline__ void lds_dma16(buf_desc_t desc, uint32_t dst, uint32_
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(dst), "v"(off), "s"(desc) : "memory");
 }
+// the same by the lower 32 lanes only (512 bytes; every lane is active when it is called)
+__device__ __forceinline__ void lds_dma16_lower(buf_desc_t desc, uint32_t dst, uint32_t off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_hi, 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n\ts_mov_b32 exec_hi, -1" ::"s"(dst), "v"(off), "s"(desc) : "memory");
+}
 // the same with 4 bytes per lane
 template <bool NT = false>
 __device__ __forceinline__ void lds_dma4(buf_desc_t desc, uint32_t dst, uint32_t off) {

@@ -80,6 +80,7 @@ int32_t gemm_launch_mxn(const GemmParams& p, int block_m, int grid_m, bool swigl
 int32_t gemm_launch_mxn_mx(const GemmParams& p, int block_m, int grid_m, bool swiglu, hipStream_t st);  // block_m 128 / 256, MX-quantised output
 int32_t gemm_launch_mxd(const GemmParams& p, int block_m, int grid_m, bool swiglu, hipStream_t st);
 int32_t gemm_launch_mxs(const GemmParams& p, int grid_m, bool swiglu, bool once, hipStream_t st);  // block_m 32; once: about one row block per slice
+int32_t gemm_launch_mxw(const GemmParams& p, bool mx_act, bool swiglu, bool mx_out, hipStream_t st);  // block_m 256
 int32_t gemm_launch_f8n(const GemmParams& p, int block_m, int grid_m, bool swiglu, hipStream_t st);
 int32_t gemm_launch_mx8n(const GemmParams& p, int block_m, int grid_m, bool swiglu, bool mx_out, hipStream_t st);
 

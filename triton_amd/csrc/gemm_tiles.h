@@ -50,9 +50,15 @@ struct TileList {
     grid_n = p.grid_n;
     const int xcd = blockIdx.x & 7;
     t_step = gridDim.x >> 3;
-    f_beg = (int)(((int64_t)full * grid_n * xcd) >> 3), f_len = (int)(((int64_t)full * grid_n * (xcd + 1)) >> 3) - f_beg;
-    s_beg = (int)(((int64_t)brief * grid_n * xcd) >> 3);
-    t_end = f_len + (int)(((int64_t)brief * grid_n * (xcd + 1)) >> 3) - s_beg;
+    // An eighth of the full tiles, and of the short ones what makes an eighth of all: with each list divided on its own an XCD could be two
+    // tiles over, which one workgroup then had in a round of its own (94 rows a slice, three rounds, K 2880, N 2880: 195 -> 169 us).
+    // (From eight short tiles on their bounds only grow: an eighth of all is then at least the larger eighth of the full ones.)
+    const int64_t n_f = (int64_t)full * grid_n, n_s = (int64_t)brief * grid_n, n = n_f + n_s;
+    auto full_to = [&](int x) -> int { return (int)((n_f * x) >> 3); };
+    auto short_to = [&](int x) -> int { return n_s < 8 ? (int)((n_s * x) >> 3) : (int)((n * x) >> 3) - full_to(x); };
+    f_beg = full_to(xcd), f_len = full_to(xcd + 1) - f_beg;
+    s_beg = short_to(xcd);
+    t_end = f_len + short_to(xcd + 1) - s_beg;
     return (int)(blockIdx.x >> 3);
   }
 

@@ -169,6 +169,19 @@ int64_t mxfp4_block_m(int64_t rows, int64_t n_slices, int64_t otherwise) {
   return per_slice <= 20 ? 32 : per_slice <= 56 ? 64 : std::max<int64_t>(otherwise, 128);
 }
 
+// Row blocks of 128, or 256 = the wide kernel (160 x 512 tiles), for MXFP4 weights beyond the sizes above.  Measured at K 2880, N 5760 and
+// 2880 (both GEMMs, 128 against 256).  bf16 rows: 64 per slice 571 against 582 us, 94 684 against 668, 162 1296 against 1131,
+// 250 (16 slices) 258 against 246, 1024 754 against 716 us.  MXFP8 rows: 64 per slice 444 against 451 us, 112 537 against 503, 162 932
+// against 767; past one tile per slice the smaller blocks, whose tiles of a slice share weights in L2, win (203 910 against 955, 250
+// 143 against 153 us), until a workgroup has several tiles of a slice (512: 256 us either way, 1024 469 against 440 us).
+// The wide kernel takes four stages of K (the activation scales sixteen blocks), 256 slices and x below 2 GiB.
+int64_t wide_block_m(int64_t rows, int64_t n_slices, int64_t K, int64_t x_bytes, bool mx8) {
+  n_slices = std::max<int64_t>(n_slices, 1);
+  if (K <= (mx8 ? 511 : 384) || n_slices > 256 || x_bytes >= int64_t(1) << 31) return rows <= 144 * n_slices ? 256 : 128;
+  if (rows <= 80 * n_slices) return 128;
+  return !mx8 || rows <= 176 * n_slices || rows >= 640 * n_slices ? 256 : 128;
+}
+
 int64_t default_block_m(int64_t rows, int64_t n_slices) {
   int64_t per_slice = std::max<int64_t>(1, rows / std::max<int64_t>(n_slices, 1));
   return per_slice <= 16 ? 16 : per_slice <= 32 ? 32 : per_slice <= 64 ? 64 : 128;
@@ -356,10 +369,10 @@ PyObject* run_gemm(PyObject* const* v) {
   if (tiled_fp8) {
     block_m = dma_block_m(M, K, N, n_slices);
   } else if (mx_act) {
-    block_m = M <= 144 * n_slices ? 256 : 128;
+    block_m = wide_block_m(M, n_slices, K, a_rows * a_stride, true);
   } else if (tiled) {
     if (M > 256 && short_x && n_slices <= 256 && !x_row && !w_col) block_m = mxfp4_block_m(M, n_slices, block_m);
-    if (block_m == 128 && M <= 144 * n_slices) block_m = 256;  // about 128 rows per expert: one tile per expert, the weights are read once
+    if (block_m == 128) block_m = wide_block_m(M, n_slices, K, a_rows * a_stride * 2, false);
   } else if (!(short_x && n_slices <= 256 && N * w->stride(2) < (int64_t(1) << 30))) {
     block_m = std::min<int64_t>(block_m, 128);
   } else if (block_m > 16) {
@@ -406,9 +419,9 @@ PyObject* run_gemm(PyObject* const* v) {
   };
   if ((tiled || tiled_fp8) && block_m >= 64 && !mx_act) d.tile_counters = words(B.tile_counters, true);
   // the combine inside the launch: with the decode kernel by the wave that completes a token's rows, with the prefill kernel by
-  // the persistent grid at its end; the streaming kernel (block_m 32) has none
+  // the persistent grid at its end; the streaming (block_m 32) and the wide kernel (256) have none
   if (combine_k > 0 && tiled && !mx_act && !act.swiglu && scatter && y_rows % combine_k == 0
-      && (block_m == 16 ? (y_rows / combine_k) * ((N + 31) / 32) <= (1 << 16) : block_m >= 64 && N % 8 == 0)) {
+      && (block_m == 16 ? (y_rows / combine_k) * ((N + 31) / 32) <= (1 << 16) : block_m >= 64 && block_m != 256 && N % 8 == 0)) {
     combined = empty({y_rows / combine_k, N}, out, *a);
     d.combine_k = int32_t(combine_k), d.combine_out = combined.data_ptr(), d.combine_stride_m = N;
     if (block_m == 16) d.combine_counters = words(B.combine_counters, false);
@@ -706,6 +719,12 @@ PyObject* rule(PyObject* const* v, bool dma) {
   if (PyErr_Occurred()) throw PyError();
   return PyLong_FromLongLong(dma ? dma_block_m(a, b, c, d) : mxfp4_block_m(a, b, c));
 }
+PyObject* rule_wide(PyObject* const* v) {
+  int64_t a[5];
+  for (int i = 0; i < 5; ++i) a[i] = PyLong_AsLongLong(v[i]);
+  if (PyErr_Occurred()) throw PyError();
+  return PyLong_FromLongLong(wide_block_m(a[0], a[1], a[2], a[3], a[4] != 0));
+}
 PyObject* rule_dma(PyObject* const* v) { return rule(v, true); }
 PyObject* rule_mxfp4(PyObject* const* v) { return rule(v, false); }
 
@@ -757,6 +776,7 @@ PyMethodDef methods[] = {
     METHOD("decode_layer", run_decode_layer, 13),
     METHOD("dma_block_m", rule_dma, 4),
     METHOD("mxfp4_block_m", rule_mxfp4, 3),
+    METHOD("wide_block_m", rule_wide, 5),
     {nullptr, nullptr, 0, nullptr},
 };
 

@@ -3,7 +3,7 @@
 //
 //   Y[dst(r), :] = act( (X[src(r), :] @ W[e(r)]) * sx[src(r)] * sw[e(r), :] + bias[e(r), :] ) * gamma[r]
 //
-// validates the descriptor and hands it to one kernel family (moe_gemm_strided / _mxn / _mxd / _f8n / _mx8n .hip).
+// validates the descriptor and hands it to one kernel family (moe_gemm_strided / _dma / _mxn / _mxw / _mxs / _mxd / _f8n / _mx8n .hip).
 #include "gemm_common.h"
 
 using namespace tk;
@@ -12,6 +12,11 @@ using namespace tk;
 // 2 GiB (buffer resources) and the slices' sizes in its registers.
 static bool dma_ok(const GemmParams& p, const tk_gemm_desc* d, int64_t w_bytes) {
   return p.x_bytes && (!d->slice_sizes || d->n_slices <= kDmaSlices) && w_bytes < (int64_t)1 << 31 && (d->block_m == 128 || d->block_m == 256);
+}
+
+// what the wide MXFP4 kernel needs beyond its neighbours' conditions: x within a buffer resource, the slice list in registers, four stages of K
+static bool wide_ok(const GemmParams& p, const tk_gemm_desc* d) {
+  return d->block_m == 256 && p.x_bytes && (!d->slice_sizes || d->n_slices <= kDmaSlices) && p.w_nst >= 4;
 }
 
 extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
@@ -171,6 +176,7 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
         fast = fast && p.y_vec && d->y_stride_m >= cdiv(n_out, piece) * piece;
       p.y_bytes = fast ? (uint32_t)y_bytes : 0u;
     }
+    if (p.y_bytes != 0 && wide_ok(p, d)) return gemm_launch_mxw(p, true, swiglu, mx_out, st);
     return gemm_launch_mx8n(p, d->block_m, d->grid_m, swiglu, mx_out, st);
   }
   if (d->w_layout == TK_W_TILED) {
@@ -223,6 +229,7 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
       return gemm_launch_mxs(p, d->grid_m, swiglu, (int64_t)d->M <= (int64_t)d->n_slices * 16, st);
     if (d->block_m <= 32) return gemm_launch_mxd(p, d->block_m, d->grid_m, swiglu, st);
     if (mx_out_bf16) return gemm_launch_mxn_mx(p, d->block_m, d->grid_m, swiglu, st);
+    if (d->combine_k <= 0 && wide_ok(p, d)) return gemm_launch_mxw(p, false, swiglu, false, st);
     return gemm_launch_mxn(p, d->block_m, d->grid_m, swiglu, st);
   }
   if (d->w_layout != TK_W_STRIDED) return fail(TK_ERR_INVALID, "tk_moe_gemm: bad w_layout %d", d->w_layout);

@@ -755,7 +755,10 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
         block_m = forced if forced in (128, 256) else 128 if forced is not None else nt.rules().dma_block_m(M, K, N, n_slices)
     elif mx_act or (tiled and mx_out_fused):
         # the tile shapes that take MXFP8 activations / have an MX-output epilogue
-        block_m = 256 if (forced == 256 or (forced is None and is_ragged and M <= 144 * n_slices)) else 128
+        if forced is None and is_ragged:
+            block_m = nt.rules().wide_block_m(M, n_slices, K, a_rows * a_stride, 1) if mx_act else 256 if M <= 144 * n_slices else 128
+        else:
+            block_m = 256 if forced == 256 else 128
     elif tiled:
         if extras:
             block_m = min(block_m, 32)  # the decode kernel carries the shared epilogue; the prefill kernels do not take these options
@@ -763,8 +766,8 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
             if (M > 256 and a_rows * a_stride < 1 << 30 and n_slices <= 256 and a_ts is None and b_ts is None
                     and a_ragged_metadata.expected_slice_size is None):
                 block_m = nt.rules().mxfp4_block_m(M, n_slices, block_m)
-            if block_m == 128 and M <= 144 * n_slices:
-                block_m = 256  # about 128 rows per expert: one tile per expert, the weights are read once
+            if block_m == 128:
+                block_m = nt.rules().wide_block_m(M, n_slices, K, a_rows * a_stride * 2, 0)
     elif w_dtype in (_BF16, _F16):
         # (the conditions of the memory-to-LDS kernel: x and an expert's weights within 2 GiB, up to 256 slices)
         dma = a_rows * a_stride < 1 << 30 and n_slices <= 256 and N * w.stride(-1) < 1 << 30
@@ -822,8 +825,8 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
     # launch of its own at the gpt-oss shape)
     can_combine = (_combine_k and tiled and not extras and not mx_act and act == nt.TK_ACT_NONE and scatter_indx is not None
                    and y_rows % _combine_k == 0 and a_dtype == _BF16)
-    if can_combine and block_m == 32 and forced is None:
-        can_combine = False  # the streaming kernel has no combine
+    if can_combine and block_m in (32, 256) and forced is None:
+        can_combine = False  # the streaming and the wide kernel have no combine
     elif can_combine and block_m <= 32:
         # decode kernel: the wave that completes a token's rows last sums them (arrival counters per token and fragment)
         can_combine = (y_rows // _combine_k) * ((N + 31) // 32) <= _COMBINE_COUNTER_WORDS
