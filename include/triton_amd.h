@@ -282,8 +282,9 @@ typedef struct tk_gemm_desc {
   const int32_t* block_offs;     /* [n_slices + 1] for block_m */
   const int32_t* block_schedule; /* [grid_m] for block_m, (block << 16) | slice, -1 padded */
   int32_t n_slices;
-  int32_t block_m; /* 16, 32, 64 or 128; tiled MXFP4 weights also 256, and so do strided 16-bit weights with x (x_rows given) and an
-                    * expert's weights within 2 GiB and up to 256 slices; tiled e4m3 weights 128 or 256 only */
+  int32_t block_m; /* 16, 32, 64 or 128; tiled MXFP4 weights also 256, and so do strided 16-bit weights with x (x_rows given, rows
+                    * at least K apart) and an expert's weights (columns at least K apart) within 2 GiB and up to 256 slices; tiled e4m3
+                    * weights 128 or 256 only */
   int32_t grid_m;  /* number of row blocks to launch (an upper bound in ragged mode) */
   int32_t M, N, K; /* M: rows of the single slice when not ragged; N: columns of W; K: reduction */
   /* output [rows, N or N/2], unit stride along N */

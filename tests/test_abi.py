@@ -131,6 +131,21 @@ def test_gather_without_x_rows_is_refused_by_the_prefill_tiled_kernels():
     assert "x_rows is required" in nt.last_error()
 
 
+def test_row_blocks_of_256_with_16_bit_weights_are_refused_where_no_kernel_has_them():
+    """Overlapping rows of x, overlapping weight columns, too many slices: refused before any launch (fake, aligned pointers)."""
+    lib = nt.lib()
+    for name, value in (("x_stride_m", 256), ("x_stride_m", 0), ("w_stride_n", 256), ("n_slices", 257)):
+        d = nt.GemmDesc()
+        d.x, d.w, d.y = 0x1000, 0x2000, 0x3000
+        d.slice_sizes, d.slice_offs, d.block_offs, d.block_schedule = 0x4000, 0x5000, 0x6000, 0x7000
+        d.x_dtype, d.w_dtype, d.y_dtype = nt.TK_BF16, nt.TK_BF16, nt.TK_BF16
+        d.M, d.N, d.K, d.grid_m, d.block_m, d.n_slices, d.x_rows = 4096, 1024, 512, 31, 256, 16, 4096
+        d.x_stride_m, d.y_stride_m, d.w_stride_k, d.w_stride_n, d.w_stride_e = 512, 1024, 1, 512, 512 * 1024
+        setattr(d, name, value)
+        assert lib.tk_moe_gemm(ctypes.byref(d), None) == nt.TK_ERR_INVALID, name
+        assert "block_m 256" in nt.last_error()
+
+
 def test_status_to_exception_mapping():
     with pytest.raises(ValueError):
         nt.check(nt.TK_ERR_INVALID, "bad")

@@ -65,3 +65,32 @@ def test_slice_registers(device, n_slices):
     """257 slices run on the kernel without registers for them."""
     _check(device, "e4m3", 128, [(i * 37) % 9 for i in range(n_slices)], 192, 160)
     _check(device, "bfloat16", 128, [(i * 37) % 9 for i in range(n_slices)], 192, 160)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("stride", [0, 8, 56])
+def test_overlapping_rows(device, monkeypatch, dtype, stride):
+    """Rows closer together than their length (one row expanded, sliding windows) with as many of them per slice as take row blocks of
+    256 otherwise: they run on the general kernel, from the native host path and from the general one, gathered and not."""
+    import triton_amd.matmul as mm
+    from triton_amd import _native as nt
+    from triton_amd.tensor import make_ragged_tensor_metadata
+    g = torch.Generator().manual_seed(stride)
+    sizes, k, n = torch.tensor([300, 0, 129, 400], dtype=torch.int32), 64, 72
+    m, out_dtype = int(sizes.sum()), getattr(torch, dtype)
+    base = torch.randn((m * stride + k, ), generator=g).to(out_dtype)
+    x, xd = base.as_strided((m, k), (stride, 1)), base.to(device).as_strided((m, k), (stride, 1))
+    w = (torch.randn((4, n, k), generator=g) * 0.1).to(out_dtype)
+    wd = w.to(device).transpose(1, 2)
+    md = make_ragged_tensor_metadata(sizes.to(device), m)
+    for gi in (None, torch.randint(0, m, (m, ), generator=g).to(torch.int32)):
+        gd = None if gi is None else gi.to(device)
+        want = omoe.matmul(x, w.transpose(1, 2), None, sizes, gather_indx=gi, out_dtype=torch.float32)
+        native = mm.matmul(xd, wd, None, md, gather_indx=gd)
+        with monkeypatch.context() as p:
+            p.setattr(nt, "host", lambda: None)
+            general = mm.matmul(xd, wd, None, md, gather_indx=gd)
+        assert_allclose_gate(want, native, what=f"{dtype} row stride {stride}")
+        assert torch.equal(native, general)
+    assert_allclose_gate(omoe.matmul(x, w[:1].transpose(1, 2), None, torch.tensor([m], dtype=torch.int32), out_dtype=torch.float32),
+                         mm.matmul(xd, wd[:1], None), what="not ragged")

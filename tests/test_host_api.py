@@ -226,3 +226,53 @@ def test_weight_relayout_cache_key_and_invalidation():
 def test_routing_data_records_whether_every_token_has_all_its_rows():
     from triton_amd.legacy import RoutingData
     assert RoutingData.__dataclass_fields__["all_rows_live"].default is False
+
+
+@pytest.fixture
+def gemm_calls(monkeypatch):
+    """The descriptors `matmul` hands to the library, with host tensors in the place of device ones and nothing launched."""
+    from triton_amd import _native as nt
+    nt.rules()
+    real, calls = nt.lib(), []
+
+    class Recorder:
+        def tk_moe_gemm(self, d, stream):
+            calls.append({name: getattr(d, name) for name, _ in d._fields_})
+            return nt.TK_OK
+
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+    recorder = Recorder()
+    monkeypatch.setattr(nt, "lib", lambda: recorder)
+    monkeypatch.setattr(nt, "require_gpu", lambda *_: None)
+    monkeypatch.setattr(nt, "stream_ptr", lambda *_: 0)
+    return calls
+
+
+def _metadata(n_slices, rows):
+    i32 = dict(dtype=torch.int32)
+    width = RaggedTensorMetadata.max_n_blocks(n_slices, rows)
+    return RaggedTensorMetadata(torch.zeros(n_slices, **i32), torch.zeros(n_slices + 1, **i32), torch.zeros((5, n_slices + 1), **i32),
+                                torch.zeros((5, width), **i32))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("ragged", [True, False])
+def test_overlapping_rows_stay_off_the_256_row_blocks(gemm_calls, dtype, ragged):
+    # rows closer together than their length: the kernel with row blocks of 256 does not run on them and the general one ends at 128
+    from triton_amd.matmul import matmul, scoped_opt_flags_constraints
+    n_slices, rows, k, n = (16, 4096, 512, 1024) if ragged else (1, 4096, 512, 1024)
+    w = torch.zeros((n_slices, n, k), dtype=dtype).transpose(1, 2)
+    md = _metadata(n_slices, rows) if ragged else None
+    base = torch.zeros(rows * 512, dtype=dtype)
+    for stride, want in ((512, 256), (0, 128), (256, 128), (504, 128)):
+        x = base.as_strided((rows, k), (stride, 1))
+        matmul(x, w, None, md)
+        assert (gemm_calls[-1]["x_stride_m"], gemm_calls[-1]["block_m"]) == (stride, want)
+        with scoped_opt_flags_constraints({"block_m": 256}):
+            matmul(x, w, None, md)
+        assert gemm_calls[-1]["block_m"] == want
+    one = torch.zeros((1, k), dtype=dtype).expand(rows, k)
+    matmul(one, w, None, md)
+    assert gemm_calls[-1]["block_m"] == 128

@@ -9,6 +9,7 @@
 #include <unordered_map>
 
 #include "common.h"
+#include "gemm_limits.h"
 #include "mx_math.h"
 
 namespace tk {
@@ -70,7 +71,7 @@ struct GemmParams {
   float out_alpha;
   const uint16_t* acc_in;     // tensor of the output's shape and type added to the result (behind the gate weight), or null
   int64_t acc_in_stride_m;
-  uint32_t x_bytes;           // extent of x for a buffer resource (kernels that address x through one), 0 = not below 2 GiB
+  uint32_t x_bytes;           // extent of x for a buffer resource (kernels that address x through one), 0 = none (`x_extent`)
 };
 
 // one entry per kernel family; each returns a TK_* status
@@ -87,8 +88,6 @@ int32_t gemm_launch_mx8n(const GemmParams& p, int block_m, int grid_m, bool swig
 // Slices (experts) whose row and block offsets the persistent MXFP4 prefill kernel keeps in LDS: a tile's coordinates
 // then cost LDS reads instead of a chain of dependent global loads.  The host refuses more slices than this.
 constexpr int kMetaSlices = 1024;
-// Slices whose sizes and offsets the memory-to-LDS kernel keeps in registers; other kernels run with more.
-constexpr int kDmaSlices = 256;
 
 namespace {
 

@@ -23,6 +23,7 @@
 #include <optional>
 
 #include "../../include/triton_amd.h"
+#include "gemm_limits.h"
 
 namespace {
 
@@ -373,9 +374,7 @@ PyObject* run_gemm(PyObject* const* v) {
   } else if (tiled) {
     if (M > 256 && short_x && n_slices <= 256 && !x_row && !w_col) block_m = mxfp4_block_m(M, n_slices, block_m);
     if (block_m == 128) block_m = wide_block_m(M, n_slices, K, a_rows * a_stride * 2, false);
-  } else if (!(short_x && n_slices <= 256 && N * w->stride(2) < (int64_t(1) << 30))) {
-    block_m = std::min<int64_t>(block_m, 128);
-  } else if (block_m > 16) {
+  } else if (block_m > 16 && tk::dma_runs_16bit(tk::x_extent(a_rows, a_stride, K, 2), n_slices, K, N, w->stride(2))) {
     block_m = dma_block_m(M, 2 * K, N, n_slices);
   }
   if (tiled && block_m >= 64 && !mx_act && n_out % 8) return none();  // (through a padded buffer)
@@ -725,6 +724,13 @@ PyObject* rule_wide(PyObject* const* v) {
   if (PyErr_Occurred()) throw PyError();
   return PyLong_FromLongLong(wide_block_m(a[0], a[1], a[2], a[3], a[4] != 0));
 }
+// (rows of x, their stride, K, N, stride of a weight column, slices) -> does the memory-to-LDS kernel run on strided 16-bit weights?
+PyObject* rule_dma_16bit(PyObject* const* v) {
+  int64_t a[6];
+  for (int i = 0; i < 6; ++i) a[i] = PyLong_AsLongLong(v[i]);
+  if (PyErr_Occurred()) throw PyError();
+  return PyBool_FromLong(tk::dma_runs_16bit(tk::x_extent(a[0], a[1], a[2], 2), a[5], a[2], a[3], a[4]));
+}
 PyObject* rule_dma(PyObject* const* v) { return rule(v, true); }
 PyObject* rule_mxfp4(PyObject* const* v) { return rule(v, false); }
 
@@ -774,6 +780,7 @@ PyMethodDef methods[] = {
     METHOD("mx_upcast", run_mx_upcast, 4),
     METHOD("ragged_k", run_ragged_k, 4),
     METHOD("decode_layer", run_decode_layer, 13),
+    METHOD("dma_runs_16bit", rule_dma_16bit, 6),
     METHOD("dma_block_m", rule_dma, 4),
     METHOD("mxfp4_block_m", rule_mxfp4, 3),
     METHOD("wide_block_m", rule_wide, 5),

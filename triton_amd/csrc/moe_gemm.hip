@@ -8,15 +8,22 @@
 
 using namespace tk;
 
-// Can the kernel that stages both operands through memory-to-LDS transfers run this?  x and an expert's weights (`w_bytes`) have to lie within
-// 2 GiB (buffer resources) and the slices' sizes in its registers.
-static bool dma_ok(const GemmParams& p, const tk_gemm_desc* d, int64_t w_bytes) {
-  return p.x_bytes && (!d->slice_sizes || d->n_slices <= kDmaSlices) && w_bytes < (int64_t)1 << 31 && (d->block_m == 128 || d->block_m == 256);
+// slices of the ragged metadata (a call without it has one)
+static int64_t slices(const tk_gemm_desc* d) { return d->slice_sizes ? d->n_slices : 1; }
+
+// Strided 16-bit weights: the kernel that stages both operands through memory-to-LDS transfers for full row blocks where it runs, else the
+// general one, which has no row blocks of 256.
+static int32_t launch_16bit(const GemmParams& p, const tk_gemm_desc* d, int wk, bool swiglu, hipStream_t st) {
+  const bool dma = dma_runs_16bit(p.x_bytes, slices(d), d->K, d->N, d->w_stride_n);
+  if (dma && (d->block_m == 128 || d->block_m == 256)) return gemm_launch_dma(p, wk, d->block_m, d->grid_m, swiglu, st);
+  if (d->block_m == 256)
+    return fail(TK_ERR_INVALID, "tk_moe_gemm: block_m 256 with 16-bit weights needs x (x_rows rows, none closer than K) and an expert's weights within 2 GiB and up to %d slices", kDmaSlices);
+  return gemm_launch_strided(p, wk, d->block_m, d->grid_m, swiglu, st);
 }
 
 // what the wide MXFP4 kernel needs beyond its neighbours' conditions: x within a buffer resource, the slice list in registers, four stages of K
 static bool wide_ok(const GemmParams& p, const tk_gemm_desc* d) {
-  return d->block_m == 256 && p.x_bytes && (!d->slice_sizes || d->n_slices <= kDmaSlices) && p.w_nst >= 4;
+  return d->block_m == 256 && p.x_bytes && slices(d) <= kDmaSlices && p.w_nst >= 4;
 }
 
 extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
@@ -126,8 +133,7 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
   {
     // extent of x for the kernels that address it through a buffer resource
     const int64_t rows = d->x_rows > 0 ? d->x_rows : (d->gather_indx ? 0 : d->M);
-    const int64_t bytes = rows * d->x_stride_m * (d->x_dtype == TK_E4M3 ? 1 : 2);
-    p.x_bytes = bytes > 0 && d->x_stride_m >= d->K && bytes < (int64_t)1 << 31 ? (uint32_t)bytes : 0u;
+    p.x_bytes = x_extent(rows, d->x_stride_m, d->K, d->x_dtype == TK_E4M3 ? 1 : 2);
   }
   if (d->w_layout == TK_W_TILED && d->w_dtype == TK_E4M3) {
     if (d->w_mx_scale) return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: MX scales with e4m3 weights");
@@ -138,7 +144,7 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
     if (d->n_slices > 1 && d->w_stride_e < nfr * nst * 8192) return fail(TK_ERR_INVALID, "tk_moe_gemm: expert stride smaller than one tiled expert");
     p.w_stride_e = d->w_stride_e;
     p.w_nst = (int32_t)nst;
-    if (dma_ok(p, d, nfr * nst * 8192)) return gemm_launch_dma(p, WK_FP8, d->block_m, d->grid_m, swiglu, st);
+    if (dma_runs(p.x_bytes, slices(d), nfr * nst * 8192)) return gemm_launch_dma(p, WK_FP8, d->block_m, d->grid_m, swiglu, st);
     return gemm_launch_f8n(p, d->block_m, d->grid_m, swiglu, st);
   }
   if (mx_act) {
@@ -225,7 +231,7 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
     p.w_nst = (int32_t)nst;
     // row blocks of 32: the streaming kernel, unless something asks for the decode kernel's epilogue or fused combine (or x is too large
     // for a buffer resource, or there are more slices than it has registers for)
-    if (d->block_m == 32 && p.x_bytes && (!d->slice_sizes || d->n_slices <= kDmaSlices) && !extras && d->combine_k <= 0 && !d->x_row_scale && !d->w_col_scale)
+    if (d->block_m == 32 && p.x_bytes && slices(d) <= kDmaSlices && !extras && d->combine_k <= 0 && !d->x_row_scale && !d->w_col_scale)
       return gemm_launch_mxs(p, d->grid_m, swiglu, (int64_t)d->M <= (int64_t)d->n_slices * 16, st);
     if (d->block_m <= 32) return gemm_launch_mxd(p, d->block_m, d->grid_m, swiglu, st);
     if (mx_out_bf16) return gemm_launch_mxn_mx(p, d->block_m, d->grid_m, swiglu, st);
@@ -248,8 +254,7 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
     if (d->w_stride_n % 8 || d->w_stride_e % 8 || (reinterpret_cast<uintptr_t>(d->w) & 15)) return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: weight columns must be 16-byte aligned");
     p.w_stride_e = d->w_stride_e * 2;
     p.w_stride_n = d->w_stride_n * 2;
-    if (dma_ok(p, d, (int64_t)(d->N - 1) * p.w_stride_n + d->K * 2) && p.w_stride_n >= d->K * 2) return gemm_launch_dma(p, WK_BF16, d->block_m, d->grid_m, swiglu, st);
-    return gemm_launch_strided(p, WK_BF16, d->block_m, d->grid_m, swiglu, st);
+    return launch_16bit(p, d, WK_BF16, swiglu, st);
   }
   if (d->w_dtype == TK_F16) {
     // fp16 x fp16 -> fp16 (v_mfma_f32_*_f16); same data path as bf16
@@ -258,8 +263,7 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
     if (d->w_stride_n % 8 || d->w_stride_e % 8 || (reinterpret_cast<uintptr_t>(d->w) & 15)) return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: weight columns must be 16-byte aligned");
     p.w_stride_e = d->w_stride_e * 2;
     p.w_stride_n = d->w_stride_n * 2;
-    if (dma_ok(p, d, (int64_t)(d->N - 1) * p.w_stride_n + d->K * 2) && p.w_stride_n >= d->K * 2) return gemm_launch_dma(p, WK_F16, d->block_m, d->grid_m, swiglu, st);
-    return gemm_launch_strided(p, WK_F16, d->block_m, d->grid_m, swiglu, st);
+    return launch_16bit(p, d, WK_F16, swiglu, st);
   }
   if (d->w_dtype == TK_E4M3) {
     if (d->w_mx_scale) return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: MX scales with e4m3 weights");

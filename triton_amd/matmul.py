@@ -769,12 +769,11 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
             if block_m == 128:
                 block_m = nt.rules().wide_block_m(M, n_slices, K, a_rows * a_stride * 2, 0)
     elif w_dtype in (_BF16, _F16):
-        # (the conditions of the memory-to-LDS kernel: x and an expert's weights within 2 GiB, up to 256 slices)
-        dma = a_rows * a_stride < 1 << 30 and n_slices <= 256 and N * w.stride(-1) < 1 << 30
-        if not dma:
-            block_m = min(block_m, 128)
-        elif forced is None and block_m > 16:
-            block_m = nt.rules().dma_block_m(M, 2 * K, N, n_slices)
+        if block_m > 16:
+            if not nt.rules().dma_runs_16bit(a_rows, a_stride, K, N, w.stride(-1), n_slices):
+                block_m = min(block_m, 128)  # (the general kernel's largest)
+            elif forced is None:
+                block_m = nt.rules().dma_block_m(M, 2 * K, N, n_slices)
     elif block_m == 256:
         block_m = 128
     if is_ragged:
