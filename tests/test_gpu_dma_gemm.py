@@ -94,3 +94,28 @@ def test_overlapping_rows(device, monkeypatch, dtype, stride):
         assert torch.equal(native, general)
     assert_allclose_gate(omoe.matmul(x, w[:1].transpose(1, 2), None, torch.tensor([m], dtype=torch.int32), out_dtype=torch.float32),
                          mm.matmul(xd, wd[:1], None), what="not ragged")
+
+
+@pytest.mark.parametrize("sizes", [[300, 0, 129, 400], [1100, 1030, 1000]])
+@pytest.mark.parametrize("stride", [0, 16])
+def test_overlapping_rows_tiled_e4m3(device, monkeypatch, sizes, stride):
+    """The same with tiled e4m3 weights, on the kernel that takes rows anywhere: row blocks of 128, and from 1024 rows per slice on of 256."""
+    import triton_amd.matmul as mm
+    from triton_amd import _native as nt
+    from triton_amd.tensor import convert_layout, make_ragged_tensor_metadata, wrap_torch_tensor
+    from triton_amd.tensor_details.layout import make_default_matmul_fp8_w_layout
+    g = torch.Generator().manual_seed(stride + len(sizes))
+    E, m, k, n = len(sizes), sum(sizes), 272, 72
+    sizes = torch.tensor(sizes, dtype=torch.int32)
+    base = torch.randn((m * stride + k, ), generator=g).to(torch.float8_e4m3fn)
+    x, xd = base.as_strided((m, k), (stride, 1)), base.to(device).as_strided((m, k), (stride, 1))
+    w = (torch.randn((E, n, k), generator=g) * 0.1).to(torch.float8_e4m3fn)
+    wd = convert_layout(wrap_torch_tensor(w.to(device).transpose(1, 2)), make_default_matmul_fp8_w_layout())
+    gi, pc, md = torch.randint(0, m, (m, ), generator=g).to(torch.int32), mm.PrecisionConfig(out_dtype=torch.bfloat16), make_ragged_tensor_metadata(sizes.to(device), m)
+    native = mm.matmul(xd, wd, None, md, gather_indx=gi.to(device), precision_config=pc)
+    with monkeypatch.context() as p:
+        p.setattr(nt, "host", lambda: None)
+        general = mm.matmul(xd, wd, None, md, gather_indx=gi.to(device), precision_config=pc)
+    want = omoe.matmul(x.contiguous(), w.transpose(1, 2), None, sizes, gather_indx=gi, out_dtype=torch.float32)
+    assert_allclose_gate(want, native, what=f"e4m3 row stride {stride}")
+    assert torch.equal(native, general)

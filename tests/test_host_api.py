@@ -276,3 +276,32 @@ def test_overlapping_rows_stay_off_the_256_row_blocks(gemm_calls, dtype, ragged)
     one = torch.zeros((1, k), dtype=dtype).expand(rows, k)
     matmul(one, w, None, md)
     assert gemm_calls[-1]["block_m"] == 128
+
+
+def _tiled(kind, n_slices, k, n):
+    from triton_amd.tensor_details import layout as L
+    if kind == "fp8":
+        w = torch.zeros((n_slices, n, k), dtype=torch.float8_e4m3fn).transpose(1, 2)
+        return convert_layout(wrap_torch_tensor(w), L.make_default_matmul_fp8_w_layout()), None
+    w, s = torch.zeros((n_slices, n, k // 2), dtype=torch.uint8).transpose(1, 2), torch.zeros((n_slices, n, k // 32), dtype=torch.uint8).transpose(1, 2)
+    return (convert_layout(wrap_torch_tensor(w, dtype=FP4), L.make_default_matmul_mxfp4_w_layout(mx_axis=1)),
+            convert_layout(wrap_torch_tensor(s), L.make_default_matmul_mxfp4_w_scale_layout(mx_axis=1)))
+
+
+@pytest.mark.parametrize("kind, n_slices, per_slice, want, overlapping", [
+    ("fp8", 4, 250, 256, 128), ("fp8", 4, 1023, 256, 128), ("fp8", 4, 1024, 256, 256), ("fp8", 4, 64, 128, 128), ("fp8", 257, 200, 128, 128),
+    ("mxfp4", 16, 30, 64, 32), ("mxfp4", 16, 60, 128, 64), ("mxfp4", 16, 162, 256, 128), ("mxfp4", 257, 60, 64, 64),
+    ("mxfp8", 16, 162, 256, 128), ("mxfp8", 16, 250, 128, 128), ("mxfp8", 257, 60, 256, 256),
+])
+def test_row_blocks_follow_the_kernel_that_runs(gemm_calls, kind, n_slices, per_slice, want, overlapping):
+    # the rules measured for the kernels that address x through a buffer resource hold where those run (not with overlapping rows, not
+    # with more than 256 slices); elsewhere the other kernels' own rules do
+    from triton_amd.matmul import PrecisionConfig, matmul
+    k, n, rows = 512, 64, n_slices * per_slice
+    w, s = _tiled(kind, n_slices, k, n)
+    dtype = torch.bfloat16 if kind == "mxfp4" else torch.float8_e4m3fn
+    xs = torch.zeros((rows, k // 32), dtype=torch.uint8) if kind == "mxfp8" else None
+    pc, md = PrecisionConfig(a_mx_scale=xs, b_mx_scale=s, out_dtype=torch.bfloat16), _metadata(n_slices, rows)
+    for stride, block_m in ((k, want), (0, overlapping), (k - 16, overlapping)):
+        matmul(torch.zeros(rows * k, dtype=dtype).as_strided((rows, k), (stride, 1)), w, None, md, precision_config=pc)
+        assert (gemm_calls[-1]["x_stride_m"], gemm_calls[-1]["block_m"]) == (stride, block_m)

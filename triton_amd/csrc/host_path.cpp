@@ -20,6 +20,7 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <algorithm>
+#include <array>
 #include <optional>
 
 #include "../../include/triton_amd.h"
@@ -161,10 +162,20 @@ int64_t dma_block_m(int64_t rows, int64_t row_bytes, int64_t N, int64_t n_slices
   return per_slice >= 192 || tiles >= 192 || row_bytes >= 8192 ? 256 : 128;
 }
 
+// Row blocks for tiled e4m3 weights: by the rule above where that kernel runs (`x_bytes` as in gemm_limits.h).  The other kernel walks a
+// block of 256 rows in two passes, which pays from 1024 rows per slice on (8 slices, K 4096, N 8192: 512 rows 147 us with either, 1024
+// 296 with blocks of 128 against 289 with 256; 2048 rows, N 28672: 1930 against 1853, K 14336, N 4096: 846 against 819 us) and costs up to twice
+// the time below (256 rows, K 14336: 133 against 273 us; 300 slices of 256 rows, K and N 2048: 474 against 544 us).
+int64_t fp8_block_m(int64_t rows, uint32_t x_bytes, int64_t K, int64_t N, int64_t n_slices) {
+  if (tk::dma_runs(x_bytes, n_slices, (N + 31) / 32 * ((K + 255) / 256) * 8192)) return dma_block_m(rows, K, N, n_slices);
+  return rows >= 1024 * n_slices ? 256 : 128;
+}
+
 // Row blocks for tiled MXFP4 weights with more routed rows than the decode kernel is made for.  32 = the streaming kernel, faster
 // than the decode kernel's 16-row blocks from 160 rows on (128 slices, K 2880, N 5760: 300 tokens 210 against 232 us, 32 slices,
 // 200 tokens 28 against 57 us) and than the prefill kernel's 64-row blocks up to about 20 rows per slice (18: 245 against 258 us,
 // 31: 331 against 290 us); those give way to the larger ones at about 56 (47: 340 against 372 us, 62: 410 against 399 us).
+// (For calls that the streaming kernel takes: x as a buffer resource, slices in registers, no row or column scales.)
 int64_t mxfp4_block_m(int64_t rows, int64_t n_slices, int64_t otherwise) {
   int64_t per_slice = rows / std::max<int64_t>(n_slices, 1);
   return per_slice <= 20 ? 32 : per_slice <= 56 ? 64 : std::max<int64_t>(otherwise, 128);
@@ -175,10 +186,10 @@ int64_t mxfp4_block_m(int64_t rows, int64_t n_slices, int64_t otherwise) {
 // 250 (16 slices) 258 against 246, 1024 754 against 716 us.  MXFP8 rows: 64 per slice 444 against 451 us, 112 537 against 503, 162 932
 // against 767; past one tile per slice the smaller blocks, whose tiles of a slice share weights in L2, win (203 910 against 955, 250
 // 143 against 153 us), until a workgroup has several tiles of a slice (512: 256 us either way, 1024 469 against 440 us).
-// The wide kernel takes four stages of K (the activation scales sixteen blocks), 256 slices and x below 2 GiB.
-int64_t wide_block_m(int64_t rows, int64_t n_slices, int64_t K, int64_t x_bytes, bool mx8) {
+// The wide kernel takes four stages of K (the activation scales sixteen blocks), slices in registers and x as a buffer resource.
+int64_t wide_block_m(int64_t rows, int64_t n_slices, int64_t K, uint32_t x_bytes, bool mx8) {
   n_slices = std::max<int64_t>(n_slices, 1);
-  if (K <= (mx8 ? 511 : 384) || n_slices > 256 || x_bytes >= int64_t(1) << 31) return rows <= 144 * n_slices ? 256 : 128;
+  if (K <= (mx8 ? 511 : 384) || n_slices > tk::kDmaSlices || !x_bytes) return rows <= 144 * n_slices ? 256 : 128;
   if (rows <= 80 * n_slices) return 128;
   return !mx8 || rows <= 176 * n_slices || rows >= 640 * n_slices ? 256 : 128;
 }
@@ -366,15 +377,15 @@ PyObject* run_gemm(PyObject* const* v) {
 
   // ---- row blocks
   int64_t block_m = default_block_m(M, n_slices);
-  const bool short_x = a_rows * a_stride < (int64_t(1) << 30);
+  const uint32_t x_bytes = tk::x_extent(a_rows, a_stride, K, a->element_size());
   if (tiled_fp8) {
-    block_m = dma_block_m(M, K, N, n_slices);
+    block_m = fp8_block_m(M, x_bytes, K, N, n_slices);
   } else if (mx_act) {
-    block_m = wide_block_m(M, n_slices, K, a_rows * a_stride, true);
+    block_m = wide_block_m(M, n_slices, K, x_bytes, true);
   } else if (tiled) {
-    if (M > 256 && short_x && n_slices <= 256 && !x_row && !w_col) block_m = mxfp4_block_m(M, n_slices, block_m);
-    if (block_m == 128) block_m = wide_block_m(M, n_slices, K, a_rows * a_stride * 2, false);
-  } else if (block_m > 16 && tk::dma_runs_16bit(tk::x_extent(a_rows, a_stride, K, 2), n_slices, K, N, w->stride(2))) {
+    if (M > 256 && x_bytes && n_slices <= tk::kDmaSlices && !x_row && !w_col) block_m = mxfp4_block_m(M, n_slices, block_m);
+    if (block_m == 128) block_m = wide_block_m(M, n_slices, K, x_bytes, false);
+  } else if (block_m > 16 && tk::dma_runs_16bit(x_bytes, n_slices, K, N, w->stride(2))) {
     block_m = dma_block_m(M, 2 * K, N, n_slices);
   }
   if (tiled && block_m >= 64 && !mx_act && n_out % 8) return none();  // (through a padded buffer)
@@ -713,26 +724,38 @@ PyObject* call(PyObject*, PyObject* const* args, Py_ssize_t given) {
   END_HANDLE_TH_ERRORS
 }
 
-PyObject* rule(PyObject* const* v, bool dma) {
-  const int64_t a = PyLong_AsLongLong(v[0]), b = PyLong_AsLongLong(v[1]), c = PyLong_AsLongLong(v[2]), d = dma ? PyLong_AsLongLong(v[3]) : 0;
+// The rules and conditions for the general host path, on integers.
+template <size_t n>
+std::array<int64_t, n> integers(PyObject* const* v) {
+  std::array<int64_t, n> a;
+  for (size_t i = 0; i < n; ++i) a[i] = PyLong_AsLongLong(v[i]);
   if (PyErr_Occurred()) throw PyError();
-  return PyLong_FromLongLong(dma ? dma_block_m(a, b, c, d) : mxfp4_block_m(a, b, c));
+  return a;
+}
+PyObject* rule_x_extent(PyObject* const* v) {
+  const auto [rows, stride, K, itemsize] = integers<4>(v);
+  return PyLong_FromUnsignedLong(tk::x_extent(rows, stride, K, itemsize));
+}
+PyObject* rule_dma_16bit(PyObject* const* v) {
+  const auto [x_bytes, n_slices, K, N, w_stride_n] = integers<5>(v);
+  return PyBool_FromLong(tk::dma_runs_16bit(uint32_t(x_bytes), n_slices, K, N, w_stride_n));
+}
+PyObject* rule_dma(PyObject* const* v) {
+  const auto [rows, row_bytes, N, n_slices] = integers<4>(v);
+  return PyLong_FromLongLong(dma_block_m(rows, row_bytes, N, n_slices));
+}
+PyObject* rule_fp8(PyObject* const* v) {
+  const auto [rows, x_bytes, K, N, n_slices] = integers<5>(v);
+  return PyLong_FromLongLong(fp8_block_m(rows, uint32_t(x_bytes), K, N, n_slices));
+}
+PyObject* rule_mxfp4(PyObject* const* v) {
+  const auto [rows, n_slices, otherwise] = integers<3>(v);
+  return PyLong_FromLongLong(mxfp4_block_m(rows, n_slices, otherwise));
 }
 PyObject* rule_wide(PyObject* const* v) {
-  int64_t a[5];
-  for (int i = 0; i < 5; ++i) a[i] = PyLong_AsLongLong(v[i]);
-  if (PyErr_Occurred()) throw PyError();
-  return PyLong_FromLongLong(wide_block_m(a[0], a[1], a[2], a[3], a[4] != 0));
+  const auto [rows, n_slices, K, x_bytes, mx8] = integers<5>(v);
+  return PyLong_FromLongLong(wide_block_m(rows, n_slices, K, uint32_t(x_bytes), mx8 != 0));
 }
-// (rows of x, their stride, K, N, stride of a weight column, slices) -> does the memory-to-LDS kernel run on strided 16-bit weights?
-PyObject* rule_dma_16bit(PyObject* const* v) {
-  int64_t a[6];
-  for (int i = 0; i < 6; ++i) a[i] = PyLong_AsLongLong(v[i]);
-  if (PyErr_Occurred()) throw PyError();
-  return PyBool_FromLong(tk::dma_runs_16bit(tk::x_extent(a[0], a[1], a[2], 2), a[5], a[2], a[3], a[4]));
-}
-PyObject* rule_dma(PyObject* const* v) { return rule(v, true); }
-PyObject* rule_mxfp4(PyObject* const* v) { return rule(v, false); }
 
 // bind(dict): the addresses of the entry points (integers) and the Python objects above
 PyObject* bind(PyObject*, PyObject* dict) {
@@ -780,8 +803,10 @@ PyMethodDef methods[] = {
     METHOD("mx_upcast", run_mx_upcast, 4),
     METHOD("ragged_k", run_ragged_k, 4),
     METHOD("decode_layer", run_decode_layer, 13),
-    METHOD("dma_runs_16bit", rule_dma_16bit, 6),
+    METHOD("x_extent", rule_x_extent, 4),
+    METHOD("dma_runs_16bit", rule_dma_16bit, 5),
     METHOD("dma_block_m", rule_dma, 4),
+    METHOD("fp8_block_m", rule_fp8, 5),
     METHOD("mxfp4_block_m", rule_mxfp4, 3),
     METHOD("wide_block_m", rule_wide, 5),
     {nullptr, nullptr, 0, nullptr},

@@ -751,26 +751,27 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
         g = g.contiguous()
         d.gammas, d.gammas_dtype = g.data_ptr(), nt.TORCH_TO_TK[g.dtype]
         keep.append(g)
+    x_bytes = nt.rules().x_extent(a_rows, a_stride, K, a.itemsize)  # 0: rows that the buffer-resource kernels do not take
     if tiled_fp8:
-        block_m = forced if forced in (128, 256) else 128 if forced is not None else nt.rules().dma_block_m(M, K, N, n_slices)
+        block_m = forced if forced in (128, 256) else 128 if forced is not None else nt.rules().fp8_block_m(M, x_bytes, K, N, n_slices)
     elif mx_act or (tiled and mx_out_fused):
         # the tile shapes that take MXFP8 activations / have an MX-output epilogue
         if forced is None and is_ragged:
-            block_m = nt.rules().wide_block_m(M, n_slices, K, a_rows * a_stride, 1) if mx_act else 256 if M <= 144 * n_slices else 128
+            block_m = nt.rules().wide_block_m(M, n_slices, K, x_bytes, 1) if mx_act else 256 if M <= 144 * n_slices else 128
         else:
             block_m = 256 if forced == 256 else 128
     elif tiled:
         if extras:
             block_m = min(block_m, 32)  # the decode kernel carries the shared epilogue; the prefill kernels do not take these options
         elif forced is None and is_ragged:
-            if (M > 256 and a_rows * a_stride < 1 << 30 and n_slices <= 256 and a_ts is None and b_ts is None
+            if (M > 256 and x_bytes and n_slices <= 256 and a_ts is None and b_ts is None
                     and a_ragged_metadata.expected_slice_size is None):
                 block_m = nt.rules().mxfp4_block_m(M, n_slices, block_m)
             if block_m == 128:
-                block_m = nt.rules().wide_block_m(M, n_slices, K, a_rows * a_stride * 2, 0)
+                block_m = nt.rules().wide_block_m(M, n_slices, K, x_bytes, 0)
     elif w_dtype in (_BF16, _F16):
         if block_m > 16:
-            if not nt.rules().dma_runs_16bit(a_rows, a_stride, K, N, w.stride(-1), n_slices):
+            if not nt.rules().dma_runs_16bit(x_bytes, n_slices, K, N, w.stride(-1)):
                 block_m = min(block_m, 128)  # (the general kernel's largest)
             elif forced is None:
                 block_m = nt.rules().dma_block_m(M, 2 * K, N, n_slices)
