@@ -146,6 +146,23 @@ def test_row_blocks_of_256_with_16_bit_weights_are_refused_where_no_kernel_has_t
         assert "block_m 256" in nt.last_error()
 
 
+def test_inline_assembly_tells_the_compiler_about_m0():
+    """Memory-to-LDS transfers read m0: as an operand of the statement, which the compiler then keeps track of.  No statement writes m0 behind
+    its back."""
+    csrc = os.path.join(ROOT, "triton_amd", "csrc")
+    transfers = 0
+    for name in sorted(os.listdir(csrc)):
+        if not name.endswith((".h", ".hip")):
+            continue
+        for m in re.finditer(r"\basm\s+volatile\s*\((.*?)\);", open(os.path.join(csrc, name)).read(), flags=re.S):
+            text = m.group(1)
+            assert not re.search(r"\bs_\w+\s+m0\b", text) or '"m0"' in text, (name, text)
+            if re.search(r"buffer_load_\w+[^\n]*\blds\b", text):
+                transfers += 1
+                assert '"{m0}"' in text, (name, text)
+    assert transfers
+
+
 def test_status_to_exception_mapping():
     with pytest.raises(ValueError):
         nt.check(nt.TK_ERR_INVALID, "bad")
