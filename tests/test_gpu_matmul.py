@@ -603,6 +603,21 @@ def test_idle_sms_keeps_results(mods, device, idle):
     assert torch.equal(base, y)
 
 
+@pytest.mark.parametrize("idle", [None, 0, 3, 3.0, -1, True])
+def test_matmul_set_idle_sms(mods, device, idle):
+    """The process-wide setting, with None for "use all" and whatever else counts as a number."""
+    mm, _, tensor = mods
+    g = torch.Generator().manual_seed(7)
+    x, w = torch.randn((300, 64), generator=g).to(torch.bfloat16).to(device), torch.randn((2, 96, 64), generator=g).to(torch.bfloat16).to(device)
+    md = tensor.make_ragged_tensor_metadata(torch.tensor([100, 200], dtype=torch.int32, device=device), 300)
+    base = mm.matmul(x, w.transpose(1, 2), None, md)
+    mm.matmul_set_idle_sms(idle)
+    try:
+        assert torch.equal(base, mm.matmul(x, w.transpose(1, 2), None, md))
+    finally:
+        mm.matmul_set_idle_sms(0)
+
+
 def test_standalone_swiglu_with_routing_data(mods, device):
     """`swiglu(a, alpha, pc, routing_data=rdata)` bounds the rows by the routed row count read on the device
     (swiglu.py:53-55 of the reference): rows past it are left unwritten, the rest match the oracle."""

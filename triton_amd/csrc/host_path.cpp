@@ -290,9 +290,13 @@ PyObject* run_gemm(PyObject* const* v) {
     gammas = tensor_of(gam_o);
     if (!gammas || !gammas->is_contiguous() || !f32_or_bf16(*gammas)) return none();
   }
-  const long combine_k = is_none(v[10]) ? 0 : PyLong_AsLong(v[10]);
-  const long idle = PyLong_AsLong(v[11]);
-  if (PyErr_Occurred()) throw PyError();
+  // (whole numbers; the general path says what it makes of anything else, None and floats among them)
+  if ((!is_none(v[10]) && !PyLong_Check(v[10])) || !PyLong_Check(v[11])) return none();
+  const long combine_k = is_none(v[10]) ? 0 : PyLong_AsLong(v[10]), idle = PyLong_AsLong(v[11]);
+  if (PyErr_Occurred()) {
+    PyErr_Clear();
+    return none();
+  }
 
   // ---- weights
   int64_t kn[2];
