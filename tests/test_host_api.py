@@ -305,3 +305,23 @@ def test_row_blocks_follow_the_kernel_that_runs(gemm_calls, kind, n_slices, per_
     for stride, block_m in ((k, want), (0, overlapping), (k - 16, overlapping)):
         matmul(torch.zeros(rows * k, dtype=dtype).as_strided((rows, k), (stride, 1)), w, None, md, precision_config=pc)
         assert (gemm_calls[-1]["x_stride_m"], gemm_calls[-1]["block_m"]) == (stride, block_m)
+
+
+@pytest.mark.parametrize("kind, block_m", [("bf16", 16), ("bf16", 32), ("bf16", 64), ("bf16", 128), ("mxfp4", 16), ("mxfp4", 64), ("mxfp4", 128), ("fp8", 128)])
+def test_a_callers_row_block_is_the_one_that_runs(gemm_calls, kind, block_m):
+    # named by a constraint or by flags of the caller's own, where the rules would take 256
+    import dataclasses
+    from triton_amd.matmul import PrecisionConfig, matmul, scoped_opt_flags, scoped_opt_flags_constraints
+    n_slices, rows, k, n = 4, 1000, 512, 64
+    w, s = (torch.zeros((n_slices, n, k), dtype=torch.bfloat16).transpose(1, 2), None) if kind == "bf16" else _tiled(kind, n_slices, k, n)
+    x = torch.zeros((rows, k), dtype=torch.float8_e4m3fn if kind == "fp8" else torch.bfloat16)
+    pc, md = PrecisionConfig(b_mx_scale=s, out_dtype=torch.bfloat16), _metadata(n_slices, rows)
+    matmul(x, w, None, md, precision_config=pc)
+    assert gemm_calls[-1]["block_m"] == 256
+    with scoped_opt_flags_constraints({"block_m": block_m}):
+        matmul(x, w, None, md, precision_config=pc)
+    assert gemm_calls[-1]["block_m"] == block_m
+    flags = dataclasses.replace(of.make_opt_flags(torch.bfloat16, torch.bfloat16, torch.bfloat16, pc, 1, rows, n, k, md), block_m=block_m)
+    with scoped_opt_flags(flags):
+        matmul(x, w, None, md, precision_config=pc)
+    assert gemm_calls[-1]["block_m"] == block_m

@@ -32,7 +32,7 @@ from typing import Callable
 import torch
 
 from . import _native as nt
-from .matmul_details.opt_flags import (InapplicableConstraint, OptFlags, _get_idle_sms, _get_opt_flags_constraints,  # noqa: F401
+from .matmul_details.opt_flags import (InapplicableConstraint, OptFlags, _get_idle_sms, block_m_is_forced,  # noqa: F401
                                         default_block_m, make_opt_flags, scoped_opt_flags, scoped_opt_flags_constraints, set_idle_sms,
                                         unconstrained)
 from .numerics import InFlexData, OutFlexData
@@ -654,7 +654,7 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
     else:
         opt_flags = make_opt_flags(torch_dtype_to_dtype(out_dtype), torch_dtype_to_dtype(a_dtype),
                                    FP4 if fp4 else torch_dtype_to_dtype(w_dtype if strided else _E4M3), precision_config, 1, M, N, K, a_ragged_metadata, epilogue_reduction_n=reduction_n)
-        block_m, forced, idle = opt_flags.block_m, _get_opt_flags_constraints().get("block_m"), opt_flags.idle_sms
+        block_m, forced, idle = opt_flags.block_m, opt_flags.block_m if block_m_is_forced() else None, opt_flags.idle_sms
     if M * N == 0:
         return c
     if a.stride(1) != 1:

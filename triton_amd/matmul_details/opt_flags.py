@@ -96,6 +96,11 @@ def unconstrained() -> bool:
     return not _opt_flags_constraints.get() and _opt_flags.get() is None
 
 
+def block_m_is_forced() -> bool:
+    """The caller names the row block, by a constraint or by flags of its own."""
+    return _opt_flags.get() is not None or bool(_get_opt_flags_constraints().get("block_m"))
+
+
 def update_opt_flags_constraints(constraints: dict):
     updated = dict(_get_opt_flags_constraints())
     updated.update(constraints)
