@@ -238,3 +238,22 @@ def test_topk_backward(device, T, E, k, dt, apply_softmax):
     (sm.vals.float() * dy.to(device).float()).sum().backward()
     full = ort.topk_backward(x, indx, dy, apply_softmax)
     assert torch.allclose(xg.grad.cpu().float(), full.float(), **tol)
+
+
+@pytest.mark.parametrize("tokens, e, k", [(1, 16, 2), (300, 128, 4), (4096, 700, 8)])
+@pytest.mark.parametrize("native", [True, False])
+def test_results_that_are_kept_hold_no_scratch_memory(device, monkeypatch, tokens, e, k, native):
+    """A kept (or saved) histogram is its E words; the permutations and the gather index are three times T * k words; the metadata is its own."""
+    from triton_amd import _native as nt
+    from triton_amd.legacy import routing
+    if not native:
+        monkeypatch.setattr(nt, "host", lambda: None)
+    rd, gather, scatter = routing(torch.randn((tokens, e), device=device), k)
+    r, md = tokens * k, rd.expt_data
+    words = lambda t: t.untyped_storage().nbytes() // 4
+    assert words(rd.expt_hist) == e and md.slice_sizes is rd.expt_hist
+    for t in (gather.src_indx, gather.dst_indx, scatter.src_indx, scatter.dst_indx, rd.token_indx):
+        assert words(t) == 3 * r
+    blocks = 6 * (e + 1) + 5 * md.block_schedule_data.shape[1]
+    for t in (md.slice_offs, md.block_offs_data, md.block_schedule_data):
+        assert words(t) <= blocks

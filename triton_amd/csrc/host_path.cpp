@@ -466,25 +466,26 @@ PyObject* run_route(PyObject* const* v) {
   if (T == 0 || E == 0 || E >= 32768 || k < 1 || k > 32 || (k & (k - 1))) return none();
   auto stream = stream_of(*logits);
   if (!stream) return none();
-  // [E] histogram, the two permutations, [R] gather index, [E + 1] row offsets, [5, E + 1] block offsets, [5, width] schedules
-  // (the schedules' readers load single words), and the kernels' scratch, which starts on 16 bytes
-  const int64_t width = n_blocks(E, R, 16), used = E + 3 * R + 6 * (E + 1) + 5 * width, start = (used + 3) / 4 * 4;
-  const int64_t scratch = (std::max<int64_t>(1, B.route_workspace_bytes(int32_t(T), int32_t(E))) + 3) / 4;
-  Tensor buf = empty({start + scratch}, ScalarType::Int, *logits);
+  // Allocations by what a caller keeps or saves together: the [E] histogram by itself, the two permutations with the [R] gather index, and
+  // the metadata ([E + 1] row offsets, [5, E + 1] block offsets, [5, width] schedules, whose readers load single words).  The kernels'
+  // scratch ends with this call.
+  const int64_t width = n_blocks(E, R, 16), scratch = std::max<int64_t>(1, B.route_workspace_bytes(int32_t(T), int32_t(E)));
+  Tensor hist_t = empty({E}, ScalarType::Int, *logits), perm = empty({3 * R}, ScalarType::Int, *logits),
+         meta = empty({6 * (E + 1) + 5 * width}, ScalarType::Int, *logits), work = empty({scratch}, ScalarType::Byte, *logits);
   Tensor vals = empty({T, k}, t, *logits), indx = empty({T, k}, ScalarType::Short, *logits), gammas = empty({R}, t, *logits);
-  int32_t* base = static_cast<int32_t*>(buf.data_ptr());
-  const int64_t col = E, row = col + R, gat = row + R, offs = gat + R, blocks = offs + E + 1, sched = blocks + 5 * (E + 1);
+  int32_t *perms = static_cast<int32_t*>(perm.data_ptr()), *metas = static_cast<int32_t*>(meta.data_ptr());
+  const int64_t row = R, gat = 2 * R, blocks = E + 1, sched = blocks + 5 * (E + 1);
   tk_route_desc d{};
   d.logits = logits->data_ptr(), d.logits_dtype = dtype_code(t), d.logits_stride_m = logits->stride(0);
   d.n_tokens = int32_t(T), d.n_rows = -1, d.n_experts = int32_t(E), d.k = int32_t(k), d.apply_softmax = softmax;
   d.vals = vals.data_ptr(), d.indx = indx.data_ptr(), d.indx_dtype = TK_I16, d.gammas = gammas.data_ptr();
-  d.col_sum = base, d.col_sorted_indx = base + col, d.row_sorted_indx = base + row, d.gather_indx = base + gat;
-  d.slice_offs = base + offs, d.block_offs = base + blocks, d.block_offs_stride = E + 1;
-  d.block_schedule = base + sched, d.block_schedule_stride = width, d.max_n_blocks = int32_t(width);
-  d.workspace = base + start;
+  d.col_sum = static_cast<int32_t*>(hist_t.data_ptr()), d.col_sorted_indx = perms, d.row_sorted_indx = perms + row, d.gather_indx = perms + gat;
+  d.slice_offs = metas, d.block_offs = metas + blocks, d.block_offs_stride = E + 1;
+  d.block_schedule = metas + sched, d.block_schedule_stride = width, d.max_n_blocks = int32_t(width);
+  d.workspace = work.data_ptr();
   launch([&] { return B.route(&d, *stream); });
-  Ref hist(part_of(buf, 0, {E})), col_o(part_of(buf, col, {R})), row_o(part_of(buf, row, {R})), gat_o(part_of(buf, gat, {R})),
-      offs_o(part_of(buf, offs, {E + 1})), blocks_o(part_of(buf, blocks, {5, E + 1})), sched_o(part_of(buf, sched, {5, width})),
+  Ref hist(THPVariable_Wrap(hist_t)), col_o(part_of(perm, 0, {R})), row_o(part_of(perm, row, {R})), gat_o(part_of(perm, gat, {R})),
+      offs_o(part_of(meta, 0, {E + 1})), blocks_o(part_of(meta, blocks, {5, E + 1})), sched_o(part_of(meta, sched, {5, width})),
       vals_o(THPVariable_Wrap(vals)), indx_o(THPVariable_Wrap(indx)), gam_o(THPVariable_Wrap(gammas)), e_o(PyLong_FromLongLong(E));
   for (PyObject* o : {hist.p, col_o.p, row_o.p, gat_o.p, offs_o.p, blocks_o.p, sched_o.p, vals_o.p, indx_o.p, gam_o.p, e_o.p})
     if (!o) throw PyError();
