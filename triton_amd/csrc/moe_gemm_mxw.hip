@@ -23,9 +23,9 @@
 namespace tk {
 namespace {
 
-template <bool MX8, int NWAVES>
+template <bool MX8>
 struct MxwCfg {
-  static constexpr int MFW = 5, NW = NWAVES;                  // row fragments, waves (each all rows x 64 columns)
+  static constexpr int MFW = 5, NW = 8;                       // row fragments, waves (each all rows x 64 columns)
   static constexpr int BM = MFW * 32, BN = NW * 64;
   static constexpr int ROW = MX8 ? 128 : 256;            // bytes of a row and stage (128 k)
   static constexpr int RPT = 1024 / ROW;                 // rows of a transfer
@@ -42,9 +42,9 @@ struct MxwCfg {
   static constexpr int LDS = RINGS + 2 * (SIDE + OPERANDS) + LISTS;
 };
 
-template <bool MX8, int NWAVES, bool SWIGLU, bool MXOUT>
-__global__ __launch_bounds__(NWAVES * 64, NWAVES / 4) void moe_gemm_mxw_kernel(const GemmParams p) {
-  typedef MxwCfg<MX8, NWAVES> C;
+template <bool MX8, bool SWIGLU, bool MXOUT>
+__global__ __launch_bounds__(MxwCfg<MX8>::NW * 64, 2) void moe_gemm_mxw_kernel(const GemmParams p) {
+  typedef MxwCfg<MX8> C;
   constexpr int MFW = C::MFW, AI = C::AI;
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -371,9 +371,9 @@ __global__ __launch_bounds__(NWAVES * 64, NWAVES / 4) void moe_gemm_mxw_kernel(c
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no transfer into this workgroup's LDS is left behind
 }
 
-template <bool MX8, int NWAVES>
+template <bool MX8>
 int32_t launch_cfg(const GemmParams& p, bool swiglu, bool mx_out, hipStream_t st) {
-  typedef MxwCfg<MX8, NWAVES> C;
+  typedef MxwCfg<MX8> C;
   static_assert(C::LDS <= 160 * 1024, "one workgroup per CU");
   GemmParams q = p;
   q.grid_n = (int)cdiv(p.N, C::BN);
@@ -388,18 +388,15 @@ int32_t launch_cfg(const GemmParams& p, bool swiglu, bool mx_out, hipStream_t st
     return check_launch("moe_gemm_mxw_kernel");
   };
   if constexpr (MX8) {
-    if (mx_out) return swiglu ? launch(moe_gemm_mxw_kernel<true, NWAVES, true, true>) : launch(moe_gemm_mxw_kernel<true, NWAVES, false, true>);
+    if (mx_out) return swiglu ? launch(moe_gemm_mxw_kernel<true, true, true>) : launch(moe_gemm_mxw_kernel<true, false, true>);
   }
-  return swiglu ? launch(moe_gemm_mxw_kernel<MX8, NWAVES, true, false>) : launch(moe_gemm_mxw_kernel<MX8, NWAVES, false, false>);
+  return swiglu ? launch(moe_gemm_mxw_kernel<MX8, true, false>) : launch(moe_gemm_mxw_kernel<MX8, false, false>);
 }
 
 }  // namespace
 
 int32_t gemm_launch_mxw(const GemmParams& p, bool mx_act, bool swiglu, bool mx_out, hipStream_t st) {
-#ifndef MXW_NW
-#define MXW_NW 8
-#endif
-  return mx_act ? launch_cfg<true, MXW_NW>(p, swiglu, mx_out, st) : launch_cfg<false, MXW_NW>(p, swiglu, false, st);
+  return mx_act ? launch_cfg<true>(p, swiglu, mx_out, st) : launch_cfg<false>(p, swiglu, false, st);
 }
 
 }  // namespace tk
