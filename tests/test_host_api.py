@@ -325,3 +325,20 @@ def test_a_callers_row_block_is_the_one_that_runs(gemm_calls, kind, block_m):
     with scoped_opt_flags(flags):
         matmul(x, w, None, md, precision_config=pc)
     assert gemm_calls[-1]["block_m"] == block_m
+
+
+def test_16_bit_tiles_at_256_rows_are_the_kernels_own(gemm_calls):
+    # 256 x 256 with eight waves; the 128 x 128 tile stays accepted beside block_m = 256 and is then the one that runs
+    from triton_amd.matmul import matmul, scoped_opt_flags_constraints
+    n_slices, rows, k, n = 4, 1000, 512, 64
+    w, x, md = torch.zeros((n_slices, n, k), dtype=torch.bfloat16).transpose(1, 2), torch.zeros((rows, k), dtype=torch.bfloat16), _metadata(n_slices, rows)
+    for constraints, block_m, block_n in (({}, 256, 256), ({"block_n": 256}, 256, 256), ({"block_n": 256, "num_warps": 8, "block_k": 64}, 256, 256),
+                                          ({"block_n": 128}, 128, 128), ({"block_k": 128, "num_warps": 4}, 128, 128)):
+        with scoped_opt_flags_constraints({"block_m": 256, **constraints}):
+            f = of.make_opt_flags(None, None, torch.bfloat16, None, 1, rows, n, k, md)
+            assert (f.block_m, f.block_n) == (block_m, block_n)
+            matmul(x, w, None, md)
+        assert gemm_calls[-1]["block_m"] == block_m
+    for constraints in ({"block_n": 64}, {"block_n": 256, "num_warps": 4}, {"block_n": 128, "block_k": 64}):
+        with scoped_opt_flags_constraints({"block_m": 256, **constraints}), pytest.raises(of.InapplicableConstraint):
+            of.make_opt_flags(None, None, torch.bfloat16, None, 1, rows, n, k, md)

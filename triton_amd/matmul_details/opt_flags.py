@@ -1,19 +1,24 @@
 """Tile selection for the ragged GEMM and the constraint-scoping API
 (mirrors the user interface of `triton_kernels/matmul_details/opt_flags.py:20-38,482-603`).
 
-The HIP GEMM is compiled for a fixed set of tile shapes, selected by `block_m` (rows of one expert per
-workgroup) and the weight format:
+The HIP GEMM is compiled for a fixed set of tile shapes.  A caller names one by `block_m`, the rows of an expert per
+row block; `block_n`, `block_k` and `num_warps` constraints are checked against this table (narrow = 4- and 8-bit weights):
 
-    block_m   mxfp4 / fp8 weights        bf16 weights           use
-              block_n  block_k  waves    block_n  block_k
-      16        128      256      4        128      128         decode: a few rows per expert
-      32        128      256      4        128      128
-      64        256      128      4        128      128
-     128        256      128      4        128      128         prefill: ~128 rows per expert
-     256        256      128      4        256       64         pre-tiled MXFP4: a whole expert (<= 160 rows) per tile; 16-bit and
-                                                                tiled e4m3 weights: from about 128 rows per expert on
+    block_m   narrow weights             16-bit weights             use
+              block_n  block_k  waves    block_n  block_k  waves
+      16        128      256      4        128      128      4      decode: a few rows per expert
+      32        128      256      4        128      128      4
+      64        256      128      4        128      128      4
+     128        256      128      4        128      128      4      prefill
+     256        256      128      4        256       64      8      prefill, many rows per expert
 
-so only `block_m` can be forced; `block_n`, `block_k` and `num_warps` constraints must match the table.
+The kernel that runs follows from `block_m`, the weight format and the operands, and may walk the row block in a tile
+of its own: tiled MXFP4 weights at 32 the streaming kernel (32 x 256; elsewhere the decode kernel), at 256 the
+wide kernel (160 x 512, eight waves; elsewhere one with 256 columns); tiled e4m3 and 16-bit weights at 128 and 256 the
+memory-to-LDS kernel (128 x 128 with four waves and 256 x 256 with eight, 128 bytes of K a stage), 16-bit weights elsewhere the
+general kernel, whose largest row block is 128.  A call with 16-bit weights that names `block_m=256` together with the 128 x 128
+tile (`block_n=128`, `block_k=128` or `num_warps=4`) gets that tile, with row blocks of 128.
+
 `split_k > 1` and `is_persistent=True` cannot be honoured and raise `InapplicableConstraint`, which is
 what the reference's own tests skip on AMD (tests/test_matmul.py:377-383).
 """
@@ -28,17 +33,22 @@ TILE_TABLE = {  # narrow (4-bit / 8-bit) weights
     32: dict(block_n=128, block_k=256, num_warps=4),
     64: dict(block_n=256, block_k=128, num_warps=4),
     128: dict(block_n=256, block_k=128, num_warps=4),
-    256: dict(block_n=256, block_k=128, num_warps=4),  # pre-tiled MXFP4 weights only: one tile per expert of <= 160 rows
+    256: dict(block_n=256, block_k=128, num_warps=4),
 }
-TILE_TABLE_16BIT = {bm: dict(block_n=128, block_k=128, num_warps=4) for bm in TILE_TABLE}
+TILE_TABLE_16BIT = {bm: dict(block_n=128, block_k=128, num_warps=4) for bm in (16, 32, 64, 128)}
+TILE_TABLE_16BIT[256] = dict(block_n=256, block_k=64, num_warps=8)
+
+
+def _is_16bit(rhs_dtype) -> bool:
+    bits = getattr(rhs_dtype, "bitwidth", None)
+    if bits is None:
+        bits = getattr(rhs_dtype, "itemsize", 1) * 8
+    return bits >= 16
 
 
 def tile_for(block_m: int, rhs_dtype=None) -> dict:
     """The compiled tile for `block_m` and a weight dtype (torch dtype, package dtype or None = narrow)."""
-    bits = getattr(rhs_dtype, "bitwidth", None)
-    if bits is None:
-        bits = getattr(rhs_dtype, "itemsize", 1) * 8
-    return (TILE_TABLE_16BIT if bits >= 16 else TILE_TABLE)[block_m]
+    return (TILE_TABLE_16BIT if _is_16bit(rhs_dtype) else TILE_TABLE)[block_m]
 
 
 @dataclass
@@ -182,10 +192,12 @@ def make_opt_flags(out_dtype, lhs_dtype, rhs_dtype, precision_config, batch_size
     block_m = constraints.get("block_m") or default_block_m(m, ragged_metadata)
     if block_m not in TILE_TABLE:
         raise InapplicableConstraint(f"block_m={block_m} is not one of {sorted(TILE_TABLE)}")
+    wanted = {key: constraints[key] for key in ("block_n", "block_k", "num_warps") if constraints.get(key) is not None}
     tile = tile_for(block_m, rhs_dtype)
-    for key in ("block_n", "block_k", "num_warps"):
-        want = constraints.get(key)
-        if want is not None and want != tile[key]:
+    if block_m == 256 and _is_16bit(rhs_dtype) and wanted and wanted.items() <= TILE_TABLE_16BIT[128].items():
+        block_m, tile = 128, TILE_TABLE_16BIT[128]
+    for key, want in wanted.items():
+        if want != tile[key]:
             raise InapplicableConstraint(f"{key}={want} does not match the compiled tile for block_m={block_m} ({tile[key]})")
     return OptFlags(
         block_m=block_m,
