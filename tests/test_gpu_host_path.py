@@ -76,16 +76,64 @@ def _weights(kind, e, k, n, g, device):
             convert_layout(wrap_torch_tensor(s), L.make_default_matmul_mxfp4_w_scale_layout(mx_axis=1)))
 
 
-@pytest.mark.parametrize("kind", ["bf16", "fp16", "fp8", "mxfp4", "mxfp8", "mxfp8_out"])
-@pytest.mark.parametrize("tokens", [1, 40, 200, 500, 1200])
-def test_layer_gemms(device, monkeypatch, kind, tokens):
-    """16 experts, 2 choices: 2 to 2400 rows, so that every row block is chosen; with activation and gather, scatter and combine."""
+@pytest.fixture
+def gemm_descriptors(monkeypatch):
+    """What the GEMM entry of the library gets from either host path, recorded on the way to it."""
+    import ctypes
+
+    from triton_amd import _native as nt
+    real, seen = nt.lib(), []
+
+    @ctypes.CFUNCTYPE(ctypes.c_int32, ctypes.POINTER(nt.GemmDesc), ctypes.c_void_p)
+    def entry(d, stream):
+        seen.append({name: getattr(d.contents, name) for name, _ in nt.GemmDesc._fields_})
+        return real.tk_moe_gemm(d, stream)
+
+    class Library:
+        tk_moe_gemm = entry
+
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+    with monkeypatch.context() as m:
+        m.setattr(nt, "_lib", Library())
+        m.setattr(nt, "_host", None)  # bound again, to this library
+        yield seen
+    nt._host = None
+    nt.host()
+
+
+def _same_descriptors(fast, slow):
+    """Every number, and every pointer to the caller's operands; buffers made by the call are there or not."""
+    made = {"y", "combine_out"}
+    for name, value in fast.items():
+        assert (bool(value), bool(slow[name])) == (True, True) if name in made and value else value == slow[name], (name, value, slow[name])
+
+
+# 16 experts, 2 choices.  The row blocks that the rules choose, and with them every kernel that a layer can meet: 16-bit weights the general
+# kernel (16) and both tiles of the memory-to-LDS one, e4m3 those two, MXFP4 the decode (16), streaming (32), prefill (64, 128) and wide
+# (256) kernels, MXFP8 activations the prefill and the wide kernel (with K of 256 and 320 the form of the prefill kernel for a short K).
+SMALL, LARGE = (256, 320), (512, 544)
+LAYERS = [
+    *[(kind, tokens, dims, bm) for kind in ("bf16", "fp16") for tokens, dims, bm in ((1, SMALL, 16), (40, LARGE, 16), (200, SMALL, 128), (1600, LARGE, 256))],
+    *[("fp8", tokens, dims, bm) for tokens, dims, bm in ((1, SMALL, 128), (40, LARGE, 128), (1600, LARGE, 256))],
+    *[("mxfp4", tokens, dims, bm) for tokens, dims, bm in ((1, SMALL, 16), (40, LARGE, 16), (140, SMALL, 32), (150, LARGE, 32), (300, LARGE, 64),
+                                                           (560, LARGE, 128), (700, LARGE, 256), (1600, SMALL, 128))],
+    *[(kind, tokens, dims, bm) for kind in ("mxfp8", "mxfp8_out") for tokens, dims, bm in ((1, SMALL, 256), (40, LARGE, 128), (700, LARGE, 256),
+                                                                                         (1600, LARGE, 128), (1600, SMALL, 128))],
+]
+
+
+@pytest.mark.parametrize("kind, tokens, dims, block_m", LAYERS)
+def test_layer_gemms(device, monkeypatch, gemm_descriptors, kind, tokens, dims, block_m):
+    """Both GEMMs of a layer, with activation and gather, scatter and combine: the same descriptor from both host paths, with the row
+    block that is written above, and the same result."""
     import triton_amd.matmul as mm
     from triton_amd.legacy import matmul_ogs, routing
     from triton_amd.numerics_details.mxfp import downcast_to_mxfp, quantize_mxfp8_fn
     from triton_amd.numerics_details.rowwise_fp8 import quantize_fp8_rowwise
     from triton_amd.swiglu import swiglu_fn
-    e, k, d, f = 16, 2, 256, 320
+    (d, f), e, k = dims, 16, 2
     g = torch.Generator().manual_seed(tokens)
     x = torch.randn((tokens, d), generator=g).to(torch.float16 if kind == "fp16" else torch.bfloat16).to(device)
     rd, gather, scatter = routing(torch.randn((tokens, e), generator=g).to(device), k)
@@ -120,6 +168,9 @@ def test_layer_gemms(device, monkeypatch, kind, tokens):
         pc2 = P(b_mx_scale=s2) if s2 is not None else P()
     gam = rd.gate_scal
     _both(monkeypatch, lambda: matmul_ogs(h, w2, b2, rd, scatter_indx=scatter, precision_config=pc2, gammas=gam))
+    assert [c["block_m"] for c in gemm_descriptors] == [block_m] * 4
+    for fast, slow in (gemm_descriptors[:2], gemm_descriptors[2:]):
+        _same_descriptors(fast, slow)
     # left to the general path: operands and options that are not of the plain form
     xt = x.t().contiguous().t()
     _both(monkeypatch, lambda: matmul_ogs(xt, w1, b1, rd, gather_indx=gather, precision_config=pc1, fused_activation=act, epilogue=epi), served=tokens == 1)
