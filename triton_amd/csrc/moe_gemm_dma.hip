@@ -18,8 +18,9 @@
 //   * Workgroups are persistent and the ring runs on across tiles: the first stages of the next tile are on their way during the
 //     last stages and the epilogue of this one.
 //
-// What bounds it: the board's power with the matrix pipe about 65 % busy at 1.85 GHz (a square bf16 product of 8192 runs at 1390 TFLOP/s,
-// 0.93 of what the vendor's library reaches on the same board), then the epilogues (12 % of the e4m3 GEMM with K = 4096).  16384 routed rows
+// What bounds it: the board's power (a square bf16 product of 8192: matrix pipe 87 % busy at 1.58 GHz, 1390 TFLOP/s, 0.93 of what the
+// vendor's library reaches on the same board), with shorter K also the epilogues (e4m3, K 4096: 12 % of the time; matrix pipe 67 % busy at 1.8
+// GHz, K 14336: 77 % at 1.75), with a few rows per expert (128 x 128 tiles) the weight stream at 5.3 to 5.6 TB/s.  16384 routed rows
 // of 8 experts in e4m3: K 4096, N 28672, swiglu 1840 -> 1590 us (2.42 PFLOP/s), K 14336, N 4096 850 -> 805 us; 4096 rows of 16
 // experts in bf16, K 2048: N 4096 231 -> 94 us, N 2048 133 -> 51 us (the kernels before: weights in registers with one wave
 // per SIMD, and both operands through registers into LDS).

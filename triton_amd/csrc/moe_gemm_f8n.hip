@@ -6,6 +6,8 @@ namespace {
 // ------------------------------------------------------------------------------------------------
 // e4m3 weights in a tile-native layout x e4m3 activations (prefill): FP8 MFMA, no conversion in the loop
 // ------------------------------------------------------------------------------------------------
+// For the calls that the memory-to-LDS kernel does not take (gemm_limits.h): overlapping activation rows, more than 256 slices, activations or
+// an expert's weights of 2 GiB and more.
 // Weight layout (built once per model by the host from the K-contiguous form): per expert, per fragment F of 32
 // output columns (N padded to 32), per K-block s of 128 (K padded to 256 with zero weights, so the number of
 // blocks is even): one 4 KiB block [q:4][lane:64][16 B]; lane = h*32 + lr holds the e4m3 bytes of column

@@ -9,7 +9,7 @@
 //   * e2m1 -> bf16 in registers (v_cvt_scalef32_pk_bf16_fp4) in front of v_mfma_f32_32x32x16_bf16, transposed like the other kernels.
 //   * Persistent workgroups, two per CU; the ring runs on across tiles.
 //
-// What bounds it: reading the weights, 5.0 to 5.8 TB/s.  128 experts, K = 2880, 8 routed rows per expert and more (300 tokens, top-4): N 5760 232 ->
+// What bounds it: reading the weights, 5.1 to 5.4 TB/s at 300 tokens with the matrix pipe 35 % busy.  128 experts, K = 2880, 8 routed rows per expert and more (300 tokens, top-4): N 5760 232 ->
 // 210 us, N 2880 149 -> 115 us against the decode kernel; 18 rows: 340 -> 245 and 211 -> 128 us.  More rows multiply more than they stream: at
 // 31 rows the prefill kernel's 64-row blocks win (290 against 331 us).  Measured and left out: 64-row blocks (slower than both from 8 to 31
 // rows), two or four stages in the ring (no difference).

@@ -13,8 +13,9 @@
 //     stages before this one's end, parked in LDS two before, used from the last on.  The epilogue has no branch around a store, so the
 //     wait in front of the next tile's first stage counts them and does not wait for them.
 //
-// What bounds it: the board's power in bf16 (fetching zeros instead of the weights, the operands then all zero, 558 -> 417 us), in MXFP8 also
-// LDS reads and the epilogue (without its arithmetic and stores 363 -> 316 us).  128 experts, K 2880, 4096 tokens, top-4, whole layer:
+// What bounds it: the board's power in bf16 (fetching zeros instead of the weights, the operands then all zero, 558 -> 417 us; matrix pipe 68 %
+// busy at 1.9 GHz), in MXFP8 also LDS reads and the epilogue (without its arithmetic and stores 363 -> 316 us; 42 % busy at 2.3 GHz,
+// ten vector instructions per MFMA with the quantised output, seven with bf16).  128 experts, K 2880, 4096 tokens, top-4, whole layer:
 // bf16 861 -> 830 us, MXFP8 609 -> 586 us against the kernels that keep weights in registers with one wave per SIMD (moe_gemm_mxn, _mx8n, which
 // serve what this one does not take).  Measured and left out: transfers spread over the whole bf16 stage (576 against 558
 // us: the last ones are late); weights brought into L2 a stage ahead of their transfer (570 against 558, MXFP8 387 against 363 us).
