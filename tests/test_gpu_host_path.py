@@ -210,3 +210,15 @@ def test_decode_layer(device, monkeypatch, tokens, skip_bias):
     act = mm.FusedActivation(mm.FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0))
     pc1, pc2 = mm.PrecisionConfig(b_mx_scale=s1), mm.PrecisionConfig(b_mx_scale=s2)
     _both(monkeypatch, lambda: moe_mlp(x, logits, k, w1, b1, w2, None, pc1, pc2, act))
+
+
+@pytest.mark.parametrize("reduction_n", [None, 1, 4, "2", 1 << 70])
+def test_activations_of_another_form_are_refused_by_the_general_path(device, reduction_n):
+    import triton_amd.matmul as mm
+    from triton_amd.swiglu import swiglu_fn
+    from triton_amd.tensor import make_ragged_tensor_metadata
+    x, w = torch.zeros((4, 64), dtype=torch.bfloat16, device=device), torch.zeros((1, 32, 64), dtype=torch.bfloat16, device=device).transpose(1, 2)
+    md = make_ragged_tensor_metadata(torch.tensor([4], dtype=torch.int32, device=device), 4)
+    act = mm.FusedActivation(mm.FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=reduction_n), (1.702, 7.0))
+    with pytest.raises(NotImplementedError):
+        mm.matmul(x, w, None, md, fused_activation=act)

@@ -252,7 +252,12 @@ struct Activation {
   bool read(PyObject* act) {
     if (is_none(act) || act == B.no_activation) return true;
     Ref specs(attr(act, N_.specs)), red(attr(specs, N_.reduction_n)), args(attr(act, N_.fn_args));
-    if (!named(specs, N_.name, "swiglu") || PyLong_AsLong(red) != 2 || !PyTuple_Check(args.p)) return false;
+    const long columns = PyLong_AsLong(red);
+    if (PyErr_Occurred()) {
+      PyErr_Clear();
+      return false;
+    }
+    if (!named(specs, N_.name, "swiglu") || columns != 2 || !PyTuple_Check(args.p)) return false;
     Py_ssize_t n = PyTuple_GET_SIZE(args.p);
     if (n < 1) return false;
     alpha = PyFloat_AsDouble(PyTuple_GET_ITEM(args.p, 0));
