@@ -26,4 +26,8 @@ inline bool dma_runs_16bit(uint32_t x_bytes, int64_t n_slices, int64_t K, int64_
   return w_stride_n >= K && dma_runs(x_bytes, n_slices, ((N - 1) * w_stride_n + K) * 2);
 }
 
+// Row blocks (of 64) that the kernel for few rows launches side by side: one a slice at least, and what slices of up to five quarters of
+// the mean make, as a random routing does (at 62 rows per slice half of the slices have a second block).
+inline int64_t few_row_blocks(int64_t rows, int64_t n_slices) { return n_slices * (rows * 5 / (n_slices * 256) + 1); }
+
 }  // namespace tk

@@ -194,6 +194,18 @@ int64_t wide_block_m(int64_t rows, int64_t n_slices, int64_t K, uint32_t x_bytes
   return !mx8 || rows <= 176 * n_slices || rows >= 640 * n_slices ? 256 : 128;
 }
 
+// Columns a workgroup of the kernel for few rows, 0 = the kernels above: up to 64 rows per slice and one workgroup per CU at most, with 32
+// columns while they fit, then 64.  Measured (us, this kernel against the one that ran before): 16 slices, 2 or 8 rows each, K 512,
+// N 1024 4.2 against 6.6, K 256, N 512 4.2 against 4.9; 32 rows each, 8 slices, K 512, N 2048 6.3 against 9.4, K 1024, N 512 5.7 against
+// 12.1; 64 rows, K 1024, N 512 6.7 against 12.4; 16 slices of 32 rows, K 1024, N 1024 8.5 against 14.5.  With two workgroups per CU to be
+// run in turn the others are as fast or faster (16 slices, K 1024, N 2048: 8 rows 16.8 against 15.5, 32 rows 19.6 against 16.8; 8 slices of
+// 125 rows, K 512, N 1024: 12.0 against 9.9).
+int64_t few_block_n(int64_t rows, int64_t N, int64_t n_slices) {
+  if (n_slices < 1 || rows > 64 * n_slices) return 0;
+  const int64_t blocks = tk::few_row_blocks(rows, n_slices);
+  return blocks * ((N + 31) / 32) <= 256 ? 32 : blocks * ((N + 63) / 64) <= 256 ? 64 : 0;
+}
+
 int64_t default_block_m(int64_t rows, int64_t n_slices) {
   int64_t per_slice = std::max<int64_t>(1, rows / std::max<int64_t>(n_slices, 1));
   return per_slice <= 16 ? 16 : per_slice <= 32 ? 32 : per_slice <= 64 ? 64 : 128;
@@ -385,7 +397,7 @@ PyObject* run_gemm(PyObject* const* v) {
     return none();
 
   // ---- row blocks
-  int64_t block_m = default_block_m(M, n_slices);
+  int64_t block_m = default_block_m(M, n_slices), block_n = 0;
   const uint32_t x_bytes = tk::x_extent(a_rows, a_stride, K, a->element_size());
   if (tiled_fp8) {
     block_m = fp8_block_m(M, x_bytes, K, N, n_slices);
@@ -394,8 +406,9 @@ PyObject* run_gemm(PyObject* const* v) {
   } else if (tiled) {
     if (M > 256 && x_bytes && n_slices <= tk::kDmaSlices && !x_row && !w_col) block_m = mxfp4_block_m(M, n_slices, block_m);
     if (block_m == 128) block_m = wide_block_m(M, n_slices, K, x_bytes, false);
-  } else if (block_m > 16 && tk::dma_runs_16bit(x_bytes, n_slices, K, N, w->stride(2))) {
-    block_m = dma_block_m(M, 2 * K, N, n_slices);
+  } else if (tk::dma_runs_16bit(x_bytes, n_slices, K, N, w->stride(2))) {
+    if (idle <= 0) block_n = few_block_n(M, N, n_slices);
+    if (block_m > 16) block_m = dma_block_m(M, 2 * K, N, n_slices);
   }
   if (tiled && block_m >= 64 && !mx_act && n_out % 8) return none();  // (through a padded buffer)
 
@@ -422,7 +435,7 @@ PyObject* run_gemm(PyObject* const* v) {
   d.slice_sizes = static_cast<const int32_t*>(md.sizes->data_ptr()), d.slice_offs = static_cast<const int32_t*>(md.offs->data_ptr());
   d.block_offs = static_cast<const int32_t*>(md.block_offs->data_ptr()) + row * md.block_offs->stride(0);
   d.block_schedule = static_cast<const int32_t*>(md.schedule->data_ptr()) + row * md.schedule->stride(0);
-  d.n_slices = int32_t(n_slices), d.block_m = int32_t(block_m);
+  d.n_slices = int32_t(n_slices), d.block_m = int32_t(block_m), d.block_n = int32_t(block_n);
   d.grid_m = int32_t(std::min(n_blocks(n_slices, M, block_m), md.schedule->size(1)));
   d.M = int32_t(M), d.N = int32_t(N), d.K = int32_t(K);
   d.y = y.data_ptr(), d.y_dtype = dtype_code(out), d.y_stride_m = n_out;
@@ -754,6 +767,10 @@ PyObject* rule_dma(PyObject* const* v) {
   const auto [rows, row_bytes, N, n_slices] = integers<4>(v);
   return PyLong_FromLongLong(dma_block_m(rows, row_bytes, N, n_slices));
 }
+PyObject* rule_few(PyObject* const* v) {
+  const auto [rows, N, n_slices] = integers<3>(v);
+  return PyLong_FromLongLong(few_block_n(rows, N, n_slices));
+}
 PyObject* rule_fp8(PyObject* const* v) {
   const auto [rows, x_bytes, K, N, n_slices] = integers<5>(v);
   return PyLong_FromLongLong(fp8_block_m(rows, uint32_t(x_bytes), K, N, n_slices));
@@ -816,6 +833,7 @@ PyMethodDef methods[] = {
     METHOD("x_extent", rule_x_extent, 4),
     METHOD("dma_runs_16bit", rule_dma_16bit, 5),
     METHOD("dma_block_m", rule_dma, 4),
+    METHOD("few_block_n", rule_few, 3),
     METHOD("fp8_block_m", rule_fp8, 5),
     METHOD("mxfp4_block_m", rule_mxfp4, 3),
     METHOD("wide_block_m", rule_wide, 5),

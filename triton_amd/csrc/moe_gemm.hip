@@ -15,6 +15,7 @@ static int64_t slices(const tk_gemm_desc* d) { return d->slice_sizes ? d->n_slic
 // general one, which has no row blocks of 256.
 static int32_t launch_16bit(const GemmParams& p, const tk_gemm_desc* d, int wk, bool swiglu, hipStream_t st) {
   const bool dma = dma_runs_16bit(p.x_bytes, slices(d), d->K, d->N, d->w_stride_n);
+  if (dma && (d->block_n == 32 || d->block_n == 64) && d->idle_cus <= 0) return gemm_launch_few(p, wk, d->block_n, swiglu, st);
   if (dma && (d->block_m == 128 || d->block_m == 256)) return gemm_launch_dma(p, wk, d->block_m, d->grid_m, swiglu, st);
   if (d->block_m == 256)
     return fail(TK_ERR_INVALID, "tk_moe_gemm: block_m 256 with 16-bit weights needs x (x_rows rows, none closer than K) and an expert's weights within 2 GiB and up to %d slices", kDmaSlices);

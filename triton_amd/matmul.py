@@ -770,10 +770,12 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
             if block_m == 128:
                 block_m = nt.rules().wide_block_m(M, n_slices, K, x_bytes, 0)
     elif w_dtype in (_BF16, _F16):
-        if block_m > 16:
-            if not nt.rules().dma_runs_16bit(x_bytes, n_slices, K, N, w.stride(-1)):
-                block_m = min(block_m, 128)  # (the general kernel's largest)
-            elif forced is None:
+        if not nt.rules().dma_runs_16bit(x_bytes, n_slices, K, N, w.stride(-1)):
+            block_m = min(block_m, 128)  # (the general kernel's largest)
+        elif forced is None:
+            if not idle or int(idle) <= 0:
+                d.block_n = nt.rules().few_block_n(M, N, n_slices)
+            if block_m > 16:
                 block_m = nt.rules().dma_block_m(M, 2 * K, N, n_slices)
     elif block_m == 256:
         block_m = 128
