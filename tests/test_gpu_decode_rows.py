@@ -1,0 +1,82 @@
+"""The decode layer row by row (two launches, small streams of weights) against the CPU oracle and against the single launch on the same
+arguments, which a caller gets by naming a spin limit: one token and the most rows, one expert a token and the most, experts met by several
+tokens, fragments and stages that are partly filled, the largest K, both router widths, 16-bit logits, with and without biases."""
+import pytest
+import torch
+
+from oracle import moe as omoe
+from oracle import mxfp as omx
+from oracle import routing as ort
+from oracle.checks import assert_close, assert_equal
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("T, E, k, d_model, d_ff, bias_dtype, limit, logits_dtype", [
+    (1, 4, 1, 8, 8, torch.bfloat16, 7.0, torch.float32),
+    (1, 6, 4, 2880, 2880, torch.bfloat16, 7.0, torch.float32),
+    (1, 8, 8, 3072, 3072, torch.float32, None, torch.bfloat16),
+    (3, 5, 2, 136, 264, torch.float32, 7.0, torch.bfloat16),
+    (64, 130, 1, 360, 248, None, 7.0, torch.float32),
+    (16, 6, 4, 520, 1144, torch.bfloat16, None, torch.float32),
+    (8, 512, 8, 144, 96, torch.bfloat16, 7.0, torch.float32),
+])
+def test_rows_against_oracle_and_single_launch(device, monkeypatch, T, E, k, d_model, d_ff, bias_dtype, limit, logits_dtype):
+    from bench import to_matmul_layout
+    from triton_amd import _native as nt
+    from triton_kernels import moe_decode
+    from triton_kernels.matmul import FnSpecs, FusedActivation, PrecisionConfig
+    from triton_kernels.swiglu import swiglu_fn
+    g = torch.Generator().manual_seed(T * 131 + E)
+    x = torch.randn((T, d_model), generator=g).to(torch.bfloat16)
+    logits = torch.randn((T, E), generator=g).to(logits_dtype)
+    dev = lambda t: None if t is None else t.to(device)
+    w = [(torch.randn(s, generator=g) / s[1]**0.5).to(torch.bfloat16) for s in ((E, d_model, 2 * d_ff), (E, d_ff, d_model))]
+    q = []
+    for m in w:  # K is no multiple of the block in some cases: padded with zeros, as a loader does
+        pad = -m.shape[1] % 32
+        q += omx.downcast_to_mxfp(torch.nn.functional.pad(m, (0, 0, 0, pad)), torch.uint8, axis=1)
+    b1 = b2 = None
+    if bias_dtype is not None:
+        b1, b2 = (torch.randn((E, n), generator=g).mul(0.1).to(bias_dtype) for n in (2 * d_ff, d_model))
+    tiled = to_matmul_layout({n: dev(t) for n, t in dict(w1=q[0], w1s=q[1], w2=q[2], w2s=q[3], b1=b1, b2=b2).items()})
+    for name, m in (("w1", w[0]), ("w2", w[1])):
+        tiled[name].shape[-2] = m.shape[1]
+    act = FusedActivation(FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, limit))
+    args = (dev(x), dev(logits), k, tiled["w1"], tiled["b1"], tiled["w2"], tiled["b2"], PrecisionConfig(b_mx_scale=tiled["w1s"]),
+            PrecisionConfig(b_mx_scale=tiled["w2s"]), act)
+    assert moe_decode.one_launch_reason(*args) is None
+    out, indx, vals = moe_decode.moe_decode_layer(*args, return_routing=True)
+    assert torch.equal(moe_decode.moe_mlp(*args), out)
+
+    class Bounded(nt.DecodeLayerDesc):
+        def __init__(self):
+            super().__init__()
+            self.spin_limit = 1 << 22
+
+    with monkeypatch.context() as p:
+        p.setattr(nt, "DecodeLayerDesc", Bounded)
+        one, one_indx, one_vals = moe_decode.moe_decode_layer(*args, return_routing=True)
+    r = ort.routing(logits.float(), k)  # (both launches keep the gate values in fp32)
+    assert_equal(r.indx, indx.to(torch.int32), "indx")
+    assert torch.equal(indx, one_indx)
+    assert_close(r.vals.float(), vals, what="gate values")
+    xp = torch.nn.functional.pad(x, (0, -d_model % 32))
+    h = omoe.matmul(xp, q[0], b1, r.meta.col_sum, gather_indx=r.gather_indx, w_mx_scale=q[1])
+    a = torch.nn.functional.pad(omoe.swiglu(h, 1.702, limit), (0, -d_ff % 32))
+    y = omoe.matmul(a, q[2], b2, r.meta.col_sum, scatter_indx=r.scatter_indx, gammas=r.gammas, w_mx_scale=q[3])
+    assert_close(omoe.reduce_k(y, k), out, maxtol=3e-2, what="row by row against the oracle")
+    # the two kernels sum K in different groupings: an ulp of a hidden value here and there
+    assert_close(one.cpu(), out, maxtol=2e-2, what="row by row against the single launch")
+
+
+def test_a_k_that_routing_refuses_stays_refused(device):
+    from triton_kernels.moe_decode import moe_mlp
+    from bench import make_moe_weights, to_matmul_layout
+    from triton_kernels.matmul import FnSpecs, FusedActivation, PrecisionConfig
+    from triton_kernels.swiglu import swiglu_fn
+    W = to_matmul_layout(make_moe_weights(8, 128, 256, seed=1, device=device)[0])
+    act = FusedActivation(FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0))
+    x, logits = torch.zeros((2, 128), dtype=torch.bfloat16, device=device), torch.zeros((2, 8), device=device)
+    with pytest.raises(ValueError):
+        moe_mlp(x, logits, 3, W["w1"], W["b1"], W["w2"], W["b2"], PrecisionConfig(b_mx_scale=W["w1s"]), PrecisionConfig(b_mx_scale=W["w2s"]), act)

@@ -24,6 +24,7 @@
 //
 // Every wait is bounded: a spin that exceeds `spin_limit` polls raises the error word of the workspace and goes on
 // (the result is then wrong, but every wave exits).
+#include "decode_params.h"
 #include "gemm_common.h"
 #include "route_common.h"
 
@@ -38,40 +39,6 @@ constexpr int kDecXS = 3;                              // K-stages (of 128) per 
 constexpr int kDecRing = 3;                            // units of weight blocks a wave holds or has requested
 constexpr int kDecBlockStride = 32;                    // words between two row blocks' counters (a cache line each)
 constexpr int kDecBlockWords = (kDecMaxRows + kDecMaxRows / 16) * kDecBlockStride;  // 16-row blocks: at most min(E, R) + R / 16
-
-struct DecodeParams {
-  const uint8_t* x;  // bf16 [T, K1]
-  int64_t x_stride;  // elements
-  uint32_t x_bytes;  // extent of x (the rows are read through a buffer resource)
-  const void* logits;
-  int64_t logits_stride;
-  int32_t logits_is_bf16;
-  int32_t T, E, k, apply_softmax;
-  const uint8_t* w1;
-  const uint8_t* w1s;
-  int64_t w1_stride_e, w1s_stride_e;  // bytes
-  const void* b1;
-  int64_t b1_stride_e;
-  int32_t b1_is_f32;
-  const uint8_t* w2;
-  const uint8_t* w2s;
-  int64_t w2_stride_e, w2s_stride_e;
-  const void* b2;
-  int64_t b2_stride_e;
-  int32_t b2_is_f32;
-  int32_t K1, N1, K2, N2;  // K2 = N1 / 2
-  int32_t nst1, nst2, nfr1, nfr2;
-  float alpha, limit;
-  int32_t has_limit;
-  uint16_t* h;      // scratch [T*k, K2] bf16, expert-sorted rows
-  uint16_t* y;      // scratch [T*k, N2] bf16, flat rows t*k + j
-  int32_t* sync;    // [0] finished workgroups, [1] error word, then kDecBlockWords GEMM-1 units done per row block, then [T*nfr2] arrivals
-  uint16_t* out;    // [T, N2] bf16
-  int64_t out_stride;
-  int16_t* indx_out;  // optional [T, k]
-  float* vals_out;    // optional [T, k]
-  int32_t spin_limit;
-};
 
 struct DecUnit {
   const uint8_t* w;  // first K-stage of the unit's weight fragment
@@ -831,6 +798,16 @@ extern "C" int32_t tk_moe_decode_layer(const tk_decode_layer_desc* d, tk_stream_
   p.indx_out = static_cast<int16_t*>(d->indx_out);
   p.vals_out = d->vals_out;
   p.spin_limit = d->spin_limit > 0 ? d->spin_limit : (1 << 22);
+  // Row by row in two launches (moe_decode_rows.hip), where the rows' weights, counted for every row, are a small stream: the single
+  // launch costs some 20 us around its stream, the two launches 7, but they read an expert's weights again for each of its rows.  Measured
+  // (us, row by row against single launch; 2880 x 5760 and 2880 x 2880 but where noted): 8 rows, 106 MB, 29.8 against 37.1; 10 rows of 8
+  // experts, 132 MB, 31.5 against 37.0; 12 rows of 10 experts, 159 MB, 39.9 against 40.0; 16 rows of 12, 211 MB, 46.8 against 44.8.  Smaller
+  // layers: d and d_ff 512, 64 rows of 13 experts, 27 MB, 15.7 against 28.1; 1024, 64 rows, 107 MB, 30.3 against 39.0; 1024 and 2048, 32 rows
+  // of 4 experts, 107 MB, 26.8 against 30.6; 512, 256 rows of 21 experts, 107 MB, 52.5 against 32.1.  (A caller that names a spin limit asks
+  // for the launch whose waits it bounds.)
+  constexpr int64_t kRowsMax = 64, kRowsBytes = 135'000'000;
+  const int64_t expert_bytes = ((int64_t)p.nfr1 * p.nst1 + (int64_t)p.nfr2 * p.nst2) * (2048 + 128);
+  if (d->spin_limit <= 0 && k <= kDecRowsMaxK && R <= kRowsMax && R * expert_bytes <= kRowsBytes) return decode_launch_rows(p, static_cast<hipStream_t>(stream));
   const bool small_e = E <= 128;
   int grid = small_e ? resident_workgroups<8>() : resident_workgroups<kDecMaxExperts / 16>();
   if (grid <= 0) return fail(TK_ERR_LAUNCH, "tk_moe_decode_layer: cannot determine how many workgroups are resident together");

@@ -8,7 +8,8 @@ The reference's MoE block is a sequence of calls (python/triton_kernels/bench/be
 
 `moe_mlp` computes the same `out` from the same arguments.  With a handful of tokens (T * k <= 256 routed rows), tiled
 MXFP4 weights and d_model, d_ff <= 3072 it is ONE kernel launch (`tk_moe_decode_layer`: router, both expert GEMMs and
-the top-k combine in a persistent grid); any other case runs the three calls above.  At these sizes the layer is a
+the top-k combine in a persistent grid), or two where the rows' weights are a small stream (one GEMM each, routed and combined
+inside); any other case runs the three calls above.  At these sizes the layer is a
 stream of the active experts' weights, and launch boundaries plus the serial router in front of the first weight byte
 cost a third of the three-call time.
 """
@@ -23,7 +24,7 @@ from .tensor import FP4, Tensor
 from .tensor_details.layout_details.gfx950_mx import GFX950MXScaleLayout, GFX950MXValueLayout
 
 MAX_ROWS = 256
-MIN_ROWS = 8  # below this `moe_mlp` prefers the three calls
+MIN_ROWS = 1  # below this `moe_mlp` prefers the three calls
 MAX_EXPERTS = 512
 MAX_DIM = 3072
 
@@ -158,11 +159,10 @@ def moe_decode_layer(x, logits, n_expts_act, w1, b1, w2, b2, pc1: PrecisionConfi
 def moe_mlp(x, logits, n_expts_act, w1, b1, w2, b2, pc1: PrecisionConfig, pc2: PrecisionConfig,
             fused_activation: FusedActivation):
     """`routing` + gather-`matmul_ogs` (+ fused activation) + scatter-`matmul_ogs` (gate weighted, k rows summed) as one
-    call: one kernel launch at decode sizes, the three calls otherwise.  Returns `[tokens, d_model]`."""
-    # (with fewer than 8 routed rows the launch's fixed part, every workgroup routing the batch before its first weight
-    # byte, outweighs the two launch boundaries it saves: 41 against 29 us for one token at the gpt-oss shape)
+    call: one or two kernel launches at decode sizes, the three calls otherwise.  Returns `[tokens, d_model]`."""
     rows = logits.shape[0] * n_expts_act
-    if MIN_ROWS <= rows <= MAX_ROWS:
+    # (up to 7 rows only with a k that `routing` takes: other k are refused there at every size)
+    if MIN_ROWS <= rows <= MAX_ROWS and (rows > 7 or n_expts_act & (n_expts_act - 1) == 0):
         host = nt.host()
         out = None
         if host is not None:
