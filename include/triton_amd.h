@@ -343,8 +343,9 @@ typedef struct tk_gemm_desc {
    * `reduce(y.view(T, k, -1), dim=1)` launch of tk/reduce.py:1143-1165 after the scatter of
    * tk/matmul_details/_matmul.py:535-569. */
   int32_t combine_k;
-  /* 32 or 64 = the kernel for few rows per expert with that many columns a workgroup, in place of the one that block_m names; taken
-   * with 16-bit weights where the memory-to-LDS kernel runs and no compute units are left idle, else not looked at.  0 = by block_m. */
+  /* Another kernel or tile than the one that block_m names, where the memory-to-LDS kernel runs (else not looked at): 32 or 64 = the kernel
+   * for few rows per expert with that many columns a workgroup (16-bit weights, no compute units left idle); 128 = 128 x 128 tiles
+   * beside block_m 256 (16-bit and tiled e4m3 weights).  0 = by block_m. */
   int32_t block_n;
   void* combine_out; /* bf16 [tokens, N], unit stride along N */
   int64_t combine_stride_m;

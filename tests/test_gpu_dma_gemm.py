@@ -119,3 +119,30 @@ def test_overlapping_rows_tiled_e4m3(device, monkeypatch, sizes, stride):
     want = omoe.matmul(x.contiguous(), w.transpose(1, 2), None, sizes, gather_indx=gi, out_dtype=torch.float32)
     assert_allclose_gate(want, native, what=f"e4m3 row stride {stride}")
     assert torch.equal(native, general)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "e4m3"])
+def test_few_large_tiles_run_as_small_ones(device, monkeypatch, dtype):
+    """Where the rows say 256 x 256 and the chip would have few such tiles: the unforced choice against the oracle and, bit for bit, against
+    the small tiles asked for by name, from both host paths."""
+    import triton_amd.matmul as mm
+    from triton_amd import _native as nt
+    from triton_amd.tensor import convert_layout, make_ragged_tensor_metadata, wrap_torch_tensor
+    from triton_amd.tensor_details.layout import make_default_matmul_fp8_w_layout
+    g = torch.Generator().manual_seed(11)
+    sizes, k, n = torch.tensor([0, 250, 700, 129, 513], dtype=torch.int32), 272, 264
+    m, e = int(sizes.sum()), len(sizes)
+    assert nt.rules().dma_block_m(m, k, n, e) == 256 and nt.rules().dma_block_n(m, n, e, 256) == 128
+    dt = torch.bfloat16 if dtype == "bfloat16" else torch.float8_e4m3fn
+    x, w = torch.randn((m, k), generator=g).to(dt), (torch.randn((e, n, k), generator=g) * 0.1).to(dt)
+    wd = w.to(device).transpose(1, 2)
+    wd = wd if dtype == "bfloat16" else convert_layout(wrap_torch_tensor(wd), make_default_matmul_fp8_w_layout())
+    md, pc = make_ragged_tensor_metadata(sizes.to(device), m), mm.PrecisionConfig(out_dtype=torch.bfloat16)
+    native = mm.matmul(x.to(device), wd, None, md, precision_config=pc)
+    with monkeypatch.context() as p:
+        p.setattr(nt, "host", lambda: None)
+        general = mm.matmul(x.to(device), wd, None, md, precision_config=pc)
+    with mm.scoped_opt_flags_constraints({"block_m": 128}):
+        small = mm.matmul(x.to(device), wd, None, md, precision_config=pc)
+    assert_allclose_gate(omoe.matmul(x, w.transpose(1, 2), None, sizes, out_dtype=torch.float32), native, what=f"{dtype} few large tiles")
+    assert torch.equal(native, general) and torch.equal(native, small)

@@ -26,6 +26,11 @@ inline bool dma_runs_16bit(uint32_t x_bytes, int64_t n_slices, int64_t K, int64_
   return w_stride_n >= K && dma_runs(x_bytes, n_slices, ((N - 1) * w_stride_n + K) * 2);
 }
 
+// ... on tiled e4m3 weights (fragments of 32 columns, stages of 256 k, 8 KiB each).
+inline bool dma_runs_e4m3(uint32_t x_bytes, int64_t n_slices, int64_t K, int64_t N) {
+  return dma_runs(x_bytes, n_slices, (N + 31) / 32 * ((K + 255) / 256) * 8192);
+}
+
 // Row blocks (of 64) that the kernel for few rows launches side by side: one a slice at least, and what slices of up to five quarters of
 // the mean make, as a random routing does (at 62 rows per slice half of the slices have a second block).
 inline int64_t few_row_blocks(int64_t rows, int64_t n_slices) { return n_slices * (rows * 5 / (n_slices * 256) + 1); }

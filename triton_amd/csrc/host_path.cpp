@@ -162,12 +162,21 @@ int64_t dma_block_m(int64_t rows, int64_t row_bytes, int64_t N, int64_t n_slices
   return per_slice >= 192 || tiles >= 192 || row_bytes >= 8192 ? 256 : 128;
 }
 
+// 128 = the kernel's 128 x 128 tiles although the rule above says 256: up to 96 of the large tiles leave most of the 256 CUs without one.
+// Measured with a random routing (us, 128 against 256): bf16, K 2048, N 2048, 8 slices of 256 rows (64 large tiles) 29 against 42; N 1536, 16
+// slices (96) 34 against 41; N 2048, 16 slices (128) 51 against 49; K 1024, N 1024, 16 slices (64) 19 against 27, N 512 (32) 11 against 23;
+// K 4096, N 1024, 16 slices (64) 55 against 72; e4m3, K 14336, N 2048, 8 slices (64) 92 against 126, N 4096 (128) 193 against 158.
+int64_t dma_block_n(int64_t rows, int64_t N, int64_t n_slices, int64_t block_m) {
+  const int64_t per_slice = rows / std::max<int64_t>(n_slices, 1);
+  return block_m == 256 && n_slices * ((per_slice + 255) / 256) * ((N + 255) / 256) <= 96 ? 128 : 0;
+}
+
 // Row blocks for tiled e4m3 weights: by the rule above where that kernel runs (`x_bytes` as in gemm_limits.h).  The other kernel walks a
 // block of 256 rows in two passes, which pays from 1024 rows per slice on (8 slices, K 4096, N 8192: 512 rows 147 us with either, 1024
 // 296 with blocks of 128 against 289 with 256; 2048 rows, N 28672: 1930 against 1853, K 14336, N 4096: 846 against 819 us) and costs up to twice
 // the time below (256 rows, K 14336: 133 against 273 us; 300 slices of 256 rows, K and N 2048: 474 against 544 us).
 int64_t fp8_block_m(int64_t rows, uint32_t x_bytes, int64_t K, int64_t N, int64_t n_slices) {
-  if (tk::dma_runs(x_bytes, n_slices, (N + 31) / 32 * ((K + 255) / 256) * 8192)) return dma_block_m(rows, K, N, n_slices);
+  if (tk::dma_runs_e4m3(x_bytes, n_slices, K, N)) return dma_block_m(rows, K, N, n_slices);
   return rows >= 1024 * n_slices ? 256 : 128;
 }
 
@@ -401,6 +410,7 @@ PyObject* run_gemm(PyObject* const* v) {
   const uint32_t x_bytes = tk::x_extent(a_rows, a_stride, K, a->element_size());
   if (tiled_fp8) {
     block_m = fp8_block_m(M, x_bytes, K, N, n_slices);
+    if (tk::dma_runs_e4m3(x_bytes, n_slices, K, N)) block_n = dma_block_n(M, N, n_slices, block_m);
   } else if (mx_act) {
     block_m = wide_block_m(M, n_slices, K, x_bytes, true);
   } else if (tiled) {
@@ -409,6 +419,7 @@ PyObject* run_gemm(PyObject* const* v) {
   } else if (tk::dma_runs_16bit(x_bytes, n_slices, K, N, w->stride(2))) {
     if (idle <= 0) block_n = few_block_n(M, N, n_slices);
     if (block_m > 16) block_m = dma_block_m(M, 2 * K, N, n_slices);
+    if (!block_n) block_n = dma_block_n(M, N, n_slices, block_m);
   }
   if (tiled && block_m >= 64 && !mx_act && n_out % 8) return none();  // (through a padded buffer)
 
@@ -771,6 +782,14 @@ PyObject* rule_few(PyObject* const* v) {
   const auto [rows, N, n_slices] = integers<3>(v);
   return PyLong_FromLongLong(few_block_n(rows, N, n_slices));
 }
+PyObject* rule_dma_n(PyObject* const* v) {
+  const auto [rows, N, n_slices, block_m] = integers<4>(v);
+  return PyLong_FromLongLong(dma_block_n(rows, N, n_slices, block_m));
+}
+PyObject* rule_dma_e4m3(PyObject* const* v) {
+  const auto [x_bytes, n_slices, K, N] = integers<4>(v);
+  return PyBool_FromLong(tk::dma_runs_e4m3(uint32_t(x_bytes), n_slices, K, N));
+}
 PyObject* rule_fp8(PyObject* const* v) {
   const auto [rows, x_bytes, K, N, n_slices] = integers<5>(v);
   return PyLong_FromLongLong(fp8_block_m(rows, uint32_t(x_bytes), K, N, n_slices));
@@ -833,6 +852,8 @@ PyMethodDef methods[] = {
     METHOD("x_extent", rule_x_extent, 4),
     METHOD("dma_runs_16bit", rule_dma_16bit, 5),
     METHOD("dma_block_m", rule_dma, 4),
+    METHOD("dma_runs_e4m3", rule_dma_e4m3, 4),
+    METHOD("dma_block_n", rule_dma_n, 4),
     METHOD("few_block_n", rule_few, 3),
     METHOD("fp8_block_m", rule_fp8, 5),
     METHOD("mxfp4_block_m", rule_mxfp4, 3),

@@ -11,12 +11,19 @@ using namespace tk;
 // slices of the ragged metadata (a call without it has one)
 static int64_t slices(const tk_gemm_desc* d) { return d->slice_sizes ? d->n_slices : 1; }
 
+// Row blocks of 256 rows or, asked for by block_n, 128 x 128 tiles in their place (grid_m counts row blocks of block_m).
+static int32_t launch_dma(const GemmParams& p, const tk_gemm_desc* d, int wk, bool swiglu, hipStream_t st) {
+  if (d->block_m != 256 || d->block_n != 128) return gemm_launch_dma(p, wk, d->block_m, d->grid_m, swiglu, st);
+  const int64_t n = slices(d), blocks = d->M <= n ? d->M : n - 1 + cdiv(d->M + 1 - n, 128);
+  return gemm_launch_dma(p, wk, 128, (int)blocks, swiglu, st);
+}
+
 // Strided 16-bit weights: the kernel that stages both operands through memory-to-LDS transfers for full row blocks where it runs, else the
 // general one, which has no row blocks of 256.
 static int32_t launch_16bit(const GemmParams& p, const tk_gemm_desc* d, int wk, bool swiglu, hipStream_t st) {
   const bool dma = dma_runs_16bit(p.x_bytes, slices(d), d->K, d->N, d->w_stride_n);
   if (dma && (d->block_n == 32 || d->block_n == 64) && d->idle_cus <= 0) return gemm_launch_few(p, wk, d->block_n, swiglu, st);
-  if (dma && (d->block_m == 128 || d->block_m == 256)) return gemm_launch_dma(p, wk, d->block_m, d->grid_m, swiglu, st);
+  if (dma && (d->block_m == 128 || d->block_m == 256)) return launch_dma(p, d, wk, swiglu, st);
   if (d->block_m == 256)
     return fail(TK_ERR_INVALID, "tk_moe_gemm: block_m 256 with 16-bit weights needs x (x_rows rows, none closer than K) and an expert's weights within 2 GiB and up to %d slices", kDmaSlices);
   return gemm_launch_strided(p, wk, d->block_m, d->grid_m, swiglu, st);
@@ -145,7 +152,7 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
     if (d->n_slices > 1 && d->w_stride_e < nfr * nst * 8192) return fail(TK_ERR_INVALID, "tk_moe_gemm: expert stride smaller than one tiled expert");
     p.w_stride_e = d->w_stride_e;
     p.w_nst = (int32_t)nst;
-    if (dma_runs(p.x_bytes, slices(d), nfr * nst * 8192)) return gemm_launch_dma(p, WK_FP8, d->block_m, d->grid_m, swiglu, st);
+    if (dma_runs(p.x_bytes, slices(d), nfr * nst * 8192)) return launch_dma(p, d, WK_FP8, swiglu, st);
     return gemm_launch_f8n(p, d->block_m, d->grid_m, swiglu, st);
   }
   if (mx_act) {

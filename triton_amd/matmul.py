@@ -754,6 +754,8 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
     x_bytes = nt.rules().x_extent(a_rows, a_stride, K, a.itemsize)  # 0: rows that the buffer-resource kernels do not take
     if tiled_fp8:
         block_m = forced if forced in (128, 256) else 128 if forced is not None else nt.rules().fp8_block_m(M, x_bytes, K, N, n_slices)
+        if forced is None and nt.rules().dma_runs_e4m3(x_bytes, n_slices, K, N):
+            d.block_n = nt.rules().dma_block_n(M, N, n_slices, block_m)
     elif mx_act or (tiled and mx_out_fused):
         # the tile shapes that take MXFP8 activations / have an MX-output epilogue
         if forced is None and is_ragged:
@@ -777,6 +779,7 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
                 d.block_n = nt.rules().few_block_n(M, N, n_slices)
             if block_m > 16:
                 block_m = nt.rules().dma_block_m(M, 2 * K, N, n_slices)
+            d.block_n = d.block_n or nt.rules().dma_block_n(M, N, n_slices, block_m)
     elif block_m == 256:
         block_m = 128
     if is_ragged:
