@@ -167,6 +167,31 @@ def test_baseline_router_shape(tk, device):
         assert_close(r.vals, sm.vals, what="vals")
 
 
+@pytest.mark.parametrize("T, E, k", [
+    *[(t, e, 4) for t in (16, 17, 1021, 5000) for e in (4, 36, 252, 256, 260)],
+    (1, 1, 1), (256, 16, 4), (257, 16, 4), (255, 7, 1), (300, 12, 2), (128, 32, 8), (129, 32, 8), (60, 17, 4), (1, 32, 8), (128, 64, 2),
+    (16, 50, 16), (129, 64, 1), (128, 128, 2), (15, 128, 16), (32, 100, 8), (33, 128, 8), (2, 129, 8), (40, 10, 8)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_every_way_through_the_router(device, T, E, k, dtype):
+    """Around the sizes where the pass changes its kernels (lanes and passes of a row, entries, experts, several rows per wave), experts of
+    very different popularity: everything that `routing` returns, bit for bit, in the order of the oracle."""
+    from triton_amd.legacy import routing
+    g = torch.Generator().manual_seed(T + E)
+    x = (torch.randn((T, E), generator=g) + 3 * torch.randn((E, ), generator=g)).to(dtype) + 0.0
+    r = ort.routing(x, k)
+    rd, gather, scatter = routing(x.to(device), k)
+    assert_equal(r.indx, rd.expt_indx.to(torch.int32), "indx")
+    assert_equal(r.meta.col_sum, rd.expt_hist, "col_sum")
+    assert_equal(r.meta.col_sorted_indx, gather.src_indx, "col_sorted_indx")
+    assert_equal(r.meta.row_sorted_indx, scatter.src_indx, "row_sorted_indx")
+    assert_equal(r.gather_indx, rd.token_indx, "gather index")
+    assert torch.equal(rd.gate_scal, rd.gate_vals.flatten()[gather.src_indx.long()])
+    ref = ort.make_ragged_tensor_metadata(r.meta.col_sum, T * k)
+    assert_equal(ref.slice_offs, rd.expt_data.slice_offs, "slice_offs")
+    assert_equal(ref.block_offs_data, rd.expt_data.block_offs_data, "block_offs")
+    assert_equal(ref.block_schedule_data, rd.expt_data.block_schedule_data, "block_schedule")
+
+
 @pytest.mark.parametrize("n_slices", [9, 32, 911, 1025])
 def test_remap_ragged_tensor_metadata(device, n_slices):
     """Mirrors tests/test_tensor.py:259-277 of the reference: random sizes with an empty slice, a random permutation as

@@ -1,7 +1,8 @@
 // Top-k softmax router, expert histogram / gather-scatter indices and ragged block schedule for gfx950.
 //
 // The reference spends six dependent launches here (top-k, vertical popcount, two metadata stages,
-// two ragged-metadata kernels).  Here the work is three launches, all latency-bound integer work:
+// two ragged-metadata kernels).  Here the work is two launches (three with more than 256
+// experts or a number that is no multiple of four, one for few rows), all latency-bound integer work:
 //
 //   route_topk_kernel    one wave64 owns a run of `rows_per_wave` tokens.  A row's logits sit in
 //                        registers (lane l holds experts l, l+64, ...); each of the k rounds is a
@@ -18,6 +19,8 @@
 //   route_scatter_kernel each wave re-reads its tokens' expert ids in flat (token-major) order, ranks
 //                        equal ids with ballots (stable), and writes both permutations plus the
 //                        optional gather index / gate value in expert-sorted order.
+//   route_place_kernel   the last two in one launch.
+//   route_few_kernel, route_small_kernel   all of it in one workgroup.
 #include <mutex>
 
 #include "common.h"
@@ -567,10 +570,10 @@ __global__ __launch_bounds__(kScanThreads) void ragged_remap_kernel(const RemapP
 // reads, all lanes reading the same address), and the ragged metadata follows.  One launch instead of three:
 // at decode batch sizes the pass is pure launch latency.
 constexpr int kSmallEntries = 1024;
-// ... and is USED up to this many entries: the single workgroup is bound by one CU's instruction rate (sixteen waves share
-// four SIMDs), so its top-k phase grows with the batch (inside the launch 6.6 us at 64 entries, 9.9 at 256, 22.7 at 1024)
-// while the three kernels, spread over the chip, stay at 20 us from launch to end: at 384 / 512 / 768 / 1024 entries a
-// replayed graph measured 24.8 / 27.2 / 34.4 / 42.6 us for the single launch against 19.8 / 20.5 / 19.8 / 20.5.
+// ... and is USED for what route_few_kernel does not take (given indices, more experts) up to 256 entries: the single workgroup is bound by one
+// CU's instruction rate (sixteen waves share four SIMDs), so its top-k phase grows with the batch, while several launches spread over the
+// chip: 384 / 512 / 768 / 1024 entries take 24.8 / 27.2 / 34.4 / 42.6 us against 19.8 / 20.5 / 19.8 / 20.5 of three launches in a replayed graph.
+// Against route_topk_kernel and route_place_kernel it wins up to 16 rows (128 experts, top 4: 16 rows 7.6 against 8.0 us, 64 15.2 against 8.2).
 constexpr int kSmallCut = 256;
 
 struct SmallParams {
@@ -831,6 +834,174 @@ __global__ __launch_bounds__(kScanThreads) void route_small_kernel(const SmallPa
   }
 }
 
+// ---- the whole pass in one workgroup for up to 128 experts ------------------------------------------------
+// A row belongs to LPR lanes with VPL keys each, so that the workgroup has all rows in hand at once where it can (128 rows of up to 16
+// experts, 64 of up to 128); an entry's rank comes from bit masks of the entries of each expert (eight words for 256 entries), as does the
+// histogram; the row offsets and the block offsets of the five sizes are scanned by a wave each.
+// What bounds it: a chain of latencies of one workgroup (logits, k selections, masks, scan, stores), and its instructions, which every launch
+// fetches from memory.  Against route_small_kernel, which did these sizes (us, in a replayed graph): 8 experts, top 2: 32 tokens 6.0 -> 3.3, 128
+// 10.1 -> 3.5; 128 experts, top 4: 1 token 5.8 -> 4.5, 64 15.2 -> 8.0.
+
+template <int LPR, class F>
+__device__ __forceinline__ int row_reduce(int x, F&& f) {
+  x = f(x, __builtin_amdgcn_update_dpp(0, x, TK_DPP_QUAD_XOR1, 0xF, 0xF, false));
+  x = f(x, __builtin_amdgcn_update_dpp(0, x, TK_DPP_QUAD_XOR2, 0xF, 0xF, false));
+  if constexpr (LPR >= 8) x = f(x, __builtin_amdgcn_update_dpp(0, x, TK_DPP_ROW_HALF_MIRROR, 0xF, 0xF, false));
+  if constexpr (LPR >= 16) x = f(x, __builtin_amdgcn_update_dpp(0, x, TK_DPP_ROW_MIRROR, 0xF, 0xF, false));
+  return x;
+}
+
+template <int DT, int LPR, int VPL, int WORDS>
+__global__ __launch_bounds__(LPR == 16 ? 1024 : 512) void route_few_kernel(const SmallParams q) {
+  constexpr int NT = LPR == 16 ? 1024 : 512, RPP = NT / LPR;  // rows of a pass
+  constexpr int kExperts = LPR * VPL, kEntries = WORDS * 32;
+  __shared__ __attribute__((aligned(16))) uint32_t mask_s[kExperts][WORDS];  // entries of an expert
+  __shared__ int16_t eid_s[kEntries];
+  __shared__ uint32_t val_s[kEntries];
+  __shared__ int32_t offs_s[kQuantities][kExperts + 1];
+  const TopkParams& p = q.t;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int E = p.E, k = p.k, T = p.T, R = T * k, words = (E + 31) / 32;
+  const int n_rows = p.n_rows_ptr ? *p.n_rows_ptr : p.n_rows_imm, n_live = T < n_rows ? T : n_rows;
+  const int l = tid % LPR;
+  for (int i = tid; i < E * WORDS; i += NT) (&mask_s[0][0])[i] = 0u;
+  for (int i = tid; i < R; i += NT) eid_s[i] = -1;
+  __syncthreads();
+#pragma unroll 1
+  for (int row0 = wave * (64 / LPR); row0 < n_live; row0 += RPP) {  // (a wave without rows leaves the SIMD to the others)
+    const int row = row0 + lane / LPR;
+    const bool row_ok = row < n_live;
+    uint32_t key[VPL];
+    uint32_t retired = 0;
+    const int64_t at = (int64_t)(row < T ? row : T - 1) * p.stride_m;
+    float v[VPL];
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) {
+      const int e = l * VPL + i;
+      v[i] = load_logit<DT>(p.logits, at + (e < E ? e : E - 1));
+      retired |= (e >= E ? 1u : 0u) << i;
+    }
+#pragma unroll
+    for (int i = 0; i < VPL; ++i) key[i] = ordered_key(v[i]);
+    // as row16_topk: the largest key still in the running, ties to the lowest expert; round j's winner stays with lane j of the row
+    uint32_t my_key = 0, key0 = 0;
+    int my_idx = -1;
+#pragma unroll 1
+    for (int j = 0; j < k; ++j) {
+      uint32_t m = 0;
+#pragma unroll
+      for (int i = 0; i < VPL; ++i) m = (!((retired >> i) & 1u) && key[i] > m) ? key[i] : m;
+      m = (uint32_t)row_reduce<LPR>((int)m, [](int x, int y) { return (uint32_t)x > (uint32_t)y ? x : y; });
+      int idx = 0x7FFFFFFF;
+#pragma unroll
+      for (int i = VPL - 1; i >= 0; --i) idx = (!((retired >> i) & 1u) && key[i] == m) ? l * VPL + i : idx;
+      idx = row_reduce<LPR>(idx, [](int x, int y) { return x < y ? x : y; });
+      const int mine = idx - l * VPL;
+      if (mine >= 0 && mine < VPL) retired |= 1u << mine;
+      if (j == 0) key0 = m;
+      if (j == l) my_key = m, my_idx = idx;
+    }
+    float out = key_to_float(my_key);
+    if (p.apply_softmax) {
+      const float z = l < k ? expf(out - key_to_float(key0)) : 0.f;
+      const float sum = __builtin_bit_cast(float, row_reduce<LPR>(__builtin_bit_cast(int, z), [](int x, int y) {
+        return __builtin_bit_cast(int, __builtin_bit_cast(float, x) + __builtin_bit_cast(float, y));
+      }));
+      out = z / sum;
+    }
+    const bool live = row_ok && l < k && my_idx >= 0 && my_idx < E;
+    if (row_ok && l < k) {
+      const int f = row * k + l;
+      if (p.vals) store_val<DT>(p.vals, f, out);
+      p.indx[f] = (int16_t)(live ? my_idx : -1);
+      val_s[f] = DT == TK_F32 ? f32_bits(out) : DT == TK_BF16 ? f32_to_bf16_bits(out) : f32_to_f16_bits(out);
+      if (live) {
+        eid_s[f] = (int16_t)my_idx;
+        atomicOr(&mask_s[my_idx][f >> 5], 1u << (f & 31));
+      }
+    }
+    if (p.bitmatrix) {
+#pragma unroll
+      for (int w = 0; w < kExperts / 32 || w == 0; ++w) {
+        const int bits = row_reduce<LPR>(live && (my_idx >> 5) == w ? (int)(1u << (my_idx & 31)) : 0, [](int x, int y) { return x | y; });
+        if (row_ok && l == w && w < words) p.bitmatrix[(int64_t)w * p.bm_stride_w + row] = (uint32_t)bits;
+      }
+    }
+  }
+  __syncthreads();
+  if (!q.col_sum) return;  // top-k only
+  if (wave < (q.want_ragged ? kQuantities : 1)) {
+    // wave 0: the experts' rows; wave 1 + b: their row blocks of size 16 << b
+    const int up = wave == 0 ? 0 : kFirstBlockLog2 + wave - 1, most = wave == 0 ? 0 : (1 << up) - 1;
+    int32_t* to = !q.want_ragged ? nullptr : wave == 0 ? q.r.slice_offs : q.r.block_offs + (wave - 1) * q.r.block_offs_stride;
+    int run = 0;
+#pragma unroll 1
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane;
+      int rows = 0;
+      if (e < E) {
+#pragma unroll
+        for (int w = 0; w < WORDS; w += 4) {
+          const uint4 a = *reinterpret_cast<const uint4*>(&mask_s[e][w]);
+          rows += __popc(a.x) + __popc(a.y) + __popc(a.z) + __popc(a.w);
+        }
+        if (wave == 0) q.col_sum[e] = rows;
+      }
+      const int v = (rows + most) >> up, inc = wave_scan_i32(v);
+      if (e < E) {
+        offs_s[wave][e] = run + inc - v;
+        if (to) to[e] = run + inc - v;
+      }
+      run += __builtin_amdgcn_readlane(inc, 63);
+    }
+    if (lane == 0) {
+      offs_s[wave][E] = run;
+      if (to) to[E] = run;
+    }
+  }
+  __syncthreads();
+  const int total = offs_s[0][E];
+#pragma unroll 1
+  for (int f = tid; f < R; f += NT) {
+    const int e = eid_s[f];
+    int pos = -1;
+    if (e >= 0) {
+      pos = offs_s[0][e] + __popc(mask_s[e][f >> 5] & ((1u << (f & 31)) - 1u));
+#pragma unroll 4
+      for (int w = 0; w < f >> 5; ++w) pos += __popc(mask_s[e][w]);
+      q.col_sorted[pos] = f;
+      if (q.gather_out) q.gather_out[pos] = f / k;
+      if (q.gammas_out) {
+        if (q.vals_bytes == 4)
+          static_cast<uint32_t*>(q.gammas_out)[pos] = val_s[f];
+        else
+          static_cast<uint16_t*>(q.gammas_out)[pos] = (uint16_t)val_s[f];
+      }
+    }
+    q.row_sorted[f] = pos;
+    // positions past the routed entries
+    if (f >= total) {
+      q.col_sorted[f] = -1;
+      if (q.gather_out) q.gather_out[f] = -1;
+    }
+  }
+  if (!q.want_ragged) return;
+  for (int slot = NT - 1 - tid; slot < kNumBlockSizes * q.r.max_n_blocks; slot += NT) {
+    const int b = slot / q.r.max_n_blocks, i = slot - b * q.r.max_n_blocks;
+    const int32_t* offs = offs_s[1 + b];
+    int val = -1;
+    if (i < offs[E]) {
+      int lo = 0, hi = E;  // largest e with offs[e] <= i; empty slices share an offset, the last one wins
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (offs[mid] <= i) lo = mid; else hi = mid;
+      }
+      val = ((i - offs[lo]) << 16) | lo;
+    }
+    q.r.block_sched[b * q.r.block_sched_stride + i] = val;
+  }
+}
+
 struct ScatterParams {
   const int16_t* indx16;  // [T, k] (one of indx16 / indx32)
   const int32_t* indx32;
@@ -849,28 +1020,10 @@ struct ScatterParams {
   int32_t vals_bytes;       // 2 or 4
 };
 
-__global__ __launch_bounds__(kWaves * 64) void route_scatter_kernel(const ScatterParams p) {
-  __shared__ int32_t base_s[kWaves][kMaxExperts];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int unit = blockIdx.x * kWaves + wave;
+// A wave's rows [row_begin, row_end): ranks equal experts in flat order and writes the permutations; base[e] = position of the wave's
+// next entry of expert e.
+__device__ __forceinline__ void scatter_rows(const ScatterParams& p, int32_t* base, int row_begin, int row_end, int n_rows, int lane) {
   const int E = p.E, k = p.k;
-  const int n_rows = p.n_rows_ptr ? *p.n_rows_ptr : p.n_rows_imm;
-  const int row_begin = unit * p.rows_per_wave;
-  if (row_begin >= p.T) return;
-  int row_end = row_begin + p.rows_per_wave;
-  row_end = row_end < p.T ? row_end : p.T;
-  // first position of this wave's entries of expert e: the expert's offset, its entries in earlier workgroups and in
-  // the earlier waves of this one (all loads independent of each other)
-  for (int e = lane; e < E; e += 64) {
-    int b = p.col_offs[e] + p.wg_prefix[(int64_t)blockIdx.x * E + e];
-    int prev[kWaves - 1];
-#pragma unroll
-    for (int w = 0; w < kWaves - 1; ++w) prev[w] = w < wave ? p.partials[(int64_t)(blockIdx.x * kWaves + w) * E + e] : 0;
-#pragma unroll
-    for (int w = 0; w < kWaves - 1; ++w) b += prev[w];
-    base_s[wave][e] = b;
-  }
-  wave_sync();
   const int64_t f_begin = (int64_t)row_begin * k, f_end = (int64_t)row_end * k;
   const int64_t n_valid = (int64_t)(n_rows < p.T ? n_rows : p.T) * k;
   const unsigned long long lt_mask = (1ull << lane) - 1ull;
@@ -890,9 +1043,9 @@ __global__ __launch_bounds__(kWaves * 64) void route_scatter_kernel(const Scatte
       const int leader = __ffsll((long long)todo) - 1;
       const int e0 = __shfl(e, leader);
       const unsigned long long same = __ballot(valid && e == e0);
-      if (valid && e == e0) pos = base_s[wave][e0] + __popcll(same & lt_mask);
+      if (valid && e == e0) pos = base[e0] + __popcll(same & lt_mask);
       wave_sync();
-      if (lane == leader) base_s[wave][e0] = base_s[wave][e0] + __popcll(same);
+      if (lane == leader) base[e0] = base[e0] + __popcll(same);
       wave_sync();
       todo &= ~same;
     }
@@ -907,6 +1060,141 @@ __global__ __launch_bounds__(kWaves * 64) void route_scatter_kernel(const Scatte
           static_cast<uint16_t*>(p.gammas_out)[pos] = (uint16_t)gate_bits;
       }
     }
+  }
+}
+
+__global__ __launch_bounds__(kWaves * 64) void route_scatter_kernel(const ScatterParams p) {
+  __shared__ int32_t base_s[kWaves][kMaxExperts];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int unit = blockIdx.x * kWaves + wave;
+  const int E = p.E;
+  const int n_rows = p.n_rows_ptr ? *p.n_rows_ptr : p.n_rows_imm;
+  const int row_begin = unit * p.rows_per_wave;
+  if (row_begin >= p.T) return;
+  int row_end = row_begin + p.rows_per_wave;
+  row_end = row_end < p.T ? row_end : p.T;
+  // first position of this wave's entries of expert e: the expert's offset, its entries in earlier workgroups and in
+  // the earlier waves of this one (all loads independent of each other)
+  for (int e = lane; e < E; e += 64) {
+    int b = p.col_offs[e] + p.wg_prefix[(int64_t)blockIdx.x * E + e];
+    int prev[kWaves - 1];
+#pragma unroll
+    for (int w = 0; w < kWaves - 1; ++w) prev[w] = w < wave ? p.partials[(int64_t)(blockIdx.x * kWaves + w) * E + e] : 0;
+#pragma unroll
+    for (int w = 0; w < kWaves - 1; ++w) b += prev[w];
+    base_s[wave][e] = b;
+  }
+  wave_sync();
+  scatter_rows(p, base_s[wave], row_begin, row_end, n_rows, lane);
+}
+
+// The scan and the scatter in one launch, for up to kPlaceExperts experts: every workgroup sums the workgroups' histograms for itself (all of
+// them for the experts' offsets, those in front of it for its own entries: at most 256 rows of 1 KiB, from L2) instead of waiting for a
+// launch in which one workgroup does; six more write the totals, offsets and schedules meanwhile.
+// What bounds it: a chain of latencies (totals, scan, ranks, stores).  The pass (top-k, this) of
+// 4096 tokens, 128 experts, top 4: 23.0 -> 15.5 us, 300 tokens 14.3 -> 9.2, 2048 tokens, 16 experts, top 2: 13.0 -> 8.7.
+constexpr int kPlaceExperts = 256, kPlaceThreads = kWaves * 64;
+struct PlaceParams {
+  ScatterParams s;
+  const int32_t* totals;  // [workgroups][E]
+  int32_t workgroups;
+  int32_t* col_sum;
+  RaggedOut r;
+};
+
+__global__ __launch_bounds__(kPlaceThreads) void route_place_kernel(const PlaceParams q) {
+  __shared__ int4 sum_s[2][kPlaceThreads];  // a group's sums: all workgroups, those in front
+  __shared__ int32_t total_s[kPlaceExperts], offs_s[kPlaceExperts + 1], front_s[kPlaceExperts];
+  __shared__ int32_t base_s[kWaves][kPlaceExperts];
+  const ScatterParams& p = q.s;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int E = p.E, n_wg = q.workgroups, wg = blockIdx.x;
+  const int w4 = E / 4, c = tid % w4, g = tid / w4;  // four experts; the rows g, g + groups, ...
+  int groups = kPlaceThreads / w4;
+  groups = groups < 16 ? groups : 16;
+  if (g < groups) {
+    const int4* rows = reinterpret_cast<const int4*>(q.totals);
+    int4 all = make_int4(0, 0, 0, 0), front = all;
+    constexpr int kBatch = 8;
+#pragma unroll 1
+    for (int r0 = g; r0 < n_wg; r0 += groups * kBatch) {
+      int4 v[kBatch];
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        const int r = r0 + i * groups;
+        v[i] = r < n_wg ? rows[(int64_t)r * w4 + c] : make_int4(0, 0, 0, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < kBatch; ++i) {
+        all.x += v[i].x, all.y += v[i].y, all.z += v[i].z, all.w += v[i].w;
+        if (r0 + i * groups < wg) front.x += v[i].x, front.y += v[i].y, front.z += v[i].z, front.w += v[i].w;
+      }
+    }
+    sum_s[0][g * w4 + c] = all;
+    sum_s[1][g * w4 + c] = front;
+  }
+  __syncthreads();
+  if (tid < E) {
+    const int32_t *a = reinterpret_cast<const int32_t*>(sum_s[0]) + tid, *f = reinterpret_cast<const int32_t*>(sum_s[1]) + tid;
+    int all = 0, front = 0;
+    for (int i = 0; i < groups; ++i) all += a[i * E], front += f[i * E];
+    total_s[tid] = all;
+    front_s[tid] = front;
+  }
+  __syncthreads();
+  // workgroup n_wg: offsets of the experts' rows; n_wg + 1 ..: of their row blocks
+  const int block = wg - n_wg - 1, up = block < 0 ? 0 : kFirstBlockLog2 + block, most = block < 0 ? 0 : (1 << up) - 1;
+  if (wave == 0) {
+    int run = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane, v = e < E ? (total_s[e] + most) >> up : 0, inc = wave_scan_i32(v);
+      if (e < E) offs_s[e] = run + inc - v;
+      run += __builtin_amdgcn_readlane(inc, 63);
+    }
+    if (lane == 0) offs_s[E] = run;
+  }
+  if (wg < n_wg) {
+    const int unit = wg * kWaves + wave, row_begin = unit * p.rows_per_wave;
+    int row_end = row_begin + p.rows_per_wave;
+    row_end = row_end < p.T ? row_end : p.T;
+    const int n_rows = p.n_rows_ptr ? *p.n_rows_ptr : p.n_rows_imm;
+    int prev[kPlaceExperts / 64];
+    for (int i = 0; i < kPlaceExperts / 64; ++i) {
+      const int e = i * 64 + lane;
+      prev[i] = 0;
+      if (e < E)
+        for (int w = 0; w < wave; ++w) prev[i] += p.partials[(int64_t)(wg * kWaves + w) * E + e];
+    }
+    __syncthreads();
+    if (row_begin >= p.T) return;
+    for (int i = 0; i < kPlaceExperts / 64; ++i) {
+      const int e = i * 64 + lane;
+      if (e < E) base_s[wave][e] = offs_s[e] + front_s[e] + prev[i];
+    }
+    wave_sync();
+    scatter_rows(p, base_s[wave], row_begin, row_end, n_rows, lane);
+    return;
+  }
+  __syncthreads();
+  if (block < 0) {
+    for (int e = tid; e < E; e += kPlaceThreads) q.col_sum[e] = total_s[e];
+    if (q.r.slice_offs)
+      for (int e = tid; e <= E; e += kPlaceThreads) q.r.slice_offs[e] = offs_s[e];
+    return;
+  }
+  for (int e = tid; e <= E; e += kPlaceThreads) q.r.block_offs[block * q.r.block_offs_stride + e] = offs_s[e];
+  const int n = offs_s[E];
+  for (int i = tid; i < q.r.max_n_blocks; i += kPlaceThreads) {
+    int val = -1;
+    if (i < n) {
+      int lo = 0, hi = E;  // largest e with offs[e] <= i; empty slices share an offset, the last one wins
+      while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (offs_s[mid] <= i) lo = mid; else hi = mid;
+      }
+      val = ((i - offs_s[lo]) << 16) | lo;
+    }
+    q.r.block_sched[block * q.r.block_sched_stride + i] = val;
   }
 }
 
@@ -943,8 +1231,35 @@ int32_t launch_topk(const TopkParams& p, int units, hipStream_t st) {
   return fail(TK_ERR_UNSUPPORTED, "tk_route: more than %d experts", kMaxExperts);
 }
 
+// What route_few_kernel takes: k up to the lanes of a row and its entries, where its workgroup is done in two passes.  Measured in a replayed
+// graph (us, against route_topk_kernel and route_place_kernel): 16 experts, top 4, 256 tokens 7.2 against 7.5; 8 experts, top 2: 256 tokens 5.1
+// against 7.1, 512 (four passes) 7.5 against 7.2; 32 experts, top 4: 128 tokens 6.6 against 7.4, 256 (four) 10.0 against 7.7.
+bool few_takes(int T, int E, int k) {
+  const int64_t R = (int64_t)T * k;
+  if (E <= 16 && k <= 4) return T <= 256 && R <= 1024;
+  if (E <= 32 && k <= 8) return T <= 128 && R <= 1024;
+  return E <= 128 && k <= 16 && T <= 128 && R <= 256;
+}
+
+template <int DT>
+bool launch_few(const SmallParams& q, hipStream_t st) {
+  const int E = q.t.E, k = q.t.k, R = q.t.T * k;
+  if (q.t.use_provided_indx || !few_takes(q.t.T, E, k)) return false;
+  auto launch = [&](auto kern, int threads) { hipLaunchKernelGGL(kern, dim3(1), dim3(threads), 0, st, q); };
+  if (E <= 16 && k <= 4)
+    R <= 256 ? launch(route_few_kernel<DT, 4, 4, 8>, 512) : launch(route_few_kernel<DT, 4, 4, 32>, 512);
+  else if (E <= 32 && k <= 8)
+    R <= 256 ? launch(route_few_kernel<DT, 8, 4, 8>, 512) : launch(route_few_kernel<DT, 8, 4, 32>, 512);
+  else if (E <= 64)
+    launch(route_few_kernel<DT, 16, 4, 8>, 1024);
+  else
+    launch(route_few_kernel<DT, 16, 8, 8>, 1024);
+  return true;
+}
+
 template <int DT>
 int32_t launch_small_dt(const SmallParams& q, hipStream_t st) {
+  if (launch_few<DT>(q, st)) return check_launch("route_few_kernel");
   const int epl = (q.t.E + 63) / 64;
 #define TK_EPL(N)                                                                                              \
   if (epl <= N) {                                                                                              \
@@ -1024,7 +1339,9 @@ static int32_t route_impl(const tk_route_desc* d, void* workspace, tk_stream_t s
   tp.fill_a = want_meta ? d->col_sorted_indx : nullptr;
   tp.fill_b = want_meta ? d->row_sorted_indx : nullptr;
   tp.fill_c = want_meta ? d->gather_indx : nullptr;
-  if ((int64_t)T * k <= kSmallCut) {
+  const bool place = E <= kPlaceExperts && E % 4 == 0 && (reinterpret_cast<uintptr_t>(wg_totals) & 15) == 0;
+  const bool few = !d->use_provided_indx && few_takes(T, E, k);
+  if (few || ((int64_t)T * k <= kSmallCut && (d->use_provided_indx || T <= 16 || !place))) {
     // small batch: the whole pass in one launch
     SmallParams sq;
     sq.t = tp;
@@ -1068,10 +1385,6 @@ static int32_t route_impl(const tk_route_desc* d, void* workspace, tk_stream_t s
   ro.max_n_blocks = d->max_n_blocks;
   const int want_ragged = d->slice_offs != nullptr;
   if (want_ragged && (!d->block_offs || (!d->block_schedule && d->max_n_blocks > 0))) return fail(TK_ERR_INVALID, "tk_route: incomplete ragged outputs");
-  hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3(kScanThreads), 0, st, wg_totals, units_pad / kWaves, E, d->col_sum, col_offs, want_ragged, ro);
-  rc = check_launch("route_scan_kernel");
-  if (rc != TK_OK) return rc;
-
   ScatterParams sp;
   sp.indx16 = static_cast<const int16_t*>(d->indx);
   sp.indx32 = nullptr;
@@ -1090,7 +1403,16 @@ static int32_t route_impl(const tk_route_desc* d, void* workspace, tk_stream_t s
   sp.vals = d->vals;
   sp.gammas_out = d->vals ? d->gammas : nullptr;
   sp.vals_bytes = (d->logits_dtype == TK_F32 || !d->logits) ? 4 : 2;
-  hipLaunchKernelGGL(route_scatter_kernel, dim3(units_pad / kWaves), dim3(kWaves * 64), 0, st, sp);
+  const int workgroups = units_pad / kWaves;
+  if (place) {
+    const PlaceParams pp{sp, wg_totals, workgroups, d->col_sum, ro};
+    hipLaunchKernelGGL(route_place_kernel, dim3(workgroups + (want_ragged ? 1 + kNumBlockSizes : 1)), dim3(kPlaceThreads), 0, st, pp);
+    return check_launch("route_place_kernel");
+  }
+  hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3(kScanThreads), 0, st, wg_totals, workgroups, E, d->col_sum, col_offs, want_ragged, ro);
+  rc = check_launch("route_scan_kernel");
+  if (rc != TK_OK) return rc;
+  hipLaunchKernelGGL(route_scatter_kernel, dim3(workgroups), dim3(kWaves * 64), 0, st, sp);
   return check_launch("route_scatter_kernel");
 }
 
