@@ -313,14 +313,19 @@ __global__ __launch_bounds__(256) void ragged_k_gemm_kernel(const RaggedKParams 
 // get an offset beyond the buffer resource; the hardware then writes zeros to LDS.
 //
 // What bounds it: writing y.  The same kernel without its loads writes 128 x [2880, 5760] bf16 in 0.77 ms (5.5 TB/s),
-// without its stores it takes 0.85 ms; together 1.21 ms (3.1 ms with the transposition in registers; 2880 x 2880: 1.5 -> 0.62).
+// without its stores it takes 0.85 ms; together 1.13 ms (3.1 ms with the transposition in registers; 2880 x 2880: 1.5 -> 0.62).
 //   * the results go through LDS so that a store instruction writes whole 128-byte lines, with the non-temporal hint
 //     (pieces of 32 bytes: 1.76 ms; with the hint on such pieces 4.0, plain whole lines 1.55, whole lines with the hint 1.40);
 //   * stages of 16 k, five buffers, four workgroups per CU: four fifths of the LDS are loads in flight (three buffers
 //     of 32 k and three workgroups: 1.44), and a slice is padded to 16 k only;
 //   * every XCD gets an eighth of EVERY slice: slices differ in length by factors, and with whole slices dealt to the
 //     XCDs the longest sum decided (1.40 -> 1.21 ms); columns of tiles run first, so an XCD's eighth touches all of a and
-//     an eighth of b.
+//     an eighth of b;
+//   * a tile of 128 k is two turns of the ring, and each waited for its first touch of memory behind the stream of stores: the lines are
+//     asked for two slices ahead (128 equal slices of 128 k 1.19 -> 1.06 ms, random lengths 1.22 -> 1.13; one slice ahead 1.17, three 1.16, every
+//     tile asking for b 1.22).
+// Measured and left out: 128 x 256 tiles, with the same ring or by persistent workgroups whose ring runs on across tiles, with loading
+// and storing waves apart (1.22 to 1.40 ms); slices mixed over an XCD's workgroups (1.25).
 constexpr int kTrK = 16;
 constexpr int kTrBufs = 5;
 constexpr int kTrOperand = kTrK * kTile * 2;   // bytes of one operand's stage
@@ -362,6 +367,7 @@ __global__ __launch_bounds__(256, 4) void ragged_k_tr_kernel(const RaggedKParams
     pid = (round * 8 + x) * q + (l - round * q);
   }
   if (pid >= p.n_slices * per_e) return;
+  const int later = pid + 16 * p.chunk;  // the tile that this XCD comes to two rounds later
   const int e = pid / per_e;
   pid -= e * per_e;
   const int tn = pid / p.tiles_m;
@@ -450,6 +456,19 @@ __global__ __launch_bounds__(256, 4) void ragged_k_tr_kernel(const RaggedKParams
       wr = wr == kLast ? 0 : wr + kTrStage;
     }
   }
+  // ---- ask for lines of the later tile's operands (128 k of a's columns; of b's, which more tiles share, one tile in eight), so that L2 has them.
+  // Nothing waits for these loads but the end, behind the stores.
+  uint32_t ahead_a = 0, ahead_b = 0;
+  if (later < p.n_slices * per_e) {
+    const int e2 = later / per_e, in_e2 = later - e2 * per_e, tn2 = in_e2 / p.tiles_m, tm2 = in_e2 - tn2 * p.tiles_m;
+    const int k = tid >> 1, col = (tid & 1) * 64;
+    if (k < p.sizes[e2]) {
+      const __amdgpu_buffer_rsrc_t qa = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.a), 0, p.a_bytes, 0x00020000);
+      const __amdgpu_buffer_rsrc_t qb = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.b), 0, p.b_bytes, 0x00020000);
+      ahead_a = __builtin_amdgcn_raw_buffer_load_b32(qa, (uint32_t)(p.a_offs[e2] + k) * a_step + (uint32_t)(tm2 * kTile + col) * 2u, 0, 0);
+      if ((tm2 & 7) == 0) ahead_b = __builtin_amdgcn_raw_buffer_load_b32(qb, (uint32_t)(p.b_offs[e2] + k) * b_step + (uint32_t)(tn2 * kTile + col) * 2u, 0, 0);
+    }
+  }
   // ---- store: a lane's accumulator quad is four columns of one row; the lane halves exchange quads, so a lane stores
   // eight consecutive columns (16-bit) or four (fp32), through a resource that drops rows past M and columns past N ----
   constexpr uint32_t ES = YT == TK_F32 ? 4 : 2;
@@ -506,6 +525,7 @@ __global__ __launch_bounds__(256, 4) void ragged_k_tr_kernel(const RaggedKParams
       __builtin_amdgcn_raw_buffer_store_b128(q, ry, off, 0, kNonTemporal);
     }
   }
+  asm volatile("" ::"v"(ahead_a), "v"(ahead_b));
 }
 
 }  // namespace
