@@ -122,3 +122,21 @@ def test_ragged_k_stage_and_tile_edges(device, m, n, out_dtype):
               precision_config=mm.PrecisionConfig(out_dtype=out_dtype))
     ref = omoe.matmul_ragged_k(a.t(), b, sizes, offs, offs, out_dtype=torch.float32)
     assert_allclose_gate(ref, out.float(), what="ragged-K matmul")
+
+
+@pytest.mark.parametrize("n_slices, m, n", [(70, 2040, 2168), (64, 2048, 2048), (63, 2040, 2168), (64, 1920, 2168)])
+def test_operands_asked_for_ahead(device, n_slices, m, n):
+    """From 64 slices and 32 tiles of a slice per XCD on, tiles ask for lines of later slices: some of these are empty, some long, the last
+    ones have no successor, and both sides of the line.  The sum is exact but for its order (fp32) and the result's rounding to bf16, half of 2^-8."""
+    import triton_amd.matmul as mm
+    g = torch.Generator().manual_seed(n_slices + m)
+    sizes = torch.randint(0, 12, (n_slices, ), generator=g).to(torch.int32)
+    sizes[3], sizes[5], sizes[-1] = 0, 250, 200
+    offs = _offsets(sizes, None)
+    a, b = torch.randn((int(offs[-1]), m), generator=g).to(torch.bfloat16).to(device), torch.randn((int(offs[-1]), n), generator=g).to(torch.bfloat16).to(device)
+    md = _metadata(sizes, offs, device)
+    out = mm.matmul(a.t(), b, None, a_ragged_metadata=md, b_ragged_metadata=md)
+    for e in range(n_slices):
+        k = slice(int(offs[e]), int(offs[e + 1]))
+        ref = a[k].float().t() @ b[k].float()
+        assert ((out[e].float() - ref).abs() <= ref.abs() * 2**-8 + 1e-4).all(), e

@@ -37,6 +37,7 @@ struct RaggedKParams {
   int M, N;
   int tiles_m, tiles_n;
   int chunk, n_slices;  // aligned variant: tiles per XCD and turn
+  int ahead;            // ... how many tiles ahead operands are asked for, 0 = not at all
   int y_dtype;
   uint32_t a_bytes, b_bytes, y_bytes;  // extents for the buffer resources of the aligned variant (y: one slice)
   int a_vec, b_vec;  // the operand's base and strides allow 16-byte loads along its contiguous dimension
@@ -322,8 +323,8 @@ __global__ __launch_bounds__(256) void ragged_k_gemm_kernel(const RaggedKParams 
 //     XCDs the longest sum decided (1.40 -> 1.21 ms); columns of tiles run first, so an XCD's eighth touches all of a and
 //     an eighth of b;
 //   * a tile of 128 k is two turns of the ring, and each waited for its first touch of memory behind the stream of stores: the lines are
-//     asked for two slices ahead (128 equal slices of 128 k 1.19 -> 1.06 ms, random lengths 1.22 -> 1.13; one slice ahead 1.17, three 1.16, every
-//     tile asking for b 1.22).
+//     asked for whole slices ahead, beyond the 128 tiles that an XCD has in flight (128 equal slices of 128 k, 258 tiles or two slices ahead,
+//     1.19 -> 1.06 ms, random lengths 1.22 -> 1.13; one slice 1.17, three 1.16, every tile asking for b 1.22).
 // Measured and left out: 128 x 256 tiles, with the same ring or by persistent workgroups whose ring runs on across tiles, with loading
 // and storing waves apart (1.22 to 1.40 ms); slices mixed over an XCD's workgroups (1.25).
 constexpr int kTrK = 16;
@@ -367,7 +368,7 @@ __global__ __launch_bounds__(256, 4) void ragged_k_tr_kernel(const RaggedKParams
     pid = (round * 8 + x) * q + (l - round * q);
   }
   if (pid >= p.n_slices * per_e) return;
-  const int later = pid + 16 * p.chunk;  // the tile that this XCD comes to two rounds later
+  const int later = pid + p.ahead;  // a tile that this XCD comes to some rounds later
   const int e = pid / per_e;
   pid -= e * per_e;
   const int tn = pid / p.tiles_m;
@@ -459,7 +460,7 @@ __global__ __launch_bounds__(256, 4) void ragged_k_tr_kernel(const RaggedKParams
   // ---- ask for lines of the later tile's operands (128 k of a's columns; of b's, which more tiles share, one tile in eight), so that L2 has them.
   // Nothing waits for these loads but the end, behind the stores.
   uint32_t ahead_a = 0, ahead_b = 0;
-  if (later < p.n_slices * per_e) {
+  if (p.ahead && later < p.n_slices * per_e) {
     const int e2 = later / per_e, in_e2 = later - e2 * per_e, tn2 = in_e2 / p.tiles_m, tm2 = in_e2 - tn2 * p.tiles_m;
     const int k = tid >> 1, col = (tid & 1) * 64;
     if (k < p.sizes[e2]) {
@@ -585,6 +586,11 @@ extern "C" int32_t tk_ragged_k_gemm(const tk_ragged_k_desc* d, tk_stream_t strea
     const int per_e = p.tiles_m * p.tiles_n;
     p.chunk = per_e >= 8 ? per_e / 8 : 1;
     p.n_slices = d->n_slices;
+    // An XCD's part of a slice below 32 tiles: lines asked for six and more slices ahead are gone again or not yet of use (both products of a layer,
+    // 16384 rows, 128 slices, 15 and 8 tiles: 165 us without against 173; 23 and 12: 385 / 391; 36 and 18: 545 / 556; 31 and 16: 420 / 420;
+    // 33 and 17: 478 / 477; 45 and 23: 685 / 659; 68 and 35: 1010 / 970).  Fewer than 64 slices: what there is to wait for is less (2880 x 5760 and
+    // 2880 x 2880, 32 slices of 128 389 / 393, 8 of 2048 933 / 942; 2048 x 4096 and 2048 x 2048, 64 slices of 128 472 / 462).
+    p.ahead = p.chunk >= 32 && d->n_slices >= 64 ? 8 * p.chunk * (int)cdiv(192, p.chunk) : 0;
     const int64_t chunks = cdiv((int64_t)d->n_slices * per_e, p.chunk);
     grid = cdiv(chunks, 8) * 8 * p.chunk;
     auto with_y = [&](auto dt) {
