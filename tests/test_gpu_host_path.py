@@ -222,3 +222,40 @@ def test_activations_of_another_form_are_refused_by_the_general_path(device, red
     act = mm.FusedActivation(mm.FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=reduction_n), (1.702, 7.0))
     with pytest.raises(NotImplementedError):
         mm.matmul(x, w, None, md, fused_activation=act)
+
+
+@pytest.mark.parametrize("dtype, swiglu", [(torch.bfloat16, False), (torch.float16, True)])
+def test_rows_of_a_token_are_summed_by_the_same_call(device, monkeypatch, dtype, swiglu):
+    """The GEMM's native call launches the combine too; results are seen by a dispatch mode, and filled in deterministic mode, as torch's own are."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    from triton_amd.legacy import matmul_ogs, routing
+    from triton_amd.matmul import FnSpecs, FusedActivation
+    from triton_amd.swiglu import swiglu_fn
+    g = torch.Generator().manual_seed(3)
+    x, w = torch.randn((40, 72), generator=g).to(dtype).to(device), torch.randn((6, 24, 72), generator=g).to(dtype).to(device).transpose(1, 2)
+    bias, logits = torch.randn((6, 24), generator=g).to(device), torch.randn((40, 6), generator=g).to(device)
+    act = FusedActivation(FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0)) if swiglu else None
+    rd, gather, scatter = routing(logits, 2)
+
+    def run():
+        return matmul_ogs(x, w, bias, rd, gather_indx=gather, scatter_indx=scatter, gammas=rd.gate_scal, fused_activation=act)
+    plain = _both(monkeypatch, run)
+    assert plain.shape == (40, 12 if swiglu else 24)
+
+    class Seen(TorchDispatchMode):
+        ops = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.ops.append(func)
+            return func(*args, **(kwargs or {}))
+    with Seen() as mode:
+        _same(run(), plain)
+    assert mode.ops.count(torch.ops.aten.empty.memory_format) == 2
+    with torch.inference_mode():
+        assert run().is_inference()
+    torch.use_deterministic_algorithms(True)
+    try:
+        filled = run()
+    finally:
+        torch.use_deterministic_algorithms(False)
+    assert torch.equal(filled, plain) and filled._version == 1  # (the fill)

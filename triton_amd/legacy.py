@@ -99,7 +99,7 @@ def matmul_ogs(x, w, bias, routing_data: RoutingData | None = None, gather_indx:
     if scatter_indx is None:
         return y
     combined = getattr(y, "_tk_combined", None)
-    if combined is not None:  # decode shapes: the GEMM's last wave per token has already summed its k rows
+    if combined is not None:  # by the GEMM itself (decode shapes: its last wave per token), or launched with it
         return combined
     return combine_rows(y, k)
 

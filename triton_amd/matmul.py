@@ -465,7 +465,8 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
         Y[idxs_y_m(e), :] += matmul(X[idxs_x_m(e), :], W[e, :, :])
 
     `_combine_k` (used by `legacy.matmul_ogs`, not part of the reference's signature): with `scatter_indx` mapping rows
-    to flat positions t * k + j, the decode kernel may also sum the k rows of every token; the result is then attached to
+    to flat positions t * k + j, the k rows of every token may also be summed (inside the decode and the prefill kernel, or by a
+    launch that the native host path makes in the same call); the result is then attached to
     the returned tensor as `._tk_combined` ([tokens, N]) and the caller skips its `reduce`.  The caller vouches that
     EVERY token has exactly k routed rows: a token with fewer leaves its arrival counter non-zero for the next launch.
     """
