@@ -146,3 +146,12 @@ def test_few_large_tiles_run_as_small_ones(device, monkeypatch, dtype):
         small = mm.matmul(x.to(device), wd, None, md, precision_config=pc)
     assert_allclose_gate(omoe.matmul(x, w.transpose(1, 2), None, sizes, out_dtype=torch.float32), native, what=f"{dtype} few large tiles")
     assert torch.equal(native, general) and torch.equal(native, small)
+
+
+@pytest.mark.parametrize("swiglu", [False, True])
+@pytest.mark.parametrize("k", [32, 160, 272, 400])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16", "e4m3"])
+def test_narrow_tiles_of_short_row_blocks(device, dtype, k, swiglu):
+    """256 full tiles, one round, and short row blocks of 1, 128, 64 and 31 rows in tiles of 128 columns behind them: an odd and an even number of
+    stages' halves, and less than one."""
+    _check(device, dtype, 256, [257, 384, 320, 0, 31, 256, 256, 512, 256], k, 8184, swiglu=swiglu)

@@ -11,6 +11,7 @@ constexpr int kSliceRegs = kDmaSlices / 64;
 
 struct Tile {
   int expert, off_m, start_m, eM, n_tile;
+  bool narrow;
 };
 
 // Two lists: row blocks that are more than half full, then the short last blocks of the experts, which cost a fraction of a tile;
@@ -18,10 +19,14 @@ struct Tile {
 // XCD (workgroup b runs on XCD b % 8) takes a contiguous part, walked side by side by its workgroups, the short tiles behind the
 // others: the workgroups without a tile in the last round of full ones begin with them.
 // Slice sizes and offsets stay in registers, lane l of register c holding slice c * 64 + l.
-template <int BM, int BN>
+// SBN < BN: short row blocks may be cut into tiles of SBN columns instead ("narrow"): where those of the whole width neither find room beside the
+// last full tiles nor keep more than half of the workgroups busy behind them.  (256 workgroups, K 2048, N 4096: 256 full and 112 short
+// tiles 95.5 -> 85 us; 128 full and 128 short tiles, which are one round, 47 against 59 in narrow ones.)
+template <int BM, int BN, int SBN = BN>
 struct TileList {
   int sz[kSliceRegs], so[kSliceRegs];
-  int f_beg, f_len, s_beg, t_end, t_step, grid_n;
+  int f_beg, f_len, s_beg, t_end, t_step, grid_n, grid_s;
+  bool narrow;
 
   static __device__ __forceinline__ int n_full(int rows) { return (rows + BM / 2 - 1) / BM; }
   static __device__ __forceinline__ int n_short(int rows) { return rows > n_full(rows) * BM ? 1 : 0; }
@@ -48,12 +53,19 @@ struct TileList {
       brief += __builtin_amdgcn_readlane(wave_scan_i32(n_short(sz[c])), 63);
     }
     grid_n = p.grid_n;
+    narrow = false;
+    grid_s = grid_n;
+    if constexpr (SBN < BN) {
+      const uint32_t wgs = gridDim.x, over = (uint32_t)(full * grid_n) % wgs, wide = (uint32_t)(brief * grid_n);
+      narrow = wide > (over ? wgs - over : 0) && wide * 2 <= wgs;
+      if (narrow) grid_s = (p.N + SBN - 1) / SBN;
+    }
     const int xcd = blockIdx.x & 7;
     t_step = gridDim.x >> 3;
     // An eighth of the full tiles, and of the short ones what makes an eighth of all: with each list divided on its own an XCD could be two
     // tiles over, which one workgroup then had in a round of its own (94 rows a slice, three rounds, K 2880, N 2880: 195 -> 169 us).
     // (From eight short tiles on their bounds only grow: an eighth of all is then at least the larger eighth of the full ones.)
-    const int64_t n_f = (int64_t)full * grid_n, n_s = (int64_t)brief * grid_n, n = n_f + n_s;
+    const int64_t n_f = (int64_t)full * grid_n, n_s = (int64_t)brief * grid_s, n = n_f + n_s;
     auto full_to = [&](int x) -> int { return (int)((n_f * x) >> 3); };
     auto short_to = [&](int x) -> int { return n_s < 8 ? (int)((n_s * x) >> 3) : (int)((n * x) >> 3) - full_to(x); };
     f_beg = full_to(xcd), f_len = full_to(xcd + 1) - f_beg;
@@ -63,10 +75,12 @@ struct TileList {
   }
 
   __device__ __forceinline__ Tile locate(int t) const {
-    Tile r = {0, 0, 0, 0, 0};
+    Tile r = {0, 0, 0, 0, 0, false};
     const bool is_full = t < f_len;
     const int g = is_full ? f_beg + t : s_beg + t - f_len;
+    const int grid_n = is_full ? this->grid_n : grid_s;
     const int q = g / grid_n;
+    r.narrow = narrow && !is_full;
     int base = 0;
     bool found = false;
 #pragma unroll
@@ -89,7 +103,7 @@ struct TileList {
         const int bh = nb - band * 8 < 8 ? nb - band * 8 : 8;
         i -= band * 8 * grid_n;
         const int pn = i / bh;
-        r.n_tile = pn * BN;
+        r.n_tile = pn * (r.narrow ? SBN : BN);
         r.off_m = (is_full ? band * 8 + i - pn * bh : n_full(r.eM)) * BM;
       }
       base += total;

@@ -17,6 +17,9 @@
 //     read and are filled again.
 //   * Workgroups are persistent and the ring runs on across tiles: the first stages of the next tile are on their way during the
 //     last stages and the epilogue of this one.
+//   * Short row blocks behind the last full round take half of the columns and twice the K a stage, so that all CUs have one and there are half
+//     as many stages, each as long as its way from memory (bf16, us: 8 slices of about 1024 rows, K 2048, N 2048 79 -> 70, K 4096, N 4096 262 -> 240,
+//     of about 512 rows 80 -> 73 and 156 -> 135; 16 of about 256, N 4096 85 to 95 -> 81).
 //
 // What bounds it: the board's power (a square bf16 product of 8192: matrix pipe 87 % busy at 1.58 GHz, 1390 TFLOP/s, 0.93 of what the
 // vendor's library reaches on the same board), with shorter K also the epilogues (e4m3, K 4096: 12 % of the time; matrix pipe 67 % busy at 1.8
@@ -38,11 +41,13 @@ struct DmaCfg {
   static constexpr int ABYTES = BM * 128, BBYTES = BN * 128;
   static constexpr int ABUFS = 2, BBUFS = 3;
   static constexpr int LDS = ABUFS * ABYTES + BBUFS * BBYTES;
+  static constexpr int SBN = BN / 2;  // columns of a narrow tile
   static constexpr int AI = BM / 8 / NW, BI = BN / 8 / NW;  // transfers of a wave and stage
 };
 static_assert(DmaCfg<true>::LDS == 160 * 1024 && DmaCfg<false>::LDS == 80 * 1024, "one / two workgroups fill a CU's LDS");
 
-template <int WK, bool LARGE, bool SWIGLU>
+// NARROW: short row blocks may be cut into narrow tiles (gemm_tiles.h).
+template <int WK, bool LARGE, bool SWIGLU, bool NARROW>
 __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel(const GemmParams p) {
   typedef DmaCfg<LARGE> C;
   constexpr bool F8 = WK == WK_FP8;
@@ -57,7 +62,7 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
   const int nst = (KB + 127) >> 7;
   const uint32_t lds0 = lds_addr(lds);
 
-  TileList<C::BM, C::BN> tiles;
+  TileList<C::BM, C::BN, NARROW ? C::SBN : C::BN> tiles;
   int tile = tiles.init(p, lane);
   const int t_step = tiles.t_step, t_end = tiles.t_end;
   if (tile >= t_end) return;
@@ -72,10 +77,19 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
   uint32_t a_off[C::AI], b_off[C::BI];
   const uint32_t x_row = (uint32_t)(p.x_stride_m * ES);
   static_assert(C::AI % 2 == 0 && C::BI % 2 == 0, "a transfer's parity is that of its index in the wave");
+  // A narrow tile's stage is twice as long: the first half of the waves fetches its first 128 bytes of K, for half of the rows and columns that the
+  // buffers have room for, the others the second.
+  int f_step = 128, f_kh = 0;  // bytes of K of a stage, and where this wave's transfers begin in it
   auto aim = [&](const Tile& c) __attribute__((always_inline)) {
+    const bool nar = NARROW && c.narrow;
+    if constexpr (NARROW) {
+      f_step = nar ? 256 : 128;
+      f_kh = nar ? wave / (C::NW / 2) * 128 : 0;
+    }
+    const int w_in = nar ? wave % (C::NW / 2) : wave;
 #pragma unroll
     for (int i = 0; i < C::AI; ++i) {
-      const int row = c.off_m + (wave * C::AI + i) * 8 + (lane >> 3);
+      const int row = c.off_m + (w_in * C::AI + i) * 8 + (lane >> 3);
       const int sr = c.start_m + (row < c.eM ? row : c.eM - 1);
       const uint32_t src = p.gather ? (uint32_t)p.gather[sr] : (uint32_t)sr;
       a_off[i] = row < c.eM ? src * x_row + (uint32_t)((i & 1) ? pc1 : pc0) * 16u : kOutOfRange;
@@ -87,29 +101,29 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
       wdesc = make_buf_desc(w + (int64_t)f0 * fsz, (uint32_t)(nfr - f0 < nf ? nfr - f0 : nf) * fsz);
 #pragma unroll
       for (int i = 0; i < C::BI; ++i) {
-        const int id = wave * C::BI + i;  // KiB id % 4 of fragment id / 4's block
+        const int id = w_in * C::BI + i;  // KiB id % 4 of fragment id / 4's block
         b_off[i] = (uint32_t)(id >> 2) * fsz + (uint32_t)(id & 3) * 1024u + (uint32_t)lane * 16u;
       }
     } else {
-      const int cols = p.N - c.n_tile < C::BN ? p.N - c.n_tile : C::BN;
+      const int bn = nar ? C::SBN : C::BN, cols = p.N - c.n_tile < bn ? p.N - c.n_tile : bn;
       wdesc = make_buf_desc(w + (int64_t)c.n_tile * p.w_stride_n, (uint32_t)(cols - 1) * (uint32_t)p.w_stride_n + (uint32_t)KB);
 #pragma unroll
       for (int i = 0; i < C::BI; ++i) {
-        const int n = (wave * C::BI + i) * 8 + (lane >> 3);
+        const int n = (w_in * C::BI + i) * 8 + (lane >> 3);
         b_off[i] = n < cols ? (uint32_t)n * (uint32_t)p.w_stride_n + (uint32_t)((i & 1) ? pc1 : pc0) * 16u : kOutOfRange;
       }
     }
   };
-  // transfer i of this wave for stage s of the tile aimed at (none left: zeros into a buffer that nobody reads)
-  auto fetch_a = [&](int i, int s, uint32_t buf, bool more) __attribute__((always_inline)) {
-    const uint32_t kb = (uint32_t)s * 128u;
-    const bool in = more && (int)kb + ((i & 1) ? pc1 : pc0) * 16 < KB;
-    lds_dma16(xdesc, lds0 + buf + (wave * C::AI + i) * 1024, in ? a_off[i] + kb : kOutOfRange);
+  // transfer i of this wave for the stage at byte kb of K of the tile aimed at (none left: zeros into a buffer that nobody reads)
+  auto fetch_a = [&](int i, int kb, uint32_t buf, bool more) __attribute__((always_inline)) {
+    kb += f_kh;
+    const bool in = more && kb + ((i & 1) ? pc1 : pc0) * 16 < KB;
+    lds_dma16(xdesc, lds0 + buf + (wave * C::AI + i) * 1024, in ? a_off[i] + (uint32_t)kb : kOutOfRange);
   };
-  auto fetch_b = [&](int i, int s, uint32_t buf, bool more) __attribute__((always_inline)) {
-    const uint32_t kb = (uint32_t)s * (F8 ? 4096u : 128u);
-    const bool in = more && (F8 || (int)kb + ((i & 1) ? pc1 : pc0) * 16 < KB);  // (tiled weights are padded with zeros)
-    lds_dma16(wdesc, lds0 + buf + (wave * C::BI + i) * 1024, in ? b_off[i] + kb : kOutOfRange);
+  auto fetch_b = [&](int i, int kb, uint32_t buf, bool more) __attribute__((always_inline)) {
+    kb += f_kh;
+    const bool in = more && kb + (F8 ? 0 : ((i & 1) ? pc1 : pc0) * 16) < KB;  // (blocks of tiled weights are padded with zeros)
+    lds_dma16(wdesc, lds0 + buf + (wave * C::BI + i) * 1024, in ? b_off[i] + (uint32_t)kb * (F8 ? 32u : 1u) : kOutOfRange);
   };
 
   // ---- LDS read side ----------------------------------------------------------------------------------------------------------------------------
@@ -131,13 +145,13 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
   Tile cur = tiles.locate(tile);
   aim(cur);
   uint32_t aw = 0, bw = kAEnd;  // buffers the next transfers fill
-  int fs = 0;                   // next stage to fetch
+  int fs = 0;                   // where the next stage to fetch begins
   bool more = true;
   int f_tile = tile;
   auto advance = [&]() __attribute__((always_inline)) {
     aw = aw + C::ABYTES == kAEnd ? 0 : aw + C::ABYTES;
     bw = bw + C::BBYTES == kBEnd ? kAEnd : bw + C::BBYTES;
-    if (++fs == nst) {
+    if ((fs += f_step) >= KB) {
       fs = 0;
       f_tile += t_step;
       more = more && f_tile < t_end;
@@ -243,7 +257,62 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
       for (int j = 0; j < MFW / 2; ++j) a8[0][j] = both(read_a(ab, j, 0), read_a(ab, j, 1));
     }
   };
+  // A narrow tile, BM / 2 rows by SBN columns, 32 columns a wave: what takes its time is not the multiplications but a stage's way from memory,
+  // and a stage is as many bytes as a full tile's.
+  auto narrow_tile = [&]() __attribute__((always_inline)) {
+    constexpr int MH = MFW / 2;
+    f32x16_t part[1][MH];
+#pragma unroll
+    for (int j = 0; j < MH; ++j)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) part[0][j][i] = 0.f;
+    const int jn = __builtin_amdgcn_readfirstlane((((cur.eM - cur.off_m + 31) >> 5) - mw + C::WM - 1) / C::WM);
+#pragma unroll 1
+    for (int s = 0; s < (nst + 1) >> 1; ++s) {
+#pragma unroll
+      for (int i = 0; i < C::BI; ++i) fetch_b(i, fs, bw, more);
+      if (jn > 0) {
+#pragma unroll
+        for (int kh = 0; kh < 2; ++kh) {
+          const uint32_t a0 = ab + kh * (C::ABYTES / 2) + (uint32_t)(mw * 4096), b0 = bb + kh * (C::BBYTES / 2) + (uint32_t)(nw * 4096);
+          u32x4_t w[4];
+#pragma unroll
+          for (int t = 0; t < 4; ++t) w[t] = F8 ? ld(b0 + (uint32_t)lane * 16u + t * 1024) : ld(b0 + pos[t]);
+#pragma unroll
+          for (int j = 0; j < MH; ++j) {
+            if (j >= jn) break;
+            u32x4_t x[4];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) x[t] = ld(a0 + pos[t] + j * (C::WM * 4096));
+            if constexpr (F8) {
+#pragma unroll
+              for (int u = 0; u < 2; ++u)
+                part[0][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(both(w[2 * u], w[2 * u + 1]), both(x[2 * u], x[2 * u + 1]), part[0][j], 0, 0, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
+            } else {
+#pragma unroll
+              for (int t = 0; t < 4; ++t) part[0][j] = mma16(w[t], x[t], part[0][j]);
+            }
+          }
+        }
+      }
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::BI) : "memory");
+      barrier();
+#pragma unroll
+      for (int i = 0; i < C::AI; ++i) fetch_a(i, fs, aw, more);
+      ab = ab + C::ABYTES == kAEnd ? 0 : ab + C::ABYTES;
+      bb = bb + C::BBYTES == kBEnd ? kAEnd : bb + C::BBYTES;
+      advance();
+    }
+    gemm_epilogue<32, C::WM, MH, 1, SWIGLU, WK == WK_F16>(p, part, cur.expert, cur.off_m, cur.start_m, cur.eM, cur.n_tile + nw * 32, cur.n_tile + C::SBN <= p.N, mw, lr, h);
+  };
   while (true) {
+    if (NARROW && cur.narrow) {
+      narrow_tile();
+      tile += t_step;
+      if (tile >= t_end) break;
+      cur = tiles.locate(tile);
+      continue;
+    }
     prime();
 #pragma unroll
     for (int f = 0; f < NFW; ++f)
@@ -300,7 +369,12 @@ int32_t launch_cfg(const GemmParams& p, int grid_m, bool swiglu, hipStream_t st)
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NW * 64), C::LDS, st, q);
     return check_launch("moe_gemm_dma_kernel");
   };
-  return swiglu ? launch(moe_gemm_dma_kernel<WK, LARGE, true>) : launch(moe_gemm_dma_kernel<WK, LARGE, false>);
+  if constexpr (LARGE) {
+    // (the other kernel, half a microsecond faster to start, where all tiles are one round, and its stages are half a percent shorter where they
+    // are many: e4m3, K 4096, 31 rounds)
+    if (tiles > grid && tiles <= 8 * grid) return swiglu ? launch(moe_gemm_dma_kernel<WK, LARGE, true, true>) : launch(moe_gemm_dma_kernel<WK, LARGE, false, true>);
+  }
+  return swiglu ? launch(moe_gemm_dma_kernel<WK, LARGE, true, false>) : launch(moe_gemm_dma_kernel<WK, LARGE, false, false>);
 }
 
 }  // namespace
