@@ -25,8 +25,8 @@ struct Tile {
 template <int BM, int BN, int SBN = BN>
 struct TileList {
   int sz[kSliceRegs], so[kSliceRegs];
-  int f_beg, f_len, s_beg, t_end, t_step, grid_n, grid_s;
-  bool narrow;
+  int f_beg, f_len, s_beg, t_end, t_step, grid_n;
+  int grid_s = 0;  // SBN < BN: tiles of a short row block if those are narrow, else 0
 
   static __device__ __forceinline__ int n_full(int rows) { return (rows + BM / 2 - 1) / BM; }
   static __device__ __forceinline__ int n_short(int rows) { return rows > n_full(rows) * BM ? 1 : 0; }
@@ -53,19 +53,16 @@ struct TileList {
       brief += __builtin_amdgcn_readlane(wave_scan_i32(n_short(sz[c])), 63);
     }
     grid_n = p.grid_n;
-    narrow = false;
-    grid_s = grid_n;
     if constexpr (SBN < BN) {
       const uint32_t wgs = gridDim.x, over = (uint32_t)(full * grid_n) % wgs, wide = (uint32_t)(brief * grid_n);
-      narrow = wide > (over ? wgs - over : 0) && wide * 2 <= wgs;
-      if (narrow) grid_s = (p.N + SBN - 1) / SBN;
+      if (wide > (over ? wgs - over : 0) && wide * 2 <= wgs) grid_s = (p.N + SBN - 1) / SBN;
     }
     const int xcd = blockIdx.x & 7;
     t_step = gridDim.x >> 3;
     // An eighth of the full tiles, and of the short ones what makes an eighth of all: with each list divided on its own an XCD could be two
     // tiles over, which one workgroup then had in a round of its own (94 rows a slice, three rounds, K 2880, N 2880: 195 -> 169 us).
     // (From eight short tiles on their bounds only grow: an eighth of all is then at least the larger eighth of the full ones.)
-    const int64_t n_f = (int64_t)full * grid_n, n_s = (int64_t)brief * grid_s, n = n_f + n_s;
+    const int64_t n_f = (int64_t)full * grid_n, n_s = (int64_t)brief * (grid_s ? grid_s : grid_n), n = n_f + n_s;
     auto full_to = [&](int x) -> int { return (int)((n_f * x) >> 3); };
     auto short_to = [&](int x) -> int { return n_s < 8 ? (int)((n_s * x) >> 3) : (int)((n * x) >> 3) - full_to(x); };
     f_beg = full_to(xcd), f_len = full_to(xcd + 1) - f_beg;
@@ -78,9 +75,9 @@ struct TileList {
     Tile r = {0, 0, 0, 0, 0, false};
     const bool is_full = t < f_len;
     const int g = is_full ? f_beg + t : s_beg + t - f_len;
-    const int grid_n = is_full ? this->grid_n : grid_s;
+    r.narrow = SBN < BN && !is_full && grid_s;
+    const int grid_n = r.narrow ? grid_s : this->grid_n;
     const int q = g / grid_n;
-    r.narrow = narrow && !is_full;
     int base = 0;
     bool found = false;
 #pragma unroll
