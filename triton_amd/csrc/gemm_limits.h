@@ -31,6 +31,17 @@ inline bool dma_runs_e4m3(uint32_t x_bytes, int64_t n_slices, int64_t K, int64_t
   return dma_runs(x_bytes, n_slices, (N + 31) / 32 * ((K + 255) / 256) * 8192);
 }
 
+// Whether the weights (`row_bytes` a column) are fetched with the non-temporal hint: few slices have a second row block, and they are more than
+// half of the 256 MiB of the cache in front of memory, so that next to nothing of them is there when the call is made again.  Measured (us of a
+// layer, with against without it; other weights each call).  e4m3, 8 experts, d 4096, d_ff 14336: 8 rows each 238 against 267, 62 rows 295 / 313; d 2048, d_ff
+// 4096, 16 rows (201 MB in all) 70 / 74, but with the same weights again 66 / 64.  bf16, d and d_ff 2048: 16 experts, 25 rows 112 / 120, 32 experts, 31
+// rows 203 / 217; tiles of 256 rows: 32 experts, 200 rows 254 / 271; where row blocks share their weights it costs: 16 experts, 256 rows 193 / 187;
+// tiles of 128 rows, 125 rows 149 / 146.  MXFP4, 128 experts, d and d_ff 2880, 128 rows 806 / 824, MXFP8 572 / 580, 94 rows 497 / 520.
+inline bool reads_once(int64_t rows, int64_t n_slices, int64_t block_rows, int64_t N, int64_t row_bytes) {
+  const int64_t read = n_slices < rows ? n_slices : rows;
+  return rows * 16 <= n_slices * block_rows * 13 && read * N * row_bytes > 128 << 20;
+}
+
 // Row blocks (of 64) that the kernel for few rows launches side by side: one a slice at least, and what slices of up to five quarters of
 // the mean make, as a random routing does (at 62 rows per slice half of the slices have a second block).
 inline int64_t few_row_blocks(int64_t rows, int64_t n_slices) { return n_slices * (rows * 5 / (n_slices * 256) + 1); }

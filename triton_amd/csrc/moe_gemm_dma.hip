@@ -23,7 +23,8 @@
 //
 // What bounds it: the board's power (a square bf16 product of 8192: matrix pipe 87 % busy at 1.58 GHz, 1390 TFLOP/s, 0.93 of what the
 // vendor's library reaches on the same board), with shorter K also the epilogues (e4m3, K 4096: 12 % of the time; matrix pipe 67 % busy at 1.8
-// GHz, K 14336: 77 % at 1.75), with a few rows per expert (128 x 128 tiles) the weight stream at 5.3 to 5.6 TB/s.  16384 routed rows
+// GHz, K 14336: 77 % at 1.75), with a few rows per expert (128 x 128 tiles) the weight stream at 5.9 TB/s (5.3 without the
+// non-temporal hint).  16384 routed rows
 // of 8 experts in e4m3: K 4096, N 28672, swiglu 1840 -> 1590 us (2.42 PFLOP/s), K 14336, N 4096 850 -> 805 us; 4096 rows of 16
 // experts in bf16, K 2048: N 4096 231 -> 94 us, N 2048 133 -> 51 us (the kernels before: weights in registers with one wave
 // per SIMD, and both operands through registers into LDS).
@@ -46,8 +47,8 @@ struct DmaCfg {
 };
 static_assert(DmaCfg<true>::LDS == 160 * 1024 && DmaCfg<false>::LDS == 80 * 1024, "one / two workgroups fill a CU's LDS");
 
-// NARROW: short row blocks may be cut into narrow tiles (gemm_tiles.h).
-template <int WK, bool LARGE, bool SWIGLU, bool NARROW>
+// NARROW: short row blocks may be cut into narrow tiles (gemm_tiles.h).  ONCE: the weights are fetched with the non-temporal hint (reads_once).
+template <int WK, bool LARGE, bool SWIGLU, bool NARROW, bool ONCE>
 __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel(const GemmParams p) {
   typedef DmaCfg<LARGE> C;
   constexpr bool F8 = WK == WK_FP8;
@@ -123,7 +124,7 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
   auto fetch_b = [&](int i, int kb, uint32_t buf, bool more) __attribute__((always_inline)) {
     kb += f_kh;
     const bool in = more && kb + (F8 ? 0 : ((i & 1) ? pc1 : pc0) * 16) < KB;  // (blocks of tiled weights are padded with zeros)
-    lds_dma16(wdesc, lds0 + buf + (wave * C::BI + i) * 1024, in ? b_off[i] + (uint32_t)kb * (F8 ? 32u : 1u) : kOutOfRange);
+    lds_dma16<ONCE>(wdesc, lds0 + buf + (wave * C::BI + i) * 1024, in ? b_off[i] + (uint32_t)kb * (F8 ? 32u : 1u) : kOutOfRange);
   };
 
   // ---- LDS read side ----------------------------------------------------------------------------------------------------------------------------
@@ -369,12 +370,15 @@ int32_t launch_cfg(const GemmParams& p, int grid_m, bool swiglu, hipStream_t st)
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NW * 64), C::LDS, st, q);
     return check_launch("moe_gemm_dma_kernel");
   };
+  if (reads_once(p.M, p.slice_sizes ? p.n_slices : 1, C::BM, p.N, p.K * (WK == WK_FP8 ? 1 : 2)))
+    return swiglu ? launch(moe_gemm_dma_kernel<WK, LARGE, true, false, true>) : launch(moe_gemm_dma_kernel<WK, LARGE, false, false, true>);
   if constexpr (LARGE) {
     // (the other kernel, half a microsecond faster to start, where all tiles are one round, and its stages are half a percent shorter where they
     // are many: e4m3, K 4096, 31 rounds)
-    if (tiles > grid && tiles <= 8 * grid) return swiglu ? launch(moe_gemm_dma_kernel<WK, LARGE, true, true>) : launch(moe_gemm_dma_kernel<WK, LARGE, false, true>);
+    if (tiles > grid && tiles <= 8 * grid)
+      return swiglu ? launch(moe_gemm_dma_kernel<WK, LARGE, true, true, false>) : launch(moe_gemm_dma_kernel<WK, LARGE, false, true, false>);
   }
-  return swiglu ? launch(moe_gemm_dma_kernel<WK, LARGE, true, false>) : launch(moe_gemm_dma_kernel<WK, LARGE, false, false>);
+  return swiglu ? launch(moe_gemm_dma_kernel<WK, LARGE, true, false, false>) : launch(moe_gemm_dma_kernel<WK, LARGE, false, false, false>);
 }
 
 }  // namespace

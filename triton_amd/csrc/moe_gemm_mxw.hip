@@ -16,7 +16,7 @@
 // What bounds it: the board's power in bf16 (fetching zeros instead of the weights, the operands then all zero, 558 -> 417 us; matrix pipe 68 %
 // busy at 1.9 GHz), in MXFP8 also LDS reads and the epilogue (without its arithmetic and stores 363 -> 316 us; 42 % busy at 2.3 GHz,
 // ten vector instructions per MFMA with the quantised output, seven with bf16).  128 experts, K 2880, 4096 tokens, top-4, whole layer:
-// bf16 861 -> 830 us, MXFP8 609 -> 586 us against the kernels that keep weights in registers with one wave per SIMD (moe_gemm_mxn, _mx8n, which
+// bf16 861 -> 815 us, MXFP8 609 -> 563 us against the kernels that keep weights in registers with one wave per SIMD (moe_gemm_mxn, _mx8n, which
 // serve what this one does not take).  Measured and left out: transfers spread over the whole bf16 stage (576 against 558
 // us: the last ones are late); weights brought into L2 a stage ahead of their transfer (570 against 558, MXFP8 387 against 363 us).
 #include "gemm_tiles.h"
@@ -43,7 +43,8 @@ struct MxwCfg {
   static constexpr int LDS = RINGS + 2 * (SIDE + OPERANDS) + LISTS;
 };
 
-template <bool MX8, bool SWIGLU, bool MXOUT>
+// ONCE: the weights are fetched with the non-temporal hint (reads_once)
+template <bool MX8, bool SWIGLU, bool MXOUT, bool ONCE>
 __global__ __launch_bounds__(MxwCfg<MX8>::NW * 64, 2) void moe_gemm_mxw_kernel(const GemmParams p) {
   typedef MxwCfg<MX8> C;
   constexpr int MFW = C::MFW, AI = C::AI;
@@ -159,9 +160,9 @@ __global__ __launch_bounds__(MxwCfg<MX8>::NW * 64, 2) void moe_gemm_mxw_kernel(c
     const uint32_t dst = lds0 + buf + wave * C::WWAVE;
     if (i < 4) {
       const int f = i >> 1, q = i & 1;
-      lds_dma16(wdesc, dst + f * 2048 + q * 1024, (on ? (uint32_t)f * f_val + (uint32_t)s * 2048u + q * 1024u : kOutOfRange) + w_off);
+      lds_dma16<ONCE>(wdesc, dst + f * 2048 + q * 1024, (on ? (uint32_t)f * f_val + (uint32_t)s * 2048u + q * 1024u : kOutOfRange) + w_off);
     } else {
-      lds_dma4(sdesc, dst + 4096, (on ? (uint32_t)s * 128u : kOutOfRange) + s_off);
+      lds_dma4<ONCE>(sdesc, dst + 4096, (on ? (uint32_t)s * 128u : kOutOfRange) + s_off);
     }
   };
   // activation scales: sixteen blocks (four stages) of row `tid` at a time, the last group of a row moved back to stay inside it
@@ -388,10 +389,14 @@ int32_t launch_cfg(const GemmParams& p, bool swiglu, bool mx_out, hipStream_t st
     hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(C::NW * 64), C::LDS, st, q);
     return check_launch("moe_gemm_mxw_kernel");
   };
-  if constexpr (MX8) {
-    if (mx_out) return swiglu ? launch(moe_gemm_mxw_kernel<true, true, true>) : launch(moe_gemm_mxw_kernel<true, false, true>);
-  }
-  return swiglu ? launch(moe_gemm_mxw_kernel<MX8, true, false>) : launch(moe_gemm_mxw_kernel<MX8, false, false>);
+  auto with = [&](auto once) -> int32_t {
+    constexpr bool ONCE = decltype(once)::value;
+    if constexpr (MX8) {
+      if (mx_out) return swiglu ? launch(moe_gemm_mxw_kernel<true, true, true, ONCE>) : launch(moe_gemm_mxw_kernel<true, false, true, ONCE>);
+    }
+    return swiglu ? launch(moe_gemm_mxw_kernel<MX8, true, false, ONCE>) : launch(moe_gemm_mxw_kernel<MX8, false, false, ONCE>);
+  };
+  return reads_once(p.M, p.slice_sizes ? p.n_slices : 1, C::BM, p.N, p.K / 2) ? with(std::true_type{}) : with(std::false_type{});
 }
 
 }  // namespace
