@@ -123,7 +123,7 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
   };
   auto fetch_b = [&](int i, int kb, uint32_t buf, bool more) __attribute__((always_inline)) {
     kb += f_kh;
-    const bool in = more && kb + (F8 ? 0 : ((i & 1) ? pc1 : pc0) * 16) < KB;  // (blocks of tiled weights are padded with zeros)
+    const bool in = more && (F8 ? !NARROW || kb < KB : kb + ((i & 1) ? pc1 : pc0) * 16 < KB);  // (blocks of tiled weights are padded with zeros)
     lds_dma16<ONCE>(wdesc, lds0 + buf + (wave * C::BI + i) * 1024, in ? b_off[i] + (uint32_t)kb * (F8 ? 32u : 1u) : kOutOfRange);
   };
 
