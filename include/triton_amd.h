@@ -106,7 +106,7 @@ int32_t tk_mx_upcast(const void* vals, const void* scales, int32_t kind, int64_t
  * ---------------------------------------------------------------------------------------------- */
 
 /*
- * One routing pass.  Replaces, in three launches, the reference's
+ * One routing pass.  Replaces, in one to three launches, the reference's
  *   `_topk_forward[(pids,)](...)`                          tk/topk.py:59-67
  *   `_sum_bitmatrix_rows[(grid_m, grid_n)](...)`           tk/tensor_details/bitmatrix_details/sum_bitmatrix_rows.py:89-97
  *   `_bitmatrix_metadata_compute_stage1/2[...]`            tk/tensor_details/bitmatrix.py:128-145
@@ -418,6 +418,8 @@ int32_t tk_ragged_k_gemm(const tk_ragged_k_desc* desc, tk_stream_t stream);
  * Limits: n_tokens * k <= TK_DECODE_MAX_ROWS, n_experts <= TK_DECODE_MAX_EXPERTS, d_model and d_ff <= 3072 and
  * multiples of 8; otherwise TK_ERR_UNSUPPORTED (callers then take tk_route + tk_moe_gemm).
  *
+ * With spin_limit 0, k <= 8, up to 64 rows and at most 135 MB of weights counted once per row, the layer runs row by row in two launches that
+ * wait for nothing (callers need not serialise those; nothing of the workspace's synchronisation words is touched).  Otherwise it is one launch:
  * The kernel is persistent: its workgroups must all be resident together (the grid is sized from the occupancy the
  * runtime reports) because workgroups of the second GEMM wait for the first GEMM's rows of other workgroups.  Two
  * launches of it that overlap in time on one device (different streams) could each hold part of the GPU and wait
