@@ -1,0 +1,65 @@
+"""The memory that decode layers are launched with, on the CPU (the descriptors are looked at, nothing is launched): the two launches of a layer that
+goes row by row get memory of the call's own, so that a captured graph's belongs to the graph."""
+import pytest
+import torch
+
+from triton_amd import _native as nt
+from triton_amd import moe_decode
+
+
+class _Library:
+    def __init__(self, real):
+        self.real, self.given = real, []
+
+    def __getattr__(self, name):
+        return getattr(self.real, name)
+
+    def tk_moe_decode_layer(self, d, stream):
+        self.given.append(d.workspace)
+        return 0
+
+
+class _Weights:  # a tiled tensor, its storage and its scales, as far as the call looks at them
+    def __init__(self, e, k, n):
+        self.shape = (e, k, n)
+        self.storage = self
+        self.data = self.b_mx_scale = torch.zeros((e, 16), dtype=torch.uint8)
+
+
+@pytest.fixture
+def layer(monkeypatch):
+    """layer(T, k, dims): a decode layer on CPU tensors with a library that only notes the workspace; layer.given: those."""
+    lib = _Library(nt.lib())
+    nt.rules()
+    monkeypatch.setattr(nt, "lib", lambda: lib)
+    monkeypatch.setattr(nt, "stream_ptr", lambda device=None: 0)
+    monkeypatch.setattr(moe_decode, "one_launch_reason", lambda *a: None)
+    monkeypatch.setattr(moe_decode, "_swiglu_args", lambda act: (1.702, 7.0, 1))
+    monkeypatch.setattr(moe_decode, "_WORKSPACES", {})
+
+    class PC:
+        def __init__(self, w):
+            self.b_mx_scale = w
+
+    def call(T, k, dims=2880, E=128):
+        w1, w2 = _Weights(E, dims, 2 * dims), _Weights(E, dims, dims)
+        return moe_decode.moe_decode_layer(torch.zeros((T, dims), dtype=torch.bfloat16), torch.zeros((T, E)), k, w1, None, w2, None, PC(w1), PC(w2), None)
+
+    call.given = lib.given
+    return call
+
+
+@pytest.mark.parametrize("T, k, dims", [(1, 1, 2880), (1, 4, 2880), (8, 1, 2880), (64, 1, 512)])
+def test_row_by_row_memory_is_the_calls_own(layer, T, k, dims):
+    assert nt.rules().decode_by_rows(T, k, dims, dims)
+    layer(T, k, dims)
+    assert len(layer.given) == 1 and layer.given[0] and moe_decode._WORKSPACES == {}
+
+
+@pytest.mark.parametrize("T, k, dims", [(16, 4, 2880), (65, 1, 512), (4, 16, 512)])
+def test_the_single_launch_keeps_its_counters(layer, T, k, dims):
+    assert not nt.rules().decode_by_rows(T, k, dims, dims)
+    layer(T, k, dims)
+    layer(T, k, dims)
+    (ws, ) = moe_decode._WORKSPACES.values()
+    assert layer.given == [ws.data_ptr()] * 2

@@ -80,3 +80,74 @@ def test_a_k_that_routing_refuses_stays_refused(device):
     x, logits = torch.zeros((2, 128), dtype=torch.bfloat16, device=device), torch.zeros((2, 8), device=device)
     with pytest.raises(ValueError):
         moe_mlp(x, logits, 3, W["w1"], W["b1"], W["w2"], W["b2"], PrecisionConfig(b_mx_scale=W["w1s"]), PrecisionConfig(b_mx_scale=W["w2s"]), act)
+
+
+@pytest.fixture(scope="module")
+def small_layer(device):
+    """call(x, logits): a layer of 8 experts through `moe_mlp`, top 4, row by row at the sizes below."""
+    from bench import make_moe_weights, to_matmul_layout
+    from triton_kernels import moe_decode
+    from triton_kernels.matmul import FnSpecs, FusedActivation, PrecisionConfig
+    from triton_kernels.swiglu import swiglu_fn
+    W = to_matmul_layout(make_moe_weights(8, 256, 512, seed=4, device=device)[0])
+    act = FusedActivation(FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0))
+    pc1, pc2 = PrecisionConfig(b_mx_scale=W["w1s"]), PrecisionConfig(b_mx_scale=W["w2s"])
+    return lambda x, logits: moe_decode.moe_mlp(x, logits, 4, W["w1"], W["b1"], W["w2"], W["b2"], pc1, pc2, act)
+
+
+def _inputs(T, device, g):
+    return torch.randn((T, 256), generator=g).to(torch.bfloat16).to(device), torch.randn((T, 8), generator=g).to(device)
+
+
+@pytest.mark.parametrize("T", [1, 3])
+def test_a_graph_owns_its_memory(device, small_layer, T):
+    """Warmed up and captured on one stream, replayed with new inputs after the workspaces of more shapes than are kept, with other tensors in
+    whatever memory they have left: bit for bit the eager layer's result."""
+    from triton_kernels import moe_decode
+    g = torch.Generator().manual_seed(T)
+    x, logits = _inputs(T, device, g)
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.stream(side):
+        small_layer(x, logits)
+        with torch.cuda.graph(graph, stream=side):
+            got = small_layer(x, logits)
+        for t in range(1, 71):
+            moe_decode._workspace(device, t, 2, 8, 256, 256)
+    torch.cuda.synchronize()
+    for rep in range(3):
+        a, b = _inputs(T, device, g)
+        x.copy_(a), logits.copy_(b)
+        others = [torch.full((n, ), 0x7F, dtype=torch.uint8, device=device) for n in (512, 4096, 65536, 1 << 20)]
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(bool((o == 0x7F).all()) for o in others)
+        assert torch.equal(got, small_layer(x, logits)), f"replay {rep}"
+
+
+def test_graphs_of_one_stream_replayed_side_by_side(device, small_layer):
+    """Two graphs captured on one stream at one shape share no memory: replayed on two streams at a time each gives its own result."""
+    g = torch.Generator().manual_seed(9)
+    side, ins, graphs, outs = torch.cuda.Stream(), [], [], []
+    for _ in range(2):
+        x, logits = _inputs(4, device, g)
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            small_layer(x, logits)
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                out = [small_layer(x, logits) for _ in range(4)]
+        torch.cuda.synchronize()
+        ins.append((x, logits)), graphs.append(graph), outs.append(out)
+    want = [small_layer(*i) for i in ins]
+    assert not torch.equal(*want)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    torch.cuda.synchronize()
+    for rep in range(20):
+        for s, graph in zip(streams, graphs):
+            with torch.cuda.stream(s):
+                graph.replay()
+        torch.cuda.synchronize()
+        for w, out in zip(want, outs):
+            assert all(torch.equal(w, o) for o in out), f"replay {rep}"

@@ -152,7 +152,7 @@ def lib():
 
 _host = None
 _HOST_ENTRIES = ("tk_moe_gemm", "tk_route", "tk_route_workspace_bytes", "tk_reduce_mid", "tk_quant_fp8_rows", "tk_mx_downcast",
-                 "tk_mx_upcast", "tk_ragged_k_gemm", "tk_moe_decode_layer")
+                 "tk_mx_upcast", "tk_ragged_k_gemm", "tk_moe_decode_layer", "tk_moe_decode_layer_workspace_bytes")
 
 
 def _load_host():

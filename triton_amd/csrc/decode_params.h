@@ -1,6 +1,7 @@
 // What the kernels of the decode layer are given (moe_decode_layer.hip and, for small streams of weights, moe_decode_rows.hip).
 #pragma once
 #include "common.h"
+#include "gemm_limits.h"
 
 namespace tk {
 
@@ -38,8 +39,7 @@ struct DecodeParams {
   int32_t spin_limit;
 };
 
-// The layer row by row in two launches (up to kDecRowsMaxK experts a token); the workspace's y serves as the table between them.
-constexpr int kDecRowsMaxK = 8;
+// The layer row by row in two launches (decode_by_rows); the workspace's y serves as the table between them.
 int32_t decode_launch_rows(const DecodeParams& p, hipStream_t st);
 
 }  // namespace tk

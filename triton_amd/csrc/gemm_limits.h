@@ -1,6 +1,7 @@
 // What a call has to be like for the expert-GEMM kernels that address x through one buffer resource.  Plain C++: the entry point
 // (moe_gemm.hip) picks the kernel by it and the host path (host_path.cpp, for both of its callers) the row blocks, so that row
-// blocks which only such a kernel has are never chosen for a call that it cannot run.
+// blocks which only such a kernel has are never chosen for a call that it cannot run.  And how a decode layer is launched: its entry
+// point (moe_decode_layer.hip) and those who make its workspace go by the same rule.
 #pragma once
 #include <stdint.h>
 
@@ -45,5 +46,20 @@ inline bool reads_once(int64_t rows, int64_t n_slices, int64_t block_rows, int64
 // Row blocks (of 64) that the kernel for few rows launches side by side: one a slice at least, and what slices of up to five quarters of
 // the mean make, as a random routing does (at 62 rows per slice half of the slices have a second block).
 inline int64_t few_row_blocks(int64_t rows, int64_t n_slices) { return n_slices * (rows * 5 / (n_slices * 256) + 1); }
+
+// The decode layer row by row in two launches (moe_decode_rows.hip; up to kDecRowsMaxK experts a token), which keep nothing between calls: where the
+// rows' weights, counted for every row, are a small stream.  The single launch costs some 20 us around its stream, the two launches 7, but they read
+// an expert's weights again for each of its rows.  Measured (us, row by row against single launch; 2880 x 5760 and 2880 x 2880 but where noted): 8
+// rows, 106 MB, 29.8 against 37.1; 10 rows of 8 experts, 132 MB, 31.5 against 37.0; 12 rows of 10 experts, 159 MB, 39.9 against 40.0; 16 rows of 12,
+// 211 MB, 46.8 against 44.8.  Smaller layers: d and d_ff 512, 64 rows of 13 experts, 27 MB, 15.7 against 28.1; 1024, 64 rows, 107 MB, 30.3 against
+// 39.0; 1024 and 2048, 32 rows of 4 experts, 107 MB, 26.8 against 30.6; 512, 256 rows of 21 experts, 107 MB, 52.5 against 32.1.  (A caller that
+// names a spin limit asks for the launch whose waits it bounds.)
+constexpr int kDecRowsMaxK = 8;
+inline bool decode_by_rows(int64_t T, int64_t k, int64_t d_ff, int64_t d_model) {
+  constexpr int64_t kRowsMax = 64, kRowsBytes = 135'000'000;
+  auto parts = [](int64_t n, int64_t of) { return (n + of - 1) / of; };
+  const int64_t expert_bytes = (parts(2 * d_ff, 32) * parts(d_model, 128) + parts(d_model, 32) * parts(d_ff, 128)) * (2048 + 128);
+  return k <= kDecRowsMaxK && T * k <= kRowsMax && T * k * expert_bytes <= kRowsBytes;
+}
 
 }  // namespace tk

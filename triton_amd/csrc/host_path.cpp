@@ -45,6 +45,7 @@ struct Bound {
   decltype(&tk_mx_upcast) mx_upcast = nullptr;
   decltype(&tk_ragged_k_gemm) ragged_k_gemm = nullptr;
   decltype(&tk_moe_decode_layer) decode_layer = nullptr;
+  decltype(&tk_moe_decode_layer_workspace_bytes) decode_workspace_bytes = nullptr;
   PyObject *check, *raw_stream, *current_device;              // _native.check, torch's raw stream and device getters
   PyObject *tile_counters, *combine_counters, *decode_workspace;  // per device and stream
   PyObject *tensor_type, *mx_value, *mx_scale, *fp8_value, *fp4;  // Tensor, its layouts, the FP4 data type
@@ -743,11 +744,17 @@ PyObject* run_decode_layer(PyObject* const* v) {
     return none();
   auto stream = stream_of(*x);
   if (!stream) return none();
-  Ref dev(attr(v[0], N_.device)), t_o(PyLong_FromLongLong(T)), e_o(PyLong_FromLongLong(E)), f_o(PyLong_FromLongLong(ff)),
-      d_o(PyLong_FromLongLong(dm));
-  PyObject* args[6] = {dev, t_o, v[2], e_o, f_o, d_o};
-  Ref ws(PyObject_Vectorcall(B.decode_workspace, args, 6, nullptr));
-  if (!ws) throw PyError();
+  Tensor ws;  // (row by row: this call's own; a graph's belongs to the graph)
+  if (tk::decode_by_rows(T, k, ff, dm)) {
+    ws = empty({B.decode_workspace_bytes(int32_t(T), int32_t(k), int32_t(E), int32_t(ff), int32_t(dm))}, ScalarType::Byte, *x);
+  } else {
+    Ref dev(attr(v[0], N_.device)), t_o(PyLong_FromLongLong(T)), e_o(PyLong_FromLongLong(E)), f_o(PyLong_FromLongLong(ff)),
+        d_o(PyLong_FromLongLong(dm));
+    PyObject* args[6] = {dev, t_o, v[2], e_o, f_o, d_o};
+    Ref kept(PyObject_Vectorcall(B.decode_workspace, args, 6, nullptr));
+    if (!kept) throw PyError();
+    ws = THPVariable_Unpack(kept.p);
+  }
   Tensor out = empty({T, dm}, ScalarType::BFloat16, *x);
   tk_decode_layer_desc d{};
   d.x = x->data_ptr(), d.x_stride_m = x->stride(0);
@@ -761,7 +768,7 @@ PyObject* run_decode_layer(PyObject* const* v) {
   if (w2.bias) d.b2 = w2.bias->data_ptr(), d.b2_dtype = dtype_code(w2.bias->scalar_type()), d.b2_stride_e = w2.bias->stride(0);
   d.act_alpha = float(act.alpha), d.act_limit = float(act.limit), d.act_has_limit = act.has_limit;
   d.out = out.data_ptr(), d.out_stride_m = dm;
-  d.workspace = THPVariable_Unpack(ws.p).data_ptr();
+  d.workspace = ws.data_ptr();
   launch([&] { return B.decode_layer(&d, *stream); });
   return THPVariable_Wrap(std::move(out));
 }
@@ -813,6 +820,10 @@ PyObject* rule_dma_e4m3(PyObject* const* v) {
   const auto [x_bytes, n_slices, K, N] = integers<4>(v);
   return PyBool_FromLong(tk::dma_runs_e4m3(uint32_t(x_bytes), n_slices, K, N));
 }
+PyObject* rule_decode_rows(PyObject* const* v) {
+  const auto [T, k, d_ff, d_model] = integers<4>(v);
+  return PyBool_FromLong(tk::decode_by_rows(T, k, d_ff, d_model));
+}
 PyObject* rule_fp8(PyObject* const* v) {
   const auto [rows, x_bytes, K, N, n_slices] = integers<5>(v);
   return PyLong_FromLongLong(fp8_block_m(rows, uint32_t(x_bytes), K, N, n_slices));
@@ -849,6 +860,7 @@ PyObject* bind(PyObject*, PyObject* dict) {
   ENTRY(mx_upcast, tk_mx_upcast)
   ENTRY(ragged_k_gemm, tk_ragged_k_gemm)
   ENTRY(decode_layer, tk_moe_decode_layer)
+  ENTRY(decode_workspace_bytes, tk_moe_decode_layer_workspace_bytes)
 #undef ENTRY
 #define OBJECT(name)                            \
   if (!(B.name = get(#name))) return nullptr;   \
@@ -878,6 +890,7 @@ PyMethodDef methods[] = {
     METHOD("dma_runs_e4m3", rule_dma_e4m3, 4),
     METHOD("dma_block_n", rule_dma_n, 4),
     METHOD("few_block_n", rule_few, 3),
+    METHOD("decode_by_rows", rule_decode_rows, 4),
     METHOD("fp8_block_m", rule_fp8, 5),
     METHOD("mxfp4_block_m", rule_mxfp4, 3),
     METHOD("wide_block_m", rule_wide, 5),

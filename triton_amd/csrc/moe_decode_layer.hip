@@ -798,16 +798,7 @@ extern "C" int32_t tk_moe_decode_layer(const tk_decode_layer_desc* d, tk_stream_
   p.indx_out = static_cast<int16_t*>(d->indx_out);
   p.vals_out = d->vals_out;
   p.spin_limit = d->spin_limit > 0 ? d->spin_limit : (1 << 22);
-  // Row by row in two launches (moe_decode_rows.hip), where the rows' weights, counted for every row, are a small stream: the single
-  // launch costs some 20 us around its stream, the two launches 7, but they read an expert's weights again for each of its rows.  Measured
-  // (us, row by row against single launch; 2880 x 5760 and 2880 x 2880 but where noted): 8 rows, 106 MB, 29.8 against 37.1; 10 rows of 8
-  // experts, 132 MB, 31.5 against 37.0; 12 rows of 10 experts, 159 MB, 39.9 against 40.0; 16 rows of 12, 211 MB, 46.8 against 44.8.  Smaller
-  // layers: d and d_ff 512, 64 rows of 13 experts, 27 MB, 15.7 against 28.1; 1024, 64 rows, 107 MB, 30.3 against 39.0; 1024 and 2048, 32 rows
-  // of 4 experts, 107 MB, 26.8 against 30.6; 512, 256 rows of 21 experts, 107 MB, 52.5 against 32.1.  (A caller that names a spin limit asks
-  // for the launch whose waits it bounds.)
-  constexpr int64_t kRowsMax = 64, kRowsBytes = 135'000'000;
-  const int64_t expert_bytes = ((int64_t)p.nfr1 * p.nst1 + (int64_t)p.nfr2 * p.nst2) * (2048 + 128);
-  if (d->spin_limit <= 0 && k <= kDecRowsMaxK && R <= kRowsMax && R * expert_bytes <= kRowsBytes) return decode_launch_rows(p, static_cast<hipStream_t>(stream));
+  if (d->spin_limit <= 0 && decode_by_rows(T, k, d->d_ff, d->d_model)) return decode_launch_rows(p, static_cast<hipStream_t>(stream));
   const bool small_e = E <= 128;
   int grid = small_e ? resident_workgroups<8>() : resident_workgroups<kDecMaxExperts / 16>();
   if (grid <= 0) return fail(TK_ERR_LAUNCH, "tk_moe_decode_layer: cannot determine how many workgroups are resident together");

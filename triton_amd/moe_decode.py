@@ -32,7 +32,7 @@ _WORKSPACES: dict = {}
 
 
 def _workspace(device, T, k, E, d_ff, d_model) -> torch.Tensor:
-    """Scratch of the launch (hidden activations, the k partial rows, counters), one per (device, stream, shape), made
+    """Scratch of the single launch (hidden activations, the k partial rows, counters), one per (device, stream, shape), made
     on first use with its counter words zero; the kernel leaves them zero, so launches in stream order share it."""
     key = (device.index, nt.stream_ptr(device), T, k, E, d_ff, d_model)
     ws = _WORKSPACES.get(key)
@@ -47,9 +47,12 @@ def _workspace(device, T, k, E, d_ff, d_model) -> torch.Tensor:
 
 def workspace_error_word(x, logits, n_expts_act, w1) -> int:
     """The sticky error word of the workspace `moe_mlp` uses for these arguments on the current stream (synchronises;
-    for tests): 0 = fine, bit 0 = a bounded wait ran out, bit 1 = the unit table overflowed."""
+    for tests): 0 = fine, bit 0 = a bounded wait ran out, bit 1 = the unit table overflowed.  A layer that goes row by row waits for
+    nothing and has none: 0."""
     T, E = logits.shape
     d_model, n1 = w1.shape[-2:]
+    if nt.rules().decode_by_rows(T, n_expts_act, n1 // 2, d_model):
+        return 0
     ws = _workspace(x.device, T, n_expts_act, E, n1 // 2, d_model)
     words = ws[-(2 + (MAX_ROWS + MAX_ROWS // 16) * 32 + T * ((d_model + 31) // 32)) * 4:].view(torch.int32)
     return int(words[1].item())
@@ -123,8 +126,12 @@ def moe_decode_layer(x, logits, n_expts_act, w1, b1, w2, b2, pc1: PrecisionConfi
         assert out.shape == (T, d_model) and out.dtype == torch.bfloat16 and out.stride(-1) == 1
     if T == 0:
         return (out, None, None) if return_routing else out
-    ws = _workspace(x.device, T, k, E, d_ff, d_model)
     d = nt.DecodeLayerDesc()
+    if d.spin_limit <= 0 and nt.rules().decode_by_rows(T, k, d_ff, d_model):
+        # two launches that keep nothing between calls: memory of this call's own, which a captured graph's pool then owns
+        ws = torch.empty(nt.lib().tk_moe_decode_layer_workspace_bytes(T, k, E, d_ff, d_model), dtype=torch.uint8, device=x.device)
+    else:
+        ws = _workspace(x.device, T, k, E, d_ff, d_model)
     d.x, d.x_stride_m = x.data_ptr(), x.stride(0)
     d.logits, d.logits_dtype, d.logits_stride_m = logits.data_ptr(), nt.TORCH_TO_TK[logits.dtype], logits.stride(0)
     d.n_tokens, d.n_experts, d.k, d.apply_softmax = T, E, k, int(apply_softmax)
