@@ -57,6 +57,9 @@ enum tk_mx_rounding {
 /* Library version (major*10000 + minor*100 + patch). */
 int32_t tk_version(void);
 
+/* A number of the graph capture that `stream` is in, 0 = none: for callers that keep a workspace whose words a captured graph may have to zero. */
+int64_t tk_stream_capture_id(tk_stream_t stream);
+
 /* Message of the last error raised on the calling thread ("" if none).  Host pointer. */
 const char* tk_last_error(void);
 

@@ -1,5 +1,6 @@
 """The memory that decode layers are launched with, on the CPU (the descriptors are looked at, nothing is launched): the two launches of a layer that
-goes row by row get memory of the call's own, so that a captured graph's belongs to the graph."""
+goes row by row get memory of the call's own, so that a captured graph's belongs to the graph, and the single launch's workspace, which keeps
+counters between calls, stays where a graph has its address."""
 import pytest
 import torch
 
@@ -9,10 +10,13 @@ from triton_amd import moe_decode
 
 class _Library:
     def __init__(self, real):
-        self.real, self.given = real, []
+        self.real, self.given, self.capture = real, [], 0
 
     def __getattr__(self, name):
         return getattr(self.real, name)
+
+    def tk_stream_capture_id(self, stream):
+        return self.capture
 
     def tk_moe_decode_layer(self, d, stream):
         self.given.append(d.workspace)
@@ -36,6 +40,7 @@ def layer(monkeypatch):
     monkeypatch.setattr(moe_decode, "one_launch_reason", lambda *a: None)
     monkeypatch.setattr(moe_decode, "_swiglu_args", lambda act: (1.702, 7.0, 1))
     monkeypatch.setattr(moe_decode, "_WORKSPACES", {})
+    monkeypatch.setattr(moe_decode, "_CAPTURED", {})
 
     class PC:
         def __init__(self, w):
@@ -61,5 +66,54 @@ def test_the_single_launch_keeps_its_counters(layer, T, k, dims):
     assert not nt.rules().decode_by_rows(T, k, dims, dims)
     layer(T, k, dims)
     layer(T, k, dims)
-    (ws, ) = moe_decode._WORKSPACES.values()
+    ((ws, _), ) = moe_decode._WORKSPACES.values()
     assert layer.given == [ws.data_ptr()] * 2
+
+
+@pytest.fixture
+def capturing(layer):
+    """capturing(id): the current stream counts as being captured, 0 = no longer."""
+    return lambda capture: setattr(nt.lib(), "capture", capture)
+
+
+def _others(n):
+    for t in range(n):
+        moe_decode._workspace(torch.device("cpu"), 1 + t, 32, 512, 64, 64)
+
+
+def test_a_captured_workspace_is_never_dropped(layer, capturing):
+    """Warmed up, captured, then more other shapes than are kept: the graph's address is still this workspace's, and no other one's."""
+    layer(16, 4)
+    capturing(7)
+    layer(16, 4)
+    capturing(0)
+    warm, captured = layer.given
+    assert warm == captured
+    ws = moe_decode._workspace(torch.device("cpu"), 16, 4, 128, 2880, 2880)
+    assert ws.data_ptr() == captured
+    _others(150)
+    assert len(moe_decode._WORKSPACES) <= 64
+    assert moe_decode._workspace(torch.device("cpu"), 16, 4, 128, 2880, 2880) is ws
+    layer(16, 4)
+    assert layer.given[-1] == captured
+
+
+def test_workspaces_without_a_graph_are_dropped(layer):
+    import weakref
+    first = weakref.ref(moe_decode._workspace(torch.device("cpu"), 16, 4, 128, 2880, 2880))
+    _others(64)
+    assert first() is None and len(moe_decode._WORKSPACES) == 64
+
+
+def test_a_workspace_made_in_a_capture_is_that_captures_own(layer, capturing):
+    """Its counters are zero only once that graph has run, so neither an eager call nor another capture may be given it."""
+    get = lambda: moe_decode._workspace(torch.device("cpu"), 16, 4, 128, 2880, 2880)
+    capturing(7)
+    first = get()
+    assert get() is first
+    capturing(8)
+    second = get()
+    assert second is not first and get() is second
+    capturing(0)
+    eager = get()
+    assert eager is not first and eager is not second and get() is eager

@@ -250,3 +250,44 @@ def test_padded_activation_rows_give_what_contiguous_rows_give(api, device, gpto
     torch.cuda.synchronize()
     assert api.md.workspace_error_word(x, logits, 4, W["w1"]) == 0
     assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("warm", [True, False])
+def test_graphs_keep_their_workspace(api, device, gptoss_weights, warm):
+    """Two graphs of two layers each captured on one stream, with and without eager launches on it before; then eager launches on that stream and
+    workspaces of more shapes than are kept.  Replayed one after the other, the later one first, each gives the eager launch's result bit for bit."""
+    from triton_amd import _native as nt
+    g = torch.Generator().manual_seed(37)
+    T, E, k, d = 16, 128, 4, 2880
+    W, act = gptoss_weights["tiled"], api.act(1.702, 7.0)
+    inputs = lambda: (torch.randn((T, d), generator=g).to(torch.bfloat16).to(device), (torch.randn((T, E), generator=g)).to(device))
+    ins = [inputs(), inputs()]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    graphs, outs = [], []
+    with torch.cuda.stream(side):
+        assert nt.lib().tk_stream_capture_id(nt.stream_ptr(device)) == 0
+        if warm:
+            _run(api, W, *ins[0], k, act)
+        ids = []
+        for x, logits in ins:
+            graph = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graph, stream=side):
+                ids.append(nt.lib().tk_stream_capture_id(nt.stream_ptr(device)))
+                outs.append([_run(api, W, x, logits, k, act) for _ in range(2)])
+            graphs.append(graph)
+        assert ids[0] and ids[1] and ids[0] != ids[1]
+        eager = [_run(api, W, x, logits, k, act) for x, logits in ins]
+        for t in range(1, 71):
+            api.md._workspace(device, t, 1, 128, 64, 64)
+        others = [torch.full((n, ), 0x7F, dtype=torch.uint8, device=device) for n in (65536, 1 << 20, 1 << 20, 4 << 20)]
+    torch.cuda.synchronize()
+    want = [_run(api, W, x, logits, k, act) for x, logits in ins]
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(eager, want))
+    for rep in range(3):
+        for i in (1, 0):
+            graphs[i].replay()
+            torch.cuda.synchronize()
+            assert all(torch.equal(o, want[i]) for o in outs[i]), f"graph {i}, replay {rep}"
+    assert all(bool((o == 0x7F).all()) for o in others)

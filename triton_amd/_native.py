@@ -99,6 +99,7 @@ class DecodeLayerDesc(_c.Structure):
 # name -> (restype, argtypes); must list every symbol include/triton_amd.h declares.
 SIGNATURES = {
     "tk_version": (_i32, []),
+    "tk_stream_capture_id": (_i64, [_ptr]),
     "tk_last_error": (_c.c_char_p, []),
     "tk_mx_downcast": (_i32, [_ptr, _i32, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _i32, _i32, _ptr]),
     "tk_route_workspace_bytes": (_i64, [_i32, _i32]),

@@ -1,4 +1,4 @@
-// Library-wide pieces of the C ABI: version, per-thread error string, and host-side evaluation of the
+// Library-wide pieces of the C ABI: version, per-thread error string, what capture a stream is in, and host-side evaluation of the
 // scalar MX conversions (so their bit-exactness can be checked on a machine without a GPU).
 #include <string.h>
 
@@ -21,6 +21,16 @@ int32_t fail(int32_t code, const char* fmt, ...) {
 extern "C" int32_t tk_version(void) { return 100; }
 
 extern "C" const char* tk_last_error(void) { return tk::g_last_error; }
+
+extern "C" int64_t tk_stream_capture_id(tk_stream_t stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  if (hipStreamGetCaptureInfo(static_cast<hipStream_t>(stream), &status, &id) != hipSuccess) {
+    (void)hipGetLastError();  // (asked of the default stream while another one is captured)
+    return 0;
+  }
+  return status == hipStreamCaptureStatusActive ? (int64_t)id + 1 : 0;
+}
 
 extern "C" int32_t tk_host_mx_convert(const float* in, int64_t n, int32_t kind, uint8_t* out) {
   if (!in || !out || n < 0) return tk::fail(TK_ERR_INVALID, "tk_host_mx_convert: bad argument");

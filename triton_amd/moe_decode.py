@@ -28,20 +28,33 @@ MIN_ROWS = 1  # below this `moe_mlp` prefers the three calls
 MAX_EXPERTS = 512
 MAX_DIM = 3072
 
-_WORKSPACES: dict = {}
+_WORKSPACES: dict = {}  # key -> (workspace, the graph capture that it was made in or 0)
+_CAPTURED: dict = {}  # key -> workspace that a graph has the address of
 
 
 def _workspace(device, T, k, E, d_ff, d_model) -> torch.Tensor:
     """Scratch of the single launch (hidden activations, the k partial rows, counters), one per (device, stream, shape), made
-    on first use with its counter words zero; the kernel leaves them zero, so launches in stream order share it."""
-    key = (device.index, nt.stream_ptr(device), T, k, E, d_ff, d_model)
-    ws = _WORKSPACES.get(key)
-    if ws is None:
+    on first use with its counter words zero; the kernel leaves them zero, so launches in stream order share it.  The oldest of 64 is
+    dropped, but one that a call under graph capture was given is kept for the life of the process (a graph does not say when it ends):
+    graphs captured on one stream at one shape must not be replayed concurrently with each other.  One first made under capture lies in
+    the graph's memory and is zeroed by its replays, so only that capture's calls share it."""
+    stream = nt.stream_ptr(device)
+    key = (device.index, stream, T, k, E, d_ff, d_model)
+    ws = _CAPTURED.get(key)
+    if ws is not None:
+        return ws
+    capture = nt.lib().tk_stream_capture_id(stream)
+    ws, made_in = _WORKSPACES.get(key, (None, 0))
+    if ws is None or made_in not in (0, capture):
         nbytes = nt.lib().tk_moe_decode_layer_workspace_bytes(T, k, E, d_ff, d_model)
         ws = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+        _WORKSPACES.pop(key, None)
         if len(_WORKSPACES) >= 64:
             _WORKSPACES.pop(next(iter(_WORKSPACES)))
-        _WORKSPACES[key] = ws
+        _WORKSPACES[key] = (ws, capture)
+    elif capture and not made_in:
+        _CAPTURED[key] = ws
+        del _WORKSPACES[key]
     return ws
 
 
