@@ -422,7 +422,10 @@ int32_t tk_ragged_k_gemm(const tk_ragged_k_desc* desc, tk_stream_t stream);
  * multiples of 8; otherwise TK_ERR_UNSUPPORTED (callers then take tk_route + tk_moe_gemm).
  *
  * With spin_limit 0, k <= 8, up to 64 rows and at most 135 MB of weights counted once per row, the layer runs row by row in two launches that
- * wait for nothing (callers need not serialise those; nothing of the workspace's synchronisation words is touched).  Otherwise it is one launch:
+ * wait for nothing, so calls may overlap in time; but the first leaves the hidden activations and the routing in the workspace for the second, so
+ * calls that are not in stream order need workspaces of their own.  Of the workspace's synchronisation words nothing is read or written, and they
+ * need not be zero.  (Calls of several threads on one stream may share a workspace: the two launches of a call are enqueued together.)
+ * Otherwise it is one launch:
  * The kernel is persistent: its workgroups must all be resident together (the grid is sized from the occupancy the
  * runtime reports) because workgroups of the second GEMM wait for the first GEMM's rows of other workgroups.  Two
  * launches of it that overlap in time on one device (different streams) could each hold part of the GPU and wait

@@ -151,3 +151,44 @@ def test_graphs_of_one_stream_replayed_side_by_side(device, small_layer):
         torch.cuda.synchronize()
         for w, out in zip(want, outs):
             assert all(torch.equal(w, o) for o in out), f"replay {rep}"
+
+
+def test_threads_of_one_stream_may_share_a_workspace(device, monkeypatch):
+    """The two launches of a call are enqueued together: calls of two threads on one stream with one workspace give what each gives alone."""
+    import threading
+
+    from bench import make_moe_weights, to_matmul_layout
+    from triton_amd import _native as nt
+    from triton_kernels import moe_decode
+    from triton_kernels.matmul import FnSpecs, FusedActivation, PrecisionConfig
+    from triton_kernels.swiglu import swiglu_fn
+    W = to_matmul_layout(make_moe_weights(8, 256, 512, seed=4, device=device)[0])
+    act = FusedActivation(FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0))
+    pc1, pc2 = PrecisionConfig(b_mx_scale=W["w1s"]), PrecisionConfig(b_mx_scale=W["w2s"])
+    layer = lambda x, logits: moe_decode.moe_decode_layer(x, logits, 4, W["w1"], W["b1"], W["w2"], W["b2"], pc1, pc2, act)
+    g = torch.Generator().manual_seed(13)
+    ins = [_inputs(2, device, g) for _ in range(2)]
+    want = [layer(*i) for i in ins]
+    real = nt.rules()
+
+    class Rules:  # (the workspace of the single launch, which calls of one stream and shape share, for the same two launches)
+        def __getattr__(self, name):
+            return (lambda *a: False) if name == "decode_by_rows" else getattr(real, name)
+
+    monkeypatch.setattr(nt, "rules", lambda: Rules())
+    outs, errors = [[], []], []
+
+    def work(i):
+        try:
+            outs[i] += [layer(*ins[i]) for _ in range(200)]
+        except Exception as e:
+            errors.append(e)
+    threads = [threading.Thread(target=work, args=(i, )) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not errors
+    for i in range(2):
+        assert len(outs[i]) == 200 and all(torch.equal(o, want[i]) for o in outs[i])

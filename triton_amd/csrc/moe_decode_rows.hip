@@ -212,7 +212,7 @@ __global__ __launch_bounds__(kDownWaves * 64) void decode_rows_down_kernel(const
 int32_t decode_launch_rows(const DecodeParams& p, hipStream_t st) {
   const dim3 up((unsigned)p.nfr1, (unsigned)(p.T * p.k)), down((unsigned)cdiv(p.N2, 16), (unsigned)p.T);
   auto launch = [&](auto up_kern, auto down_kern) -> int32_t {
-    // the two launches of a call stay together: another thread's on the same stream has the same workspace
+    // the two launches of a call stay together: another thread's on the same stream may have the same workspace
     static std::mutex together;
     std::lock_guard<std::mutex> lock(together);
     hipLaunchKernelGGL(up_kern, up, dim3(kUpWaves * 64), 0, st, p);
