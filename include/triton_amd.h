@@ -421,7 +421,8 @@ int32_t tk_ragged_k_gemm(const tk_ragged_k_desc* desc, tk_stream_t stream);
  * Limits: n_tokens * k <= TK_DECODE_MAX_ROWS, n_experts <= TK_DECODE_MAX_EXPERTS, d_model and d_ff <= 3072 and
  * multiples of 8; otherwise TK_ERR_UNSUPPORTED (callers then take tk_route + tk_moe_gemm).
  *
- * With spin_limit 0, k <= 8, up to 64 rows and at most 135 MB of weights counted once per row, the layer runs row by row in two launches that
+ * With spin_limit 0, k <= 8 and up to 64 rows whose weights, counted once per row, are a small stream (at most some 170 MB, less the more rows
+ * and tokens there are: decode_by_rows in gemm_limits.h), the layer runs row by row in two launches that
  * wait for nothing, so calls may overlap in time; but the first leaves the hidden activations and the routing in the workspace for the second, so
  * calls that are not in stream order need workspaces of their own.  Of the workspace's synchronisation words nothing is read or written, and they
  * need not be zero.  (Calls of several threads on one stream may share a workspace: the two launches of a call are enqueued together.)

@@ -117,3 +117,16 @@ def test_a_workspace_made_in_a_capture_is_that_captures_own(layer, capturing):
     capturing(0)
     eager = get()
     assert eager is not first and eager is not second and get() is eager
+
+
+@pytest.mark.parametrize("T, k, d_ff, d_model, by_rows", [
+    (1, 4, 2880, 2880, True), (7, 1, 3072, 3072, True), (2, 4, 2880, 2880, True), (9, 1, 2880, 2880, True), (5, 2, 2880, 2880, True),
+    (3, 4, 2880, 2880, False), (12, 1, 2880, 2880, False), (4, 4, 2880, 2880, False),
+    (16, 1, 2048, 2048, True), (10, 2, 2048, 2048, True), (21, 1, 2048, 2048, False), (13, 2, 2048, 2048, False),
+    (24, 1, 1536, 1536, True), (4, 8, 1536, 1536, True), (32, 1, 1536, 1536, False), (20, 2, 1536, 1536, False),
+    (32, 1, 1024, 1024, True), (24, 2, 1024, 1024, True), (8, 8, 1024, 1024, True), (48, 1, 1024, 1024, False), (64, 1, 1024, 1024, False),
+    (32, 2, 1024, 1024, False), (16, 2, 2048, 1024, True), (32, 1, 2048, 1024, False), (64, 1, 512, 512, True), (4, 16, 512, 512, False),
+])
+def test_which_layers_go_row_by_row(T, k, d_ff, d_model, by_rows):
+    """Both sides of the line, at sizes where each form of launch was measured to be the faster one (or, in the end, is the only one)."""
+    assert nt.rules().decode_by_rows(T, k, d_ff, d_model) == by_rows

@@ -20,6 +20,7 @@ pytestmark = pytest.mark.gpu
     (64, 130, 1, 360, 248, None, 7.0, torch.float32),
     (16, 6, 4, 520, 1144, torch.bfloat16, None, torch.float32),
     (8, 512, 8, 144, 96, torch.bfloat16, 7.0, torch.float32),
+    (5, 8, 2, 2880, 2880, torch.bfloat16, 7.0, torch.float32),
 ])
 def test_rows_against_oracle_and_single_launch(device, monkeypatch, T, E, k, d_model, d_ff, bias_dtype, limit, logits_dtype):
     from bench import to_matmul_layout

@@ -47,19 +47,25 @@ inline bool reads_once(int64_t rows, int64_t n_slices, int64_t block_rows, int64
 // the mean make, as a random routing does (at 62 rows per slice half of the slices have a second block).
 inline int64_t few_row_blocks(int64_t rows, int64_t n_slices) { return n_slices * (rows * 5 / (n_slices * 256) + 1); }
 
-// The decode layer row by row in two launches (moe_decode_rows.hip; up to kDecRowsMaxK experts a token), which keep nothing between calls: where the
-// rows' weights, counted for every row, are a small stream.  The single launch costs some 20 us around its stream, the two launches 7, but they read
-// an expert's weights again for each of its rows.  Measured (us, row by row against single launch; 2880 x 5760 and 2880 x 2880 but where noted): 8
-// rows, 106 MB, 29.8 against 37.1; 10 rows of 8 experts, 132 MB, 31.5 against 37.0; 12 rows of 10 experts, 159 MB, 39.9 against 40.0; 16 rows of 12,
-// 211 MB, 46.8 against 44.8.  Smaller layers: d and d_ff 512, 64 rows of 13 experts, 27 MB, 15.7 against 28.1; 1024, 64 rows, 107 MB, 30.3 against
-// 39.0; 1024 and 2048, 32 rows of 4 experts, 107 MB, 26.8 against 30.6; 512, 256 rows of 21 experts, 107 MB, 52.5 against 32.1.  (A caller that
-// names a spin limit asks for the launch whose waits it bounds.)
+// The decode layer row by row in two launches (moe_decode_rows.hip; up to kDecRowsMaxK experts a token), which keep nothing between calls: where that
+// is the smaller stream.  The single launch costs some 30 us around its stream but reads an expert once; the two launches cost 4, but they read
+// an expert's weights (padded, as they lie in memory) again for each of its rows, at about 4 MB/us, and the second one's workgroups, one for a token and
+// 16 columns, take 5.5 ns each, as long as 22 KB do.  The more rows, the more of them share an expert, which nobody knows here: 1 MB a row.
+// Measured (us, row by row against single launch, with all experts alike; with a few that most tokens choose), at MB of this sum:
+//   d and d_ff 2880, 128 experts: 8 rows, top 4, 124 MB, 31 / 38; 30 / 37; 10 rows, top 2, 165, 38 / 42; 33 / 39; 12, top 4, 186, 44 / 45; 40 / 40
+//   2048, 64 experts: 16, top 1, 168, 36 / 41; 33 / 34; 20, top 2, 182, 36 / 45; 32 / 36; 21, top 1, 221, 46 / 46; 41 / 35; 26, top 2, 236, 46 / 50; 40 / 38
+//   1536, 32 experts: 32, top 8, 161, 36 / 44; 35 / 38; 24, top 1, 165, 35 / 39; 31 / 32; 40, top 2, 233, 37 / 42; 35 / 31; 32, top 1, 220, 44 / 42; 40 / 33
+//   1024, 32 experts: 48, top 2, 162, 31 / 40; 28 / 31; 64, top 8, 182, 36 / 41; 35 / 36; 64, top 2, 216, 39 / 41; 35 / 31; 48, top 1, 196, 41 / 41; 36 / 32;
+//     64, top 1, 261, 51 / 42; 47 / 32
+//   1024 and 2048, 8 experts: 32, top 2, 162, 30 / 31; 29 / 31; 32, top 1, 184, 36 / 31; 33 / 30
+//   512, 32 experts: 64, top 1, 136, 26 / 31; 26 / 29
+// (A caller that names a spin limit asks for the launch whose waits it bounds.)
 constexpr int kDecRowsMaxK = 8;
 inline bool decode_by_rows(int64_t T, int64_t k, int64_t d_ff, int64_t d_model) {
-  constexpr int64_t kRowsMax = 64, kRowsBytes = 135'000'000;
+  constexpr int64_t kRowsMax = 64, kRowsBytes = 183'000'000, kWorkgroupBytes = 22'000, kRowBytes = 1'000'000;
   auto parts = [](int64_t n, int64_t of) { return (n + of - 1) / of; };
   const int64_t expert_bytes = (parts(2 * d_ff, 32) * parts(d_model, 128) + parts(d_model, 32) * parts(d_ff, 128)) * (2048 + 128);
-  return k <= kDecRowsMaxK && T * k <= kRowsMax && T * k * expert_bytes <= kRowsBytes;
+  return k <= kDecRowsMaxK && T * k <= kRowsMax && T * k * (expert_bytes + kRowBytes) + T * parts(d_model, 16) * kWorkgroupBytes <= kRowsBytes;
 }
 
 }  // namespace tk
