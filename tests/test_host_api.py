@@ -342,3 +342,12 @@ def test_16_bit_tiles_at_256_rows_are_the_kernels_own(gemm_calls):
     for constraints in ({"block_n": 64}, {"block_n": 256, "num_warps": 4}, {"block_n": 128, "block_k": 64}):
         with scoped_opt_flags_constraints({"block_m": 256, **constraints}), pytest.raises(of.InapplicableConstraint):
             of.make_opt_flags(None, None, torch.bfloat16, None, 1, rows, n, k, md)
+
+
+@pytest.mark.parametrize("per_slice, N, n_slices, want", [
+    (32, 1024, 8, 32), (32, 2048, 8, 64), (48, 1024, 16, 64), (49, 1024, 16, 0), (51, 1024, 16, 0), (48, 512, 32, 64), (51, 512, 32, 0),
+    (51, 2048, 8, 64), (51, 16384, 1, 64), (51, 256, 32, 32), (51, 512, 16, 32), (62, 512, 16, 64), (62, 1024, 16, 0), (64, 1024, 8, 64), (65, 64, 8, 0)])
+def test_columns_of_the_kernel_for_few_rows(per_slice, N, n_slices, want):
+    """Both sides of the line: with 64 columns a second round for slices of over 64 rows costs more than the kernel gains."""
+    from triton_amd import _native as nt
+    assert nt.rules().few_block_n(per_slice * n_slices, N, n_slices) == want

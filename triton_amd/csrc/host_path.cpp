@@ -220,15 +220,23 @@ int64_t wide_block_m(int64_t rows, int64_t n_slices, int64_t K, uint32_t x_bytes
 }
 
 // Columns a workgroup of the kernel for few rows, 0 = the kernels above: up to 64 rows per slice and one workgroup per CU at most, with 32
-// columns while they fit, then 64.  Measured (us, this kernel against the one that ran before): 16 slices, 2 or 8 rows each, K 512,
-// N 1024 4.2 against 6.6, K 256, N 512 4.2 against 4.9; 32 rows each, 8 slices, K 512, N 2048 6.3 against 9.4, K 1024, N 512 5.7 against
-// 12.1; 64 rows, K 1024, N 512 6.7 against 12.4; 16 slices of 32 rows, K 1024, N 1024 8.5 against 14.5.  With two workgroups per CU to be
+// columns while they fit, then 64.  Measured (us, this kernel against the one that ran before; other weights each call): 8 slices of 32
+// rows, N 2048: K 512 9.1 against 12.1, K 2048 20 against 28, K 8192 60 against 76; N 512: K 1024 7.6 against 15.4, K 8192 26 against 72; 64 rows, N
+// 1024: K 512 9.0 against 11.6, K 8192 47 against 77; one slice of 50 rows, N 16384: K 512 10.4 against 12.3, K 8192 67 against 77; 16 slices
+// of 28 rows, some of them over 64, N 1024: K 512 11.7 against 12.3, K 2048 24 against 28.  The same weights again: 8 slices of 32 rows, K 512,
+// N 2048 6.3 against 9.4; 16 slices, 2 or 8 rows each, K 512, N 1024 4.2 against 6.6.
+// 64 columns only up to 48 rows per slice where one row block of more than eight slices each is counted on: a slice of more than 64 rows is then a
+// second round, which takes as long as the first (16 slices, N 1024, of 48 rows: K 512 11.1 against 12.7, K 2048 22 against 28; of 51: 12.4 against
+// 12.7 and 29 against 28, with such a slice in every routing 15.2 against 12.3; 32 slices of 51, N 512, K 1024 19 against 18).  Eight slices seldom
+// have one (of 51 rows, N 2048: K 512 11.2 against 12.8, K 2048 24 against 28), and with 32 columns it is the faster way all the same (32
+// slices of 51, N 256: K 512 9.6 against 10.6, K 2048 19 against 25).  With two workgroups per CU to be
 // run in turn the others are as fast or faster (16 slices, K 1024, N 2048: 8 rows 16.8 against 15.5, 32 rows 19.6 against 16.8; 8 slices of
 // 125 rows, K 512, N 1024: 12.0 against 9.9).
 int64_t few_block_n(int64_t rows, int64_t N, int64_t n_slices) {
   if (n_slices < 1 || rows > 64 * n_slices) return 0;
   const int64_t blocks = tk::few_row_blocks(rows, n_slices);
-  return blocks * ((N + 31) / 32) <= 256 ? 32 : blocks * ((N + 63) / 64) <= 256 ? 64 : 0;
+  if (blocks * ((N + 31) / 32) <= 256) return 32;
+  return blocks * ((N + 63) / 64) <= 256 && (rows <= 48 * n_slices || n_slices <= 8 || blocks > n_slices) ? 64 : 0;
 }
 
 int64_t default_block_m(int64_t rows, int64_t n_slices) {
