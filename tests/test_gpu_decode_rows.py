@@ -21,6 +21,12 @@ pytestmark = pytest.mark.gpu
     (16, 6, 4, 520, 1144, torch.bfloat16, None, torch.float32),
     (8, 512, 8, 144, 96, torch.bfloat16, 7.0, torch.float32),
     (5, 8, 2, 2880, 2880, torch.bfloat16, 7.0, torch.float32),
+    # (k that does not divide the second launch's sixteen waves: some have no expert, and the others uneven shares of the stages)
+    (5, 9, 3, 264, 392, torch.bfloat16, 7.0, torch.float32),
+    (4, 7, 5, 520, 1656, torch.float32, 7.0, torch.bfloat16),
+    (2, 140, 6, 136, 3072, torch.bfloat16, None, torch.float32),
+    (9, 7, 7, 128, 640, None, 7.0, torch.float32),
+    (2, 8, 7, 1032, 2440, torch.bfloat16, 7.0, torch.float32),
 ])
 def test_rows_against_oracle_and_single_launch(device, monkeypatch, T, E, k, d_model, d_ff, bias_dtype, limit, logits_dtype):
     from bench import to_matmul_layout
@@ -66,7 +72,9 @@ def test_rows_against_oracle_and_single_launch(device, monkeypatch, T, E, k, d_m
     h = omoe.matmul(xp, q[0], b1, r.meta.col_sum, gather_indx=r.gather_indx, w_mx_scale=q[1])
     a = torch.nn.functional.pad(omoe.swiglu(h, 1.702, limit), (0, -d_ff % 32))
     y = omoe.matmul(a, q[2], b2, r.meta.col_sum, scatter_indx=r.scatter_indx, gammas=r.gammas, w_mx_scale=q[3])
-    assert_close(omoe.reduce_k(y, k), out, maxtol=3e-2, what="row by row against the oracle")
+    # (the oracle rounds the pre-activations to bf16, which the kernels keep in fp32: these layers in 64 bits, rounded only where the kernels
+    # round, are 3.5e-3 to 4.02e-3 away from it)
+    assert_close(omoe.reduce_k(y, k), out, maxtol=3e-2, rmstol=4.5e-3, what="row by row against the oracle")
     # the two kernels sum K in different groupings: an ulp of a hidden value here and there
     assert_close(one.cpu(), out, maxtol=2e-2, what="row by row against the single launch")
 

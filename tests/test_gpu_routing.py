@@ -192,6 +192,63 @@ def test_every_way_through_the_router(device, T, E, k, dtype):
     assert_equal(ref.block_schedule_data, rd.expt_data.block_schedule_data, "block_schedule")
 
 
+@pytest.mark.parametrize("T, E, k", [(100, 16, 2), (128, 32, 8), (60, 17, 4), (64, 128, 4), (3, 8, 2), (300, 128, 4), (1021, 252, 4), (5000, 8, 1), (300, 260, 4)])
+@pytest.mark.parametrize("rows", ["none", "one", "some", "all but one", "more than there are"])
+@pytest.mark.parametrize("on_device", [False, True])
+def test_a_row_mask_on_every_way(device, T, E, k, rows, on_device):
+    """Rows from `n_rows` on are not routed, whichever kernels take the call and whether the number lies on the host or on the device."""
+    from triton_amd.legacy import routing
+    n = {"none": 0, "one": 1, "some": T * 2 // 3, "all but one": T - 1, "more than there are": T + 5}[rows]
+    x = _logits(T, E, torch.float32, seed=T + E)
+    rd, gather, scatter = routing(x.to(device), k, n_rows=torch.tensor([n], dtype=torch.int32, device=device) if on_device else n)
+    vals, indx, _ = ort.topk(x, k, n_rows=min(n, T))
+    m = ort.make_bitmatrix_metadata(indx, E)
+    live = min(n, T)
+    assert_equal(indx[:live], rd.expt_indx[:live].to(torch.int32), "indx")
+    if live:
+        assert_close(vals[:live], rd.gate_vals[:live], what="vals")
+    assert_equal(m.col_sum, rd.expt_hist, "col_sum")
+    assert_equal(m.col_sorted_indx, gather.src_indx, "col_sorted_indx")
+    assert_equal(m.row_sorted_indx, scatter.src_indx, "row_sorted_indx")
+    col = m.col_sorted_indx[:live * k]
+    assert_equal(torch.div(col, k, rounding_mode="floor").to(torch.int32), rd.token_indx[:live * k], "gather index")
+    assert bool((rd.token_indx[live * k:] == -1).all())
+    assert torch.equal(rd.gate_scal[:live * k], rd.gate_vals.flatten()[col.long().to(device)])
+    ref = ort.make_ragged_tensor_metadata(m.col_sum, T * k)
+    assert_equal(ref.slice_offs, rd.expt_data.slice_offs, "slice_offs")
+    assert_equal(ref.block_offs_data, rd.expt_data.block_offs_data, "block_offs")
+    assert_equal(ref.block_schedule_data, rd.expt_data.block_schedule_data, "block_schedule")
+
+
+@pytest.mark.parametrize("E, k", [(8, 2), (16, 4), (32, 8), (64, 4), (128, 8)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_logits_that_are_no_numbers(device, E, k, dtype):
+    """Experts masked with -inf or the lowest finite value against the oracle; and rows with infinities and NaN, whose order no oracle
+    defines, select and weigh the same in a batch of their own (one workgroup) as among many rows (several)."""
+    from triton_amd.legacy import routing
+    x = _logits(16, E, torch.float32, seed=E)
+    x[0, ::2] = float("-inf")  # (E / 2 >= k are left)
+    x[1, k:] = float("-inf")
+    x[2, 1:] = torch.finfo(dtype).min
+    x = x.to(dtype)
+    rd, _, _ = routing(x.to(device), k)
+    vals, indx, _ = ort.topk(x, k)
+    assert_equal(indx, rd.expt_indx.to(torch.int32), "indx")
+    assert_close(vals, rd.gate_vals, what="vals")
+    x[3] = float("-inf")
+    x[4] = float("nan")
+    x[5, E // 2] = float("inf")
+    x[6, 1], x[6, E - 1] = float("nan"), float("inf")
+    x[7, ::3] = float("nan")
+    x[8, 2:] = float("nan")
+    x[9, 0], x[9, 1] = float("inf"), float("-inf")
+    few, _, _ = routing(x.to(device), k)
+    many, _, _ = routing(torch.cat([x, _logits(2000, E, dtype, seed=1)]).to(device), k)
+    assert torch.equal(few.expt_indx, many.expt_indx[:16])
+    assert int(few.expt_indx.min()) >= 0 and int(few.expt_indx.max()) < E
+    torch.testing.assert_close(few.gate_vals, many.gate_vals[:16], equal_nan=True, rtol=1e-6 if dtype == torch.float32 else 2**-7, atol=0)
+
+
 @pytest.mark.parametrize("n_slices", [9, 32, 911, 1025])
 def test_remap_ragged_tensor_metadata(device, n_slices):
     """Mirrors tests/test_tensor.py:259-277 of the reference: random sizes with an empty slice, a random permutation as
