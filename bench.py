@@ -270,9 +270,10 @@ def bench_decode(device, steps, warmup, n_layers=10):
     with their own weight copies are captured in ONE HIP graph, as a serving loop captures a decode step over all its
     layers (gpt-oss-120b has 36); the time of a layer is the replay time / n_layers.  Ten copies rotate at least
     530 MB of touched weights at every T (the last-level cache holds 256 MB), so no layer finds its weights cached.
-    Two paths are timed on the same inputs: `moe_mlp` (one launch per layer, two for one token) and the three-call
+    Two paths are timed on the same inputs: `moe_mlp` (one launch per layer, two where it goes row by row) and the three-call
     sequence routing -> matmul_ogs -> matmul_ogs.  Every layer's output of every checked replay is compared with the
     eager result before timing."""
+    from triton_amd._native import rules
     from triton_kernels.moe_decode import moe_mlp
     E, k, d, f2 = 128, 4, 2880, 5760
     copies = [to_matmul_layout(w) for w in make_moe_weights(E, d, f2, seed=3, device=device, n_copies=n_layers)]
@@ -312,7 +313,7 @@ def bench_decode(device, steps, warmup, n_layers=10):
                 timed[name]["board_under_replay"] = board_state_under(graph.replay)
             del graph
         best = min(timed, key=lambda n: timed[n]["ms"])
-        res[f"T{T}"] = dict(ms=timed[best]["ms"], path=best, launches_per_layer=3 if best != "moe_mlp" else 2 if T * k < 8 else 1,
+        res[f"T{T}"] = dict(ms=timed[best]["ms"], path=best, launches_per_layer=3 if best != "moe_mlp" else 2 if rules().decode_by_rows(T, k, f2 // 2, d) else 1,
                             active_experts=active, weight_GB=round(gbytes, 4), GBps=timed[best]["GBps"], frac_hbm=timed[best]["frac_hbm"],
                             layers_per_graph=n_layers, rotated_weight_GB=round(gbytes * n_layers, 3), **{n: timed[n] for n in timed})
     return res
