@@ -8,7 +8,7 @@ python/triton_kernels/tests/test_distributed.py:203-220 composes them:
     y        = matmul(x, w, bias, metadata, gather_indx=gather, scatter_indx=scatter, gammas=...)
     out      = reduce(y.view(T, k, -1), dim=1)                   when scattering
 
-`routing` obtains all of it from ONE fused routing pass (three kernel launches).  The router's own choice for every row
+`routing` obtains all of it from ONE fused routing pass (one to three kernel launches).  The router's own choice for every row
 is served by the native host path, where the bitmatrix, which `RoutingData` does not carry, is not made.  The histogram
 has memory of its own; the permutations and the gather index share theirs, and so does the block metadata.
 """

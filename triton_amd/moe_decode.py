@@ -1,4 +1,4 @@
-"""One-launch MoE FFN layer for decode-sized batches (no counterpart function in the reference).
+"""MoE FFN layer in one or two launches for decode-sized batches (no counterpart function in the reference).
 
 The reference's MoE block is a sequence of calls (python/triton_kernels/bench/bench_mlp.py:72-79):
 
@@ -24,7 +24,7 @@ from .tensor import FP4, Tensor
 from .tensor_details.layout_details.gfx950_mx import GFX950MXScaleLayout, GFX950MXValueLayout
 
 MAX_ROWS = 256
-MIN_ROWS = 1  # below this `moe_mlp` prefers the three calls
+MIN_ROWS = 1  # (a call without rows goes through the three calls)
 MAX_EXPERTS = 512
 MAX_DIM = 3072
 
@@ -120,7 +120,7 @@ def one_launch_reason(x, logits, n_expts_act, w1, b1, w2, b2, pc1, pc2, act) -> 
 
 def moe_decode_layer(x, logits, n_expts_act, w1, b1, w2, b2, pc1: PrecisionConfig, pc2: PrecisionConfig,
                      fused_activation: FusedActivation, *, apply_softmax: bool = True, out=None, return_routing: bool = False):
-    """The layer in one launch; raises NotImplementedError when `one_launch_reason` names an obstacle."""
+    """The layer in one launch, or two where it goes row by row; raises NotImplementedError when `one_launch_reason` names an obstacle."""
     why = one_launch_reason(x, logits, n_expts_act, w1, b1, w2, b2, pc1, pc2, fused_activation)
     if why is not None:
         raise NotImplementedError(f"moe_decode_layer: {why}")
