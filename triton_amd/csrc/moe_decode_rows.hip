@@ -9,8 +9,8 @@
 //     costs nothing beside the stream.
 //
 // What bounds it: launch 1 two dependent trips to memory (logits, weights) and launch 2 two (table, weights) around the streams of 35 and
-// 18 MB.  One token, 4 of 128 experts, K 2880, N 5760 and 2880: 18.6 us; with routing, a GEMM, and a GEMM that counts its rows for the sum
-// as launches of their own 29.7 us.
+// 18 MB.  One token, 4 of 128 experts, K 2880, N 5760 and 2880: 17.9 us (ten such layers in a graph, one after the
+// other); with routing, a GEMM, and a GEMM that counts its rows for the sum as launches of their own 28.4 us.
 #include "decode_params.h"
 #include "gemm_common.h"
 #include "route_common.h"

@@ -21,8 +21,8 @@
 //     as many stages, each as long as its way from memory (bf16, us: 8 slices of about 1024 rows, K 2048, N 2048 79 -> 70, K 4096, N 4096 262 -> 240,
 //     of about 512 rows 80 -> 73 and 156 -> 135; 16 of about 256, N 4096 85 to 95 -> 81).
 //
-// What bounds it: the board's power (a square bf16 product of 8192: matrix pipe 87 % busy at 1.58 GHz, 1390 TFLOP/s, 0.93 of what the
-// vendor's library reaches on the same board), with shorter K also the epilogues (e4m3, K 4096: 12 % of the time; matrix pipe 67 % busy at 1.8
+// What bounds it: the board's power (a square bf16 product of 8192: matrix pipe 87 % busy at 1.58 GHz, 1390 TFLOP/s, 0.87 to 0.93 of what
+// the vendor's library reaches on the same board), with shorter K also the epilogues (e4m3, K 4096: 12 % of the time; matrix pipe 67 % busy at 1.8
 // GHz, K 14336: 77 % at 1.75), with a few rows per expert (128 x 128 tiles) the weight stream at 5.9 TB/s (5.3 without the
 // non-temporal hint).  16384 routed rows
 // of 8 experts in e4m3: K 4096, N 28672, swiglu 1840 -> 1590 us (2.42 PFLOP/s), K 14336, N 4096 850 -> 805 us; 4096 rows of 16

@@ -14,7 +14,8 @@
 // What bounds it: a chain of latencies (slice sizes, row indices, rows, sums, store), 4.2 us at K 512 with next to nothing to do; its
 // instructions come from memory as well, once per launch: with the ring's first turns unrolled and every option of the epilogue in line
 // (4900 instructions) the same kernel took 1.2 to 2.3 us longer than now (2300).  Layer of 128 tokens, 8 experts, top 2, d 512,
-// d_ff 1024: first GEMM 9.4 -> 6.3 us, second 12.1 -> 5.7.
+// d_ff 1024: first GEMM 12.1 -> 9.1 us, second 15.4 -> 7.6 with other weights each call; with the same ones again, as far as they are in the
+// caches, 9.4 -> 6.3 and 12.1 -> 5.7.
 #include "gemm_common.h"
 #include "route_common.h"
 
