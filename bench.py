@@ -26,9 +26,9 @@ sys.path.insert(0, ROOT)
 PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA
 PEAK_HBM_GBPS = 8000.0  # MI355X HBM3E
 # HBM bytes one launch of the first expert GEMM moves at this workload, from two counter runs over this script
-# (FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000 KiB, factors from the 1 GiB copy of --calibrate-copy): 1480.7 MB read
+# (FETCH_SIZE x 2.000 + WRITE_SIZE x 1.000 KiB, factors from the 1 GiB copy of --calibrate-copy): 1303.9 MB read
 # + 96.5 MB written, against 1318.3 MB of algorithmic bytes.
-GEMM1_TRAFFIC_BYTES = 1.5772e9
+GEMM1_TRAFFIC_BYTES = 1.4004e9
 
 
 def make_moe_weights(E, d_model, d_ff2, seed, device, n_copies=1):
