@@ -68,27 +68,30 @@ __device__ __forceinline__ buf_desc_t make_buf_desc(const void* base, uint32_t b
 // 16 bytes per lane from `desc` at byte offset `off` into LDS at `dst` (wave-uniform byte address) + 16 * lane.  Written
 // as assembly because the compiler puts a wait for ALL outstanding memory operations in front of every LDS read that
 // follows the builtin form; here the kernel places its own vmcnt waits (the instruction counts as one).  m0, from which the transfer takes
-// its LDS address, is an operand, so that the compiler knows of it and computes the address straight into it; the s_nop is the wait
-// state that a write of m0 needs in front of such a transfer.
+// its LDS address, is an operand, so that the compiler knows of it and computes the address straight into it.
+// Wait states: a vector memory instruction may read a scalar register no sooner than five wait states after a vector instruction wrote it, and the
+// compiler, which keeps that distance for its own instructions, does not look into assembly.  A descriptor's words come from v_readfirstlane, or
+// back from a spill by v_readlane, at whatever distance the scheduler likes (two in one kernel: its first transfers now and then went by the
+// register's old contents, and read zeros or past the operand).  So every transfer brings its five; one is also what a write of m0 needs.
 // NT = with the non-temporal hint (streams that are read once).
 template <bool NT = false>
 __device__ __forceinline__ void lds_dma16(buf_desc_t desc, uint32_t dst, uint32_t off) {
   if constexpr (NT)
-    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"{m0}"(dst), "v"(off), "s"(desc) : "memory");
+    asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"{m0}"(dst), "v"(off), "s"(desc) : "memory");
   else
-    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"{m0}"(dst), "v"(off), "s"(desc) : "memory");
+    asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"{m0}"(dst), "v"(off), "s"(desc) : "memory");
 }
-// the same by the lower 32 lanes only (512 bytes; every lane is active when it is called; the write of exec_hi is the wait state)
+// the same by the lower 32 lanes only (512 bytes; every lane is active when it is called; the write of exec_hi is a wait state, too)
 __device__ __forceinline__ void lds_dma16_lower(buf_desc_t desc, uint32_t dst, uint32_t off) {
-  asm volatile("s_mov_b32 exec_hi, 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n\ts_mov_b32 exec_hi, -1" ::"{m0}"(dst), "v"(off), "s"(desc) : "memory");
+  asm volatile("s_nop 3\n\ts_mov_b32 exec_hi, 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds\n\ts_mov_b32 exec_hi, -1" ::"{m0}"(dst), "v"(off), "s"(desc) : "memory");
 }
 // the same with 4 bytes per lane
 template <bool NT = false>
 __device__ __forceinline__ void lds_dma4(buf_desc_t desc, uint32_t dst, uint32_t off) {
   if constexpr (NT)
-    asm volatile("s_nop 0\n\tbuffer_load_dword %1, %2, 0 offen nt lds" ::"{m0}"(dst), "v"(off), "s"(desc) : "memory");
+    asm volatile("s_nop 4\n\tbuffer_load_dword %1, %2, 0 offen nt lds" ::"{m0}"(dst), "v"(off), "s"(desc) : "memory");
   else
-    asm volatile("s_nop 0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"{m0}"(dst), "v"(off), "s"(desc) : "memory");
+    asm volatile("s_nop 4\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"{m0}"(dst), "v"(off), "s"(desc) : "memory");
 }
 // LDS byte address of a __shared__ object
 __device__ __forceinline__ uint32_t lds_addr(const void* p) {
