@@ -85,3 +85,70 @@ def test_wide_gemm_quantised_output(device, swiglu):
     step = torch.exp2(scale.float() - 127).repeat_interleave(32, 1)
     # (2^-8: the bf16 value's own rounding)
     assert torch.all((back - plain).abs() <= plain.abs() * (2.0**-4 + 2.0**-8) + step * 2.0**-10)
+
+
+# mean rows per slice, slices, K, N, sizes dealt in turn: every tile that the rules name, at the edges of its row blocks (one more, one less, none at
+# all), of its columns and of a wave's 64, with four stages of K (the fewest), remainders of K and of the scales' groups
+RULED = [
+    ("bf16", "32x256", 40, 512, 528, [0, 1, 31, 32, 33, 2, 13]),
+    ("bf16", "64x256", 64, 544, 1056, [63, 64, 65, 1, 0, 33, 127, 128, 129]),
+    ("bf16", "64x256", 64, 1312, 1040, [95, 32, 31, 97]),
+    ("bf16", "64x512", 256, 512, 544, [0, 1, 31, 32, 33, 63, 64, 65, 10]),
+    ("bf16", "96x512", 256, 736, 528, [95, 96, 97, 1, 33, 65, 64, 100]),
+    ("bf16", "160x512", 256, 512, 576, [159, 160, 161, 81, 80, 1, 33]),
+    ("mxfp8", "32x256", 128, 512, 576, [0, 1, 31, 32, 33, 2, 13]),
+    ("mxfp8", "64x512", 128, 672, 544, [0, 1, 31, 32, 33, 63, 64, 65, 10]),
+    ("mxfp8", "64x512", 256, 544, 1088, [0, 1, 31, 32, 63, 64, 65, 10, 2, 1, 0]),
+    ("mxfp8", "128x512", 128, 736, 576, [95, 96, 97, 1, 33, 65, 40]),
+    ("mxfp8", "128x512", 128, 928, 544, [127, 128, 129, 65, 64, 1, 33, 97, 96]),
+]
+
+
+@pytest.mark.parametrize("kind, tile, e, k, n, sizes", RULED)
+@pytest.mark.parametrize("swiglu, routed", [(True, True), (False, False), (False, True)])
+def test_tiles_by_the_rules(device, kind, tile, e, k, n, sizes, swiglu, routed):
+    """The tile of the wide kernel that the rules name gives, bit for bit, what the kernel for row blocks of 128 gives (whose sums over K run in the
+    same order): gathered and scattered rows, gate weights, rows without a destination, a quantised output."""
+    import triton_amd._native as nt
+    import triton_amd.matmul as mm
+    from triton_amd.numerics_details.mxfp import downcast_to_mxfp, quantize_mxfp8_fn
+    from triton_amd.swiglu import swiglu_fn
+    from triton_amd.tensor import FP4, convert_layout, make_ragged_tensor_metadata, wrap_torch_tensor
+    from triton_amd.tensor_details.layout import make_default_matmul_mxfp4_w_layout, make_default_matmul_mxfp4_w_scale_layout
+    g = torch.Generator(device=device).manual_seed(k + n)
+    sizes = torch.tensor([sizes[i % len(sizes)] for i in range(e)], dtype=torch.int32, device=device)
+    m = int(sizes.sum())
+    mx8 = kind == "mxfp8"
+    assert nt.rules().wide_block_n(m, e, k, n, m * k, mx8) == int(tile.split("x")[1])
+    x = torch.randn((m, k), generator=g, device=device).to(torch.bfloat16)
+    wq, ws = downcast_to_mxfp((torch.randn((e, k, n), generator=g, device=device) * 0.1).to(torch.bfloat16), torch.uint8, axis=1)
+    w = convert_layout(wrap_torch_tensor(wq, dtype=FP4), make_default_matmul_mxfp4_w_layout(mx_axis=1))
+    s = convert_layout(wrap_torch_tensor(ws), make_default_matmul_mxfp4_w_scale_layout(mx_axis=1))
+    bias = torch.randn((e, n), generator=g, device=device)
+    args = dict(fused_activation=mm.FusedActivation(mm.FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0)) if swiglu else None)
+    if routed:
+        args.update(gammas=torch.rand((m, ), generator=g, device=device) + 0.5, gather_indx=torch.randint(0, m, (m, ), generator=g, device=device).to(torch.int32),
+                    scatter_indx=torch.randperm(m, generator=g, device=device).to(torch.int32))
+        args["scatter_indx"][::7] = -1
+    md = make_ragged_tensor_metadata(sizes, m)
+    n_out = n // 2 if swiglu else n
+    quantised = mx8 and n_out % 32 == 0
+
+    def run():
+        out = torch.zeros((m, n_out), dtype=torch.bfloat16, device=device)
+        a, pc = x, mm.PrecisionConfig(b_mx_scale=s, out_dtype=torch.bfloat16)
+        if mx8:
+            a, pc.a_mx_scale = downcast_to_mxfp(x, torch.float8_e4m3fn, axis=-1)
+        got = [mm.matmul(a, w, bias, md, precision_config=pc, c=out, **args).clone()]
+        if quantised:
+            pc.c_mx_scale, pc.out_dtype = torch.zeros((m, n_out // 32), dtype=torch.uint8, device=device), torch.float8_e4m3fn
+            epi = mm.Epilogue(mm.FnSpecs(mm.FnName.QUANTIZE_MXFP8.name, quantize_mxfp8_fn, (), ()), tuple(), tuple(), effective_itemsize=1.0)
+            q = torch.zeros((m, n_out), dtype=torch.float8_e4m3fn, device=device)
+            got += [mm.matmul(a, w, bias, md, precision_config=pc, epilogue=epi, c=q, **args).view(torch.uint8).clone(), pc.c_mx_scale]
+        return got
+    by_rule = run()
+    with mm.scoped_opt_flags_constraints({"block_m": 128}):
+        want = run()
+    for a, b in zip(by_rule, want):
+        assert torch.equal(a, b)
+    assert not torch.isnan(by_rule[0]).any() and by_rule[0].any()

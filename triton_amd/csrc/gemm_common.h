@@ -82,7 +82,10 @@ int32_t gemm_launch_mxn(const GemmParams& p, int block_m, int grid_m, bool swigl
 int32_t gemm_launch_mxn_mx(const GemmParams& p, int block_m, int grid_m, bool swiglu, hipStream_t st);  // block_m 128 / 256, MX-quantised output
 int32_t gemm_launch_mxd(const GemmParams& p, int block_m, int grid_m, bool swiglu, hipStream_t st);
 int32_t gemm_launch_mxs(const GemmParams& p, int grid_m, bool swiglu, bool once, hipStream_t st);  // block_m 32; once: about one row block per slice
-int32_t gemm_launch_mxw(const GemmParams& p, bool mx_act, bool swiglu, bool mx_out, hipStream_t st);  // block_m 256
+int32_t gemm_launch_mxw(const GemmParams& p, MxwTile tile, bool swiglu, hipStream_t st);  // tile: mxw_tile, or 160 rows
+int32_t gemm_launch_mxw_low(const GemmParams& p, MxwTile tile, bool swiglu, hipStream_t st);
+int32_t gemm_launch_mxw_mx8(const GemmParams& p, MxwTile tile, bool swiglu, bool mx_out, hipStream_t st);  // the same, MXFP8 activations
+int32_t gemm_launch_mxw_mx8_low(const GemmParams& p, MxwTile tile, bool swiglu, bool mx_out, hipStream_t st);
 int32_t gemm_launch_f8n(const GemmParams& p, int block_m, int grid_m, bool swiglu, hipStream_t st);
 int32_t gemm_launch_mx8n(const GemmParams& p, int block_m, int grid_m, bool swiglu, bool mx_out, hipStream_t st);
 
@@ -541,9 +544,10 @@ inline int busy_cu_count(int idle) {
 // HOIST: all LDS operands (a lane's 16 * NFW bias values, its rows' gate weights and destinations) are read into
 // registers up front, one LDS round trip instead of one per row fragment and column group; for kernels whose registers
 // are free behind the K loop.
+// nj: row fragments that hold rows; the ones behind issue no stores (for kernels whose own waits count the stores).
 template <int G, int MFW, int NFW, int NFV, bool SWIGLU, bool HOIST = false>
 __device__ __forceinline__ void staged_epilogue(const GemmParams& p, f32x16_t (&acc)[NFW][MFW], __amdgpu_buffer_rsrc_t yrsrc, const float* bias_s,
-                                                const float* gam_s, const int* dst_s, int ncol_tile, int ncol0, int grp, int lr, int h) {
+                                                const float* gam_s, const int* dst_s, int ncol_tile, int ncol0, int grp, int lr, int h, int nj = MFW) {
   const int NOUT = SWIGLU ? p.N / 2 : p.N;
   const float nalpha_log2e = -p.alpha * 1.4426950408889634f;
   const float limit = p.has_limit ? p.limit : INFINITY;
@@ -567,6 +571,7 @@ __device__ __forceinline__ void staged_epilogue(const GemmParams& p, f32x16_t (&
   }
 #pragma unroll
   for (int j = 0; j < MFW; ++j) {
+    if (j >= nj) continue;
     const int r = (j * G + grp) * 32 + lr;
     const float g = HOIST ? gh[j] : gam_s[r];
     const int dst = HOIST ? dh[j] : dst_s[r];
@@ -626,7 +631,7 @@ __device__ __forceinline__ void staged_epilogue(const GemmParams& p, f32x16_t (&
 template <int MFW, int NFW, bool SWIGLU>
 __device__ __forceinline__ void staged_mx_epilogue(const GemmParams& p, f32x16_t (&acc)[NFW][MFW], __amdgpu_buffer_rsrc_t yrsrc,
                                                    __amdgpu_buffer_rsrc_t ysrsrc, const float* bias_s, const float* gam_s, const int* dst_s,
-                                                   int ncol_tile, int ncol0, int lr, int h) {
+                                                   int ncol_tile, int ncol0, int lr, int h, int nj = MFW) {
   const int NOUT = SWIGLU ? p.N / 2 : p.N;
   const float nalpha_log2e = -p.alpha * 1.4426950408889634f;
   const float limit = p.has_limit ? p.limit : INFINITY;
@@ -650,6 +655,7 @@ __device__ __forceinline__ void staged_mx_epilogue(const GemmParams& p, f32x16_t
   }
 #pragma unroll
   for (int j = 0; j < MFW; ++j) {
+    if (j >= nj) continue;
     const float g = gh[j];
     const int dst = dh[j];
     float o[NFW][2][VO];

@@ -49,6 +49,45 @@ inline bool reads_once(int64_t rows, int64_t n_slices, int64_t block_rows, int64
   return rows * 16 <= n_slices * block_rows * 13 && read * N * row_bytes > 128 << 20;
 }
 
+// Tile of the wide MXFP4 kernel (moe_gemm_mxw_kernel.h) for a call whose rows are more than the decode kernel is made for; rows 0 = the kernels before it.
+// Figures: us, both GEMMs of a layer; "before" = the streaming kernel's 32-row blocks, or 64 and 128 rows of the ones with weights in registers.
+// bf16 rows.  32 x 256 (two workgroups a CU) is the shortest chain where it is one round; otherwise up to 20 rows the streaming kernel, which waits for no
+// other wave (real layers, 128 slices, K 2880: 3 rows 274 against 284, 9 rows 323 against 355).  64 x 256, two workgroups a CU as well, divides a small
+// product evenly; where the tiles of 512 columns are two rounds and more, those: half the reads of the rows, and three stages of weights in flight.
+//   128 slices, K 2880, N 5760 and 2880: 28 rows before 415, 370 (64 x 512), 42 471, 416, 56 525, 475 (96; 64 x 512 498), 72 607, 544 (96; 160 563,
+//   64 x 256 743), 84 646, 602 (160; 96 613)
+//   128 slices, K 2048, N 4096: 28 rows 131, 117 (64 x 512; 64 x 256 123), 69 203, 177 (96), 109 271, 236 (160; 64 x 256 268)
+//   96 slices, K 1088 and 1024, N 2048 and 1088: 39 rows 76, 60 (64 x 256; 64 x 512 72), 62 91, 74 (96 89, 160 98), 94 105, 90
+//   64 slices, K 1344 and 992, N 1984 and 1344: 44 rows 68, 54, 62 80, 66, 94 93, 76 (160: 78)
+//   32 slices, K 1536 and 640, N 1280 and 1536: 16 rows 32, 25 (32; 64 x 256 28), 64 46, 32 (32 or 64 x 256), 82 51, 37
+//   32 slices, K 1024, N 4096: 62 rows 32, 29 (64 x 256), 500 163, 134 (160; 64 x 256 145); 16 slices, K 1024, N 2048: 50 rows 18.6, 13.1 (32; 64 x
+//   256 15.1), 375 45, 34 (64 x 256)
+//   (against: 32 slices, K 2400, N 1920, 256 tiles of the kernel before, one for each CU: 12 rows 19.1, 21, 31 22.3, 24.9)
+// MXFP8 rows, whose stage is half as long to multiply: the kernel before (128 x 256 tiles, weights in registers) stays where its tiles are one round (32
+// slices, K 2400, N 1920: 18 rows 21 against 24, 50 22 against 30).  Beyond that tiles as high as a routing with favourites needs as well, since the epilogue
+// costs by rows: 128 x 512 from 24 rows; 64 x 512 below, and longer where the tiles of 512 columns are less than three a CU, where 32 x 256 divides better below.
+// (slices all alike; by favourites, the last one's expectation five times the first's):
+//   128 slices, K 2880, N 5760 and 2880: 4 rows 348, 287 (64); 139, 135.  14 354, 305 (64); 209, 204.  28 378, 341 (128; 64 334); 262, 276 (64 289).
+//   43 401, 369 (128); 322, 313 (64 357).  72 452, 418 (160 435); 427, 413.  94 485, 458 (160 467); 500, 486.  128 658, 656 (160 531); 603, 580
+//   96 slices, K 1696 and 1088, N 2176 and 1696: 11 rows 92, 72 (32; 64 76); 65, 54 (64).  36 98, 86 (64; 128 90, 32 107); 88, 84 (128 96).  58 108,
+//   97 (128); 106, 99.  83 121, 110; 122, 129.  125 154, 138 (160; 128 147); 153, 161 (128 144)
+struct MxwTile {
+  int32_t rows, cols;
+};
+inline MxwTile mxw_tile(int64_t rows, int64_t n_slices, int64_t N, bool mx8) {
+  const int64_t n256 = (N + 255) / 256, n512 = (N + 511) / 512;
+  if (mx8) {
+    if ((rows <= 96 * n_slices ? 256 * n_slices : 2 * rows + 128 * n_slices) * n256 <= 256 * 256) return {0, 0};  // (256ths of its row blocks)
+    const bool few = n_slices * n512 < 3 * 256;
+    if (few && rows <= 24 * n_slices) return {32, 256};
+    return rows <= (few ? 40 : 24) * n_slices ? MxwTile{64, 512} : rows <= 104 * n_slices ? MxwTile{128, 512} : MxwTile{0, 0};
+  }
+  if ((rows + 16 * n_slices) * n256 <= 512 * 32) return {32, 256};
+  if (rows <= 20 * n_slices) return {0, 0};
+  if ((rows + 160 * n_slices - 1) / (160 * n_slices) * n_slices * n512 < 512) return {64, 256};
+  return rows <= 48 * n_slices ? MxwTile{64, 512} : rows <= 80 * n_slices ? MxwTile{96, 512} : MxwTile{160, 512};
+}
+
 // Row blocks (of 64) that the kernel for few rows launches side by side: one a slice at least, and what slices of up to five quarters of
 // the mean make, as a random routing does (at 62 rows per slice half of the slices have a second block).
 inline int64_t few_row_blocks(int64_t rows, int64_t n_slices) { return n_slices * (rows * 5 / (n_slices * 256) + 1); }

@@ -219,6 +219,12 @@ int64_t wide_block_m(int64_t rows, int64_t n_slices, int64_t K, uint32_t x_bytes
   return !mx8 || rows <= 176 * n_slices || rows >= 640 * n_slices ? 256 : 128;
 }
 
+// Columns of the wide kernel's tiles that gemm_limits.h names for such weights, 0 = the kernel of the row block.
+int64_t wide_block_n(int64_t rows, int64_t n_slices, int64_t K, int64_t N, uint32_t x_bytes, bool mx8) {
+  n_slices = std::max<int64_t>(n_slices, 1);
+  return K <= (mx8 ? 511 : 384) || n_slices > tk::kDmaSlices || !x_bytes ? 0 : tk::mxw_tile(rows, n_slices, N, mx8).cols;
+}
+
 // Columns a workgroup of the kernel for few rows, 0 = the kernels above: up to 64 rows per slice and one workgroup per CU at most, with 32
 // columns while they fit, then 64.  Measured (us, this kernel against the one that ran before; other weights each call): 8 slices of 32
 // rows, N 2048: K 512 9.1 against 12.1, K 2048 20 against 28, K 8192 60 against 76; N 512: K 1024 7.6 against 15.4, K 8192 26 against 72; 64 rows, N
@@ -437,8 +443,12 @@ PyObject* run_gemm(PyObject* const* v) {
     if (tk::dma_runs_e4m3(x_bytes, n_slices, K, N)) block_n = dma_block_n(M, N, n_slices, block_m);
   } else if (mx_act) {
     block_m = wide_block_m(M, n_slices, K, x_bytes, true);
+    block_n = wide_block_n(M, n_slices, K, N, x_bytes, true);
   } else if (tiled) {
-    if (M > 256 && x_bytes && n_slices <= tk::kDmaSlices && !x_row && !w_col) block_m = mxfp4_block_m(M, n_slices, block_m);
+    if (M > 256 && x_bytes && n_slices <= tk::kDmaSlices && !x_row && !w_col) {
+      block_m = mxfp4_block_m(M, n_slices, block_m);
+      if (n_out % 8 == 0) block_n = wide_block_n(M, n_slices, K, N, x_bytes, false);
+    }
     if (block_m == 128) block_m = wide_block_m(M, n_slices, K, x_bytes, false);
   } else if (tk::dma_runs_16bit(x_bytes, n_slices, K, N, w->stride(2))) {
     if (idle <= 0) block_n = few_block_n(M, N, n_slices);
@@ -485,13 +495,14 @@ PyObject* run_gemm(PyObject* const* v) {
     return static_cast<int32_t*>(THPVariable_Unpack(t.p).data_ptr());  // (kept for the life of the process)
   };
   if ((tiled || tiled_fp8) && block_m >= 64 && !mx_act) d.tile_counters = words(B.tile_counters, true);
-  // the combine inside the launch: with the decode kernel by the wave that completes a token's rows, with the prefill kernel by
-  // the persistent grid at its end; the streaming (block_m 32) and the wide kernel (256) have none
-  if (combine_k > 0 && tiled && !mx_act && !act.swiglu && scatter && y_rows % combine_k == 0
-      && (block_m == 16 ? (y_rows / combine_k) * ((N + 31) / 32) <= (1 << 16) : block_m >= 64 && block_m != 256 && N % 8 == 0)) {
+  // the combine inside the launch, by the wave that completes a token's rows: the decode kernel only.  (The prefill kernel for row blocks of 64 and 128
+  // can sum at the end of its persistent grid, which costs more than a launch: 96 slices of 39 rows, N 1088 79 us against 33 and 5, 32 slices of 64
+  // rows, N 1536 56 against 21 and 4, 128 slices of 29 rows, N 2880 167 against 140 and 10.)
+  if (combine_k > 0 && tiled && !mx_act && !act.swiglu && scatter && y_rows % combine_k == 0 && block_m == 16
+      && (y_rows / combine_k) * ((N + 31) / 32) <= (1 << 16)) {
     combined = empty({y_rows / combine_k, N}, out, *a);
     d.combine_k = int32_t(combine_k), d.combine_out = combined.data_ptr(), d.combine_stride_m = N;
-    if (block_m == 16) d.combine_counters = words(B.combine_counters, false);
+    d.combine_counters = words(B.combine_counters, false);
   }
   launch([&] { return B.moe_gemm(&d, *stream); });
   // or by a launch of its own, from here
@@ -840,6 +851,10 @@ PyObject* rule_mxfp4(PyObject* const* v) {
   const auto [rows, n_slices, otherwise] = integers<3>(v);
   return PyLong_FromLongLong(mxfp4_block_m(rows, n_slices, otherwise));
 }
+PyObject* rule_wide_n(PyObject* const* v) {
+  const auto [rows, n_slices, K, N, x_bytes, mx8] = integers<6>(v);
+  return PyLong_FromLongLong(wide_block_n(rows, n_slices, K, N, uint32_t(x_bytes), mx8 != 0));
+}
 PyObject* rule_wide(PyObject* const* v) {
   const auto [rows, n_slices, K, x_bytes, mx8] = integers<5>(v);
   return PyLong_FromLongLong(wide_block_m(rows, n_slices, K, uint32_t(x_bytes), mx8 != 0));
@@ -902,6 +917,7 @@ PyMethodDef methods[] = {
     METHOD("fp8_block_m", rule_fp8, 5),
     METHOD("mxfp4_block_m", rule_mxfp4, 3),
     METHOD("wide_block_m", rule_wide, 5),
+    METHOD("wide_block_n", rule_wide_n, 6),
     {nullptr, nullptr, 0, nullptr},
 };
 

@@ -29,9 +29,15 @@ static int32_t launch_16bit(const GemmParams& p, const tk_gemm_desc* d, int wk, 
   return gemm_launch_strided(p, wk, d->block_m, d->grid_m, swiglu, st);
 }
 
-// what the wide MXFP4 kernel needs beyond its neighbours' conditions: x within a buffer resource, the slice list in registers, four stages of K
-static bool wide_ok(const GemmParams& p, const tk_gemm_desc* d) {
-  return d->block_m == 256 && p.x_bytes && slices(d) <= kDmaSlices && p.w_nst >= 4;
+// The wide MXFP4 kernel's tile for this call, rows 0 = it runs on another kernel: asked for by block_n (256, 512), or row blocks of 256; it needs x within
+// a buffer resource, the slice list in registers, four stages of K.
+static MxwTile wide_tile(const GemmParams& p, const tk_gemm_desc* d, bool mx8) {
+  if (!p.x_bytes || slices(d) > kDmaSlices || p.w_nst < 4) return {0, 0};
+  if (d->block_n == 256 || d->block_n == 512) {
+    const MxwTile tile = mxw_tile(d->M, slices(d), d->N, mx8);
+    if (tile.rows && tile.cols == d->block_n) return tile;
+  }
+  return d->block_m == 256 ? MxwTile{160, 512} : MxwTile{0, 0};
 }
 
 extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
@@ -190,7 +196,7 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
         fast = fast && p.y_vec && d->y_stride_m >= cdiv(n_out, piece) * piece;
       p.y_bytes = fast ? (uint32_t)y_bytes : 0u;
     }
-    if (p.y_bytes != 0 && wide_ok(p, d)) return gemm_launch_mxw(p, true, swiglu, mx_out, st);
+    if (const MxwTile tile = p.y_bytes != 0 ? wide_tile(p, d, true) : MxwTile{0, 0}; tile.rows) return gemm_launch_mxw_mx8(p, tile, swiglu, mx_out, st);
     return gemm_launch_mx8n(p, d->block_m, d->grid_m, swiglu, mx_out, st);
   }
   if (d->w_layout == TK_W_TILED) {
@@ -237,13 +243,20 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
     if (d->n_slices > 1 && (d->w_stride_e < nfr * nst * 2048 || d->ws_stride_e < nfr * nst * 128)) return fail(TK_ERR_INVALID, "tk_moe_gemm: expert stride smaller than one tiled expert");
     p.w_stride_e = d->w_stride_e;
     p.w_nst = (int32_t)nst;
+    if (d->combine_k <= 0 && !mx_out_bf16 && !extras && !d->x_row_scale && !d->w_col_scale) {
+      const MxwTile tile = wide_tile(p, d, false);
+      const int64_t n_out = swiglu ? d->N / 2 : d->N, piece = swiglu ? 4 : 8, y_bytes = (int64_t)(d->scatter_indx ? d->scatter_len : d->M) * d->y_stride_m * 2;
+      if (tile.rows && p.y_vec && d->y_stride_m >= cdiv(n_out, piece) * piece && y_bytes < (int64_t)1 << 31) {  // (as above, where row blocks are below 64)
+        p.y_bytes = (uint32_t)y_bytes;
+        return gemm_launch_mxw(p, tile, swiglu, st);
+      }
+    }
     // row blocks of 32: the streaming kernel, unless something asks for the decode kernel's epilogue or fused combine (or x is too large
     // for a buffer resource, or there are more slices than it has registers for)
     if (d->block_m == 32 && p.x_bytes && slices(d) <= kDmaSlices && !extras && d->combine_k <= 0 && !d->x_row_scale && !d->w_col_scale)
       return gemm_launch_mxs(p, d->grid_m, swiglu, (int64_t)d->M <= (int64_t)d->n_slices * 16, st);
     if (d->block_m <= 32) return gemm_launch_mxd(p, d->block_m, d->grid_m, swiglu, st);
     if (mx_out_bf16) return gemm_launch_mxn_mx(p, d->block_m, d->grid_m, swiglu, st);
-    if (d->combine_k <= 0 && wide_ok(p, d)) return gemm_launch_mxw(p, false, swiglu, false, st);
     return gemm_launch_mxn(p, d->block_m, d->grid_m, swiglu, st);
   }
   if (d->w_layout != TK_W_STRIDED) return fail(TK_ERR_INVALID, "tk_moe_gemm: bad w_layout %d", d->w_layout);

@@ -1,32 +1,37 @@
-// Expert GEMM on tiled MXFP4 weights for about 80 rows per expert and more, bf16 or MXFP8 activations: tiles of 160 rows x 512 columns
-// with both operands staged by memory-to-LDS transfers.
+// Expert GEMM on tiled MXFP4 weights for more than a few rows per expert, bf16 or MXFP8 activations: tiles of 32 to 160 rows x 256 or 512
+// columns with both operands staged by memory-to-LDS transfers.  Which tile a call gets, and why there: mxw_tile (gemm_limits.h).
 //
-//   * Eight waves, each all rows x 64 columns, two to a SIMD: 160 accumulators of its 256 registers.  A stage (128 k) moves 40 or 20 KiB of rows
-//     and 34 KiB of weights per 5120 / 2560 matrix cycles; with tiles of 256 columns the rows cross from L2 twice as often.  160 rows: an
-//     expert with 128 +- 11 rows is one tile, so its weights are read once.
+//   * Four or eight waves, each all rows x 64 columns, two to a SIMD (four waves: two workgroups a CU).  Tiles of 512 columns halve what the rows cross from
+//     L2.  160 rows (160 accumulators of a wave's 256 registers; a stage of 128 k moves 40 or 20 KiB of rows and 34 KiB of weights per 5120 / 2560
+//     matrix cycles): an expert with 128 +- 11 rows is one tile, so its weights are read once.  The smaller ones bring fewer rows that are not there, and
+//     their LDS holds three stages of both: what few rows per expert wait for is the weights.
 //   * Everything comes by `buffer_load ... lds`: no registers wait for memory, rows past the slice, columns past N and k past K are a matter of
-//     the lanes' offsets (past the resource's range the hardware writes zeros).  Rings of two stages of rows and two (bf16) or three
-//     (MXFP8, whose stage is half as long) of weights run on across the tiles of a persistent workgroup.
+//     the lanes' offsets (past the resource's range the hardware writes zeros).  Rings of two or three stages of rows and of weights run on
+//     across the tiles of a persistent workgroup.
 //   * bf16: e2m1 -> bf16 in registers in front of v_mfma_f32_32x32x16_bf16.  MXFP8: both operands as stored to
 //     v_mfma_scale_f32_32x32x64_f8f6f4; a row's activation scales arrive sixteen blocks at a time and wait in LDS for four stages.
-//   * What the next tile needs before its transfers (source rows) and in its epilogue (bias, gate weights, destinations) is requested three
-//     stages before this one's end, parked in LDS two before, used from the last on.  The epilogue has no branch around a store, so the
-//     wait in front of the next tile's first stage counts them and does not wait for them.
+//   * What the next tile needs before its transfers (source rows) and in its epilogue (bias, gate weights, destinations) is requested one stage before
+//     the rows' ring needs it parked in LDS, and used a stage after that.  The epilogue's stores depend on nothing but the row fragments that hold
+//     rows, so the wait in front of the next tile's first stage counts them and does not wait for them.
 //
-// What bounds it: the board's power in bf16 (fetching zeros instead of the weights, the operands then all zero, 558 -> 417 us; matrix pipe 68 %
-// busy at 1.9 GHz), in MXFP8 also LDS reads and the epilogue (without its arithmetic and stores 363 -> 316 us; 42 % busy at 2.3 GHz,
+// What bounds the 160-row tile: the board's power in bf16 (fetching zeros instead of the weights, the operands then all zero, 558 -> 417 us; matrix pipe
+// 68 % busy at 1.9 GHz), in MXFP8 also LDS reads and the epilogue (without its arithmetic and stores 363 -> 316 us; 42 % busy at 2.3 GHz,
 // ten vector instructions per MFMA with the quantised output, seven with bf16).  128 experts, K 2880, 4096 tokens, top-4, whole layer:
 // bf16 861 -> 815 us, MXFP8 609 -> 563 us against the kernels that keep weights in registers with one wave per SIMD (moe_gemm_mxn, _mx8n, which
-// serve what this one does not take).  Measured and left out: transfers spread over the whole bf16 stage (576 against 558
-// us: the last ones are late); weights brought into L2 a stage ahead of their transfer (570 against 558, MXFP8 387 against 363 us).
+// serve what this one does not take).  The smaller ones: reading the weights (128 experts, 14 MXFP8 rows each, both GEMMs 305 us for 1.63 GB).  Measured
+// and left out: transfers spread over the whole bf16 stage (576 against 558 us: the last ones are late); weights brought into L2 a stage ahead
+// of their transfer (570 against 558, MXFP8 387 against 363 us); rings of four and six stages with 32 and 64 rows (no change); all four row fragments'
+// epilogue whether they hold rows or not (128 x 512, 28 MXFP8 rows, both GEMMs 377 against 341 us).
+#pragma once
 #include "gemm_tiles.h"
 
 namespace tk {
 namespace {
 
-template <bool MX8>
+// MFW_ row fragments, NW_ waves (each all rows x 64 columns), rings of ABUFS_ stages of rows and WBUFS_ of weights
+template <bool MX8, int MFW_, int NW_, int ABUFS_, int WBUFS_>
 struct MxwCfg {
-  static constexpr int MFW = 5, NW = 8;                       // row fragments, waves (each all rows x 64 columns)
+  static constexpr int MFW = MFW_, NW = NW_;
   static constexpr int BM = MFW * 32, BN = NW * 64;
   static constexpr int ROW = MX8 ? 128 : 256;            // bytes of a row and stage (128 k)
   static constexpr int RPT = 1024 / ROW;                 // rows of a transfer
@@ -35,18 +40,19 @@ struct MxwCfg {
   static_assert(!HALF || (BM / RPT) * 2 == (2 * AI - 1) * NW, "every wave has the same number of transfers");
   static constexpr int AWAVE = AI * 1024 - (HALF ? 512 : 0), ABYTES = AWAVE * NW;
   static constexpr int WWAVE = 4096 + 256, WBYTES = WWAVE * NW;  // a wave's two weight fragments: values, scales
-  static constexpr int ABUFS = 2, WBUFS = MX8 ? 3 : 2;
+  static constexpr int ABUFS = ABUFS_, WBUFS = WBUFS_;
   static constexpr int RINGS = ABUFS * ABYTES + WBUFS * WBYTES;
   static constexpr int SIDE = MX8 ? BM * 16 : 0;         // a row's activation scales of four stages
   static constexpr int OPERANDS = (BN + 2 * BM) * 4;     // a tile's bias, gate weights, destination rows
-  static constexpr int LISTS = 2 * kDmaSlices * 4;       // slice sizes and offsets
+  static constexpr bool LISTED = MFW == 5;               // the slice sizes and offsets wait in LDS: no registers are left for them
+  static constexpr int LISTS = LISTED ? 2 * kDmaSlices * 4 : 0;
   static constexpr int LDS = RINGS + 2 * (SIDE + OPERANDS) + LISTS;
 };
 
 // ONCE: the weights are fetched with the non-temporal hint (reads_once)
-template <bool MX8, bool SWIGLU, bool MXOUT, bool ONCE>
-__global__ __launch_bounds__(MxwCfg<MX8>::NW * 64, 2) void moe_gemm_mxw_kernel(const GemmParams p) {
-  typedef MxwCfg<MX8> C;
+template <bool MX8, int MFW_, int NW_, int ABUFS_, int WBUFS_, bool SWIGLU, bool MXOUT, bool ONCE>
+__global__ __launch_bounds__(NW_ * 64, 2) void moe_gemm_mxw_kernel(const GemmParams p) {
+  typedef MxwCfg<MX8, MFW_, NW_, ABUFS_, WBUFS_> C;
   constexpr int MFW = C::MFW, AI = C::AI;
   extern __shared__ __attribute__((aligned(1024))) uint8_t lds[];
   const int tid = threadIdx.x, lane = tid & 63;
@@ -58,21 +64,20 @@ __global__ __launch_bounds__(MxwCfg<MX8>::NW * 64, 2) void moe_gemm_mxw_kernel(c
   uint8_t* const side = lds + C::RINGS;
   float* const operands = reinterpret_cast<float*>(lds + C::RINGS + 2 * C::SIDE);
 
-  // the tile list's slice sizes and offsets wait in LDS between two tiles (every wave stores the same words)
+  // the tile list; its slice sizes and offsets in LDS between two tiles where they are LISTED (every wave stores the same words)
   int* const lists = reinterpret_cast<int*>(lds + C::RINGS + 2 * (C::SIDE + C::OPERANDS));
   typedef TileList<C::BM, C::BN> Tiles;
-  int tile, t_step, t_end, f_beg, f_len, s_beg;
-  Tile cur, nxt;
-  {
-    Tiles t;
-    tile = t.init(p, lane);
-    t_step = t.t_step, t_end = t.t_end, f_beg = t.f_beg, f_len = t.f_len, s_beg = t.s_beg;
-    if (tile >= t_end) return;
-    cur = nxt = t.locate(tile);
+  Tiles list;
+  int tile = list.init(p, lane);
+  const int t_step = list.t_step, t_end = list.t_end, f_beg = list.f_beg, f_len = list.f_len, s_beg = list.s_beg;
+  if (tile >= t_end) return;
+  Tile cur = list.locate(tile), nxt = cur;
+  if constexpr (C::LISTED) {
 #pragma unroll
-    for (int c = 0; c < kSliceRegs; ++c) lists[c * 64 + lane] = t.sz[c], lists[kDmaSlices + c * 64 + lane] = t.so[c];
+    for (int c = 0; c < kSliceRegs; ++c) lists[c * 64 + lane] = list.sz[c], lists[kDmaSlices + c * 64 + lane] = list.so[c];
   }
   auto locate = [&](int i) __attribute__((always_inline)) -> Tile {
+    if constexpr (!C::LISTED) return list.locate(i);
     Tiles t;
 #pragma unroll
     for (int c = 0; c < kSliceRegs; ++c) t.sz[c] = lists[c * 64 + lane], t.so[c] = lists[kDmaSlices + c * 64 + lane];
@@ -205,18 +210,22 @@ __global__ __launch_bounds__(MxwCfg<MX8>::NW * 64, 2) void moe_gemm_mxw_kernel(c
   scales_park(0, 0);
   // the rings: activations one stage ahead, weights, which come from further away, WBUFS - 1
   constexpr uint32_t kW0 = C::ABUFS * C::ABYTES, kWEnd = C::RINGS;
-  constexpr int WA = C::WBUFS - 1;
+  constexpr int AA = C::ABUFS - 1, WA = C::WBUFS - 1;
   uint32_t ab = 0, wb = kW0, wf_buf = kW0 + WA * C::WBYTES;  // buffers being read; the next one of the weights to fill
   aim_w(cur);
 #pragma unroll
   for (int i = 0; i < 5; ++i) fetch_w(i, 0, kW0, true);
 #pragma unroll
   for (int i = 0; i < AI; ++i) fetch_a(i, 0, 0, KB);
-  if constexpr (WA == 2) {
 #pragma unroll
-    for (int i = 0; i < 5; ++i) fetch_w(i, 1, kW0 + C::WBYTES, true);
+  for (int n = 1; n < (AA > WA ? AA : WA); ++n) {
+#pragma unroll
+    for (int i = 0; i < AI && n < AA; ++i) fetch_a(i, n, n * C::ABYTES, KB);
+#pragma unroll
+    for (int i = 0; i < 5 && n < WA; ++i) fetch_w(i, n, kW0 + n * C::WBYTES, true);
   }
-  bool more = true, stored = false;
+  bool more = true;
+  int stored = 0;  // row fragments that the last epilogue has stored
 
   f32x16_t acc[2][MFW];
   // NJ = row fragments that hold rows (0: this wave has no columns)
@@ -225,30 +234,37 @@ __global__ __launch_bounds__(MxwCfg<MX8>::NW * 64, 2) void moe_gemm_mxw_kernel(c
     for (int s = 0; s < nst; ++s) {
       // stage s has landed when only what was fetched behind it, the next stage's weights, is outstanding (and, in a tile's first stage, the
       // stores of the last epilogue); the buffers of stage s - 1 have been read
-      constexpr int kBehind = (WA - 1) * 5, kStores = MXOUT ? MFW * (SWIGLU ? 5 : 6) : MFW * 4;
-      if (s == 0 && stored)
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kBehind + kStores) : "memory");
-      else
+      constexpr int kBehind = AA == WA ? (AA - 1) * (AI + 5) : (WA - 1) * 5, kStores = MXOUT ? (SWIGLU ? 5 : 6) : 4;  // (stores of a fragment)
+      static_assert(kBehind + MFW * kStores < 64, "what a wait can count");
+      if (s == 0) {
+        static_for<0, MFW + 1>([&](auto n_c) __attribute__((always_inline)) {
+          if (stored == decltype(n_c)::value) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kBehind + decltype(n_c)::value * kStores) : "memory");
+        });
+      } else {
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kBehind) : "memory");
+      }
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      int fs = s + 1, ws = s + WA;  // stages to fetch
+      int fs = s + AA, ws = s + WA;  // stages to fetch
       // the next tile, a step a stage: its words requested, then parked, then its transfers begin
-      if (s == nst - 3) {
+      if (s == nst - AA - 2) {
         more = tile + t_step < t_end;
         if (more) nxt = locate(tile + t_step);
         request(nxt);
-      } else if (s == nst - 2) {
+      } else if (s == nst - AA - 1) {
         arrived();
         park(nxt, set ^ 1);
-        if constexpr (MX8) xs_row = (uint32_t)raw_xs * (uint32_t)p.xs_stride_m;
-        scales_request(0);
-        if (WA == 2) aim_w(nxt);
-      } else if (s == nst - 1) {
+      } else if (s == nst - AA) {
         aim(nxt);
-        if (WA == 1) aim_w(nxt);
-        fs = 0;
-        scales_park(0, xset ^ 1);
+      }
+      if (s == nst - WA) aim_w(nxt);
+      if constexpr (MX8) {
+        if (s == nst - 2) {
+          xs_row = (uint32_t)raw_xs * (uint32_t)p.xs_stride_m;
+          scales_request(0);
+        } else if (s == nst - 1) {
+          scales_park(0, xset ^ 1);
+        }
       }
       if constexpr (MX8) {
         if ((s & 3) == 1 && (s >> 2) + 1 <= ((nst - 1) >> 2)) scales_request((s >> 2) + 1);
@@ -256,8 +272,10 @@ __global__ __launch_bounds__(MxwCfg<MX8>::NW * 64, 2) void moe_gemm_mxw_kernel(c
       }
       const bool w_on = more || ws < nst;
       ws = ws < nst ? ws : ws - nst;
-      const int k_end = more || fs != 0 ? KB : 0;
-      const uint32_t af_buf = ab ^ C::ABYTES;
+      const int k_end = more || fs < nst ? KB : 0;
+      fs = fs < nst ? fs : fs - nst;
+      // (of the ring's buffers the one before the one being read)
+      const uint32_t af_buf = AA == 1 ? ab ^ C::ABYTES : ab == 0 ? AA * C::ABYTES : ab - C::ABYTES;
       const uint8_t* a = lds + ab;
       const uint8_t* w = lds + wb + wave * C::WWAVE;
       auto fetch = [&](int i) __attribute__((always_inline)) {
@@ -339,7 +357,7 @@ __global__ __launch_bounds__(MxwCfg<MX8>::NW * 64, 2) void moe_gemm_mxw_kernel(c
 #pragma unroll
           for (int j = 0; j < MFW; ++j) asm volatile("" : "+v"(acc[f][j]));
       }
-      ab ^= C::ABYTES;
+      ab = AA == 1 ? ab ^ C::ABYTES : ab + C::ABYTES == kW0 ? 0 : ab + C::ABYTES;
       wb = wb + C::WBYTES == kWEnd ? kW0 : wb + C::WBYTES;
       wf_buf = wf_buf + C::WBYTES == kWEnd ? kW0 : wf_buf + C::WBYTES;
       if constexpr (MX8) xset ^= (s & 3) == 3 || s == nst - 1;
@@ -361,27 +379,29 @@ __global__ __launch_bounds__(MxwCfg<MX8>::NW * 64, 2) void moe_gemm_mxw_kernel(c
     });
     const float* o = operands + set * (C::OPERANDS / 4);
     if constexpr (MXOUT)
-      staged_mx_epilogue<MFW, 2, SWIGLU>(p, acc, yrsrc, ysrsrc, o, o + C::BN, reinterpret_cast<const int*>(o) + C::BN + C::BM, wave * 64, ncol0, lr, h);
+      staged_mx_epilogue<MFW, 2, SWIGLU>(p, acc, yrsrc, ysrsrc, o, o + C::BN, reinterpret_cast<const int*>(o) + C::BN + C::BM, wave * 64, ncol0, lr, h, nj);
     else
-      staged_epilogue<1, MFW, 2, 2, SWIGLU>(p, acc, yrsrc, o, o + C::BN, reinterpret_cast<const int*>(o) + C::BN + C::BM, wave * 64, ncol0, 0, lr, h);
+      staged_epilogue<1, MFW, 2, 2, SWIGLU>(p, acc, yrsrc, o, o + C::BN, reinterpret_cast<const int*>(o) + C::BN + C::BM, wave * 64, ncol0, 0, lr, h, nj);
     if (!more) break;
     tile += t_step;
     cur = nxt;
     set ^= 1;
-    stored = true;
+    stored = nj;
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no transfer into this workgroup's LDS is left behind
 }
 
-template <bool MX8>
-int32_t launch_cfg(const GemmParams& p, bool swiglu, bool mx_out, hipStream_t st) {
-  typedef MxwCfg<MX8> C;
-  static_assert(C::LDS <= 160 * 1024, "one workgroup per CU");
+template <bool MX8, int MFW, int NW, int ABUFS, int WBUFS>
+int32_t launch_mxw(const GemmParams& p, bool swiglu, bool mx_out, hipStream_t st) {
+  typedef MxwCfg<MX8, MFW, NW, ABUFS, WBUFS> C;
+  constexpr int kPerCu = C::LDS <= 80 * 1024 && NW == 4 ? 2 : 1;  // workgroups of a CU
+  static_assert(C::LDS * kPerCu <= 160 * 1024 && (NW == 8 || kPerCu == 2), "workgroups of a CU");
+  static_assert(ABUFS + 1 <= 4, "a tile's events, the first of which comes ABUFS + 1 stages before its end, within the fewest stages of K that the kernel takes");
   GemmParams q = p;
   q.grid_n = (int)cdiv(p.N, C::BN);
   const int64_t tiles = (cdiv(p.M, C::BM) + (p.slice_sizes ? p.n_slices : 0)) * q.grid_n;  // at most
   if (tiles > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: grid too large");
-  int64_t grid = (int64_t)busy_cu_count(p.idle_cus) / 8 * 8;  // every XCD walks its share of the tiles
+  int64_t grid = (int64_t)busy_cu_count(p.idle_cus) * kPerCu / 8 * 8;  // every XCD walks its share of the tiles
   grid = grid < 8 ? 8 : grid;
   grid = grid < cdiv(tiles, 8) * 8 ? grid : cdiv(tiles, 8) * 8;
   auto launch = [&](auto kern) -> int32_t {
@@ -392,17 +412,12 @@ int32_t launch_cfg(const GemmParams& p, bool swiglu, bool mx_out, hipStream_t st
   auto with = [&](auto once) -> int32_t {
     constexpr bool ONCE = decltype(once)::value;
     if constexpr (MX8) {
-      if (mx_out) return swiglu ? launch(moe_gemm_mxw_kernel<true, true, true, ONCE>) : launch(moe_gemm_mxw_kernel<true, false, true, ONCE>);
+      if (mx_out) return swiglu ? launch(moe_gemm_mxw_kernel<true, MFW, NW, ABUFS, WBUFS, true, true, ONCE>) : launch(moe_gemm_mxw_kernel<true, MFW, NW, ABUFS, WBUFS, false, true, ONCE>);
     }
-    return swiglu ? launch(moe_gemm_mxw_kernel<MX8, true, false, ONCE>) : launch(moe_gemm_mxw_kernel<MX8, false, false, ONCE>);
+    return swiglu ? launch(moe_gemm_mxw_kernel<MX8, MFW, NW, ABUFS, WBUFS, true, false, ONCE>) : launch(moe_gemm_mxw_kernel<MX8, MFW, NW, ABUFS, WBUFS, false, false, ONCE>);
   };
   return reads_once(p.M, p.slice_sizes ? p.n_slices : 1, C::BM, p.N, p.K / 2) ? with(std::true_type{}) : with(std::false_type{});
 }
 
 }  // namespace
-
-int32_t gemm_launch_mxw(const GemmParams& p, bool mx_act, bool swiglu, bool mx_out, hipStream_t st) {
-  return mx_act ? launch_cfg<true>(p, swiglu, mx_out, st) : launch_cfg<false>(p, swiglu, false, st);
-}
-
 }  // namespace tk

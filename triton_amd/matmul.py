@@ -761,6 +761,8 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
         # the tile shapes that take MXFP8 activations / have an MX-output epilogue
         if forced is None and is_ragged:
             block_m = nt.rules().wide_block_m(M, n_slices, K, x_bytes, 1) if mx_act else 256 if M <= 144 * n_slices else 128
+            if mx_act and not extras:
+                d.block_n = nt.rules().wide_block_n(M, n_slices, K, N, x_bytes, 1)
         else:
             block_m = 256 if forced == 256 else 128
     elif tiled:
@@ -770,6 +772,8 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
             if (M > 256 and x_bytes and n_slices <= 256 and a_ts is None and b_ts is None
                     and a_ragged_metadata.expected_slice_size is None):
                 block_m = nt.rules().mxfp4_block_m(M, n_slices, block_m)
+                if out_shape[1] % 8 == 0:
+                    d.block_n = nt.rules().wide_block_n(M, n_slices, K, N, x_bytes, 0)
             if block_m == 128:
                 block_m = nt.rules().wide_block_m(M, n_slices, K, x_bytes, 0)
     elif w_dtype in (_BF16, _F16):
@@ -831,8 +835,8 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
     # launch of its own at the gpt-oss shape)
     can_combine = (_combine_k and tiled and not extras and not mx_act and act == nt.TK_ACT_NONE and scatter_indx is not None
                    and y_rows % _combine_k == 0 and a_dtype == _BF16)
-    if can_combine and block_m in (32, 256) and forced is None:
-        can_combine = False  # the streaming and the wide kernel have no combine
+    if can_combine and block_m != 16 and forced is None:
+        can_combine = False  # (the streaming and the wide kernel have none, and the one behind the prefill kernel's tiles costs more than a launch)
     elif can_combine and block_m <= 32:
         # decode kernel: the wave that completes a token's rows last sums them (arrival counters per token and fragment)
         can_combine = (y_rows // _combine_k) * ((N + 31) // 32) <= _COMBINE_COUNTER_WORDS
