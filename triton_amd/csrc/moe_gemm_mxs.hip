@@ -75,12 +75,8 @@ __global__ __launch_bounds__(MxsCfg::NW * 64, 2) void moe_gemm_mxs_kernel(const 
   };
   auto fetch = [&](int s, uint32_t buf, bool more) __attribute__((always_inline)) {
     const uint32_t wdst = lds0 + buf + C::ABYTES + wave * C::WBYTES;
-#pragma unroll
-    for (int f = 0; f < 2; ++f)
-#pragma unroll
-      for (int q = 0; q < 2; ++q)
-        lds_dma16<ONCE>(wdesc, wdst + f * 2048 + q * 1024, more ? w_off + (uint32_t)f * f_val + (uint32_t)s * 2048u + q * 1024u : kOutOfRange);
-    lds_dma4<ONCE>(sdesc, wdst + 4096, more ? s_off + (uint32_t)s * 128u : kOutOfRange);
+    const uint32_t at = w_off + (uint32_t)s * 2048u;
+    lds_dma_mxfp4<ONCE>(wdesc, sdesc, wdst, more ? at : kOutOfRange, more ? at + (f_val - 2048u) : kOutOfRange, more ? s_off + (uint32_t)s * 128u : kOutOfRange);
 #pragma unroll
     for (int i = 0; i < C::AI; ++i)
       lds_dma16(xdesc, lds0 + buf + (wave * C::AI + i) * 1024, more && s * 128 + a_k[i] < p.K ? a_off[i] + (uint32_t)s * 256u : kOutOfRange);
