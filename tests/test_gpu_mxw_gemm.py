@@ -152,3 +152,37 @@ def test_tiles_by_the_rules(device, kind, tile, e, k, n, sizes, swiglu, routed):
     for a, b in zip(by_rule, want):
         assert torch.equal(a, b)
     assert not torch.isnan(by_rule[0]).any() and by_rule[0].any()
+
+
+# slices, K, N, sizes: each tile with MXFP8 rows (32, 64, 128 and 160 rows; eight, sixteen and twenty rows' scales a wave)
+SCALED = [(128, 544, 576, [0, 1, 31, 32, 33, 2, 13]), (256, 672, 544, [33, 63, 64, 65, 10, 1]), (128, 800, 544, [95, 96, 97, 1, 33, 65, 40]), (128, 928, 544, [159, 160, 161, 33, 97])]
+
+
+@pytest.mark.parametrize("e, k, n, sizes", SCALED)
+@pytest.mark.parametrize("offset, pad", [(0, 0), (1, 3), (2, 1), (3, 6), (1, 7)])
+def test_scales_at_any_byte(device, e, k, n, sizes, offset, pad):
+    """Rows of activation scales that begin at any byte, between bytes that are no scales (NaN): the result is, bit for bit, that of scales in a
+    tensor of their own, and nothing of a neighbour gets into the last blocks of a row."""
+    import triton_amd.matmul as mm
+    from triton_amd.numerics_details.mxfp import downcast_to_mxfp
+    from triton_amd.tensor import FP4, convert_layout, make_ragged_tensor_metadata, wrap_torch_tensor
+    from triton_amd.tensor_details.layout import make_default_matmul_mxfp4_w_layout, make_default_matmul_mxfp4_w_scale_layout
+    g = torch.Generator(device=device).manual_seed(k + n + offset)
+    sizes = torch.tensor([sizes[i % len(sizes)] for i in range(e)], dtype=torch.int32, device=device)
+    m = int(sizes.sum())
+    a, scale = downcast_to_mxfp(torch.randn((m, k), generator=g, device=device).to(torch.bfloat16), torch.float8_e4m3fn, axis=-1)
+    wq, ws = downcast_to_mxfp((torch.randn((e, k, n), generator=g, device=device) * 0.1).to(torch.bfloat16), torch.uint8, axis=1)
+    w = convert_layout(wrap_torch_tensor(wq, dtype=FP4), make_default_matmul_mxfp4_w_layout(mx_axis=1))
+    s = convert_layout(wrap_torch_tensor(ws), make_default_matmul_mxfp4_w_scale_layout(mx_axis=1))
+    md, gather = make_ragged_tensor_metadata(sizes, m), torch.randint(0, m, (m, ), generator=g, device=device).to(torch.int32)
+
+    def run(x_scale):
+        return mm.matmul(a, w, None, md, gather_indx=gather, precision_config=mm.PrecisionConfig(a_mx_scale=x_scale, b_mx_scale=s, out_dtype=torch.bfloat16))
+    with mm.scoped_opt_flags_constraints({"block_m": 128}):
+        want = run(scale)
+    stride = k // 32 + pad
+    room = torch.full((offset + m * stride, ), 255, dtype=torch.uint8, device=device)
+    view = room[offset:].view(m, stride)[:, :k // 32]
+    view.copy_(scale)
+    got = run(view)
+    assert torch.equal(got, want) and not torch.isnan(got).any()

@@ -60,6 +60,7 @@ struct GemmParams {
   int64_t combine_stride;
   int32_t* combine_counters;  // zeroed [tokens * ceil(N / 32)] words, left zero
   const uint8_t* x_mx_scale;  // e8m0 block scales of MXFP8 activations [rows, K/32], or null
+  uint32_t xs_bytes = 0;      // ... their extent where a kernel addresses them through a buffer resource
   int64_t xs_stride_m;
   uint8_t* y_mx_scale;        // e8m0 block scales of an MX-quantised output [rows, N_out/32], or null
   int64_t ys_stride_m;

@@ -195,8 +195,11 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
       else
         fast = fast && p.y_vec && d->y_stride_m >= cdiv(n_out, piece) * piece;
       p.y_bytes = fast ? (uint32_t)y_bytes : 0u;
+      // (the wide kernel reads the scales through a buffer resource)
+      const int64_t xs_bytes = fast ? (x_rows - 1) * d->xs_stride_m + d->K / 32 : 0;
+      p.xs_bytes = xs_bytes < ((int64_t)1 << 31) - 8 ? (uint32_t)xs_bytes : 0u;
     }
-    if (const MxwTile tile = p.y_bytes != 0 ? wide_tile(p, d, true) : MxwTile{0, 0}; tile.rows) return gemm_launch_mxw_mx8(p, tile, swiglu, mx_out, st);
+    if (const MxwTile tile = p.xs_bytes != 0 ? wide_tile(p, d, true) : MxwTile{0, 0}; tile.rows) return gemm_launch_mxw_mx8(p, tile, swiglu, mx_out, st);
     return gemm_launch_mx8n(p, d->block_m, d->grid_m, swiglu, mx_out, st);
   }
   if (d->w_layout == TK_W_TILED) {

@@ -9,14 +9,17 @@
 //     the lanes' offsets (past the resource's range the hardware writes zeros).  Rings of two or three stages of rows and of weights run on
 //     across the tiles of a persistent workgroup.
 //   * bf16: e2m1 -> bf16 in registers in front of v_mfma_f32_32x32x16_bf16.  MXFP8: both operands as stored to
-//     v_mfma_scale_f32_32x32x64_f8f6f4; a row's activation scales arrive sixteen blocks at a time and wait in LDS for four stages.
-//   * What the next tile needs before its transfers (source rows) and in its epilogue (bias, gate weights, destinations) is requested one stage before
-//     the rows' ring needs it parked in LDS, and used a stage after that.  The epilogue's stores depend on nothing but the row fragments that hold
+//     v_mfma_scale_f32_32x32x64_f8f6f4; a row's activation scales arrive sixteen blocks at a time, by transfers as well, and wait in LDS for four stages.
+//   * What the next tile needs before its transfers (source rows) and in its epilogue (bias, gate weights, destinations) is fetched and parked in LDS one
+//     stage before the rows' ring needs it.  No load into registers is on its way anywhere else: the compiler, which cannot count the transfers, waits
+//     for all of them wherever such a load may be outstanding, and one that is requested in one stage and used in another may be in every
+//     stage (128 experts of MXFP8 rows, layer, us: 9 rows 368 -> 293, 44 431 -> 395, 72 488 -> 444, 94 505 -> 479).  The epilogue's stores depend on nothing but the row fragments that hold
 //     rows, so the wait in front of the next tile's first stage counts them and does not wait for them.
 //
 // What bounds the 160-row tile: the board's power in bf16 (fetching zeros instead of the weights, the operands then all zero, 558 -> 417 us; matrix pipe
-// 68 % busy at 1.9 GHz), in MXFP8 also LDS reads and the epilogue (without its arithmetic and stores 363 -> 316 us; 42 % busy at 2.3 GHz,
-// ten vector instructions per MFMA with the quantised output, seven with bf16).  128 experts, K 2880, 4096 tokens, top-4, whole layer:
+// 68 % busy at 1.9 GHz), in MXFP8 no single part (360 us; without its multiplications 325, with the weights from L2 307, hardly any LDS reads 343, without
+// the epilogue's arithmetic and stores 316): of a stage's 5500 cycles 2160 go into its multiplications, 1770 into waiting for transfers and the other waves,
+// 870 into the epilogue's share and 370 into the next tile's words.  128 experts, K 2880, 4096 tokens, top-4, whole layer:
 // bf16 861 -> 815 us, MXFP8 609 -> 563 us against the kernels that keep weights in registers with one wave per SIMD (moe_gemm_mxn, _mx8n, which
 // serve what this one does not take).  The smaller ones: reading the weights (128 experts, 14 MXFP8 rows each, both GEMMs 305 us for 1.63 GB).  Measured
 // and left out: transfers spread over the whole bf16 stage (576 against 558 us: the last ones are late); weights brought into L2 a stage ahead
@@ -43,10 +46,13 @@ struct MxwCfg {
   static constexpr int ABUFS = ABUFS_, WBUFS = WBUFS_;
   static constexpr int RINGS = ABUFS * ABYTES + WBUFS * WBYTES;
   static constexpr int SIDE = MX8 ? BM * 16 : 0;         // a row's activation scales of four stages
+  static constexpr int RW = BM / NW, RAWI = (RW + 11) / 12;  // rows whose scales a wave fetches, its transfers for that (twelve rows each)
+  static constexpr int RAW = MX8 ? RAWI * 256 * NW : 0;  // the scales as they arrive
   static constexpr int OPERANDS = (BN + 2 * BM) * 4;     // a tile's bias, gate weights, destination rows
   static constexpr bool LISTED = MFW == 5;               // the slice sizes and offsets wait in LDS: no registers are left for them
   static constexpr int LISTS = LISTED ? 2 * kDmaSlices * 4 : 0;
-  static constexpr int LDS = RINGS + 2 * (SIDE + OPERANDS) + LISTS;
+  static constexpr int LDS = RINGS + 2 * (SIDE + OPERANDS) + LISTS + RAW;
+  static_assert(LDS <= 160 * 1024, "a CU's LDS");
 };
 
 // ONCE: the weights are fetched with the non-temporal hint (reads_once)
@@ -104,6 +110,7 @@ __global__ __launch_bounds__(NW_ * 64, 2) void moe_gemm_mxw_kernel(const GemmPar
   };
   const int nfr = (p.N + 31) >> 5;
   const uint32_t f_val = (uint32_t)nst * 2048u, f_scale = (uint32_t)nst * 128u;  // bytes of a fragment
+  const int scale_row = wave * C::RW + (lane < C::RW ? lane : C::RW - 1);  // the row whose activation scales this lane parks
   const uint32_t w_off = (uint32_t)lane * 16u, s_off = (uint32_t)h * f_scale + (uint32_t)lr * 4u;
   // what a tile needs from memory before its first transfers: source rows; and before its epilogue: bias, gate weights, destinations
   auto request = [&](const Tile& c) __attribute__((always_inline)) {
@@ -122,7 +129,11 @@ __global__ __launch_bounds__(NW_ * 64, 2) void moe_gemm_mxw_kernel(const GemmPar
     const int sr = c.start_m + (row < c.eM ? row : c.eM - 1);
     if (p.gammas) raw_gam = p.gammas_is_f32 ? static_cast<const uint32_t*>(p.gammas)[sr] : (uint32_t)static_cast<const uint16_t*>(p.gammas)[sr];
     if (p.scatter) raw_dst = p.scatter[sr < p.scatter_len ? sr : p.scatter_len - 1];
-    if (MX8) raw_xs = p.gather ? p.gather[sr] : sr;
+    if constexpr (MX8) {
+      row = c.off_m + scale_row;
+      const int xr = c.start_m + (row < c.eM ? row : c.eM - 1);
+      raw_xs = p.gather ? p.gather[xr] : xr;
+    }
   };
   auto arrived = [&]() __attribute__((always_inline)) {  // (holds the uses of the requested words behind the wait in front of it)
 #pragma unroll
@@ -170,32 +181,42 @@ __global__ __launch_bounds__(NW_ * 64, 2) void moe_gemm_mxw_kernel(const GemmPar
       lds_dma4<ONCE>(sdesc, dst + 4096, (on ? (uint32_t)s * 128u : kOutOfRange) + s_off);
     }
   };
-  // activation scales: sixteen blocks (four stages) of row `tid` at a time, the last group of a row moved back to stay inside it
+  // Activation scales: sixteen blocks (four stages) of a row at a time.  They begin at any byte, so a transfer fetches the five words that hold them
+  // (twelve rows a transfer), and a stage later the wave that fetched a row shifts them into place.  (Loads into registers, which the compiler knows of,
+  // made it wait for everything outstanding in front of each stage's first operands.)
   const int kblocks = p.K >> 5;
-  u32x4_t xsq = {};
   uint32_t xs_row = 0;
+  const uint32_t xs_mis = MX8 ? (uint32_t)(reinterpret_cast<uintptr_t>(p.x_mx_scale) & 3) : 0u;
+  const buf_desc_t xsdesc = make_buf_desc(p.x_mx_scale - xs_mis, MX8 ? (p.xs_bytes + xs_mis + 3u) & ~3u : 0u);
+  const uint32_t raw0 = (uint32_t)(C::RINGS + 2 * (C::SIDE + C::OPERANDS) + C::LISTS + wave * C::RAWI * 256);
+  auto scales_aim = [&]() __attribute__((always_inline)) { xs_row = (uint32_t)raw_xs * (uint32_t)p.xs_stride_m + xs_mis; };
   auto scales_request = [&](int g) __attribute__((always_inline)) {
     if constexpr (MX8) {
-      const int b0 = g * 16 < kblocks - 16 ? g * 16 : kblocks - 16;
-      __builtin_memcpy(&xsq, p.x_mx_scale + (xs_row + (uint32_t)b0), 16);
+      const int r = (lane * 205) >> 10;  // lane / 5
+#pragma unroll
+      for (int i = 0; i < C::RAWI; ++i) {
+        const uint32_t row = (uint32_t)__builtin_amdgcn_ds_bpermute((i * 12 + r) * 4, (int)xs_row);
+        lds_dma4(xsdesc, lds0 + raw0 + i * 256, r < 12 ? ((row + (uint32_t)g * 16u) & ~3u) + (uint32_t)(lane - r * 5) * 4u : kOutOfRange);
+      }
     }
   };
   auto scales_park = [&](int g, int set) __attribute__((always_inline)) {
     if constexpr (MX8) {
-      asm volatile("" : "+v"(xsq));
-      const int back = g * 16 < kblocks - 16 ? 0 : g * 16 - (kblocks - 16);  // 0 .. 15
-      // bytes back .. of xsq, 2^0 behind its end
-      const uint32_t one = 0x7F7F7F7Fu;
-      const uint32_t w[9] = {xsq.x, xsq.y, xsq.z, xsq.w, one, one, one, one, one};
-      u32x4_t o = {};
+      if (lane < C::RW) {
+        const int t = lane >= 12 ? 1 : 0;
+        const uint32_t* raw = reinterpret_cast<const uint32_t*>(lds + raw0 + t * 256 + (lane - t * 12) * 20);
+        uint32_t w[5];
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        if ((back >> 2) == d) {
+        for (int d = 0; d < 5; ++d) w[d] = raw[d];
+        u32x4_t o;
 #pragma unroll
-          for (int i = 0; i < 4; ++i) o[i] = (uint32_t)((((uint64_t)w[i + d + 1] << 32) | w[i + d]) >> ((back & 3) * 8));
+        for (int d = 0; d < 4; ++d) {
+          const int in = kblocks - g * 16 - d * 4;  // blocks of this word inside the row; 2^0 behind its end
+          const uint32_t keep = in >= 4 ? ~0u : in <= 0 ? 0u : (1u << (8 * in)) - 1u;
+          o[d] = (__builtin_amdgcn_alignbyte(w[d + 1], w[d], xs_row) & keep) | (0x7F7F7F7Fu & ~keep);
         }
+        *reinterpret_cast<u32x4_t*>(side + set * C::SIDE + scale_row * 16) = o;
       }
-      if (tid < C::BM) *reinterpret_cast<u32x4_t*>(side + set * C::SIDE + tid * 16) = o;
     }
   };
 
@@ -205,9 +226,8 @@ __global__ __launch_bounds__(NW_ * 64, 2) void moe_gemm_mxw_kernel(const GemmPar
   arrived();
   park(cur, 0);
   aim(cur);
-  if constexpr (MX8) xs_row = (uint32_t)raw_xs * (uint32_t)p.xs_stride_m;
+  if constexpr (MX8) scales_aim();
   scales_request(0);
-  scales_park(0, 0);
   // the rings: activations one stage ahead, weights, which come from further away, WBUFS - 1
   constexpr uint32_t kW0 = C::ABUFS * C::ABYTES, kWEnd = C::RINGS;
   constexpr int AA = C::ABUFS - 1, WA = C::WBUFS - 1;
@@ -223,6 +243,10 @@ __global__ __launch_bounds__(NW_ * 64, 2) void moe_gemm_mxw_kernel(const GemmPar
     for (int i = 0; i < AI && n < AA; ++i) fetch_a(i, n, n * C::ABYTES, KB);
 #pragma unroll
     for (int i = 0; i < 5 && n < WA; ++i) fetch_w(i, n, kW0 + n * C::WBYTES, true);
+  }
+  if constexpr (MX8) {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(5 * WA + AI * AA) : "memory");  // (everything behind the scales)
+    scales_park(0, 0);
   }
   bool more = true;
   int stored = 0;  // row fragments that the last epilogue has stored
@@ -246,12 +270,12 @@ __global__ __launch_bounds__(NW_ * 64, 2) void moe_gemm_mxw_kernel(const GemmPar
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
       int fs = s + AA, ws = s + WA;  // stages to fetch
-      // the next tile, a step a stage: its words requested, then parked, then its transfers begin
-      if (s == nst - AA - 2) {
+      // the next tile: its words fetched and parked, a stage later its transfers begin.  (Requested a stage ahead the words are on their way across the
+      // loop's other paths, and the compiler puts a wait for everything outstanding into every stage.)
+      if (s == nst - AA - 1) {
         more = tile + t_step < t_end;
         if (more) nxt = locate(tile + t_step);
         request(nxt);
-      } else if (s == nst - AA - 1) {
         arrived();
         park(nxt, set ^ 1);
       } else if (s == nst - AA) {
@@ -260,7 +284,7 @@ __global__ __launch_bounds__(NW_ * 64, 2) void moe_gemm_mxw_kernel(const GemmPar
       if (s == nst - WA) aim_w(nxt);
       if constexpr (MX8) {
         if (s == nst - 2) {
-          xs_row = (uint32_t)raw_xs * (uint32_t)p.xs_stride_m;
+          scales_aim();
           scales_request(0);
         } else if (s == nst - 1) {
           scales_park(0, xset ^ 1);
@@ -288,40 +312,45 @@ __global__ __launch_bounds__(NW_ * 64, 2) void moe_gemm_mxw_kernel(const GemmPar
 #pragma unroll
         for (int i = 0; i < AI + 5; ++i) fetch(i);
       } else {
-        uint32_t sc[2];
         auto weights = [&](int f, int q) __attribute__((always_inline)) -> u32x4_t {
           return *reinterpret_cast<const u32x4_t*>(w + f * 2048 + q * 1024 + lane * 16);
         };
+        // (a lane's two blocks of the stage)
+        uint32_t sc[2];
 #pragma unroll
-        for (int f = 0; f < 2; ++f) sc[f] = *reinterpret_cast<const uint32_t*>(w + 4096 + f * 128 + lr * 4) >> (16 * h);
+        for (int f = 0; f < 2; ++f) sc[f] = *reinterpret_cast<const uint16_t*>(w + 4096 + f * 128 + lr * 4 + 2 * h);
         if constexpr (MX8) {
-          const uint8_t* xsc = side + xset * C::SIDE + lr * 16 + (s & 3) * 4;
+          const uint8_t* xsc = side + xset * C::SIDE + lr * 16 + (s & 3) * 4 + 2 * h;
           const int sw = (lr >> 1) & 7;
-          // one row fragment of one half stage ahead: activations, their scales; the second half's weights with its first one
-          i32x8_t xf[2];
-          uint32_t xs[2];
+          // two row fragments of a half stage ahead: activations, their scales; the second half's weights with its first one
+          i32x8_t xf[3];
+          uint32_t xs[3];
           u32x4_t wr[2][2];
           auto read = [&](auto i_c) __attribute__((always_inline)) {
             constexpr int i = decltype(i_c)::value, q = i / NJ, j = i % NJ;
             if constexpr (j == 0) wr[q][0] = weights(0, q), wr[q][1] = weights(1, q);
             const u32x4_t lo = *reinterpret_cast<const u32x4_t*>(a + (j * 32 + lr) * 128 + (((q * 2 + h) ^ sw) * 16));
             const u32x4_t hi = *reinterpret_cast<const u32x4_t*>(a + (j * 32 + lr) * 128 + (((4 + q * 2 + h) ^ sw) * 16));
-            xf[i & 1] = __builtin_bit_cast(i32x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
-            xs[i & 1] = *reinterpret_cast<const uint32_t*>(xsc + j * 512) >> (16 * h);
+            xf[i % 3] = __builtin_bit_cast(i32x8_t, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+            xs[i % 3] = *reinterpret_cast<const uint16_t*>(xsc + j * 512);
           };
           constexpr int NI = 2 * NJ;
           read(template_int<0>{});
           __builtin_amdgcn_sched_barrier(0);
+          read(template_int<1>{});
+          __builtin_amdgcn_sched_barrier(0);
           static_for<0, NI>([&](auto i_c) __attribute__((always_inline)) {
             constexpr int i = decltype(i_c)::value, q = i / NJ, j = i % NJ;
-            if constexpr (i + 1 < NI) read(template_int<i + 1>{});
+            if constexpr (i + 2 < NI) read(template_int<i + 2>{});
 #pragma unroll
             for (int f = 0; f < 2; ++f) {
               // (an fp4 operand is the low four of the eight registers the builtin's type has; the others stay undefined)
               const i32x8_t wv = __builtin_bit_cast(i32x8_t, __builtin_shufflevector(wr[q][f], wr[q][f], 0, 1, 2, 3, -1, -1, -1, -1));
-              acc[f][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wv, xf[i & 1], acc[f][j], 4 /* A: e2m1 */, 0 /* B: e4m3 */, q, (int)sc[f], q, (int)xs[i & 1]);
+              acc[f][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(wv, xf[i % 3], acc[f][j], 4 /* A: e2m1 */, 0 /* B: e4m3 */, q, (int)sc[f], q, (int)xs[i % 3]);
             }
-            static_for<i*(AI + 5) / NI, (i + 1) * (AI + 5) / NI>([&](auto t_c) __attribute__((always_inline)) { fetch(decltype(t_c)::value); });
+            // (two transfers a step: late ones are waited for, four a step hold up the first multiplications; 94 rows of 128 experts, layer: 479 us,
+            // 488 spread over the whole stage, 487 four a step)
+            static_for<(2 * i < AI + 5 ? 2 * i : AI + 5), (2 * i + 2 < AI + 5 && i + 1 < NI ? 2 * i + 2 : AI + 5)>([&](auto t_c) __attribute__((always_inline)) { fetch(decltype(t_c)::value); });
             __builtin_amdgcn_sched_barrier(0);
           });
         } else {
