@@ -347,8 +347,9 @@ typedef struct tk_gemm_desc {
    * tk/matmul_details/_matmul.py:535-569. */
   int32_t combine_k;
   /* Another kernel or tile than the one that block_m names, where the memory-to-LDS kernel runs (else not looked at): 32 or 64 = the kernel
-   * for few rows per expert with that many columns a workgroup (16-bit weights, no compute units left idle); 128 = 128 x 128 tiles
-   * beside block_m 256 (16-bit and tiled e4m3 weights); 256 or 512 = the wide kernel with tiles of so many columns, and of as many rows as
+   * for few rows per expert with that many columns a workgroup (16-bit weights, no compute units left idle); 128 or 256, beside
+   * block_m 256 with 16-bit weights = tiles of 320 rows and so many columns, where such a tile is meant for M, N and n_slices; else 128 = 128 x 128
+   * tiles beside block_m 256 (16-bit and tiled e4m3 weights); 256 or 512 = the wide kernel with tiles of so many columns, and of as many rows as
    * suit the rows per slice, where such a tile is meant for M, N and n_slices (tiled MXFP4 weights; not with combine_k, betas, out_alpha, acc_in,
    * row or column scales, an MX-quantised output from bf16 activations, or output rows that block_m 64 would not take).  0 = by block_m. */
   int32_t block_n;

@@ -88,6 +88,27 @@ inline MxwTile mxw_tile(int64_t rows, int64_t n_slices, int64_t N, bool mx8) {
   return rows <= 48 * n_slices ? MxwTile{64, 512} : rows <= 80 * n_slices ? MxwTile{96, 512} : MxwTile{160, 512};
 }
 
+// Tile of the memory-to-LDS kernel (moe_gemm_dma.hip) for 16-bit operands in place of 256 x 256 ones: 320 rows, so that a slice of about 256 rows, of which
+// a random routing makes half a few longer, is one row block.  (An eighth above the mean is 2.5 deviations at 400 rows, 2 at 256.)  rows 0 = those.
+//   320 x 128 where its tiles are one round and 128 x 128 ones (up to 96 of 256 x 256, dma_block_n) are not better; 320 x 256 beyond, from 248 rows on.
+// Measured (us of a GEMM with a random routing, 256 x 256 / 320 x 256 / 320 x 128; slices, K, N):
+//   16, 2048, 4096: 224 rows 89 / 100 / 92, 240 101 / 95 / 92, 256 105 / 96 / 92, 272 130 / 101 / 107, 288 136 / 122 / 126, 320 142 / 150 / 152
+//   16, 2048, 2048: 224 rows 56 / 72 / 50, 256 56 / 74 / 53, 272 57 / 78 / 58, 288 56 / 78 / 67; K 1024: 224 30 / 35 / 25, 272 32 / 40 / 28, 288 33 / 40 / 35
+//   16, 2880, 2880: 240 rows 89 / 101 / 108, 256 111 / 102 / 111, 272 127 / 107 / 128; 32, 2048, 4096: 240 175 / 182 / 176, 256 225 / 184 / 181, 288 280 /
+//   229 / 232; 32, 1024, 2048: 224 48 / 50 / 55, 256 65 / 55 / 59; 8, 4096, 4096: 224 102 / 120 / 83, 256 101 / 124 / 84, 272 103 / 132 / 108
+//   8, 2048, 2048 (128 x 128 / 320 x 128): 256 30 / 34; 272 (256 x 256) 43 / 35; two blocks: 448 45 / 41, 544 47 / 43, 608 49 / 55
+// (Slices that all have 256 rows to the row are as fast in the tiles of 256 or faster; how a routing divides the rows is not known here.)
+struct DmaTile {
+  int32_t rows, cols;
+};
+inline DmaTile dma_tile(int64_t rows, int64_t n_slices, int64_t N) {
+  if (n_slices < 8) return {0, 0};
+  const int64_t per_slice = rows / n_slices, n256 = (N + 255) / 256, blocks = (per_slice * 9 / 8 + 319) / 320;
+  if (per_slice >= (blocks == 1 ? 192 : 448) && blocks <= 2 && n_slices * blocks * ((N + 127) / 128) <= 256 && n_slices * ((per_slice + 255) / 256) * n256 > 96)
+    return {320, 128};
+  return per_slice >= 248 && per_slice <= 288 && n_slices * n256 > 128 ? DmaTile{320, 256} : DmaTile{0, 0};
+}
+
 // Row blocks (of 64) that the kernel for few rows launches side by side: one a slice at least, and what slices of up to five quarters of
 // the mean make, as a random routing does (at 62 rows per slice half of the slices have a second block).
 inline int64_t few_row_blocks(int64_t rows, int64_t n_slices) { return n_slices * (rows * 5 / (n_slices * 256) + 1); }

@@ -182,7 +182,10 @@ int64_t dma_block_m(int64_t rows, int64_t row_bytes, int64_t N, int64_t n_slices
 // Measured with a random routing (us, 128 against 256): bf16, K 2048, N 2048, 8 slices of 256 rows (64 large tiles) 29 against 42; N 1536, 16
 // slices (96) 34 against 41; N 2048, 16 slices (128) 51 against 49; K 1024, N 1024, 16 slices (64) 19 against 27, N 512 (32) 11 against 23;
 // K 4096, N 1024, 16 slices (64) 55 against 72; e4m3, K 14336, N 2048, 8 slices (64) 92 against 126, N 4096 (128) 193 against 158.
-int64_t dma_block_n(int64_t rows, int64_t N, int64_t n_slices, int64_t block_m) {
+// With 16-bit operands, columns of the tiles of 320 rows where gemm_limits.h names those.
+int64_t dma_block_n(int64_t rows, int64_t N, int64_t n_slices, int64_t block_m, bool bits16) {
+  const int64_t cols = block_m == 256 && bits16 ? tk::dma_tile(rows, n_slices, N).cols : 0;
+  if (cols) return cols;
   const int64_t per_slice = rows / std::max<int64_t>(n_slices, 1);
   return block_m == 256 && n_slices * ((per_slice + 255) / 256) * ((N + 255) / 256) <= 96 ? 128 : 0;
 }
@@ -440,7 +443,7 @@ PyObject* run_gemm(PyObject* const* v) {
   const uint32_t x_bytes = tk::x_extent(a_rows, a_stride, K, a->element_size());
   if (tiled_fp8) {
     block_m = fp8_block_m(M, x_bytes, K, N, n_slices);
-    if (tk::dma_runs_e4m3(x_bytes, n_slices, K, N)) block_n = dma_block_n(M, N, n_slices, block_m);
+    if (tk::dma_runs_e4m3(x_bytes, n_slices, K, N)) block_n = dma_block_n(M, N, n_slices, block_m, false);
   } else if (mx_act) {
     block_m = wide_block_m(M, n_slices, K, x_bytes, true);
     block_n = wide_block_n(M, n_slices, K, N, x_bytes, true);
@@ -453,7 +456,7 @@ PyObject* run_gemm(PyObject* const* v) {
   } else if (tk::dma_runs_16bit(x_bytes, n_slices, K, N, w->stride(2))) {
     if (idle <= 0) block_n = few_block_n(M, N, n_slices);
     if (block_m > 16) block_m = dma_block_m(M, 2 * K, N, n_slices);
-    if (!block_n) block_n = dma_block_n(M, N, n_slices, block_m);
+    if (!block_n) block_n = dma_block_n(M, N, n_slices, block_m, true);
   }
   if (tiled && block_m >= 64 && !mx_act && n_out % 8) return none();  // (through a padded buffer)
 
@@ -833,7 +836,11 @@ PyObject* rule_few(PyObject* const* v) {
 }
 PyObject* rule_dma_n(PyObject* const* v) {
   const auto [rows, N, n_slices, block_m] = integers<4>(v);
-  return PyLong_FromLongLong(dma_block_n(rows, N, n_slices, block_m));
+  return PyLong_FromLongLong(dma_block_n(rows, N, n_slices, block_m, false));
+}
+PyObject* rule_dma_n_16bit(PyObject* const* v) {
+  const auto [rows, N, n_slices, block_m] = integers<4>(v);
+  return PyLong_FromLongLong(dma_block_n(rows, N, n_slices, block_m, true));
 }
 PyObject* rule_dma_e4m3(PyObject* const* v) {
   const auto [x_bytes, n_slices, K, N] = integers<4>(v);
@@ -912,6 +919,7 @@ PyMethodDef methods[] = {
     METHOD("dma_block_m", rule_dma, 4),
     METHOD("dma_runs_e4m3", rule_dma_e4m3, 4),
     METHOD("dma_block_n", rule_dma_n, 4),
+    METHOD("dma_block_n_16bit", rule_dma_n_16bit, 4),
     METHOD("few_block_n", rule_few, 3),
     METHOD("decode_by_rows", rule_decode_rows, 4),
     METHOD("fp8_block_m", rule_fp8, 5),

@@ -11,11 +11,16 @@ using namespace tk;
 // slices of the ragged metadata (a call without it has one)
 static int64_t slices(const tk_gemm_desc* d) { return d->slice_sizes ? d->n_slices : 1; }
 
-// Row blocks of 256 rows or, asked for by block_n, 128 x 128 tiles in their place (grid_m counts row blocks of block_m).
+// Row blocks of 256 rows or, asked for by block_n, 128 x 128 tiles or those of 320 rows in their place (grid_m counts row blocks of block_m).
 static int32_t launch_dma(const GemmParams& p, const tk_gemm_desc* d, int wk, bool swiglu, hipStream_t st) {
-  if (d->block_m != 256 || d->block_n != 128) return gemm_launch_dma(p, wk, d->block_m, d->grid_m, swiglu, st);
-  const int64_t n = slices(d), blocks = d->M <= n ? d->M : n - 1 + cdiv(d->M + 1 - n, 128);
-  return gemm_launch_dma(p, wk, 128, (int)blocks, swiglu, st);
+  const int64_t n = slices(d);
+  if (d->block_m == 256 && (d->block_n == 128 || d->block_n == 256) && wk != WK_FP8) {
+    const DmaTile tile = dma_tile(d->M, n, d->N);
+    if (tile.rows && tile.cols == d->block_n) return gemm_launch_dma(p, wk, tile, d->grid_m, swiglu, st);
+  }
+  if (d->block_m != 256 || d->block_n != 128) return gemm_launch_dma(p, wk, DmaTile{d->block_m, d->block_m}, d->grid_m, swiglu, st);
+  const int64_t blocks = d->M <= n ? d->M : n - 1 + cdiv(d->M + 1 - n, 128);
+  return gemm_launch_dma(p, wk, DmaTile{128, 128}, (int)blocks, swiglu, st);
 }
 
 // Strided 16-bit weights: the kernel that stages both operands through memory-to-LDS transfers for full row blocks where it runs, else the

@@ -1,12 +1,13 @@
 // Expert GEMM for full row blocks with both operands staged by memory-to-LDS transfers: bf16 / fp16 (strided, K-contiguous weights)
 // and e4m3 (tiled weights), fp32 accumulation, the shared epilogue.
 //
-//   * A workgroup multiplies BM rows of one expert by BN columns: 256 x 256 with eight waves of 128 x 64 (one workgroup per CU), or
-//     128 x 128 with four waves of 64 x 64 (two per CU).  Either way a SIMD holds two waves: while one waits for LDS or at the
+//   * A workgroup multiplies BM rows of one expert by BN columns: 256 x 256 with eight waves of 128 x 64 (one workgroup per CU),
+//     128 x 128 with four waves of 64 x 64 (two per CU), or with 16-bit operands 320 x 256 or 320 x 128, eight waves of 160 x 64 or 160 x 32, for slices of
+//     about 256 rows (dma_tile in gemm_limits.h).  Either way a SIMD holds two waves: while one waits for LDS or at the
 //     barrier the other feeds the matrix pipe.
 //   * A stage is 128 bytes of K of every row and column, i.e. whole cache lines: with 64-byte stages every line crossed from L2 to
 //     the CU twice, 37 bytes per cycle for 18 useful ones.  The LDS holds two stages of activations and three of weights (which come
-//     from further away).  Every transfer is a `buffer_load ... lds` of 1 KiB per wave, eight rows of a line each: no registers, no VALU, no
+//     from further away; two beside 320 rows and 256 columns).  Every transfer is a `buffer_load ... lds` of 1 KiB per wave, eight rows of a line each: no registers, no VALU, no
 //     LDS write instructions; gathered rows, rows past the slice, columns past N and k past K are a matter of the lanes'
 //     offsets (past the resource's range the hardware writes zeros).
 //   * Rows lie 128 bytes apart without padding (the transfer writes lane-contiguously); the 16-byte pieces of row r are stored at
@@ -26,6 +27,8 @@
 // GHz, K 14336: 77 % at 1.75), with a few rows per expert (128 x 128 tiles) the weight stream at 5.9 TB/s (5.3 without the
 // non-temporal hint).  16384 routed rows
 // of 8 experts in e4m3: K 4096, N 28672, swiglu 1840 -> 1590 us (2.42 PFLOP/s), K 14336, N 4096 850 -> 805 us; 4096 rows of 16
+// experts in bf16, K 2048, about 256 rows each: a stage takes 1.9 to 2.4 us, twice its multiplications, and the CU's cache has about 90 lines of 128 bytes under way
+// whatever is asked for ahead (weights two stages at a time into a ring of four: no change).  4096 rows of 16
 // experts in bf16, K 2048: N 4096 231 -> 94 us, N 2048 133 -> 51 us (the kernels before: weights in registers with one wave
 // per SIMD, and both operands through registers into LDS).
 #include "gemm_tiles.h"
@@ -33,24 +36,27 @@
 namespace tk {
 namespace {
 
-template <bool LARGE>
+// 128 x 128 tiles (kDma128), 256 x 256 (kDma256), 320 x 256 and 320 x 128 (kDma320, kDma320Half; 16-bit operands)
+enum { kDma128, kDma256, kDma320, kDma320Half };
+template <int TILE>
 struct DmaCfg {
-  static constexpr int WM = 2, WN = LARGE ? 4 : 2;       // waves along rows / columns
-  static constexpr int MFW = LARGE ? 4 : 2, NFW = 2;     // fragments of a wave
+  static constexpr int WM = 2, WN = TILE == kDma128 ? 2 : 4;                                       // waves along rows / columns
+  static constexpr int MFW = TILE == kDma128 ? 2 : TILE == kDma256 ? 4 : 5, NFW = TILE == kDma320Half ? 1 : 2;  // fragments of a wave
   static constexpr int BM = WM * MFW * 32, BN = WN * NFW * 32;
   static constexpr int NW = WM * WN;
   static constexpr int ABYTES = BM * 128, BBYTES = BN * 128;
-  static constexpr int ABUFS = 2, BBUFS = 3;
+  static constexpr int ABUFS = 2, BBUFS = TILE == kDma320 ? 2 : 3;
   static constexpr int LDS = ABUFS * ABYTES + BBUFS * BBYTES;
   static constexpr int SBN = BN / 2;  // columns of a narrow tile
   static constexpr int AI = BM / 8 / NW, BI = BN / 8 / NW;  // transfers of a wave and stage
+  static constexpr int PER_CU = TILE == kDma128 ? 2 : 1;    // workgroups
 };
-static_assert(DmaCfg<true>::LDS == 160 * 1024 && DmaCfg<false>::LDS == 80 * 1024, "one / two workgroups fill a CU's LDS");
+static_assert(DmaCfg<kDma256>::LDS == 160 * 1024 && DmaCfg<kDma128>::LDS == 80 * 1024 && DmaCfg<kDma320>::LDS <= 160 * 1024, "one / two workgroups of a CU");
 
 // NARROW: short row blocks may be cut into narrow tiles (gemm_tiles.h).  ONCE: the weights are fetched with the non-temporal hint (reads_once).
-template <int WK, bool LARGE, bool SWIGLU, bool NARROW, bool ONCE>
-__global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel(const GemmParams p) {
-  typedef DmaCfg<LARGE> C;
+template <int WK, int TILE, bool SWIGLU, bool NARROW, bool ONCE>
+__global__ __launch_bounds__(DmaCfg<TILE>::NW * 64, 2) void moe_gemm_dma_kernel(const GemmParams p) {
+  typedef DmaCfg<TILE> C;
   constexpr bool F8 = WK == WK_FP8;
   constexpr int ES = F8 ? 1 : 2;
   constexpr int MFW = C::MFW, NFW = C::NFW;
@@ -71,13 +77,14 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
   // ---- transfer side ------------------------------------------------------------------------------------------------------------------------------
   // transfer i of an operand: rows i * 8 .. + 7, lane -> row lane / 8, LDS position lane % 8, i.e. piece (lane % 8) ^ (row >> 1 & 7);
   // with eight rows a transfer, row >> 1 & 7 = (i & 1) * 4 + (lane >> 4)
-  // (a wave's transfers start at an even index, so the parity of i counts)
+  // (pc0, pc1: of a wave's transfers of even and odd index, which start at an even index or, of activations, at wave * AI)
   const int pc0 = (lane & 7) ^ (lane >> 4), pc1 = pc0 ^ 4;
+  const int pa0 = C::AI % 2 ? pc0 ^ ((wave & 1) << 2) : pc0, pa1 = pa0 ^ 4;
   const buf_desc_t xdesc = make_buf_desc(p.x, p.x_bytes);
   buf_desc_t wdesc;
   uint32_t a_off[C::AI], b_off[C::BI];
   const uint32_t x_row = (uint32_t)(p.x_stride_m * ES);
-  static_assert(C::AI % 2 == 0 && C::BI % 2 == 0, "a transfer's parity is that of its index in the wave");
+  static_assert(C::BI % 2 == 0 && (C::AI % 2 == 0 || !NARROW), "a transfer's parity is that of its index in the wave");
   // A narrow tile's stage is twice as long: the first half of the waves fetches its first 128 bytes of K, for half of the rows and columns that the
   // buffers have room for, the others the second.
   int f_step = 128, f_kh = 0;  // bytes of K of a stage, and where this wave's transfers begin in it
@@ -93,7 +100,7 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
       const int row = c.off_m + (w_in * C::AI + i) * 8 + (lane >> 3);
       const int sr = c.start_m + (row < c.eM ? row : c.eM - 1);
       const uint32_t src = p.gather ? (uint32_t)p.gather[sr] : (uint32_t)sr;
-      a_off[i] = row < c.eM ? src * x_row + (uint32_t)((i & 1) ? pc1 : pc0) * 16u : kOutOfRange;
+      a_off[i] = row < c.eM ? src * x_row + (uint32_t)((i & 1) ? pa1 : pa0) * 16u : kOutOfRange;
     }
     const uint8_t* w = p.w + (int64_t)c.expert * p.w_stride_e;
     if constexpr (F8) {
@@ -118,7 +125,7 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
   // transfer i of this wave for the stage at byte kb of K of the tile aimed at (none left: zeros into a buffer that nobody reads)
   auto fetch_a = [&](int i, int kb, uint32_t buf, bool more) __attribute__((always_inline)) {
     kb += f_kh;
-    const bool in = more && kb + ((i & 1) ? pc1 : pc0) * 16 < KB;
+    const bool in = more && kb + ((i & 1) ? pa1 : pa0) * 16 < KB;
     lds_dma16(xdesc, lds0 + buf + (wave * C::AI + i) * 1024, in ? a_off[i] + (uint32_t)kb : kOutOfRange);
   };
   auto fetch_b = [&](int i, int kb, uint32_t buf, bool more) __attribute__((always_inline)) {
@@ -175,29 +182,39 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
   u32x4_t ar[2][F8 ? 1 : MFW], wr[2][F8 ? 1 : NFW];
   i32x8_t a8[2][F8 ? MFW / 2 : 1], w8[2][F8 ? NFW : 1];
   // quarter Q of the stage at (abuf, bbuf), while the operands of the next quarter are read: of the same stage, or for Q = 3 of the next
-  auto quarter = [&](auto full_c, auto q_c, int jc, uint32_t abuf, uint32_t bbuf) __attribute__((always_inline)) {
-    constexpr bool FULL = decltype(full_c)::value;
+  // (NJ row fragments if that is not 0, else those of the wave's MFW that hold rows)
+  auto quarter = [&](auto nj_c, auto q_c, int jc, uint32_t abuf, uint32_t bbuf) __attribute__((always_inline)) {
+    constexpr int NJ = decltype(nj_c)::value, JN = NJ ? NJ : MFW;
+    constexpr bool FULL = NJ != 0;
     constexpr int Q = decltype(q_c)::value, QN = (Q + 1) & 3, P = Q & 1;
     // A wave's transfers are spread over the stage (the CU takes one per sixteen cycles or so; all eight behind the barrier held up
     // its first multiplications): activations, which the next barrier waits for, in quarter 3, weights in quarters 0 and 1.
-    auto transfer = [&](int k) __attribute__((always_inline)) {
-      if constexpr (Q == 3) {
-        fetch_a(2 * k, fs, aw, more);
-        fetch_a(2 * k + 1, fs, aw, more);
+    // (With two stages of weights these wait for the barrier as well, and go first: they come from further away.)
+    constexpr int QB = C::BBUFS == 2 ? (Q == 3 ? C::BI : 0) : Q < 2 ? C::BI / 2 : 0, QT = QB + (Q == 3 ? C::AI : 0);
+    auto transfer = [&](int k, int of) __attribute__((always_inline)) {
+#pragma unroll
+      for (int i = k * QT / of; i < (k + 1) * QT / of; ++i) {
+        if (i < QB)
+          fetch_b(C::BBUFS == 2 ? i : Q * QB + i, fs, bw, more);
+        else
+          fetch_a(i - QB, fs, aw, more);
       }
-      if constexpr (Q < 2) fetch_b(2 * Q + k, fs, bw, more);
     };
     if constexpr (!F8) {
 #pragma unroll
       for (int f = 0; f < NFW; ++f) wr[1 - P][f] = read_b(bbuf, f, QN);
 #pragma unroll
-      for (int j = 0; j < MFW; ++j) {
+      for (int j = 0; j < JN; ++j) {
         ar[1 - P][j] = read_a(abuf, j, QN);
         if (FULL || j < jc) {
 #pragma unroll
           for (int f = 0; f < NFW; ++f) acc[f][j] = mma16(wr[P][f], ar[P][j], acc[f][j]);
         }
-        if (j % (MFW / 2) == MFW / 2 - 1) transfer(j / (MFW / 2));
+        if constexpr (MFW % 2 == 0) {
+          if (j % (MFW / 2) == MFW / 2 - 1) transfer(j / (MFW / 2), 2);
+        } else {
+          transfer(j, JN);
+        }
         if constexpr (FULL) __builtin_amdgcn_sched_barrier(0);
       }
     } else {
@@ -215,7 +232,7 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
             acc[f][P * HJ + j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w8[U][f], a8[P][j], acc[f][P * HJ + j], 0, 0, 0, 0x7F7F7F7F, 0, 0x7F7F7F7F);
         }
 #pragma unroll
-        for (int k = 0; k < 2 / HJ; ++k) transfer(HJ == 2 ? j : k);
+        for (int k = 0; k < 2 / HJ; ++k) transfer(HJ == 2 ? j : k, 2);
         if constexpr (FULL) {
           // (an empty use of the results: the compiler otherwise sinks the multiplications to the end of the loop)
 #pragma unroll
@@ -232,16 +249,15 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
     asm volatile("" ::: "memory");
   };
   // stages 0 and 1 of both operands: as the loop finds them in front of its quarter 0
-  static_assert(C::AI == 4 && C::BI == 4, "transfers as dealt to the quarters");
 #pragma unroll
   for (int n = 0; n < 2; ++n) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) fetch_b(i, fs, bw, more);
+    for (int i = 0; i < C::BI; ++i) fetch_b(i, fs, bw, more);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) fetch_a(i, fs, aw, more);
+    for (int i = 0; i < C::AI; ++i) fetch_a(i, fs, aw, more);
     advance();
   }
-  asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::AI + C::BI) : "memory");
   barrier();
   uint32_t ab = 0, bb = kAEnd;
   // the operands of a tile's first quarter (read again behind an epilogue, which needs the registers)
@@ -323,26 +339,28 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
         for (int i = 0; i < 16; ++i) acc[f][j][i] = 0.f;
     const int rows = cur.eM - cur.off_m < C::BM ? cur.eM - cur.off_m : C::BM;
     const int jc = __builtin_amdgcn_readfirstlane((((rows + 31) >> 5) - mw + C::WM - 1) / C::WM);  // this wave's row fragments (j * WM + mw) that hold rows
-    auto stages = [&](auto full_c) __attribute__((always_inline)) {
+    auto stages = [&](auto nj_c) __attribute__((always_inline)) {
       for (int s = 0; s < nst; ++s) {
-        quarter(full_c, template_int<0>{}, jc, ab, bb);
-        quarter(full_c, template_int<1>{}, jc, ab, bb);
-        quarter(full_c, template_int<2>{}, jc, ab, bb);
-        // the next stage has landed (this wave's part) when only the four transfers of quarters 0 and 1 are outstanding
-        asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        quarter(nj_c, template_int<0>{}, jc, ab, bb);
+        quarter(nj_c, template_int<1>{}, jc, ab, bb);
+        quarter(nj_c, template_int<2>{}, jc, ab, bb);
+        // the next stage has landed (this wave's part) when only the transfers of quarters 0 and 1 are outstanding
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::BBUFS == 2 ? 0 : C::BI) : "memory");
         barrier();
         ab = ab + C::ABYTES == kAEnd ? 0 : ab + C::ABYTES;
         bb = bb + C::BBYTES == kBEnd ? kAEnd : bb + C::BBYTES;
-        quarter(full_c, template_int<3>{}, jc, ab, bb);
+        quarter(nj_c, template_int<3>{}, jc, ab, bb);
         // (the one branch of a stage stands at its end: with one in between, the compiler moves the multiplications in front of it
         // down behind it, and their operands pile up)
         advance();
       }
     };
     if (jc >= MFW)
-      stages(std::true_type{});
+      stages(template_int<MFW>{});
+    else if (MFW == 5 && jc == 4)
+      stages(template_int<MFW == 5 ? 4 : 0>{});
     else
-      stages(std::false_type{});
+      stages(template_int<0>{});
     gemm_epilogue<32, C::WM, MFW, NFW, SWIGLU, WK == WK_F16>(p, acc, cur.expert, cur.off_m, cur.start_m, cur.eM, cur.n_tile + nw * NFW * 32,
                                                              cur.n_tile + C::BN <= p.N, mw, lr, h);
     tile += t_step;
@@ -352,9 +370,9 @@ __global__ __launch_bounds__(DmaCfg<LARGE>::NW * 64, 2) void moe_gemm_dma_kernel
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no transfer into this workgroup's LDS is left behind
 }
 
-template <int WK, bool LARGE>
+template <int WK, int TILE>
 int32_t launch_cfg(const GemmParams& p, int grid_m, bool swiglu, hipStream_t st) {
-  typedef DmaCfg<LARGE> C;
+  typedef DmaCfg<TILE> C;
   GemmParams q = p;
   q.grid_n = (int)cdiv(p.N, C::BN);
   const int64_t tiles = (int64_t)grid_m * q.grid_n;
@@ -362,7 +380,7 @@ int32_t launch_cfg(const GemmParams& p, int grid_m, bool swiglu, hipStream_t st)
   if (tiles > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: grid too large");
   q.total_tiles = (int32_t)tiles;
   // a multiple of 8 workgroups (every XCD walks its share of the tiles), one or two per CU
-  int64_t grid = (int64_t)busy_cu_count(p.idle_cus) * (LARGE ? 1 : 2) / 8 * 8;
+  int64_t grid = (int64_t)busy_cu_count(p.idle_cus) * C::PER_CU / 8 * 8;
   grid = grid < 8 ? 8 : grid;
   grid = grid < cdiv(tiles, 8) * 8 ? grid : cdiv(tiles, 8) * 8;
   auto launch = [&](auto kern) -> int32_t {
@@ -371,26 +389,31 @@ int32_t launch_cfg(const GemmParams& p, int grid_m, bool swiglu, hipStream_t st)
     return check_launch("moe_gemm_dma_kernel");
   };
   if (reads_once(p.M, p.slice_sizes ? p.n_slices : 1, C::BM, p.N, p.K * (WK == WK_FP8 ? 1 : 2)))
-    return swiglu ? launch(moe_gemm_dma_kernel<WK, LARGE, true, false, true>) : launch(moe_gemm_dma_kernel<WK, LARGE, false, false, true>);
-  if constexpr (LARGE) {
+    return swiglu ? launch(moe_gemm_dma_kernel<WK, TILE, true, false, true>) : launch(moe_gemm_dma_kernel<WK, TILE, false, false, true>);
+  if constexpr (TILE == kDma256) {
     // (the other kernel, half a microsecond faster to start, where all tiles are one round, and its stages are half a percent shorter where they
     // are many: e4m3, K 4096, 31 rounds)
     if (tiles > grid && tiles <= 8 * grid)
-      return swiglu ? launch(moe_gemm_dma_kernel<WK, LARGE, true, true, false>) : launch(moe_gemm_dma_kernel<WK, LARGE, false, true, false>);
+      return swiglu ? launch(moe_gemm_dma_kernel<WK, TILE, true, true, false>) : launch(moe_gemm_dma_kernel<WK, TILE, false, true, false>);
   }
-  return swiglu ? launch(moe_gemm_dma_kernel<WK, LARGE, true, false, false>) : launch(moe_gemm_dma_kernel<WK, LARGE, false, false, false>);
+  return swiglu ? launch(moe_gemm_dma_kernel<WK, TILE, true, false, false>) : launch(moe_gemm_dma_kernel<WK, TILE, false, false, false>);
 }
 
 }  // namespace
 
-int32_t gemm_launch_dma(const GemmParams& p, int wk, int block_m, int grid_m, bool swiglu, hipStream_t st) {
+int32_t gemm_launch_dma(const GemmParams& p, int wk, DmaTile tile, int grid_m, bool swiglu, hipStream_t st) {
+  auto launch_16bit = [&](auto wk_c) -> int32_t {
+    constexpr int WK = decltype(wk_c)::value;
+    if (tile.rows == 320) return tile.cols == 256 ? launch_cfg<WK, kDma320>(p, grid_m, swiglu, st) : launch_cfg<WK, kDma320Half>(p, grid_m, swiglu, st);
+    return tile.rows == 256 ? launch_cfg<WK, kDma256>(p, grid_m, swiglu, st) : launch_cfg<WK, kDma128>(p, grid_m, swiglu, st);
+  };
   switch (wk) {
     case WK_BF16:
-      return block_m == 256 ? launch_cfg<WK_BF16, true>(p, grid_m, swiglu, st) : launch_cfg<WK_BF16, false>(p, grid_m, swiglu, st);
+      return launch_16bit(template_int<WK_BF16>{});
     case WK_F16:
-      return block_m == 256 ? launch_cfg<WK_F16, true>(p, grid_m, swiglu, st) : launch_cfg<WK_F16, false>(p, grid_m, swiglu, st);
+      return launch_16bit(template_int<WK_F16>{});
     case WK_FP8:
-      return block_m == 256 ? launch_cfg<WK_FP8, true>(p, grid_m, swiglu, st) : launch_cfg<WK_FP8, false>(p, grid_m, swiglu, st);
+      return tile.rows == 256 ? launch_cfg<WK_FP8, kDma256>(p, grid_m, swiglu, st) : launch_cfg<WK_FP8, kDma128>(p, grid_m, swiglu, st);
   }
   return fail(TK_ERR_INVALID, "tk_moe_gemm: bad weight kind %d", wk);
 }

@@ -784,7 +784,7 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
                 d.block_n = nt.rules().few_block_n(M, N, n_slices)
             if block_m > 16:
                 block_m = nt.rules().dma_block_m(M, 2 * K, N, n_slices)
-            d.block_n = d.block_n or nt.rules().dma_block_n(M, N, n_slices, block_m)
+            d.block_n = d.block_n or nt.rules().dma_block_n_16bit(M, N, n_slices, block_m)
     elif block_m == 256:
         block_m = 128
     if is_ragged:
