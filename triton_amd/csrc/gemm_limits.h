@@ -51,9 +51,11 @@ inline bool reads_once(int64_t rows, int64_t n_slices, int64_t block_rows, int64
 
 // Tile of the wide MXFP4 kernel (moe_gemm_mxw_kernel.h) for a call whose rows are more than the decode kernel is made for; rows 0 = the kernels before it.
 // Figures: us, both GEMMs of a layer; "before" = the streaming kernel's 32-row blocks, or 64 and 128 rows of the ones with weights in registers.
-// bf16 rows.  32 x 256 (two workgroups a CU) is the shortest chain where it is one round; otherwise up to 20 rows the streaming kernel, which waits for no
-// other wave (real layers, 128 slices, K 2880: 3 rows 274 against 284, 9 rows 323 against 355).  64 x 256, two workgroups a CU as well, divides a small
-// product evenly; where the tiles of 512 columns are two rounds and more, those: half the reads of the rows, and three stages of weights in flight.
+// bf16 rows.  32 x 256 (two workgroups a CU) is the shortest chain and divides best, for one round and up to 20 rows; beyond four rows 64 x 512, half the reads of the
+// rows, where its tiles are three a CU (real layers, the streaming kernel / 32 x 256 / 64 x 512: 128 slices, K 2880: 3 rows 277 / 268 / 275, 5 302 / 292 /
+// 286, 9 315 / 310 / 301, 19 370 / 351 / 332; K 2048: 9 rows 170 / 163 / 162, 16 178 / 176 / 171; 96 slices, K 1088, 12 rows 62 / 60 / 71; 64 slices, K 1536: 9
+// rows 66 / 63 / 68, 19 75 / 76 / 75; 32 slices, K 2880, 19 rows 109 / 104 / 106).  64 x 256, two workgroups a CU as well, divides a small
+// product of more rows evenly; where the tiles of 512 columns are two rounds and more, those: half the reads of the rows, and three stages of weights in flight.
 //   128 slices, K 2880, N 5760 and 2880: 28 rows before 415, 370 (64 x 512), 42 471, 416, 56 525, 475 (96; 64 x 512 498), 72 607, 544 (96; 160 563,
 //   64 x 256 743), 84 646, 602 (160; 96 613)
 //   128 slices, K 2048, N 4096: 28 rows 131, 117 (64 x 512; 64 x 256 123), 69 203, 177 (96), 109 271, 236 (160; 64 x 256 268)
@@ -83,7 +85,7 @@ inline MxwTile mxw_tile(int64_t rows, int64_t n_slices, int64_t N, bool mx8) {
     return rows <= (few ? 40 : 24) * n_slices ? MxwTile{64, 512} : rows <= 104 * n_slices ? MxwTile{128, 512} : MxwTile{0, 0};
   }
   if ((rows + 16 * n_slices) * n256 <= 512 * 32) return {32, 256};
-  if (rows <= 20 * n_slices) return {0, 0};
+  if (rows <= 20 * n_slices) return rows > 4 * n_slices && n_slices * n512 >= 3 * 256 ? MxwTile{64, 512} : MxwTile{32, 256};
   if ((rows + 160 * n_slices - 1) / (160 * n_slices) * n_slices * n512 < 512) return {64, 256};
   return rows <= 48 * n_slices ? MxwTile{64, 512} : rows <= 80 * n_slices ? MxwTile{96, 512} : MxwTile{160, 512};
 }

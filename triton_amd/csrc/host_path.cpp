@@ -203,7 +203,8 @@ int64_t fp8_block_m(int64_t rows, uint32_t x_bytes, int64_t K, int64_t N, int64_
 // than the decode kernel's 16-row blocks from 160 rows on (128 slices, K 2880, N 5760: 300 tokens 210 against 232 us, 32 slices,
 // 200 tokens 28 against 57 us) and than the prefill kernel's 64-row blocks up to about 20 rows per slice (18: 245 against 258 us,
 // 31: 331 against 290 us); those give way to the larger ones at about 56 (47: 340 against 372 us, 62: 410 against 399 us).
-// (For calls that the streaming kernel takes: x as a buffer resource, slices in registers, no row or column scales.)
+// (For calls that the streaming kernel takes: x as a buffer resource, slices in registers, no row or column scales.  Where the wide kernel runs, its tiles
+// (mxw_tile) come in place of all of these.)
 int64_t mxfp4_block_m(int64_t rows, int64_t n_slices, int64_t otherwise) {
   int64_t per_slice = rows / std::max<int64_t>(n_slices, 1);
   return per_slice <= 20 ? 32 : per_slice <= 56 ? 64 : std::max<int64_t>(otherwise, 128);
