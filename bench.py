@@ -313,8 +313,7 @@ def bench_decode(device, steps, warmup, n_layers=10):
                 timed[name]["board_under_replay"] = board_state_under(graph.replay)
             del graph
         best = min(timed, key=lambda n: timed[n]["ms"])
-        res[f"T{T}"] = dict(ms=timed[best]["ms"], path=best, launches_per_layer=4 if rules().decode_by_gemms(T, k, E, f2 // 2, d) else 3 if best != "moe_mlp"
-                            else 2 if rules().decode_by_rows(T, k, f2 // 2, d) else 1,
+        res[f"T{T}"] = dict(ms=timed[best]["ms"], path=best, launches_per_layer=3 if best != "moe_mlp" else 2 if rules().decode_by_rows(T, k, f2 // 2, d) else 1,
                             active_experts=active, weight_GB=round(gbytes, 4), GBps=timed[best]["GBps"], frac_hbm=timed[best]["frac_hbm"],
                             layers_per_graph=n_layers, rotated_weight_GB=round(gbytes * n_layers, 3), **{n: timed[n] for n in timed})
     return res

@@ -473,6 +473,22 @@ def test_fused_combine_with_many_row_blocks_on_one_expert(api, device, gptoss_we
         assert outside(got) <= outside(want) + LAYER_GATE_SLACK * ref.numel()
 
 
+@pytest.mark.parametrize("T", [1, 16, 25, 64])
+def test_up_to_256_rows_ask_for_the_fused_combine(api, device, gptoss_weights, monkeypatch, T):
+    """What the tests of the combine inside the decode GEMM run: its row blocks, with the sum over a token's rows in the same launch."""
+    from triton_amd import _native as nt
+    g = torch.Generator().manual_seed(T)
+    E, k, d = 128, 4, 2880
+    W = gptoss_weights["tiled"]
+    rdata, _, scatter = api.routing(torch.randn((T, E), generator=g).to(device), k)
+    h = torch.randn((T * k, d), generator=g).to(torch.bfloat16).to(device)
+    asked, real = [], nt.submit
+    monkeypatch.setattr(nt, "host", lambda: None)
+    monkeypatch.setattr(nt, "submit", lambda entry, desc, *a, **kw: (asked.append((desc.block_m, desc.block_n, desc.combine_k)), real(entry, desc, *a, **kw))[1])
+    api.matmul_ogs(h, W["w2"], W["b2"], rdata, scatter_indx=scatter, gammas=rdata.gate_scal, precision_config=api.PrecisionConfig(b_mx_scale=W["w2s"]))
+    assert asked == [(16, 0, k)]
+
+
 def test_config5_full_shape_sampled_tokens(api, device):
     """Benchmark config 5 at its real shape: the FINAL output rows of six sampled tokens, i.e. the second GEMM at
     K = 14336 with per-token and per-channel scales, the gate weight, the scatter and the combine over the eight

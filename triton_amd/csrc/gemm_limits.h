@@ -136,18 +136,4 @@ inline bool decode_by_rows(int64_t T, int64_t k, int64_t d_ff, int64_t d_model) 
   return k <= kDecRowsMaxK && T * k <= kRowsMax && T * k * (expert_bytes + kRowBytes) + T * parts(d_model, 16) * kWorkgroupBytes <= kRowsBytes;
 }
 
-// Calls of up to 256 rows that the wide MXFP4 kernel takes as well: beyond 96 rows (below, the decode kernel), and tiles for half of the CUs at least
-// if every slice has rows (one slice's columns are too few for tiles of 256, and the decode kernel also divides K).
-inline bool mxw_few(int64_t rows, int64_t n_slices, int64_t N) { return rows > 96 && n_slices <= kDmaSlices && n_slices * ((N + 255) / 256) >= 128; }
-
-// A decode layer (T tokens, k experts each) as router, two GEMMs of the wide kernel and combine instead of one launch: four launches cost about 25 us around their
-// streams where the single launch costs 30 and streams slower, the more so the more experts have rows (a 16-row unit each, and a second unit reads its weights
-// again).  Measured (us of a layer, single launch / the calls): 128 experts, d and d_ff 2880, top 4, routing with favourites: 16 tokens 78 / 84, 24 86 / 87, 32 91 / 89,
-// 48 105 / 100, 61 122 / 109; all experts alike: 24 184 / 167, 40 240 / 211, 64 299 / 256; 64 experts, 2048: 32 tokens 90 / 80, 64 102 / 87; with
-// favourites 66 / 53; 32 experts, 1536, top 8, 32 tokens 49 / 42; 32 experts, 1024, top 4, 64 tokens 41 / 30.
-// (A k that is no power of two has only the single launch.)
-inline bool decode_by_gemms(int64_t T, int64_t k, int64_t n_experts, int64_t d_ff, int64_t d_model) {
-  return k > 0 && (k & (k - 1)) == 0 && d_ff > 384 && d_model > 384 && mxw_few(T * k, n_experts, 2 * d_ff) && mxw_few(T * k, n_experts, d_model);
-}
-
 }  // namespace tk

@@ -449,9 +449,9 @@ PyObject* run_gemm(PyObject* const* v) {
     block_m = wide_block_m(M, n_slices, K, x_bytes, true);
     block_n = wide_block_n(M, n_slices, K, N, x_bytes, true);
   } else if (tiled) {
-    if (x_bytes && n_slices <= tk::kDmaSlices && !x_row && !w_col) {
-      if (n_out % 8 == 0 && (M > 256 || tk::mxw_few(M, n_slices, N))) block_n = wide_block_n(M, n_slices, K, N, x_bytes, false);
-      if (M > 256 || block_n) block_m = mxfp4_block_m(M, n_slices, block_m);
+    if (M > 256 && x_bytes && n_slices <= tk::kDmaSlices && !x_row && !w_col) {
+      block_m = mxfp4_block_m(M, n_slices, block_m);
+      if (n_out % 8 == 0) block_n = wide_block_n(M, n_slices, K, N, x_bytes, false);
     }
     if (block_m == 128) block_m = wide_block_m(M, n_slices, K, x_bytes, false);
   } else if (tk::dma_runs_16bit(x_bytes, n_slices, K, N, w->stride(2))) {
@@ -851,14 +851,6 @@ PyObject* rule_decode_rows(PyObject* const* v) {
   const auto [T, k, d_ff, d_model] = integers<4>(v);
   return PyBool_FromLong(tk::decode_by_rows(T, k, d_ff, d_model));
 }
-PyObject* rule_decode_gemms(PyObject* const* v) {
-  const auto [T, k, n_experts, d_ff, d_model] = integers<5>(v);
-  return PyBool_FromLong(tk::decode_by_gemms(T, k, n_experts, d_ff, d_model));
-}
-PyObject* rule_mxw_few(PyObject* const* v) {
-  const auto [rows, n_slices, N] = integers<3>(v);
-  return PyBool_FromLong(tk::mxw_few(rows, n_slices, N));
-}
 PyObject* rule_fp8(PyObject* const* v) {
   const auto [rows, x_bytes, K, N, n_slices] = integers<5>(v);
   return PyLong_FromLongLong(fp8_block_m(rows, uint32_t(x_bytes), K, N, n_slices));
@@ -931,8 +923,6 @@ PyMethodDef methods[] = {
     METHOD("dma_block_n_16bit", rule_dma_n_16bit, 4),
     METHOD("few_block_n", rule_few, 3),
     METHOD("decode_by_rows", rule_decode_rows, 4),
-    METHOD("decode_by_gemms", rule_decode_gemms, 5),
-    METHOD("mxw_few", rule_mxw_few, 3),
     METHOD("fp8_block_m", rule_fp8, 5),
     METHOD("mxfp4_block_m", rule_mxfp4, 3),
     METHOD("wide_block_m", rule_wide, 5),

@@ -769,12 +769,11 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
         if extras:
             block_m = min(block_m, 32)  # the decode kernel carries the shared epilogue; the prefill kernels do not take these options
         elif forced is None and is_ragged:
-            if (x_bytes and n_slices <= 256 and a_ts is None and b_ts is None
+            if (M > 256 and x_bytes and n_slices <= 256 and a_ts is None and b_ts is None
                     and a_ragged_metadata.expected_slice_size is None):
-                if out_shape[1] % 8 == 0 and (M > 256 or nt.rules().mxw_few(M, n_slices, N)):
+                block_m = nt.rules().mxfp4_block_m(M, n_slices, block_m)
+                if out_shape[1] % 8 == 0:
                     d.block_n = nt.rules().wide_block_n(M, n_slices, K, N, x_bytes, 0)
-                if M > 256 or d.block_n:
-                    block_m = nt.rules().mxfp4_block_m(M, n_slices, block_m)
             if block_m == 128:
                 block_m = nt.rules().wide_block_m(M, n_slices, K, x_bytes, 0)
     elif w_dtype in (_BF16, _F16):

@@ -9,7 +9,7 @@ The reference's MoE block is a sequence of calls (python/triton_kernels/bench/be
 `moe_mlp` computes the same `out` from the same arguments.  With a handful of tokens (T * k <= 256 routed rows), tiled
 MXFP4 weights and d_model, d_ff <= 3072 it is ONE kernel launch (`tk_moe_decode_layer`: router, both expert GEMMs and
 the top-k combine in a persistent grid), or two where the rows' weights are a small stream (one GEMM each, routed and combined
-inside); any other case runs the three calls above, as do more than 96 rows of enough experts (`decode_by_gemms` in csrc/gemm_limits.h).  At these sizes the layer is a
+inside); any other case runs the three calls above.  At these sizes the layer is a
 stream of the active experts' weights, and launch boundaries plus the serial router in front of the first weight byte
 cost a third of the three-call time.
 """
@@ -60,11 +60,11 @@ def _workspace(device, T, k, E, d_ff, d_model) -> torch.Tensor:
 
 def workspace_error_word(x, logits, n_expts_act, w1) -> int:
     """The sticky error word of the workspace `moe_mlp` uses for these arguments on the current stream (synchronises;
-    for tests): 0 = fine, bit 0 = a bounded wait ran out, bit 1 = the unit table overflowed.  A layer that goes row by row or as
-    calls waits for nothing and has none: 0."""
+    for tests): 0 = fine, bit 0 = a bounded wait ran out, bit 1 = the unit table overflowed.  A layer that goes row by row waits for
+    nothing and has none: 0."""
     T, E = logits.shape
     d_model, n1 = w1.shape[-2:]
-    if nt.rules().decode_by_rows(T, n_expts_act, n1 // 2, d_model) or _by_gemms(logits, n_expts_act, n1 // 2, d_model):
+    if nt.rules().decode_by_rows(T, n_expts_act, n1 // 2, d_model):
         return 0
     ws = _workspace(x.device, T, n_expts_act, E, n1 // 2, d_model)
     words = ws[-(2 + (MAX_ROWS + MAX_ROWS // 16) * 32 + T * ((d_model + 31) // 32)) * 4:].view(torch.int32)
@@ -118,22 +118,9 @@ def one_launch_reason(x, logits, n_expts_act, w1, b1, w2, b2, pc1, pc2, act) -> 
     return None
 
 
-def _by_gemms(logits, k, d_ff, d_model) -> bool:
-    """Whether a layer that one launch could run goes as the three calls (with bf16 logits those round the gate values to bf16, which the launch does not)."""
-    T, E = logits.shape
-    return T * k > 96 and logits.dtype == torch.float32 and nt.rules().decode_by_gemms(T, k, E, d_ff, d_model)
-
-
-def _calls(x, logits, k, w1, b1, w2, b2, pc1, pc2, act, apply_softmax):
-    rdata, gather, scatter = routing(logits, k, apply_softmax)
-    h = matmul_ogs(x, w1, b1, rdata, gather_indx=gather, precision_config=pc1, fused_activation=act)
-    out = matmul_ogs(h, w2, b2, rdata, scatter_indx=scatter, precision_config=pc2, gammas=rdata.gate_scal)
-    return out, rdata
-
-
 def moe_decode_layer(x, logits, n_expts_act, w1, b1, w2, b2, pc1: PrecisionConfig, pc2: PrecisionConfig,
                      fused_activation: FusedActivation, *, apply_softmax: bool = True, out=None, return_routing: bool = False):
-    """The layer in one launch, two where it goes row by row, or (without `out`) the three calls where those are faster; raises NotImplementedError when `one_launch_reason` names an obstacle."""
+    """The layer in one launch, or two where it goes row by row; raises NotImplementedError when `one_launch_reason` names an obstacle."""
     why = one_launch_reason(x, logits, n_expts_act, w1, b1, w2, b2, pc1, pc2, fused_activation)
     if why is not None:
         raise NotImplementedError(f"moe_decode_layer: {why}")
@@ -141,9 +128,6 @@ def moe_decode_layer(x, logits, n_expts_act, w1, b1, w2, b2, pc1: PrecisionConfi
     k = n_expts_act
     d_model, n1 = w1.shape[-2:]
     d_ff = n1 // 2
-    if out is None and _by_gemms(logits, k, d_ff, d_model):
-        out, rdata = _calls(x, logits, k, w1, b1, w2, b2, pc1, pc2, fused_activation, apply_softmax)
-        return (out, rdata.expt_indx, rdata.gate_vals) if return_routing else out
     alpha, limit, has_limit = _swiglu_args(fused_activation)
     if x.stride(-1) != 1:
         x = x.contiguous()
@@ -195,11 +179,10 @@ def moe_decode_layer(x, logits, n_expts_act, w1, b1, w2, b2, pc1: PrecisionConfi
 def moe_mlp(x, logits, n_expts_act, w1, b1, w2, b2, pc1: PrecisionConfig, pc2: PrecisionConfig,
             fused_activation: FusedActivation):
     """`routing` + gather-`matmul_ogs` (+ fused activation) + scatter-`matmul_ogs` (gate weighted, k rows summed) as one
-    call: one or two kernel launches for a few rows, the three calls otherwise.  Returns `[tokens, d_model]`."""
+    call: one or two kernel launches at decode sizes, the three calls otherwise.  Returns `[tokens, d_model]`."""
     rows = logits.shape[0] * n_expts_act
     # (up to 7 rows only with a k that `routing` takes: other k are refused there at every size)
-    if (MIN_ROWS <= rows <= MAX_ROWS and (rows > 7 or n_expts_act & (n_expts_act - 1) == 0)
-            and not _by_gemms(logits, n_expts_act, w2.shape[-2], x.shape[-1])):
+    if MIN_ROWS <= rows <= MAX_ROWS and (rows > 7 or n_expts_act & (n_expts_act - 1) == 0):
         host = nt.host()
         out = None
         if host is not None:
@@ -208,4 +191,6 @@ def moe_mlp(x, logits, n_expts_act, w1, b1, w2, b2, pc1: PrecisionConfig, pc2: P
             out = moe_decode_layer(x, logits, n_expts_act, w1, b1, w2, b2, pc1, pc2, fused_activation)
         if out is not None:
             return out
-    return _calls(x, logits, n_expts_act, w1, b1, w2, b2, pc1, pc2, fused_activation, True)[0]
+    rdata, gather, scatter = routing(logits, n_expts_act)
+    h = matmul_ogs(x, w1, b1, rdata, gather_indx=gather, precision_config=pc1, fused_activation=fused_activation)
+    return matmul_ogs(h, w2, b2, rdata, scatter_indx=scatter, precision_config=pc2, gammas=rdata.gate_scal)
