@@ -274,10 +274,18 @@ __global__ __launch_bounds__(NW_ * 64, 2) void moe_gemm_mxw_kernel(const GemmPar
       // loop's other paths, and the compiler puts a wait for everything outstanding into every stage.)
       if (s == nst - AA - 1) {
         more = tile + t_step < t_end;
-        if (more) nxt = locate(tile + t_step);
-        request(nxt);
-        arrived();
-        park(nxt, set ^ 1);
+        if (more) {
+          nxt = locate(tile + t_step);
+          request(nxt);
+          arrived();
+          park(nxt, set ^ 1);
+        } else {
+          // (behind the last tile nothing is fetched: the words' wait, which is one for everything, cost products of one round 3 to 5 %, 64 slices of 8 bf16
+          // rows, K 2880, N 512 21.2 us against 20.5, a layer of 1000 MXFP8 rows 102.5 against 99.9; the words get a value so that the old ones need no registers until here)
+#pragma unroll
+          for (int i = 0; i < AI; ++i) raw_src[i] = 0;
+          raw_xs = 0;
+        }
       } else if (s == nst - AA) {
         aim(nxt);
       }
