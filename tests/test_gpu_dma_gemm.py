@@ -203,3 +203,40 @@ def test_tiles_of_320_rows(device, monkeypatch, tile, e, k, n, sizes, dtype, swi
         want = run()
     assert torch.equal(by_rule, want) and torch.equal(general, want)
     assert not torch.isnan(want).any() and want.any()
+
+
+@pytest.mark.parametrize("e, k, n, sizes", [
+    (16, 136, 2048, [1100, 20, 0, 511, 130, 1, 700, 31, 257, 640, 90, 320, 5, 0, 33, 258]),  # where 320 x 128 is more than a round
+    (32, 72, 2312, [700, 129, 1, 384, 0, 256, 33, 512]),                                     # 320 x 256: full square tiles, short ones beside them
+    (16, 400, 4096, [257, 384, 320, 0, 31, 256, 512, 230]),                                  # ... and in narrow tiles behind them
+])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float16"])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_square_tiles_where_a_routing_divides_worse_into_tall_ones(device, dtype, e, k, n, sizes, swiglu):
+    """The rows that a tile of 320 is meant for, dealt so that the kernel goes by 256 x 256 tiles: against the oracle on a row of every row block's kind."""
+    import triton_amd.matmul as mm
+    from triton_amd import _native as nt
+    from triton_amd.swiglu import swiglu_fn
+    from triton_amd.tensor import make_ragged_tensor_metadata
+    sizes = [sizes[i % len(sizes)] for i in range(e)]
+    m, dt = sum(sizes), getattr(torch, dtype)
+    cols = nt.rules().dma_block_n_16bit(m, n, e, 256)
+    assert cols in (128, 256)
+    tall, square = (sum(-(-s // b) for s in sizes) * -(-n // c) / 256 for b, c in ((320, cols), (256, 256)))  # rounds on 256 compute units
+    assert (tall > 1) if cols == 128 else 0.73 * square < (tall if tall < 1 else int(tall) + (0.43 if tall > int(tall) else 0))
+    g = torch.Generator(device=device).manual_seed(k + n)
+    x = torch.randn((m, k), generator=g, device=device).to(dt)
+    w = (torch.randn((e, n, k), generator=g, device=device) * 0.1).to(dt).transpose(1, 2)
+    bias, gam = torch.randn((e, n), generator=g, device=device), torch.rand((m, ), generator=g, device=device) + 0.5
+    gi, sc = torch.randint(0, m, (m, ), generator=g, device=device).to(torch.int32), torch.randperm(m, generator=g, device=device).to(torch.int32)
+    act = mm.FusedActivation(mm.FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0)) if swiglu else None
+    out = torch.full((m, n // 2 if swiglu else n), float("nan"), dtype=dt, device=device)
+    mm.matmul(x, w, bias, make_ragged_tensor_metadata(torch.tensor(sizes, dtype=torch.int32, device=device), m), gather_indx=gi, scatter_indx=sc, gammas=gam, fused_activation=act, c=out)
+    assert not torch.isnan(out).any()
+    first = [sum(sizes[:i]) for i in range(e)]
+    pick = sorted({r for i, s in enumerate(sizes) for r in (first[i], first[i] + s // 2, first[i] + s - 1) if s})
+    counts = torch.tensor([sum(first[i] <= r < first[i] + s for r in pick) for i, s in enumerate(sizes)], dtype=torch.int32)
+    rows = torch.tensor(pick)
+    ref = omoe.matmul(x.cpu(), w.cpu(), bias.cpu(), counts, gather_indx=gi.cpu()[rows], out_dtype=torch.float32)
+    ref = (omoe.swiglu(ref, 1.702, 7.0).float() if swiglu else ref) * gam.cpu()[rows][:, None]
+    assert_allclose_gate(ref, out.cpu()[sc.cpu()[rows].long()], what=f"{dtype} square tiles")

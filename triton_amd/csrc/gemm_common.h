@@ -78,6 +78,7 @@ struct GemmParams {
 // one entry per kernel family; each returns a TK_* status
 int32_t gemm_launch_strided(const GemmParams& p, int wk, int block_m, int grid_m, bool swiglu, hipStream_t st);
 int32_t gemm_launch_dma(const GemmParams& p, int wk, DmaTile tile, int grid_m, bool swiglu, hipStream_t st);  // 128 x 128, 256 x 256, dma_tile
+int32_t gemm_launch_dma_tall(const GemmParams& p, int wk, DmaTile tile, int grid_m, bool swiglu, hipStream_t st);  // dma_tile, 16-bit operands
 int32_t gemm_launch_few(const GemmParams& p, int wk, int block_n, bool swiglu, hipStream_t st);  // block_n 32 / 64
 int32_t gemm_launch_mxn(const GemmParams& p, int block_m, int grid_m, bool swiglu, hipStream_t st);
 int32_t gemm_launch_mxn_mx(const GemmParams& p, int block_m, int grid_m, bool swiglu, hipStream_t st);  // block_m 128 / 256, MX-quantised output

@@ -90,7 +90,7 @@ inline MxwTile mxw_tile(int64_t rows, int64_t n_slices, int64_t N, bool mx8) {
   return rows <= 48 * n_slices ? MxwTile{64, 512} : rows <= 80 * n_slices ? MxwTile{96, 512} : MxwTile{160, 512};
 }
 
-// Tile of the memory-to-LDS kernel (moe_gemm_dma.hip) for 16-bit operands in place of 256 x 256 ones: 320 rows, so that a slice of about 256 rows, of which
+// Tile of the memory-to-LDS kernel (moe_gemm_dma_kernel.h) for 16-bit operands beside 256 x 256 ones: 320 rows, so that a slice of about 256 rows, of which
 // a random routing makes half a few longer, is one row block.  (An eighth above the mean is 2.5 deviations at 400 rows, 2 at 256.)  rows 0 = those.
 //   320 x 128 where its tiles are one round and 128 x 128 ones (up to 96 of 256 x 256, dma_block_n) are not better; 320 x 256 beyond, from 248 rows on.
 // Measured (us of a GEMM with a random routing, 256 x 256 / 320 x 256 / 320 x 128; slices, K, N):
@@ -99,7 +99,8 @@ inline MxwTile mxw_tile(int64_t rows, int64_t n_slices, int64_t N, bool mx8) {
 //   16, 2880, 2880: 240 rows 89 / 101 / 108, 256 111 / 102 / 111, 272 127 / 107 / 128; 32, 2048, 4096: 240 175 / 182 / 176, 256 225 / 184 / 181, 288 280 /
 //   229 / 232; 32, 1024, 2048: 224 48 / 50 / 55, 256 65 / 55 / 59; 8, 4096, 4096: 224 102 / 120 / 83, 256 101 / 124 / 84, 272 103 / 132 / 108
 //   8, 2048, 2048 (128 x 128 / 320 x 128): 256 30 / 34; 272 (256 x 256) 43 / 35; two blocks: 448 45 / 41, 544 47 / 43, 608 49 / 55
-// (Slices that all have 256 rows to the row are as fast in the tiles of 256 or faster; how a routing divides the rows is not known here.)
+// (Slices that all have 256 rows to the row, or with favourites any number, are faster in the tiles of 256.  How a routing divides the rows is not known
+// here: the kernel counts both kinds of tiles and goes on with the better one, moe_gemm_dma_tall.hip.)
 struct DmaTile {
   int32_t rows, cols;
 };

@@ -31,8 +31,8 @@ struct TileList {
   static __device__ __forceinline__ int n_full(int rows) { return (rows + BM / 2 - 1) / BM; }
   static __device__ __forceinline__ int n_short(int rows) { return rows > n_full(rows) * BM ? 1 : 0; }
 
-  // returns this workgroup's first index (it has none if that is not below t_end; the following ones are t_step apart)
-  __device__ __forceinline__ int init(const GemmParams& p, int lane) {
+  // n_cols = tiles of a row block; returns this workgroup's first index (it has none if that is not below t_end; the following ones are t_step apart)
+  __device__ __forceinline__ int init(const GemmParams& p, int lane, int n_cols) {
     int full = 0, brief = 0;
 #pragma unroll
     for (int c = 0; c < kSliceRegs; ++c) {
@@ -52,7 +52,7 @@ struct TileList {
       full += __builtin_amdgcn_readlane(wave_scan_i32(n_full(sz[c])), 63);
       brief += __builtin_amdgcn_readlane(wave_scan_i32(n_short(sz[c])), 63);
     }
-    grid_n = p.grid_n;
+    grid_n = n_cols;
     if constexpr (SBN < BN) {
       const uint32_t wgs = gridDim.x, over = (uint32_t)(full * grid_n) % wgs, wide = (uint32_t)(brief * grid_n);
       if (wide > (over ? wgs - over : 0) && wide * 2 <= wgs) grid_s = (p.N + SBN - 1) / SBN;

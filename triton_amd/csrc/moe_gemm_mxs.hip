@@ -44,7 +44,7 @@ __global__ __launch_bounds__(MxsCfg::NW * 64, 2) void moe_gemm_mxs_kernel(const 
   const uint32_t lds0 = lds_addr(lds);
 
   TileList<C::BM, C::BN> tiles;
-  int tile = tiles.init(p, lane);
+  int tile = tiles.init(p, lane, p.grid_n);
   const int t_step = tiles.t_step, t_end = tiles.t_end;
   if (tile >= t_end) return;
 

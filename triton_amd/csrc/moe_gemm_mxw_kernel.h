@@ -74,7 +74,7 @@ __global__ __launch_bounds__(NW_ * 64, 2) void moe_gemm_mxw_kernel(const GemmPar
   int* const lists = reinterpret_cast<int*>(lds + C::RINGS + 2 * (C::SIDE + C::OPERANDS));
   typedef TileList<C::BM, C::BN> Tiles;
   Tiles list;
-  int tile = list.init(p, lane);
+  int tile = list.init(p, lane, p.grid_n);
   const int t_step = list.t_step, t_end = list.t_end, f_beg = list.f_beg, f_len = list.f_len, s_beg = list.s_beg;
   if (tile >= t_end) return;
   Tile cur = list.locate(tile), nxt = cur;
