@@ -328,11 +328,9 @@ typedef struct tk_gemm_desc {
    * NULL = plain bf16 output.  Other operand combinations quantise in a second pass (tk_mx_downcast on the bf16 result). */
   void* y_mx_scale;
   int64_t ys_stride_m;
-  /* Fused top-k combine behind the scatter (bf16 activations, tiled MXFP4 weights, no activation).  At block_m >= 64
-   * the persistent kernel sums when all its workgroups have written their tiles (a device-wide arrival count in words
-   * 9..31 of tile_counters, which must be given; word 11 is raised, and stays, if a bounded wait for the other
-   * workgroups runs out; combine_counters is not used; N % 8 == 0, 16-byte aligned rows of combine_out, and the
-   * launch must not share the GPU with another launch that waits for its own workgroups).  At block_m 16 or 32:
+  /* Top-k combine behind the scatter (bf16 activations, tiled MXFP4 weights, no activation).  At block_m >= 64 it is a
+   * launch of its own behind the GEMM's (tk_reduce_mid; tile_counters must be given, combine_counters is not used; N % 8
+   * == 0, 16-byte aligned rows of combine_out).  At block_m 16 or 32 it is part of the GEMM's launch:
    * scatter_indx maps expert-sorted row r to flat position t * combine_k + j; besides y [tokens * combine_k, N] the
    * kernel writes combine_out[t, :] = sum over j of y[t * combine_k + j, :] (fp32 sum in j order, bf16 result: what
    * tk_reduce_mid computes from y), by the wave that completes token t's rows last.  combine_counters:

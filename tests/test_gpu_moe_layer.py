@@ -588,10 +588,8 @@ def test_config3_full_shape_mxfp8_activations_sampled_tokens(api, device, gptoss
 
 @pytest.mark.parametrize("T", [300, 4096])
 def test_fused_combine_at_prefill_equals_reduce(api, device, gptoss_weights, T):
-    """At prefill shapes `matmul_ogs(..., scatter_indx=...)` sums the k rows of every token at the end of the second
-    GEMM's own launch (the persistent grid waits until all its workgroups have written their tiles).  Bit-equal to
-    `reduce` over the scattered rows, three calls in a row on the same counters (left clean), error word clear."""
-    import triton_amd.matmul as mm
+    """At prefill shapes `matmul_ogs(..., scatter_indx=...)` sums the k rows of every token by a launch behind the second GEMM, from the same
+    native call.  Bit-equal to `reduce` over the scattered rows, three calls in a row."""
     g = torch.Generator().manual_seed(6 + T)
     E, k, d = 128, 4, 2880
     x = torch.randn((T, d), generator=g).to(torch.bfloat16).to(device)
@@ -606,9 +604,37 @@ def test_fused_combine_at_prefill_equals_reduce(api, device, gptoss_weights, T):
     for rep in range(3):
         got = api.matmul_ogs(h, W["w2"], W["b2"], rdata, scatter_indx=scatter, precision_config=pc2, gammas=rdata.gate_scal)
         assert got.shape == (T, d)
-        assert torch.equal(got, want), f"call {rep}: fused combine differs from reduce"
-    ctr = mm._tile_counters(device).cpu()
-    assert int(ctr[9]) == 0 and int(ctr[10]) == 0 and int(ctr[11]) == 0, f"tile counters after the launches: {ctr.tolist()}"
+        assert torch.equal(got, want), f"call {rep}: combine differs from reduce"
+
+
+@pytest.mark.parametrize("block_m", [64, 128, 256])
+def test_combine_asked_of_the_gemm_at_row_blocks_of_64_and_more(api, device, gptoss_weights, monkeypatch, block_m):
+    """`combine_k` in the descriptor of a GEMM in row blocks of 64, 128 and 256: the call writes the sums beside the scattered rows, bit-equal to `reduce`
+    over them, twice on the same counters, which it leaves zero."""
+    import triton_amd.matmul as mm
+    from triton_amd import _native as nt
+    from triton_amd.matmul_details.opt_flags import scoped_opt_flags_constraints
+    g = torch.Generator().manual_seed(block_m)
+    T, E, k, d = 300, 128, 4, 2880
+    W = gptoss_weights["tiled"]
+    rdata, _, scatter = api.routing(torch.randn((T, E), generator=g).to(device), k)
+    h = torch.randn((T * k, d), generator=g).to(torch.bfloat16).to(device)
+    sums, asked, real = torch.full((T, d), float("nan"), dtype=torch.bfloat16, device=device), [], nt.submit
+
+    def submit(entry, desc, *a, **kw):
+        desc.combine_k, desc.combine_out, desc.combine_stride_m = k, sums.data_ptr(), d
+        asked.append((desc.block_m, bool(desc.tile_counters)))
+        return real(entry, desc, *a, **kw)
+
+    monkeypatch.setattr(nt, "host", lambda: None)
+    monkeypatch.setattr(nt, "submit", submit)
+    for rep in range(2):
+        sums.fill_(float("nan"))
+        with scoped_opt_flags_constraints({"block_m": block_m}):
+            y = api.matmul(h, W["w2"], W["b2"], rdata.expt_data, scatter_indx=scatter.dst_indx, gammas=rdata.gate_scal,
+                           precision_config=api.PrecisionConfig(b_mx_scale=W["w2s"]))
+        assert torch.equal(sums, api.reduce(y.view(T, k, -1), dim=1)[0]) and not torch.isnan(sums).any()
+    assert asked == [(block_m, True)] * 2 and not mm._tile_counters(device).any()
 
 
 @pytest.mark.parametrize("T", [300, 4096])

@@ -53,7 +53,7 @@ struct GemmParams {
   int32_t w_nst;     // tile-native weight layout: K-stages of 128 per column fragment
   int32_t total_tiles;  // persistent kernels, non-ragged case: row blocks x column tiles
   int32_t idle_cus;     // persistent kernels: compute units to leave without a workgroup
-  int32_t* tile_counters;  // persistent kernels: 32 zeroed words (tile claiming: 0..8; prefill combine: 9..31), or null
+  int32_t* tile_counters;  // persistent kernels: zeroed words for tile claiming (0..8), or null
   uint32_t y_bytes;        // persistent MXFP4 kernels: bytes of the output buffer that rows may be written to (< 2 GiB)
   int32_t combine_k;          // decode kernel: > 0 = sum the k rows of every token into combine_out (fused top-k combine)
   uint16_t* combine_out;      // bf16 [tokens, N]
@@ -755,110 +755,6 @@ __device__ __forceinline__ void staged_mx_epilogue(const GemmParams& p, f32x16_t
           }
         }
       }
-    }
-  }
-}
-
-
-// Top-k combine behind the scatter of a persistent prefill kernel (reduce.py:1143-1165 after matmul_details/_matmul.py:535-569 in the reference,
-// a launch of its own there): out[t, :] = sum over j of y[t * k + j, :], fp32 in j order, bf16 result.  The k rows of a
-// token come from k experts, i.e. from tiles of workgroups all over the chip, so the sum runs when EVERY workgroup
-// has written its tiles: the grid is persistent and fits the GPU (one workgroup per CU).
-//   1. a workgroup whose stores have all reached its XCD's L2 counts itself in (per XCD and in total);
-//   2. when all have, ONE workgroup per XCD (the first to claim it) has that L2 write its dirty lines back (a release
-//      fence; one per L2, not one per wave: every fence walks the whole cache) and reports it;
-//   3. when every XCD in use has reported, the rows of y are in memory: the workgroups sum the tokens blockIdx.x,
-//      blockIdx.x + grid, ..., reading y around their own L2 (sc0 sc1: lines another XCD wrote are not coherent in it);
-//   4. the last workgroup to leave clears the words for the next launch.
-// Words of `tile_counters`: 9 arrivals, 10 departures, 11 error (raised, and kept, if a bounded wait runs out),
-// 12 XCDs in use, 13 XCDs written back, 16..23 arrivals per XCD, 24..31 write-back claimed per XCD.
-template <int NT>
-__device__ __forceinline__ void fused_prefill_combine(const GemmParams& p, int tid, int grid) {
-  const int N = p.N;
-  int32_t* ctr = p.tile_counters;
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  if (tid == 0) {
-    int xcc;
-    asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
-    xcc &= 7;
-    auto wait_for = [&](int32_t* word, int want) {
-      int spins = 0;
-      while (__hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < want) {
-        __builtin_amdgcn_s_sleep(16);
-        if (++spins > (1 << 22)) {
-          atomicOr(&ctr[11], 1);
-          break;
-        }
-      }
-    };
-    if (__hip_atomic_fetch_add(&ctr[16 + xcc], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0)
-      __hip_atomic_fetch_add(&ctr[12], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __hip_atomic_fetch_add(&ctr[9], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    wait_for(&ctr[9], grid);
-    if (__hip_atomic_fetch_add(&ctr[24 + xcc], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // this XCD's L2 writes back its dirty lines
-      __hip_atomic_fetch_add(&ctr[13], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    wait_for(&ctr[13], __hip_atomic_load(&ctr[12], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-  }
-  __syncthreads();
-  const int k = p.combine_k, T = p.scatter_len / k;
-  const int n8 = N >> 3;  // (N is a multiple of 8: host check)
-  const __amdgpu_buffer_rsrc_t ysrc = __builtin_amdgcn_make_buffer_rsrc(p.y, 0, p.y_bytes, 0x00020000);
-  const uint32_t row_bytes = (uint32_t)(p.y_stride_m * 2);
-  constexpr int kAround = 1 | 16;  // sc0 | sc1
-  // The tokens of this workgroup and their 8-column groups form one index space, H items of it per lane and pass:
-  // their rows are all requested before any is summed (4 * H 16-byte loads in flight per lane when k <= 4).
-  constexpr int H = 2;
-  const int n_tok = blockIdx.x < T ? (T - 1 - blockIdx.x) / grid + 1 : 0;
-  const int items = n_tok * n8;
-  for (int i0 = tid; i0 < items; i0 += H * NT) {
-    int tt[H], cc[H];
-#pragma unroll
-    for (int h = 0; h < H; ++h) {
-      const int i = i0 + h * NT;
-      const int lt = i / n8;
-      tt[h] = i < items ? blockIdx.x + lt * grid : -1;
-      cc[h] = i - lt * n8;
-    }
-    float sum[H][8];
-#pragma unroll
-    for (int h = 0; h < H; ++h)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) sum[h][e] = 0.f;
-    for (int j0 = 0; j0 < k; j0 += 4) {
-      u32x4_t v[H][4];
-#pragma unroll
-      for (int h = 0; h < H; ++h)
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          const uint32_t off =
-              (tt[h] >= 0 && j0 + q < k) ? (uint32_t)(tt[h] * k + j0 + q) * row_bytes + (uint32_t)cc[h] * 16u : kDroppedStore;
-          v[h][q] = __builtin_amdgcn_raw_buffer_load_b128(ysrc, off, 0, kAround);  // (dropped offsets read zero)
-        }
-#pragma unroll
-      for (int h = 0; h < H; ++h)
-#pragma unroll
-        for (int q = 0; q < 4; ++q)
-#pragma unroll
-          for (int e = 0; e < 4; ++e) {
-            sum[h][2 * e] += bits_f32(v[h][q][e] << 16);
-            sum[h][2 * e + 1] += bits_f32(v[h][q][e] & 0xFFFF0000u);
-          }
-    }
-#pragma unroll
-    for (int h = 0; h < H; ++h)
-      if (tt[h] >= 0)
-        *reinterpret_cast<u32x4_t*>(p.combine_out + (int64_t)tt[h] * p.combine_stride + cc[h] * 8) =
-            u32x4_t{pack_bf16x2(sum[h][0], sum[h][1]), pack_bf16x2(sum[h][2], sum[h][3]), pack_bf16x2(sum[h][4], sum[h][5]),
-                    pack_bf16x2(sum[h][6], sum[h][7])};
-  }
-  __syncthreads();
-  if (tid == 0) {
-    if (__hip_atomic_fetch_add(&ctr[10], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == grid - 1) {
-      for (int w = 9; w < 32; ++w)
-        if (w != 11) __hip_atomic_store(&ctr[w], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
   }
 }

@@ -499,9 +499,7 @@ PyObject* run_gemm(PyObject* const* v) {
     return static_cast<int32_t*>(THPVariable_Unpack(t.p).data_ptr());  // (kept for the life of the process)
   };
   if ((tiled || tiled_fp8) && block_m >= 64 && !mx_act) d.tile_counters = words(B.tile_counters, true);
-  // the combine inside the launch, by the wave that completes a token's rows: the decode kernel only.  (The prefill kernel for row blocks of 64 and 128
-  // can sum at the end of its persistent grid, which costs more than a launch: 96 slices of 39 rows, N 1088 79 us against 33 and 5, 32 slices of 64
-  // rows, N 1536 56 against 21 and 4, 128 slices of 29 rows, N 2880 167 against 140 and 10.)
+  // the combine inside the launch, by the wave that completes a token's rows: the decode kernel only
   if (combine_k > 0 && tiled && !mx_act && !act.swiglu && scatter && y_rows % combine_k == 0 && block_m == 16
       && (y_rows / combine_k) * ((N + 31) / 32) <= (1 << 16)) {
     combined = empty({y_rows / combine_k, N}, out, *a);

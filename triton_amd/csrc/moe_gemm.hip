@@ -45,7 +45,8 @@ static MxwTile wide_tile(const GemmParams& p, const tk_gemm_desc* d, bool mx8) {
   return d->block_m == 256 ? MxwTile{160, 512} : MxwTile{0, 0};
 }
 
-extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
+// tk_moe_gemm but for the top-k combine behind row blocks of 64 and more.
+static int32_t moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
   if (!d) return fail(TK_ERR_INVALID, "tk_moe_gemm: null descriptor");
   if (d->M < 0 || d->N < 0 || d->K < 0) return fail(TK_ERR_INVALID, "tk_moe_gemm: negative size");
   if (d->M == 0 || d->N == 0 || d->grid_m == 0) return TK_OK;
@@ -117,20 +118,22 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
     const bool decode_tile = d->block_m == 16 || d->block_m == 32;
     if (!(d->w_layout == TK_W_TILED && d->w_dtype == TK_E2M1 && d->x_dtype == TK_BF16 && !d->x_mx_scale))
       return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: the fused top-k combine needs bf16 activations and tiled MXFP4 weights");
-    // block_m 16 / 32: arrival counters per (token, fragment); block_m >= 64: the persistent kernel's tile counters
+    // block_m 16 / 32: arrival counters per (token, fragment); block_m >= 64: a launch behind the GEMM
     if (!d->scatter_indx || !d->combine_out || !(decode_tile ? d->combine_counters != nullptr : d->tile_counters != nullptr) || d->activation != TK_ACT_NONE)
       return fail(TK_ERR_INVALID, "tk_moe_gemm: the fused top-k combine needs scatter_indx, combine_out, its counters (combine_counters at block_m 16 / 32, tile_counters above) and no activation");
     if (!decode_tile && (d->N % 8 || d->combine_stride_m % 8 || (reinterpret_cast<uintptr_t>(d->combine_out) & 15)))
-      return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: the fused top-k combine at block_m >= 64 needs N %% 8 == 0 and 16-byte aligned rows of combine_out");
+      return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: the top-k combine at block_m >= 64 needs N %% 8 == 0 and 16-byte aligned rows of combine_out");
     if (d->scatter_len % d->combine_k) return fail(TK_ERR_INVALID, "tk_moe_gemm: scatter_len %d is not a multiple of combine_k %d", d->scatter_len, d->combine_k);
     const int64_t yb = (int64_t)d->scatter_len * d->y_stride_m * 2;
     if (yb >= (int64_t)1 << 31 || d->y_stride_m % 4 || (reinterpret_cast<uintptr_t>(d->y) & 7) || d->N % 4)
       return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: the fused top-k combine needs N %% 4 == 0 and 8-byte aligned output rows spanning less than 2 GiB");
     p.y_bytes = (uint32_t)yb;
-    p.combine_k = d->combine_k;
-    p.combine_out = static_cast<uint16_t*>(d->combine_out);
-    p.combine_stride = d->combine_stride_m;
-    p.combine_counters = d->combine_counters;
+    if (decode_tile) {
+      p.combine_k = d->combine_k;
+      p.combine_out = static_cast<uint16_t*>(d->combine_out);
+      p.combine_stride = d->combine_stride_m;
+      p.combine_counters = d->combine_counters;
+    }
   }
   p.betas = d->betas;
   p.betas_is_f32 = d->betas_dtype == TK_F32;
@@ -304,3 +307,13 @@ extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
   return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: weight dtype %d is not supported", d->w_dtype);
 }
 
+
+// The combine behind row blocks of 64 and more: the launch that would follow otherwise.  (A sum at the end of the persistent grid, which waits there for its
+// slowest workgroup, took longer than that launch: 96 slices of 39 rows, N 1088 79 us against 33 and 5, 32 slices of 64 rows, N 1536 56 against 21 and
+// 4, 128 slices of 29 rows, N 2880 167 against 140 and 10.)
+extern "C" int32_t tk_moe_gemm(const tk_gemm_desc* d, tk_stream_t stream) {
+  if (const int32_t rc = moe_gemm(d, stream)) return rc;
+  if (d->combine_k <= 0 || d->block_m < 64 || d->M == 0 || d->N == 0 || d->grid_m == 0) return TK_OK;
+  return tk_reduce_mid(d->y, TK_BF16, d->scatter_len / d->combine_k, d->combine_k, d->N, d->combine_k * d->y_stride_m, d->y_stride_m, nullptr, 0, 0, 0, nullptr, 0,
+                       0, 0, d->combine_out, d->combine_stride_m, stream);
+}

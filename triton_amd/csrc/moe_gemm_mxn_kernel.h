@@ -521,9 +521,6 @@ __global__ __launch_bounds__(256 * G) void moe_gemm_mxn_kernel(const GemmParams 
     }
   }
   if (dyn) claimer.finish();
-  if constexpr (!SWIGLU && !MXOUT) {
-    if (p.combine_k > 0 && p.tile_counters != nullptr) fused_prefill_combine<NT>(p, tid, grid);
-  }
 }
 
 template <int BLKM, int MFW, int NFW, int G, int WD, int XD, bool MXOUT>

@@ -4,7 +4,8 @@
 //   * Four or eight waves, each all rows x 64 columns, two to a SIMD (four waves: two workgroups a CU).  Tiles of 512 columns halve what the rows cross from
 //     L2.  160 rows (160 accumulators of a wave's 256 registers; a stage of 128 k moves 40 or 20 KiB of rows and 34 KiB of weights per 5120 / 2560
 //     matrix cycles): an expert with 128 +- 11 rows is one tile, so its weights are read once.  The smaller ones bring fewer rows that are not there, and
-//     their LDS holds three stages of both: what few rows per expert wait for is the weights.
+//     have LDS for three stages of weights, which is what few rows per expert wait for (but 64 x 256, two workgroups a CU with two each), and up to 64 rows of three of
+//     the rows too.
 //   * Everything comes by `buffer_load ... lds`: no registers wait for memory, rows past the slice, columns past N and k past K are a matter of
 //     the lanes' offsets (past the resource's range the hardware writes zeros).  Rings of two or three stages of rows and of weights run on
 //     across the tiles of a persistent workgroup.
@@ -260,6 +261,7 @@ __global__ __launch_bounds__(NW_ * 64, 2) void moe_gemm_mxw_kernel(const GemmPar
       // stores of the last epilogue); the buffers of stage s - 1 have been read
       constexpr int kBehind = AA == WA ? (AA - 1) * (AI + 5) : (WA - 1) * 5, kStores = MXOUT ? (SWIGLU ? 5 : 6) : 4;  // (stores of a fragment)
       static_assert(kBehind + MFW * kStores < 64, "what a wait can count");
+      static_assert(WA <= AA + 1, "weights further ahead would let rows through that have not landed, and be aimed at the next tile before its words are there");
       if (s == 0) {
         static_for<0, MFW + 1>([&](auto n_c) __attribute__((always_inline)) {
           if (stored == decltype(n_c)::value) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(kBehind + decltype(n_c)::value * kStores) : "memory");

@@ -465,7 +465,7 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
         Y[idxs_y_m(e), :] += matmul(X[idxs_x_m(e), :], W[e, :, :])
 
     `_combine_k` (used by `legacy.matmul_ogs`, not part of the reference's signature): with `scatter_indx` mapping rows
-    to flat positions t * k + j, the k rows of every token may also be summed (inside the decode and the prefill kernel, or by a
+    to flat positions t * k + j, the k rows of every token may also be summed (inside the decode kernel, or by a
     launch that the native host path makes in the same call); the result is then attached to
     the returned tensor as `._tk_combined` ([tokens, N]) and the caller skips its `reduce`.  The caller vouches that
     EVERY token has exactly k routed rows: a token with fewer leaves its arrival counter non-zero for the next launch.
@@ -831,23 +831,14 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
     if (tiled or tiled_fp8) and block_m >= 64 and not _STATIC_TILES and not mx_act:
         d.tile_counters = _tile_counters(device).data_ptr()
     combined = None
-    # (not with MXFP8 activations: at the end of that kernel's launch the combine measured 22 us slower than `reduce` in a
-    # launch of its own at the gpt-oss shape)
+    # decode kernel: the wave that completes a token's rows last sums them (arrival counters per token and fragment)
     can_combine = (_combine_k and tiled and not extras and not mx_act and act == nt.TK_ACT_NONE and scatter_indx is not None
-                   and y_rows % _combine_k == 0 and a_dtype == _BF16)
-    if can_combine and block_m != 16 and forced is None:
-        can_combine = False  # (the streaming and the wide kernel have none, and the one behind the prefill kernel's tiles costs more than a launch)
-    elif can_combine and block_m <= 32:
-        # decode kernel: the wave that completes a token's rows last sums them (arrival counters per token and fragment)
-        can_combine = (y_rows // _combine_k) * ((N + 31) // 32) <= _COMBINE_COUNTER_WORDS
-    elif can_combine:
-        # prefill kernel: the persistent grid sums when all its workgroups have written their tiles
-        can_combine = bool(d.tile_counters) and N % 8 == 0 and y_buf is c
+                   and y_rows % _combine_k == 0 and a_dtype == _BF16 and (block_m == 16 or block_m == 32 and forced is not None)
+                   and (y_rows // _combine_k) * ((N + 31) // 32) <= _COMBINE_COUNTER_WORDS)
     if can_combine:
         combined = torch.empty((y_rows // _combine_k, N), dtype=out_dtype, device=device)
         d.combine_k, d.combine_out, d.combine_stride_m = int(_combine_k), combined.data_ptr(), combined.stride(0)
-        if block_m <= 32:
-            d.combine_counters = _combine_counters(device).data_ptr()
+        d.combine_counters = _combine_counters(device).data_ptr()
     nt.submit(nt.lib().tk_moe_gemm, d, device)
     del keep
     if y_buf is not c:
