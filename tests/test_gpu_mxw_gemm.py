@@ -93,6 +93,8 @@ RULED = [
     ("bf16", "64x512", 256, 544, 1056, [0, 1, 31, 32, 33, 5, 2, 9, 64, 65]),
     ("bf16", "32x256", 192, 736, 1072, [0, 1, 31, 32, 33, 5, 2, 9]),
     ("bf16", "32x256", 256, 512, 2080, [0, 1, 3, 2, 0, 33, 0, 0, 0, 0]),
+    ("bf16", "32x256", 256, 512, 2080, [0, 1, 31, 2, 0, 33, 0, 0, 0, 0]),
+    ("bf16", "64x512", 256, 512, 1056, [0, 1, 31, 2, 9, 33, 0, 65, 0, 0, 0, 0]),
     ("bf16", "32x256", 40, 512, 528, [0, 1, 31, 32, 33, 2, 13]),
     ("bf16", "64x256", 64, 544, 1056, [63, 64, 65, 1, 0, 33, 127, 128, 129]),
     ("bf16", "64x256", 64, 1312, 1040, [95, 32, 31, 97]),

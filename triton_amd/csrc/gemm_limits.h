@@ -51,10 +51,13 @@ inline bool reads_once(int64_t rows, int64_t n_slices, int64_t block_rows, int64
 
 // Tile of the wide MXFP4 kernel (moe_gemm_mxw_kernel.h) for a call whose rows are more than the decode kernel is made for; rows 0 = the kernels before it.
 // Figures: us, both GEMMs of a layer; "before" = the streaming kernel's 32-row blocks, or 64 and 128 rows of the ones with weights in registers.
-// bf16 rows.  32 x 256 (two workgroups a CU) is the shortest chain and divides best, for one round and up to 20 rows; beyond four rows 64 x 512, half the reads of the
-// rows, where its tiles are three a CU (real layers, the streaming kernel / 32 x 256 / 64 x 512: 128 slices, K 2880: 3 rows 277 / 268 / 275, 5 302 / 292 /
-// 286, 9 315 / 310 / 301, 19 370 / 351 / 332; K 2048: 9 rows 170 / 163 / 162, 16 178 / 176 / 171; 96 slices, K 1088, 12 rows 62 / 60 / 71; 64 slices, K 1536: 9
-// rows 66 / 63 / 68, 19 75 / 76 / 75; 32 slices, K 2880, 19 rows 109 / 104 / 106).  64 x 256, two workgroups a CU as well, divides a small
+// bf16 rows.  32 x 256 (two workgroups a CU) is the shortest chain and divides best, for one round and up to 20 rows; beyond seven rows 64 x 512, half the reads of the
+// rows, where its tiles are three a CU.  Not below: there only slices with favourites fill such a tile, and they are few (real layers, the streaming
+// kernel / 32 x 256 / 64 x 512; 128 slices, K 2880, random: 3 rows 277 / 268 / 275, 5 306 / 293 / 299, 8 325 / 317 / 313, 13 340 / 326 / 325, 19 368 / 341 / 339;
+// with favourites, the logits' spread 1.5 times their noise: 5 rows 149 / 136 / 170, 8 192 / 189 / 177, 13 241 / 219 / 225, 19 292 / 282 / 266; all tokens on the same four: 5
+// rows 70 / 64 / 87, 8 104 / 99 / 92.  K 2048: 8 rows 170 / 168 / 163, favourites 109 / 102 / 99, 16 178 / 176 / 171; 96 slices, K 1088, 12 rows 62 / 60 / 71; 64
+// slices, K 1536: 9 rows 66 / 63 / 68, 19 75 / 76 / 75; 32 slices, K 2880, 19 rows 109 / 104 / 106; K 1024, N 2048, 64 slices, the first GEMM alone: 4 rows 19.0 / 18.0 /
+// 17.8, favourites 11.8 / 12.5 / 18.6).  64 x 256, two workgroups a CU as well, divides a small
 // product of more rows evenly; where the tiles of 512 columns are two rounds and more, those: half the reads of the rows, and three stages of weights in flight.
 //   128 slices, K 2880, N 5760 and 2880: 28 rows before 415, 370 (64 x 512), 42 471, 416, 56 525, 475 (96; 64 x 512 498), 72 607, 544 (96; 160 563,
 //   64 x 256 743), 84 646, 602 (160; 96 613)
@@ -64,7 +67,8 @@ inline bool reads_once(int64_t rows, int64_t n_slices, int64_t block_rows, int64
 //   32 slices, K 1536 and 640, N 1280 and 1536: 16 rows 32, 25 (32; 64 x 256 28), 64 46, 32 (32 or 64 x 256), 82 51, 37
 //   32 slices, K 1024, N 4096: 62 rows 32, 29 (64 x 256), 500 163, 134 (160; 64 x 256 145); 16 slices, K 1024, N 2048: 50 rows 18.6, 13.1 (32; 64 x
 //   256 15.1), 375 45, 34 (64 x 256)
-//   (against: 32 slices, K 2400, N 1920, 256 tiles of the kernel before, one for each CU: 12 rows 19.1, 21, 31 22.3, 24.9)
+//   (Against: products of one round with a random routing, one GEMM: 32 slices, K 2400, N 1920, 31 rows 23.7, 24.9, 16 slices, K 1024, N 4096, 37 rows 15.9, 16.9; with
+//   favourites 37.6, 24.8 and 31.4, 16.5; the whole layers 101, 54 and 56, 42.)
 // MXFP8 rows, whose stage is half as long to multiply: the kernel before (128 x 256 tiles, weights in registers) stays where its tiles are one round (32
 // slices, K 2400, N 1920: 18 rows 21 against 24, 50 22 against 30).  Beyond that tiles as high as a routing with favourites needs as well, since the epilogue
 // costs by rows: 128 x 512 from 24 rows; 64 x 512 below, and longer where the tiles of 512 columns are less than three a CU, where 32 x 256 divides better below.
@@ -85,7 +89,7 @@ inline MxwTile mxw_tile(int64_t rows, int64_t n_slices, int64_t N, bool mx8) {
     return rows <= (few ? 40 : 24) * n_slices ? MxwTile{64, 512} : rows <= 104 * n_slices ? MxwTile{128, 512} : MxwTile{0, 0};
   }
   if ((rows + 16 * n_slices) * n256 <= 512 * 32) return {32, 256};
-  if (rows <= 20 * n_slices) return rows > 4 * n_slices && n_slices * n512 >= 3 * 256 ? MxwTile{64, 512} : MxwTile{32, 256};
+  if (rows <= 20 * n_slices) return rows > 7 * n_slices && n_slices * n512 >= 3 * 256 ? MxwTile{64, 512} : MxwTile{32, 256};
   if ((rows + 160 * n_slices - 1) / (160 * n_slices) * n_slices * n512 < 512) return {64, 256};
   return rows <= 48 * n_slices ? MxwTile{64, 512} : rows <= 80 * n_slices ? MxwTile{96, 512} : MxwTile{160, 512};
 }
