@@ -102,10 +102,12 @@ RULED = [
     ("bf16", "96x512", 256, 736, 528, [95, 96, 97, 1, 33, 65, 64, 100]),
     ("bf16", "160x512", 256, 512, 576, [159, 160, 161, 81, 80, 1, 33]),
     ("mxfp8", "32x256", 128, 512, 576, [0, 1, 31, 32, 33, 2, 13]),
-    ("mxfp8", "64x512", 128, 672, 544, [0, 1, 31, 32, 33, 63, 64, 65, 10]),
+    ("mxfp8", "128x512", 128, 672, 544, [0, 1, 31, 32, 33, 63, 64, 65, 10]),
+    ("mxfp8", "64x512", 128, 672, 544, [0, 1, 31, 32, 33, 63, 64, 65, 10, 0]),
     ("mxfp8", "64x512", 256, 544, 1088, [0, 1, 31, 32, 63, 64, 65, 10, 2, 1, 0]),
     ("mxfp8", "128x512", 128, 736, 576, [95, 96, 97, 1, 33, 65, 40]),
     ("mxfp8", "128x512", 128, 928, 544, [127, 128, 129, 65, 64, 1, 33, 97, 96]),
+    ("mxfp8", "128x512", 64, 544, 1024, [127, 128, 129, 150, 255, 256, 1, 160]),
 ]
 
 

@@ -72,7 +72,14 @@ inline bool reads_once(int64_t rows, int64_t n_slices, int64_t block_rows, int64
 // MXFP8 rows, whose stage is half as long to multiply: the kernel before (128 x 256 tiles, weights in registers) stays where its tiles are one round (32
 // slices, K 2400, N 1920: 18 rows 21 against 24, 50 22 against 30).  Beyond that tiles as high as a routing with favourites needs as well, since the epilogue
 // costs by rows: 128 x 512 from 24 rows; 64 x 512 below, and longer where the tiles of 512 columns are less than three a CU, where 32 x 256 divides better below.
-// (slices all alike; by favourites, the last one's expectation five times the first's):
+// Where these are just one round if all slices have rows, a routing with favourites makes 64-row blocks a second one from about 32 rows on (64 slices, K and N
+// 2048: 37 rows, random / favourites, before 38 / 39, 64 x 512 33 / 42, 128 x 512 33 / 36; 32 slices, N 4096: 37 / 38, 32 / 42, 33 / 36; 160 tiles, K 960, N 2400: 19 /
+// 21, 17 / 17, 18 / 23).  160 x 512 takes over at 104 rows, or where two row blocks of 128 are more than a round (before / 128 x 512 / 160 x 512: 16 slices, K 1024, N
+// 4096: 125 rows 30 / 26 / 32, 175 32 / 28 / 33; 32 slices, K 2400, N 1920: 125 rows 47 / 41 / 49, 176 50 / 43 / 52; K 960, N 2400: 125 rows 28 / 25 / 29, 162 30 / 35 / 30).
+// (All tokens on the same few experts, which a balanced router does not do, leave the tiles of 512 columns fewer than CUs, or just over a round, more often
+// than the 128 x 256 ones before; layers: 128 experts of 2880, four of them live, 300 tokens 90, 83, 700 139, 162, 1400 206, 237, 2300 312, 292; 96 experts, K 1696 and 1088, 900 tokens
+// 74, 78; 64 experts of 1024, two live, 300 41, 37, 1500 51, 60.)
+// Before and by these rules (slices all alike; by favourites, the last one's expectation five times the first's):
 //   128 slices, K 2880, N 5760 and 2880: 4 rows 348, 287 (64); 139, 135.  14 354, 305 (64); 209, 204.  28 378, 341 (128; 64 334); 262, 276 (64 289).
 //   43 401, 369 (128); 322, 313 (64 357).  72 452, 418 (160 435); 427, 413.  94 485, 458 (160 467); 500, 486.  128 658, 656 (160 531); 603, 580
 //   96 slices, K 1696 and 1088, N 2176 and 1696: 11 rows 92, 72 (32; 64 76); 65, 54 (64).  36 98, 86 (64; 128 90, 32 107); 88, 84 (128 96).  58 108,
@@ -84,9 +91,13 @@ inline MxwTile mxw_tile(int64_t rows, int64_t n_slices, int64_t N, bool mx8) {
   const int64_t n256 = (N + 255) / 256, n512 = (N + 511) / 512;
   if (mx8) {
     if ((rows <= 96 * n_slices ? 256 * n_slices : 2 * rows + 128 * n_slices) * n256 <= 256 * 256) return {0, 0};  // (256ths of its row blocks)
-    const bool few = n_slices * n512 < 3 * 256;
+    const int64_t alike = n_slices * n512;
+    const bool few = alike < 3 * 256;
     if (few && rows <= 24 * n_slices) return {32, 256};
-    return rows <= (few ? 40 : 24) * n_slices ? MxwTile{64, 512} : rows <= 104 * n_slices ? MxwTile{128, 512} : MxwTile{0, 0};
+    if (rows <= (!few ? 24 : alike > 192 && alike <= 256 ? 32 : 40) * n_slices) return {64, 512};
+    // (from 104 to 152 rows on a slice's second row block of 128 becomes the rule)
+    const int64_t second = rows - 104 * n_slices < 48 * n_slices ? rows - 104 * n_slices : 48 * n_slices;
+    return second <= 0 || (rows <= 176 * n_slices && n512 * (48 * n_slices + second) <= 256 * 48) ? MxwTile{128, 512} : MxwTile{0, 0};
   }
   if ((rows + 16 * n_slices) * n256 <= 512 * 32) return {32, 256};
   if (rows <= 20 * n_slices) return rows > 7 * n_slices && n_slices * n512 >= 3 * 256 ? MxwTile{64, 512} : MxwTile{32, 256};
