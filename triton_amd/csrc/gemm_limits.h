@@ -36,14 +36,16 @@ inline bool dma_runs_e4m3(uint32_t x_bytes, int64_t n_slices, int64_t K, int64_t
 // half of the 256 MiB of the cache in front of memory, so that next to nothing of them is there when the call is made again.  Measured (us of a
 // layer, with against without it; other weights each call).  e4m3, 8 experts, d 4096, d_ff 14336: 8 rows each 238 against 267, 62 rows 295 / 313; d 2048, d_ff
 // 4096, 16 rows (201 MB in all) 70 / 74, but with the same weights again 66 / 64.  bf16, d and d_ff 2048: 16 experts, 25 rows 112 / 120, 32 experts, 31
-// rows 203 / 217; tiles of 256 rows: 32 experts, 200 rows 254 / 271; where row blocks share their weights it costs: 16 experts, 256 rows 193 / 187;
+// rows 203 / 217; tiles of 256 rows: 32 experts, 200 rows 254 / 271; where row blocks of 256 share their weights it costs: 16 experts, 256 rows 193 / 187;
 // tiles of 128 rows, 125 rows 149 / 146.  MXFP4, 128 experts, d and d_ff 2880, 128 rows 806 / 824, MXFP8 572 / 580, 94 rows 497 / 520.
 // Why the line lies at 13/16 of a block (a first GEMM by itself, two sets of weights in turn, random routing): with tiles of 256 rows it turns between
 // 0.85 and 0.90, where slices begin to have a second block, which the kernel without the hint cuts into narrow tiles: bf16, 32 slices, K 2048, N
 // 4096: 205 rows 143 / 149, 218 144 / 150, 230 172 / 165, 243 180 / 170; 64 slices, N 1024: 218 rows 74 / 82, 230 105 / 96; e4m3, 16 slices, K 4096,
 // N 8192: 218 rows 127 / 135, 230 131 / 135, 243 162 / 148 (all slices alike 3 to 14 % for the hint up to a whole block).  Smaller tiles have no
 // narrow ones and gain beyond the line as well: 128 rows, 16 slices, K 2048, N 3072: 102 rows 52 / 56, 109 54 / 57, 122 53 / 57; the wide kernel's
-// 160, 128 slices, K 2880, N 5760: MXFP4 128 rows 537 / 546, 136 570 / 578, 152 640 / 644, MXFP8 128 rows 358 / 357, 136 363 / 373, 152 417 / 421.
+// 160, 128 slices, K 2880, N 5760: MXFP4 128 rows 537 / 546, 136 570 / 578, 152 640 / 644, MXFP8 128 rows 358 / 357, 136 363 / 373, 152 417 / 421.  Tiles of 320
+// rows, one block for a slice of 256: 32 slices, K and N 2048, 256 rows 102 / 109, N 4096 190 / 191, K 1440 163 / 152, K 2048, N 1440 92 / 100; 8 slices, K and N 4096, 256 rows 96 /
+// 103; beyond the line, 285 rows, 16 slices, K 2048, N 4096 117 / 126, N 2048 58 / 65, 32 slices 123 / 127.
 inline bool reads_once(int64_t rows, int64_t n_slices, int64_t block_rows, int64_t N, int64_t row_bytes) {
   const int64_t read = n_slices < rows ? n_slices : rows;
   return rows * 16 <= n_slices * block_rows * 13 && read * N * row_bytes > 128 << 20;
