@@ -212,3 +212,51 @@ def test_infinite_inputs_match_oracle(mx, device, dt):
         qo, so = omx.downcast_to_mxfp(xs, torch.uint8, axis=1)
         _same(qo, q, "values")
         _same(so, s, "scales")
+
+
+@pytest.mark.parametrize("inner", [4, 5, 7, 255, 257, 258, 261])
+@pytest.mark.parametrize("qdt", QTYPES)
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_columns_that_are_no_multiple_of_four(mx, device, dt, qdt, inner):
+    """The last lane of a row moves back to end with the row, and a tile of fewer than four columns starts in front of
+    its place."""
+    x = torch.randn((2, 96, inner), generator=torch.Generator().manual_seed(inner)).to(dt)
+    x[0, 32:64, inner - 1] = 0  # a block of zeros and one with a scale of its own beside it
+    x[1, 5, inner - 2] = 30000.0
+    q, s = mx.downcast_to_mxfp(x.to(device), qdt, axis=1)
+    qo, so = omx.downcast_to_mxfp(x, qdt, axis=1)
+    _same(qo, q, "values")
+    _same(so, s, "scales")
+    _same(omx.upcast_from_mxfp(qo, so, dt, axis=1).contiguous(), mx.upcast_from_mxfp(q, s, dt, axis=1), "dequant")
+
+
+@pytest.mark.parametrize("qdt", [torch.float8_e4m3fn, torch.float8_e5m2])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_every_code_under_every_scale(mx, device, dt, qdt):
+    """All 256 codes under all 256 scale bytes: the packed conversions inside their range, the clamp outside it.  Finite
+    results and infinities exactly; NaN where the oracle has NaN."""
+    codes = torch.arange(256, dtype=torch.int32).to(torch.uint8).view(1, 1, 256).expand(256, 8, 256)  # [scale, column, axis]
+    scales = torch.arange(256, dtype=torch.int32).to(torch.uint8).view(256, 1, 1).expand(256, 8, 8).contiguous()
+    for finite in (False, True):  # with the special codes in every block of 32 that has them, and without any
+        c = codes.contiguous()
+        if finite:
+            special = (c & 0x7F) == 0x7F if qdt == torch.float8_e4m3fn else (c & 0x7C) == 0x7C
+            c = torch.where(special, torch.zeros_like(c), c)
+        q = c.view(qdt).transpose(1, 2)  # [scale, axis, column], unit stride along the axis
+        s = scales.transpose(1, 2)
+        d = mx.upcast_from_mxfp(q.to(device), s.to(device), dt, axis=1).cpu()
+        ref = omx.upcast_from_mxfp(q, s, dt, axis=1)
+        assert torch.equal(ref.isnan(), d.isnan())
+        _same(torch.nan_to_num(ref, 0.0, float("inf"), float("-inf")), torch.nan_to_num(d, 0.0, float("inf"), float("-inf")), "dequant")
+
+
+@pytest.mark.parametrize("qdt", QTYPES)
+def test_sources_read_with_the_non_temporal_hint(mx, device, qdt):
+    """A source past the size from which the rows are read with the hint: the same bytes as its halves below that size."""
+    g = torch.Generator(device=device).manual_seed(2)
+    x = torch.randn((2, 1024, 26624), generator=g, device=device, dtype=torch.bfloat16)
+    q, s = mx.downcast_to_mxfp(x, qdt, axis=1)
+    for i in range(2):
+        qi, si = mx.downcast_to_mxfp(x[i:i + 1], qdt, axis=1)
+        _same(qi, q[i:i + 1], "values")
+        _same(si, s[i:i + 1], "scales")

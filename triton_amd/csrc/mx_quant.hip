@@ -6,8 +6,8 @@
 //   cols : the quantised axis is strided and the INNER axis is unit-stride (a weight [E, K, N]
 //          quantised along K); a lane owns one or two columns and walks 32 rows, so every load of a
 //          wave is one contiguous row segment and the 32-element reduction is register-local.
-//   tile : the cols case for 16-bit tensors, with an LDS transpose so that the quantised bytes of a column move
-//          as full 128-byte lines (mx_down_tile / mx_up_tile).
+//   tile : the cols case for 16-bit tensors of four columns and more, with an LDS transpose so that the quantised
+//          bytes of a column move as full 128-byte lines (mx_down_tile / mx_up_tile).
 #include "mx_math.h"
 
 namespace tk {
@@ -49,10 +49,123 @@ __device__ inline int64_t line_of(int64_t o, int64_t col, int64_t inner, int64_t
   return (o * inner_last + l) * (inner / inner_last) + m;
 }
 
+typedef __attribute__((ext_vector_type(2))) unsigned short u16x2_t;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
+typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
+__device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
+  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, a), __builtin_bit_cast(u16x2_t, b)));
+}
+// two 16-bit floats (low half first) / scale -> two e2m1 codes in byte `SEL` of `old` (first value in the low nibble)
+template <int SRC>
+__device__ __forceinline__ uint32_t cvt_pk_fp4(uint32_t old, uint32_t pair, float scale, int sel) {
+  if constexpr (SRC == TK_BF16) {
+    const bf16x2_t v = __builtin_bit_cast(bf16x2_t, pair);
+    return sel == 0   ? __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(old, v, scale, 0)
+           : sel == 1 ? __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(old, v, scale, 1)
+           : sel == 2 ? __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(old, v, scale, 2)
+                      : __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(old, v, scale, 3);
+  } else {
+    const f16x2_t v = __builtin_bit_cast(f16x2_t, pair);
+    return sel == 0   ? __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(old, v, scale, 0)
+           : sel == 1 ? __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(old, v, scale, 1)
+           : sel == 2 ? __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(old, v, scale, 2)
+                      : __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(old, v, scale, 3);
+  }
+}
+
+// byte pair `SEL` of `w` (two e2m1 codes, low nibble first) * scale -> two 16-bit floats (first value in the low half)
+template <int DST>
+__device__ __forceinline__ uint32_t cvt_pk_from_fp4(uint32_t w, float scale, int sel) {
+  if constexpr (DST == TK_BF16) {
+    const bf16x2_t r = sel == 0   ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 0)
+                       : sel == 1 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 1)
+                       : sel == 2 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 2)
+                                  : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 3);
+    return __builtin_bit_cast(uint32_t, r);
+  } else {
+    const f16x2_t r = sel == 0   ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 0)
+                      : sel == 1 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 1)
+                      : sel == 2 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 2)
+                                 : __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 3);
+    return __builtin_bit_cast(uint32_t, r);
+  }
+}
+
+// The hardware's 8-bit float conversions give the bytes of the bit algorithms in mx_math.h: compared on the GPU over every 16-bit pattern under every
+// scale (down) and every code under every scale (up), they differ in overflow (a value past the largest finite one gives NaN; here it saturates), in the
+// sign and payload of NaN, and where a product with the scale leaves the target type's range.  Calls clamp, or exclude, those.
+// Two fp32 -> two bytes (first in the low one), saturating; NaN becomes 0x7F with its sign.
 template <int KIND>
-__device__ inline uint32_t quant_byte(float q) {
-  if (KIND == TK_E4M3) return e4m3_byte(mx_clamp(q, 448.0f));
-  return e5m2_byte(mx_clamp(q, 57344.0f));
+__device__ __forceinline__ uint32_t quant_pair(float q0, float q1) {
+  const float mq = KIND == TK_E4M3 ? 448.0f : 57344.0f;
+  const uint32_t w = (uint32_t)(KIND == TK_E4M3 ? __builtin_amdgcn_cvt_pk_fp8_f32(mx_clamp(q0, mq), mx_clamp(q1, mq), 0, false)
+                                                : __builtin_amdgcn_cvt_pk_bf8_f32(mx_clamp(q0, mq), mx_clamp(q1, mq), 0, false));
+  const uint32_t lo = q0 != q0 ? ((hd_f32_bits(q0) >> 24) & 0x80u) | 0x7Fu : w & 0xFFu;
+  const uint32_t hi = q1 != q1 ? ((hd_f32_bits(q1) >> 16) & 0x8000u) | 0x7F00u : w & 0xFF00u;
+  return lo | hi;
+}
+
+// two 16-bit floats (low half first) / scale -> two bytes in half `sel` of `old`; the quotients must be finite and within the format's range
+template <int SRC, int KIND>
+__device__ __forceinline__ uint32_t cvt_pk_8(uint32_t old, uint32_t pair, float scale, int sel) {
+  typedef __attribute__((ext_vector_type(2))) short s16x2_t;
+  const s16x2_t o = __builtin_bit_cast(s16x2_t, old);
+  s16x2_t r;
+  if constexpr (SRC == TK_BF16) {
+    const bf16x2_t v = __builtin_bit_cast(bf16x2_t, pair);
+    if constexpr (KIND == TK_E4M3)
+      r = sel == 0 ? __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(o, v, scale, false) : __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(o, v, scale, true);
+    else
+      r = sel == 0 ? __builtin_amdgcn_cvt_scalef32_pk_bf8_bf16(o, v, scale, false) : __builtin_amdgcn_cvt_scalef32_pk_bf8_bf16(o, v, scale, true);
+  } else {
+    const f16x2_t v = __builtin_bit_cast(f16x2_t, pair);
+    if constexpr (KIND == TK_E4M3)
+      r = sel == 0 ? __builtin_amdgcn_cvt_scalef32_pk_fp8_f16(o, v, scale, false) : __builtin_amdgcn_cvt_scalef32_pk_fp8_f16(o, v, scale, true);
+    else
+      r = sel == 0 ? __builtin_amdgcn_cvt_scalef32_pk_bf8_f16(o, v, scale, false) : __builtin_amdgcn_cvt_scalef32_pk_bf8_f16(o, v, scale, true);
+  }
+  return __builtin_bit_cast(uint32_t, r);
+}
+
+// half `sel` of `w` (two bytes, low one first) * scale -> two 16-bit floats; no NaN or infinity among the codes and a scale of `up_scale_ok`
+template <int KIND, int DST>
+__device__ __forceinline__ uint32_t cvt_pk_from_8(uint32_t w, float scale, int sel) {
+  if constexpr (DST == TK_BF16) {
+    bf16x2_t r;
+    if constexpr (KIND == TK_E4M3)
+      r = sel == 0 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, scale, false) : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w, scale, true);
+    else
+      r = sel == 0 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(w, scale, false) : __builtin_amdgcn_cvt_scalef32_pk_bf16_bf8(w, scale, true);
+    return __builtin_bit_cast(uint32_t, r);
+  } else {
+    f16x2_t r;
+    if constexpr (KIND == TK_E4M3)
+      r = sel == 0 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, scale, false) : __builtin_amdgcn_cvt_scalef32_pk_f16_fp8(w, scale, true);
+    else
+      r = sel == 0 ? __builtin_amdgcn_cvt_scalef32_pk_f16_bf8(w, scale, false) : __builtin_amdgcn_cvt_scalef32_pk_f16_bf8(w, scale, true);
+    return __builtin_bit_cast(uint32_t, r);
+  }
+}
+
+// Scales (e8m0 bytes) under which the conversion above equals dequantising in fp32, clamping to the target's range and rounding: no finite code leaves
+// that range.  (e2m1: see mx_up_tile.)
+template <int KIND, int DST>
+__device__ __forceinline__ bool up_scale_ok(uint32_t sb) {
+  if (KIND == TK_E2M1) return DST == TK_BF16 ? (sb >= 8 && sb <= 248) : (sb >= 114 && sb <= 139);
+  const uint32_t top = KIND == TK_E4M3 ? (DST == TK_BF16 ? 246u : 134u) : (DST == TK_BF16 ? 239u : 127u);
+  return sb >= 1 && sb <= top;
+}
+// scale bits under which the packed conversions of finite 16-bit elements need no clamp and lose nothing.  (e2m1 saturates by itself; extreme scales, where
+// subnormal elements could matter, are left out.  fp8: the scale rounded up, so that max / scale is within the format's range.)
+template <int KIND>
+__device__ __forceinline__ bool down_scale_ok(uint32_t sb, int rounding) {
+  if (KIND == TK_E2M1) return sb >= (16u << 23) && sb <= (250u << 23);
+  return rounding == TK_MX_ROUND_UP && sb >= (1u << 23) && sb <= (254u << 23);
+}
+// nonzero where one of a word's four codes is NaN (e4m3) or NaN or an infinity (e5m2)
+template <int KIND>
+__device__ __forceinline__ uint32_t special_codes(uint32_t w) {
+  return ((w & 0x7F7F7F7Fu) + (KIND == TK_E4M3 ? 0x01010101u : 0x04040404u)) & 0x80808080u;
 }
 
 template <int KIND>
@@ -64,23 +177,59 @@ __device__ inline float elem_f32(uint32_t b) {
 // ---------------------------------------------------------------------------------------------
 // downcast, quantised axis contiguous: src [rows, L] with row stride `ld`
 // ---------------------------------------------------------------------------------------------
+// One lane takes eight elements (16 bytes of a 16-bit tensor in one load), the four lanes of a block share its maximum.  16-bit sources whose block is finite
+// (and, for fp8, whose scale is rounded up, so that no quotient passes the largest finite code) go through the packed conversions, one instruction for
+// two elements; everything else takes the fp32 path.  A row index is a division, in 32 bits where the indices fit.
 template <int SRC, int KIND>
 __global__ __launch_bounds__(kThreads) void mx_down_rows(const typename Elem<SRC>::T* __restrict__ src, int64_t ld,
                                                          int64_t rows, int64_t L, uint8_t* __restrict__ out_vals,
                                                          uint8_t* __restrict__ out_scales, int rounding) {
+  typedef typename Elem<SRC>::T T;
   const int64_t groups_per_row = L / 8;
   const int64_t total = rows * groups_per_row;
   const int64_t gid = (int64_t)blockIdx.x * kThreads + threadIdx.x;
   if (gid >= total) return;  // total % 4 == 0, so a quad of lanes is either fully in or fully out
-  const int64_t row = gid / groups_per_row;
+  const int64_t row = total <= 0xFFFFFFFFll ? (int64_t)((uint32_t)gid / (uint32_t)groups_per_row) : gid / groups_per_row;
   const int64_t g = gid - row * groups_per_row;
-  const typename Elem<SRC>::T* p = src + row * ld + g * 8;
+  T e[8];
+  __builtin_memcpy(e, src + row * ld + g * 8, sizeof(e));
+  uint8_t* const dst = out_vals + row * (KIND == TK_E2M1 ? L / 2 : L) + g * (KIND == TK_E2M1 ? 4 : 8);
+  uint8_t* const sdst = out_scales + row * (L / 32) + (g >> 2);
+  float m = 0.0f;
+  if constexpr (sizeof(T) == 2) {
+    uint32_t w[4], mx = 0;
+    __builtin_memcpy(w, e, 16);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mx = pk_max_u16(mx, w[i] & 0x7FFF7FFFu);
+    mx = pk_max_u16(mx, (uint32_t)__shfl_xor((int)mx, 1));
+    mx = pk_max_u16(mx, (uint32_t)__shfl_xor((int)mx, 2));
+    const uint32_t m16 = mx >> 16 > (mx & 0xFFFFu) ? mx >> 16 : mx & 0xFFFFu;
+    const float mf = SRC == TK_BF16 ? hd_bits_f32(m16 << 16) : f16_bits_to_f32((uint16_t)m16);
+    const uint32_t sb = mx_scale_bits(mf, KIND, rounding);
+    const bool finite = SRC == TK_BF16 ? m16 < 0x7F80u : m16 < 0x7C00u;
+    if (finite && down_scale_ok<KIND>(sb, rounding)) {
+      const float scale = hd_bits_f32(sb);
+      if constexpr (KIND == TK_E2M1) {
+        uint32_t o = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o = cvt_pk_fp4<SRC>(o, w[i], scale, i);
+        *reinterpret_cast<uint32_t*>(dst) = o;
+      } else {
+        uint32_t o[2] = {0, 0};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[i >> 1] = cvt_pk_8<SRC, KIND>(o[i >> 1], w[i], scale, i & 1);
+        *reinterpret_cast<uint2*>(dst) = make_uint2(o[0], o[1]);
+      }
+      if ((g & 3) == 0) *sdst = (uint8_t)(sb >> 23);
+      return;  // all four lanes of a block come to the same answer
+    }
+  }
   float v[8];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = Elem<SRC>::load(p + i);
-  float m = 0.0f;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) m = fmaxf(m, fabsf(v[i]));
+  for (int i = 0; i < 8; ++i) {
+    v[i] = Elem<SRC>::load(e + i);
+    m = fmaxf(m, fabsf(v[i]));
+  }
   m = fmaxf(m, __shfl_xor(m, 1));
   m = fmaxf(m, __shfl_xor(m, 2));
   const uint32_t sbits = mx_scale_bits(m, KIND, rounding);
@@ -89,16 +238,14 @@ __global__ __launch_bounds__(kThreads) void mx_down_rows(const typename Elem<SRC
     uint32_t packed = 0;
 #pragma unroll
     for (int i = 0; i < 8; ++i) packed |= e2m1_code(v[i] * inv) << (4 * i);
-    *reinterpret_cast<uint32_t*>(out_vals + row * (L / 2) + g * 4) = packed;
+    *reinterpret_cast<uint32_t*>(dst) = packed;
   } else {
-    uint32_t lo = 0, hi = 0;
+    uint32_t o[2];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) lo |= quant_byte<KIND>(v[i] * inv) << (8 * i);
-#pragma unroll
-    for (int i = 0; i < 4; ++i) hi |= quant_byte<KIND>(v[4 + i] * inv) << (8 * i);
-    *reinterpret_cast<uint2*>(out_vals + row * L + g * 8) = make_uint2(lo, hi);
+    for (int h = 0; h < 2; ++h) o[h] = quant_pair<KIND>(v[4 * h] * inv, v[4 * h + 1] * inv) | quant_pair<KIND>(v[4 * h + 2] * inv, v[4 * h + 3] * inv) << 16;
+    *reinterpret_cast<uint2*>(dst) = make_uint2(o[0], o[1]);
   }
-  if ((g & 3) == 0) out_scales[row * (L / 32) + (g >> 2)] = (uint8_t)(sbits >> 23);
+  if ((g & 3) == 0) *sdst = (uint8_t)(sbits >> 23);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -155,9 +302,10 @@ __global__ __launch_bounds__(kThreads) void mx_down_cols(const typename Elem<SRC
       for (int i = 0; i < 32; ++i) w[i >> 3] |= e2m1_code(v[i][c] * inv) << (4 * (i & 7));
       *reinterpret_cast<uint4*>(out_vals + line * (L / 2) + blk * 16) = make_uint4(w[0], w[1], w[2], w[3]);
     } else {
-      uint32_t w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+      uint32_t w[8];
 #pragma unroll
-      for (int i = 0; i < 32; ++i) w[i >> 2] |= quant_byte<KIND>(v[i][c] * inv) << (8 * (i & 3));
+      for (int i = 0; i < 8; ++i)
+        w[i] = quant_pair<KIND>(v[4 * i][c] * inv, v[4 * i + 1][c] * inv) | quant_pair<KIND>(v[4 * i + 2][c] * inv, v[4 * i + 3][c] * inv) << 16;
       uint4* dst = reinterpret_cast<uint4*>(out_vals + line * L + blk * 32);
       dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
       dst[1] = make_uint4(w[4], w[5], w[6], w[7]);
@@ -271,6 +419,17 @@ constexpr int kTilePitch = 128 + 16;  // LDS bytes per column
 // consecutive lanes (columns c, c + 4, ...) fall 144 bytes apart and take different banks
 constexpr int kTileRows = 64 + 65 * 3;
 __device__ __forceinline__ int tile_row(int c) { return (c >> 2) + 65 * (c & 3); }
+// First column of tile `ct`, and the first of a lane's four columns inside it.  Where the number of columns is no multiple of four (it is at least four),
+// the last lane moves back to end with the last column and does up to three columns again that its neighbour does, with the same result.  Rows then start
+// at any even address: the memory takes 8 bytes a lane at any alignment, and the 512 bytes of a wave's row touch one line more.  (6 x 1632 x 1093 to e4m3 and
+// back, a column per lane and 16 or 32 bytes of a line per store: 15.3 + 15.2 us; this way 9.6 + 10.4.)
+__device__ __forceinline__ int64_t tile_col0(int64_t ct, int64_t inner) { return ct * kTileCols < inner - 4 ? ct * kTileCols : inner - 4; }
+__device__ __forceinline__ int tile_cols_of(int lane, int64_t col0, int64_t inner) {
+  const int64_t last = inner - 4 - col0;
+  return lane * 4 < last ? lane * 4 : (int)last;
+}
+// 8 bytes at any even address
+typedef __attribute__((ext_vector_type(2), aligned(2))) uint32_t u32x2_any_t;
 
 // Workgroups are dealt round-robin to the 8 XCDs, each with its own L2.  Tiles are renumbered so that consecutive
 // tiles run on ONE XCD at about the same time, and the tiles of one column range are numbered consecutively along
@@ -281,49 +440,6 @@ __device__ __forceinline__ int64_t tile_order(int64_t pid, int64_t total) {
   const int64_t per = total / 8, extra = total % 8;
   const int64_t grp = pid % 8, local = pid / 8;
   return grp * per + (grp < extra ? grp : extra) + local;
-}
-
-typedef __attribute__((ext_vector_type(2))) unsigned short u16x2_t;
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
-typedef __attribute__((ext_vector_type(2))) uint32_t u32x2_t;
-typedef __attribute__((ext_vector_type(2))) _Float16 half2_t;
-__device__ __forceinline__ uint32_t pk_max_u16(uint32_t a, uint32_t b) {
-  return __builtin_bit_cast(uint32_t, __builtin_elementwise_max(__builtin_bit_cast(u16x2_t, a), __builtin_bit_cast(u16x2_t, b)));
-}
-// two 16-bit floats (low half first) / scale -> two e2m1 codes in byte `SEL` of `old` (first value in the low nibble)
-template <int SRC>
-__device__ __forceinline__ uint32_t cvt_pk_fp4(uint32_t old, uint32_t pair, float scale, int sel) {
-  if constexpr (SRC == TK_BF16) {
-    const bf16x2_t v = __builtin_bit_cast(bf16x2_t, pair);
-    return sel == 0   ? __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(old, v, scale, 0)
-           : sel == 1 ? __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(old, v, scale, 1)
-           : sel == 2 ? __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(old, v, scale, 2)
-                      : __builtin_amdgcn_cvt_scalef32_pk_fp4_bf16(old, v, scale, 3);
-  } else {
-    const half2_t v = __builtin_bit_cast(half2_t, pair);
-    return sel == 0   ? __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(old, v, scale, 0)
-           : sel == 1 ? __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(old, v, scale, 1)
-           : sel == 2 ? __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(old, v, scale, 2)
-                      : __builtin_amdgcn_cvt_scalef32_pk_fp4_f16(old, v, scale, 3);
-  }
-}
-
-// byte pair `SEL` of `w` (two e2m1 codes, low nibble first) * scale -> two 16-bit floats (first value in the low half)
-template <int DST>
-__device__ __forceinline__ uint32_t cvt_pk_from_fp4(uint32_t w, float scale, int sel) {
-  if constexpr (DST == TK_BF16) {
-    const bf16x2_t r = sel == 0   ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 0)
-                       : sel == 1 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 1)
-                       : sel == 2 ? __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 2)
-                                  : __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(w, scale, 3);
-    return __builtin_bit_cast(uint32_t, r);
-  } else {
-    const f16x2_t r = sel == 0   ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 0)
-                      : sel == 1 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 1)
-                      : sel == 2 ? __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 2)
-                                 : __builtin_amdgcn_cvt_scalef32_pk_f16_fp4(w, scale, 3);
-    return __builtin_bit_cast(uint32_t, r);
-  }
 }
 
 template <int KIND>
@@ -386,87 +502,102 @@ __device__ __forceinline__ void tile_move(uint8_t* vals_s, uint8_t* sc_s, uint8_
 template <int SRC, int KIND>
 __device__ __forceinline__ void quantise_block_to_lds(const uint2 (&raw)[32], uint8_t* vals_s, uint8_t* sc_s, int c4, int b, int rounding) {
   constexpr int BB = TileGeom<KIND>::BB, NB = TileGeom<KIND>::NB;
-    auto elem = [&](int i, int c) __attribute__((always_inline)) {
-      const uint32_t w = c < 2 ? raw[i].x : raw[i].y;
-      const uint16_t e = (uint16_t)((c & 1) ? (w >> 16) : (w & 0xFFFFu));
-      return Elem<SRC>::load(&e);
-    };
-    // e2m1: the block maxima come from the 16-bit patterns themselves (|x| orders like its bits without the sign, two
-    // elements per instruction) and the hardware converts two 16-bit floats to two e2m1 codes while dividing by the
-    // power-of-two scale (round to nearest even, saturating at +-6, exact), so a pair of rows costs one byte permute
-    // and one conversion.  Blocks that hold an infinity or a NaN, or whose scale is so extreme that subnormal inputs
-    // could matter, take the fp32 path below.
-    uint32_t max01 = 0, max23 = 0;
-    if constexpr (KIND == TK_E2M1) {
+  // The block maxima come from the 16-bit patterns themselves (|x| orders like its bits without the sign, two elements per instruction) and the
+  // hardware converts two 16-bit floats to two codes while dividing by the power-of-two scale (round to nearest even, exact), so a pair of rows costs
+  // one byte permute and one conversion.  A lane with a block that holds an infinity or a NaN, or whose scale is outside `down_scale_ok`, takes the fp32
+  // path below, as a loop over its columns: the bit algorithms of fp8, unrolled over the 128 elements, were 25 KB of instructions, and fetching those was
+  // most of the time of a small tensor (2 x 64 x 528 e5m2: 20 us a launch, 4.6 now; 32 x 2880 x 5760 e4m3: 395 us, 300 with the hint below).
+  uint32_t max01 = 0, max23 = 0;
 #pragma unroll
-      for (int i = 0; i < 32; ++i) {
-        max01 = pk_max_u16(max01, raw[i].x & 0x7FFF7FFFu);
-        max23 = pk_max_u16(max23, raw[i].y & 0x7FFF7FFFu);
-      }
-    }
+  for (int i = 0; i < 32; ++i) {
+    max01 = pk_max_u16(max01, raw[i].x & 0x7FFF7FFFu);
+    max23 = pk_max_u16(max23, raw[i].y & 0x7FFF7FFFu);
+  }
+  uint32_t sb[4];
+  bool fast = true;
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const uint32_t mx = c < 2 ? max01 : max23;
+    const uint32_t m16 = (c & 1) ? (mx >> 16) : (mx & 0xFFFFu);
+    sb[c] = mx_scale_bits(SRC == TK_BF16 ? hd_bits_f32(m16 << 16) : f16_bits_to_f32((uint16_t)m16), KIND, rounding);
+    fast = fast && (SRC == TK_BF16 ? m16 < 0x7F80u : m16 < 0x7C00u) && down_scale_ok<KIND>(sb[c], rounding);
+  }
+  if (fast) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
       uint4* dst = reinterpret_cast<uint4*>(vals_s + tile_row(c4 + c) * kTilePitch + b * BB);
-      if constexpr (KIND == TK_E2M1) {
-        const uint32_t mx = c < 2 ? max01 : max23;
-        const uint32_t m16 = (c & 1) ? (mx >> 16) : (mx & 0xFFFFu);
-        const float mf = SRC == TK_BF16 ? hd_bits_f32(m16 << 16) : f16_bits_to_f32((uint16_t)m16);
-        const uint32_t sb = mx_scale_bits(mf, KIND, rounding);
-        const bool finite = SRC == TK_BF16 ? m16 < 0x7F80u : m16 < 0x7C00u;
-        if (finite && sb >= (16u << 23) && sb <= (250u << 23)) {
-          const float scale = hd_bits_f32(sb);
-          uint32_t w[4] = {0, 0, 0, 0};
+      const float scale = hd_bits_f32(sb[c]);
+      uint32_t w[BB / 4];
 #pragma unroll
-          for (int i = 0; i < 32; i += 2) {
-            const uint32_t lo = c < 2 ? raw[i].x : raw[i].y, hi = c < 2 ? raw[i + 1].x : raw[i + 1].y;
-            const uint32_t pair = __builtin_amdgcn_perm(hi, lo, (c & 1) ? 0x07060302u : 0x05040100u);  // (row i, row i+1) of column c
-            w[i >> 3] = cvt_pk_fp4<SRC>(w[i >> 3], pair, scale, (i >> 1) & 3);
-          }
-          dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
-          sc_s[(c4 + c) * NB + b] = (uint8_t)(sb >> 23);
-          continue;
-        }
+      for (int i = 0; i < BB / 4; ++i) w[i] = 0;
+#pragma unroll
+      for (int i = 0; i < 32; i += 2) {
+        const uint32_t lo = c < 2 ? raw[i].x : raw[i].y, hi = c < 2 ? raw[i + 1].x : raw[i + 1].y;
+        const uint32_t pair = __builtin_amdgcn_perm(hi, lo, (c & 1) ? 0x07060302u : 0x05040100u);  // (row i, row i+1) of column c
+        if constexpr (KIND == TK_E2M1)
+          w[i >> 3] = cvt_pk_fp4<SRC>(w[i >> 3], pair, scale, (i >> 1) & 3);
+        else
+          w[i >> 2] = cvt_pk_8<SRC, KIND>(w[i >> 2], pair, scale, (i >> 1) & 1);
       }
-      float m = 0.0f;
 #pragma unroll
-      for (int i = 0; i < 32; ++i) m = fmaxf(m, fabsf(elem(i, c)));
-      const uint32_t sbits = mx_scale_bits(m, KIND, rounding);
-      const float inv = mx_inv_scale(sbits);
-      if (KIND == TK_E2M1) {
-        // hardware conversion (round to nearest even, saturating at +-6); NaN is first turned into the infinity of
-        // its sign so that it saturates like the reference's bit algorithm (mxfp.py:298-327)
-        uint32_t w[4] = {0, 0, 0, 0};
-#pragma unroll
-        for (int i = 0; i < 32; i += 2) {
-          float q0 = elem(i, c) * inv, q1 = elem(i + 1, c) * inv;
-          q0 = q0 != q0 ? __builtin_copysignf(INFINITY, q0) : q0;
-          q1 = q1 != q1 ? __builtin_copysignf(INFINITY, q1) : q1;
-          if ((i & 6) == 0) w[i >> 3] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w[i >> 3], q0, q1, 1.0f, 0);
-          if ((i & 6) == 2) w[i >> 3] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w[i >> 3], q0, q1, 1.0f, 1);
-          if ((i & 6) == 4) w[i >> 3] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w[i >> 3], q0, q1, 1.0f, 2);
-          if ((i & 6) == 6) w[i >> 3] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w[i >> 3], q0, q1, 1.0f, 3);
-        }
-        dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
-      } else {
-        uint32_t w[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll
-        for (int i = 0; i < 32; ++i) w[i >> 2] |= quant_byte<KIND>(elem(i, c) * inv) << (8 * (i & 3));
-        dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
-        dst[BB / 32] = make_uint4(w[4], w[5], w[6], w[7]);
-      }
-      sc_s[(c4 + c) * NB + b] = (uint8_t)(sbits >> 23);
+      for (int i = 0; i < BB / 16; ++i) dst[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
+      sc_s[(c4 + c) * NB + b] = (uint8_t)(sb[c] >> 23);
     }
+    return;
+  }
+#pragma unroll 1
+  for (int c = 0; c < 4; ++c) {
+    auto elem = [&](int i) __attribute__((always_inline)) {
+      const uint16_t e = (uint16_t)((c < 2 ? raw[i].x : raw[i].y) >> (16 * (c & 1)));
+      return Elem<SRC>::load(&e);
+    };
+    uint4* dst = reinterpret_cast<uint4*>(vals_s + tile_row(c4 + c) * kTilePitch + b * BB);
+    float m = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) m = fmaxf(m, fabsf(elem(i)));
+    const uint32_t sbits = mx_scale_bits(m, KIND, rounding);
+    const float inv = mx_inv_scale(sbits);
+    uint32_t w[BB / 4];
+#pragma unroll
+    for (int i = 0; i < BB / 4; ++i) w[i] = 0;
+    if constexpr (KIND == TK_E2M1) {
+      // hardware conversion (round to nearest even, saturating at +-6); NaN is first turned into the infinity of
+      // its sign so that it saturates like the reference's bit algorithm (mxfp.py:298-327)
+#pragma unroll
+      for (int i = 0; i < 32; i += 2) {
+        float q0 = elem(i) * inv, q1 = elem(i + 1) * inv;
+        q0 = q0 != q0 ? __builtin_copysignf(INFINITY, q0) : q0;
+        q1 = q1 != q1 ? __builtin_copysignf(INFINITY, q1) : q1;
+        if ((i & 6) == 0) w[i >> 3] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w[i >> 3], q0, q1, 1.0f, 0);
+        if ((i & 6) == 2) w[i >> 3] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w[i >> 3], q0, q1, 1.0f, 1);
+        if ((i & 6) == 4) w[i >> 3] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w[i >> 3], q0, q1, 1.0f, 2);
+        if ((i & 6) == 6) w[i >> 3] = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(w[i >> 3], q0, q1, 1.0f, 3);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 32; i += 2) w[i >> 2] |= quant_pair<KIND>(elem(i) * inv, elem(i + 1) * inv) << (8 * (i & 2));
+    }
+#pragma unroll
+    for (int i = 0; i < BB / 16; ++i) dst[i] = make_uint4(w[4 * i], w[4 * i + 1], w[4 * i + 2], w[4 * i + 3]);
+    sc_s[(c4 + c) * NB + b] = (uint8_t)(sbits >> 23);
+  }
 }
 
-// 8 bytes of a stream that is read exactly once: the non-temporal hint keeps the lines from displacing what the L2
+// 8 bytes of a stream that is read exactly once: the non-temporal hint (NT) keeps the lines from displacing what the L2
 // still has to merge (the output lines at the tiles' seams); measured 0.281 -> 0.264 ms on [32, 2880, 5760] bf16.
 // (The same hint on the dequantiser's row stores costs 5 %: 0.275 -> 0.288 ms.)
+template <bool NT>
 __device__ __forceinline__ uint2 load_once_u2(const uint16_t* p) {
-  const u32x2_t t = __builtin_nontemporal_load(reinterpret_cast<const u32x2_t*>(p));
+  const u32x2_any_t* a = reinterpret_cast<const u32x2_any_t*>(p);
+  const u32x2_any_t t = NT ? __builtin_nontemporal_load(a) : *a;
   return make_uint2(t.x, t.y);
 }
 
-template <int SRC, int KIND>
+// Sources of this size and more are read with the non-temporal hint.  Two in turn, plain loads / with the hint, us a launch, bf16 [b, 2880, 5760] to e4m3:
+// b 2 (66 MB) 18.1 / 23.8, b 4 47.8 / 39.5, b 8 107 / 75, b 16 181 / 153, b 32 343 / 300; to e2m1: b 2 18.9 / 21.8, b 4 42.6 / 36.8, b 8 95 / 68.  What
+// was used a moment ago is still in the memory-side cache up to about a hundred megabytes, and a read with the hint does not profit from that.
+constexpr int64_t kOnceBytes = 96ll << 20;
+template <int SRC, int KIND, bool NT>
 __global__ __launch_bounds__(kThreads) void mx_down_tile(const uint16_t* __restrict__ src, int64_t stride_outer, int64_t stride_axis,
                                                          int64_t L, int64_t inner, int64_t inner_last, int64_t col_tiles,
                                                          int64_t blk_tiles, uint8_t* __restrict__ out_vals,
@@ -480,36 +611,37 @@ __global__ __launch_bounds__(kThreads) void mx_down_tile(const uint16_t* __restr
   const int64_t ct = bid % col_tiles;
   const int64_t o = bid / col_tiles;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: row addresses stay scalar
-  const int64_t col0 = ct * kTileCols, blk0 = bt * NB;
-  const int c4 = lane * 4;  // this lane's four columns inside the tile
+  const int64_t col0 = tile_col0(ct, inner), blk0 = bt * NB;
+  const bool live = col0 + lane * 4 < inner;
+  const int c4 = tile_cols_of(lane, col0, inner);  // this lane's four columns inside the tile
   if constexpr (NB / 4 == 2) {
     // e2m1 (two blocks per wave): the rows of BOTH blocks are requested before either is converted.  That takes 171
     // registers, so two workgroups share a CU instead of four, each wave with 32 KB on its way instead of 16: measured
     // 0.314 -> 0.281 ms on [32, 2880, 5760] bf16.  (Fewer resident workgroups help on their own, 0.289 ms with the one-block
     // loop held to two waves per SIMD; one wave per SIMD is too few, 0.317 ms.)
     uint2 raw0[32], raw1[32];
-    const bool ok0 = blk0 + wave < L / 32 && col0 + c4 < inner, ok1 = blk0 + wave + 4 < L / 32 && col0 + c4 < inner;
+    const bool ok0 = blk0 + wave < L / 32 && live, ok1 = blk0 + wave + 4 < L / 32 && live;
     const int64_t bb0 = ok0 ? blk0 + wave : 0, bb1 = ok1 ? blk0 + wave + 4 : bb0;
-    const int64_t cc = col0 + c4 < inner ? col0 + c4 : 0;
+    const int64_t cc = live ? col0 + c4 : 0;
     const uint16_t* p0 = src + o * stride_outer + bb0 * 32 * stride_axis + cc;
     const uint16_t* p1 = src + o * stride_outer + bb1 * 32 * stride_axis + cc;
 #pragma unroll
-    for (int i = 0; i < 32; ++i) raw0[i] = load_once_u2(p0 + i * stride_axis);
+    for (int i = 0; i < 32; ++i) raw0[i] = load_once_u2<NT>(p0 + i * stride_axis);
 #pragma unroll
-    for (int i = 0; i < 32; ++i) raw1[i] = load_once_u2(p1 + i * stride_axis);
+    for (int i = 0; i < 32; ++i) raw1[i] = load_once_u2<NT>(p1 + i * stride_axis);
     if (ok0) quantise_block_to_lds<SRC, KIND>(raw0, vals_s, sc_s, c4, wave, rounding);
     if (ok1) quantise_block_to_lds<SRC, KIND>(raw1, vals_s, sc_s, c4, wave + 4, rounding);
   } else
 #pragma unroll 1
   for (int pass = 0; pass < NB / 4; ++pass) {
     const int b = wave + 4 * pass;
-    if (blk0 + b >= L / 32 || col0 + c4 >= inner) continue;
+    if (blk0 + b >= L / 32 || !live) continue;
     const uint16_t* p = src + o * stride_outer + (blk0 + b) * 32 * stride_axis + col0 + c4;
     // the 32 rows stay packed (two 16-bit elements per register) and are widened where they are used: half the
     // registers of an fp32 copy, which is what lets four workgroups share a CU and overlap their load phases
     uint2 raw[32];
 #pragma unroll
-    for (int i = 0; i < 32; ++i) raw[i] = *reinterpret_cast<const uint2*>(p + i * stride_axis);
+    for (int i = 0; i < 32; ++i) raw[i] = load_once_u2<NT>(p + i * stride_axis);
     quantise_block_to_lds<SRC, KIND>(raw, vals_s, sc_s, c4, b, rounding);
   }
   __syncthreads();
@@ -529,92 +661,88 @@ __global__ __launch_bounds__(kThreads) void mx_up_tile(const uint8_t* __restrict
   const int64_t ct = bid % col_tiles;
   const int64_t o = bid / col_tiles;
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // uniform: row addresses stay scalar
-  const int64_t col0 = ct * kTileCols, blk0 = bt * NB;
-  const int c4 = lane * 4;
+  const int64_t col0 = tile_col0(ct, inner), blk0 = bt * NB;
+  const bool live = col0 + lane * 4 < inner;
+  const int c4 = tile_cols_of(lane, col0, inner);
   tile_move<KIND, false>(vals_s, sc_s, const_cast<uint8_t*>(vals), const_cast<uint8_t*>(scales), o, col0, blk0, L, inner, inner_last);
   __syncthreads();
   const float mf = Elem<DST>::max_finite();
 #pragma unroll 1
   for (int pass = 0; pass < NB / 4; ++pass) {
     const int b = wave + 4 * pass;
-    if (blk0 + b >= L / 32 || col0 + c4 >= inner) continue;
+    if (blk0 + b >= L / 32 || !live) continue;
     uint16_t* q = out + o * ostride_outer + (blk0 + b) * 32 * ostride_axis + col0 + c4;
-    if constexpr (KIND == TK_E2M1) {
-      // Common case, all four blocks of the lane have a scale for which element * scale is a normal number of the
-      // target type whatever the element: the hardware conversion (two codes -> two scaled 16-bit floats, exact, no
-      // clamp needed) yields rows (i, i+1) of one column, a byte permute per output dword regroups two columns'
-      // results into (column c, column c+1) of one row, and every 8 rows are stored as soon as they are complete.
-      uint32_t sb4[4];
-      bool all_fast = true;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        sb4[c] = sc_s[(c4 + c) * NB + b];
-        all_fast = all_fast && (DST == TK_BF16 ? (sb4[c] >= 8 && sb4[c] <= 248) : (sb4[c] >= 114 && sb4[c] <= 139));
-      }
-      if (all_fast) {
-        uint4 w4[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) w4[c] = *reinterpret_cast<const uint4*>(vals_s + tile_row(c4 + c) * kTilePitch + b * BB);
-#pragma unroll
-        for (int d = 0; d < 4; ++d) {
-          uint32_t pr[4][4];  // [column][row pair of this group of 8 rows]
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            const uint32_t w = d == 0 ? w4[c].x : d == 1 ? w4[c].y : d == 2 ? w4[c].z : w4[c].w;
-            const float scale = hd_bits_f32(sb4[c] << 23);
-#pragma unroll
-            for (int g = 0; g < 4; ++g) pr[c][g] = cvt_pk_from_fp4<DST>(w, scale, g);
-          }
-#pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const int i = d * 8 + g * 2;
-            *reinterpret_cast<uint2*>(q + i * ostride_axis) =
-                make_uint2(__builtin_amdgcn_perm(pr[1][g], pr[0][g], 0x05040100u), __builtin_amdgcn_perm(pr[3][g], pr[2][g], 0x05040100u));
-            *reinterpret_cast<uint2*>(q + (i + 1) * ostride_axis) =
-                make_uint2(__builtin_amdgcn_perm(pr[1][g], pr[0][g], 0x07060302u), __builtin_amdgcn_perm(pr[3][g], pr[2][g], 0x07060302u));
-          }
-        }
-        continue;
-      }
-    }
-    // general path (fp8 values, or a block with an extreme scale): element by element with the clamp, eight rows at a
-    // time so that only those rows' results are held in registers
-    uint4 wa[4], wb[4];
-    uint32_t sb4g[4];
+    // Common case, all four blocks of the lane have a scale for which element * scale is a normal number of the target type whatever the element (fp8:
+    // what `up_scale_ok` says, and no NaN or infinity among the codes): the hardware conversion (two codes -> two scaled 16-bit floats, exact, no
+    // clamp needed) yields rows (i, i+1) of one column, a byte permute per output dword regroups two columns' results into (column c, column c+1) of one
+    // row, and every 8 rows are stored as soon as they are complete.
+    uint32_t sb4[4];
+    uint4 w4[4][BB / 16];
+    bool all_fast = true;
+    uint32_t special = 0;
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
+      sb4[c] = sc_s[(c4 + c) * NB + b];
+      all_fast = all_fast && up_scale_ok<KIND, DST>(sb4[c]);
       const uint4* srcp = reinterpret_cast<const uint4*>(vals_s + tile_row(c4 + c) * kTilePitch + b * BB);
-      wa[c] = srcp[0];
-      wb[c] = KIND == TK_E2M1 ? wa[c] : srcp[BB / 32];
-      sb4g[c] = sc_s[(c4 + c) * NB + b];
-    }
-    auto word = [](const uint4& v, int k) __attribute__((always_inline)) { return k == 0 ? v.x : k == 1 ? v.y : k == 2 ? v.z : v.w; };
 #pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      uint32_t hp[8][2];
+      for (int h = 0; h < BB / 16; ++h) {
+        w4[c][h] = srcp[h];
+        if constexpr (KIND != TK_E2M1)
+          special |= special_codes<KIND>(w4[c][h].x) | special_codes<KIND>(w4[c][h].y) | special_codes<KIND>(w4[c][h].z) | special_codes<KIND>(w4[c][h].w);
+      }
+    }
+    if (all_fast && special == 0) {
+      auto word = [](const uint4& v, int k) __attribute__((always_inline)) { return k == 0 ? v.x : k == 1 ? v.y : k == 2 ? v.z : v.w; };
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        uint32_t pr[4][4];  // [column][row pair of this group of 8 rows]
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+          const float scale = hd_bits_f32(sb4[c] << 23);
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            if constexpr (KIND == TK_E2M1)
+              pr[c][g] = cvt_pk_from_fp4<DST>(word(w4[c][0], d), scale, g);
+            else
+              pr[c][g] = cvt_pk_from_8<KIND, DST>(word(w4[c][d >> 1], 2 * (d & 1) + (g >> 1)), scale, g & 1);
+          }
+        }
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int i = d * 8 + g * 2;
+          *reinterpret_cast<u32x2_any_t*>(q + i * ostride_axis) =
+              u32x2_any_t{__builtin_amdgcn_perm(pr[1][g], pr[0][g], 0x05040100u), __builtin_amdgcn_perm(pr[3][g], pr[2][g], 0x05040100u)};
+          *reinterpret_cast<u32x2_any_t*>(q + (i + 1) * ostride_axis) =
+              u32x2_any_t{__builtin_amdgcn_perm(pr[1][g], pr[0][g], 0x07060302u), __builtin_amdgcn_perm(pr[3][g], pr[2][g], 0x07060302u)};
+        }
+      }
+      continue;
+    }
+    // general path: element by element with the clamp, two rows at a time; a loop, since unrolled over fp8's 128 elements it was most of the time of a
+    // small tensor to fetch (2 x 64 x 528 e5m2: 15 to 18 us a launch, 4.5 now; 32 x 2880 x 5760 e4m3 490 us, 345 now, of which the packed conversions are most)
+#pragma unroll 1
+    for (int i = 0; i < 32; i += 2) {
+      uint32_t hp[2][2] = {{0, 0}, {0, 0}};
 #pragma unroll
       for (int c = 0; c < 4; ++c) {
+        const uint8_t* srcp = vals_s + tile_row(c4 + c) * kTilePitch + b * BB;
+        const uint32_t sb = sc_s[(c4 + c) * NB + b];
+        const uint32_t two = KIND == TK_E2M1 ? srcp[i >> 1] : *reinterpret_cast<const uint16_t*>(srcp + i);
 #pragma unroll
-        for (int r = 0; r < 8; ++r) {
+        for (int r = 0; r < 2; ++r) {
           float f;
-          if (KIND == TK_E2M1) {
-            const uint32_t code = (word(wa[c], d) >> (4 * r)) & 0xFu;
-            f = mx_dequant(bf16_bits_to_f32((uint16_t)e2m1_to_bf16_bits(code)), sb4g[c], mf, false);
-          } else {
-            const int k = 2 * d + (r >> 2);  // dword of the block's 32 bytes
-            const uint32_t byte = (word(k < 4 ? wa[c] : wb[c], k & 3) >> (8 * (r & 3))) & 0xFFu;
-            f = mx_dequant(elem_f32<KIND>(byte), sb4g[c], mf, KIND == TK_E5M2);
-          }
+          if (KIND == TK_E2M1)
+            f = mx_dequant(bf16_bits_to_f32((uint16_t)e2m1_to_bf16_bits((two >> (4 * r)) & 0xFu)), sb, mf, false);
+          else
+            f = mx_dequant(elem_f32<KIND>((two >> (8 * r)) & 0xFFu), sb, mf, KIND == TK_E5M2);
           uint16_t e;
           Elem<DST>::store(&e, f);
-          if (c & 1)
-            hp[r][c >> 1] |= (uint32_t)e << 16;
-          else
-            hp[r][c >> 1] = e;
+          hp[r][c >> 1] |= (uint32_t)e << (16 * (c & 1));
         }
       }
 #pragma unroll
-      for (int r = 0; r < 8; ++r) *reinterpret_cast<uint2*>(q + (d * 8 + r) * ostride_axis) = make_uint2(hp[r][0], hp[r][1]);
+      for (int r = 0; r < 2; ++r) *reinterpret_cast<u32x2_any_t*>(q + (i + r) * ostride_axis) = u32x2_any_t{hp[r][0], hp[r][1]};
     }
   }
 }
@@ -639,13 +767,13 @@ int32_t launch_down(const void* src, int64_t outer, int64_t L, int64_t inner, in
   if (si != 1 && inner != 1) return fail(TK_ERR_UNSUPPORTED, "tk_mx_downcast: inner stride must be 1");
   const int64_t nblk = L / 32;
   if constexpr (sizeof(T) == 2) {
-    if (inner % 4 == 0 && sa % 4 == 0 && so % 4 == 0 && (reinterpret_cast<uintptr_t>(src) % 8) == 0 &&
-        (reinterpret_cast<uintptr_t>(out_vals) % 16) == 0) {
+    if (inner >= 4 && (reinterpret_cast<uintptr_t>(out_vals) % 16) == 0) {
       const int64_t col_tiles = cdiv(inner, kTileCols), blk_tiles = cdiv(nblk, TileGeom<KIND>::NB);
       const int64_t grid = col_tiles * blk_tiles * outer;
       if (grid > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_mx_downcast: tensor too large for one launch");
-      hipLaunchKernelGGL((mx_down_tile<SRC, KIND>), dim3((unsigned)grid), dim3(kThreads), 0, st, reinterpret_cast<const uint16_t*>(s), so, sa,
-                         L, inner, inner_last, col_tiles, blk_tiles, ov, os, rounding);
+      const bool once = outer * L * inner * 2 >= kOnceBytes;
+      hipLaunchKernelGGL((once ? mx_down_tile<SRC, KIND, true> : mx_down_tile<SRC, KIND, false>), dim3((unsigned)grid), dim3(kThreads), 0, st,
+                         reinterpret_cast<const uint16_t*>(s), so, sa, L, inner, inner_last, col_tiles, blk_tiles, ov, os, rounding);
       return check_launch("mx_down_tile");
     }
   }
@@ -685,8 +813,7 @@ int32_t launch_up(const void* vals, const void* scales, int64_t outer, int64_t L
   if (osi != 1 && inner != 1) return fail(TK_ERR_UNSUPPORTED, "tk_mx_upcast: output inner stride must be 1");
   const int64_t nblk = L / 32;
   if constexpr (sizeof(T) == 2) {
-    if (inner % 4 == 0 && osa % 4 == 0 && oso % 4 == 0 && (reinterpret_cast<uintptr_t>(out) % 8) == 0 &&
-        (reinterpret_cast<uintptr_t>(vals) % 16) == 0) {
+    if (inner >= 4 && (reinterpret_cast<uintptr_t>(vals) % 16) == 0) {
       const int64_t col_tiles = cdiv(inner, kTileCols), blk_tiles = cdiv(nblk, TileGeom<KIND>::NB);
       const int64_t grid = col_tiles * blk_tiles * outer;
       if (grid > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_mx_upcast: tensor too large for one launch");
