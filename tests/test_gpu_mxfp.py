@@ -214,6 +214,27 @@ def test_infinite_inputs_match_oracle(mx, device, dt):
         _same(so, s, "scales")
 
 
+@pytest.mark.parametrize("K", [8, 504, 1024, 1032, 2048, 2056, 8192, 8200])
+def test_quantize_fp8_rowwise_every_magnitude(device, K):
+    """Rows from the smallest to the largest magnitudes (scales with and without a reciprocal in the normal range), a
+    count that is no multiple of the rows per workgroup, every kernel and the lengths at which they change."""
+    from oracle import moe as omoe
+    from triton_amd.numerics_details.rowwise_fp8 import quantize_fp8_rowwise
+    g = torch.Generator().manual_seed(K)
+    x = torch.randn((257, K), generator=g) * (2.0**torch.linspace(-125, 124, 257))[:, None]
+    x = x * 2.0**torch.randint(-12, 1, x.shape, generator=g)  # quotients down to the subnormal codes and zero
+    x = x.to(torch.bfloat16)
+    x[0] = 0
+    x[5::9, ::3] = -0.0
+    x[3, K // 2] = float("-inf")
+    q, s = quantize_fp8_rowwise(x.to(device))
+    q_ref, s_ref = omoe.quantize_fp8_rowwise(x)
+    assert torch.equal(s.cpu(), s_ref)
+    bad = q.cpu().view(torch.uint8) != q_ref.view(torch.uint8)
+    bad[3, K // 2] = False  # inf / inf is NaN, whose sign is open
+    assert not bad.any()
+
+
 @pytest.mark.parametrize("inner", [4, 5, 7, 255, 257, 258, 261])
 @pytest.mark.parametrize("qdt", QTYPES)
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])

@@ -102,6 +102,44 @@ __global__ __launch_bounds__(256) void reduce_mid_bf16x8_kernel(const uint16_t* 
   }
 }
 
+// Eight elements of a row / its scale to e4m3.  The quotient is the correctly rounded fp32 one, as `x / s` gives it, from the row's reciprocal: with r = 1 / s
+// correctly rounded and q = x * r, q - (q * s - x) * r, two fused operations, is x / s rounded to nearest (P. Markstein, "Computation of elementary functions on the
+// IBM RISC System/6000 processor", 1990), three instructions in the place of a division's ten.  That needs r and the remainder in the normal range: rows
+// whose scale is not between 2^-60 and 2^100 (an infinity among the elements makes it infinite) divide.  (Elements so far below the row's maximum that the remainder
+// is subnormal become zero either way.)  No quotient passes 448 by more than its rounding, so it needs no clamp; NaN stays NaN.
+__device__ __forceinline__ bool scale_has_reciprocal(float s) { return s >= 8.6736173798840355e-19f && s <= 1.2676506002282294e30f; }
+__device__ __forceinline__ uint2 quant8_recip(uint4 v, float s, float r) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  float q8[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    const float x = bits_f32(c & 1 ? w[c >> 1] & 0xFFFF0000u : w[c >> 1] << 16);
+    const float q = x * r;
+    q8[c] = __builtin_fmaf(-__builtin_fmaf(q, s, -x), r, q);  // (in this order -0 stays -0)
+  }
+  int o0 = 0, o1 = 0;
+  o0 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[0], q8[1], o0, false);
+  o0 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[2], q8[3], o0, true);
+  o1 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[4], q8[5], o1, false);
+  o1 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[6], q8[7], o1, true);
+  return make_uint2((uint32_t)o0, (uint32_t)o1);
+}
+__device__ __forceinline__ uint2 quant8_div(uint4 v, float s) {
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  float q8[8];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    q8[2 * c] = mx_clamp(bits_f32(w[c] << 16) / s, 448.0f);
+    q8[2 * c + 1] = mx_clamp(bits_f32(w[c] & 0xFFFF0000u) / s, 448.0f);
+  }
+  int o0 = 0, o1 = 0;
+  o0 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[0], q8[1], o0, false);
+  o0 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[2], q8[3], o0, true);
+  o1 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[4], q8[5], o1, false);
+  o1 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[6], q8[7], o1, true);
+  return make_uint2((uint32_t)o0, (uint32_t)o1);
+}
+
 // Per-row dynamic quantisation to OCP e4m3: s = amax / 448 (1 for an all-zero row), q = sat(x / s).
 // One wave per row; the row is read twice (second pass hits L2), 16 bytes per lane and load where aligned.
 __global__ __launch_bounds__(256) void quant_fp8_rows_kernel(const uint16_t* x, int64_t stride_m, int64_t M, int64_t K,
@@ -128,45 +166,35 @@ __global__ __launch_bounds__(256) void quant_fp8_rows_kernel(const uint16_t* x, 
   float s = m / 448.0f;
   if (s == 0.f) s = 1.0f;
   if (lane == 0) scales[row] = s;
+  const bool recip = scale_has_reciprocal(s);
+  const float r = 1.0f / s;
 #pragma unroll 4
   for (int64_t k = lane * 8; k < kv; k += 512) {
     const uint4 v = *reinterpret_cast<const uint4*>(xr + k);
-    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
-    // hardware conversion (OCP e4m3 on this GPU, round to nearest even) of the clamped quotients, two per instruction
-    float q8[8];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      q8[2 * i] = mx_clamp(bits_f32(w[i] << 16) / s, 448.0f);
-      q8[2 * i + 1] = mx_clamp(bits_f32(w[i] & 0xFFFF0000u) / s, 448.0f);
-    }
-    int o0 = 0, o1 = 0;
-    o0 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[0], q8[1], o0, false);
-    o0 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[2], q8[3], o0, true);
-    o1 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[4], q8[5], o1, false);
-    o1 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[6], q8[7], o1, true);
-    *reinterpret_cast<uint2*>(qr + k) = make_uint2((uint32_t)o0, (uint32_t)o1);
+    *reinterpret_cast<uint2*>(qr + k) = recip ? quant8_recip(v, s, r) : quant8_div(v, s);
   }
   for (int64_t k = kv + lane; k < K; k += 64) qr[k] = (uint8_t)e4m3_byte(mx_clamp(bf16_bits_to_f32(xr[k]) / s, 448.0f));
 }
 
 // The same with the row held in registers between the two passes (rows 16-byte aligned, K a multiple of 8 and at most
-// NV * 2048): a WORKGROUP per row, NV 16-byte pieces per thread, the row maximum through LDS, one read of x instead of
+// NV * 8 * TPR): TPR threads to a row, a workgroup or one of its waves, NV 16-byte pieces per thread, one read of x instead of
 // two.  (With a wave per row and two passes some thirty rows per CU are between their passes at any time, 29 MB per XCD
 // at K = 14336 against an L2 of 4 MB, so the second pass came from memory again: 16384 x 14336 in 189 us, 134 us this
-// way.  A wave per row with the row in registers needs 4 NV registers per lane for a row four times as long per lane and
-// was slower than two passes from 8192 elements on; for rows of 4096 it took 25 us at 8192 rows, this takes 21.)
-template <int NV>
-__global__ __launch_bounds__(256) void quant_fp8_rows_wg_kernel(const uint16_t* x, int64_t stride_m, int64_t M, int64_t K, uint8_t* q,
-                                                                int64_t stride_qm, float* scales) {
+// way, 127 us = 5.5 TB/s without the division.  A wave per row needs four times the registers per lane: from 4096 elements on a workgroup is faster,
+// 8192 x 4096 16.5 us, of which the division was 5.)
+template <int NV, int TPR>
+__global__ __launch_bounds__(256) void quant_fp8_rows_regs_kernel(const uint16_t* x, int64_t stride_m, int64_t M, int64_t K, uint8_t* q,
+                                                                  int64_t stride_qm, float* scales) {
   __shared__ float wmax_s[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t row = blockIdx.x;
+  const int tid = threadIdx.x % TPR, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t row = (int64_t)blockIdx.x * (256 / TPR) + threadIdx.x / TPR;
+  if (TPR == 64 && row >= M) return;
   const uint16_t* xr = x + row * stride_m;
   uint8_t* qr = q + row * stride_qm;
   uint4 v[NV];
 #pragma unroll
   for (int i = 0; i < NV; ++i) {
-    const int64_t k = (int64_t)i * 2048 + tid * 8;
+    const int64_t k = (int64_t)i * (TPR * 8) + tid * 8;
     v[i] = k < K ? *reinterpret_cast<const uint4*>(xr + k) : make_uint4(0u, 0u, 0u, 0u);
   }
   float m = 0.f;
@@ -178,28 +206,27 @@ __global__ __launch_bounds__(256) void quant_fp8_rows_wg_kernel(const uint16_t* 
   }
 #pragma unroll
   for (int off = 32; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off));
-  if (lane == 0) wmax_s[wave] = m;
-  __syncthreads();
-  m = fmaxf(fmaxf(wmax_s[0], wmax_s[1]), fmaxf(wmax_s[2], wmax_s[3]));
+  if (TPR == 256) {
+    if (lane == 0) wmax_s[wave] = m;
+    __syncthreads();
+    m = fmaxf(fmaxf(wmax_s[0], wmax_s[1]), fmaxf(wmax_s[2], wmax_s[3]));
+  }
   float s = m / 448.0f;
   if (s == 0.f) s = 1.0f;
   if (tid == 0) scales[row] = s;
+  if (scale_has_reciprocal(s)) {
+    const float r = 1.0f / s;
 #pragma unroll
-  for (int i = 0; i < NV; ++i) {
-    const int64_t k = (int64_t)i * 2048 + tid * 8;
-    const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-    float q8[8];
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      q8[2 * c] = mx_clamp(bits_f32(w[c] << 16) / s, 448.0f);
-      q8[2 * c + 1] = mx_clamp(bits_f32(w[c] & 0xFFFF0000u) / s, 448.0f);
+    for (int i = 0; i < NV; ++i) {
+      const int64_t k = (int64_t)i * (TPR * 8) + tid * 8;
+      if (k < K) *reinterpret_cast<uint2*>(qr + k) = quant8_recip(v[i], s, r);
     }
-    int o0 = 0, o1 = 0;
-    o0 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[0], q8[1], o0, false);
-    o0 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[2], q8[3], o0, true);
-    o1 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[4], q8[5], o1, false);
-    o1 = __builtin_amdgcn_cvt_pk_fp8_f32(q8[6], q8[7], o1, true);
-    if (k < K) *reinterpret_cast<uint2*>(qr + k) = make_uint2((uint32_t)o0, (uint32_t)o1);
+  } else {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int64_t k = (int64_t)i * (TPR * 8) + tid * 8;
+      if (k < K) *reinterpret_cast<uint2*>(qr + k) = quant8_div(v[i], s);
+    }
   }
 }
 
@@ -369,15 +396,22 @@ extern "C" int32_t tk_quant_fp8_rows(const void* x, int32_t dtype, int64_t M, in
   const uint16_t* xs = static_cast<const uint16_t*>(x);
   uint8_t* qd = static_cast<uint8_t*>(q);
   const bool aligned = K % 8 == 0 && stride_m % 8 == 0 && stride_qm % 8 == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0 && (reinterpret_cast<uintptr_t>(q) & 7) == 0;
-  if (aligned && K > 2048 && K <= 32768 && M <= 0x7FFFFFFF) {
+  if (aligned && K <= 32768 && M <= 0x7FFFFFFF) {
     const dim3 rows((unsigned)M);
-    if (K <= 4096)
-      hipLaunchKernelGGL(quant_fp8_rows_wg_kernel<2>, rows, block, 0, st, xs, stride_m, M, K, qd, stride_qm, scales);
+    // rows of up to 2048 elements by a wave each: 16384 x 1024 9.7 us, a workgroup per row 15.4, two passes 15.1; 5416 x 1920 9.3, 9.6, 17.4
+    if (K <= 1024)
+      hipLaunchKernelGGL((quant_fp8_rows_regs_kernel<2, 64>), grid, block, 0, st, xs, stride_m, M, K, qd, stride_qm, scales);
+    else if (K <= 2048)
+      hipLaunchKernelGGL((quant_fp8_rows_regs_kernel<4, 64>), grid, block, 0, st, xs, stride_m, M, K, qd, stride_qm, scales);
+    else if (K <= 4096)
+      hipLaunchKernelGGL((quant_fp8_rows_regs_kernel<2, 256>), rows, block, 0, st, xs, stride_m, M, K, qd, stride_qm, scales);
+    else if (K <= 8192)
+      hipLaunchKernelGGL((quant_fp8_rows_regs_kernel<4, 256>), rows, block, 0, st, xs, stride_m, M, K, qd, stride_qm, scales);
     else if (K <= 16384)
-      hipLaunchKernelGGL(quant_fp8_rows_wg_kernel<8>, rows, block, 0, st, xs, stride_m, M, K, qd, stride_qm, scales);
+      hipLaunchKernelGGL((quant_fp8_rows_regs_kernel<8, 256>), rows, block, 0, st, xs, stride_m, M, K, qd, stride_qm, scales);
     else
-      hipLaunchKernelGGL(quant_fp8_rows_wg_kernel<16>, rows, block, 0, st, xs, stride_m, M, K, qd, stride_qm, scales);
-    return check_launch("quant_fp8_rows_wg_kernel");
+      hipLaunchKernelGGL((quant_fp8_rows_regs_kernel<16, 256>), rows, block, 0, st, xs, stride_m, M, K, qd, stride_qm, scales);
+    return check_launch("quant_fp8_rows_regs_kernel");
   }
   hipLaunchKernelGGL(quant_fp8_rows_kernel, grid, block, 0, st, xs, stride_m, M, K, qd, stride_qm, scales);
   return check_launch("quant_fp8_rows_kernel");
