@@ -140,3 +140,31 @@ def test_operands_asked_for_ahead(device, n_slices, m, n):
         k = slice(int(offs[e]), int(offs[e + 1]))
         ref = a[k].float().t() @ b[k].float()
         assert ((out[e].float() - ref).abs() <= ref.abs() * 2**-8 + 1e-4).all(), e
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("n_slices, m, n, rest", [(12, 264, 1032, 300), (9, 8, 136, 2000), (128, 520, 264, 170), (1, 264, 520, 700), (128, 520, 776, 170), (129, 264, 264, 170)])
+def test_long_slices(device, n_slices, m, n, rest, out_dtype):
+    """Slices long enough on average for the kernel of long ones: lengths around its stages of 32 and its four buffers, empty ones, tiles of 128 and
+    of 256 with remainders, more and fewer tiles than workgroups and XCDs, one slice more than it keeps.  The sum is exact but for its order (fp32: some
+    2000 terms of size one, 2^-24 each time, far below the gate) and the result's rounding."""
+    import triton_amd.matmul as mm
+    g = torch.Generator().manual_seed(n_slices + m + n)
+    sizes = torch.full((n_slices, ), rest, dtype=torch.int32)
+    edges = [0, 1, 31, 32, 33, 64, 65, 96, 97, 128, 129, 3 * rest]
+    for i, s in enumerate(edges[:n_slices if n_slices > 1 else 0]):
+        sizes[(i * 5) % n_slices] = s
+    offs = _offsets(sizes, 8)
+    k = max(int(offs[-1]), 160 * n_slices + 8)  # (some rows belong to no slice)
+    a, b = torch.randn((k, m), generator=g).to(torch.bfloat16), torch.randn((k, n), generator=g).to(torch.bfloat16)
+    used = torch.zeros(k, dtype=torch.bool)
+    for e, s in enumerate(sizes.tolist()):
+        used[int(offs[e]):int(offs[e]) + s] = True
+    a[~used], b[~used] = float("nan"), float("nan")
+    out = torch.full((n_slices, m + 8, n + 8), float("nan"), dtype=out_dtype, device=device)
+    md = _metadata(sizes, offs, device)
+    mm.matmul(a.to(device).t(), b.to(device), None, a_ragged_metadata=md, b_ragged_metadata=md, c=out[:, :m, :n],
+              precision_config=mm.PrecisionConfig(out_dtype=out_dtype))
+    ref = omoe.matmul_ragged_k(a.t(), b, sizes, offs, offs, out_dtype=torch.float32)
+    assert_allclose_gate(ref, out[:, :m, :n].float(), what="ragged-K matmul")
+    assert torch.isnan(out[:, m:]).all() and torch.isnan(out[:, :, n:]).all()  # nothing written beside the result

@@ -14,34 +14,13 @@
 //
 // The problem is bound by writing y (n_slices * M * N outputs from short reductions), not by the MFMAs: at 128
 // experts x 2880 x 5760 from 256 rows each the output is 4.2 GB against 1.1 TFLOP.
+#include <algorithm>
 #include <type_traits>
 
-#include "common.h"
+#include "ragged_k.h"
 
 namespace tk {
 namespace {
-
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8_t;
-typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
-
-struct RaggedKParams {
-  const uint8_t* a;
-  int64_t a_stride_m, a_stride_k;  // elements
-  const uint8_t* b;
-  int64_t b_stride_k, b_stride_n;
-  uint8_t* y;
-  int64_t y_stride_e, y_stride_m;
-  const int32_t* sizes;
-  const int32_t* a_offs;
-  const int32_t* b_offs;
-  int M, N;
-  int tiles_m, tiles_n;
-  int chunk, n_slices;  // aligned variant: tiles per XCD and turn
-  int ahead;            // ... how many tiles ahead operands are asked for, 0 = not at all
-  int y_dtype;
-  uint32_t a_bytes, b_bytes, y_bytes;  // extents for the buffer resources of the aligned variant (y: one slice)
-  int a_vec, b_vec;  // the operand's base and strides allow 16-byte loads along its contiguous dimension
-};
 
 constexpr int kTile = 128;  // output tile edge (rows and columns)
 constexpr int kKC = 32;     // k per pipeline stage
@@ -309,11 +288,12 @@ __global__ __launch_bounds__(256) void ragged_k_gemm_kernel(const RaggedKParams 
 // A stage is kTrK k rows x 128 m (and 128 n) in the operands' own order: the rows go from memory straight into LDS
 // (buffer_load ... lds, 1 KiB = 4 k rows per wave instruction, no registers, no VALU) and ds_read_b64_tr_b16 hands a
 // lane four consecutive k of ITS row, so nothing is transposed in registers.  Row pitch 256 bytes without padding (the
-// DMA writes lane-contiguously): the 16-byte pieces of k row r are stored at piece ^ 2 * (r & 3), which puts the four
-// rows that sixteen lanes of a transposing read touch on disjoint banks.  Pieces past the slice end or the matrix edge
+// DMA writes lane-contiguously): the 16-byte pieces of k row r are stored at piece ^ 4 * (r & 3), which puts the four
+// rows of 64 bytes that 32 lanes of a transposing read touch on disjoint banks (^ 2 * (r & 3), disjoint for sixteen lanes only: half of the
+// LDS cycles were conflicts; 16 slices of 256, 1024 x 2048 and 1024 x 1024 63 -> 57 us).  Pieces past the slice end or the matrix edge
 // get an offset beyond the buffer resource; the hardware then writes zeros to LDS.
 //
-// What bounds it: writing y.  The same kernel without its loads writes 128 x [2880, 5760] bf16 in 0.77 ms (5.5 TB/s),
+// What bounds it: writing y (long slices: ragged_k_long.hip).  The same kernel without its loads writes 128 x [2880, 5760] bf16 in 0.77 ms (5.5 TB/s),
 // without its stores it takes 0.85 ms; together 1.13 ms (3.1 ms with the transposition in registers; 2880 x 2880: 1.5 -> 0.62).
 //   * the results go through LDS so that a store instruction writes whole 128-byte lines, with the non-temporal hint
 //     (pieces of 32 bytes: 1.76 ms; with the hint on such pieces 4.0, plain whole lines 1.55, whole lines with the hint 1.40);
@@ -325,30 +305,12 @@ __global__ __launch_bounds__(256) void ragged_k_gemm_kernel(const RaggedKParams 
 //   * a tile of 128 k is two turns of the ring, and each waited for its first touch of memory behind the stream of stores: the lines are
 //     asked for whole slices ahead, beyond the 128 tiles that an XCD has in flight (128 equal slices of 128 k, 258 tiles or two slices ahead,
 //     1.19 -> 1.06 ms, random lengths 1.22 -> 1.13; one slice 1.17, three 1.16, every tile asking for b 1.22).
-// Measured and left out: 128 x 256 tiles, with the same ring or by persistent workgroups whose ring runs on across tiles, with loading
+// Measured and left out (256 x 256 tiles: ragged_k_long.hip): 128 x 256 tiles, with the same ring or by persistent workgroups whose ring runs on across tiles, with loading
 // and storing waves apart (1.22 to 1.40 ms); slices mixed over an XCD's workgroups (1.25).
 constexpr int kTrK = 16;
 constexpr int kTrBufs = 5;
 constexpr int kTrOperand = kTrK * kTile * 2;   // bytes of one operand's stage
 constexpr int kTrStage = 2 * kTrOperand;
-constexpr int kNonTemporal = 2;  // buffer store: streaming
-
-__device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
-  const f32x2_t v = {a, b};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2_t));
-}
-__device__ __forceinline__ uint32_t pack_f16x2(float a, float b) {
-  const f32x2_t v = {a, b};
-  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, f16x2_t));
-}
-
-template <int DT>
-__device__ __forceinline__ f32x16_t mfma_k16(u32x4_t a, u32x4_t b, f32x16_t c) {
-  if constexpr (DT == TK_BF16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8_t, a), __builtin_bit_cast(bf16x8_t, b), c, 0, 0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a), __builtin_bit_cast(f16x8_t, b), c, 0, 0, 0);
-}
 
 // YT = element type of y (TK_BF16, TK_F16, TK_F32)
 template <int DT, int YT>
@@ -383,7 +345,7 @@ __global__ __launch_bounds__(256, 4) void ragged_k_tr_kernel(const RaggedKParams
   const buf_desc_t ra = make_buf_desc(p.a, p.a_bytes), rb = make_buf_desc(p.b, p.b_bytes);
   constexpr uint32_t kOutOfRange = 0x80000000u;
   const int krow = lane >> 4;                  // k row within the instruction's four
-  const int piece = (lane & 15) ^ (krow * 2);  // the 16-byte piece of the row this lane fetches
+  const int piece = (lane & 15) ^ (krow * 4);  // the 16-byte piece of the row this lane fetches
   const int k_lane = wave * 4 + krow;
   static_assert(kTrK == 16, "one instruction per wave, operand and stage");
   const uint32_t a_step = (uint32_t)p.a_stride_k * 2u, b_step = (uint32_t)p.b_stride_k * 2u;
@@ -408,21 +370,16 @@ __global__ __launch_bounds__(256, 4) void ragged_k_tr_kernel(const RaggedKParams
 
   // ---- fragment reads: lane addresses of a transposing read (row (lane & 15) >> 2 of four k, four columns) ------------
   const int l16 = lane & 15;
-  const int v = ((((lane >> 4) & 1) * 2) + ((l16 & 3) >> 1)) ^ ((l16 >> 2) * 2);
+  const int v = ((lane >> 4) & 1) * 2 + ((l16 & 3) >> 1), swz = (l16 >> 2) * 4;
   const uint32_t rd0 = lds0 + (uint32_t)((h * 8 + (l16 >> 2)) * (kTile * 2) + (l16 & 1) * 8);
-  // (the second fragment of a quadrant flips piece bit 2, which the rows' exclusive-or also touches)
-  const uint32_t frag_a[2] = {rd0 + mw * 128 + v * 16, rd0 + mw * 128 + (v ^ 4) * 16};
-  const uint32_t frag_b[2] = {rd0 + kTrOperand + nw * 128 + v * 16, rd0 + kTrOperand + nw * 128 + (v ^ 4) * 16};
-  auto read_frag = [&](uint32_t at) __attribute__((always_inline)) -> u32x4_t {
-    const uint64_t lo = lds_read_tr16(at), hi = lds_read_tr16(at + 4 * kTile * 2);
-    return u32x4_t{(uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32)};
-  };
+  const uint32_t frag_a[2] = {rd0 + ((mw * 8 + v) ^ swz) * 16, rd0 + ((mw * 8 + 4 + v) ^ swz) * 16};
+  const uint32_t frag_b[2] = {rd0 + kTrOperand + ((nw * 8 + v) ^ swz) * 16, rd0 + kTrOperand + ((nw * 8 + 4 + v) ^ swz) * 16};
   auto compute = [&](uint32_t buf) __attribute__((always_inline)) {
     u32x4_t af[2], bf[2];
 #pragma unroll
-    for (int j = 0; j < 2; ++j) af[j] = read_frag(frag_a[j] + buf);
+    for (int j = 0; j < 2; ++j) af[j] = read_frag_tr(frag_a[j] + buf, kTile * 2);
 #pragma unroll
-    for (int f = 0; f < 2; ++f) bf[f] = read_frag(frag_b[f] + buf);
+    for (int f = 0; f < 2; ++f) bf[f] = read_frag_tr(frag_b[f] + buf, kTile * 2);
 #pragma unroll
     for (int f = 0; f < 2; ++f)
 #pragma unroll
@@ -491,42 +448,43 @@ __global__ __launch_bounds__(256, 4) void ragged_k_tr_kernel(const RaggedKParams
         }
     }
   } else {
-    // through LDS (16-byte pieces exchanged by row to spread the banks), so that a store instruction writes eight whole
-    // 128-byte lines of the quadrant
+    // through LDS, so that a store instruction writes eight whole 128-byte lines of the quadrant
     static_assert(kTrBufs * kTrStage >= 4 * 8192, "the four quadrants fit the operand buffers");
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     uint8_t* sp = lds + wave * 8192;
 #pragma unroll
-    for (int j = 0; j < 2; ++j)
-#pragma unroll
-      for (int f = 0; f < 2; ++f)
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          uint32_t q[4];  // columns 16u + 4h + {01, 23} and 16u + 8 + 4h + {01, 23}
-#pragma unroll
-          for (int i = 0; i < 4; ++i)
-            q[i] = YT == TK_BF16 ? pack_bf16x2(acc[f][j][8 * u + 2 * i], acc[f][j][8 * u + 2 * i + 1])
-                                 : pack_f16x2(acc[f][j][8 * u + 2 * i], acc[f][j][8 * u + 2 * i + 1]);
-          // after the exchange lanes 0..31 hold columns 16u .. 16u + 7 of their row, lanes 32..63 columns 16u + 8 .. 16u + 15
-          const auto s0 = __builtin_amdgcn_permlane32_swap(q[0], q[2], false, false);
-          const auto s1 = __builtin_amdgcn_permlane32_swap(q[1], q[3], false, false);
-          const int r = j * 32 + lr;
-          *reinterpret_cast<u32x4_t*>(sp + r * 128 + (((f * 4 + u * 2 + h) ^ (r & 7)) * 16)) = u32x4_t{s0[0], s1[0], s0[1], s1[1]};
-        }
+    for (int j = 0; j < 2; ++j) stage_out_rows<YT>(sp, j, lane, acc[0][j], acc[1][j]);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
     for (int it = 0; it < 8; ++it) {
       const int r = it * 8 + (lane >> 3), pc = lane & 7;
-      const u32x4_t q = *reinterpret_cast<const u32x4_t*>(sp + r * 128 + ((pc ^ (r & 7)) * 16));
+      const u32x4_t q = staged_piece(sp, r, pc);
       const int m = m0 + mw * 64 + r, n = n0 + nw * 64 + pc * 8;
       const uint32_t off = (m < p.M && n < p.N) ? ((uint32_t)m * (uint32_t)p.y_stride_m + (uint32_t)n) * ES : kOutOfRange;
       __builtin_amdgcn_raw_buffer_store_b128(q, ry, off, 0, kNonTemporal);
     }
   }
   asm volatile("" ::"v"(ahead_a), "v"(ahead_b));
+}
+
+// Tile of the kernel for long slices (ragged_k_long.hip) for aligned operands, 0 = the one above, whose four small workgroups a CU write best where
+// writing is what takes the time.  256 x 256 needs a few rounds of tiles over the 256 CUs, 128 x 128 starts sooner; from 90 k a slice on the former
+// is as good where rounds are many and hardly any of it hangs over the edges.  Measured (us of both products [d, 2 f] and [f, d] of
+// a layer with slices of random lengths; above / 128 / 256):
+//   slices, k of one, d, f: 8, 2048, 2880, 2880 936 / 916 / 827; 8, 256, 2880, 2880 162 / 163 / 155; 16, 1024, 2048, 2048 498 / 491 / 423; 16, 375, 1600, 1200 121 / 110 / 110
+//   32, 512, 2880, 2880 1069 / 1104 / 935; 32, 187, 2880, 2880 477 / 512 / 464; 32, 187, 1600, 1200 135 / 132 / 135; 64, 256, 1024, 1024 168 / 172 / 146; 64, 256, 2880, 2880 1309 / 1357 / 1149
+//   8, 2048, 512, 512 132 / 85 / 192; 8, 256, 512, 512 26 / 21 / 40; 8, 2048, 1024, 1024 162 / 134 / 210; 8, 750, 800, 1024 71 / 55 / 87; 16, 375, 320, 448 39 / 30 / 54; 16, 256,
+//   1024, 1024 60 / 47 / 55; 32, 187, 320, 448 35 / 30 / 48; 32, 187, 800, 1024 77 / 69 / 73; 64, 256, 320, 448 50 / 47 / 54
+//   128, 128, 2880, 2880 1742 / 1903 / 1623; 128, 128, 1440, 1440 456 / 472 / 421; 64, 93, 2880, 2880 706 / 733 / 681; 32, 128, 2880, 2880 407 / 418 / 396; 16, 128, 2880, 2880 202 / 223 / 208
+//   128, 128, 1600, 1200 404 / 438 / 411; 64, 93, 1600, 1200 184 / 196 / 197; 64, 125, 1440, 1440 226 / 242 / 231; 8, 128, 512, 512 15 / 14 / 23; 128, 128, 512, 512 76 / 82 / 76; 128, 46, 2880,
+//   2880 1171 / 1275 / 1221; 16, 64, 1600, 1200 25 / 29 / 30
+int long_tile(int64_t k, int64_t M, int64_t N, int64_t n_slices) {
+  const int64_t tiles = cdiv(M, 256) * cdiv(N, 256) * n_slices;
+  if (k >= 160) return tiles >= 4 * 256 ? 256 : 128;
+  return k >= 90 && tiles >= 24 * 256 && tiles * 256 * 256 * 8 <= M * N * n_slices * 9 ? 256 : 0;
 }
 
 }  // namespace
@@ -584,9 +542,13 @@ extern "C" int32_t tk_ragged_k_gemm(const tk_ragged_k_desc* d, tk_stream_t strea
   const bool bf16 = d->dtype == TK_BF16;
   if (fast && y_ok) {
     const int per_e = p.tiles_m * p.tiles_n;
-    p.chunk = per_e >= 8 ? per_e / 8 : 1;
     p.n_slices = d->n_slices;
-    // An XCD's part of a slice below 32 tiles: lines asked for six and more slices ahead are gone again or not yet of use (both products of a layer,
+    // (rows past M of a long slice's last tiles go by offsets beyond the resource, which may not wrap)
+    const bool long_runs = d->n_slices <= kRaggedKLongSlices && (int64_t)(d->M + 256) * d->y_stride_m * es < (int64_t(1) << 32);
+    const int tile = long_runs ? long_tile(std::min(d->a_k_extent, d->b_k_extent) / d->n_slices, d->M, d->N, d->n_slices) : 0;
+    if (tile) return ragged_k_launch_long(p, d->dtype, tile, st);
+    p.chunk = per_e >= 8 ? per_e / 8 : 1;
+    // An XCD's part of a slice below 32 tiles: lines asked for six and more slices ahead are gone again or not yet of use (both products of a layer, all by this kernel,
     // 16384 rows, 128 slices, 15 and 8 tiles: 165 us without against 173; 23 and 12: 385 / 391; 36 and 18: 545 / 556; 31 and 16: 420 / 420;
     // 33 and 17: 478 / 477; 45 and 23: 685 / 659; 68 and 35: 1010 / 970).  Fewer than 64 slices: what there is to wait for is less (2880 x 5760 and
     // 2880 x 2880, 32 slices of 128 389 / 393, 8 of 2048 933 / 942; 2048 x 4096 and 2048 x 2048, 64 slices of 128 472 / 462).
