@@ -12,7 +12,10 @@
 //   3. The NW waves of a workgroup split the K-stages of a unit (K-slices of XS stages); a wave keeps its slice of the
 //      block's activation rows in REGISTERS for as long as the (expert, row block) stays the same, so the inner loop
 //      is: 2 KiB weight block global -> registers (ring, one unit ahead), e2m1 -> bf16 in registers, 16x16x32 MFMA.
-//      The slices meet in LDS once per unit (one barrier); the waves take turns at summing them and running the epilogue.
+//      The slices meet in LDS once per unit (one barrier); four of the waves, in turn, sum them and run the
+//      epilogue.  (One wave in turn: its next unit started late, and the others met it at the barrier; all waves: a quarter of a microsecond of each
+//      one's time.  49 tokens, 64 experts, top 2, d 1952, d_ff 960: 60.7 / 59.4 with four / 59.9 us; 60 tokens, 96 experts, top 4, 2048: 69.5 / 68.9 / 70.1;
+//      61 tokens, 128 experts, top 4, 2880, with favourites: 116.1 / 114.5 / 116.0.)
 //   4. GEMM 1 writes its swiglu'd rows (bf16) to a scratch tensor h with write-through stores; a workgroup that has
 //      finished its GEMM-1 share counts its units in at a per-expert counter.  GEMM-2 units of an expert wait for that
 //      counter (their weight blocks are already on their way) and read h around the L2 (the eight XCDs' L2s are not
@@ -57,6 +60,12 @@ __device__ long long dec_stamps[1024][20];
 #define DEC_STAMP(n) do {} while (0)
 #endif
 
+// x of another lane of the lane's four (DPP quad permutation)
+template <int PERM>
+__device__ __forceinline__ float quad_swap(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), PERM, 0xF, 0xF, true));
+}
+
 constexpr int kThrough = 1 | 16;  // aux bits of the buffer instructions: sc0 | sc1 (write through / read around the L2)
 
 // ONCE: no expert has more than one row block (the host knows it from T <= 16: a token's k experts differ), so every
@@ -75,9 +84,9 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
   __shared__ int32_t bpre_s[kDecMaxExperts + 1];  // a -> 16-row blocks of the active experts before a
   __shared__ int32_t misc_s[4];                   // [0] number of active experts
   __shared__ DecUnit tab_s[kDecMaxUnits + kDecRing];
-  // partial sums of a unit: [unit parity][wave][half][lane] (a lane's two quads 1 KiB apart: 16-byte accesses of
-  // neighbouring lanes are then contiguous, without bank conflicts)
-  __shared__ f32x4_t red_s[2][NW][2][64];
+  // partial sums of a unit: [unit parity][wave][row][column], the 16-byte pieces of row r stored at piece ^ (r & 7): neither the waves' quads nor the
+  // rows of columns that a wave sums conflict in a bank
+  __shared__ __attribute__((aligned(16))) float red_s[2][NW][16][32];
   __shared__ __attribute__((aligned(16))) float bias_s[kDecMaxUnits][32];  // bias of a unit's 32 columns
   __shared__ u32x4_t xst_s[NW][4][64];  // per wave: one K-stage of a row block's activations on its way into MFMA order
 
@@ -521,7 +530,6 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
       x_settle();
     }
     if (i == 0) DEC_STAMP(14);
-    const bool leader = (i % NW) == wave;
     const int F = cur.frag;
     // ---- this wave's K-slice of the unit; the next unit's blocks follow into the slots as they fall free ----
     typename FR::acc_t acc[2];
@@ -549,14 +557,13 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
       }
       load_w(h_c, j, nxt, nst_next);
     }
-    // ---- the slices meet in LDS; the leader sums them in slice order and runs the epilogue ----
+    // ---- the slices meet in LDS; half of the waves, in turn, sum two of the 16 x 32 results a lane in slice order and
+    // finish them (one wave for all of them held up the others' next unit where units are short; all waves: themselves where they are long) ----
     if (i == 0) DEC_STAMP(15);
     DEC_UNIT_STAMP(i);
     if (i == 0) bias_park(0);
-    {
-      red_s[i & 1][wave][0][lane] = acc[0];
-      red_s[i & 1][wave][1][lane] = acc[1];
-    }
+#pragma unroll
+    for (int g = 0; g < 2; ++g) *reinterpret_cast<f32x4_t*>(&red_s[i & 1][wave][lr][((g * 4 + kg) ^ (lr & 7)) * 4]) = acc[g];
     __syncthreads();
     if (i == 0) DEC_STAMP(16);
     if (i == nr0 && !signalled0) {  // the first unit behind run 0 (it exists and opened a new row block)
@@ -567,41 +574,23 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
       signalled = true;
       signal_blocks(r1b, r1b + nr1);
     }
-    if (leader) {
-      const int row_c = lr < rows ? lr : rows - 1;
-      const int flat = rowflat_s[row0 + row_c];
+    if ((wave & 1) == (i & 1)) {
+      const int r = (wave >> 1) * 4 + (lane >> 4), c = (lane & 15) * 2;
+      const int flat = rowflat_s[row0 + (r < rows ? r : rows - 1)];
       const float gam = gate_s[flat];
-      const f32x4_t bias_lo = *reinterpret_cast<const f32x4_t*>(&bias_s[i][kg * 4]);
-      const f32x4_t bias_hi = *reinterpret_cast<const f32x4_t*>(&bias_s[i][16 + kg * 4]);
-      f32x4_t s0 = {0.f, 0.f, 0.f, 0.f}, s1 = {0.f, 0.f, 0.f, 0.f};
+      const f32x2_t bias = *reinterpret_cast<const f32x2_t*>(&bias_s[i][c]);
+      f32x2_t s = {0.f, 0.f};
 #pragma unroll
-      for (int q = 0; q < NW; ++q) {
-        s0 += red_s[i & 1][q][0][lane];
-        s1 += red_s[i & 1][q][1][lane];
-      }
-      const bool row_ok = lr < rows;
-      if (ph == 1) {
-        // bias, swiglu over the interleaved (gate, linear) pairs, bf16, row (row0 + lr) of h
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          const f32x4_t s = (g == 0 ? s0 : s1) + (g == 0 ? bias_lo : bias_hi);
-          const int n0 = F * 32 + g * 16 + kg * 4;
-          const float o0 = swiglu_f(s[0], s[1], nalpha_log2e, limit);
-          const float o1 = swiglu_f(s[2], s[3], nalpha_log2e, limit);
-          const uint32_t off = (row_ok && n0 < p.N1) ? (uint32_t)(row0 + lr) * (uint32_t)(p.K2 * 2) + (uint32_t)(n0 / 2) * 2u : kDroppedStore;
-          __builtin_amdgcn_raw_buffer_store_b32(pack_bf16x2(o0, o1), hrsrc, off, 0, kThrough);
-        }
-      } else {
-        // bias, gate weight, bf16, flat row t*k + j of y
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          const f32x4_t s = (g == 0 ? s0 : s1) + (g == 0 ? bias_lo : bias_hi);
-          const int n0 = F * 32 + g * 16 + kg * 4;
-          const u32x2_t w = {pack_bf16x2(s[0] * gam, s[1] * gam), pack_bf16x2(s[2] * gam, s[3] * gam)};
-          const uint32_t off = (row_ok && n0 < p.N2) ? (uint32_t)flat * (uint32_t)(p.N2 * 2) + (uint32_t)n0 * 2u : kDroppedStore;
-          __builtin_amdgcn_raw_buffer_store_b64(w, yrsrc, off, 0, kThrough);
-        }
-      }
+      for (int q = 0; q < NW; ++q) s += *reinterpret_cast<const f32x2_t*>(&red_s[i & 1][q][r][((c >> 2) ^ (r & 7)) * 4 + (c & 3)]);
+      s += bias;
+      // One store for either GEMM, of two bf16 results: of y (flat row t*k + j) the gate-weighted columns c and c + 1; of h (row row0 + r), by every
+      // second lane, its and its neighbour's swiglu over the (gate, linear) pair
+      const float o = swiglu_f(s[0], s[1], nalpha_log2e, limit);
+      const float right = quad_swap<0xB1>(o);  // lanes 1 0 3 2 of four
+      const int n = F * 32 + c;
+      const bool up = ph == 1, mine = r < rows && n < (up ? p.N1 : p.N2) && !(up && (lane & 1));
+      const uint32_t off = up ? (uint32_t)(row0 + r) * (uint32_t)(p.K2 * 2) + (uint32_t)n : (uint32_t)flat * (uint32_t)(p.N2 * 2) + (uint32_t)n * 2u;
+      __builtin_amdgcn_raw_buffer_store_b32(up ? pack_bf16x2(o, right) : pack_bf16x2(s[0] * gam, s[1] * gam), up ? hrsrc : yrsrc, mine ? off : kDroppedStore, 0, kThrough);
     }
   };
   // Whole rounds of RD units run without a test between the units: with one, the compiler has to allow for a round
