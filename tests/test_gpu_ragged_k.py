@@ -168,3 +168,23 @@ def test_long_slices(device, n_slices, m, n, rest, out_dtype):
     ref = omoe.matmul_ragged_k(a.t(), b, sizes, offs, offs, out_dtype=torch.float32)
     assert_allclose_gate(ref, out[:, :m, :n].float(), what="ragged-K matmul")
     assert torch.isnan(out[:, m:]).all() and torch.isnan(out[:, :, n:]).all()  # nothing written beside the result
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("m, n, beside", [(8, 8, 8), (72, 56, 8), (136, 200, 0), (120, 328, 24), (264, 120, 16)])
+def test_short_slices_rows_of_broken_lines(device, m, n, beside, out_dtype):
+    """Results whose rows begin and end inside a 128-byte line, tiles that end inside a wave's rows or columns: nothing is written beside them.  One
+    rounding of a sum of at most 40 terms."""
+    import triton_amd.matmul as mm
+    g = torch.Generator().manual_seed(m * n)
+    sizes = torch.tensor([0, 1, 17, 40, 16], dtype=torch.int32)
+    offs = _offsets(sizes, 8)
+    k = int(offs[-1])
+    a, b = torch.randn((k, m), generator=g).to(torch.bfloat16), torch.randn((k, n), generator=g).to(torch.bfloat16)
+    out = torch.full((len(sizes), m + 8, n + beside), float("nan"), dtype=out_dtype, device=device)
+    md = _metadata(sizes, offs, device)
+    mm.matmul(a.to(device).t(), b.to(device), None, a_ragged_metadata=md, b_ragged_metadata=md, c=out[:, :m, :n],
+              precision_config=mm.PrecisionConfig(out_dtype=out_dtype))
+    ref = omoe.matmul_ragged_k(a.t(), b, sizes, offs, offs, out_dtype=torch.float32)
+    assert_allclose_gate(ref, out[:, :m, :n].float(), what="ragged-K matmul")
+    assert torch.isnan(out[:, m:]).all() and torch.isnan(out[:, :, n:]).all()

@@ -296,7 +296,10 @@ __global__ __launch_bounds__(256) void ragged_k_gemm_kernel(const RaggedKParams 
 // What bounds it: writing y (long slices: ragged_k_long.hip).  The same kernel without its loads writes 128 x [2880, 5760] bf16 in 0.77 ms (5.5 TB/s),
 // without its stores it takes 0.85 ms; together 1.13 ms (3.1 ms with the transposition in registers; 2880 x 2880: 1.5 -> 0.62).
 //   * the results go through LDS so that a store instruction writes whole 128-byte lines, with the non-temporal hint
-//     (pieces of 32 bytes: 1.76 ms; with the hint on such pieces 4.0, plain whole lines 1.55, whole lines with the hint 1.40);
+//     (pieces of 32 bytes: 1.76 ms; with the hint on such pieces 4.0, plain whole lines 1.55, whole lines with the hint 1.40) and rows of y that are no multiple
+//     of a line, whose pieces begin and end inside one, by whole rows of the tile: 256 bytes an instruction have two broken lines, 128 of each wave's columns nothing
+//     else (both products of a layer, us: 128 slices of 31 k, 1000 x 2000 and 1000 x 1000 365 -> 295; of 93 k, 864 x 2800 and 1400 x 864 349 -> 313; of 7 k, 1888 x 960 and
+//     480 x 1888 141 -> 134; of 39 k, 2784 x 5568 and 2784 x 2784 1196 -> 1151; whole lines 140 -> 138, 2880 x 5760 and 2880 x 2880 the same);
 //   * stages of 16 k, five buffers, four workgroups per CU: four fifths of the LDS are loads in flight (three buffers
 //     of 32 k and three workgroups: 1.44), and a slice is padded to 16 k only;
 //   * every XCD gets an eighth of EVERY slice: slices differ in length by factors, and with whole slices dealt to the
@@ -448,21 +451,20 @@ __global__ __launch_bounds__(256, 4) void ragged_k_tr_kernel(const RaggedKParams
         }
     }
   } else {
-    // through LDS, so that a store instruction writes eight whole 128-byte lines of the quadrant
+    // through LDS, so that a store instruction writes four whole rows of the tile
     static_assert(kTrBufs * kTrStage >= 4 * 8192, "the four quadrants fit the operand buffers");
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
-    uint8_t* sp = lds + wave * 8192;
 #pragma unroll
-    for (int j = 0; j < 2; ++j) stage_out_rows<YT>(sp, j, lane, acc[0][j], acc[1][j]);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    for (int j = 0; j < 2; ++j) stage_out_rows<YT>(lds + wave * 8192, j, lane, acc[0][j], acc[1][j]);
+    __syncthreads();
+    // a store instruction writes four rows of the whole tile: 256 bytes that lie together
+    const int pc = lane & 15, n = n0 + pc * 8;
+    const uint8_t* sp = lds + ((wave >> 1) + (pc >> 3) * 2) * 8192;
 #pragma unroll
     for (int it = 0; it < 8; ++it) {
-      const int r = it * 8 + (lane >> 3), pc = lane & 7;
-      const u32x4_t q = staged_piece(sp, r, pc);
-      const int m = m0 + mw * 64 + r, n = n0 + nw * 64 + pc * 8;
+      const int r = wave * 32 + it * 4 + (lane >> 4), m = m0 + r;
+      const u32x4_t q = staged_piece(sp, r & 63, pc & 7);
       const uint32_t off = (m < p.M && n < p.N) ? ((uint32_t)m * (uint32_t)p.y_stride_m + (uint32_t)n) * ES : kOutOfRange;
       __builtin_amdgcn_raw_buffer_store_b128(q, ry, off, 0, kNonTemporal);
     }
