@@ -172,6 +172,51 @@ def test_odd_shapes(api, device, T, E, k, d_model, d_ff, bias_dtype, limit):
         assert_close(three, out, maxtol=3e-2, what="one launch against three calls")
 
 
+@pytest.mark.parametrize("T, E, k, d_model, d_ff, bias_dtype, limit", [
+    (12, 24, 4, 992, 544, torch.bfloat16, 7.0),     # one K-stage a wave, two fragments a unit: an odd number of fragments in the second GEMM
+    (40, 20, 4, 1024, 1024, torch.float32, None),   # ... all eight waves with a stage in both
+    (9, 8, 2, 1056, 288, None, 7.0),                # two stages a wave, one fragment: nine stages, and three
+    (14, 96, 8, 1632, 1056, torch.bfloat16, 7.0),   # two stages, two fragments (an odd number of them)
+    (32, 40, 8, 288, 2048, torch.float32, 7.0),     # ... many short units in front of few long ones
+    (2, 3, 1, 2080, 32, None, None),                # three stages, hardly a unit a workgroup
+])
+def test_units_by_k(api, device, T, E, k, d_model, d_ff, bias_dtype, limit):
+    """The stages a wave and the fragments a unit that the length of K and the number of units select."""
+    test_odd_shapes(api, device, T, E, k, d_model, d_ff, bias_dtype, limit)
+
+
+@pytest.mark.parametrize("d, T, k, spread", [
+    (1024, 16, 8, 0.0),  # no second row blocks: known from the tokens
+    (1024, 20, 8, 0.0),  # found by the routing
+    (1024, 32, 8, 3.0),  # experts with two blocks, fewer weights than the caches hold
+    (2880, 20, 4, 0.0),
+    (2880, 40, 4, 1.5),  # a few experts with two blocks: by unit
+    (2880, 64, 4, 4.0),  # many
+])
+def test_weights_fetched_with_the_hint_and_without(api, device, gptoss_weights, d, T, k, spread):
+    """More weights than the caches hold, read once or by several row blocks: the layer against the oracle, twice the same."""
+    from bench import make_moe_weights, to_matmul_layout
+    g = torch.Generator().manual_seed(T + d)
+    x = torch.randn((T, d), generator=g).to(torch.bfloat16)
+    logits = torch.randn((T, 128), generator=g) + spread * torch.randn((128, ), generator=g)
+    if d == 2880:
+        W0, W = gptoss_weights["strided"], gptoss_weights["tiled"]
+    else:
+        W0 = make_moe_weights(128, d, 2 * d, seed=4, device=device)[0]
+        W = to_matmul_layout(W0)
+    ref, r = _oracle_layer(x, logits, k, W0)
+    xd, ld = x.to(device), logits.to(device)
+    outs = []
+    for rep in range(2):
+        out, indx, _ = _run(api, W, xd, ld, k, api.act(1.702, 7.0), return_routing=True)
+        torch.cuda.synchronize()
+        assert api.md.workspace_error_word(xd, ld, k, W["w1"]) == 0
+        assert_equal(r.indx, indx.to(torch.int32), "indx")
+        assert_close(ref, out, maxtol=3e-2, what=f"decode layer T={T} (launch {rep})")
+        outs.append(out.clone())
+    assert torch.equal(outs[0], outs[1])
+
+
 def test_one_launch_layer_in_a_hip_graph(api, device, gptoss_weights):
     """Captured once, replayed three times with new inputs and eager launches in between; every replay must equal the
     eager launch on the same inputs bit for bit."""

@@ -7,9 +7,9 @@
 //
 //   1. EVERY workgroup routes all T tokens itself (the logits are a few KiB): top-k by wave-wide max rounds, softmax,
 //      expert histogram, stable expert-sorted row order - into LDS, no global round trip, no dependence on others.
-//   2. The work is cut into units = (active expert, 16-row block, 32-column weight fragment) of GEMM 1 followed by
+//   2. The work is cut into units = (active expert, 16-row block, one or two 32-column weight fragments) of GEMM 1 followed by
 //      those of GEMM 2; every workgroup takes an equal contiguous share of each list, derived from the LDS tables.
-//   3. The NW waves of a workgroup split the K-stages of a unit (K-slices of XS stages); a wave keeps its slice of the
+//   3. The NW waves of a workgroup take the K-stages of a unit in turn (XS = 1 to 3 each); a wave keeps its part of the
 //      block's activation rows in REGISTERS for as long as the (expert, row block) stays the same, so the inner loop
 //      is: 2 KiB weight block global -> registers (ring, one unit ahead), e2m1 -> bf16 in registers, 16x16x32 MFMA.
 //      The slices meet in LDS once per unit (one barrier); four of the waves, in turn, sum them and run the
@@ -36,10 +36,9 @@ namespace {
 
 constexpr int kDecMaxRows = TK_DECODE_MAX_ROWS;        // T * k
 constexpr int kDecMaxExperts = TK_DECODE_MAX_EXPERTS;  // one expert per thread in the placement pass
-constexpr int kDecMaxUnits = 192;                      // units of one workgroup (the host bounds it)
+constexpr int kDecMaxUnits = 192;                      // units (of one fragment) of a workgroup (the host bounds it)
 constexpr int kDecNW = 8;                              // waves per workgroup = K-slices of a unit
-constexpr int kDecXS = 3;                              // K-stages (of 128) per slice: K <= NW * XS * 128 = 3072
-constexpr int kDecRing = 3;                            // units of weight blocks a wave holds or has requested
+constexpr int kDecXS = 3;                              // K-stages (of 128) per slice at most: K <= NW * XS * 128 = 3072
 constexpr int kDecBlockStride = 32;                    // words between two row blocks' counters (a cache line each)
 constexpr int kDecBlockWords = (kDecMaxRows + kDecMaxRows / 16) * kDecBlockStride;  // 16-row blocks: at most min(E, R) + R / 16
 
@@ -47,7 +46,18 @@ struct DecUnit {
   const uint8_t* w;  // first K-stage of the unit's weight fragment
   const uint8_t* s;
   int32_t key;       // phase << 24 | expert slot a << 8 | row block
-  int32_t frag;      // column fragment F
+  int32_t frag;      // first column fragment F
+  int32_t once;      // its expert has one row block only
+};
+
+// XS: K-stages of a wave's slice, FPU: column fragments of a unit.  A unit costs its chain (weights, products, sums through LDS, barrier) whatever its
+// bytes, so short K take fewer stages a wave, which leaves registers for a deeper ring or for two fragments a unit.
+template <int XS_, int FPU_>
+struct DecCfg {
+  static constexpr int XS = XS_, FPU = FPU_;
+  static constexpr int RING = XS * FPU >= 3 ? 3 : 4;      // units of weight blocks a wave holds or has requested
+  static constexpr int UNITS = kDecMaxUnits / FPU;        // of one workgroup
+  static constexpr int COLS = 32 * FPU;
 };
 
 #ifdef TK_DEC_STAMPS
@@ -66,14 +76,23 @@ __device__ __forceinline__ float quad_swap(float x) {
   return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), PERM, 0xF, 0xF, true));
 }
 
+constexpr int kNonTemporalLoad = 2;
+
+// How the weights are fetched.  With the non-temporal hint where they are read once by the whole grid and more than the caches keep for the next call
+// anyway; the later row blocks of an expert find a fragment in the caches that the hint would take away.  Up to 16 tokens no expert has a second block (a
+// token's k experts differ); beyond, the kernel knows the blocks after its routing: hardly any second ones, all with the hint; up to a third, by unit
+// (whole K of 24 stages only: the branch costs the compiler's wait counts, a drained ring a unit, which shorter units feel more than they gain).  Three
+// copies of the loop are code to be fetched (0.8 us a call), so the host rules out what cannot be.
+// us, 128 experts, top 4, 2880, without and with: no second blocks, 17 tokens 143 / 130, 32 215 / 192, 64 291 / 260; with favourites, 32 tokens (27.6 blocks of
+// 25.7 experts) 90.5 / 83.6, 40 (32.8 of 30.4) 96.5 / 93.0, by unit 89.5, 61 (39.9 of 33.9) 117.2 / 119.1, by unit 111.5; 33 tokens, 96 experts, 768 and 1824, favourites, 100 MB 37.9 / 40.5.
+enum { kFetchPlain, kFetchOnce, kFetchEither };
+constexpr int kLargeBlocks = (128 << 20) / 2176;  // blocks of 32 columns x 128 k, values and scales
 constexpr int kThrough = 1 | 16;  // aux bits of the buffer instructions: sc0 | sc1 (write through / read around the L2)
 
-// ONCE: no expert has more than one row block (the host knows it from T <= 16: a token's k experts differ), so every
-// weight byte is read exactly once by the whole grid and is fetched with the non-temporal hint; with several row
-// blocks on an expert the later ones find the fragment in the L2 and the hint would take that away.
-template <int VPL, bool ONCE>
+template <int VPL, int XS_, int FPU_, int FETCH>
 __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void moe_decode_layer_kernel(const DecodeParams p) {
-  constexpr int NW = kDecNW, XS = kDecXS, NT = NW * 64;
+  typedef DecCfg<XS_, FPU_> C;
+  constexpr int NW = kDecNW, XS = C::XS, FPU = C::FPU, NT = NW * 64;
   typedef Frag<16> FR;
   __shared__ int16_t eid_s[kDecMaxRows];      // expert of flat entry f = t*k + j
   __shared__ float gate_s[kDecMaxRows];       // its gate value
@@ -83,11 +102,11 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
   __shared__ int16_t act_s[kDecMaxExperts];       // a -> expert id, active experts in ascending order
   __shared__ int32_t bpre_s[kDecMaxExperts + 1];  // a -> 16-row blocks of the active experts before a
   __shared__ int32_t misc_s[4];                   // [0] number of active experts
-  __shared__ DecUnit tab_s[kDecMaxUnits + kDecRing];
+  __shared__ DecUnit tab_s[C::UNITS + C::RING];
   // partial sums of a unit: [unit parity][wave][row][column], the 16-byte pieces of row r stored at piece ^ (r & 7): neither the waves' quads nor the
   // rows of columns that a wave sums conflict in a bank
-  __shared__ __attribute__((aligned(16))) float red_s[2][NW][16][32];
-  __shared__ __attribute__((aligned(16))) float bias_s[kDecMaxUnits][32];  // bias of a unit's 32 columns
+  __shared__ __attribute__((aligned(16))) float red_s[2][NW][16][C::COLS];
+  __shared__ __attribute__((aligned(16))) float bias_s[C::UNITS][C::COLS];  // bias of a unit's columns
   __shared__ u32x4_t xst_s[NW][4][64];  // per wave: one K-stage of a row block's activations on its way into MFMA order
 
   const int tid = threadIdx.x;
@@ -233,8 +252,9 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
   const int bh = (nblk + 1) >> 1;  // row blocks of the first half
   // (32-bit arithmetic: nblk <= 272 and nfr1 + nfr2 <= 288, so G * (U1 + U2) stays below 2^25; a 64-bit division is
   // a hundred instructions, and a dozen of them stood between the routing and the first weight request)
-  const int U1 = nblk * p.nfr1, U2 = nblk * p.nfr2;
-  const int L0 = bh * p.nfr1, L1 = U1 - L0, L2 = bh * p.nfr2, L3 = U2 - L2;
+  const int nu1 = (p.nfr1 + FPU - 1) / FPU, nu2 = (p.nfr2 + FPU - 1) / FPU;  // units of a row block
+  const int U1 = nblk * nu1, U2 = nblk * nu2;
+  const int L0 = bh * nu1, L1 = U1 - L0, L2 = bh * nu2, L3 = U2 - L2;
   const int wg = blockIdx.x;
   auto udiv = [](int a, int b) -> int { return (int)((uint32_t)a / (uint32_t)b); };
   // Shares.  The four runs are cut as one list: cut i of a run = floor(i * (S + L) / G) - floor(i * S / G), S = the
@@ -259,29 +279,30 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
   const int r0b = c0b, r0e = c0e, r1b = L0 + c1b, r1e = L0 + c1e;
   const int r2b = c2b, r2e = c2e, r3b = L2 + c3b, r3e = L2 + c3e;
   int nr0 = r0e - r0b, nr1 = r1e - r1b, nr2 = r2e - r2b, nr3 = r3e - r3b;
-  if (nr0 + nr1 + nr2 + nr3 > kDecMaxUnits) {  // (the host's bound rules this out)
+  if (nr0 + nr1 + nr2 + nr3 > C::UNITS) {  // (the host's bound rules this out)
     if (tid == 0) atomicOr(&p.sync[1], 2);
-    nr0 = nr0 < kDecMaxUnits ? nr0 : kDecMaxUnits;
-    nr1 = nr1 < kDecMaxUnits - nr0 ? nr1 : kDecMaxUnits - nr0;
-    nr2 = nr2 < kDecMaxUnits - nr0 - nr1 ? nr2 : kDecMaxUnits - nr0 - nr1;
-    nr3 = nr3 < kDecMaxUnits - nr0 - nr1 - nr2 ? nr3 : kDecMaxUnits - nr0 - nr1 - nr2;
+    nr0 = nr0 < C::UNITS ? nr0 : C::UNITS;
+    nr1 = nr1 < C::UNITS - nr0 ? nr1 : C::UNITS - nr0;
+    nr2 = nr2 < C::UNITS - nr0 - nr1 ? nr2 : C::UNITS - nr0 - nr1;
+    nr3 = nr3 < C::UNITS - nr0 - nr1 - nr2 ? nr3 : C::UNITS - nr0 - nr1 - nr2;
   }
   const int n1 = nr0 + nr1, n2 = nr2 + nr3;
   const int n_units = n1 + n2;
   // (no barrier here: the table below is built from the scan's results, like the row order above)
-  for (int i = tid; i < n_units + kDecRing; i += NT) {
+  for (int i = tid; i < n_units + C::RING; i += NT) {
     DecUnit u;
-    if (i >= n_units) {  // what the loads issued during the last units fetch: one fixed block, never used
+    if (i >= n_units) {  // behind the last unit nothing is fetched
       u.w = p.w1;
       u.s = p.w1s;
       u.key = -1;
       u.frag = 0;
+      u.once = 1;
     } else {
       const bool ph2 = i >= n1;
       const int uu = i < nr0 ? r0b + i : i < n1 ? r1b + (i - nr0) : i < n1 + nr2 ? r2b + (i - n1) : r3b + (i - n1 - nr2);
-      const int nfr = ph2 ? p.nfr2 : p.nfr1;
+      const int nu = ph2 ? nu2 : nu1;
       const int nst = ph2 ? p.nst2 : p.nst1;
-      const int B = udiv(uu, nfr), F = uu - B * nfr;
+      const int B = udiv(uu, nu), F = (uu - B * nu) * FPU;
       int lo = 0, hi = A;  // last a with bpre[a] <= B
       while (hi - lo > 1) {
         const int mid = (lo + hi) >> 1;
@@ -293,6 +314,7 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
       u.s = (ph2 ? p.w2s + (int64_t)e * p.w2s_stride_e : p.w1s + (int64_t)e * p.w1s_stride_e) + (int64_t)F * nst * 128;
       u.key = ((ph2 ? 2 : 1) << 24) | (a << 8) | rb;
       u.frag = F;
+      u.once = bpre_s[a + 1] - bpre_s[a] == 1;
     }
     tab_s[i] = u;
   }
@@ -301,39 +323,14 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
 
   // ---- 3. the stream ----------------------------------------------------------------------------------------
   // lane (lr, kg): weight columns g*16 + lr of the fragment, k-block kg (32 k = 16 packed bytes) of every stage;
-  // this wave's stages of a unit are wave*XS + j
+  // this wave's stages of a unit are wave + j * NW: the waves of a short K have the same share of it
   const uint32_t wlane = (uint32_t)((kg & 1) * 1024 + ((kg >> 1) * 32 + lr) * 16);
   const uint32_t slane = (uint32_t)(lr * 4);
   // weight registers: RD sets of XS stages; unit i lives in set i % RD and, stage by stage as it is consumed, is
   // replaced by unit i + RD.  A wave's requests are answered in order, one unit per unit time, so a block must be
   // requested RD unit times before it is used: with a loaded memory latency of about 4 us, two sets bound a unit at
   // 2 us (what was measured), three at 1.3 us, which is below what HBM delivers (19 KiB per wave on its way).
-  constexpr int RD = kDecRing;
-  u32x4_t wr[RD][XS][2];
-  uint32_t sr[RD][XS][2];
-  u32x4_t xr[XS][4];
-  auto load_w = [&](auto h_c, int j, const DecUnit& u, int nst) __attribute__((always_inline)) {
-    constexpr int H = decltype(h_c)::value;
-    int s = wave * XS + j;
-    s = s < nst ? s : nst - 1;  // stages past the last re-read it (no branch around a load: the compiler's wait counts
-                                // stay exact only in straight-line code); their scales are taken as zero when they are used
-#pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      // (global address space spelled out: the pointers come out of the LDS table, the compiler takes them for generic
-      // ones, and with FLAT loads in flight every wait for memory on this target is a wait for ALL of it, i.e. the ring
-      // of weight blocks would be drained at the head of every unit)
-      const auto* wp = (const __attribute__((address_space(1))) u32x4_t*)(u.w + (int64_t)s * 2048 + g * 256 + wlane);
-      const auto* sp = (const __attribute__((address_space(1))) uint32_t*)(u.s + (int64_t)s * 128 + g * 64 + slane);
-      if constexpr (ONCE) {
-        wr[H][j][g] = __builtin_nontemporal_load(wp);
-        sr[H][j][g] = __builtin_nontemporal_load(sp);
-      } else {
-        wr[H][j][g] = *wp;
-        sr[H][j][g] = *sp;
-      }
-    }
-  };
-  auto unit_nst = [&](const DecUnit& u) __attribute__((always_inline)) -> int { return (u.key >> 24) == 2 ? p.nst2 : p.nst1; };
+  constexpr int RD = C::RING;
   const __amdgpu_buffer_rsrc_t hrsrc = __builtin_amdgcn_make_buffer_rsrc(p.h, 0, (uint32_t)((int64_t)R * p.K2 * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(p.y, 0, (uint32_t)((int64_t)R * p.N2 * 2), 0x00020000);
   const float nalpha_log2e = -p.alpha * 1.4426950408889634f;
@@ -348,19 +345,96 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
     u.s = (const uint8_t*)(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(sc >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)sc));
     u.key = __builtin_amdgcn_readfirstlane(v.key);
     u.frag = __builtin_amdgcn_readfirstlane(v.frag);
+    u.once = XS == 3 ? __builtin_amdgcn_readfirstlane(v.once) : 0;
     return u;
   };
-  // counts GEMM-1 units [from, to) of this workgroup in at their row blocks' counters (unit u belongs to block u / nfr1)
+  // counts GEMM-1 units [from, to) of this workgroup in at their row blocks' counters (unit u belongs to block u / nu1)
   auto signal_blocks = [&](int ub, int ue) __attribute__((always_inline)) {
     if (ue > ub) {
-      const int b_first = udiv(ub, p.nfr1), b_last = udiv(ue - 1, p.nfr1);
+      const int b_first = udiv(ub, nu1), b_last = udiv(ue - 1, nu1);
       for (int b = b_first + tid; b <= b_last; b += NT) {
-        const int lo = b * p.nfr1, hi = lo + p.nfr1;
+        const int lo = b * nu1, hi = lo + nu1;
         const int from = lo > ub ? lo : ub, to = hi < ue ? hi : ue;
         __hip_atomic_fetch_add(&p.sync[2 + b * kDecBlockStride], to - from, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
     }
   };
+  // ---- the biases of this workgroup's units, to LDS: requested in front of the first weight blocks (what is requested behind them is answered behind
+  // them, and the wait would be one for the whole ring), written when the first activations have come.  Four values a thread cover 2048 columns; more take
+  // another round.  As two halves (of a bf16 bias the same one twice), from the activations where there is nothing: a load under a condition is waited for at its end. ----
+  constexpr int BPT = 4, kBiasRound = BPT * NT / C::COLS;  // values of a thread, units of a round
+  uint64_t b1 = (uint64_t)p.b1, b2 = (uint64_t)p.b2;
+  int64_t b1_stride = p.b1_stride_e, b2_stride = p.b2_stride_e;
+  int b1_f32 = p.b1_is_f32, b2_f32 = p.b2_is_f32, n_of1 = p.N1, n_of2 = p.N2;
+  // (opaque: a choice between two of the kernel's arguments by a lane's GEMM becomes a load of them otherwise)
+  asm volatile("" : "+s"(b1), "+s"(b2), "+s"(b1_stride), "+s"(b2_stride), "+s"(b1_f32), "+s"(b2_f32), "+s"(n_of1), "+s"(n_of2));
+  uint16_t bias_lo[BPT], bias_hi[BPT];
+  auto bias_fetch = [&](int first_unit) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < BPT; ++q) {
+      const int idx = first_unit * C::COLS + q * NT + tid, ui = idx / C::COLS;
+      const DecUnit u = tab_s[ui < n_units ? ui : 0];
+      const bool ph2 = (u.key >> 24) == 2, f32 = ph2 ? b2_f32 : b1_f32;
+      const int n = u.frag * 32 + idx % C::COLS;
+      const uint64_t bp = ph2 ? b2 : b1;
+      const bool have = bp && n < (ph2 ? n_of2 : n_of1);
+      const int64_t el = (int64_t)act_s[(u.key >> 8) & 0xFFFF] * (ph2 ? b2_stride : b1_stride) + n;
+      const uint64_t at = have ? bp + ((uint64_t)el << (f32 ? 2 : 1)) : (uint64_t)p.x;
+      bias_lo[q] = *(const __attribute__((address_space(1))) uint16_t*)at;
+      bias_hi[q] = *(const __attribute__((address_space(1))) uint16_t*)(have && f32 ? at + 2 : at);
+    }
+  };
+  auto bias_park = [&](int first_unit) __attribute__((always_inline)) {
+#pragma unroll
+    for (int q = 0; q < BPT; ++q) {
+      const int idx = first_unit * C::COLS + q * NT + tid, ui = idx / C::COLS;
+      if (ui < n_units) {
+        const DecUnit u = tab_s[ui];
+        const bool ph2 = (u.key >> 24) == 2, f32 = ph2 ? b2_f32 : b1_f32;
+        const bool have = (ph2 ? b2 : b1) && u.frag * 32 + idx % C::COLS < (ph2 ? n_of2 : n_of1);
+        const uint32_t hi = bias_hi[q];
+        (&bias_s[0][0])[idx] = bits_f32(!have ? 0u : f32 ? hi << 16 | bias_lo[q] : hi << 16);
+      }
+    }
+  };
+  for (int u0 = kBiasRound; u0 < n_units; u0 += kBiasRound) {
+    bias_fetch(u0);
+    bias_park(u0);
+  }
+  bool signalled0 = nr0 == 0, signalled = n1 == 0;  // see below
+  auto stream = [&](auto mode_c) __attribute__((always_inline)) {
+  constexpr int MODE = decltype(mode_c)::value;
+  u32x4_t wr[RD][XS][FPU][2];
+  uint32_t sr[RD][XS][FPU][2];
+  u32x4_t xr[XS][4];
+  // (Stages and fragments past the unit's last are past the resource's end: zeros, and no memory is asked for them.  No branch around a load: the compiler's wait
+  // counts stay exact only in straight-line code.)
+  uint32_t w_at[XS], s_at[XS];
+#pragma unroll
+  for (int j = 0; j < XS; ++j) w_at[j] = wlane + (uint32_t)(wave + j * NW) * 2048u, s_at[j] = slane + (uint32_t)(wave + j * NW) * 128u;
+  auto load_w = [&](auto h_c, int j, const DecUnit& u, int nst, int nfr) __attribute__((always_inline)) {
+    constexpr int H = decltype(h_c)::value;
+    auto fetch = [&](auto aux_c) __attribute__((always_inline)) {
+      constexpr int AUX = decltype(aux_c)::value;
+#pragma unroll
+      for (int f = 0; f < FPU; ++f) {
+        const int stages = FPU == 1 || u.frag + f < nfr ? nst : 0;
+        const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(u.w + (int64_t)f * nst * 2048), 0, stages * 2048, 0x00020000);
+        const __amdgpu_buffer_rsrc_t srsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(u.s + (int64_t)f * nst * 128), 0, stages * 128, 0x00020000);
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          wr[H][j][f][g] = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_at[j] + g * 256, 0, AUX);
+          sr[H][j][f][g] = __builtin_amdgcn_raw_buffer_load_b32(srsrc, s_at[j] + g * 64, 0, AUX);
+        }
+      }
+    };
+    if (MODE == kFetchOnce || (MODE == kFetchEither && u.once))
+      fetch(template_int<kNonTemporalLoad>{});
+    else
+      fetch(template_int<0>{});
+  };
+  auto unit_nst = [&](const DecUnit& u) __attribute__((always_inline)) -> int { return u.key < 0 ? 0 : (u.key >> 24) == 2 ? p.nst2 : p.nst1; };
+  auto unit_nfr = [&](const DecUnit& u) __attribute__((always_inline)) -> int { return (u.key >> 24) == 2 ? p.nfr2 : p.nfr1; };
   // This wave's K-slice of a row block's activation rows: x through the expert-sorted order for GEMM 1, h for GEMM 2.
   // The MFMA wants row lr's k-block kg in lane (lr, kg): loaded that way, the sixteen lanes that one pass of a load
   // serves touch sixteen rows, i.e. sixteen cache lines for 16 bytes each.  So the rows are loaded four lanes to a row
@@ -380,7 +454,7 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
     const int K = ph == 2 ? p.K2 : p.K1;
     // first k of this lane in its wave's slice (opaque: otherwise the twelve addresses below are computed once, ahead
     // of the loop, and parked in scratch memory, which turns every reload into a chain of dependent memory round trips)
-    int kb = wave * (XS * 128) + c * 8;
+    int kb = wave * 128 + c * 8;
     asm volatile("" : "+v"(kb));
     uint32_t base;
     if constexpr (ph == 2) {
@@ -393,8 +467,8 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
     for (int j = 0; j < XS; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int k0 = kb + j * 128 + q * 32;
-        // past K the weights are zero (padding) or their scales are zeroed (stages past the last): zeros will do
+        const int k0 = kb + j * (NW * 128) + q * 32;
+        // past K the weights are zero (padding, stages past the last): zeros will do
         const uint32_t off = (valid && k0 < K) ? base + (uint32_t)k0 * 2u : kDroppedStore;
         if constexpr (ph == 2)
           xr[j][q] = __builtin_amdgcn_raw_buffer_load_b128(hrsrc, off, 0, kThrough);
@@ -419,6 +493,7 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
   };
   int cur_key = 0;
   if (n_units > 0) {
+    bias_fetch(0);
     // the first unit's activation slice is requested in front of the weight blocks (a wave's requests are answered in
     // order, and the three units of weight blocks primed below keep the memory system busy for microseconds)
     const DecUnit first = uniform_unit(0);
@@ -430,53 +505,13 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
     static_for<0, RD>([&](auto h_c) __attribute__((always_inline)) {
       const DecUnit u = uniform_unit(decltype(h_c)::value);
 #pragma unroll
-      for (int j = 0; j < XS; ++j) load_w(h_c, j, u, unit_nst(u));
+      for (int j = 0; j < XS; ++j) load_w(h_c, j, u, unit_nst(u), unit_nfr(u));
     });
     // (here, in straight-line code behind the requests, the wait in front of the LDS writes counts the weight blocks
     // out: behind the bias loops below it would be a wait for everything requested so far)
     if (x_first) x_settle();
+    bias_park(0);
   }
-  // The biases of this workgroup's units (32 columns each) go to LDS once: requested behind the first weight blocks,
-  // written in front of the first unit's barrier.  Four values per thread cover 64 units; more take another round.
-  constexpr int BPT = 4;
-  uint32_t bias_raw[BPT];
-  auto bias_fetch = [&](int first_unit) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < BPT; ++q) {
-      const int idx = first_unit * 32 + q * NT + tid, ui = idx >> 5, c = idx & 31;
-      bias_raw[q] = 0u;
-      if (ui < n_units) {
-        const DecUnit u = tab_s[ui];
-        const bool ph2 = (u.key >> 24) == 2;
-        const void* bp = ph2 ? p.b2 : p.b1;
-        const int n = u.frag * 32 + c;
-        if (bp && n < (ph2 ? p.N2 : p.N1)) {
-          const int64_t at = (int64_t)act_s[(u.key >> 8) & 0xFFFF] * (ph2 ? p.b2_stride_e : p.b1_stride_e) + n;
-          // (raw bits: anything computed from the value here would wait for it, behind the weight blocks just requested)
-          bias_raw[q] = (ph2 ? p.b2_is_f32 : p.b1_is_f32) ? static_cast<const uint32_t*>(bp)[at] : (uint32_t)static_cast<const uint16_t*>(bp)[at];
-        }
-      }
-    }
-  };
-  auto bias_park = [&](int first_unit) __attribute__((always_inline)) {
-#pragma unroll
-    for (int q = 0; q < BPT; ++q) {
-      const int idx = first_unit * 32 + q * NT + tid;
-      const int ui = idx >> 5;
-      if (ui < n_units) {
-        const bool f32 = (tab_s[ui].key >> 24) == 2 ? p.b2_is_f32 : p.b1_is_f32;
-        (&bias_s[0][0])[idx] = bits_f32(f32 ? bias_raw[q] : bias_raw[q] << 16);
-      }
-    }
-  };
-  constexpr int kBiasRound = BPT * NT / 32;  // units per round
-  for (int u0 = kBiasRound; u0 < n_units; u0 += kBiasRound) {  // (more than 64 units: the later rounds up front)
-    bias_fetch(u0);
-    bias_park(u0);
-  }
-  DEC_STAMP(12);
-  bias_fetch(0);
-  DEC_STAMP(13);
   // A finished GEMM-1 run is counted in without draining the wave's memory queue.  A wave's loads and stores complete
   // in issue order.  The epilogue of a run's last unit stores its rows of h right behind that unit's barrier; the
   // next unit opens another row block (or the other GEMM), so EVERY wave starts it by fetching new activation rows
@@ -484,7 +519,6 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
   // reached memory, and the run is counted in there.  (A wait that comes earlier than that, possible only for a
   // workgroup with next to no units, drains the queue and counts in first: a workgroup must never wait for rows
   // that it has not counted in itself.)
-  bool signalled0 = nr0 == 0, signalled = n1 == 0;
   auto unit_body = [&](auto h_c, int i) __attribute__((always_inline)) {
     constexpr int H = decltype(h_c)::value;
     const DecUnit cur = uniform_unit(i);
@@ -508,12 +542,12 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
           if (!signalled) signal_blocks(r1b, r1b + nr1);
           signalled0 = signalled = true;
         }
-        // the block's rows of h are complete when all nfr1 GEMM-1 units of the block have been counted in
+        // the block's rows of h are complete when all nu1 GEMM-1 units of the block have been counted in
         if (tid == 0) {
           int spins = 0;
           // (polled gently, and every block's counter in a cache line of its own: a few hundred workgroups polling
           // one line at full speed slow down every stream that crosses that memory channel)
-          while (__hip_atomic_load(&p.sync[2 + blk * kDecBlockStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < p.nfr1) {
+          while (__hip_atomic_load(&p.sync[2 + blk * kDecBlockStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < nu1) {
             __builtin_amdgcn_s_sleep(16);
             if (++spins > p.spin_limit) {
               atomicOr(&p.sync[1], 1);
@@ -532,38 +566,38 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
     if (i == 0) DEC_STAMP(14);
     const int F = cur.frag;
     // ---- this wave's K-slice of the unit; the next unit's blocks follow into the slots as they fall free ----
-    typename FR::acc_t acc[2];
+    typename FR::acc_t acc[FPU][2];
 #pragma unroll
-    for (int g = 0; g < 2; ++g)
+    for (int f = 0; f < FPU; ++f)
 #pragma unroll
-      for (int c = 0; c < 4; ++c) acc[g][c] = 0.f;
-    const int nst_next = unit_nst(nxt);
-    const int nst_cur = ph == 2 ? p.nst2 : p.nst1;
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) acc[f][g][c] = 0.f;
+    const int nst_next = unit_nst(nxt), nfr_next = unit_nfr(nxt);
 #pragma unroll
     for (int j = 0; j < XS; ++j) {
-      const uint32_t live = wave * XS + j < nst_cur ? 0xFFu : 0u;  // (uniform) a stage past the last contributes nothing
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        bf16x8_t wf[2];
-#pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          const u32x4_t v = wr[H][j][g];
-          const uint32_t raw = t == 0 ? v.x : t == 1 ? v.y : t == 2 ? v.z : v.w;
-          wf[g] = dequant8(raw, bits_f32(((sr[H][j][g] >> (8 * kg)) & live) << 23));
-        }
         const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, xr[j][t]);
 #pragma unroll
-        for (int g = 0; g < 2; ++g) acc[g] = FR::mma(wf[g], xf, acc[g]);
+        for (int f = 0; f < FPU; ++f)
+#pragma unroll
+          for (int g = 0; g < 2; ++g) {
+            const u32x4_t v = wr[H][j][f][g];
+            const uint32_t raw = t == 0 ? v.x : t == 1 ? v.y : t == 2 ? v.z : v.w;
+            acc[f][g] = FR::mma(dequant8(raw, bits_f32(((sr[H][j][f][g] >> (8 * kg)) & 0xFFu) << 23)), xf, acc[f][g]);
+          }
       }
-      load_w(h_c, j, nxt, nst_next);
+      load_w(h_c, j, nxt, nst_next, nfr_next);
     }
     // ---- the slices meet in LDS; half of the waves, in turn, sum two of the 16 x 32 results a lane in slice order and
     // finish them (one wave for all of them held up the others' next unit where units are short; all waves: themselves where they are long) ----
     if (i == 0) DEC_STAMP(15);
     DEC_UNIT_STAMP(i);
-    if (i == 0) bias_park(0);
 #pragma unroll
-    for (int g = 0; g < 2; ++g) *reinterpret_cast<f32x4_t*>(&red_s[i & 1][wave][lr][((g * 4 + kg) ^ (lr & 7)) * 4]) = acc[g];
+    for (int f = 0; f < FPU; ++f)
+#pragma unroll
+      for (int g = 0; g < 2; ++g) *reinterpret_cast<f32x4_t*>(&red_s[i & 1][wave][lr][f * 32 + ((g * 4 + kg) ^ (lr & 7)) * 4]) = acc[f][g];
     __syncthreads();
     if (i == 0) DEC_STAMP(16);
     if (i == nr0 && !signalled0) {  // the first unit behind run 0 (it exists and opened a new row block)
@@ -578,19 +612,21 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
       const int r = (wave >> 1) * 4 + (lane >> 4), c = (lane & 15) * 2;
       const int flat = rowflat_s[row0 + (r < rows ? r : rows - 1)];
       const float gam = gate_s[flat];
-      const f32x2_t bias = *reinterpret_cast<const f32x2_t*>(&bias_s[i][c]);
-      f32x2_t s = {0.f, 0.f};
-#pragma unroll
-      for (int q = 0; q < NW; ++q) s += *reinterpret_cast<const f32x2_t*>(&red_s[i & 1][q][r][((c >> 2) ^ (r & 7)) * 4 + (c & 3)]);
-      s += bias;
       // One store for either GEMM, of two bf16 results: of y (flat row t*k + j) the gate-weighted columns c and c + 1; of h (row row0 + r), by every
       // second lane, its and its neighbour's swiglu over the (gate, linear) pair
-      const float o = swiglu_f(s[0], s[1], nalpha_log2e, limit);
-      const float right = quad_swap<0xB1>(o);  // lanes 1 0 3 2 of four
-      const int n = F * 32 + c;
-      const bool up = ph == 1, mine = r < rows && n < (up ? p.N1 : p.N2) && !(up && (lane & 1));
-      const uint32_t off = up ? (uint32_t)(row0 + r) * (uint32_t)(p.K2 * 2) + (uint32_t)n : (uint32_t)flat * (uint32_t)(p.N2 * 2) + (uint32_t)n * 2u;
-      __builtin_amdgcn_raw_buffer_store_b32(up ? pack_bf16x2(o, right) : pack_bf16x2(s[0] * gam, s[1] * gam), up ? hrsrc : yrsrc, mine ? off : kDroppedStore, 0, kThrough);
+#pragma unroll
+      for (int f = 0; f < FPU; ++f) {
+        f32x2_t s = {0.f, 0.f};
+#pragma unroll
+        for (int q = 0; q < NW; ++q) s += *reinterpret_cast<const f32x2_t*>(&red_s[i & 1][q][r][f * 32 + ((c >> 2) ^ (r & 7)) * 4 + (c & 3)]);
+        s += *reinterpret_cast<const f32x2_t*>(&bias_s[i][f * 32 + c]);
+        const float o = swiglu_f(s[0], s[1], nalpha_log2e, limit);
+        const float right = quad_swap<0xB1>(o);  // lanes 1 0 3 2 of four
+        const int n = (F + f) * 32 + c;
+        const bool up = ph == 1, mine = r < rows && n < (up ? p.N1 : p.N2) && !(up && (lane & 1));
+        const uint32_t off = up ? (uint32_t)(row0 + r) * (uint32_t)(p.K2 * 2) + (uint32_t)n : (uint32_t)flat * (uint32_t)(p.N2 * 2) + (uint32_t)n * 2u;
+        __builtin_amdgcn_raw_buffer_store_b32(up ? pack_bf16x2(o, right) : pack_bf16x2(s[0] * gam, s[1] * gam), up ? hrsrc : yrsrc, mine ? off : kDroppedStore, 0, kThrough);
+      }
     }
   };
   // Whole rounds of RD units run without a test between the units: with one, the compiler has to allow for a round
@@ -602,6 +638,19 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
   static_for<0, RD - 1>([&](auto h_c) __attribute__((always_inline)) {
     if (i_unit + decltype(h_c)::value < n_units) unit_body(h_c, i_unit + decltype(h_c)::value);
   });
+  };  // stream
+  if constexpr (FETCH != kFetchEither) {
+    stream(template_int<FETCH>{});
+  } else {
+    const int again = nblk - A;
+    const bool large = A * (p.nfr1 * p.nst1 + p.nfr2 * p.nst2) > kLargeBlocks;
+    if (large && again * (XS == 3 ? 20 : 10) <= nblk)
+      stream(template_int<kFetchOnce>{});
+    else if (XS == 3 && large && again * 3 <= nblk)
+      stream(template_int<kFetchEither>{});
+    else
+      stream(template_int<kFetchPlain>{});
+  }
   DEC_STAMP(6);
   // ---- 4./5. hand-over of whatever is still to be counted in, then the combine of this workgroup's rows of y ----
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -611,17 +660,17 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
   DEC_STAMP(7);
   int32_t* arrivals = p.sync + 2 + kDecBlockWords;
   const bool out_vec = (p.out_stride & 7) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
-  for (int it0 = 0; it0 < n2 * 64; it0 += NT) {
-    // item = (unit, row of its block, group of 8 columns): the group-0 thread counts the row in and tells the other three
+  for (int it0 = 0; it0 < n2 * (64 * FPU); it0 += NT) {
+    // item = (unit, its fragment, row of its block, group of 8 columns): the group-0 thread counts the row in and tells the other three
     const int it = it0 + tid;
     int seen = -1, token = 0, F = 0;
-    if (it < n2 * 64) {
-      const DecUnit u = tab_s[n1 + (it >> 6)];
+    if (it < n2 * (64 * FPU)) {
+      const DecUnit u = tab_s[n1 + it / (64 * FPU)];
       const int r = (it >> 2) & 15;
       const int a = (u.key >> 8) & 0xFFFF, rb = u.key & 0xFF;
       const int e = act_s[a];
-      F = u.frag;
-      if (rb * 16 + r < hist_s[e]) {
+      F = u.frag + (FPU == 1 ? 0 : (it >> 6) % FPU);
+      if (rb * 16 + r < hist_s[e] && (FPU == 1 || F < p.nfr2)) {
         token = rowflat_s[offs_s[e] + rb * 16 + r] / k;
         if ((it & 3) == 0) seen = __hip_atomic_fetch_add(&arrivals[token * p.nfr2 + F], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
@@ -677,7 +726,7 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
 }
 
 // workgroups of the kernel that are resident together on the current device (cached per device and variant)
-template <int VPL>
+template <int VPL, int XS, int FPU, int FETCH>
 int resident_workgroups() {
   static std::atomic<int> cached[64];
   int dev = 0;
@@ -685,13 +734,52 @@ int resident_workgroups() {
   int n = cached[dev].load(std::memory_order_relaxed);
   if (n == 0) {
     int per_cu = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(moe_decode_layer_kernel<VPL, false>), kDecNW * 64, 0) != hipSuccess || per_cu <= 0)
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(moe_decode_layer_kernel<VPL, XS, FPU, FETCH>), kDecNW * 64, 0) != hipSuccess || per_cu <= 0)
       return 0;
     per_cu = 1;  // (a wave holds up to two units of weight blocks in its registers: one workgroup fills a CU)
     n = per_cu * device_cu_count();
     cached[dev].store(n, std::memory_order_relaxed);
   }
   return n;
+}
+
+// Units of one workgroup: at most min(E, R) + R / 16 row blocks, dealt evenly (+1 per run)
+bool units_fit(const DecodeParams& p, int64_t units_of_block, int grid, int max_units) {
+  const int64_t R = (int64_t)p.T * p.k, max_blocks = (R < p.E ? R : p.E) + R / 16;
+  return max_blocks * units_of_block / grid + 4 <= max_units;
+}
+
+template <int VPL, int XS, int FPU, int FETCH>
+int32_t launch_layer(const DecodeParams& p, hipStream_t st) {
+  typedef DecCfg<XS, FPU> C;
+  const int grid = resident_workgroups<VPL, XS, FPU, FETCH>();
+  if (grid <= 0) return fail(TK_ERR_LAUNCH, "tk_moe_decode_layer: cannot determine how many workgroups are resident together");
+  if (!units_fit(p, cdiv(p.nfr1, FPU) + cdiv(p.nfr2, FPU), grid, C::UNITS)) {
+    if constexpr (FPU > 1) return launch_layer<VPL, kDecXS, 1, FETCH>(p, st);
+    return fail(TK_ERR_UNSUPPORTED, "tk_moe_decode_layer: row blocks of %d x %d rows x %d fragments over %d workgroups exceed the kernel's unit table", p.T, p.k, p.nfr1 + p.nfr2, grid);
+  }
+  hipLaunchKernelGGL((moe_decode_layer_kernel<VPL, XS, FPU, FETCH>), dim3((unsigned)grid), dim3(kDecNW * 64), 0, st, p);
+  return check_launch("moe_decode_layer_kernel");
+}
+
+// K of up to 8 stages: one a wave, two fragments a unit; up to 16: two, and two fragments where there are some twenty units of one a workgroup (with fewer the
+// last ones are too long).  us, stages of three a wave and one fragment a unit / two stages and one / two and two: 60 tokens, 96 experts, top 4, 2048 136 / 123 /
+// 116, 16 experts 48.3 / 46.4 / 49.2; 20 tokens, 32 experts, top 2, 1600 39.5 / 36.6 / 38.1.  One stage and two fragments: 100 tokens, 64 experts, top 2, 1024 58 -> 46; 12 tokens, 32 experts,
+// top 8, 1024 40 -> 31.
+template <int VPL, int FETCH>
+int32_t launch_layer(const DecodeParams& p, hipStream_t st) {
+  const int nst = p.nst1 > p.nst2 ? p.nst1 : p.nst2, R = p.T * p.k;
+  const bool two = (int64_t)(R < p.E ? R : p.E) * (p.nfr1 + p.nfr2) >= 20 * device_cu_count();
+  if (nst <= kDecNW) return launch_layer<VPL, 1, 2, FETCH>(p, st);
+  if (nst <= 2 * kDecNW) return two ? launch_layer<VPL, 2, 2, FETCH>(p, st) : launch_layer<VPL, 2, 1, FETCH>(p, st);
+  return launch_layer<VPL, kDecXS, 1, FETCH>(p, st);
+}
+
+template <int VPL>
+int32_t launch_layer(const DecodeParams& p, hipStream_t st) {
+  const int R = p.T * p.k;
+  if ((int64_t)(R < p.E ? R : p.E) * (p.nfr1 * p.nst1 + p.nfr2 * p.nst2) <= kLargeBlocks) return launch_layer<VPL, kFetchPlain>(p, st);
+  return p.T <= 16 ? launch_layer<VPL, kFetchOnce>(p, st) : launch_layer<VPL, kFetchEither>(p, st);
 }
 
 }  // namespace
@@ -788,27 +876,6 @@ extern "C" int32_t tk_moe_decode_layer(const tk_decode_layer_desc* d, tk_stream_
   p.vals_out = d->vals_out;
   p.spin_limit = d->spin_limit > 0 ? d->spin_limit : (1 << 22);
   if (d->spin_limit <= 0 && decode_by_rows(T, k, d->d_ff, d->d_model)) return decode_launch_rows(p, static_cast<hipStream_t>(stream));
-  const bool small_e = E <= 128;
-  int grid = small_e ? resident_workgroups<8>() : resident_workgroups<kDecMaxExperts / 16>();
-  if (grid <= 0) return fail(TK_ERR_LAUNCH, "tk_moe_decode_layer: cannot determine how many workgroups are resident together");
-  // units of one workgroup: at most min(E, R) + R / 16 row blocks, each with nfr1 + nfr2 fragments, dealt evenly (+1 per run)
-  const int64_t max_blocks = (R < E ? R : E) + R / 16;
-  if (max_blocks * (p.nfr1 + p.nfr2) / grid + 4 > kDecMaxUnits)
-    return fail(TK_ERR_UNSUPPORTED, "tk_moe_decode_layer: %lld row blocks x %d fragments over %d workgroups exceed the kernel's unit table", (long long)max_blocks, p.nfr1 + p.nfr2, grid);
   hipStream_t st = static_cast<hipStream_t>(stream);
-  const bool once = T <= 16;  // at most 16 rows, i.e. one row block, per expert: measured 43.0 -> 41.5 us at T = 4, 63.9 -> 61.1 at 16
-                              // (gpt-oss shape), and 102 -> 107 us at T = 64 with skewed routing, hence the switch
-  const dim3 g((unsigned)grid), b(kDecNW * 64);
-  if (small_e) {
-    if (once)
-      hipLaunchKernelGGL((moe_decode_layer_kernel<8, true>), g, b, 0, st, p);
-    else
-      hipLaunchKernelGGL((moe_decode_layer_kernel<8, false>), g, b, 0, st, p);
-  } else {
-    if (once)
-      hipLaunchKernelGGL((moe_decode_layer_kernel<kDecMaxExperts / 16, true>), g, b, 0, st, p);
-    else
-      hipLaunchKernelGGL((moe_decode_layer_kernel<kDecMaxExperts / 16, false>), g, b, 0, st, p);
-  }
-  return check_launch("moe_decode_layer_kernel");
+  return E <= 128 ? launch_layer<8>(p, st) : launch_layer<kDecMaxExperts / 16>(p, st);
 }
