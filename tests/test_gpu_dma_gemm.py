@@ -240,3 +240,11 @@ def test_square_tiles_where_a_routing_divides_worse_into_tall_ones(device, dtype
     ref = omoe.matmul(x.cpu(), w.cpu(), bias.cpu(), counts, gather_indx=gi.cpu()[rows], out_dtype=torch.float32)
     ref = (omoe.swiglu(ref, 1.702, 7.0).float() if swiglu else ref) * gam.cpu()[rows][:, None]
     assert_allclose_gate(ref, out.cpu()[sc.cpu()[rows].long()], what=f"{dtype} square tiles")
+
+
+@pytest.mark.parametrize("sizes", [[0, 1, 31, 32, 33, 63, 64, 40], [2, 0, 31, 33, 64, 65, 129, 2], [5]])
+@pytest.mark.parametrize("k, n", [(32, 8), (144, 264), (528, 1032), (1040, 72)])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_narrow_tiles_of_few_rows(device, sizes, k, n, swiglu):
+    """e4m3, few rows a slice and few columns: tiles of 64 x 64 and 256 of K a stage, beside whole ones for a slice of more."""
+    _check(device, "e4m3", 128, sizes, k, n, swiglu=swiglu)

@@ -13,13 +13,27 @@ int32_t launch_cfg(const GemmParams& p, int grid_m, bool swiglu, hipStream_t st)
   if (tiles <= 0) return TK_OK;
   if (tiles > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_moe_gemm: grid too large");
   q.total_tiles = (int32_t)tiles;
-  const unsigned grid = dma_grid(p, C::PER_CU, tiles);
+  unsigned grid = dma_grid(p, C::PER_CU, tiles);
   auto launch = [&](auto kern) -> int32_t {
     if (const int32_t rc = allow_dynamic_lds(reinterpret_cast<const void*>(kern), C::LDS)) return rc;
     hipLaunchKernelGGL(kern, dim3(grid), dim3(C::NW * 64), C::LDS, st, q);
     return check_launch("moe_gemm_dma_kernel");
   };
-  if (reads_once(p.M, p.slice_sizes ? p.n_slices : 1, C::BM, p.N, p.K * (WK == WK_FP8 ? 1 : 2)))
+  const int64_t slices = p.slice_sizes ? p.n_slices : 1;
+  const bool once = reads_once(p.M, slices, C::BM, p.N, p.K * (WK == WK_FP8 ? 1 : 2));
+  // Tiles of 64 x 64 and 256 of K a stage (the narrow ones of short row blocks) where slices have few rows and those of 128 columns are not two a CU: twice
+  // the workgroups read the weights.  Layers, us: 8 experts, top 2, d 2048, d_ff 13312, 28 tokens 154 -> 130; d 1024, d_ff 8192, 128 tokens 87 -> 74; d 2048, d_ff 4096,
+  // 200 tokens 74 -> 68; 16 experts, d 1024, d_ff 2560, 108 tokens 52 -> 49; d 1152, d_ff 5120, 406 91.4 -> 90.4.  Up to 52 rows a slice, beyond which slices of over 64,
+  // whose tiles stay, are many (62: d 1536, d_ff 2048 48.0 -> 49.2).
+  if constexpr (TILE == kDma128 && WK == WK_FP8) {
+    const int64_t wide = slices * q.grid_n;
+    if (p.M <= slices * 52 && wide * 2 <= dma_grid(p, C::PER_CU, wide * 2)) {
+      grid = dma_grid(p, C::PER_CU, wide * 2);
+      if (once) return swiglu ? launch(moe_gemm_dma_kernel<WK, TILE, true, true, true>) : launch(moe_gemm_dma_kernel<WK, TILE, false, true, true>);
+      return swiglu ? launch(moe_gemm_dma_kernel<WK, TILE, true, true, false>) : launch(moe_gemm_dma_kernel<WK, TILE, false, true, false>);
+    }
+  }
+  if (once)
     return swiglu ? launch(moe_gemm_dma_kernel<WK, TILE, true, false, true>) : launch(moe_gemm_dma_kernel<WK, TILE, false, false, true>);
   if constexpr (TILE == kDma256) {
     // (the other kernel, half a microsecond faster to start, where all tiles are one round, and its stages are half a percent shorter where they
