@@ -109,6 +109,12 @@ RULED = [
     ("mxfp8", "128x512", 128, 928, 544, [127, 128, 129, 65, 64, 1, 33, 97, 96]),
     ("mxfp8", "128x512", 64, 544, 1024, [127, 128, 129, 150, 255, 256, 1, 160]),
 ]
+# MXFP8 rows of more than 104 a slice, by what the tiles cost
+RULED += [
+    ("mxfp8", "64x512", 32, 608, 864, [127, 128, 129, 192, 193, 130]),
+    ("mxfp8", "128x512", 16, 672, 2112, [255, 256, 257, 300, 260, 268]),
+    ("mxfp8", "160x512", 16, 672, 1856, [480, 481, 560, 640, 641, 340]),
+]
 
 
 @pytest.mark.parametrize("kind, tile, e, k, n, sizes", RULED)

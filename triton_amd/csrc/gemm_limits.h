@@ -3,6 +3,7 @@
 // blocks which only such a kernel has are never chosen for a call that it cannot run.  And how a decode layer is launched: its entry
 // point (moe_decode_layer.hip) and those who make its workspace go by the same rule.
 #pragma once
+#include <math.h>
 #include <stdint.h>
 
 namespace tk {
@@ -73,11 +74,12 @@ inline bool reads_once(int64_t rows, int64_t n_slices, int64_t block_rows, int64
 //   favourites 37.6, 24.8 and 31.4, 16.5; the whole layers 101, 54 and 56, 42.)
 // MXFP8 rows, whose stage is half as long to multiply: the kernel before (128 x 256 tiles, weights in registers) stays where its tiles are one round (32
 // slices, K 2400, N 1920: 18 rows 21 against 24, 50 22 against 30).  Beyond that tiles as high as a routing with favourites needs as well, since the epilogue
-// costs by rows: 128 x 512 from 24 rows; 64 x 512 below, and longer where the tiles of 512 columns are less than three a CU, where 32 x 256 divides better below.
+// costs by rows: 128 x 512 from 40 rows, 64 x 512 below (whole layers, 64 / 128 rows, random and with favourites: 128 slices of 2880, 25 rows 324 / 355 and 265 / 263, 31 340 /
+// 371 and 292 / 296, 37 353 / 386 and 303 / 329, 44 382 / 394 and 339 / 333, 50 412 / 404 and 366 / 361; of 1408, 26 rows 107 / 122 and 99 / 94, 32 112 / 128 and 100 / 108; 64 slices of 2048, 36
+// rows 105 / 110 and 107 / 109, 44 121 / 114 and 118 / 110), and 32 x 256 up to 24 where the tiles of 512 columns are less than three a CU.
 // Where these are just one round if all slices have rows, a routing with favourites makes 64-row blocks a second one from about 32 rows on (64 slices, K and N
 // 2048: 37 rows, random / favourites, before 38 / 39, 64 x 512 33 / 42, 128 x 512 33 / 36; 32 slices, N 4096: 37 / 38, 32 / 42, 33 / 36; 160 tiles, K 960, N 2400: 19 /
-// 21, 17 / 17, 18 / 23).  160 x 512 takes over at 104 rows, or where two row blocks of 128 are more than a round (before / 128 x 512 / 160 x 512: 16 slices, K 1024, N
-// 4096: 125 rows 30 / 26 / 32, 175 32 / 28 / 33; 32 slices, K 2400, N 1920: 125 rows 47 / 41 / 49, 176 50 / 43 / 52; K 960, N 2400: 125 rows 28 / 25 / 29, 162 30 / 35 / 30).
+// 21, 17 / 17, 18 / 23). 
 // (All tokens on the same few experts, which a balanced router does not do, leave the tiles of 512 columns fewer than CUs, or just over a round, more often
 // than the 128 x 256 ones before; layers: 128 experts of 2880, four of them live, 300 tokens 90, 83, 700 139, 162, 1400 206, 237, 2300 312, 292; 96 experts, K 1696 and 1088, 900 tokens
 // 74, 78; 64 experts of 1024, two live, 300 41, 37, 1500 51, 60.)
@@ -89,17 +91,51 @@ inline bool reads_once(int64_t rows, int64_t n_slices, int64_t block_rows, int64
 struct MxwTile {
   int32_t rows, cols;
 };
-inline MxwTile mxw_tile(int64_t rows, int64_t n_slices, int64_t N, bool mx8) {
+// MXFP8 rows, more than 104 a slice: by what a tile costs.  A workgroup's tile of bm rows takes `start` + `stage` us for every 128 of K, the rounds of 256
+// workgroups follow one another, and a routing makes about 1 + sum over j of P(rows > j bm) row blocks of a slice (normal, a fifth wider than random; from
+// three on, half a block more than there are rows for).  How many rounds a number of tiles is near a whole one is not known: the mean of 5 % less and
+// more.  The two constants of each tile come from products of one round (K 512 and 1600, 16 slices of 108 rows); the rest follows, within some 10 %: us, predicted /
+// measured, 64 x 512, 128 x 512, 160 x 512, and the 128 x 256 tiles with weights in registers:
+//   16 slices, K 2752, N 2368, 138 rows 30 / 31, 44 / 43, 59 / 50; K 1696, N 5440, 474 rows 114 / 115, 102 / 91, 119 / 112, 108 / 105; K 2720, N 1696 70 / 56, 64 / 65, 59 / 53, 49 / 49
+//   32 slices, K 2496, N 4608, 212 rows 126 / 130, 115 / 112, 157 / 131, 108 / 115; K 2144, N 896, 494 rows 57 / 63, 69 / 58, 49 / 47; K 608, N 3968, 486 rows 81 / 87, 79 / 76, 84 / 82,
+//   90 / 93; 64 slices, K 1696, N 4736, 136 rows with favourites 141 / 131, 145 / 112, 119 / 134; 128 x 256: K 640, N 3200, 32 slices of 332 54 / 65
+// (160 x 512 before up to 176 rows and from 640, 128 x 256 between: 16 slices of 122 rows, K 1792, N 2048 38 -> 23; layers of 1000 tokens, 16 experts, top 8, 1536 112 -> 102, of 1500, 32
+// experts, top 8, 2016 and 992 154 -> 135, of 4000, 32 experts, top 4, 2880 516 -> 473.)  Where a slice of 105 to 152 rows, one block of 160, makes three rounds of tiles
+// and more, the second blocks that a routing adds are few rows each and cost less than this counts: those stay.
+inline double mx8_row_blocks(double per_slice, int bm) {
+  if (per_slice >= 3.0 * bm) return per_slice / bm + 0.5;
+  double n = 1.0;
+  const double spread = 1.2 * sqrt(per_slice);
+  for (int j = 1; j < 5; ++j) n += 1.0 / (1.0 + exp(1.7 * (j * bm - per_slice) / spread));
+  return n;
+}
+inline MxwTile mx8_tile(int64_t rows, int64_t n_slices, int64_t K, int64_t N) {
+  if (rows <= 152 * n_slices && n_slices * ((N + 511) / 512) >= 3 * 256) return {160, 512};
+  struct Cost {
+    MxwTile tile;
+    int bm, bn;
+    double start, stage;
+  };
+  const Cost costs[] = {{{0, 0}, 128, 256, 5.1, 0.78}, {{64, 512}, 64, 512, 4.0, 1.02}, {{128, 512}, 128, 512, 7.7, 1.46}, {{160, 512}, 160, 512, 9.8, 2.05}};
+  MxwTile best = {0, 0};
+  double least = 1e30;
+  for (const Cost& c : costs) {
+    const double rounds = mx8_row_blocks((double)rows / (double)n_slices, c.bm) * (double)(n_slices * ((N + c.bn - 1) / c.bn)) / 256.0;
+    const double us = (ceil(rounds * 0.95) + ceil(rounds * 1.05)) * (c.start + (double)((K + 127) / 128) * c.stage);
+    if (us < least) least = us, best = c.tile;
+  }
+  return best;
+}
+
+inline MxwTile mxw_tile(int64_t rows, int64_t n_slices, int64_t K, int64_t N, bool mx8) {
   const int64_t n256 = (N + 255) / 256, n512 = (N + 511) / 512;
   if (mx8) {
+    if (rows > 104 * n_slices) return mx8_tile(rows, n_slices, K, N);
     if ((rows <= 96 * n_slices ? 256 * n_slices : 2 * rows + 128 * n_slices) * n256 <= 256 * 256) return {0, 0};  // (256ths of its row blocks)
     const int64_t alike = n_slices * n512;
     const bool few = alike < 3 * 256;
     if (few && rows <= 24 * n_slices) return {32, 256};
-    if (rows <= (!few ? 24 : alike > 192 && alike <= 256 ? 32 : 40) * n_slices) return {64, 512};
-    // (from 104 to 152 rows on a slice's second row block of 128 becomes the rule)
-    const int64_t second = rows - 104 * n_slices < 48 * n_slices ? rows - 104 * n_slices : 48 * n_slices;
-    return second <= 0 || (rows <= 176 * n_slices && n512 * (48 * n_slices + second) <= 256 * 48) ? MxwTile{128, 512} : MxwTile{0, 0};
+    return rows <= (alike > 192 && alike <= 256 ? 32 : 40) * n_slices ? MxwTile{64, 512} : MxwTile{128, 512};
   }
   if ((rows + 16 * n_slices) * n256 <= 512 * 32) return {32, 256};
   if (rows <= 20 * n_slices) return rows > 7 * n_slices && n_slices * n512 >= 3 * 256 ? MxwTile{64, 512} : MxwTile{32, 256};

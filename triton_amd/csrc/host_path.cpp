@@ -212,21 +212,20 @@ int64_t mxfp4_block_m(int64_t rows, int64_t n_slices, int64_t otherwise) {
 
 // Row blocks of 128, or 256 = the wide kernel (160 x 512 tiles), for MXFP4 weights beyond the sizes above.  Measured at K 2880, N 5760 and
 // 2880 (both GEMMs, 128 against 256).  bf16 rows: 64 per slice 571 against 582 us, 94 684 against 668, 162 1296 against 1131,
-// 250 (16 slices) 258 against 246, 1024 754 against 716 us.  MXFP8 rows: 64 per slice 444 against 451 us, 112 537 against 503, 162 932
-// against 767; past one tile per slice the smaller blocks, whose tiles of a slice share weights in L2, win (203 910 against 955, 250
-// 143 against 153 us), until a workgroup has several tiles of a slice (512: 256 us either way, 1024 469 against 440 us).
+// 250 (16 slices) 258 against 246, 1024 754 against 716 us.  MXFP8 rows: 64 per slice 444 against 451 us; beyond 104 by mx8_tile (gemm_limits.h), whose
+// tiles other than 160 x 512 are asked for by their columns, or are those of the kernel for row blocks of 128.
 // The wide kernel takes four stages of K (the activation scales sixteen blocks), slices in registers and x as a buffer resource.
-int64_t wide_block_m(int64_t rows, int64_t n_slices, int64_t K, uint32_t x_bytes, bool mx8) {
+int64_t wide_block_m(int64_t rows, int64_t n_slices, int64_t K, int64_t N, uint32_t x_bytes, bool mx8) {
   n_slices = std::max<int64_t>(n_slices, 1);
   if (K <= (mx8 ? 511 : 384) || n_slices > tk::kDmaSlices || !x_bytes) return rows <= 144 * n_slices ? 256 : 128;
   if (rows <= 80 * n_slices) return 128;
-  return !mx8 || rows <= 176 * n_slices || rows >= 640 * n_slices ? 256 : 128;
+  return !mx8 || rows <= 104 * n_slices || tk::mxw_tile(rows, n_slices, K, N, mx8).rows == 160 ? 256 : 128;
 }
 
 // Columns of the wide kernel's tiles that gemm_limits.h names for such weights, 0 = the kernel of the row block.
 int64_t wide_block_n(int64_t rows, int64_t n_slices, int64_t K, int64_t N, uint32_t x_bytes, bool mx8) {
   n_slices = std::max<int64_t>(n_slices, 1);
-  return K <= (mx8 ? 511 : 384) || n_slices > tk::kDmaSlices || !x_bytes ? 0 : tk::mxw_tile(rows, n_slices, N, mx8).cols;
+  return K <= (mx8 ? 511 : 384) || n_slices > tk::kDmaSlices || !x_bytes ? 0 : tk::mxw_tile(rows, n_slices, K, N, mx8).cols;
 }
 
 // Columns a workgroup of the kernel for few rows, 0 = the kernels above: up to 64 rows per slice and one workgroup per CU at most, with 32
@@ -446,14 +445,14 @@ PyObject* run_gemm(PyObject* const* v) {
     block_m = fp8_block_m(M, x_bytes, K, N, n_slices);
     if (tk::dma_runs_e4m3(x_bytes, n_slices, K, N)) block_n = dma_block_n(M, N, n_slices, block_m, false);
   } else if (mx_act) {
-    block_m = wide_block_m(M, n_slices, K, x_bytes, true);
+    block_m = wide_block_m(M, n_slices, K, N, x_bytes, true);
     block_n = wide_block_n(M, n_slices, K, N, x_bytes, true);
   } else if (tiled) {
     if (M > 256 && x_bytes && n_slices <= tk::kDmaSlices && !x_row && !w_col) {
       block_m = mxfp4_block_m(M, n_slices, block_m);
       if (n_out % 8 == 0) block_n = wide_block_n(M, n_slices, K, N, x_bytes, false);
     }
-    if (block_m == 128) block_m = wide_block_m(M, n_slices, K, x_bytes, false);
+    if (block_m == 128) block_m = wide_block_m(M, n_slices, K, N, x_bytes, false);
   } else if (tk::dma_runs_16bit(x_bytes, n_slices, K, N, w->stride(2))) {
     if (idle <= 0) block_n = few_block_n(M, N, n_slices);
     if (block_m > 16) block_m = dma_block_m(M, 2 * K, N, n_slices);
@@ -862,8 +861,8 @@ PyObject* rule_wide_n(PyObject* const* v) {
   return PyLong_FromLongLong(wide_block_n(rows, n_slices, K, N, uint32_t(x_bytes), mx8 != 0));
 }
 PyObject* rule_wide(PyObject* const* v) {
-  const auto [rows, n_slices, K, x_bytes, mx8] = integers<5>(v);
-  return PyLong_FromLongLong(wide_block_m(rows, n_slices, K, uint32_t(x_bytes), mx8 != 0));
+  const auto [rows, n_slices, K, N, x_bytes, mx8] = integers<6>(v);
+  return PyLong_FromLongLong(wide_block_m(rows, n_slices, K, N, uint32_t(x_bytes), mx8 != 0));
 }
 
 // bind(dict): the addresses of the entry points (integers) and the Python objects above
@@ -923,7 +922,7 @@ PyMethodDef methods[] = {
     METHOD("decode_by_rows", rule_decode_rows, 4),
     METHOD("fp8_block_m", rule_fp8, 5),
     METHOD("mxfp4_block_m", rule_mxfp4, 3),
-    METHOD("wide_block_m", rule_wide, 5),
+    METHOD("wide_block_m", rule_wide, 6),
     METHOD("wide_block_n", rule_wide_n, 6),
     {nullptr, nullptr, 0, nullptr},
 };

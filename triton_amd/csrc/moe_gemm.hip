@@ -39,7 +39,7 @@ static int32_t launch_16bit(const GemmParams& p, const tk_gemm_desc* d, int wk, 
 static MxwTile wide_tile(const GemmParams& p, const tk_gemm_desc* d, bool mx8) {
   if (!p.x_bytes || slices(d) > kDmaSlices || p.w_nst < 4) return {0, 0};
   if (d->block_n == 256 || d->block_n == 512) {
-    const MxwTile tile = mxw_tile(d->M, slices(d), d->N, mx8);
+    const MxwTile tile = mxw_tile(d->M, slices(d), d->K, d->N, mx8);
     if (tile.rows && tile.cols == d->block_n) return tile;
   }
   return d->block_m == 256 ? MxwTile{160, 512} : MxwTile{0, 0};

@@ -760,7 +760,7 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
     elif mx_act or (tiled and mx_out_fused):
         # the tile shapes that take MXFP8 activations / have an MX-output epilogue
         if forced is None and is_ragged:
-            block_m = nt.rules().wide_block_m(M, n_slices, K, x_bytes, 1) if mx_act else 256 if M <= 144 * n_slices else 128
+            block_m = nt.rules().wide_block_m(M, n_slices, K, N, x_bytes, 1) if mx_act else 256 if M <= 144 * n_slices else 128
             if mx_act and not extras:
                 d.block_n = nt.rules().wide_block_n(M, n_slices, K, N, x_bytes, 1)
         else:
@@ -775,7 +775,7 @@ def matmul(a, b, bias, a_ragged_metadata: RaggedTensorMetadata | None = None,
                 if out_shape[1] % 8 == 0:
                     d.block_n = nt.rules().wide_block_n(M, n_slices, K, N, x_bytes, 0)
             if block_m == 128:
-                block_m = nt.rules().wide_block_m(M, n_slices, K, x_bytes, 0)
+                block_m = nt.rules().wide_block_m(M, n_slices, K, N, x_bytes, 0)
     elif w_dtype in (_BF16, _F16):
         if not nt.rules().dma_runs_16bit(x_bytes, n_slices, K, N, w.stride(-1)):
             block_m = min(block_m, 128)  # (the general kernel's largest)
