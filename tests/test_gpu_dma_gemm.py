@@ -248,3 +248,31 @@ def test_square_tiles_where_a_routing_divides_worse_into_tall_ones(device, dtype
 def test_narrow_tiles_of_few_rows(device, sizes, k, n, swiglu):
     """e4m3, few rows a slice and few columns: tiles of 64 x 64 and 256 of K a stage, beside whole ones for a slice of more."""
     _check(device, "e4m3", 128, sizes, k, n, swiglu=swiglu)
+
+
+@pytest.mark.parametrize("dtype", ["bfloat16", "e4m3"])
+def test_small_tiles_of_one_round(device, monkeypatch, dtype):
+    """More large tiles than the chip would leave CUs without, but one round of small ones: both host paths choose these, whose results are those of small
+    tiles asked for by name, bit for bit, and agree with the oracle."""
+    import triton_amd.matmul as mm
+    from triton_amd import _native as nt
+    from triton_amd.tensor import convert_layout, make_ragged_tensor_metadata, wrap_torch_tensor
+    from triton_amd.tensor_details.layout import make_default_matmul_fp8_w_layout
+    g = torch.Generator().manual_seed(12)
+    sizes, k, n = torch.tensor([272, 250, 300, 129, 400, 256, 257, 320], dtype=torch.int32), 48, 2056
+    m, e = int(sizes.sum()), len(sizes)
+    assert nt.rules().dma_block_m(m, k, n, e) == 256 and nt.rules().dma_block_n(m, n, e, 256) == 128 and nt.rules().dma_block_n_16bit(m, n, e, 256) == 128
+    assert nt.rules().dma_block_n(m, 2 * n, e, 256) == 0
+    dt = torch.bfloat16 if dtype == "bfloat16" else torch.float8_e4m3fn
+    x, w = torch.randn((m, k), generator=g).to(dt), (torch.randn((e, n, k), generator=g) * 0.1).to(dt)
+    wd = w.to(device).transpose(1, 2)
+    wd = wd if dtype == "bfloat16" else convert_layout(wrap_torch_tensor(wd), make_default_matmul_fp8_w_layout())
+    md, pc = make_ragged_tensor_metadata(sizes.to(device), m), mm.PrecisionConfig(out_dtype=torch.bfloat16)
+    native = mm.matmul(x.to(device), wd, None, md, precision_config=pc)
+    with monkeypatch.context() as p:
+        p.setattr(nt, "host", lambda: None)
+        general = mm.matmul(x.to(device), wd, None, md, precision_config=pc)
+    with mm.scoped_opt_flags_constraints({"block_m": 128}):
+        small = mm.matmul(x.to(device), wd, None, md, precision_config=pc)
+    assert_allclose_gate(omoe.matmul(x, w.transpose(1, 2), None, sizes, out_dtype=torch.float32), native, what=f"{dtype} small tiles")
+    assert torch.equal(native, general) and torch.equal(native, small)

@@ -143,9 +143,19 @@ inline MxwTile mxw_tile(int64_t rows, int64_t n_slices, int64_t K, int64_t N, bo
   return rows <= 48 * n_slices ? MxwTile{64, 512} : rows <= 80 * n_slices ? MxwTile{96, 512} : MxwTile{160, 512};
 }
 
+// Whether 128 x 128 tiles of slices of 192 rows and more, half a row block a slice more than there are rows for, are one round of two workgroups a CU: they
+// beat larger tiles, which then leave CUs without one or are little more than a round.  Measured (us, this kernel's 128 x 128 / the best of 256 x 256 and those of 320
+// rows; slices, rows of one, K, N: 128 x 128 tiles).  bf16: 8, 272, 2048, 2048: 336 31.8 / 37.2; 8, 300: 364 33.5 / 38.1; 8, 400: 464 36.7 / 40.2; 8, 450, 1536: 514 32.6 / 34.2; 16, 272,
+// 1024, 1280: 420 22.6 / 24.9; 16, 200, 1024, 1600: 429 26.1 / 25.6; 16, 400, 704, 896: 406 18.8 / 20.7 (256 x 256 30.7); 16, 300, 512, 1600: 591 31.6 / 29.1; 32, 200, 384, 1024: 528 18.5 /
+// 18.0.  e4m3: 8, 272, 1536, 2048: 336 17.6 / 25.4; 8, 400, 2048, 2048: 464 23.0 / 30.6; 16, 272, 1024, 1152: 378 16.2 / 32.7; 16, 200, 6144, 1792: 462 64 / 68; 8, 272, 2048, 3072: 504
+// 31.2 / 30.6; 8, 600, 1280, 2048: 664 26.8 / 25.9; 8, 272, 1024, 4096: 672 29.2 / 23.2; 16, 200, 1024, 2048: 528 17.8 / 21.7.
+inline bool small_tiles_one_round(int64_t rows, int64_t n_slices, int64_t N) {
+  return rows >= 192 * n_slices && (rows + 64 * n_slices) * ((N + 127) / 128) <= 500 * 128;
+}
+
 // Tile of the memory-to-LDS kernel (moe_gemm_dma_kernel.h) for 16-bit operands beside 256 x 256 ones: 320 rows, so that a slice of about 256 rows, of which
 // a random routing makes half a few longer, is one row block.  (An eighth above the mean is 2.5 deviations at 400 rows, 2 at 256.)  rows 0 = those.
-//   320 x 128 where its tiles are one round and 128 x 128 ones (up to 96 of 256 x 256, dma_block_n) are not better; 320 x 256 beyond, from 248 rows on.
+//   320 x 128 where its tiles are one round and 128 x 128 ones (above; up to 96 of 256 x 256, dma_block_n) are not better; 320 x 256 beyond, from 248 rows on.
 // Measured (us of a GEMM with a random routing, 256 x 256 / 320 x 256 / 320 x 128; slices, K, N):
 //   16, 2048, 4096: 224 rows 89 / 100 / 92, 240 101 / 95 / 92, 256 105 / 96 / 92, 272 130 / 101 / 107, 288 136 / 122 / 126, 320 142 / 150 / 152
 //   16, 2048, 2048: 224 rows 56 / 72 / 50, 256 56 / 74 / 53, 272 57 / 78 / 58, 288 56 / 78 / 67; K 1024: 224 30 / 35 / 25, 272 32 / 40 / 28, 288 33 / 40 / 35
@@ -158,7 +168,7 @@ struct DmaTile {
   int32_t rows, cols;
 };
 inline DmaTile dma_tile(int64_t rows, int64_t n_slices, int64_t N) {
-  if (n_slices < 8) return {0, 0};
+  if (n_slices < 8 || small_tiles_one_round(rows, n_slices, N)) return {0, 0};
   const int64_t per_slice = rows / n_slices, n256 = (N + 255) / 256, blocks = (per_slice * 9 / 8 + 319) / 320;
   if (per_slice >= (blocks == 1 ? 192 : 448) && blocks <= 2 && n_slices * blocks * ((N + 127) / 128) <= 256 && n_slices * ((per_slice + 255) / 256) * n256 > 96)
     return {320, 128};

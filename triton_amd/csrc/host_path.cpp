@@ -178,7 +178,8 @@ int64_t dma_block_m(int64_t rows, int64_t row_bytes, int64_t N, int64_t n_slices
   return per_slice >= 192 || tiles >= 192 || row_bytes >= 8192 ? 256 : 128;
 }
 
-// 128 = the kernel's 128 x 128 tiles although the rule above says 256: up to 96 of the large tiles leave most of the 256 CUs without one.
+// 128 = the kernel's 128 x 128 tiles although the rule above says 256: where those are one round (small_tiles_one_round, gemm_limits.h), and with fewer rows
+// up to 96 of the large tiles, which leave most of the 256 CUs without one.
 // Measured with a random routing (us, 128 against 256): bf16, K 2048, N 2048, 8 slices of 256 rows (64 large tiles) 29 against 42; N 1536, 16
 // slices (96) 34 against 41; N 2048, 16 slices (128) 51 against 49; K 1024, N 1024, 16 slices (64) 19 against 27, N 512 (32) 11 against 23;
 // K 4096, N 1024, 16 slices (64) 55 against 72; e4m3, K 14336, N 2048, 8 slices (64) 92 against 126, N 4096 (128) 193 against 158.
@@ -187,7 +188,7 @@ int64_t dma_block_n(int64_t rows, int64_t N, int64_t n_slices, int64_t block_m, 
   const int64_t cols = block_m == 256 && bits16 ? tk::dma_tile(rows, n_slices, N).cols : 0;
   if (cols) return cols;
   const int64_t per_slice = rows / std::max<int64_t>(n_slices, 1);
-  return block_m == 256 && n_slices * ((per_slice + 255) / 256) * ((N + 255) / 256) <= 96 ? 128 : 0;
+  return block_m == 256 && (tk::small_tiles_one_round(rows, n_slices, N) || n_slices * ((per_slice + 255) / 256) * ((N + 255) / 256) <= 96) ? 128 : 0;
 }
 
 // Row blocks for tiled e4m3 weights: by the rule above where that kernel runs (`x_bytes` as in gemm_limits.h).  The other kernel walks a
