@@ -213,14 +213,15 @@ int64_t mxfp4_block_m(int64_t rows, int64_t n_slices, int64_t otherwise) {
 
 // Row blocks of 128, or 256 = the wide kernel (160 x 512 tiles), for MXFP4 weights beyond the sizes above.  Measured at K 2880, N 5760 and
 // 2880 (both GEMMs, 128 against 256).  bf16 rows: 64 per slice 571 against 582 us, 94 684 against 668, 162 1296 against 1131,
-// 250 (16 slices) 258 against 246, 1024 754 against 716 us.  MXFP8 rows: 64 per slice 444 against 451 us; beyond 104 by mx8_tile (gemm_limits.h), whose
-// tiles other than 160 x 512 are asked for by their columns, or are those of the kernel for row blocks of 128.
+// 250 (16 slices) 258 against 246, 1024 754 against 716 us.  MXFP8 rows: 64 per slice 444 against 451 us; beyond 104 by mx8_tile (gemm_limits.h).
 // The wide kernel takes four stages of K (the activation scales sixteen blocks), slices in registers and x as a buffer resource.
 int64_t wide_block_m(int64_t rows, int64_t n_slices, int64_t K, int64_t N, uint32_t x_bytes, bool mx8) {
   n_slices = std::max<int64_t>(n_slices, 1);
   if (K <= (mx8 ? 511 : 384) || n_slices > tk::kDmaSlices || !x_bytes) return rows <= 144 * n_slices ? 256 : 128;
   if (rows <= 80 * n_slices) return 128;
-  return !mx8 || rows <= 104 * n_slices || tk::mxw_tile(rows, n_slices, K, N, mx8).rows == 160 ? 256 : 128;
+  // (the wide kernel's tiles are asked for by their columns; the other kernel, where mx8_tile says so, has row blocks of 128)
+  if (mx8 && rows > 104 * n_slices && !tk::mxw_tile(rows, n_slices, K, N, mx8).rows) return 128;
+  return !mx8 || rows <= 176 * n_slices || rows >= 640 * n_slices ? 256 : 128;
 }
 
 // Columns of the wide kernel's tiles that gemm_limits.h names for such weights, 0 = the kernel of the row block.
