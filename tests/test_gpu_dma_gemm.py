@@ -242,12 +242,19 @@ def test_square_tiles_where_a_routing_divides_worse_into_tall_ones(device, dtype
     assert_allclose_gate(ref, out.cpu()[sc.cpu()[rows].long()], what=f"{dtype} square tiles")
 
 
-@pytest.mark.parametrize("sizes", [[0, 1, 31, 32, 33, 63, 64, 40], [2, 0, 31, 33, 64, 65, 129, 2], [5]])
+@pytest.mark.parametrize("sizes", [[0, 1, 31, 32, 33, 63, 64, 40], [2, 0, 31, 33, 64, 65, 129, 2], [5], [96, 97, 128, 161, 192, 1, 0, 95]])
 @pytest.mark.parametrize("k, n", [(32, 8), (144, 264), (528, 1032), (1040, 72)])
-@pytest.mark.parametrize("swiglu", [False, True])
-def test_narrow_tiles_of_few_rows(device, sizes, k, n, swiglu):
-    """e4m3, few rows a slice and few columns: tiles of 64 x 64 and 256 of K a stage, beside whole ones for a slice of more."""
-    _check(device, "e4m3", 128, sizes, k, n, swiglu=swiglu)
+@pytest.mark.parametrize("dtype, swiglu", [("e4m3", False), ("e4m3", True), ("bfloat16", True), ("float16", False)])
+def test_narrow_tiles_of_few_rows(device, sizes, k, n, dtype, swiglu):
+    """Few rows a slice, or few tiles in all: row blocks of 64 by 64 columns and twice the K a stage."""
+    _check(device, dtype, 128, sizes, k, n, swiglu=swiglu)
+
+
+@pytest.mark.parametrize("k, n", [(32, 1032), (208, 1288), (528, 1032)])
+@pytest.mark.parametrize("dtype, swiglu", [("e4m3", False), ("bfloat16", False), ("bfloat16", True), ("float16", False)])
+def test_tiles_of_128_columns(device, k, n, dtype, swiglu):
+    """More columns than the small tiles are for: the row blocks of 128 at the edges of tiles and stages."""
+    _check(device, dtype, 128, SIZES, k, n, swiglu=swiglu)
 
 
 @pytest.mark.parametrize("dtype", ["bfloat16", "e4m3"])

@@ -21,16 +21,19 @@ int32_t launch_cfg(const GemmParams& p, int grid_m, bool swiglu, hipStream_t st)
   };
   const int64_t slices = p.slice_sizes ? p.n_slices : 1;
   const bool once = reads_once(p.M, slices, C::BM, p.N, p.K * (WK == WK_FP8 ? 1 : 2));
-  // Tiles of 64 x 64 and 256 of K a stage (the narrow ones of short row blocks) where slices have few rows and those of 128 columns are not two a CU: twice
-  // the workgroups read the weights.  Layers, us: 8 experts, top 2, d 2048, d_ff 13312, 28 tokens 154 -> 130; d 1024, d_ff 8192, 128 tokens 87 -> 74; d 2048, d_ff 4096,
-  // 200 tokens 74 -> 68; 16 experts, d 1024, d_ff 2560, 108 tokens 52 -> 49; d 1152, d_ff 5120, 406 91.4 -> 90.4.  Up to 52 rows a slice, beyond which slices of over 64,
-  // whose tiles stay, are many (62: d 1536, d_ff 2048 48.0 -> 49.2).
-  if constexpr (TILE == kDma128 && WK == WK_FP8) {
-    const int64_t wide = slices * q.grid_n;
-    if (p.M <= slices * 52 && wide * 2 <= dma_grid(p, C::PER_CU, wide * 2)) {
-      grid = dma_grid(p, C::PER_CU, wide * 2);
-      if (once) return swiglu ? launch(moe_gemm_dma_kernel<WK, TILE, true, true, true>) : launch(moe_gemm_dma_kernel<WK, TILE, false, true, true>);
-      return swiglu ? launch(moe_gemm_dma_kernel<WK, TILE, true, true, false>) : launch(moe_gemm_dma_kernel<WK, TILE, false, true, false>);
+  // Tiles of 64 x 64 and twice the K a stage (the narrow ones that short row blocks have, for all) where those are about one round of two workgroups a CU: the larger
+  // ones would be a part of one, and what takes their time is the way of a stage from memory.  Layers, us, 128 x 128 / 64 x 64 (expected tiles of the first and
+  // second GEMM where they run): bf16, 8 experts, top 4, d 704, d_ff 1120, 613 tokens 68 / 50 (465 in the second); 8, top 1, 288 and 352, 567 tokens 37 / 26 (141, 64); 16, top 2, 320 and 512,
+  // 1146 39 / 31 (219); 8, top 4, 1568 and 256, 699 54 / 45 (381); e4m3, 8, top 2, 2048 and 13312, 28 154 / 130 (256); 1280 and 11904, 234 127 / 105 (226); 1024 and 8192, 128 87 / 74.  One GEMM:
+  // bf16, 8 slices of 100, K 512, N 1024 11.4 / 8.5 (264); 16 of 80, K 1024, N 1024 16.2 / 13.7 (448); e4m3, 8 of 80, K 2048, N 2048 16.2 / 14.0 (448), of 200, K 1024, N 2048 13.4 / 12.8.
+  // (Half a block a slice more than there are rows for; up to 52 rows a slice, one.)
+  if constexpr (TILE == kDma128) {
+    const int64_t blocks = p.M <= slices * 52 ? slices : (p.M + slices * 32) / 64, small = blocks * cdiv(p.N, C::SBN);
+    if (small <= 512 && small <= dma_grid(p, C::PER_CU, small)) {
+      // (a workgroup for every tile that there may be: one with two of them takes twice the time)
+      grid = dma_grid(p, C::PER_CU, (cdiv(p.M, 64) + slices) * cdiv(p.N, C::SBN));
+      if (once) return swiglu ? launch(moe_gemm_dma_kernel<WK, TILE, true, true, true, true>) : launch(moe_gemm_dma_kernel<WK, TILE, false, true, true, true>);
+      return swiglu ? launch(moe_gemm_dma_kernel<WK, TILE, true, true, false, true>) : launch(moe_gemm_dma_kernel<WK, TILE, false, true, false, true>);
     }
   }
   if (once)

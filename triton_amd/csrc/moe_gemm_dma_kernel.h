@@ -55,7 +55,8 @@ struct DmaCfg {
 static_assert(DmaCfg<kDma256>::LDS == 160 * 1024 && DmaCfg<kDma128>::LDS == 80 * 1024 && DmaCfg<kDma320>::LDS <= 160 * 1024, "one / two workgroups of a CU");
 
 // NARROW: short row blocks may be cut into narrow tiles (gemm_tiles.h).  ONCE: the weights are fetched with the non-temporal hint (reads_once).
-template <int WK, int TILE, bool SWIGLU, bool NARROW, bool ONCE>
+// SMALL: all tiles are narrow ones, of row blocks half as high.
+template <int WK, int TILE, bool SWIGLU, bool NARROW, bool ONCE, bool SMALL = false>
 __device__ __forceinline__ void dma_gemm(const GemmParams& p) {
   typedef DmaCfg<TILE> C;
   constexpr bool F8 = WK == WK_FP8;
@@ -70,8 +71,15 @@ __device__ __forceinline__ void dma_gemm(const GemmParams& p) {
   const int nst = (KB + 127) >> 7;
   const uint32_t lds0 = lds_addr(lds);
 
-  TileList<C::BM, C::BN, NARROW ? C::SBN : C::BN> tiles;
-  int tile = tiles.init(p, lane, (p.N + C::BN - 1) / C::BN);
+  static_assert(NARROW || !SMALL, "small tiles are narrow ones");
+  constexpr int LBM = SMALL ? C::BM / 2 : C::BM, LBN = SMALL ? C::SBN : C::BN;
+  TileList<LBM, LBN, NARROW ? C::SBN : C::BN> tiles;
+  int tile = tiles.init(p, lane, (p.N + LBN - 1) / LBN);
+  auto locate = [&](int i) __attribute__((always_inline)) -> Tile {
+    Tile t = tiles.locate(i);
+    if (SMALL) t.narrow = true;
+    return t;
+  };
   const int t_step = tiles.t_step, t_end = tiles.t_end;
   if (tile >= t_end) return;
 
@@ -151,7 +159,7 @@ __device__ __forceinline__ void dma_gemm(const GemmParams& p) {
 
   // ---- the rings: one cursor, two stages ahead of the multiplication --------------------------------------------------------------------------
   constexpr uint32_t kAEnd = C::ABUFS * C::ABYTES, kBEnd = kAEnd + C::BBUFS * C::BBYTES;
-  Tile cur = tiles.locate(tile);
+  Tile cur = locate(tile);
   aim(cur);
   uint32_t aw = 0, bw = kAEnd;  // buffers the next transfers fill
   int fs = 0;                   // where the next stage to fetch begins
@@ -164,7 +172,7 @@ __device__ __forceinline__ void dma_gemm(const GemmParams& p) {
       fs = 0;
       f_tile += t_step;
       more = more && f_tile < t_end;
-      if (more) aim(tiles.locate(f_tile));
+      if (more) aim(locate(f_tile));
     }
   };
 
@@ -328,9 +336,10 @@ __device__ __forceinline__ void dma_gemm(const GemmParams& p) {
       narrow_tile();
       tile += t_step;
       if (tile >= t_end) break;
-      cur = tiles.locate(tile);
+      cur = locate(tile);
       continue;
     }
+    if constexpr (!SMALL) {
     prime();
 #pragma unroll
     for (int f = 0; f < NFW; ++f)
@@ -366,14 +375,15 @@ __device__ __forceinline__ void dma_gemm(const GemmParams& p) {
                                                              cur.n_tile + C::BN <= p.N, mw, lr, h);
     tile += t_step;
     if (tile >= t_end) break;
-    cur = tiles.locate(tile);
+    cur = locate(tile);
+    }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no transfer into this workgroup's LDS is left behind
 }
 
-template <int WK, int TILE, bool SWIGLU, bool NARROW, bool ONCE>
+template <int WK, int TILE, bool SWIGLU, bool NARROW, bool ONCE, bool SMALL = false>
 __global__ __launch_bounds__(DmaCfg<TILE>::NW * 64, 2) void moe_gemm_dma_kernel(const GemmParams p) {
-  dma_gemm<WK, TILE, SWIGLU, NARROW, ONCE>(p);
+  dma_gemm<WK, TILE, SWIGLU, NARROW, ONCE, SMALL>(p);
 }
 
 // Workgroups of a launch over `tiles` tiles at most: a multiple of 8 (every XCD walks its share of the tiles), `per_cu` per CU at most.
