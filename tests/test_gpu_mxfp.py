@@ -281,3 +281,19 @@ def test_sources_read_with_the_non_temporal_hint(mx, device, qdt):
         qi, si = mx.downcast_to_mxfp(x[i:i + 1], qdt, axis=1)
         _same(qi, q[i:i + 1], "values")
         _same(si, s[i:i + 1], "scales")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("outer, length, inner", [(260, 288, 260), (520, 32, 512)])
+def test_tiles_of_many_blocks_give_what_small_ones_give(device, dtype, outer, length, inner):
+    """More tiles than the small ones are for, with a last one that holds a single block: the bytes that a few matrices at a time give."""
+    from triton_kernels.numerics_details.mxfp import downcast_to_mxfp, upcast_from_mxfp
+    g = torch.Generator(device=device).manual_seed(outer)
+    x = torch.randn((outer, length, inner), generator=g, device=device).to(dtype)
+    x[::7, ::5, ::3] *= 1000
+    q, s = downcast_to_mxfp(x, torch.uint8, axis=1)
+    back = upcast_from_mxfp(q, s, dtype, axis=1)
+    for i in range(0, outer, 20):
+        qi, si = downcast_to_mxfp(x[i:i + 20], torch.uint8, axis=1)
+        assert torch.equal(q[i:i + 20], qi) and torch.equal(s[i:i + 20], si)
+        assert torch.equal(back[i:i + 20], upcast_from_mxfp(qi, si, dtype, axis=1))

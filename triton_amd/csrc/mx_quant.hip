@@ -446,19 +446,20 @@ template <int KIND>
 struct TileGeom {
   static constexpr int BB = KIND == TK_E2M1 ? 16 : 32;  // value bytes per block and column
   static constexpr int NB = 128 / BB;                    // blocks per tile
+  static constexpr int SMALL = 4;                        // ... of a small tensor: one a wave
 };
 
 // moves the tile's value bytes and scales between LDS and global memory (TO_GLOBAL) or back
-template <int KIND, bool TO_GLOBAL>
+template <int KIND, int NB, bool TO_GLOBAL>
 __device__ __forceinline__ void tile_move(uint8_t* vals_s, uint8_t* sc_s, uint8_t* gvals, uint8_t* gscales, int64_t o, int64_t col0,
                                           int64_t blk0, int64_t L, int64_t inner, int64_t inner_last) {
-  constexpr int BB = TileGeom<KIND>::BB, NB = TileGeom<KIND>::NB;
+  constexpr int BB = TileGeom<KIND>::BB, PIECES = NB * BB / 16;  // (of a column)
   const int64_t nblk = L / 32;
   const int64_t line_bytes = KIND == TK_E2M1 ? L / 2 : L;
 #pragma unroll
-  for (int it = 0; it < 8; ++it) {
+  for (int it = 0; it < PIECES; ++it) {
     const int q = it * kThreads + threadIdx.x;
-    const int col = q >> 3, piece = q & 7;
+    const int col = q / PIECES, piece = q % PIECES;
     const int64_t blk = blk0 + piece * 16 / BB;
     if (col0 + col < inner && blk < nblk) {
       const int64_t line = line_of(o, col0 + col, inner, inner_last);
@@ -499,9 +500,9 @@ __device__ __forceinline__ void tile_move(uint8_t* vals_s, uint8_t* sc_s, uint8_
 
 // Quantises the lane's 32 rows x 4 columns of block `b` (raw[i] = row i, two 16-bit elements per dword) into the
 // tile's LDS staging arrays.
-template <int SRC, int KIND>
+template <int SRC, int KIND, int NB>
 __device__ __forceinline__ void quantise_block_to_lds(const uint2 (&raw)[32], uint8_t* vals_s, uint8_t* sc_s, int c4, int b, int rounding) {
-  constexpr int BB = TileGeom<KIND>::BB, NB = TileGeom<KIND>::NB;
+  constexpr int BB = TileGeom<KIND>::BB;
   // The block maxima come from the 16-bit patterns themselves (|x| orders like its bits without the sign, two elements per instruction) and the
   // hardware converts two 16-bit floats to two codes while dividing by the power-of-two scale (round to nearest even, exact), so a pair of rows costs
   // one byte permute and one conversion.  A lane with a block that holds an infinity or a NaN, or whose scale is outside `down_scale_ok`, takes the fp32
@@ -597,12 +598,11 @@ __device__ __forceinline__ uint2 load_once_u2(const uint16_t* p) {
 // b 2 (66 MB) 18.1 / 23.8, b 4 47.8 / 39.5, b 8 107 / 75, b 16 181 / 153, b 32 343 / 300; to e2m1: b 2 18.9 / 21.8, b 4 42.6 / 36.8, b 8 95 / 68.  What
 // was used a moment ago is still in the memory-side cache up to about a hundred megabytes, and a read with the hint does not profit from that.
 constexpr int64_t kOnceBytes = 96ll << 20;
-template <int SRC, int KIND, bool NT>
+template <int SRC, int KIND, bool NT, int NB>
 __global__ __launch_bounds__(kThreads) void mx_down_tile(const uint16_t* __restrict__ src, int64_t stride_outer, int64_t stride_axis,
                                                          int64_t L, int64_t inner, int64_t inner_last, int64_t col_tiles,
                                                          int64_t blk_tiles, uint8_t* __restrict__ out_vals,
                                                          uint8_t* __restrict__ out_scales, int rounding) {
-  constexpr int NB = TileGeom<KIND>::NB;
   __shared__ __attribute__((aligned(16))) uint8_t vals_s[kTileRows * kTilePitch];
   __shared__ uint8_t sc_s[kTileCols * NB];
   int64_t bid = tile_order(blockIdx.x, gridDim.x);
@@ -629,8 +629,8 @@ __global__ __launch_bounds__(kThreads) void mx_down_tile(const uint16_t* __restr
     for (int i = 0; i < 32; ++i) raw0[i] = load_once_u2<NT>(p0 + i * stride_axis);
 #pragma unroll
     for (int i = 0; i < 32; ++i) raw1[i] = load_once_u2<NT>(p1 + i * stride_axis);
-    if (ok0) quantise_block_to_lds<SRC, KIND>(raw0, vals_s, sc_s, c4, wave, rounding);
-    if (ok1) quantise_block_to_lds<SRC, KIND>(raw1, vals_s, sc_s, c4, wave + 4, rounding);
+    if (ok0) quantise_block_to_lds<SRC, KIND, NB>(raw0, vals_s, sc_s, c4, wave, rounding);
+    if (ok1) quantise_block_to_lds<SRC, KIND, NB>(raw1, vals_s, sc_s, c4, wave + 4, rounding);
   } else
 #pragma unroll 1
   for (int pass = 0; pass < NB / 4; ++pass) {
@@ -642,17 +642,17 @@ __global__ __launch_bounds__(kThreads) void mx_down_tile(const uint16_t* __restr
     uint2 raw[32];
 #pragma unroll
     for (int i = 0; i < 32; ++i) raw[i] = load_once_u2<NT>(p + i * stride_axis);
-    quantise_block_to_lds<SRC, KIND>(raw, vals_s, sc_s, c4, b, rounding);
+    quantise_block_to_lds<SRC, KIND, NB>(raw, vals_s, sc_s, c4, b, rounding);
   }
   __syncthreads();
-  tile_move<KIND, true>(vals_s, sc_s, out_vals, out_scales, o, col0, blk0, L, inner, inner_last);
+  tile_move<KIND, NB, true>(vals_s, sc_s, out_vals, out_scales, o, col0, blk0, L, inner, inner_last);
 }
 
-template <int KIND, int DST>
+template <int KIND, int DST, int NB>
 __global__ __launch_bounds__(kThreads) void mx_up_tile(const uint8_t* __restrict__ vals, const uint8_t* __restrict__ scales, int64_t L,
                                                        int64_t inner, int64_t inner_last, int64_t col_tiles, int64_t blk_tiles,
                                                        uint16_t* __restrict__ out, int64_t ostride_outer, int64_t ostride_axis) {
-  constexpr int BB = TileGeom<KIND>::BB, NB = TileGeom<KIND>::NB;
+  constexpr int BB = TileGeom<KIND>::BB;
   __shared__ __attribute__((aligned(16))) uint8_t vals_s[kTileRows * kTilePitch];
   __shared__ uint8_t sc_s[kTileCols * NB];
   int64_t bid = tile_order(blockIdx.x, gridDim.x);
@@ -664,7 +664,7 @@ __global__ __launch_bounds__(kThreads) void mx_up_tile(const uint8_t* __restrict
   const int64_t col0 = tile_col0(ct, inner), blk0 = bt * NB;
   const bool live = col0 + lane * 4 < inner;
   const int c4 = tile_cols_of(lane, col0, inner);
-  tile_move<KIND, false>(vals_s, sc_s, const_cast<uint8_t*>(vals), const_cast<uint8_t*>(scales), o, col0, blk0, L, inner, inner_last);
+  tile_move<KIND, NB, false>(vals_s, sc_s, const_cast<uint8_t*>(vals), const_cast<uint8_t*>(scales), o, col0, blk0, L, inner, inner_last);
   __syncthreads();
   const float mf = Elem<DST>::max_finite();
 #pragma unroll 1
@@ -748,6 +748,11 @@ __global__ __launch_bounds__(kThreads) void mx_up_tile(const uint8_t* __restrict
 }
 
 // ---- dispatch helpers --------------------------------------------------------------------------
+// e2m1: half as many blocks a tile, one a wave instead of two, where the tiles of whole lines are up to four a CU: both directions are a chain of loads, conversion and stores, and
+// half of it is shorter (us, both launches: 1 x 2368 x 592 14.6 -> 9.7, 11 x 448 x 256 14.3 -> 9.4, 5 x 544 x 2368 15.9 -> 11.6, 8 x 1024 x 1024 15.3 -> 12.5, 1 x 2880 x 5760 (276 tiles)
+// 24.5 -> 20.3, 2 x (552) 35.1 -> 32.8, 16 x 2048 x 1024 (512) 30.8 -> 29.3; 8 x 2880 x 2880 (1152) 65.1 -> 66.6, since a column's piece is half a line).
+bool small_tiles(int64_t tiles) { return tiles <= 1024; }
+
 template <int SRC, int KIND>
 int32_t launch_down(const void* src, int64_t outer, int64_t L, int64_t inner, int64_t inner_last, int64_t so, int64_t sa, int64_t si,
                     void* out_vals, void* out_scales, int rounding, hipStream_t st) {
@@ -768,11 +773,13 @@ int32_t launch_down(const void* src, int64_t outer, int64_t L, int64_t inner, in
   const int64_t nblk = L / 32;
   if constexpr (sizeof(T) == 2) {
     if (inner >= 4 && (reinterpret_cast<uintptr_t>(out_vals) % 16) == 0) {
-      const int64_t col_tiles = cdiv(inner, kTileCols), blk_tiles = cdiv(nblk, TileGeom<KIND>::NB);
+      typedef TileGeom<KIND> G;
+      const int64_t col_tiles = cdiv(inner, kTileCols);
+      const bool once = outer * L * inner * 2 >= kOnceBytes, small = small_tiles(col_tiles * cdiv(nblk, G::NB) * outer);
+      const int64_t blk_tiles = cdiv(nblk, small ? G::SMALL : G::NB);
       const int64_t grid = col_tiles * blk_tiles * outer;
       if (grid > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_mx_downcast: tensor too large for one launch");
-      const bool once = outer * L * inner * 2 >= kOnceBytes;
-      hipLaunchKernelGGL((once ? mx_down_tile<SRC, KIND, true> : mx_down_tile<SRC, KIND, false>), dim3((unsigned)grid), dim3(kThreads), 0, st,
+      hipLaunchKernelGGL((once ? mx_down_tile<SRC, KIND, true, G::NB> : small ? mx_down_tile<SRC, KIND, false, G::SMALL> : mx_down_tile<SRC, KIND, false, G::NB>), dim3((unsigned)grid), dim3(kThreads), 0, st,
                          reinterpret_cast<const uint16_t*>(s), so, sa, L, inner, inner_last, col_tiles, blk_tiles, ov, os, rounding);
       return check_launch("mx_down_tile");
     }
@@ -814,10 +821,13 @@ int32_t launch_up(const void* vals, const void* scales, int64_t outer, int64_t L
   const int64_t nblk = L / 32;
   if constexpr (sizeof(T) == 2) {
     if (inner >= 4 && (reinterpret_cast<uintptr_t>(vals) % 16) == 0) {
-      const int64_t col_tiles = cdiv(inner, kTileCols), blk_tiles = cdiv(nblk, TileGeom<KIND>::NB);
+      typedef TileGeom<KIND> G;
+      const int64_t col_tiles = cdiv(inner, kTileCols);
+      const bool small = small_tiles(col_tiles * cdiv(nblk, G::NB) * outer);
+      const int64_t blk_tiles = cdiv(nblk, small ? G::SMALL : G::NB);
       const int64_t grid = col_tiles * blk_tiles * outer;
       if (grid > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_mx_upcast: tensor too large for one launch");
-      hipLaunchKernelGGL((mx_up_tile<KIND, DST>), dim3((unsigned)grid), dim3(kThreads), 0, st, v, s, L, inner, inner_last, col_tiles,
+      hipLaunchKernelGGL((small ? mx_up_tile<KIND, DST, G::SMALL> : mx_up_tile<KIND, DST, G::NB>), dim3((unsigned)grid), dim3(kThreads), 0, st, v, s, L, inner, inner_last, col_tiles,
                          blk_tiles, reinterpret_cast<uint16_t*>(o), oso, osa);
       return check_launch("mx_up_tile");
     }
