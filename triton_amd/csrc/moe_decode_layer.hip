@@ -403,241 +403,241 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
   }
   bool signalled0 = nr0 == 0, signalled = n1 == 0;  // see below
   auto stream = [&](auto mode_c) __attribute__((always_inline)) {
-  constexpr int MODE = decltype(mode_c)::value;
-  u32x4_t wr[RD][XS][FPU][2];
-  uint32_t sr[RD][XS][FPU][2];
-  u32x4_t xr[XS][4];
-  // (Stages and fragments past the unit's last are past the resource's end: zeros, and no memory is asked for them.  No branch around a load: the compiler's wait
-  // counts stay exact only in straight-line code.)
-  uint32_t w_at[XS], s_at[XS];
+    constexpr int MODE = decltype(mode_c)::value;
+    u32x4_t wr[RD][XS][FPU][2];
+    uint32_t sr[RD][XS][FPU][2];
+    u32x4_t xr[XS][4];
+    // (Stages and fragments past the unit's last are past the resource's end: zeros, and no memory is asked for them.  No branch around a load: the compiler's wait
+    // counts stay exact only in straight-line code.)
+    uint32_t w_at[XS], s_at[XS];
 #pragma unroll
-  for (int j = 0; j < XS; ++j) w_at[j] = wlane + (uint32_t)(wave + j * NW) * 2048u, s_at[j] = slane + (uint32_t)(wave + j * NW) * 128u;
-  auto load_w = [&](auto h_c, int j, const DecUnit& u, int nst, int nfr) __attribute__((always_inline)) {
-    constexpr int H = decltype(h_c)::value;
-    auto fetch = [&](auto aux_c) __attribute__((always_inline)) {
-      constexpr int AUX = decltype(aux_c)::value;
+    for (int j = 0; j < XS; ++j) w_at[j] = wlane + (uint32_t)(wave + j * NW) * 2048u, s_at[j] = slane + (uint32_t)(wave + j * NW) * 128u;
+    auto load_w = [&](auto h_c, int j, const DecUnit& u, int nst, int nfr) __attribute__((always_inline)) {
+      constexpr int H = decltype(h_c)::value;
+      auto fetch = [&](auto aux_c) __attribute__((always_inline)) {
+        constexpr int AUX = decltype(aux_c)::value;
 #pragma unroll
-      for (int f = 0; f < FPU; ++f) {
-        const int stages = FPU == 1 || u.frag + f < nfr ? nst : 0;
-        const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(u.w + (int64_t)f * nst * 2048), 0, stages * 2048, 0x00020000);
-        const __amdgpu_buffer_rsrc_t srsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(u.s + (int64_t)f * nst * 128), 0, stages * 128, 0x00020000);
+        for (int f = 0; f < FPU; ++f) {
+          const int stages = FPU == 1 || u.frag + f < nfr ? nst : 0;
+          const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(u.w + (int64_t)f * nst * 2048), 0, stages * 2048, 0x00020000);
+          const __amdgpu_buffer_rsrc_t srsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(u.s + (int64_t)f * nst * 128), 0, stages * 128, 0x00020000);
 #pragma unroll
-        for (int g = 0; g < 2; ++g) {
-          wr[H][j][f][g] = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_at[j] + g * 256, 0, AUX);
-          sr[H][j][f][g] = __builtin_amdgcn_raw_buffer_load_b32(srsrc, s_at[j] + g * 64, 0, AUX);
+          for (int g = 0; g < 2; ++g) {
+            wr[H][j][f][g] = __builtin_amdgcn_raw_buffer_load_b128(wrsrc, w_at[j] + g * 256, 0, AUX);
+            sr[H][j][f][g] = __builtin_amdgcn_raw_buffer_load_b32(srsrc, s_at[j] + g * 64, 0, AUX);
+          }
+        }
+      };
+      if (MODE == kFetchOnce || (MODE == kFetchEither && u.once))
+        fetch(template_int<kNonTemporalLoad>{});
+      else
+        fetch(template_int<0>{});
+    };
+    auto unit_nst = [&](const DecUnit& u) __attribute__((always_inline)) -> int { return u.key < 0 ? 0 : (u.key >> 24) == 2 ? p.nst2 : p.nst1; };
+    auto unit_nfr = [&](const DecUnit& u) __attribute__((always_inline)) -> int { return (u.key >> 24) == 2 ? p.nfr2 : p.nfr1; };
+    // This wave's K-slice of a row block's activation rows: x through the expert-sorted order for GEMM 1, h for GEMM 2.
+    // The MFMA wants row lr's k-block kg in lane (lr, kg): loaded that way, the sixteen lanes that one pass of a load
+    // serves touch sixteen rows, i.e. sixteen cache lines for 16 bytes each.  So the rows are loaded four lanes to a row
+    // (lane = row * 4 + chunk: 64 contiguous bytes per row and instruction, rows past the block's last dropped, not
+    // repeated) and turned into MFMA order through a 4 KiB buffer of the wave's own in LDS, one K-stage at a time
+    // (LDS operations of a wave execute in order; 16-byte chunks swizzled by the row so that neither side conflicts).
+    const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.x), 0, p.x_bytes, 0x00020000);
+    auto x_request = [&](auto ph_c, const DecUnit& u) __attribute__((always_inline)) {
+      constexpr int ph = decltype(ph_c)::value;  // 1: rows of x, 2: rows of h
+      const int a = (u.key >> 8) & 0xFFFF, rb = u.key & 0xFF;
+      const int e = act_s[a];
+      const int cnt = hist_s[e];
+      const int row0 = offs_s[e] + rb * 16;
+      const int rows = cnt - rb * 16 < 16 ? cnt - rb * 16 : 16;
+      const int r = lane >> 2, c = lane & 3;
+      const bool valid = r < rows;
+      const int K = ph == 2 ? p.K2 : p.K1;
+      // first k of this lane in its wave's slice (opaque: otherwise the twelve addresses below are computed once, ahead
+      // of the loop, and parked in scratch memory, which turns every reload into a chain of dependent memory round trips)
+      int kb = wave * 128 + c * 8;
+      asm volatile("" : "+v"(kb));
+      uint32_t base;
+      if constexpr (ph == 2) {
+        base = (uint32_t)(row0 + r) * (uint32_t)(p.K2 * 2);
+      } else {
+        const int token = rowflat_s[row0 + (valid ? r : 0)] / k;
+        base = (uint32_t)token * (uint32_t)(p.x_stride * 2);
+      }
+#pragma unroll
+      for (int j = 0; j < XS; ++j)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int k0 = kb + j * (NW * 128) + q * 32;
+          // past K the weights are zero (padding, stages past the last): zeros will do
+          const uint32_t off = (valid && k0 < K) ? base + (uint32_t)k0 * 2u : kDroppedStore;
+          if constexpr (ph == 2)
+            xr[j][q] = __builtin_amdgcn_raw_buffer_load_b128(hrsrc, off, 0, kThrough);
+          else
+            xr[j][q] = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, off, 0, 0);
+        }
+    };
+    auto x_settle = [&]() __attribute__((always_inline)) {
+      const int r = lane >> 2, c = lane & 3;
+      const int wpos = r * 4 + (c ^ ((r >> 2) & 3));
+#pragma unroll
+      for (int j = 0; j < XS; ++j) {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int q = 0; q < 4; ++q) xst_s[wave][q][wpos] = xr[j][q];
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int t = 0; t < 4; ++t) xr[j][t] = xst_s[wave][kg][lr * 4 + (t ^ ((lr >> 2) & 3))];
+      }
+    };
+    int cur_key = 0;
+    if (n_units > 0) {
+      bias_fetch(0);
+      // the first unit's activation slice is requested in front of the weight blocks (a wave's requests are answered in
+      // order, and the three units of weight blocks primed below keep the memory system busy for microseconds)
+      const DecUnit first = uniform_unit(0);
+      const bool x_first = (first.key >> 24) == 1;
+      if (x_first) {
+        x_request(std::integral_constant<int, 1>{}, first);
+        cur_key = first.key;
+      }
+      static_for<0, RD>([&](auto h_c) __attribute__((always_inline)) {
+        const DecUnit u = uniform_unit(decltype(h_c)::value);
+#pragma unroll
+        for (int j = 0; j < XS; ++j) load_w(h_c, j, u, unit_nst(u), unit_nfr(u));
+      });
+      // (here, in straight-line code behind the requests, the wait in front of the LDS writes counts the weight blocks
+      // out: behind the bias loops below it would be a wait for everything requested so far)
+      if (x_first) x_settle();
+      bias_park(0);
+    }
+    // A finished GEMM-1 run is counted in without draining the wave's memory queue.  A wave's loads and stores complete
+    // in issue order.  The epilogue of a run's last unit stores its rows of h right behind that unit's barrier; the
+    // next unit opens another row block (or the other GEMM), so EVERY wave starts it by fetching new activation rows
+    // and consumes them in its K loop.  Behind that unit's barrier all stores of the finished run have therefore
+    // reached memory, and the run is counted in there.  (A wait that comes earlier than that, possible only for a
+    // workgroup with next to no units, drains the queue and counts in first: a workgroup must never wait for rows
+    // that it has not counted in itself.)
+    auto unit_body = [&](auto h_c, int i) __attribute__((always_inline)) {
+      constexpr int H = decltype(h_c)::value;
+      const DecUnit cur = uniform_unit(i);
+      const DecUnit nxt = uniform_unit(i + RD);  // the unit that takes over this set of weight registers
+      const int ph = cur.key >> 24, a = (cur.key >> 8) & 0xFFFF, rb = cur.key & 0xFF;
+      const int e = act_s[a];
+      const int cnt = hist_s[e];
+      const int row0 = offs_s[e] + rb * 16;                       // first expert-sorted row of the block
+      const int rows = cnt - rb * 16 < 16 ? cnt - rb * 16 : 16;  // valid rows of the block
+      if (i == 1) DEC_STAMP(3);
+      if (i == n1) DEC_STAMP(4);
+      if (cur.key != cur_key) {
+        cur_key = cur.key;
+        // ---- a new (expert, row block): this wave's K-slice of its activation rows goes into registers ----
+        if (ph == 2) {
+          const int blk = bpre_s[a] + rb;  // a block of the first half was computed by run 0 alone
+          if (!signalled0 || (blk >= bh && !signalled)) {  // (uniform) see above: count in what this workgroup itself still owes
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+            if (!signalled0) signal_blocks(r0b, r0b + nr0);
+            if (!signalled) signal_blocks(r1b, r1b + nr1);
+            signalled0 = signalled = true;
+          }
+          // the block's rows of h are complete when all nu1 GEMM-1 units of the block have been counted in
+          if (tid == 0) {
+            int spins = 0;
+            // (polled gently, and every block's counter in a cache line of its own: a few hundred workgroups polling
+            // one line at full speed slow down every stream that crosses that memory channel)
+            while (__hip_atomic_load(&p.sync[2 + blk * kDecBlockStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < nu1) {
+              __builtin_amdgcn_s_sleep(16);
+              if (++spins > p.spin_limit) {
+                atomicOr(&p.sync[1], 1);
+                break;
+              }
+            }
+          }
+          __syncthreads();
+          if (i == n1) DEC_STAMP(5);
+          x_request(std::integral_constant<int, 2>{}, cur);
+        } else {
+          x_request(std::integral_constant<int, 1>{}, cur);
+        }
+        x_settle();
+      }
+      if (i == 0) DEC_STAMP(14);
+      const int F = cur.frag;
+      // ---- this wave's K-slice of the unit; the next unit's blocks follow into the slots as they fall free ----
+      typename FR::acc_t acc[FPU][2];
+#pragma unroll
+      for (int f = 0; f < FPU; ++f)
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+          for (int c = 0; c < 4; ++c) acc[f][g][c] = 0.f;
+      const int nst_next = unit_nst(nxt), nfr_next = unit_nfr(nxt);
+#pragma unroll
+      for (int j = 0; j < XS; ++j) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+          const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, xr[j][t]);
+#pragma unroll
+          for (int f = 0; f < FPU; ++f)
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+              const u32x4_t v = wr[H][j][f][g];
+              const uint32_t raw = t == 0 ? v.x : t == 1 ? v.y : t == 2 ? v.z : v.w;
+              acc[f][g] = FR::mma(dequant8(raw, bits_f32(((sr[H][j][f][g] >> (8 * kg)) & 0xFFu) << 23)), xf, acc[f][g]);
+            }
+        }
+        load_w(h_c, j, nxt, nst_next, nfr_next);
+      }
+      // ---- the slices meet in LDS; half of the waves, in turn, sum two of the 16 x 32 results a lane in slice order and
+      // finish them (one wave for all of them held up the others' next unit where units are short; all waves: themselves where they are long) ----
+      if (i == 0) DEC_STAMP(15);
+      DEC_UNIT_STAMP(i);
+#pragma unroll
+      for (int f = 0; f < FPU; ++f)
+#pragma unroll
+        for (int g = 0; g < 2; ++g) *reinterpret_cast<f32x4_t*>(&red_s[i & 1][wave][lr][f * 32 + ((g * 4 + kg) ^ (lr & 7)) * 4]) = acc[f][g];
+      __syncthreads();
+      if (i == 0) DEC_STAMP(16);
+      if (i == nr0 && !signalled0) {  // the first unit behind run 0 (it exists and opened a new row block)
+        signalled0 = true;
+        signal_blocks(r0b, r0b + nr0);
+      }
+      if (i == n1 && !signalled) {  // the first GEMM-2 unit
+        signalled = true;
+        signal_blocks(r1b, r1b + nr1);
+      }
+      if ((wave & 1) == (i & 1)) {
+        const int r = (wave >> 1) * 4 + (lane >> 4), c = (lane & 15) * 2;
+        const int flat = rowflat_s[row0 + (r < rows ? r : rows - 1)];
+        const float gam = gate_s[flat];
+        // One store for either GEMM, of two bf16 results: of y (flat row t*k + j) the gate-weighted columns c and c + 1; of h (row row0 + r), by every
+        // second lane, its and its neighbour's swiglu over the (gate, linear) pair
+#pragma unroll
+        for (int f = 0; f < FPU; ++f) {
+          f32x2_t s = {0.f, 0.f};
+#pragma unroll
+          for (int q = 0; q < NW; ++q) s += *reinterpret_cast<const f32x2_t*>(&red_s[i & 1][q][r][f * 32 + ((c >> 2) ^ (r & 7)) * 4 + (c & 3)]);
+          s += *reinterpret_cast<const f32x2_t*>(&bias_s[i][f * 32 + c]);
+          const float o = swiglu_f(s[0], s[1], nalpha_log2e, limit);
+          const float right = quad_swap<0xB1>(o);  // lanes 1 0 3 2 of four
+          const int n = (F + f) * 32 + c;
+          const bool up = ph == 1, mine = r < rows && n < (up ? p.N1 : p.N2) && !(up && (lane & 1));
+          const uint32_t off = up ? (uint32_t)(row0 + r) * (uint32_t)(p.K2 * 2) + (uint32_t)n : (uint32_t)flat * (uint32_t)(p.N2 * 2) + (uint32_t)n * 2u;
+          __builtin_amdgcn_raw_buffer_store_b32(up ? pack_bf16x2(o, right) : pack_bf16x2(s[0] * gam, s[1] * gam), up ? hrsrc : yrsrc, mine ? off : kDroppedStore, 0, kThrough);
         }
       }
     };
-    if (MODE == kFetchOnce || (MODE == kFetchEither && u.once))
-      fetch(template_int<kNonTemporalLoad>{});
-    else
-      fetch(template_int<0>{});
-  };
-  auto unit_nst = [&](const DecUnit& u) __attribute__((always_inline)) -> int { return u.key < 0 ? 0 : (u.key >> 24) == 2 ? p.nst2 : p.nst1; };
-  auto unit_nfr = [&](const DecUnit& u) __attribute__((always_inline)) -> int { return (u.key >> 24) == 2 ? p.nfr2 : p.nfr1; };
-  // This wave's K-slice of a row block's activation rows: x through the expert-sorted order for GEMM 1, h for GEMM 2.
-  // The MFMA wants row lr's k-block kg in lane (lr, kg): loaded that way, the sixteen lanes that one pass of a load
-  // serves touch sixteen rows, i.e. sixteen cache lines for 16 bytes each.  So the rows are loaded four lanes to a row
-  // (lane = row * 4 + chunk: 64 contiguous bytes per row and instruction, rows past the block's last dropped, not
-  // repeated) and turned into MFMA order through a 4 KiB buffer of the wave's own in LDS, one K-stage at a time
-  // (LDS operations of a wave execute in order; 16-byte chunks swizzled by the row so that neither side conflicts).
-  const __amdgpu_buffer_rsrc_t xrsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p.x), 0, p.x_bytes, 0x00020000);
-  auto x_request = [&](auto ph_c, const DecUnit& u) __attribute__((always_inline)) {
-    constexpr int ph = decltype(ph_c)::value;  // 1: rows of x, 2: rows of h
-    const int a = (u.key >> 8) & 0xFFFF, rb = u.key & 0xFF;
-    const int e = act_s[a];
-    const int cnt = hist_s[e];
-    const int row0 = offs_s[e] + rb * 16;
-    const int rows = cnt - rb * 16 < 16 ? cnt - rb * 16 : 16;
-    const int r = lane >> 2, c = lane & 3;
-    const bool valid = r < rows;
-    const int K = ph == 2 ? p.K2 : p.K1;
-    // first k of this lane in its wave's slice (opaque: otherwise the twelve addresses below are computed once, ahead
-    // of the loop, and parked in scratch memory, which turns every reload into a chain of dependent memory round trips)
-    int kb = wave * 128 + c * 8;
-    asm volatile("" : "+v"(kb));
-    uint32_t base;
-    if constexpr (ph == 2) {
-      base = (uint32_t)(row0 + r) * (uint32_t)(p.K2 * 2);
-    } else {
-      const int token = rowflat_s[row0 + (valid ? r : 0)] / k;
-      base = (uint32_t)token * (uint32_t)(p.x_stride * 2);
-    }
-#pragma unroll
-    for (int j = 0; j < XS; ++j)
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        const int k0 = kb + j * (NW * 128) + q * 32;
-        // past K the weights are zero (padding, stages past the last): zeros will do
-        const uint32_t off = (valid && k0 < K) ? base + (uint32_t)k0 * 2u : kDroppedStore;
-        if constexpr (ph == 2)
-          xr[j][q] = __builtin_amdgcn_raw_buffer_load_b128(hrsrc, off, 0, kThrough);
-        else
-          xr[j][q] = __builtin_amdgcn_raw_buffer_load_b128(xrsrc, off, 0, 0);
-      }
-  };
-  auto x_settle = [&]() __attribute__((always_inline)) {
-    const int r = lane >> 2, c = lane & 3;
-    const int wpos = r * 4 + (c ^ ((r >> 2) & 3));
-#pragma unroll
-    for (int j = 0; j < XS; ++j) {
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int q = 0; q < 4; ++q) xst_s[wave][q][wpos] = xr[j][q];
-      __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-#pragma unroll
-      for (int t = 0; t < 4; ++t) xr[j][t] = xst_s[wave][kg][lr * 4 + (t ^ ((lr >> 2) & 3))];
-    }
-  };
-  int cur_key = 0;
-  if (n_units > 0) {
-    bias_fetch(0);
-    // the first unit's activation slice is requested in front of the weight blocks (a wave's requests are answered in
-    // order, and the three units of weight blocks primed below keep the memory system busy for microseconds)
-    const DecUnit first = uniform_unit(0);
-    const bool x_first = (first.key >> 24) == 1;
-    if (x_first) {
-      x_request(std::integral_constant<int, 1>{}, first);
-      cur_key = first.key;
-    }
-    static_for<0, RD>([&](auto h_c) __attribute__((always_inline)) {
-      const DecUnit u = uniform_unit(decltype(h_c)::value);
-#pragma unroll
-      for (int j = 0; j < XS; ++j) load_w(h_c, j, u, unit_nst(u), unit_nfr(u));
+    // Whole rounds of RD units run without a test between the units: with one, the compiler has to allow for a round
+    // that skips its later units and comes back to the first, i.e. for weight blocks that nothing younger follows, and
+    // its waits then drain the wave's memory queue once per round.
+    int i_unit = 0;
+    for (; i_unit + RD <= n_units; i_unit += RD)
+      static_for<0, RD>([&](auto h_c) __attribute__((always_inline)) { unit_body(h_c, i_unit + decltype(h_c)::value); });
+    static_for<0, RD - 1>([&](auto h_c) __attribute__((always_inline)) {
+      if (i_unit + decltype(h_c)::value < n_units) unit_body(h_c, i_unit + decltype(h_c)::value);
     });
-    // (here, in straight-line code behind the requests, the wait in front of the LDS writes counts the weight blocks
-    // out: behind the bias loops below it would be a wait for everything requested so far)
-    if (x_first) x_settle();
-    bias_park(0);
-  }
-  // A finished GEMM-1 run is counted in without draining the wave's memory queue.  A wave's loads and stores complete
-  // in issue order.  The epilogue of a run's last unit stores its rows of h right behind that unit's barrier; the
-  // next unit opens another row block (or the other GEMM), so EVERY wave starts it by fetching new activation rows
-  // and consumes them in its K loop.  Behind that unit's barrier all stores of the finished run have therefore
-  // reached memory, and the run is counted in there.  (A wait that comes earlier than that, possible only for a
-  // workgroup with next to no units, drains the queue and counts in first: a workgroup must never wait for rows
-  // that it has not counted in itself.)
-  auto unit_body = [&](auto h_c, int i) __attribute__((always_inline)) {
-    constexpr int H = decltype(h_c)::value;
-    const DecUnit cur = uniform_unit(i);
-    const DecUnit nxt = uniform_unit(i + RD);  // the unit that takes over this set of weight registers
-    const int ph = cur.key >> 24, a = (cur.key >> 8) & 0xFFFF, rb = cur.key & 0xFF;
-    const int e = act_s[a];
-    const int cnt = hist_s[e];
-    const int row0 = offs_s[e] + rb * 16;                       // first expert-sorted row of the block
-    const int rows = cnt - rb * 16 < 16 ? cnt - rb * 16 : 16;  // valid rows of the block
-    if (i == 1) DEC_STAMP(3);
-    if (i == n1) DEC_STAMP(4);
-    if (cur.key != cur_key) {
-      cur_key = cur.key;
-      // ---- a new (expert, row block): this wave's K-slice of its activation rows goes into registers ----
-      if (ph == 2) {
-        const int blk = bpre_s[a] + rb;  // a block of the first half was computed by run 0 alone
-        if (!signalled0 || (blk >= bh && !signalled)) {  // (uniform) see above: count in what this workgroup itself still owes
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          __syncthreads();
-          if (!signalled0) signal_blocks(r0b, r0b + nr0);
-          if (!signalled) signal_blocks(r1b, r1b + nr1);
-          signalled0 = signalled = true;
-        }
-        // the block's rows of h are complete when all nu1 GEMM-1 units of the block have been counted in
-        if (tid == 0) {
-          int spins = 0;
-          // (polled gently, and every block's counter in a cache line of its own: a few hundred workgroups polling
-          // one line at full speed slow down every stream that crosses that memory channel)
-          while (__hip_atomic_load(&p.sync[2 + blk * kDecBlockStride], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < nu1) {
-            __builtin_amdgcn_s_sleep(16);
-            if (++spins > p.spin_limit) {
-              atomicOr(&p.sync[1], 1);
-              break;
-            }
-          }
-        }
-        __syncthreads();
-        if (i == n1) DEC_STAMP(5);
-        x_request(std::integral_constant<int, 2>{}, cur);
-      } else {
-        x_request(std::integral_constant<int, 1>{}, cur);
-      }
-      x_settle();
-    }
-    if (i == 0) DEC_STAMP(14);
-    const int F = cur.frag;
-    // ---- this wave's K-slice of the unit; the next unit's blocks follow into the slots as they fall free ----
-    typename FR::acc_t acc[FPU][2];
-#pragma unroll
-    for (int f = 0; f < FPU; ++f)
-#pragma unroll
-      for (int g = 0; g < 2; ++g)
-#pragma unroll
-        for (int c = 0; c < 4; ++c) acc[f][g][c] = 0.f;
-    const int nst_next = unit_nst(nxt), nfr_next = unit_nfr(nxt);
-#pragma unroll
-    for (int j = 0; j < XS; ++j) {
-#pragma unroll
-      for (int t = 0; t < 4; ++t) {
-        const bf16x8_t xf = __builtin_bit_cast(bf16x8_t, xr[j][t]);
-#pragma unroll
-        for (int f = 0; f < FPU; ++f)
-#pragma unroll
-          for (int g = 0; g < 2; ++g) {
-            const u32x4_t v = wr[H][j][f][g];
-            const uint32_t raw = t == 0 ? v.x : t == 1 ? v.y : t == 2 ? v.z : v.w;
-            acc[f][g] = FR::mma(dequant8(raw, bits_f32(((sr[H][j][f][g] >> (8 * kg)) & 0xFFu) << 23)), xf, acc[f][g]);
-          }
-      }
-      load_w(h_c, j, nxt, nst_next, nfr_next);
-    }
-    // ---- the slices meet in LDS; half of the waves, in turn, sum two of the 16 x 32 results a lane in slice order and
-    // finish them (one wave for all of them held up the others' next unit where units are short; all waves: themselves where they are long) ----
-    if (i == 0) DEC_STAMP(15);
-    DEC_UNIT_STAMP(i);
-#pragma unroll
-    for (int f = 0; f < FPU; ++f)
-#pragma unroll
-      for (int g = 0; g < 2; ++g) *reinterpret_cast<f32x4_t*>(&red_s[i & 1][wave][lr][f * 32 + ((g * 4 + kg) ^ (lr & 7)) * 4]) = acc[f][g];
-    __syncthreads();
-    if (i == 0) DEC_STAMP(16);
-    if (i == nr0 && !signalled0) {  // the first unit behind run 0 (it exists and opened a new row block)
-      signalled0 = true;
-      signal_blocks(r0b, r0b + nr0);
-    }
-    if (i == n1 && !signalled) {  // the first GEMM-2 unit
-      signalled = true;
-      signal_blocks(r1b, r1b + nr1);
-    }
-    if ((wave & 1) == (i & 1)) {
-      const int r = (wave >> 1) * 4 + (lane >> 4), c = (lane & 15) * 2;
-      const int flat = rowflat_s[row0 + (r < rows ? r : rows - 1)];
-      const float gam = gate_s[flat];
-      // One store for either GEMM, of two bf16 results: of y (flat row t*k + j) the gate-weighted columns c and c + 1; of h (row row0 + r), by every
-      // second lane, its and its neighbour's swiglu over the (gate, linear) pair
-#pragma unroll
-      for (int f = 0; f < FPU; ++f) {
-        f32x2_t s = {0.f, 0.f};
-#pragma unroll
-        for (int q = 0; q < NW; ++q) s += *reinterpret_cast<const f32x2_t*>(&red_s[i & 1][q][r][f * 32 + ((c >> 2) ^ (r & 7)) * 4 + (c & 3)]);
-        s += *reinterpret_cast<const f32x2_t*>(&bias_s[i][f * 32 + c]);
-        const float o = swiglu_f(s[0], s[1], nalpha_log2e, limit);
-        const float right = quad_swap<0xB1>(o);  // lanes 1 0 3 2 of four
-        const int n = (F + f) * 32 + c;
-        const bool up = ph == 1, mine = r < rows && n < (up ? p.N1 : p.N2) && !(up && (lane & 1));
-        const uint32_t off = up ? (uint32_t)(row0 + r) * (uint32_t)(p.K2 * 2) + (uint32_t)n : (uint32_t)flat * (uint32_t)(p.N2 * 2) + (uint32_t)n * 2u;
-        __builtin_amdgcn_raw_buffer_store_b32(up ? pack_bf16x2(o, right) : pack_bf16x2(s[0] * gam, s[1] * gam), up ? hrsrc : yrsrc, mine ? off : kDroppedStore, 0, kThrough);
-      }
-    }
-  };
-  // Whole rounds of RD units run without a test between the units: with one, the compiler has to allow for a round
-  // that skips its later units and comes back to the first, i.e. for weight blocks that nothing younger follows, and
-  // its waits then drain the wave's memory queue once per round.
-  int i_unit = 0;
-  for (; i_unit + RD <= n_units; i_unit += RD)
-    static_for<0, RD>([&](auto h_c) __attribute__((always_inline)) { unit_body(h_c, i_unit + decltype(h_c)::value); });
-  static_for<0, RD - 1>([&](auto h_c) __attribute__((always_inline)) {
-    if (i_unit + decltype(h_c)::value < n_units) unit_body(h_c, i_unit + decltype(h_c)::value);
-  });
   };  // stream
   if constexpr (FETCH != kFetchEither) {
     stream(template_int<FETCH>{});

@@ -340,42 +340,42 @@ __device__ __forceinline__ void dma_gemm(const GemmParams& p) {
       continue;
     }
     if constexpr (!SMALL) {
-    prime();
+      prime();
 #pragma unroll
-    for (int f = 0; f < NFW; ++f)
+      for (int f = 0; f < NFW; ++f)
 #pragma unroll
-      for (int j = 0; j < MFW; ++j)
+        for (int j = 0; j < MFW; ++j)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) acc[f][j][i] = 0.f;
-    const int rows = cur.eM - cur.off_m < C::BM ? cur.eM - cur.off_m : C::BM;
-    const int jc = __builtin_amdgcn_readfirstlane((((rows + 31) >> 5) - mw + C::WM - 1) / C::WM);  // this wave's row fragments (j * WM + mw) that hold rows
-    auto stages = [&](auto nj_c) __attribute__((always_inline)) {
-      for (int s = 0; s < nst; ++s) {
-        quarter(nj_c, template_int<0>{}, jc, ab, bb);
-        quarter(nj_c, template_int<1>{}, jc, ab, bb);
-        quarter(nj_c, template_int<2>{}, jc, ab, bb);
-        // the next stage has landed (this wave's part) when only the transfers of quarters 0 and 1 are outstanding
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::BBUFS == 2 ? 0 : C::BI) : "memory");
-        barrier();
-        ab = ab + C::ABYTES == kAEnd ? 0 : ab + C::ABYTES;
-        bb = bb + C::BBYTES == kBEnd ? kAEnd : bb + C::BBYTES;
-        quarter(nj_c, template_int<3>{}, jc, ab, bb);
-        // (the one branch of a stage stands at its end: with one in between, the compiler moves the multiplications in front of it
-        // down behind it, and their operands pile up)
-        advance();
-      }
-    };
-    if (jc >= MFW)
-      stages(template_int<MFW>{});
-    else if (MFW == 5 && jc == 4)
-      stages(template_int<MFW == 5 ? 4 : 0>{});
-    else
-      stages(template_int<0>{});
-    gemm_epilogue<32, C::WM, MFW, NFW, SWIGLU, WK == WK_F16>(p, acc, cur.expert, cur.off_m, cur.start_m, cur.eM, cur.n_tile + nw * NFW * 32,
-                                                             cur.n_tile + C::BN <= p.N, mw, lr, h);
-    tile += t_step;
-    if (tile >= t_end) break;
-    cur = locate(tile);
+          for (int i = 0; i < 16; ++i) acc[f][j][i] = 0.f;
+      const int rows = cur.eM - cur.off_m < C::BM ? cur.eM - cur.off_m : C::BM;
+      const int jc = __builtin_amdgcn_readfirstlane((((rows + 31) >> 5) - mw + C::WM - 1) / C::WM);  // this wave's row fragments (j * WM + mw) that hold rows
+      auto stages = [&](auto nj_c) __attribute__((always_inline)) {
+        for (int s = 0; s < nst; ++s) {
+          quarter(nj_c, template_int<0>{}, jc, ab, bb);
+          quarter(nj_c, template_int<1>{}, jc, ab, bb);
+          quarter(nj_c, template_int<2>{}, jc, ab, bb);
+          // the next stage has landed (this wave's part) when only the transfers of quarters 0 and 1 are outstanding
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"(C::BBUFS == 2 ? 0 : C::BI) : "memory");
+          barrier();
+          ab = ab + C::ABYTES == kAEnd ? 0 : ab + C::ABYTES;
+          bb = bb + C::BBYTES == kBEnd ? kAEnd : bb + C::BBYTES;
+          quarter(nj_c, template_int<3>{}, jc, ab, bb);
+          // (the one branch of a stage stands at its end: with one in between, the compiler moves the multiplications in front of it
+          // down behind it, and their operands pile up)
+          advance();
+        }
+      };
+      if (jc >= MFW)
+        stages(template_int<MFW>{});
+      else if (MFW == 5 && jc == 4)
+        stages(template_int<MFW == 5 ? 4 : 0>{});
+      else
+        stages(template_int<0>{});
+      gemm_epilogue<32, C::WM, MFW, NFW, SWIGLU, WK == WK_F16>(p, acc, cur.expert, cur.off_m, cur.start_m, cur.eM, cur.n_tile + nw * NFW * 32,
+                                                               cur.n_tile + C::BN <= p.N, mw, lr, h);
+      tile += t_step;
+      if (tile >= t_end) break;
+      cur = locate(tile);
     }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // no transfer into this workgroup's LDS is left behind
