@@ -217,6 +217,40 @@ def test_weights_fetched_with_the_hint_and_without(api, device, gptoss_weights, 
     assert torch.equal(outs[0], outs[1])
 
 
+@pytest.mark.parametrize("k_len", [2080, 2304, 2880, 3072])
+@pytest.mark.parametrize("second", [False, True], ids=["gemm1", "gemm2"])
+def test_long_k_is_summed_in_consecutive_slices(api, device, k_len, second):
+    """K beyond 2048: an fp32 sum per slice of 384 consecutive k, the slices added in order.  A large value and its negative inside the first slice
+    cancel, whatever comes later; in any other grouping of the stages of 128 k they swallow the 1 of the third slice."""
+    from bench import to_matmul_layout
+    T, E, big = 72, 1, 2.0**30
+    marks = {130: big, 300: -big, 1030: 1.0}  # k -> value of the summand
+    d, f = (64, k_len) if second else (k_len, 64)
+    x = torch.zeros((T, d), dtype=torch.bfloat16)
+    w1, w2 = torch.zeros((E, d, 2 * f), dtype=torch.bfloat16), torch.zeros((E, f, d), dtype=torch.bfloat16)
+    b1, b2 = torch.zeros((E, 2 * f)), torch.zeros((E, d))
+    b1[:, ::2] = 1.0  # the gate: silu(1) times (linear + 1)
+    silu = (1.0 / (1.0 + torch.exp(torch.tensor(-1.702)))).to(torch.bfloat16).float()
+    if second:
+        b1[:, 1::2] = -1.0
+        for at, v in marks.items():
+            b1[:, 2 * at + 1] = v - 1.0
+        w2[:] = 1.0
+        want = silu
+    else:
+        for at, v in marks.items():
+            x[:, at] = v
+        w1[:, :, 1::2] = 1.0
+        w2[:, 0] = 1.0
+        want = 2 * silu
+    w1q, w1s = omx.downcast_to_mxfp(w1, torch.uint8, axis=1)
+    w2q, w2s = omx.downcast_to_mxfp(w2, torch.uint8, axis=1)
+    W = to_matmul_layout({n: t.to(device) for n, t in dict(w1=w1q, w1s=w1s, w2=w2q, w2s=w2s, b1=b1, b2=b2).items()})
+    out = _run(api, W, x.to(device), torch.zeros((T, E), device=device), 1, api.act(1.702, None))
+    torch.cuda.synchronize()
+    assert torch.allclose(out.float().cpu(), want.expand(T, d), rtol=2**-7, atol=0)
+
+
 def test_one_launch_layer_in_a_hip_graph(api, device, gptoss_weights):
     """Captured once, replayed three times with new inputs and eager launches in between; every replay must equal the
     eager launch on the same inputs bit for bit."""

@@ -9,7 +9,8 @@
 //      expert histogram, stable expert-sorted row order - into LDS, no global round trip, no dependence on others.
 //   2. The work is cut into units = (active expert, 16-row block, one or two 32-column weight fragments) of GEMM 1 followed by
 //      those of GEMM 2; every workgroup takes an equal contiguous share of each list, derived from the LDS tables.
-//   3. The NW waves of a workgroup take the K-stages of a unit in turn (XS = 1 to 3 each); a wave keeps its part of the
+//   3. The NW waves of a workgroup share the K-stages of a unit (XS = 1 to 3 each; three: consecutive ones, so that the sums are those of
+//      K / 384 slices added in order; one or two: in turn, which leaves no wave idle); a wave keeps its part of the
 //      block's activation rows in REGISTERS for as long as the (expert, row block) stays the same, so the inner loop
 //      is: 2 KiB weight block global -> registers (ring, one unit ahead), e2m1 -> bf16 in registers, 16x16x32 MFMA.
 //      The slices meet in LDS once per unit (one barrier); four of the waves, in turn, sum them and run the
@@ -55,6 +56,7 @@ struct DecUnit {
 template <int XS_, int FPU_>
 struct DecCfg {
   static constexpr int XS = XS_, FPU = FPU_;
+  static constexpr int STAGE0 = XS == 3 ? 3 : 1, STEP = XS == 3 ? 1 : kDecNW;  // wave w's stages: w * STAGE0 + j * STEP
   static constexpr int RING = XS * FPU >= 3 ? 3 : 4;      // units of weight blocks a wave holds or has requested
   static constexpr int UNITS = kDecMaxUnits / FPU;        // of one workgroup
   static constexpr int COLS = 32 * FPU;
@@ -323,7 +325,7 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
 
   // ---- 3. the stream ----------------------------------------------------------------------------------------
   // lane (lr, kg): weight columns g*16 + lr of the fragment, k-block kg (32 k = 16 packed bytes) of every stage;
-  // this wave's stages of a unit are wave + j * NW: the waves of a short K have the same share of it
+  // this wave's stages of a unit are wave * STAGE0 + j * STEP
   const uint32_t wlane = (uint32_t)((kg & 1) * 1024 + ((kg >> 1) * 32 + lr) * 16);
   const uint32_t slane = (uint32_t)(lr * 4);
   // weight registers: RD sets of XS stages; unit i lives in set i % RD and, stage by stage as it is consumed, is
@@ -411,7 +413,7 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
     // counts stay exact only in straight-line code.)
     uint32_t w_at[XS], s_at[XS];
 #pragma unroll
-    for (int j = 0; j < XS; ++j) w_at[j] = wlane + (uint32_t)(wave + j * NW) * 2048u, s_at[j] = slane + (uint32_t)(wave + j * NW) * 128u;
+    for (int j = 0; j < XS; ++j) w_at[j] = wlane + (uint32_t)(wave * C::STAGE0 + j * C::STEP) * 2048u, s_at[j] = slane + (uint32_t)(wave * C::STAGE0 + j * C::STEP) * 128u;
     auto load_w = [&](auto h_c, int j, const DecUnit& u, int nst, int nfr) __attribute__((always_inline)) {
       constexpr int H = decltype(h_c)::value;
       auto fetch = [&](auto aux_c) __attribute__((always_inline)) {
@@ -454,7 +456,7 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
       const int K = ph == 2 ? p.K2 : p.K1;
       // first k of this lane in its wave's slice (opaque: otherwise the twelve addresses below are computed once, ahead
       // of the loop, and parked in scratch memory, which turns every reload into a chain of dependent memory round trips)
-      int kb = wave * 128 + c * 8;
+      int kb = wave * (C::STAGE0 * 128) + c * 8;
       asm volatile("" : "+v"(kb));
       uint32_t base;
       if constexpr (ph == 2) {
@@ -467,7 +469,7 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
       for (int j = 0; j < XS; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-          const int k0 = kb + j * (NW * 128) + q * 32;
+          const int k0 = kb + j * (C::STEP * 128) + q * 32;
           // past K the weights are zero (padding, stages past the last): zeros will do
           const uint32_t off = (valid && k0 < K) ? base + (uint32_t)k0 * 2u : kDroppedStore;
           if constexpr (ph == 2)
