@@ -351,3 +351,20 @@ def test_columns_of_the_kernel_for_few_rows(per_slice, N, n_slices, want):
     """Both sides of the line: with 64 columns a second round for slices of over 64 rows costs more than the kernel gains."""
     from triton_amd import _native as nt
     assert nt.rules().few_block_n(per_slice * n_slices, N, n_slices) == want
+
+
+@pytest.mark.parametrize("outer, length, inner", [
+    (16, 1024, 3200), (26, 2048, 1024), (8, 2048, 3328), (2, 5120, 5120), (7, 2880, 2560), (2, 1024, 26624), (3, 2880, 5760), (4, 2880, 5760), (1, 64, 528), (260, 288, 260), (5, 32, 7)])
+@pytest.mark.parametrize("e2m1", [True, False])
+@pytest.mark.parametrize("down", [True, False])
+def test_every_workgroup_of_the_mx_tiles_has_a_block(outer, length, inner, e2m1, down):
+    """The number of workgroups is that of the tiles of the kernel that runs, above all from 96 to 128 MiB, where both the rule for reading once and the
+    one for small tensors apply."""
+    from triton_amd import _native as nt
+    grid, blocks, once = nt.rules().mx_tiles(outer, length, inner, e2m1, down)
+    cols = -(-inner // 256) * outer
+    assert grid % cols == 0 and (grid // cols - 1) * blocks < length // 32 <= grid // cols * blocks
+    assert blocks in ((4, 8) if e2m1 else (4, ))
+    assert not once or down
+    if e2m1 and (outer, length, inner) == (260, 288, 260):
+        assert blocks == 8

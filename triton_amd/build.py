@@ -52,7 +52,7 @@ def _compile(src: str, force: bool) -> str:
 
 
 def _build_host(force: bool) -> None:
-    deps = [HOST_SRC, os.path.join(CSRC, "gemm_limits.h"), os.path.join(HERE, "..", "include", "triton_amd.h")]
+    deps = [HOST_SRC, os.path.join(CSRC, "gemm_limits.h"), os.path.join(CSRC, "mx_tiles.h"), os.path.join(HERE, "..", "include", "triton_amd.h")]
     if not force and os.path.exists(HOST_LIB) and all(os.path.getmtime(d) <= os.path.getmtime(HOST_LIB) for d in deps):
         return
     import torch

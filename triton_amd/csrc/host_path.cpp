@@ -28,6 +28,7 @@
 
 #include "../../include/triton_amd.h"
 #include "gemm_limits.h"
+#include "mx_tiles.h"
 
 namespace {
 
@@ -866,6 +867,11 @@ PyObject* rule_wide(PyObject* const* v) {
   const auto [rows, n_slices, K, N, x_bytes, mx8] = integers<6>(v);
   return PyLong_FromLongLong(wide_block_m(rows, n_slices, K, N, uint32_t(x_bytes), mx8 != 0));
 }
+PyObject* rule_mx_tiles(PyObject* const* v) {
+  const auto [outer, L, inner, e2m1, down] = integers<5>(v);
+  const tk::MxTiles t = tk::mx_tiles(outer, L, inner, e2m1 != 0, down != 0);
+  return Py_BuildValue("(Lii)", (long long)t.grid, (int)t.blocks, (int)t.once);
+}
 
 // bind(dict): the addresses of the entry points (integers) and the Python objects above
 PyObject* bind(PyObject*, PyObject* dict) {
@@ -926,6 +932,7 @@ PyMethodDef methods[] = {
     METHOD("mxfp4_block_m", rule_mxfp4, 3),
     METHOD("wide_block_m", rule_wide, 6),
     METHOD("wide_block_n", rule_wide_n, 6),
+    METHOD("mx_tiles", rule_mx_tiles, 5),
     {nullptr, nullptr, 0, nullptr},
 };
 

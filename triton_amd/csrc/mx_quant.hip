@@ -9,6 +9,7 @@
 //   tile : the cols case for 16-bit tensors of four columns and more, with an LDS transpose so that the quantised
 //          bytes of a column move as full 128-byte lines (mx_down_tile / mx_up_tile).
 #include "mx_math.h"
+#include "mx_tiles.h"
 
 namespace tk {
 namespace {
@@ -413,7 +414,7 @@ __global__ __launch_bounds__(kThreads) void mx_up_cols(const uint8_t* __restrict
 // 128-byte line (8 lanes x 16 bytes) instead of 16- or 32-byte pieces of 64 different lines per instruction,
 // and a lane walks its rows with 8-byte accesses (4 columns), so a wave covers 512 contiguous bytes per row.
 // ---------------------------------------------------------------------------------------------
-constexpr int kTileCols = 256;
+constexpr int kTileCols = kMxTileCols;
 constexpr int kTilePitch = 128 + 16;  // LDS bytes per column
 // LDS row of tile column c: a lane's four adjacent columns are spread 65 rows apart, so the 16-byte accesses of
 // consecutive lanes (columns c, c + 4, ...) fall 144 bytes apart and take different banks
@@ -445,8 +446,8 @@ __device__ __forceinline__ int64_t tile_order(int64_t pid, int64_t total) {
 template <int KIND>
 struct TileGeom {
   static constexpr int BB = KIND == TK_E2M1 ? 16 : 32;  // value bytes per block and column
-  static constexpr int NB = 128 / BB;                    // blocks per tile
-  static constexpr int SMALL = 4;                        // ... of a small tensor: one a wave
+  static constexpr int NB = mx_tile_blocks(KIND == TK_E2M1), SMALL = kMxSmallBlocks;  // blocks per tile
+  static_assert(NB * BB == 128, "a column of a tile is a whole line");
 };
 
 // moves the tile's value bytes and scales between LDS and global memory (TO_GLOBAL) or back
@@ -594,10 +595,7 @@ __device__ __forceinline__ uint2 load_once_u2(const uint16_t* p) {
   return make_uint2(t.x, t.y);
 }
 
-// Sources of this size and more are read with the non-temporal hint.  Two in turn, plain loads / with the hint, us a launch, bf16 [b, 2880, 5760] to e4m3:
-// b 2 (66 MB) 18.1 / 23.8, b 4 47.8 / 39.5, b 8 107 / 75, b 16 181 / 153, b 32 343 / 300; to e2m1: b 2 18.9 / 21.8, b 4 42.6 / 36.8, b 8 95 / 68.  What
-// was used a moment ago is still in the memory-side cache up to about a hundred megabytes, and a read with the hint does not profit from that.
-constexpr int64_t kOnceBytes = 96ll << 20;
+// NT: the source is read with the hint; NB: blocks of 32 in a tile (mx_tiles).
 template <int SRC, int KIND, bool NT, int NB>
 __global__ __launch_bounds__(kThreads) void mx_down_tile(const uint16_t* __restrict__ src, int64_t stride_outer, int64_t stride_axis,
                                                          int64_t L, int64_t inner, int64_t inner_last, int64_t col_tiles,
@@ -748,11 +746,6 @@ __global__ __launch_bounds__(kThreads) void mx_up_tile(const uint8_t* __restrict
 }
 
 // ---- dispatch helpers --------------------------------------------------------------------------
-// e2m1: half as many blocks a tile, one a wave instead of two, where the tiles of whole lines are up to four a CU: both directions are a chain of loads, conversion and stores, and
-// half of it is shorter (us, both launches: 1 x 2368 x 592 14.6 -> 9.7, 11 x 448 x 256 14.3 -> 9.4, 5 x 544 x 2368 15.9 -> 11.6, 8 x 1024 x 1024 15.3 -> 12.5, 1 x 2880 x 5760 (276 tiles)
-// 24.5 -> 20.3, 2 x (552) 35.1 -> 32.8, 16 x 2048 x 1024 (512) 30.8 -> 29.3; 8 x 2880 x 2880 (1152) 65.1 -> 66.6, since a column's piece is half a line).
-bool small_tiles(int64_t tiles) { return tiles <= 1024; }
-
 template <int SRC, int KIND>
 int32_t launch_down(const void* src, int64_t outer, int64_t L, int64_t inner, int64_t inner_last, int64_t so, int64_t sa, int64_t si,
                     void* out_vals, void* out_scales, int rounding, hipStream_t st) {
@@ -774,13 +767,15 @@ int32_t launch_down(const void* src, int64_t outer, int64_t L, int64_t inner, in
   if constexpr (sizeof(T) == 2) {
     if (inner >= 4 && (reinterpret_cast<uintptr_t>(out_vals) % 16) == 0) {
       typedef TileGeom<KIND> G;
-      const int64_t col_tiles = cdiv(inner, kTileCols);
-      const bool once = outer * L * inner * 2 >= kOnceBytes, small = small_tiles(col_tiles * cdiv(nblk, G::NB) * outer);
-      const int64_t blk_tiles = cdiv(nblk, small ? G::SMALL : G::NB);
-      const int64_t grid = col_tiles * blk_tiles * outer;
-      if (grid > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_mx_downcast: tensor too large for one launch");
-      hipLaunchKernelGGL((once ? mx_down_tile<SRC, KIND, true, G::NB> : small ? mx_down_tile<SRC, KIND, false, G::SMALL> : mx_down_tile<SRC, KIND, false, G::NB>), dim3((unsigned)grid), dim3(kThreads), 0, st,
-                         reinterpret_cast<const uint16_t*>(s), so, sa, L, inner, inner_last, col_tiles, blk_tiles, ov, os, rounding);
+      const MxTiles t = mx_tiles(outer, L, inner, KIND == TK_E2M1, true);
+      if (t.grid > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_mx_downcast: tensor too large for one launch");
+      auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)t.grid), dim3(kThreads), 0, st, reinterpret_cast<const uint16_t*>(s), so, sa, L, inner, inner_last, t.col_tiles, t.blk_tiles, ov, os, rounding);
+      };
+      if (t.blocks == G::NB)
+        launch(t.once ? mx_down_tile<SRC, KIND, true, G::NB> : mx_down_tile<SRC, KIND, false, G::NB>);
+      else
+        launch(mx_down_tile<SRC, KIND, false, G::SMALL>);
       return check_launch("mx_down_tile");
     }
   }
@@ -822,13 +817,10 @@ int32_t launch_up(const void* vals, const void* scales, int64_t outer, int64_t L
   if constexpr (sizeof(T) == 2) {
     if (inner >= 4 && (reinterpret_cast<uintptr_t>(vals) % 16) == 0) {
       typedef TileGeom<KIND> G;
-      const int64_t col_tiles = cdiv(inner, kTileCols);
-      const bool small = small_tiles(col_tiles * cdiv(nblk, G::NB) * outer);
-      const int64_t blk_tiles = cdiv(nblk, small ? G::SMALL : G::NB);
-      const int64_t grid = col_tiles * blk_tiles * outer;
-      if (grid > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_mx_upcast: tensor too large for one launch");
-      hipLaunchKernelGGL((small ? mx_up_tile<KIND, DST, G::SMALL> : mx_up_tile<KIND, DST, G::NB>), dim3((unsigned)grid), dim3(kThreads), 0, st, v, s, L, inner, inner_last, col_tiles,
-                         blk_tiles, reinterpret_cast<uint16_t*>(o), oso, osa);
+      const MxTiles t = mx_tiles(outer, L, inner, KIND == TK_E2M1, false);
+      if (t.grid > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_mx_upcast: tensor too large for one launch");
+      hipLaunchKernelGGL((t.blocks == G::NB ? mx_up_tile<KIND, DST, G::NB> : mx_up_tile<KIND, DST, G::SMALL>), dim3((unsigned)t.grid), dim3(kThreads), 0, st, v, s, L, inner, inner_last,
+                         t.col_tiles, t.blk_tiles, reinterpret_cast<uint16_t*>(o), oso, osa);
       return check_launch("mx_up_tile");
     }
   }
