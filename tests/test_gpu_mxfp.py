@@ -297,3 +297,18 @@ def test_tiles_of_many_blocks_give_what_small_ones_give(device, dtype, outer, le
         qi, si = downcast_to_mxfp(x[i:i + 20], torch.uint8, axis=1)
         assert torch.equal(q[i:i + 20], qi) and torch.equal(s[i:i + 20], si)
         assert torch.equal(back[i:i + 20], upcast_from_mxfp(qi, si, dtype, axis=1))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "fp16"])
+@pytest.mark.parametrize("shape", [(3, 2880, 2204), (3, 2880, 2203)])
+def test_small_tiles_read_with_the_hint_and_without(device, dtype, shape):
+    """To e2m1, small tiles just above the size from which the source is read with the hint (where its rows allow it): the bytes of one matrix at a time."""
+    from triton_amd import _native as nt
+    from triton_kernels.numerics_details.mxfp import downcast_to_mxfp
+    aligned = shape[2] % 4 == 0
+    assert nt.rules().mx_tiles(*shape, True, True, aligned)[1:] == (4, int(aligned)) and nt.rules().mx_tiles(1, *shape[1:], True, True, aligned)[1:] == (4, 0)
+    x = torch.randn(shape, generator=torch.Generator(device=device).manual_seed(7), device=device).to(dtype)
+    q, s = downcast_to_mxfp(x, torch.uint8, axis=1)
+    for i in range(shape[0]):
+        qi, si = downcast_to_mxfp(x[i:i + 1].clone(), torch.uint8, axis=1)
+        assert torch.equal(q[i:i + 1], qi) and torch.equal(s[i:i + 1], si)

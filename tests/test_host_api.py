@@ -361,10 +361,19 @@ def test_every_workgroup_of_the_mx_tiles_has_a_block(outer, length, inner, e2m1,
     """The number of workgroups is that of the tiles of the kernel that runs, above all from 96 to 128 MiB, where both the rule for reading once and the
     one for small tensors apply."""
     from triton_amd import _native as nt
-    grid, blocks, once = nt.rules().mx_tiles(outer, length, inner, e2m1, down)
+    grid, blocks, once = nt.rules().mx_tiles(outer, length, inner, e2m1, down, inner % 4 == 0)
     cols = -(-inner // 256) * outer
     assert grid % cols == 0 and (grid // cols - 1) * blocks < length // 32 <= grid // cols * blocks
     assert blocks in ((4, 8) if e2m1 else (4, ))
     assert not once or down
     if e2m1 and (outer, length, inner) == (260, 288, 260):
         assert blocks == 8
+
+
+def test_sources_to_e2m1_are_read_with_the_hint():
+    """From 36 MiB on: a tensor that the program did not touch lately, which a first call on loaded weights has, is read faster with it."""
+    from triton_amd import _native as nt
+    for outer, length, inner in [(3, 2880, 2880), (8, 2048, 2048), (2, 2880, 5760), (3, 2880, 5760), (13, 2048, 2048), (32, 2880, 5760)]:
+        assert nt.rules().mx_tiles(outer, length, inner, True, True, True)[2] == 1
+    assert nt.rules().mx_tiles(2, 2880, 2880, True, True, True)[2] == 0 and nt.rules().mx_tiles(16, 2048, 1093, True, True, False)[2] == 0
+    assert nt.rules().mx_tiles(2, 2880, 5760, False, True, True)[2] == 0 and nt.rules().mx_tiles(4, 2880, 5760, False, True, True)[2] == 1

@@ -868,8 +868,8 @@ PyObject* rule_wide(PyObject* const* v) {
   return PyLong_FromLongLong(wide_block_m(rows, n_slices, K, N, uint32_t(x_bytes), mx8 != 0));
 }
 PyObject* rule_mx_tiles(PyObject* const* v) {
-  const auto [outer, L, inner, e2m1, down] = integers<5>(v);
-  const tk::MxTiles t = tk::mx_tiles(outer, L, inner, e2m1 != 0, down != 0);
+  const auto [outer, L, inner, e2m1, down, rows8] = integers<6>(v);
+  const tk::MxTiles t = tk::mx_tiles(outer, L, inner, e2m1 != 0, down != 0, rows8 != 0);
   return Py_BuildValue("(Lii)", (long long)t.grid, (int)t.blocks, (int)t.once);
 }
 
@@ -932,7 +932,7 @@ PyMethodDef methods[] = {
     METHOD("mxfp4_block_m", rule_mxfp4, 3),
     METHOD("wide_block_m", rule_wide, 6),
     METHOD("wide_block_n", rule_wide_n, 6),
-    METHOD("mx_tiles", rule_mx_tiles, 5),
+    METHOD("mx_tiles", rule_mx_tiles, 6),
     {nullptr, nullptr, 0, nullptr},
 };
 

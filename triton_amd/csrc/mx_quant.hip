@@ -767,7 +767,8 @@ int32_t launch_down(const void* src, int64_t outer, int64_t L, int64_t inner, in
   if constexpr (sizeof(T) == 2) {
     if (inner >= 4 && (reinterpret_cast<uintptr_t>(out_vals) % 16) == 0) {
       typedef TileGeom<KIND> G;
-      const MxTiles t = mx_tiles(outer, L, inner, KIND == TK_E2M1, true);
+      const bool rows8 = inner % 4 == 0 && sa % 4 == 0 && so % 4 == 0 && (reinterpret_cast<uintptr_t>(src) % 8) == 0;
+      const MxTiles t = mx_tiles(outer, L, inner, KIND == TK_E2M1, true, rows8);
       if (t.grid > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_mx_downcast: tensor too large for one launch");
       auto launch = [&](auto kern) {
         hipLaunchKernelGGL(kern, dim3((unsigned)t.grid), dim3(kThreads), 0, st, reinterpret_cast<const uint16_t*>(s), so, sa, L, inner, inner_last, t.col_tiles, t.blk_tiles, ov, os, rounding);
@@ -775,7 +776,7 @@ int32_t launch_down(const void* src, int64_t outer, int64_t L, int64_t inner, in
       if (t.blocks == G::NB)
         launch(t.once ? mx_down_tile<SRC, KIND, true, G::NB> : mx_down_tile<SRC, KIND, false, G::NB>);
       else
-        launch(mx_down_tile<SRC, KIND, false, G::SMALL>);
+        launch(t.once ? mx_down_tile<SRC, KIND, true, G::SMALL> : mx_down_tile<SRC, KIND, false, G::SMALL>);
       return check_launch("mx_down_tile");
     }
   }
@@ -817,7 +818,7 @@ int32_t launch_up(const void* vals, const void* scales, int64_t outer, int64_t L
   if constexpr (sizeof(T) == 2) {
     if (inner >= 4 && (reinterpret_cast<uintptr_t>(vals) % 16) == 0) {
       typedef TileGeom<KIND> G;
-      const MxTiles t = mx_tiles(outer, L, inner, KIND == TK_E2M1, false);
+      const MxTiles t = mx_tiles(outer, L, inner, KIND == TK_E2M1, false, false);
       if (t.grid > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_mx_upcast: tensor too large for one launch");
       hipLaunchKernelGGL((t.blocks == G::NB ? mx_up_tile<KIND, DST, G::NB> : mx_up_tile<KIND, DST, G::SMALL>), dim3((unsigned)t.grid), dim3(kThreads), 0, st, v, s, L, inner, inner_last,
                          t.col_tiles, t.blk_tiles, reinterpret_cast<uint16_t*>(o), oso, osa);

@@ -14,10 +14,17 @@ constexpr int mx_tile_blocks(bool e2m1) { return e2m1 ? 8 : 4; }                
 // 24.5 -> 20.3, 2 x (552) 35.1 -> 32.8, 16 x 2048 x 1024 (512) 30.8 -> 29.3; 8 x 2880 x 2880 (1152) 65.1 -> 66.6, since a column's piece is half a line).
 constexpr int64_t kMxSmallTiles = 1024;
 
-// Sources of this size and more are read with the non-temporal hint, by whole-line tiles.  Two in turn, plain loads / with the hint, us a launch, bf16 [b, 2880, 5760] to e4m3:
-// b 2 (66 MB) 18.1 / 23.8, b 4 47.8 / 39.5, b 8 107 / 75, b 16 181 / 153, b 32 343 / 300; to e2m1: b 2 18.9 / 21.8, b 4 42.6 / 36.8, b 8 95 / 68.  What
-// was used a moment ago is still in the memory-side cache up to about a hundred megabytes, and a read with the hint does not profit from that.
-constexpr int64_t kMxOnceBytes = 96ll << 20;
+// Sources of this size and more are read with the non-temporal hint; to e2m1, whose values are a quarter of the source, from less on where the rows begin at multiples of 8
+// bytes.  What the program wrote or read a moment ago is in the memory-side cache up to about a hundred megabytes, and a read with the hint does not profit from that;
+// what it did not touch lately, as a first call on loaded weights has it, is read faster with the hint.  us a launch, plain loads / with the hint: the same tensor again and
+// again; others in turn; one that the kernel in front has just made.  bf16 to e2m1, small tiles:
+//   8 x 1024 x 1024 (17 MB) 4.7 / 4.7; 7.3 / 6.7; 9.6 / 13.0; 2 x 2880 x 2880 (33 MB) 9.0 / 10.7; 13.7 / 12.4; 11.7 / 12.0; 3 x (50 MB) 13.2 / 13.9; 18.3 / 15.7; 13.6 / 16.6
+//   8 x 2048 x 2048 (67 MB) 15.6 / 18.4; 22.7 / 20.1; 16.5 / 19.1; 2 x 2880 x 5760 (66 MB) 16.6 / 18.8; 22.3 / 19.8; 16.5 / 17.1; 3 x (100 MB) 22.1 / 27.1; 30.3 / 27.6; 21.7 / 27.1
+//   (whole-line tiles with the hint, as all sizes had them once, 33 MB 11.9; 13.6; 14.3; 50 MB 14.1; 15.5; 15.9; 100 MB 28.3; 28.9; 27.4)
+//   rows at any address, 16 x 2048 x 1093 (72 MB) 17.1 / 22.7; 24.4 / 22.7; 17.6 / 23.1
+// To e4m3: 3 x 2880 x 2880 15.5 / 18.1; 21.2 / 18.9; 15.1 / 18.3; 2 x 2880 x 5760 18.9 / 24.8; 26.6 / 24.7; 18.6 / 18.7; 3 x 25.5 / 34.0; 36.3 / 33.8; 24.6 / 32.4; 4 x (133 MB) 35.2 / 43.9;
+//   47.2 / 43.7; 37.2 / 46.6; two in turn: 4 x 47.8 / 39.5, 8 x 107 / 75, 16 x 181 / 153, 32 x 343 / 300.
+constexpr int64_t kMxOnceBytes = 96ll << 20, kMxOnceBytesE2m1 = 36ll << 20;
 
 struct MxTiles {
   int64_t col_tiles, blk_tiles, grid;
@@ -25,13 +32,14 @@ struct MxTiles {
   bool once;       // down: the source is read with the non-temporal hint
 };
 
-inline MxTiles mx_tiles(int64_t outer, int64_t L, int64_t inner, bool e2m1, bool down) {
+// down: a source to be quantised, rows8: its rows begin at multiples of 8 bytes
+inline MxTiles mx_tiles(int64_t outer, int64_t L, int64_t inner, bool e2m1, bool down, bool rows8) {
   const int64_t nblk = L / 32;
   MxTiles t;
   t.col_tiles = (inner + kMxTileCols - 1) / kMxTileCols;
   t.blocks = mx_tile_blocks(e2m1);
-  t.once = down && outer * L * inner * 2 >= kMxOnceBytes;
-  if (!t.once && t.col_tiles * ((nblk + t.blocks - 1) / t.blocks) * outer <= kMxSmallTiles) t.blocks = kMxSmallBlocks;
+  t.once = down && outer * L * inner * 2 >= (e2m1 && rows8 ? kMxOnceBytesE2m1 : kMxOnceBytes);
+  if (t.col_tiles * ((nblk + t.blocks - 1) / t.blocks) * outer <= kMxSmallTiles) t.blocks = kMxSmallBlocks;
   t.blk_tiles = (nblk + t.blocks - 1) / t.blocks;
   t.grid = t.col_tiles * t.blk_tiles * outer;
   return t;
