@@ -377,3 +377,12 @@ def test_sources_to_e2m1_are_read_with_the_hint():
         assert nt.rules().mx_tiles(outer, length, inner, True, True, True)[2] == 1
     assert nt.rules().mx_tiles(2, 2880, 2880, True, True, True)[2] == 0 and nt.rules().mx_tiles(16, 2048, 1093, True, True, False)[2] == 0
     assert nt.rules().mx_tiles(2, 2880, 5760, False, True, True)[2] == 0 and nt.rules().mx_tiles(4, 2880, 5760, False, True, True)[2] == 1
+
+
+def test_small_mx_tiles_up_to_two_whole_line_ones_a_cu_when_expanding():
+    """Beyond, half lines fetched twice cost more than the shorter chain gains; quantising takes them up to four a CU."""
+    from triton_amd import _native as nt
+    blocks = lambda *size: [nt.rules().mx_tiles(*size, True, down, True)[1] for down in (True, False)]
+    assert blocks(2, 2880, 2880) == blocks(8, 2048, 2048) == [4, 4]
+    assert blocks(2, 2880, 5760) == blocks(3, 2880, 5760) == [4, 8]
+    assert blocks(8, 2880, 2880) == [8, 8]

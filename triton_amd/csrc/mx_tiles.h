@@ -9,10 +9,12 @@ constexpr int kMxTileCols = 256;
 constexpr int kMxSmallBlocks = 4;                                                  // blocks of a small tile: one a wave
 constexpr int mx_tile_blocks(bool e2m1) { return e2m1 ? 8 : 4; }                   // ... of one whose columns are whole lines of 128 bytes
 
-// e2m1: small tiles, one block a wave instead of two, where those of whole lines are up to four a CU: both directions are a chain of loads, conversion and stores, and
+// e2m1: small tiles, one block a wave instead of two, where those of whole lines are up to four a CU (up: two): both directions are a chain of loads, conversion and stores, and
 // half of it is shorter (us, both launches: 1 x 2368 x 592 14.6 -> 9.7, 11 x 448 x 256 14.3 -> 9.4, 5 x 544 x 2368 15.9 -> 11.6, 8 x 1024 x 1024 15.3 -> 12.5, 1 x 2880 x 5760 (276 tiles)
 // 24.5 -> 20.3, 2 x (552) 35.1 -> 32.8, 16 x 2048 x 1024 (512) 30.8 -> 29.3; 8 x 2880 x 2880 (1152) 65.1 -> 66.6, since a column's piece is half a line).
-constexpr int64_t kMxSmallTiles = 1024;
+// Up, other tensors in turn, whole-line / small tiles: 2 x 2880 x 2880 (276) 15.1 / 12.2, 3 x (414) 16.7 / 15.0, 8 x 2048 x 2048 (512) 20.8 / 20.5, 2 x 2880 x 5760 (552) 20.5 / 22.1, 3 x
+// (828) 27.0 / 29.3: half lines are fetched twice where nothing of the tensor is in a cache.
+constexpr int64_t kMxSmallTiles = 1024, kMxSmallTilesUp = 512;
 
 // Sources of this size and more are read with the non-temporal hint; to e2m1, whose values are a quarter of the source, from less on where the rows begin at multiples of 8
 // bytes.  What the program wrote or read a moment ago is in the memory-side cache up to about a hundred megabytes, and a read with the hint does not profit from that;
@@ -39,7 +41,7 @@ inline MxTiles mx_tiles(int64_t outer, int64_t L, int64_t inner, bool e2m1, bool
   t.col_tiles = (inner + kMxTileCols - 1) / kMxTileCols;
   t.blocks = mx_tile_blocks(e2m1);
   t.once = down && outer * L * inner * 2 >= (e2m1 && rows8 ? kMxOnceBytesE2m1 : kMxOnceBytes);
-  if (t.col_tiles * ((nblk + t.blocks - 1) / t.blocks) * outer <= kMxSmallTiles) t.blocks = kMxSmallBlocks;
+  if (t.col_tiles * ((nblk + t.blocks - 1) / t.blocks) * outer <= (down ? kMxSmallTiles : kMxSmallTilesUp)) t.blocks = kMxSmallBlocks;
   t.blk_tiles = (nblk + t.blocks - 1) / t.blocks;
   t.grid = t.col_tiles * t.blk_tiles * outer;
   return t;
