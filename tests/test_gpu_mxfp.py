@@ -312,3 +312,14 @@ def test_small_tiles_read_with_the_hint_and_without(device, dtype, shape):
     for i in range(shape[0]):
         qi, si = downcast_to_mxfp(x[i:i + 1].clone(), torch.uint8, axis=1)
         assert torch.equal(q[i:i + 1], qi) and torch.equal(s[i:i + 1], si)
+
+
+@pytest.mark.parametrize("qdt", QTYPES)
+@pytest.mark.parametrize("outer, length, inner", [(1, 32, 4), (2, 160, 257), (3, 96, 255), (1, 288, 1029), (128, 160, 512), (129, 160, 512), (2, 32, 5)])
+def test_expanded_tiles_whose_bytes_are_fetched_together(mx, device, qdt, outer, length, inner):
+    """Both sides of the number of tiles (the two sizes with 512 columns), tiles of one to four blocks, columns and blocks past the last: the oracle's numbers."""
+    x = torch.randn((outer, length, inner), generator=torch.Generator(device=device).manual_seed(inner), device=device).to(torch.bfloat16)
+    q, s = mx.downcast_to_mxfp(x, qdt, axis=1)
+    back = mx.upcast_from_mxfp(q, s, torch.bfloat16, axis=1)
+    _same(omx.upcast_from_mxfp(q[-2:].cpu(), s[-2:].cpu(), torch.bfloat16, axis=1).contiguous(), back[-2:], "dequant")
+    _same(mx.upcast_from_mxfp(q[:1], s[:1], torch.bfloat16, axis=1), back[:1], "dequant of one matrix")

@@ -361,11 +361,10 @@ def test_every_workgroup_of_the_mx_tiles_has_a_block(outer, length, inner, e2m1,
     """The number of workgroups is that of the tiles of the kernel that runs, above all from 96 to 128 MiB, where both the rule for reading once and the
     one for small tensors apply."""
     from triton_amd import _native as nt
-    grid, blocks, once = nt.rules().mx_tiles(outer, length, inner, e2m1, down, inner % 4 == 0)
+    grid, blocks, _ = nt.rules().mx_tiles(outer, length, inner, e2m1, down, inner % 4 == 0)
     cols = -(-inner // 256) * outer
     assert grid % cols == 0 and (grid // cols - 1) * blocks < length // 32 <= grid // cols * blocks
     assert blocks in ((4, 8) if e2m1 else (4, ))
-    assert not once or down
     if e2m1 and (outer, length, inner) == (260, 288, 260):
         assert blocks == 8
 
@@ -386,3 +385,14 @@ def test_small_mx_tiles_up_to_two_whole_line_ones_a_cu_when_expanding():
     assert blocks(2, 2880, 2880) == blocks(8, 2048, 2048) == [4, 4]
     assert blocks(2, 2880, 5760) == blocks(3, 2880, 5760) == [4, 8]
     assert blocks(8, 2880, 2880) == [8, 8]
+
+
+@pytest.mark.parametrize("e2m1", [True, False])
+def test_tiles_of_small_launches_fetch_all_their_bytes_together(e2m1):
+    """Up to two tiles a CU nothing else runs while a tile waits for one piece after the other."""
+    from triton_amd import _native as nt
+    together = lambda *size: nt.rules().mx_tiles(*size, e2m1, False, False)[::2]
+    for size in [(1, 64, 5), (1, 960, 517), (2, 1024, 517), (1, 2880, 517), (8, 1024, 1024)]:
+        assert together(*size)[1] == 1
+    assert together(4, 2048, 2048) == (512, 1) and together(2, 2880, 2880) == (552, 0)
+    assert together(2, 2880, 5760)[1] == 0

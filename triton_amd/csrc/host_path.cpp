@@ -870,7 +870,7 @@ PyObject* rule_wide(PyObject* const* v) {
 PyObject* rule_mx_tiles(PyObject* const* v) {
   const auto [outer, L, inner, e2m1, down, rows8] = integers<6>(v);
   const tk::MxTiles t = tk::mx_tiles(outer, L, inner, e2m1 != 0, down != 0, rows8 != 0);
-  return Py_BuildValue("(Lii)", (long long)t.grid, (int)t.blocks, (int)t.once);
+  return Py_BuildValue("(Lii)", (long long)t.grid, (int)t.blocks, (int)(down ? t.once : t.together));
 }
 
 // bind(dict): the addresses of the entry points (integers) and the Python objects above

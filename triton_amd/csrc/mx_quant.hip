@@ -450,10 +450,11 @@ struct TileGeom {
   static_assert(NB * BB == 128, "a column of a tile is a whole line");
 };
 
-// moves the tile's value bytes and scales between LDS and global memory (TO_GLOBAL) or back
-template <int KIND, int NB, bool TO_GLOBAL>
-__device__ __forceinline__ void tile_move(uint8_t* vals_s, uint8_t* sc_s, uint8_t* gvals, uint8_t* gscales, int64_t o, int64_t col0,
-                                          int64_t blk0, int64_t L, int64_t inner, int64_t inner_last) {
+// The tile's value bytes and scales from LDS to global memory.  Scales: a column's NB bytes are contiguous in both places, so one thread moves them in one piece
+// (4 or 8 bytes at any alignment) unless the tile hangs over the end of the axis; single-byte accesses cost an instruction and a memory transaction each.
+template <int KIND, int NB>
+__device__ __forceinline__ void tile_store(const uint8_t* vals_s, const uint8_t* sc_s, uint8_t* gvals, uint8_t* gscales, int64_t o, int64_t col0,
+                                           int64_t blk0, int64_t L, int64_t inner, int64_t inner_last) {
   constexpr int BB = TileGeom<KIND>::BB, PIECES = NB * BB / 16;  // (of a column)
   const int64_t nblk = L / 32;
   const int64_t line_bytes = KIND == TK_E2M1 ? L / 2 : L;
@@ -464,38 +465,71 @@ __device__ __forceinline__ void tile_move(uint8_t* vals_s, uint8_t* sc_s, uint8_
     const int64_t blk = blk0 + piece * 16 / BB;
     if (col0 + col < inner && blk < nblk) {
       const int64_t line = line_of(o, col0 + col, inner, inner_last);
-      uint4* g = reinterpret_cast<uint4*>(gvals + line * line_bytes + blk0 * BB + piece * 16);
-      uint4* l = reinterpret_cast<uint4*>(vals_s + tile_row(col) * kTilePitch + piece * 16);
-      if (TO_GLOBAL)
-        *g = *l;
-      else
-        *l = *g;
+      *reinterpret_cast<uint4*>(gvals + line * line_bytes + blk0 * BB + piece * 16) = *reinterpret_cast<const uint4*>(vals_s + tile_row(col) * kTilePitch + piece * 16);
     }
   }
-  // scales: a column's NB bytes are contiguous in both places, so one thread moves them in one piece (4 or 8 bytes at
-  // any alignment) unless the tile hangs over the end of the axis; single-byte accesses cost an instruction and a
-  // memory transaction each
   static_assert(kTileCols == kThreads, "one column per thread");
-  {
-    const int col = threadIdx.x;
-    if (col0 + col < inner && blk0 < nblk) {
-      const int64_t line = line_of(o, col0 + col, inner, inner_last);
-      uint8_t* g = gscales + line * nblk + blk0;
-      uint8_t* l = sc_s + col * NB;
-      if (blk0 + NB <= nblk) {
-        if (TO_GLOBAL)
-          __builtin_memcpy(g, l, NB);
-        else
-          __builtin_memcpy(l, g, NB);
-      } else {
-        for (int b = 0; blk0 + b < nblk; ++b) {
-          if (TO_GLOBAL)
-            g[b] = l[b];
-          else
-            l[b] = g[b];
-        }
-      }
+  const int col = threadIdx.x;
+  if (col0 + col < inner && blk0 < nblk) {
+    uint8_t* g = gscales + line_of(o, col0 + col, inner, inner_last) * nblk + blk0;
+    const uint8_t* l = sc_s + col * NB;
+    if (blk0 + NB <= nblk)
+      __builtin_memcpy(g, l, NB);
+    else
+      for (int b = 0; blk0 + b < nblk; ++b) g[b] = l[b];
+  }
+}
+
+// ... and from global memory to LDS.  TOGETHER: everything is requested before any of it is written to LDS, without a condition around a load, whose end would wait for it; a
+// thread past the last column or block fetches that one again, for a place that nobody reads.  One piece after the other a tile is up to nine round trips, which is what a launch
+// of few tiles takes; with many tiles a CU others run meanwhile, and fewer requests at a time serve the memory better (mx_tiles).
+template <int KIND, int NB, bool TOGETHER>
+__device__ __forceinline__ void tile_fetch(uint8_t* vals_s, uint8_t* sc_s, const uint8_t* gvals, const uint8_t* gscales, int64_t o, int64_t col0,
+                                           int64_t blk0, int64_t L, int64_t inner, int64_t inner_last) {
+  constexpr int BB = TileGeom<KIND>::BB, PIECES = NB * BB / 16;
+  const int64_t nblk = L / 32;
+  const int64_t line_bytes = KIND == TK_E2M1 ? L / 2 : L;
+  if constexpr (!TOGETHER) {
+#pragma unroll
+    for (int it = 0; it < PIECES; ++it) {
+      const int q = it * kThreads + threadIdx.x;
+      const int col = q / PIECES, piece = q % PIECES;
+      if (col0 + col < inner && blk0 + piece * 16 / BB < nblk)
+        *reinterpret_cast<uint4*>(vals_s + tile_row(col) * kTilePitch + piece * 16) =
+            *reinterpret_cast<const uint4*>(gvals + line_of(o, col0 + col, inner, inner_last) * line_bytes + blk0 * BB + piece * 16);
     }
+    const int col = threadIdx.x;
+    if (col0 + col < inner) {
+      const uint8_t* g = gscales + line_of(o, col0 + col, inner, inner_last) * nblk + blk0;
+      uint8_t* l = sc_s + col * NB;
+      if (blk0 + NB <= nblk)
+        __builtin_memcpy(l, g, NB);
+      else
+        for (int b = 0; blk0 + b < nblk; ++b) l[b] = g[b];
+    }
+    return;
+  }
+  auto line = [&](int col) __attribute__((always_inline)) { return line_of(o, col0 + col < inner ? col0 + col : inner - 1, inner, inner_last); };
+  uint8_t sc[NB];
+  const uint8_t* gs = gscales + line(threadIdx.x) * nblk;
+  if (blk0 + NB <= nblk) {
+    __builtin_memcpy(sc, gs + blk0, NB);
+  } else {
+#pragma unroll
+    for (int b = 0; b < NB; ++b) sc[b] = gs[blk0 + b < nblk ? blk0 + b : nblk - 1];
+  }
+  uint4 v[PIECES];
+#pragma unroll
+  for (int it = 0; it < PIECES; ++it) {
+    const int q = it * kThreads + threadIdx.x, byte = q % PIECES * 16;
+    const int64_t blk = blk0 + byte / BB;
+    v[it] = *reinterpret_cast<const uint4*>(gvals + line(q / PIECES) * line_bytes + (blk < nblk ? blk : nblk - 1) * BB + byte % BB);
+  }
+  __builtin_memcpy(sc_s + threadIdx.x * NB, sc, NB);
+#pragma unroll
+  for (int it = 0; it < PIECES; ++it) {
+    const int q = it * kThreads + threadIdx.x;
+    *reinterpret_cast<uint4*>(vals_s + tile_row(q / PIECES) * kTilePitch + q % PIECES * 16) = v[it];
   }
 }
 
@@ -643,10 +677,10 @@ __global__ __launch_bounds__(kThreads) void mx_down_tile(const uint16_t* __restr
     quantise_block_to_lds<SRC, KIND, NB>(raw, vals_s, sc_s, c4, b, rounding);
   }
   __syncthreads();
-  tile_move<KIND, NB, true>(vals_s, sc_s, out_vals, out_scales, o, col0, blk0, L, inner, inner_last);
+  tile_store<KIND, NB>(vals_s, sc_s, out_vals, out_scales, o, col0, blk0, L, inner, inner_last);
 }
 
-template <int KIND, int DST, int NB>
+template <int KIND, int DST, int NB, bool TOGETHER>
 __global__ __launch_bounds__(kThreads) void mx_up_tile(const uint8_t* __restrict__ vals, const uint8_t* __restrict__ scales, int64_t L,
                                                        int64_t inner, int64_t inner_last, int64_t col_tiles, int64_t blk_tiles,
                                                        uint16_t* __restrict__ out, int64_t ostride_outer, int64_t ostride_axis) {
@@ -662,7 +696,7 @@ __global__ __launch_bounds__(kThreads) void mx_up_tile(const uint8_t* __restrict
   const int64_t col0 = tile_col0(ct, inner), blk0 = bt * NB;
   const bool live = col0 + lane * 4 < inner;
   const int c4 = tile_cols_of(lane, col0, inner);
-  tile_move<KIND, NB, false>(vals_s, sc_s, const_cast<uint8_t*>(vals), const_cast<uint8_t*>(scales), o, col0, blk0, L, inner, inner_last);
+  tile_fetch<KIND, NB, TOGETHER>(vals_s, sc_s, vals, scales, o, col0, blk0, L, inner, inner_last);
   __syncthreads();
   const float mf = Elem<DST>::max_finite();
 #pragma unroll 1
@@ -820,8 +854,13 @@ int32_t launch_up(const void* vals, const void* scales, int64_t outer, int64_t L
       typedef TileGeom<KIND> G;
       const MxTiles t = mx_tiles(outer, L, inner, KIND == TK_E2M1, false, false);
       if (t.grid > 0x7FFFFFFF) return fail(TK_ERR_UNSUPPORTED, "tk_mx_upcast: tensor too large for one launch");
-      hipLaunchKernelGGL((t.blocks == G::NB ? mx_up_tile<KIND, DST, G::NB> : mx_up_tile<KIND, DST, G::SMALL>), dim3((unsigned)t.grid), dim3(kThreads), 0, st, v, s, L, inner, inner_last,
-                         t.col_tiles, t.blk_tiles, reinterpret_cast<uint16_t*>(o), oso, osa);
+      auto launch = [&](auto kern) {
+        hipLaunchKernelGGL(kern, dim3((unsigned)t.grid), dim3(kThreads), 0, st, v, s, L, inner, inner_last, t.col_tiles, t.blk_tiles, reinterpret_cast<uint16_t*>(o), oso, osa);
+      };
+      if (t.blocks == G::SMALL)
+        launch(t.together ? mx_up_tile<KIND, DST, G::SMALL, true> : mx_up_tile<KIND, DST, G::SMALL, false>);
+      else
+        launch(mx_up_tile<KIND, DST, G::NB, false>);
       return check_launch("mx_up_tile");
     }
   }

@@ -28,10 +28,18 @@ constexpr int64_t kMxSmallTiles = 1024, kMxSmallTilesUp = 512;
 //   47.2 / 43.7; 37.2 / 46.6; two in turn: 4 x 47.8 / 39.5, 8 x 107 / 75, 16 x 181 / 153, 32 x 343 / 300.
 constexpr int64_t kMxOnceBytes = 96ll << 20, kMxOnceBytesE2m1 = 36ll << 20;
 
+// Up: a tile's bytes requested together up to this many (small) tiles, two a CU.  us, one piece after the other / together, the same tensor again and again; others in turn:
+//   from e2m1: 960 x 517 (24 tiles) 4.1 / 3.8; 5.2 / 4.3; 2 x 1024 x 517 (48) 4.4 / 4.0; 6.2 / 4.7; 8 x 1024 x 1024 (256) 6.2 / 5.9; 8.7 / 7.3; 4 x 2048 x 2048 (512) 9.9 / 9.3; 11.7 / 11.2;
+//   2 x 2880 x 2880 (552) 10.5 / 10.9; 12.2 / 13.2; 3 x (828) 13.6 / 14.2; 15.1 / 17.1
+//   from e4m3: 960 x 517 5.0 / 4.5; 6.8 / 4.9; 2 x 1024 x 517 5.3 / 4.7; 8.9 / 5.8 (7.2 by a column a lane, which calls of that kind took once); 2880 x 517 (69) 5.7 / 5.0; 9.6 / 6.6 (7.9);
+//   8 x 1024 x 1024 7.0 / 6.3; 11.3 / 8.7; 4 x 2048 x 2048 11.6 / 10.3; 15.8 / 14.4; 2 x 2880 x 2880 12.1 / 11.4; 15.1 / 16.9; 8 x 2048 x 2048 (1024) 21.7 / 20.0; 25.9 / 28.4
+constexpr int64_t kMxTogether = 512;
+
 struct MxTiles {
   int64_t col_tiles, blk_tiles, grid;
   int32_t blocks;  // of 32, in a tile
   bool once;       // down: the source is read with the non-temporal hint
+  bool together;   // up: a tile's bytes are requested together
 };
 
 // down: a source to be quantised, rows8: its rows begin at multiples of 8 bytes
@@ -44,6 +52,7 @@ inline MxTiles mx_tiles(int64_t outer, int64_t L, int64_t inner, bool e2m1, bool
   if (t.col_tiles * ((nblk + t.blocks - 1) / t.blocks) * outer <= (down ? kMxSmallTiles : kMxSmallTilesUp)) t.blocks = kMxSmallBlocks;
   t.blk_tiles = (nblk + t.blocks - 1) / t.blocks;
   t.grid = t.col_tiles * t.blk_tiles * outer;
+  t.together = !down && t.blocks == kMxSmallBlocks && t.grid <= kMxTogether;
   return t;
 }
 
