@@ -323,3 +323,20 @@ def test_expanded_tiles_whose_bytes_are_fetched_together(mx, device, qdt, outer,
     back = mx.upcast_from_mxfp(q, s, torch.bfloat16, axis=1)
     _same(omx.upcast_from_mxfp(q[-2:].cpu(), s[-2:].cpu(), torch.bfloat16, axis=1).contiguous(), back[-2:], "dequant")
     _same(mx.upcast_from_mxfp(q[:1], s[:1], torch.bfloat16, axis=1), back[:1], "dequant of one matrix")
+
+
+@pytest.mark.parametrize("qdt", QTYPES)
+@pytest.mark.parametrize("outer, length, inner", [(40, 96, 261), (80, 64, 5), (36, 160, 141)])
+def test_rows_at_any_address_by_tiles_and_by_columns(mx, device, qdt, outer, length, inner):
+    """An odd number of columns: the whole tensor by tiles, a few of its matrices by a column a lane, the same bytes, and the oracle's."""
+    from triton_amd import _native as nt
+    assert not nt.rules().mx_by_columns(outer, length, inner) and nt.rules().mx_by_columns(4, length, inner)
+    x = torch.randn((outer, length, inner), generator=torch.Generator(device=device).manual_seed(inner), device=device).to(torch.bfloat16)
+    x[1, 3, 2], x[2, 40, 1], x[3, :32, 0] = 30000.0, -0.0, 0.0
+    q, s = mx.downcast_to_mxfp(x, qdt, axis=1)
+    qi, si = mx.downcast_to_mxfp(x[:4].clone(), qdt, axis=1)
+    _same(qi, q[:4], "values")
+    _same(si, s[:4], "scales")
+    qo, so = omx.downcast_to_mxfp(x[:4].cpu(), qdt, axis=1)
+    _same(qo, q[:4], "values")
+    _same(so, s[:4], "scales")

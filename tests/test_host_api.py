@@ -396,3 +396,13 @@ def test_tiles_of_small_launches_fetch_all_their_bytes_together(e2m1):
         assert together(*size)[1] == 1
     assert together(4, 2048, 2048) == (512, 1) and together(2, 2880, 2880) == (552, 0)
     assert together(2, 2880, 5760)[1] == 0
+
+
+def test_small_sources_with_rows_at_any_address_are_quantised_by_columns():
+    """Up to 70 tiles, whose longer chain is all that there is to see, except where the last columns are few."""
+    from triton_amd import _native as nt
+    by = nt.rules().mx_by_columns
+    for size in [(1, 64, 33), (1, 480, 1093), (1, 960, 517), (1, 960, 1093), (2, 1024, 517), (1, 2880, 517), (1, 512, 2049), (1, 960, 577), (1, 2880, 261)]:
+        assert by(*size), size
+    for size in [(1, 2880, 1093), (4, 960, 517), (6, 1632, 1093), (1, 480, 65), (1, 960, 193), (1, 480, 897)]:
+        assert not by(*size), size

@@ -872,6 +872,10 @@ PyObject* rule_mx_tiles(PyObject* const* v) {
   const tk::MxTiles t = tk::mx_tiles(outer, L, inner, e2m1 != 0, down != 0, rows8 != 0);
   return Py_BuildValue("(Lii)", (long long)t.grid, (int)t.blocks, (int)(down ? t.once : t.together));
 }
+PyObject* rule_mx_by_columns(PyObject* const* v) {
+  const auto [outer, L, inner] = integers<3>(v);
+  return PyBool_FromLong(tk::mx_by_columns(outer, L, inner));
+}
 
 // bind(dict): the addresses of the entry points (integers) and the Python objects above
 PyObject* bind(PyObject*, PyObject* dict) {
@@ -933,6 +937,7 @@ PyMethodDef methods[] = {
     METHOD("wide_block_m", rule_wide, 6),
     METHOD("wide_block_n", rule_wide_n, 6),
     METHOD("mx_tiles", rule_mx_tiles, 6),
+    METHOD("mx_by_columns", rule_mx_by_columns, 3),
     {nullptr, nullptr, 0, nullptr},
 };
 

@@ -7,7 +7,8 @@
 //          quantised along K); a lane owns one or two columns and walks 32 rows, so every load of a
 //          wave is one contiguous row segment and the 32-element reduction is register-local.
 //   tile : the cols case for 16-bit tensors of four columns and more, with an LDS transpose so that the quantised
-//          bytes of a column move as full 128-byte lines (mx_down_tile / mx_up_tile).
+//          bytes of a column move as full 128-byte lines (mx_down_tile / mx_up_tile); small sources with rows at any
+//          address stay with the cols kernel (mx_by_columns).
 #include "mx_math.h"
 #include "mx_tiles.h"
 
@@ -798,8 +799,10 @@ int32_t launch_down(const void* src, int64_t outer, int64_t L, int64_t inner, in
   }
   if (si != 1 && inner != 1) return fail(TK_ERR_UNSUPPORTED, "tk_mx_downcast: inner stride must be 1");
   const int64_t nblk = L / 32;
+  const size_t esz = sizeof(T);
+  const bool pair_ok = inner % 2 == 0 && sa % 2 == 0 && so % 2 == 0 && (reinterpret_cast<uintptr_t>(src) % (2 * esz)) == 0;
   if constexpr (sizeof(T) == 2) {
-    if (inner >= 4 && (reinterpret_cast<uintptr_t>(out_vals) % 16) == 0) {
+    if (inner >= 4 && (reinterpret_cast<uintptr_t>(out_vals) % 16) == 0 && (pair_ok || !mx_by_columns(outer, L, inner))) {
       typedef TileGeom<KIND> G;
       const bool rows8 = inner % 4 == 0 && sa % 4 == 0 && so % 4 == 0 && (reinterpret_cast<uintptr_t>(src) % 8) == 0;
       const MxTiles t = mx_tiles(outer, L, inner, KIND == TK_E2M1, true, rows8);
@@ -815,8 +818,6 @@ int32_t launch_down(const void* src, int64_t outer, int64_t L, int64_t inner, in
     }
   }
   const int64_t blk_tiles = cdiv(nblk, 4);
-  const size_t esz = sizeof(T);
-  const bool pair_ok = inner % 2 == 0 && sa % 2 == 0 && so % 2 == 0 && (reinterpret_cast<uintptr_t>(src) % (2 * esz)) == 0;
   if (pair_ok) {
     const int64_t col_tiles = cdiv(inner, 128);
     const int64_t grid = col_tiles * blk_tiles * outer;

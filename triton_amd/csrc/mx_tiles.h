@@ -56,4 +56,16 @@ inline MxTiles mx_tiles(int64_t outer, int64_t L, int64_t inner, bool e2m1, bool
   return t;
 }
 
+// Whether a source whose rows begin at any address (an odd number of columns, say) is quantised by a column a lane instead: up to some 70 tiles that kernel's shorter chain is the
+// faster one.  us, bf16, by tiles / by columns, the same tensor again and again; others in turn: to e2m1, 480 x 1093 (20 tiles) 5.0 / 4.4 (others), 960 x 517 (24) 5.9 / 3.8; 6.0 / 4.4, 960 x 1093
+// (40) 4.5 / 3.8; 5.5 / 5.2, 2 x 1024 x 517 (48) 5.7 / 4.0; 6.0 / 5.0, 2880 x 517 (69) 5.6 / 4.3; 6.4 / 6.0, 480 x 4097 (68) 4.6 / 4.4; 6.3 / 6.4, 4 x 960 x 517 (96) 4.6 / 5.1; 6.3 / 6.7, 2880 x 1093 (115) 4.8 /
+// 4.8; 6.8 / 7.3; to e4m3, 960 x 517 6.1 / 4.0; 6.2 / 4.6, 4 x 960 x 517 5.2 / 4.8; 7.0 / 6.9, 2880 x 1093 5.6 / 5.6; 7.5 / 7.6.
+// Except where the last of its 64 columns are one to eight and the launch is small, which then takes 5.5 to 6.5 (a tile with as few columns takes as long): 480 x 65 4.1 / 5.8, 960 x 193 4.5 / 6.1, 480 x 897
+// (60 workgroups) 5.0 / 5.4, 960 x 577 (80) 5.0 / 4.4.
+inline bool mx_by_columns(int64_t outer, int64_t L, int64_t inner) {
+  const int64_t quads = (L / 32 + 3) / 4 * outer, last = inner % 64;
+  if ((inner + kMxTileCols - 1) / kMxTileCols * quads > 70) return false;
+  return !(last >= 1 && last <= 8 && inner % kMxTileCols > 8 && (inner + 63) / 64 * quads < 64);
+}
+
 }  // namespace tk
