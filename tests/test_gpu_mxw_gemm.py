@@ -199,3 +199,21 @@ def test_scales_at_any_byte(device, e, k, n, sizes, offset, pad):
     view.copy_(scale)
     got = run(view)
     assert torch.equal(got, want) and not torch.isnan(got).any()
+
+
+@pytest.mark.parametrize("e, k, n, sizes", [(16, 1792, 2048, [81, 104, 97, 90]), (8, 544, 1056, [96, 128, 64, 100, 33, 129, 90, 95])])
+def test_mxfp8_rows_without_a_wide_tile(device, e, k, n, sizes):
+    """81 to 104 rows a slice where the tiles of 128 x 256 are one round: they run, and give what the wide kernel's 160 x 512 give, bit for bit."""
+    import triton_amd._native as nt
+    import triton_amd.matmul as mm
+    from triton_amd.swiglu import swiglu_fn
+    c = _case(device, k, n, [sizes[i % len(sizes)] for i in range(e)], True)
+    assert 80 * e < c["m"] <= 104 * e
+    assert nt.rules().wide_block_n(c["m"], e, k, n, c["m"] * k, 1) == 0 and nt.rules().wide_block_m(c["m"], e, k, n, c["m"] * k, 1) == 128
+    act = mm.FusedActivation(mm.FnSpecs("swiglu", swiglu_fn, ("alpha", "limit"), reduction_n=2), (1.702, 7.0))
+    pc = mm.PrecisionConfig(b_mx_scale=c["s_dev"], a_mx_scale=c["xs"].to(device), out_dtype=torch.bfloat16)
+    args = dict(gather_indx=c["gi"].to(device), scatter_indx=c["sc"].to(device), gammas=c["gam"].to(device), precision_config=pc, fused_activation=act)
+    out = mm.matmul(c["xq"].to(device), c["w_dev"], c["bias"].to(device), c["md"], **args)
+    with mm.scoped_opt_flags_constraints({"block_m": 256}):
+        wide = mm.matmul(c["xq"].to(device), c["w_dev"], c["bias"].to(device), c["md"], **args)
+    assert torch.equal(out, wide) and out.any()

@@ -406,3 +406,18 @@ def test_small_sources_with_rows_at_any_address_are_quantised_by_columns():
         assert by(*size), size
     for size in [(1, 2880, 1093), (4, 960, 517), (6, 1632, 1093), (1, 480, 65), (1, 960, 193), (1, 480, 897)]:
         assert not by(*size), size
+
+
+def test_mxfp8_row_blocks_of_256_only_where_the_wide_kernel_has_a_tile():
+    """A row block of 256 without columns is that kernel's largest tile; where the rules name none of its tiles the other kernel runs, whose row blocks are 128."""
+    from triton_amd import _native as nt
+    rules, without = nt.rules(), 0
+    for n_slices in (1, 2, 8, 16, 32, 64, 128):
+        for K in (512, 960, 1792, 2880):
+            for N in (256, 960, 2048, 2880, 5760):
+                for per_slice in (1, 24, 40, 64, 80, 81, 90, 96, 97, 104, 105, 122, 152, 176, 300, 640, 1000):
+                    rows = per_slice * n_slices
+                    if not rules.wide_block_n(rows, n_slices, K, N, rows * K, 1):
+                        without += 1
+                        assert rules.wide_block_m(rows, n_slices, K, N, rows * K, 1) == 128, (n_slices, K, N, per_slice)
+    assert without > 100
