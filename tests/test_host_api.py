@@ -421,3 +421,13 @@ def test_mxfp8_row_blocks_of_256_only_where_the_wide_kernel_has_a_tile():
                         without += 1
                         assert rules.wide_block_m(rows, n_slices, K, N, rows * K, 1) == 128, (n_slices, K, N, per_slice)
     assert without > 100
+
+
+def test_decode_layers_up_to_16_tokens_read_the_weights_with_the_hint():
+    """Read once by the whole grid, whatever their size: another layer's weights come in between.  Beyond 16 tokens plain loads (0), or as the routing has it (2)."""
+    from triton_amd import _native as nt
+    blocks = lambda d, f: (2 * f // 32) * -(-d // 128) + (d // 32) * -(-f // 128)
+    for T in (1, 10, 16):
+        for E, k, d in [(16, 4, 2048), (8, 4, 2880), (32, 8, 1024), (64, 8, 768), (128, 4, 2880)]:
+            assert nt.rules().decode_fetch(T, k, E, blocks(d, d)) == 1
+    assert nt.rules().decode_fetch(17, 4, 16, blocks(2048, 2048)) == 0 and nt.rules().decode_fetch(17, 4, 128, blocks(2880, 2880)) == 2

@@ -200,4 +200,20 @@ inline bool decode_by_rows(int64_t T, int64_t k, int64_t d_ff, int64_t d_model) 
   return k <= kDecRowsMaxK && T * k <= kRowsMax && T * k * (expert_bytes + kRowBytes) + T * parts(d_model, 16) * kWorkgroupBytes <= kRowsBytes;
 }
 
+// How a decode layer in a single launch fetches the weights.  Up to 16 tokens no expert has a second row block (a token's k experts differ): they are read once by the whole grid,
+// with the non-temporal hint, which is the faster way wherever other layers run in between (us, plain loads / with the hint, the same weights again and again; other weights
+// each call: 16 tokens, 16 experts, top 4, 2048 36.3 / 36.2; 38.7 / 37.4; 16, 8, top 4, 2880 37.4 / 38.6; 40.4 / 39.8; 10, 8, top 8, 2880 39.8 / 40.8; 42.6 / 41.9; 16, 32, top 8, 1024 31.7 / 30.9; 32.5 / 32.1;
+// 16, 64, top 8, 768 33.3 / 33.3; 34.1 / 33.5).  Beyond, the later row blocks of an expert find a fragment in the caches that the hint would take away: up to kLargeBlocks, plain loads; where there
+// may be more than the caches keep for the next call anyway, the kernel decides, which knows the blocks after its routing: hardly any second ones, all with the hint; up to a third, by unit
+// (whole K of 24 stages only: the branch costs the compiler's wait counts, a drained ring a unit, which shorter units feel more than they gain).  Three
+// copies of the loop are code to be fetched (0.8 us a call), so the host rules out what cannot be.
+// us, 128 experts, top 4, 2880, without and with: no second blocks, 17 tokens 143 / 130, 32 215 / 192, 64 291 / 260; with favourites, 32 tokens (27.6 blocks of
+// 25.7 experts) 90.5 / 83.6, 40 (32.8 of 30.4) 96.5 / 93.0, by unit 89.5, 61 (39.9 of 33.9) 117.2 / 119.1, by unit 111.5; 33 tokens, 96 experts, 768 and 1824, favourites, 100 MB 37.9 / 40.5.
+enum { kFetchPlain, kFetchOnce, kFetchEither };
+constexpr int kLargeBlocks = (128 << 20) / 2176;  // blocks of 32 columns x 128 k, values and scales
+inline int decode_fetch(int64_t T, int64_t k, int64_t E, int64_t blocks_of_expert) {
+  if (T <= 16) return kFetchOnce;
+  return (T * k < E ? T * k : E) * blocks_of_expert <= kLargeBlocks ? kFetchPlain : kFetchEither;
+}
+
 }  // namespace tk

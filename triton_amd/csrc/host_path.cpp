@@ -853,6 +853,10 @@ PyObject* rule_decode_rows(PyObject* const* v) {
   const auto [T, k, d_ff, d_model] = integers<4>(v);
   return PyBool_FromLong(tk::decode_by_rows(T, k, d_ff, d_model));
 }
+PyObject* rule_decode_fetch(PyObject* const* v) {
+  const auto [T, k, E, blocks_of_expert] = integers<4>(v);
+  return PyLong_FromLong(tk::decode_fetch(T, k, E, blocks_of_expert));
+}
 PyObject* rule_fp8(PyObject* const* v) {
   const auto [rows, x_bytes, K, N, n_slices] = integers<5>(v);
   return PyLong_FromLongLong(fp8_block_m(rows, uint32_t(x_bytes), K, N, n_slices));
@@ -934,6 +938,7 @@ PyMethodDef methods[] = {
     METHOD("dma_block_n_16bit", rule_dma_n_16bit, 4),
     METHOD("few_block_n", rule_few, 3),
     METHOD("decode_by_rows", rule_decode_rows, 4),
+    METHOD("decode_fetch", rule_decode_fetch, 4),
     METHOD("fp8_block_m", rule_fp8, 5),
     METHOD("mxfp4_block_m", rule_mxfp4, 3),
     METHOD("wide_block_m", rule_wide, 6),

@@ -80,15 +80,6 @@ __device__ __forceinline__ float quad_swap(float x) {
 
 constexpr int kNonTemporalLoad = 2;
 
-// How the weights are fetched.  With the non-temporal hint where they are read once by the whole grid and more than the caches keep for the next call
-// anyway; the later row blocks of an expert find a fragment in the caches that the hint would take away.  Up to 16 tokens no expert has a second block (a
-// token's k experts differ); beyond, the kernel knows the blocks after its routing: hardly any second ones, all with the hint; up to a third, by unit
-// (whole K of 24 stages only: the branch costs the compiler's wait counts, a drained ring a unit, which shorter units feel more than they gain).  Three
-// copies of the loop are code to be fetched (0.8 us a call), so the host rules out what cannot be.
-// us, 128 experts, top 4, 2880, without and with: no second blocks, 17 tokens 143 / 130, 32 215 / 192, 64 291 / 260; with favourites, 32 tokens (27.6 blocks of
-// 25.7 experts) 90.5 / 83.6, 40 (32.8 of 30.4) 96.5 / 93.0, by unit 89.5, 61 (39.9 of 33.9) 117.2 / 119.1, by unit 111.5; 33 tokens, 96 experts, 768 and 1824, favourites, 100 MB 37.9 / 40.5.
-enum { kFetchPlain, kFetchOnce, kFetchEither };
-constexpr int kLargeBlocks = (128 << 20) / 2176;  // blocks of 32 columns x 128 k, values and scales
 constexpr int kThrough = 1 | 16;  // aux bits of the buffer instructions: sc0 | sc1 (write through / read around the L2)
 
 template <int VPL, int XS_, int FPU_, int FETCH>
@@ -779,9 +770,9 @@ int32_t launch_layer(const DecodeParams& p, hipStream_t st) {
 
 template <int VPL>
 int32_t launch_layer(const DecodeParams& p, hipStream_t st) {
-  const int R = p.T * p.k;
-  if ((int64_t)(R < p.E ? R : p.E) * (p.nfr1 * p.nst1 + p.nfr2 * p.nst2) <= kLargeBlocks) return launch_layer<VPL, kFetchPlain>(p, st);
-  return p.T <= 16 ? launch_layer<VPL, kFetchOnce>(p, st) : launch_layer<VPL, kFetchEither>(p, st);
+  const int fetch = decode_fetch(p.T, p.k, p.E, p.nfr1 * p.nst1 + p.nfr2 * p.nst2);
+  if (fetch == kFetchPlain) return launch_layer<VPL, kFetchPlain>(p, st);
+  return fetch == kFetchOnce ? launch_layer<VPL, kFetchOnce>(p, st) : launch_layer<VPL, kFetchEither>(p, st);
 }
 
 }  // namespace
