@@ -206,7 +206,7 @@ inline bool decode_by_rows(int64_t T, int64_t k, int64_t d_ff, int64_t d_model) 
 // 16, 64, top 8, 768 33.3 / 33.3; 34.1 / 33.5).  Beyond, the later row blocks of an expert find a fragment in the caches that the hint would take away: up to kLargeBlocks, plain loads; where there
 // may be more than the caches keep for the next call anyway, the kernel decides, which knows the blocks after its routing: hardly any second ones, all with the hint; up to a third, by unit
 // (whole K of 24 stages only: the branch costs the compiler's wait counts, a drained ring a unit, which shorter units feel more than they gain).  Three
-// copies of the loop are code to be fetched (0.8 us a call), so the host rules out what cannot be.
+// copies of the loop are code to be fetched (0.8 us a call for those behind the first), so the host rules out what cannot be.
 // us, 128 experts, top 4, 2880, without and with: no second blocks, 17 tokens 143 / 130, 32 215 / 192, 64 291 / 260; with favourites, 32 tokens (27.6 blocks of
 // 25.7 experts) 90.5 / 83.6, 40 (32.8 of 30.4) 96.5 / 93.0, by unit 89.5, 61 (39.9 of 33.9) 117.2 / 119.1, by unit 111.5; 33 tokens, 96 experts, 768 and 1824, favourites, 100 MB 37.9 / 40.5.
 enum { kFetchPlain, kFetchOnce, kFetchEither };
