@@ -188,3 +188,25 @@ def test_short_slices_rows_of_broken_lines(device, m, n, beside, out_dtype):
     ref = omoe.matmul_ragged_k(a.t(), b, sizes, offs, offs, out_dtype=torch.float32)
     assert_allclose_gate(ref, out[:, :m, :n].float(), what="ragged-K matmul")
     assert torch.isnan(out[:, m:]).all() and torch.isnan(out[:, :, n:]).all()
+
+
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float16, torch.float32], ids=["bf16", "fp16", "fp32"])
+@pytest.mark.parametrize("n_slices, m, n, rest, tile", [(12, 264, 1032, 300, 128), (128, 520, 776, 170, 256)])
+def test_long_slices_of_fp16(device, n_slices, m, n, rest, tile, out_dtype):
+    """fp16 operands by either tile of the kernel for long slices.  A sum of at most 900 products of values below 5 in size: far inside fp16's range, and
+    its order's error (2^-24 a term) far below the gate."""
+    import triton_amd._native as nt
+    import triton_amd.matmul as mm
+    g = torch.Generator().manual_seed(n_slices + n)
+    sizes = torch.full((n_slices, ), rest, dtype=torch.int32)
+    for i, s in enumerate([0, 1, 31, 33, 64, 97, 129, 3 * rest]):
+        sizes[(i * 5) % n_slices] = s
+    offs = _offsets(sizes, 8)
+    k = max(int(offs[-1]), 160 * n_slices + 8)
+    assert nt.rules().ragged_k_tile(k // n_slices, m, n, n_slices) == tile
+    a, b = torch.randn((k, m), generator=g).to(torch.float16), torch.randn((k, n), generator=g).to(torch.float16)
+    out = torch.full((n_slices, m, n), float("nan"), dtype=out_dtype, device=device)
+    md = _metadata(sizes, offs, device)
+    mm.matmul(a.to(device).t(), b.to(device), None, a_ragged_metadata=md, b_ragged_metadata=md, c=out, precision_config=mm.PrecisionConfig(out_dtype=out_dtype))
+    ref = omoe.matmul_ragged_k(a.t(), b, sizes, offs, offs, out_dtype=torch.float32)
+    assert_allclose_gate(ref, out.float(), what="ragged-K matmul")

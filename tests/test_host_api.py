@@ -431,3 +431,15 @@ def test_decode_layers_up_to_16_tokens_read_the_weights_with_the_hint():
         for E, k, d in [(16, 4, 2048), (8, 4, 2880), (32, 8, 1024), (64, 8, 768), (128, 4, 2880)]:
             assert nt.rules().decode_fetch(T, k, E, blocks(d, d)) == 1
     assert nt.rules().decode_fetch(17, 4, 16, blocks(2048, 2048)) == 0 and nt.rules().decode_fetch(17, 4, 128, blocks(2880, 2880)) == 2
+
+
+@pytest.mark.parametrize("k, m, n, n_slices, tile", [
+    # the sizes that test_gpu_ragged_k.py runs by each kernel
+    (160, 264, 1032, 12, 128), (160, 8, 136, 9, 128), (160, 520, 264, 128, 128), (160, 264, 520, 1, 128), (160, 520, 776, 128, 256), (160, 264, 264, 129, 0), (159, 264, 1032, 12, 0),
+    # from 90 k on: rounds, and what hangs over the edges
+    (128, 2880, 5760, 128, 256), (128, 2880, 2880, 128, 0), (128, 2880, 5760, 32, 256), (128, 2880, 5760, 16, 0), (93, 2880, 5760, 64, 256), (89, 2880, 5760, 128, 0), (128, 1600, 2400, 128, 0),
+    (256, 2880, 5760, 8, 256), (2048, 512, 1024, 8, 128)])
+def test_tile_of_a_ragged_k_gemm(k, m, n, n_slices, tile):
+    """Both sides of each line: k a slice, rounds of tiles, their overhang, the slices that the kernel for long ones keeps."""
+    from triton_amd import _native as nt
+    assert nt.rules().ragged_k_tile(k, m, n, n_slices) == tile

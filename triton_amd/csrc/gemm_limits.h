@@ -1,7 +1,7 @@
 // What a call has to be like for the expert-GEMM kernels that address x through one buffer resource.  Plain C++: the entry point
 // (moe_gemm.hip) picks the kernel by it and the host path (host_path.cpp, for both of its callers) the row blocks, so that row
 // blocks which only such a kernel has are never chosen for a call that it cannot run.  And how a decode layer is launched: its entry
-// point (moe_decode_layer.hip) and those who make its workspace go by the same rule.
+// point (moe_decode_layer.hip) and those who make its workspace go by the same rule.  And the tile of a ragged-K GEMM.
 #pragma once
 #include <math.h>
 #include <stdint.h>
@@ -214,6 +214,28 @@ constexpr int kLargeBlocks = (128 << 20) / 2176;  // blocks of 32 columns x 128 
 inline int decode_fetch(int64_t T, int64_t k, int64_t E, int64_t blocks_of_expert) {
   if (T <= 16) return kFetchOnce;
   return (T * k < E ? T * k : E) * blocks_of_expert <= kLargeBlocks ? kFetchPlain : kFetchEither;
+}
+
+// Tile of the ragged-K kernel for long slices (ragged_k_long.hip) for aligned operands, `k` a slice; 0 = the one for short slices, whose four small workgroups a CU write best where
+// writing is what takes the time.
+//   * From 160 k a slice on 256 x 256 where they are four rounds over the 256 CUs; with fewer, 128 x 128, which start sooner.
+//   * From 90 k on 256 x 256 or nothing: where they are 24 rounds (below: 16 slices of 128, 2880, 17 rounds for the larger product, lose; 32, 34 rounds, gain) and
+//     an eighth of their area at most hangs over the edges (1600 x 2400, a fifth, loses).  2880 x 2880 and 1440 x 2880, 0.138, are beyond that line, so of the layers of 2880 with 90 to 160 k only the
+//     product of 2880 x 5760 (0.094) is this kernel's, and neither of those of 1440: the table's columns are both products by one kernel (128 slices of 128, 2880: by this rule 1642).
+// Measured (us of both products [d, 2 f] and [f, d] of a layer with slices of random lengths; short / 128 / 256):
+//   slices, k of one, d, f: 8, 2048, 2880, 2880 936 / 916 / 827; 8, 256, 2880, 2880 162 / 163 / 155; 16, 1024, 2048, 2048 498 / 491 / 423; 16, 375, 1600, 1200 121 / 110 / 110
+//   32, 512, 2880, 2880 1069 / 1104 / 935; 32, 187, 2880, 2880 477 / 512 / 464; 32, 187, 1600, 1200 135 / 132 / 135; 64, 256, 1024, 1024 168 / 172 / 146; 64, 256, 2880, 2880 1309 / 1357 / 1149
+//   8, 2048, 512, 512 132 / 85 / 192; 8, 256, 512, 512 26 / 21 / 40; 8, 2048, 1024, 1024 162 / 134 / 210; 8, 750, 800, 1024 71 / 55 / 87; 16, 375, 320, 448 39 / 30 / 54; 16, 256,
+//   1024, 1024 60 / 47 / 55; 32, 187, 320, 448 35 / 30 / 48; 32, 187, 800, 1024 77 / 69 / 73; 64, 256, 320, 448 50 / 47 / 54
+//   128, 128, 2880, 2880 1742 / 1903 / 1623; 128, 128, 1440, 1440 456 / 472 / 421; 64, 93, 2880, 2880 706 / 733 / 681; 32, 128, 2880, 2880 407 / 418 / 396; 16, 128, 2880, 2880 202 / 223 / 208
+//   128, 128, 1600, 1200 404 / 438 / 411; 64, 93, 1600, 1200 184 / 196 / 197; 64, 125, 1440, 1440 226 / 242 / 231; 8, 128, 512, 512 15 / 14 / 23; 128, 128, 512, 512 76 / 82 / 76; 128, 46, 2880,
+//   2880 1171 / 1275 / 1221; 16, 64, 1600, 1200 25 / 29 / 30
+constexpr int kRaggedKLongSlices = 128;  // slices that the kernel for long ones keeps in registers
+inline int ragged_k_tile(int64_t k, int64_t M, int64_t N, int64_t n_slices) {
+  if (n_slices > kRaggedKLongSlices) return 0;
+  const int64_t tiles = (M + 255) / 256 * ((N + 255) / 256) * n_slices;
+  if (k >= 160) return tiles >= 4 * 256 ? 256 : 128;
+  return k >= 90 && tiles >= 24 * 256 && tiles * 256 * 256 * 8 <= M * N * n_slices * 9 ? 256 : 0;
 }
 
 }  // namespace tk

@@ -873,6 +873,10 @@ PyObject* rule_wide(PyObject* const* v) {
   const auto [rows, n_slices, K, N, x_bytes, mx8] = integers<6>(v);
   return PyLong_FromLongLong(wide_block_m(rows, n_slices, K, N, uint32_t(x_bytes), mx8 != 0));
 }
+PyObject* rule_ragged_k_tile(PyObject* const* v) {
+  const auto [k, M, N, n_slices] = integers<4>(v);
+  return PyLong_FromLong(tk::ragged_k_tile(k, M, N, n_slices));
+}
 PyObject* rule_mx_tiles(PyObject* const* v) {
   const auto [outer, L, inner, e2m1, down, rows8] = integers<6>(v);
   const tk::MxTiles t = tk::mx_tiles(outer, L, inner, e2m1 != 0, down != 0, rows8 != 0);
@@ -943,6 +947,7 @@ PyMethodDef methods[] = {
     METHOD("mxfp4_block_m", rule_mxfp4, 3),
     METHOD("wide_block_m", rule_wide, 6),
     METHOD("wide_block_n", rule_wide_n, 6),
+    METHOD("ragged_k_tile", rule_ragged_k_tile, 4),
     METHOD("mx_tiles", rule_mx_tiles, 6),
     METHOD("mx_by_columns", rule_mx_by_columns, 3),
     {nullptr, nullptr, 0, nullptr},

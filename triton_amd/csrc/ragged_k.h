@@ -1,6 +1,7 @@
 // Shared by the ragged-K kernels (ragged_k_gemm.hip: any layout, and aligned operands of short slices; ragged_k_long.hip: aligned operands of long ones).
 #pragma once
 #include "gemm_common.h"
+#include "gemm_limits.h"
 
 namespace tk {
 
@@ -22,8 +23,6 @@ struct RaggedKParams {
   uint32_t a_bytes, b_bytes, y_bytes;  // extents for the buffer resources of the aligned variants (y: one slice)
   int a_vec, b_vec;  // the operand's base and strides allow 16-byte loads along its contiguous dimension
 };
-
-constexpr int kRaggedKLongSlices = 128;  // slices that the kernel for long ones keeps in registers
 
 // Aligned operands (as in tk_ragged_k_gemm), long slices; `tile` = 256 or 128.
 int32_t ragged_k_launch_long(const RaggedKParams& p, int dtype, int tile, hipStream_t st);

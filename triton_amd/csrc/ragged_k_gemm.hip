@@ -472,23 +472,6 @@ __global__ __launch_bounds__(256, 4) void ragged_k_tr_kernel(const RaggedKParams
   asm volatile("" ::"v"(ahead_a), "v"(ahead_b));
 }
 
-// Tile of the kernel for long slices (ragged_k_long.hip) for aligned operands, 0 = the one above, whose four small workgroups a CU write best where
-// writing is what takes the time.  256 x 256 needs a few rounds of tiles over the 256 CUs, 128 x 128 starts sooner; from 90 k a slice on the former
-// is as good where rounds are many and hardly any of it hangs over the edges.  Measured (us of both products [d, 2 f] and [f, d] of
-// a layer with slices of random lengths; above / 128 / 256):
-//   slices, k of one, d, f: 8, 2048, 2880, 2880 936 / 916 / 827; 8, 256, 2880, 2880 162 / 163 / 155; 16, 1024, 2048, 2048 498 / 491 / 423; 16, 375, 1600, 1200 121 / 110 / 110
-//   32, 512, 2880, 2880 1069 / 1104 / 935; 32, 187, 2880, 2880 477 / 512 / 464; 32, 187, 1600, 1200 135 / 132 / 135; 64, 256, 1024, 1024 168 / 172 / 146; 64, 256, 2880, 2880 1309 / 1357 / 1149
-//   8, 2048, 512, 512 132 / 85 / 192; 8, 256, 512, 512 26 / 21 / 40; 8, 2048, 1024, 1024 162 / 134 / 210; 8, 750, 800, 1024 71 / 55 / 87; 16, 375, 320, 448 39 / 30 / 54; 16, 256,
-//   1024, 1024 60 / 47 / 55; 32, 187, 320, 448 35 / 30 / 48; 32, 187, 800, 1024 77 / 69 / 73; 64, 256, 320, 448 50 / 47 / 54
-//   128, 128, 2880, 2880 1742 / 1903 / 1623; 128, 128, 1440, 1440 456 / 472 / 421; 64, 93, 2880, 2880 706 / 733 / 681; 32, 128, 2880, 2880 407 / 418 / 396; 16, 128, 2880, 2880 202 / 223 / 208
-//   128, 128, 1600, 1200 404 / 438 / 411; 64, 93, 1600, 1200 184 / 196 / 197; 64, 125, 1440, 1440 226 / 242 / 231; 8, 128, 512, 512 15 / 14 / 23; 128, 128, 512, 512 76 / 82 / 76; 128, 46, 2880,
-//   2880 1171 / 1275 / 1221; 16, 64, 1600, 1200 25 / 29 / 30
-int long_tile(int64_t k, int64_t M, int64_t N, int64_t n_slices) {
-  const int64_t tiles = cdiv(M, 256) * cdiv(N, 256) * n_slices;
-  if (k >= 160) return tiles >= 4 * 256 ? 256 : 128;
-  return k >= 90 && tiles >= 24 * 256 && tiles * 256 * 256 * 8 <= M * N * n_slices * 9 ? 256 : 0;
-}
-
 }  // namespace
 }  // namespace tk
 
@@ -546,8 +529,8 @@ extern "C" int32_t tk_ragged_k_gemm(const tk_ragged_k_desc* d, tk_stream_t strea
     const int per_e = p.tiles_m * p.tiles_n;
     p.n_slices = d->n_slices;
     // (rows past M of a long slice's last tiles go by offsets beyond the resource, which may not wrap)
-    const bool long_runs = d->n_slices <= kRaggedKLongSlices && (int64_t)(d->M + 256) * d->y_stride_m * es < (int64_t(1) << 32);
-    const int tile = long_runs ? long_tile(std::min(d->a_k_extent, d->b_k_extent) / d->n_slices, d->M, d->N, d->n_slices) : 0;
+    const bool long_runs = (int64_t)(d->M + 256) * d->y_stride_m * es < (int64_t(1) << 32);
+    const int tile = long_runs ? ragged_k_tile(std::min(d->a_k_extent, d->b_k_extent) / d->n_slices, d->M, d->N, d->n_slices) : 0;
     if (tile) return ragged_k_launch_long(p, d->dtype, tile, st);
     p.chunk = per_e >= 8 ? per_e / 8 : 1;
     // An XCD's part of a slice below 32 tiles: lines asked for six and more slices ahead are gone again or not yet of use (both products of a layer, all by this kernel,
