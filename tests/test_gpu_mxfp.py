@@ -340,3 +340,30 @@ def test_rows_at_any_address_by_tiles_and_by_columns(mx, device, qdt, outer, len
     qo, so = omx.downcast_to_mxfp(x[:4].cpu(), qdt, axis=1)
     _same(qo, q[:4], "values")
     _same(so, s[:4], "scales")
+
+
+@pytest.mark.parametrize("rounding", [omx.ROUND_UP, omx.ROUND_DOWN], ids=["up", "down"])
+@pytest.mark.parametrize("qdt", QTYPES)
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_every_pattern_under_every_scale(mx, device, dt, qdt, rounding):
+    """All 16-bit patterns that a block of each scale can hold, i.e. up to the largest number that has the scale as a block's maximum, subnormal ones among
+    them, along the row and along the column: the oracle's bytes."""
+    import numpy as np
+    mode = mx.DequantScaleRoundingMode(rounding)
+    top = 0x7F80 if dt == torch.bfloat16 else 0x7C00
+    finite = torch.arange(top, dtype=torch.int32).to(torch.int16)
+    bits = omx.scale_bits_from_absmax(finite.view(dt).float().numpy(), omx._kind(qdt), rounding)
+    blocks = []
+    for last in np.flatnonzero(np.append(bits[1:] != bits[:-1], True)):  # (the scale grows with the maximum)
+        p = torch.arange(int(last) + 1, dtype=torch.int32)
+        p = torch.cat([p, p - 0x8000])
+        p = torch.cat([p, torch.full((-len(p) % 31, ), int(last), dtype=torch.int32)]).view(-1, 31)
+        blocks.append(torch.cat([p, torch.full((len(p), 1), int(last), dtype=torch.int32)], dim=1))
+    x = torch.cat(blocks).to(torch.int16).view(dt)
+    vo, so = omx.downcast_to_mxfp(x, qdt, 1, rounding)
+    v, s = mx.downcast_to_mxfp(x.to(device), qdt, axis=1, DEQUANT_SCALE_ROUNDING_MODE=mode)
+    _same(vo, v, "values along the row")
+    _same(so, s, "scales along the row")
+    v, s = mx.downcast_to_mxfp(x.t().contiguous().to(device)[None], qdt, axis=1, DEQUANT_SCALE_ROUNDING_MODE=mode)
+    _same(vo.t().contiguous(), v[0].contiguous(), "values along the column")
+    _same(so.t().contiguous(), s[0].contiguous(), "scales along the column")
