@@ -3,7 +3,7 @@
 //
 // At these sizes the layer is a stream of the active experts' weights (13 MB per expert at the gpt-oss shape) read
 // once from HBM; three launches spend a third of their time on launch boundaries and on the serial router in front
-// of the first weight byte.  Here the grid is persistent and co-resident (one or two workgroups per CU):
+// of the first weight byte.  Here the grid is persistent and co-resident (one workgroup per CU):
 //
 //   1. EVERY workgroup routes all T tokens itself (the logits are a few KiB): top-k by wave-wide max rounds, softmax,
 //      expert histogram, stable expert-sorted row order - into LDS, no global round trip, no dependence on others.
@@ -12,13 +12,13 @@
 //   3. The NW waves of a workgroup share the K-stages of a unit (XS = 1 to 3 each; three: consecutive ones, so that the sums are those of
 //      K / 384 slices added in order; one or two: in turn, which leaves no wave idle); a wave keeps its part of the
 //      block's activation rows in REGISTERS for as long as the (expert, row block) stays the same, so the inner loop
-//      is: 2 KiB weight block global -> registers (ring, one unit ahead), e2m1 -> bf16 in registers, 16x16x32 MFMA.
-//      The slices meet in LDS once per unit (one barrier); four of the waves, in turn, sum them and run the
+//      is: 2 KiB weight block global -> registers (ring of three or four units), e2m1 -> bf16 in registers, 16x16x32 MFMA.
+//      The waves' sums meet in LDS once per unit (one barrier); four of the waves, the even ones of an even unit and the odd ones of an odd one, add them and run the
 //      epilogue.  (One wave in turn: its next unit started late, and the others met it at the barrier; all waves: a quarter of a microsecond of each
 //      one's time.  49 tokens, 64 experts, top 2, d 1952, d_ff 960: 60.7 / 59.4 with four / 59.9 us; 60 tokens, 96 experts, top 4, 2048: 69.5 / 68.9 / 70.1;
 //      61 tokens, 128 experts, top 4, 2880, with favourites: 116.1 / 114.5 / 116.0.)
 //   4. GEMM 1 writes its swiglu'd rows (bf16) to a scratch tensor h with write-through stores; a workgroup that has
-//      finished its GEMM-1 share counts its units in at a per-expert counter.  GEMM-2 units of an expert wait for that
+//      finished its GEMM-1 share counts its units in at a counter per row block.  GEMM-2 units of a block wait for that
 //      counter (their weight blocks are already on their way) and read h around the L2 (the eight XCDs' L2s are not
 //      coherent with each other).
 //   5. GEMM 2 writes gate-weighted rows to y [T*k, N]; when a workgroup has finished its share it counts every
@@ -38,8 +38,8 @@ namespace {
 constexpr int kDecMaxRows = TK_DECODE_MAX_ROWS;        // T * k
 constexpr int kDecMaxExperts = TK_DECODE_MAX_EXPERTS;  // one expert per thread in the placement pass
 constexpr int kDecMaxUnits = 192;                      // units (of one fragment) of a workgroup (the host bounds it)
-constexpr int kDecNW = 8;                              // waves per workgroup = K-slices of a unit
-constexpr int kDecXS = 3;                              // K-stages (of 128) per slice at most: K <= NW * XS * 128 = 3072
+constexpr int kDecNW = 8;                              // waves per workgroup, which share a unit's K-stages
+constexpr int kDecXS = 3;                              // K-stages (of 128) of a wave at most: K <= NW * XS * 128 = 3072
 constexpr int kDecBlockStride = 32;                    // words between two row blocks' counters (a cache line each)
 constexpr int kDecBlockWords = (kDecMaxRows + kDecMaxRows / 16) * kDecBlockStride;  // 16-row blocks: at most min(E, R) + R / 16
 
@@ -51,7 +51,7 @@ struct DecUnit {
   int32_t once;      // its expert has one row block only
 };
 
-// XS: K-stages of a wave's slice, FPU: column fragments of a unit.  A unit costs its chain (weights, products, sums through LDS, barrier) whatever its
+// XS: K-stages of a wave, FPU: column fragments of a unit.  A unit costs its chain (weights, products, sums through LDS, barrier) whatever its
 // bytes, so short K take fewer stages a wave, which leaves registers for a deeper ring or for two fragments a unit.
 template <int XS_, int FPU_>
 struct DecCfg {
@@ -321,8 +321,9 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
   const uint32_t slane = (uint32_t)(lr * 4);
   // weight registers: RD sets of XS stages; unit i lives in set i % RD and, stage by stage as it is consumed, is
   // replaced by unit i + RD.  A wave's requests are answered in order, one unit per unit time, so a block must be
-  // requested RD unit times before it is used: with a loaded memory latency of about 4 us, two sets bound a unit at
-  // 2 us (what was measured), three at 1.3 us, which is below what HBM delivers (19 KiB per wave on its way).
+  // requested RD unit times before it is used: with a loaded memory latency of about 4 us and three stages a wave, two sets bound a unit at
+  // 2 us (what was measured), three at 1.3 us, which is below what HBM delivers (19 KiB per wave on its way).  The shorter units of less K have 17 KiB on
+  // their way (four sets of one stage and two fragments, or of two and one) or 25.5 (three of two and two).
   constexpr int RD = C::RING;
   const __amdgpu_buffer_rsrc_t hrsrc = __builtin_amdgcn_make_buffer_rsrc(p.h, 0, (uint32_t)((int64_t)R * p.K2 * 2), 0x00020000);
   const __amdgpu_buffer_rsrc_t yrsrc = __builtin_amdgcn_make_buffer_rsrc(p.y, 0, (uint32_t)((int64_t)R * p.N2 * 2), 0x00020000);
@@ -428,7 +429,7 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
     };
     auto unit_nst = [&](const DecUnit& u) __attribute__((always_inline)) -> int { return u.key < 0 ? 0 : (u.key >> 24) == 2 ? p.nst2 : p.nst1; };
     auto unit_nfr = [&](const DecUnit& u) __attribute__((always_inline)) -> int { return (u.key >> 24) == 2 ? p.nfr2 : p.nfr1; };
-    // This wave's K-slice of a row block's activation rows: x through the expert-sorted order for GEMM 1, h for GEMM 2.
+    // This wave's stages of a row block's activation rows: x through the expert-sorted order for GEMM 1, h for GEMM 2.
     // The MFMA wants row lr's k-block kg in lane (lr, kg): loaded that way, the sixteen lanes that one pass of a load
     // serves touch sixteen rows, i.e. sixteen cache lines for 16 bytes each.  So the rows are loaded four lanes to a row
     // (lane = row * 4 + chunk: 64 contiguous bytes per row and instruction, rows past the block's last dropped, not
@@ -488,7 +489,7 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
     if (n_units > 0) {
       bias_fetch(0);
       // the first unit's activation slice is requested in front of the weight blocks (a wave's requests are answered in
-      // order, and the three units of weight blocks primed below keep the memory system busy for microseconds)
+      // order, and the units of weight blocks primed below keep the memory system busy for microseconds)
       const DecUnit first = uniform_unit(0);
       const bool x_first = (first.key >> 24) == 1;
       if (x_first) {
@@ -525,7 +526,7 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
       if (i == n1) DEC_STAMP(4);
       if (cur.key != cur_key) {
         cur_key = cur.key;
-        // ---- a new (expert, row block): this wave's K-slice of its activation rows goes into registers ----
+        // ---- a new (expert, row block): this wave's stages of its activation rows go into registers ----
         if (ph == 2) {
           const int blk = bpre_s[a] + rb;  // a block of the first half was computed by run 0 alone
           if (!signalled0 || (blk >= bh && !signalled)) {  // (uniform) see above: count in what this workgroup itself still owes
@@ -558,7 +559,7 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
       }
       if (i == 0) DEC_STAMP(14);
       const int F = cur.frag;
-      // ---- this wave's K-slice of the unit; the next unit's blocks follow into the slots as they fall free ----
+      // ---- this wave's stages of the unit; the next unit's blocks follow into the slots as they fall free ----
       typename FR::acc_t acc[FPU][2];
 #pragma unroll
       for (int f = 0; f < FPU; ++f)
@@ -583,7 +584,7 @@ __global__ __launch_bounds__(kDecNW * 64) __attribute__((amdgpu_waves_per_eu(2, 
         }
         load_w(h_c, j, nxt, nst_next, nfr_next);
       }
-      // ---- the slices meet in LDS; half of the waves, in turn, sum two of the 16 x 32 results a lane in slice order and
+      // ---- the waves' sums meet in LDS; half of the waves, the other half in the next unit, add two of a fragment's 16 x 32 results a lane in the waves' order and
       // finish them (one wave for all of them held up the others' next unit where units are short; all waves: themselves where they are long) ----
       if (i == 0) DEC_STAMP(15);
       DEC_UNIT_STAMP(i);
@@ -731,7 +732,7 @@ int resident_workgroups() {
     int per_cu = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, reinterpret_cast<const void*>(moe_decode_layer_kernel<VPL, XS, FPU, FETCH>), kDecNW * 64, 0) != hipSuccess || per_cu <= 0)
       return 0;
-    per_cu = 1;  // (a wave holds up to two units of weight blocks in its registers: one workgroup fills a CU)
+    per_cu = 1;  // (more than half of a CU's LDS a workgroup)
     n = per_cu * device_cu_count();
     cached[dev].store(n, std::memory_order_relaxed);
   }

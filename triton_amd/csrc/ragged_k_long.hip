@@ -9,10 +9,10 @@
 //     nobody waits for until its fourth stage.
 //   * Slices differ in length by factors: tiles go from the longest slice to the shortest, every XCD takes an eighth of each, and its workgroups walk
 //     their list forth and back.  In a slice tiles run in bands of eight down, so that an XCD's 32 tiles share 12 operand columns instead of 15
-//     (misses of the L2 12.4 to 11.0 million lines a launch, 5 to 6 % of the time).
+//     (lines read past the L2 12.4 to 11.0 million a launch when the bands came in, 5 to 6 % of the time).
 //
-// What bounds it: 256 x 256, the board's power (8 slices of 2048 k, 2880 x 5760 and 2880 x 2880: matrix pipe 66 % busy at 1.55 to 1.6 GHz, 1.0 PFLOP/s, where the vendor's
-// library reaches 1.13 on a square product of 8192 of the same random numbers); 128 x 128, the lines that come to a CU (some 55 KB/us), and with few
+// What bounds it: 256 x 256, slices of thousands, the board's power (8 of 2048 k, 2880 x 5760 and 2880 x 2880: matrix pipe 69 % busy at 1.93 GHz, 1.0 PFLOP/s, where the vendor's
+// library reaches 1.13 on a square product of 8192 of the same random numbers), slices of a hundred, the writing of y (128 of 128, 2880 x 5760: 29 % busy, 4.9 TB/s); 128 x 128, the lines that come to a CU (some 55 KB/us), and with few
 // slices the longest.  Both products of a layer, us, the kernel for short slices / this one: 8 slices of 2048, d and f 2880 946 / 827; 32 of 512 1088 / 935; 128 of 128 1755 / 1623; 8 of
 // 2048, d and f 512 140 / 85.
 // Measured and left out: stores without the non-temporal hint (128 of 128, d and f 1440 421 -> 502), cleared accumulators in place of a first product on zero, whole rows of the tile an
