@@ -201,7 +201,7 @@ def test_scales_at_any_byte(device, e, k, n, sizes, offset, pad):
     assert torch.equal(got, want) and not torch.isnan(got).any()
 
 
-@pytest.mark.parametrize("e, k, n, sizes", [(16, 1792, 2048, [81, 104, 97, 90]), (8, 544, 1056, [96, 128, 64, 100, 33, 129, 90, 95])])
+@pytest.mark.parametrize("e, k, n, sizes", [(16, 1792, 2048, [81, 104, 97, 90]), (8, 576, 1056, [96, 128, 64, 100, 33, 129, 90, 95])])
 def test_mxfp8_rows_without_a_wide_tile(device, e, k, n, sizes):
     """81 to 104 rows a slice where the tiles of 128 x 256 are one round: they run, and give what the wide kernel's 160 x 512 give, bit for bit."""
     import triton_amd._native as nt

@@ -413,7 +413,7 @@ def test_mxfp8_row_blocks_of_256_only_where_the_wide_kernel_has_a_tile():
     from triton_amd import _native as nt
     rules, without = nt.rules(), 0
     for n_slices in (1, 2, 8, 16, 32, 64, 128):
-        for K in (512, 960, 1792, 2880):
+        for K in (576, 960, 1792, 2880):
             for N in (256, 960, 2048, 2880, 5760):
                 for per_slice in (1, 24, 40, 64, 80, 81, 90, 96, 97, 104, 105, 122, 152, 176, 300, 640, 1000):
                     rows = per_slice * n_slices

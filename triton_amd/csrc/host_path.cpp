@@ -222,8 +222,9 @@ int64_t wide_block_m(int64_t rows, int64_t n_slices, int64_t K, int64_t N, uint3
   if (rows <= 80 * n_slices) return 128;
   // (the wide kernel's tiles are asked for by their columns; the other kernel, wherever the rules name none of them, has row blocks of 128: its tiles are one round there, which
   // with row blocks of 256 were 160 x 512 of the wide kernel on a quarter of the CUs.  Layers, us, 16 slices of 90 rows, 1792 and 1024: 80 -> 56; 8 of 96, 2880 105 -> 65; 16 of 84, 1024
-  // 65 -> 48; 32 of 96, 1024 and 512 68 -> 50)
-  if (mx8 && !tk::mxw_tile(rows, n_slices, K, N, mx8).rows) return 128;
+  // 65 -> 48; 32 of 96, 1024 64 -> 50.  K of 512 and 544 with up to 104 rows keep the row block of 256, which callers can see in the descriptor and are promised for the wide
+  // kernel, although 128 is faster there as well: 16 slices of 87, K 512, N 1088 16.3 against 9.8, K 544, N 512 17.2 against 10.5)
+  if (mx8 && (K > 544 || rows > 104 * n_slices) && !tk::mxw_tile(rows, n_slices, K, N, mx8).rows) return 128;
   return !mx8 || rows <= 176 * n_slices || rows >= 640 * n_slices ? 256 : 128;
 }
 
